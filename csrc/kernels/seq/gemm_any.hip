@@ -14,6 +14,7 @@
 // (mixture of experts: rows sorted by expert, offs[g] .. offs[g+1] use weight g).
 #include "seq_common.h"
 #include "fls_seq.h"
+#include "gemm_epi.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
@@ -29,35 +30,6 @@ template <> struct Lds<float> { static constexpr int LD = BK + 1; };
 __device__ __forceinline__ void cvt_store(bf16_t* d, float v) { *d = f_to_bf16(v); }
 __device__ __forceinline__ void cvt_store(float* d, float v) { *d = v; }
 __device__ __forceinline__ void cvt_store(bf16_t* d, bf16_t v) { *d = v; }
-
-// What a kernel does with a finished accumulator element: + bias, optionally an activation (kind 1, xIELU with
-// act = {p, q}: z > 0: softplus(p) z^2 + z/2, else (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2; kind 2: the square
-// of max(z, 0); kind 3, a decay: exp(-exp(act[column / act_n]) softplus(z))), then the store as fp32 or bf16 -- so a projection whose consumer is the next matrix product writes that
-// product's operand directly and the fp32 intermediate never reaches memory.
-struct Epi {
-  const float* bias;
-  const float* act;      // the activation's numbers on the device, if it has any
-  int kind;              // 0 none, 1 xIELU, 2 squared ReLU, 3 decay
-  int tc;                // element type of C: 0 fp32, 1 bf16
-  int act_n;             // kind 3: columns per number of act
-};
-struct EpiRegs { float ap, an; };
-__device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {
-  EpiRegs r = {0.f, 0.f};
-  if (e.kind == 1) { r.ap = softplus_f(e.act[0]); r.an = 0.5f + softplus_f(e.act[1]); }
-  return r;
-}
-// (kind 3: what a lane's column needs, before its elements are emitted)
-__device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
-  if (e.kind == 3) r.ap = -expf(e.act[col / e.act_n]);
-}
-__device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e, const EpiRegs& r) {
-  if (e.kind == 2) { v = fmaxf(v, 0.f); v *= v; }
-  else if (e.kind == 3) v = expf(r.ap * softplus_f(v));
-  else if (e.kind == 1) v = v > 0.f ? r.ap * v * v + 0.5f * v : r.an * (expm1f(v) - v) + 0.5f * v;
-  if (e.tc == 1) reinterpret_cast<bf16_t*>(C)[idx] = f_to_bf16(v);
-  else reinterpret_cast<float*>(C)[idx] = v;
-}
 
 // stage rows [r0, r0 + 64) x columns [k0, k0 + 32) of X (row bound rmax, column bound K) into LDS
 template <typename TS, typename TL>
@@ -421,8 +393,12 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
     SEQ_LAUNCH_CHECK();
     return 0;
   }
-  // tile side by the rows of a group (on average, for row groups): 64, 128, or 256 when the
-  // problem still gives the chip a few hundred blocks
+  if (tw == 1 && ta == 1 && vec_a && vec_w) {
+    const int rc = seq_gemm_tile((const bf16_t*)A, (const bf16_t*)W, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_gs, a_mod, w_gs, c_gs, st0);
+    if (rc != 0) return rc == 1 ? 0 : rc;
+  }
+  // what is left has fp32 rows, ragged K or N, or fp32 weights.  Tile side by the rows of a group (on average, for row
+  // groups): 64, 128, or 256 when the problem still gives the chip a few hundred blocks
   const int gm = offs != nullptr ? M / groups : M;
   int big = 0;
   if (gm > 64 && N > 64) big = 128;

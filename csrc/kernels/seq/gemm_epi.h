@@ -1,0 +1,41 @@
+// What the matrix-product kernels (gemm_any.hip, gemm_tile.hip) do with a finished accumulator.
+#pragma once
+#include "seq_common.h"
+
+// What a kernel does with a finished accumulator element: + bias, optionally an activation (kind 1, xIELU with
+// act = {p, q}: z > 0: softplus(p) z^2 + z/2, else (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2; kind 2: the square
+// of max(z, 0); kind 3, a decay: exp(-exp(act[column / act_n]) softplus(z))), then the store as fp32 or bf16 -- so a projection whose consumer is the next matrix product writes that
+// product's operand directly and the fp32 intermediate never reaches memory.
+struct Epi {
+  const float* bias;
+  const float* act;      // the activation's numbers on the device, if it has any
+  int kind;              // 0 none, 1 xIELU, 2 squared ReLU, 3 decay
+  int tc;                // element type of C: 0 fp32, 1 bf16
+  int act_n;             // kind 3: columns per number of act
+};
+struct EpiRegs { float ap, an; };
+__device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {
+  EpiRegs r = {0.f, 0.f};
+  if (e.kind == 1) { r.ap = softplus_f(e.act[0]); r.an = 0.5f + softplus_f(e.act[1]); }
+  return r;
+}
+// (kind 3: what a lane's column needs, before its elements are emitted)
+__device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
+  if (e.kind == 3) r.ap = -expf(e.act[col / e.act_n]);
+}
+__device__ __forceinline__ float epi_value(float v, const Epi& e, const EpiRegs& r) {
+  if (e.kind == 2) { v = fmaxf(v, 0.f); v *= v; }
+  else if (e.kind == 3) v = expf(r.ap * softplus_f(v));
+  else if (e.kind == 1) v = v > 0.f ? r.ap * v * v + 0.5f * v : r.an * (expm1f(v) - v) + 0.5f * v;
+  return v;
+}
+__device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e, const EpiRegs& r) {
+  v = epi_value(v, e, r);
+  if (e.tc == 1) reinterpret_cast<bf16_t*>(C)[idx] = f_to_bf16(v);
+  else reinterpret_cast<float*>(C)[idx] = v;
+}
+
+// gemm_tile.hip: the product of bf16 rows and bf16 weights on LDS-DMA tiles.  1: launched; 0: not a shape it serves;
+// < 0: failed.
+int seq_gemm_tile(const bf16_t* A, const bf16_t* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
+                  const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s);

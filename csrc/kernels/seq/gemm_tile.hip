@@ -1,0 +1,512 @@
+// C[M,N] = epilogue(A[M,K] . W[N,K]^T), bf16 operands, fp32 accumulation: the prompt projections of the stateful models.
+//
+// Both operands go from global memory to LDS by DMA (no registers in between), 64 columns of K at a time, 1 KiB pieces of
+// 8 rows x 128 bytes whose 16-byte chunks are XOR-swizzled by the row (chunk c of row r in slot c ^ (r & 7)), so that the
+// 16-byte fragment reads of 16x16x32 MFMAs have no bank conflicts.  Rows past M and columns past N re-read the last valid row
+// (never out of bounds) and are not stored.
+#include "seq_common.h"
+#include "fls_seq.h"
+#include "gemm_epi.h"
+
+namespace {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+#define LDS_AS __attribute__((address_space(3)))
+
+struct Tile {
+  const bf16_t* A;
+  const bf16_t* W;
+  void* C;
+  Epi epi;
+  int M, N, K, lda, ldw, ldc;
+  const int* offs;          // row groups (experts): group g owns rows offs[g] .. offs[g + 1] and weight g
+  int groups;
+  long long w_gs, a_gs, c_gs;   // strided batch (grid y): operand and column offsets of group g
+  int a_mod;
+  int tiles_m, tiles_n, order;
+};
+
+// Virtual tile id -> (tile row, tile column): groups of `order` tiles of one dimension (order < 0: of N) walked along the
+// other; with consecutive ids on one XCD, an XCD's concurrent tiles are a compact patch whose operand panels its L2 holds.
+__device__ __forceinline__ int2 place(int b, int tiles_m, int tiles_n, int order) {
+  const bool by_m = order > 0;
+  const int g = by_m ? order : -order;
+  const int along = by_m ? tiles_n : tiles_m, total = by_m ? tiles_m : tiles_n;
+  const int first = b / (g * along) * g;
+  const int size = min(total - first, g);
+  const int in = b - first * along;
+  const int grouped = first + in % size, walked = in / size;
+  return by_m ? int2{grouped, walked} : int2{walked, grouped};
+}
+
+// This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
+template <int TM, int TN>
+__device__ __forceinline__ bool locate(const Tile& a, const bf16_t*& A, const bf16_t*& W, size_t& cbase, int& m0, int& mend, int& n0) {
+  const int nwg = gridDim.x;
+  int bid = blockIdx.x;
+  {                                      // blocks go to the 8 XCDs in turn: give each a run of consecutive ids
+    const int q = nwg >> 3, r = nwg & 7, xcd = bid & 7, loc = bid >> 3;
+    bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
+  }
+  const int2 t = place(bid, a.tiles_m, a.tiles_n, a.order);
+  int tm = t.x;
+  A = a.A;
+  W = a.W;
+  cbase = 0;
+  mend = a.M;
+  n0 = t.y * TN;
+  m0 = 0;
+  if (a.offs != nullptr) {               // tiles of the groups one after the other: find the one that owns tile tm
+    const int lane = threadIdx.x & 63;
+    int e = -1;
+    for (int base = 0; base < a.groups; base += 64) {
+      const int g = base + lane;
+      const int cnt = g < a.groups ? (a.offs[g + 1] - a.offs[g] + TM - 1) / TM : 0;
+      int pre = cnt;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(pre, o, 64);
+        if (lane >= o) pre += v;
+      }
+      const unsigned long long past = __ballot(pre > tm);
+      if (past != 0) {
+        const int l = __builtin_ctzll(past);
+        e = base + l;
+        tm -= __shfl(pre, l, 64) - __shfl(cnt, l, 64);
+        break;
+      }
+      tm -= __shfl(pre, 63, 64);
+    }
+    if (e < 0) return false;
+    e = __builtin_amdgcn_readfirstlane(e);
+    tm = __builtin_amdgcn_readfirstlane(tm);
+    m0 = a.offs[e];
+    mend = a.offs[e + 1];
+    W += (size_t)e * a.w_gs;
+  } else if (gridDim.y > 1) {
+    const int g = blockIdx.y;
+    A += (size_t)(g % a.a_mod) * a.a_gs;
+    W += (size_t)g * a.w_gs;
+    cbase = (size_t)g * a.c_gs;
+  }
+  m0 += tm * TM;
+  return true;
+}
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, bool live) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, live ? -1 : 0, 0x00020000);
+}
+
+// four consecutive columns as fp32, or rounded to nearest even as bf16
+template <int TC>
+__device__ __forceinline__ void store4(void* C, size_t idx, floatx4 v) {
+  if constexpr (TC == 1) {
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(C) + idx) = __builtin_convertvector(v, bf16x4);
+  } else {
+    *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(C) + idx) = v;
+  }
+}
+
+// (ACC: the accumulators are in accumulation registers, written by asm; each stays there until it is used)
+template <bool ACC>
+__device__ __forceinline__ void hold(floatx4& c) {
+  if constexpr (ACC) asm volatile("" : "+a"(c));
+}
+
+// A wave's outputs: acc[u][t] = rows mw + 16 u + (lane & 15), columns nw + 16 t + 4 (lane >> 4) .. + 3.  Without an activation
+// they leave straight from the registers.  An activation runs in a short loop over rows that the wave first lays down in
+// its own piece of LDS (PU row groups at a time): unrolled over all accumulators its code would be larger than the cache.
+template <int MI, int NJ, int PU, bool ACC, int TC>
+__device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
+  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+  const Epi& e = a.epi;
+  if (e.kind == 0) {
+#pragma unroll
+    for (int t = 0; t < NJ; ++t) {
+      asm volatile("" ::: "memory");                        // (one column group at a time: fewer live registers)
+      const int n = nw + t * 16 + 4 * grp;
+      if (n < a.N) {
+        floatx4 b = {0.f, 0.f, 0.f, 0.f};
+        if (e.bias != nullptr) b = *reinterpret_cast<const floatx4*>(e.bias + cbase + n);
+        const size_t at = cbase + (size_t)(mw + fr) * a.ldc + n;
+#pragma unroll
+        for (int u = 0; u < MI; ++u) {
+          hold<ACC>(acc[u][t]);
+          if (mw + u * 16 + fr < mend) store4<TC>(a.C, at + (size_t)(u * 16) * a.ldc, acc[u][t] + b);
+        }
+      }
+    }
+    return;
+  }
+  constexpr int CH = 4 * NJ, RI = 64 / CH;          // 16-byte chunks of a row; rows per step of the loop
+  const EpiRegs er0 = epi_regs(e);
+  const int c = lane % CH, n = nw + 4 * c;
+  EpiRegs er[4] = {er0, er0, er0, er0};
+  floatx4 b = {0.f, 0.f, 0.f, 0.f};
+  if (n < a.N) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) epi_column(e, er[i], n + i);
+    if (e.bias != nullptr) b = *reinterpret_cast<const floatx4*>(e.bias + cbase + n);
+  }
+#pragma unroll
+  for (int p = 0; p < MI / PU; ++p) {
+#pragma unroll
+    for (int u = 0; u < PU; ++u)
+#pragma unroll
+      for (int t = 0; t < NJ; ++t) {
+        const int r = u * 16 + fr;
+        hold<ACC>(acc[p * PU + u][t]);
+        *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = acc[p * PU + u][t];
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the wave's own rows: no other wave reads them)
+#pragma unroll 1
+    for (int i = 0; i < 16 * PU; i += RI) {
+      const int r = i + lane / CH;
+      floatx4 v = *reinterpret_cast<const floatx4*>(lds + (r * CH + (c ^ (r & (CH - 1)))) * 16) + b;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) v[x] = epi_value(v[x], e, er[x]);
+      const int m = mw + p * PU * 16 + r;
+      if (m < mend && n < a.N) store4<TC>(a.C, cbase + (size_t)m * a.ldc + n, v);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+template <int MI, int NJ, int PU, bool ACC = false>
+__device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
+  if (a.epi.tc == 1) finish_as<MI, NJ, PU, ACC, 1>(a, acc, cbase, mw, nw, mend, lds);
+  else finish_as<MI, NJ, PU, ACC, 0>(a, acc, cbase, mw, nw, mend, lds);
+}
+
+// ------------------------------------------------------------------------------------ 256 x 256
+// Four waves, one per SIMD, 128 x 128 outputs each: all 256 accumulation registers of a wave.  A fragment read from LDS
+// feeds 8 MFMAs.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
+// accumulation register the compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between
+// them; reads run one phase of 32 MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
+namespace t256 {
+constexpr int TM = 256, TN = 256, KT = 64, STG = 65536, WIMG = 32768, LDS_BYTES = 2 * STG;
+}
+
+__device__ __forceinline__ void mfma_in_place(floatx4& c, const bf16x8& a, const bf16x8& b) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
+}
+
+__global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
+  using namespace t256;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const bf16_t *A, *W;
+  size_t cbase;
+  int m0, mend, n0;
+  if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // DMA: a half-tile is 16 pieces, rows (j >> 3) 128 + (j & 7) 8 (+ 64: the second half); a wave moves pieces 4 wave .. + 3
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  int prow[4];
+  unsigned xo[8], wo[8];
+  const int mlast = mend - 1 - m0, nlast = a.N - 1 - n0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int j = 4 * wave + i;
+    prow[i] = (j >> 3) * 128 + (j & 7) * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      xo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, mlast) * a.lda + lc * 8) * 2u;
+      wo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, nlast) * a.ldw + lc * 8) * 2u;
+    }
+  }
+  const char* Ab = reinterpret_cast<const char*>(A + (size_t)m0 * a.lda);
+  const char* Wb = reinterpret_cast<const char*>(W + (size_t)n0 * a.ldw);
+  // (past the last K tile the DMAs go through a descriptor of no records: counted like the others, they write zeros)
+  const __amdgpu_buffer_rsrc_t rA = rsrc_of(Ab, true), rW = rsrc_of(Wb, true), r0 = rsrc_of(Ab, false);
+#define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, (k0) * 2, 0, 0)
+#define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[(h) * 4 + (i)], k0, smem + (buf) * STG + (prow[i] + (h) * 64) * 128)
+#define T_W(rs, buf, h, i, k0) T_DMA(rs, wo[(h) * 4 + (i)], k0, smem + (buf) * STG + WIMG + (prow[i] + (h) * 64) * 128)
+  const int wm = wave >> 1, wn = wave & 1;
+  const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
+  const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
+  const int xrow = (wm * 128 + fr) * 128, wrow = WIMG + (wn * 128 + fr) * 128;
+  floatx4 acc[8][8];
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 xf[8][2], wf[8][2];
+#define T_HOLD()                                                                                   \
+  _Pragma("unroll") for (int u_ = 0; u_ < 8; ++u_)                                                 \
+  _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+a"(acc[u_][t_]));
+  T_HOLD();
+  asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");          // (the zeros are written before the first MFMA reads them)
+#define T_RX(buf, f, k) xf[f][k] = *(const bf16x8*)(smem + (buf) * STG + xrow + (f) * 2048 + ((k) ? c1 : c0))
+#define T_RW(buf, f, k) wf[f][k] = *(const bf16x8*)(smem + (buf) * STG + wrow + (f) * 2048 + ((k) ? c1 : c0))
+// 32 MFMAs of the quadrant (x half xh, w half wh); after the first even ones the 8 reads of the half needed next (RX: of x),
+// after four later ones the DMAs of a half-tile (DX: of x)
+#define T_PHASE(xh, wh, RX, rbuf, rh, DX, rs, dbuf, dh, dk, SYNC)                                  \
+  {                                                                                                \
+    _Pragma("unroll") for (int i_ = 0; i_ < 32; ++i_) {                                            \
+      const int s_ = i_ >> 4, u_ = (xh) * 4 + ((i_ >> 2) & 3), t_ = (wh) * 4 + (i_ & 3);           \
+      mfma_in_place(acc[u_][t_], wf[t_][s_], xf[u_][s_]);                                          \
+      if (i_ < 16 && (i_ & 1) == 0) {                                                              \
+        const int f_ = (rh) * 4 + (i_ >> 2), k_ = (i_ >> 1) & 1;                                   \
+        if (RX) T_RX(rbuf, f_, k_);                                                                \
+        else T_RW(rbuf, f_, k_);                                                                   \
+      }                                                                                            \
+      if (i_ >= 17 && i_ <= 26 && (i_ - 17) % 3 == 0) {                                            \
+        if (DX) T_X(rs, dbuf, dh, (i_ - 17) / 3, dk);                                              \
+        else T_W(rs, dbuf, dh, (i_ - 17) / 3, dk);                                                 \
+      }                                                                                            \
+    }                                                                                              \
+    if (SYNC) {                                                                                    \
+      asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");                                 \
+      __builtin_amdgcn_s_barrier();                                                                \
+    }                                                                                              \
+  }
+// a K tile held by buffer 0: w halves 0, 1; by buffer 1: w halves 1, 0 (each phase reads one half for the next one)
+#define T_EVEN(rx, rw, dk)                                                                         \
+  T_PHASE(0, 0, 0, 0, 1, 1, rx, 0, 0, dk, 0)                                                       \
+  T_PHASE(0, 1, 1, 0, 1, 0, rw, 0, 0, dk, 1)                                                       \
+  T_PHASE(1, 1, 1, 1, 0, 0, rw, 0, 1, dk, 0)                                                       \
+  T_PHASE(1, 0, 0, 1, 1, 1, rx, 0, 1, dk, 1)
+#define T_ODD(rx, rw, dk)                                                                          \
+  T_PHASE(0, 1, 0, 1, 0, 1, rx, 1, 0, dk, 0)                                                       \
+  T_PHASE(0, 0, 1, 1, 1, 0, rw, 1, 1, dk, 1)                                                       \
+  T_PHASE(1, 0, 1, 0, 0, 0, rw, 1, 0, dk, 0)                                                       \
+  T_PHASE(1, 1, 0, 0, 0, 1, rx, 1, 1, dk, 1)
+  const int nk = a.K / KT;
+  {
+    const __amdgpu_buffer_rsrc_t rA1 = nk > 1 ? rA : r0, rW1 = nk > 1 ? rW : r0;
+    const int k1 = nk > 1 ? KT : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_X(rA, 0, 0, i, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_W(rW, 0, 0, i, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_W(rW, 0, 1, i, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_X(rA, 0, 1, i, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_X(rA1, 1, 0, i, k1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_W(rW1, 1, 1, i, k1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_W(rW1, 1, 0, i, k1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) T_X(rA1, 1, 1, i, k1);
+  }
+  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {
+    T_RX(0, f, 0); T_RX(0, f, 1);
+    T_RW(0, f, 0); T_RW(0, f, 1);
+  }
+  asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  // (an odd last K tile is followed by one of zeros, which is what a DMA without records leaves in LDS: a loop exit in the
+  // middle would have the compiler move accumulators between registers while asm MFMAs it cannot see are still writing them)
+  int kt = 0;
+  do {
+    const bool more2 = kt + 2 < nk, more3 = kt + 3 < nk;
+    const int k2 = more2 ? (kt + 2) * KT : 0, k3 = more3 ? (kt + 3) * KT : 0;
+    const __amdgpu_buffer_rsrc_t rx2 = more2 ? rA : r0, rw2 = more2 ? rW : r0, rx3 = more3 ? rA : r0, rw3 = more3 ? rW : r0;
+    T_EVEN(rx2, rw2, k2)
+    T_ODD(rx3, rw3, k3)
+    asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");      // (the last MFMAs' passes, before anything may move an accumulator)
+    kt += 2;
+  } while (kt < nk);
+  // every DMA has landed and every wave is done with the tiles before LDS changes its use; the nops give the last MFMAs,
+  // which the compiler cannot see, their passes before the accumulators are read
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#undef T_HOLD
+#undef T_RX
+#undef T_RW
+#undef T_PHASE
+#undef T_EVEN
+#undef T_ODD
+#undef T_X
+#undef T_W
+  finish<8, 8, 4, true>(a, acc, cbase, m0 + wm * 128, n0 + wn * 128, mend, smem + wave * 32768);
+}
+
+// ------------------------------------------------------------------------------------ smaller tiles
+// 32 MI x 32 NJ outputs, four waves in a 2 x 2 grid of 16 MI x 16 NJ, S stages of LDS: the DMAs of K tile t + S - 1 are issued
+// while tile t is multiplied, one barrier per K tile.  What bounds them is the chain of one K tile (wait, barrier, LDS read,
+// MFMA), 0.5 us or more for one wave a SIMD whatever the tile: KG groups of four waves take every KG-th K tile each, so that a
+// SIMD has KG chains to run (256 x 2048 x 2048 in 64 x 64 tiles: 16 us with one group, 12 with two).
+template <int MI, int NJ>
+__device__ __forceinline__ void fill(const char* Ab, const char* Wb, int kt, int nk, int wave, const unsigned* xo, const unsigned* wo,
+                                     char* stg) {
+  const bool live = kt < nk;             // (past the last K tile: a descriptor of no records; counted like the others, nothing reads what they leave)
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(Ab, live), rw = rsrc_of(Wb, live);
+  const int k0 = live ? kt * 64 : 0;
+#pragma unroll
+  for (int i = 0; i < MI; ++i) T_DMA(ra, xo[i], k0, stg + (MI * wave + i) * 1024);
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) T_DMA(rw, wo[i], k0, stg + 32 * MI * 128 + (NJ * wave + i) * 1024);
+}
+
+template <int MI, int NJ, int S, int OCC, int KG>
+__global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
+  constexpr int TM = 32 * MI, TN = 32 * NJ, STG = (TM + TN) * 128, WIMG = TM * 128;
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  const bf16_t *A, *W;
+  size_t cbase;
+  int m0, mend, n0;
+  if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
+  const int lane = threadIdx.x & 63;
+  const int wall = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = wall & 3, kg = wall >> 2;
+  char* smem = smem_all + kg * (S * STG);
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  const int mlast = mend - 1 - m0, nlast = a.N - 1 - n0;
+  unsigned xo[MI], wo[NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i) xo[i] = (unsigned)(min((MI * wave + i) * 8 + lr, mlast) * a.lda + lc * 8) * 2u;
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) wo[i] = (unsigned)(min((NJ * wave + i) * 8 + lr, nlast) * a.ldw + lc * 8) * 2u;
+  const char* Ab = reinterpret_cast<const char*>(A + (size_t)m0 * a.lda);
+  const char* Wb = reinterpret_cast<const char*>(W + (size_t)n0 * a.ldw);
+  const int nk = a.K / 64;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
+  const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
+  const int xrow = (wm * 16 * MI + fr) * 128, wrow = WIMG + (wn * 16 * NJ + fr) * 128;
+  floatx4 acc[MI][NJ];
+#pragma unroll
+  for (int u = 0; u < MI; ++u)
+#pragma unroll
+    for (int t = 0; t < NJ; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < S - 1; ++s) fill<MI, NJ>(Ab, Wb, s * KG + kg, nk, wave, xo, wo, smem + s * STG);
+  int cur = 0, nxt = S - 1;
+  for (int kt = kg; kt < nk + kg; kt += KG) {
+    // this wave's pieces of tile kt have landed and its reads of the tile before are done; after the barrier, everyone's
+    asm volatile("" ::: "memory");
+    constexpr int LEFT = (S - 2) * (MI + NJ);               // DMAs of later K tiles that may stay in flight
+    __builtin_amdgcn_s_waitcnt((LEFT & 15) | (LEFT >> 4) << 14 | 0x70);       // vmcnt(LEFT) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fill<MI, NJ>(Ab, Wb, kt + (S - 1) * KG, nk, wave, xo, wo, smem + nxt * STG);
+    const char* stg = smem + cur * STG;
+    bf16x8 x[2][MI], w[2][NJ];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const int c = k ? c1 : c0;
+#pragma unroll
+      for (int u = 0; u < MI; ++u) x[k][u] = *(const bf16x8*)(stg + xrow + u * 2048 + c);
+#pragma unroll
+      for (int t = 0; t < NJ; ++t) w[k][t] = *(const bf16x8*)(stg + wrow + t * 2048 + c);
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int u = 0; u < MI; ++u)
+#pragma unroll
+        for (int t = 0; t < NJ; ++t) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k][t], x[k][u], acc[u][t], 0, 0, 0);
+    cur = cur + 1 == S ? 0 : cur + 1;
+    nxt = nxt + 1 == S ? 0 : nxt + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  constexpr int OUT = 16 * MI * 16 * NJ * 4;                // a wave's accumulators
+  if constexpr (KG > 1) {                                    // the wave groups' partial sums meet in LDS, in the groups' order
+    if (kg > 0) {
+#pragma unroll
+      for (int u = 0; u < MI; ++u)
+#pragma unroll
+        for (int t = 0; t < NJ; ++t)
+          *reinterpret_cast<floatx4*>(smem_all + ((kg - 1) * 4 + wave) * OUT + ((u * NJ + t) * 64 + lane) * 16) = acc[u][t];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; ++g)
+#pragma unroll
+      for (int u = 0; u < MI; ++u)
+#pragma unroll
+        for (int t = 0; t < NJ; ++t)
+          acc[u][t] += *reinterpret_cast<const floatx4*>(smem_all + ((g - 1) * 4 + wave) * OUT + ((u * NJ + t) * 64 + lane) * 16);
+  }
+  finish<MI, NJ, MI>(a, acc, cbase, m0 + wm * 16 * MI, n0 + wn * 16 * NJ, mend, smem_all + wave * OUT);
+}
+#undef T_DMA
+
+int pick_order(int tiles_m, int tiles_n) {
+  if (tiles_n % 8 == 0)
+    for (int g = 4; g <= 8; ++g)
+      if ((tiles_n / 8) % g == 0) return -g;
+  if (tiles_m % 8 == 0)
+    for (int g = 4; g <= 8; ++g)
+      if ((tiles_m / 8) % g == 0) return g;
+  return -4;
+}
+
+template <auto KERNEL>
+int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
+  // (row groups: each may end in a tile of its own)
+  t.tiles_m = (t.M + tm - 1) / tm + (t.offs != nullptr ? t.groups - 1 : 0);
+  t.tiles_n = (t.N + tn - 1) / tn;
+  t.order = pick_order(t.tiles_m, t.tiles_n);
+  static const hipError_t e = hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return -(int)e;
+  hipLaunchKernelGGL(KERNEL, dim3(t.tiles_m * t.tiles_n, t.offs == nullptr ? t.groups : 1), dim3(threads), lds, s, t);
+  const hipError_t l = hipGetLastError();
+  return l == hipSuccess ? 1 : -(int)l;
+}
+
+}  // namespace
+
+// The tiles, and what a launch of each costs: rounds of `slots` blocks (what the chip holds at once), each K / 64 K tiles and
+// a start and a store.  us per K tile and per round, measured on full rounds at K = 2048 .. 8192 (one MI355X):
+//   256 x 256   1.35  12    least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
+//   128 x 128   1.0    9    two blocks a CU
+//   128 x 128   0.55   6    eight waves, two wave groups each taking every other K tile
+//    64 x 128   0.40   5    the same
+//    64 x 64    0.26   3    the same
+//    32 x 64    0.16   3.5  sixteen waves, four wave groups
+//    32 x 32    0.12   3.5  the same
+// A launch that leaves CUs idle in its last (or only) round wants smaller tiles, a long one the large tile; the cheapest sum
+// wins (1024 x 2048 x 2048: 64 x 128 at 18 us, the 256 tile 45; 256 x 2048 x 2048: 32 x 64 at 9 us, the 256 tile 45;
+// 16384 x 14336 x 4096: the 256 tile at 1.49 ms, 128 x 128 at 2.28).
+struct TileCost { int tm, tn, slots; float k_us, round_us; };
+static const TileCost TILES[] = {{256, 256, 256, 1.35f, 12.f}, {128, 128, 512, 1.0f, 9.f}, {128, 128, 256, 0.55f, 6.f}, {64, 128, 256, 0.40f, 5.f},
+                                 {64, 64, 256, 0.26f, 3.f}, {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f}};
+
+static int pick_tile(int M, int N, int K, int groups, bool by_rows) {
+  int best = 0;
+  float least = 0.f;
+  for (int v = 0; v < (int)(sizeof(TILES) / sizeof(TILES[0])); ++v) {
+    const TileCost& t = TILES[v];
+    // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average)
+    const long long rows = by_rows ? (long long)M / t.tm + (groups + 1) / 2 : (long long)((M + t.tm - 1) / t.tm) * groups;
+    const long long tiles = rows * ((N + t.tn - 1) / t.tn);
+    const float us = (float)((tiles + t.slots - 1) / t.slots) * ((float)(K / 64) * t.k_us + t.round_us);
+    if (v == 0 || us < least) {
+      least = us;
+      best = v;
+    }
+  }
+  return best;
+}
+
+int seq_gemm_tile(const bf16_t* A, const bf16_t* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
+                  const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
+  // whole K tiles; stores of four columns; 32-bit offsets within a tile
+  if (K % 64 || N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16)) return 0;
+  if ((long long)lda * 512 + K * 2LL >= (1LL << 31) || (long long)ldw * 512 + K * 2LL >= (1LL << 31)) return 0;
+  if (offs == nullptr && groups > 65535) return 0;
+  const Tile t = {A, W, C, epi, M, N, K, lda, ldw, ldc, offs, groups, w_gs, a_gs, c_gs, a_mod < 1 ? 1 : a_mod, 0, 0, 0};
+  switch (pick_tile(M, N, K, groups, offs != nullptr)) {
+    case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
+    case 1: return start<gemm_tile_mid<4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
+    case 2: return start<gemm_tile_mid<4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
+    case 3: return start<gemm_tile_mid<2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
+    case 4: return start<gemm_tile_mid<2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
+    case 5: return start<gemm_tile_mid<1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
+    default: return start<gemm_tile_mid<1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
+  }
+}

@@ -75,6 +75,29 @@ def test_matmul(ops, cdt, tol, M, N, K):
     close(H.matmul_nt(af, w), R.matmul_nt(af.to(cdt), w), 1e-5)
 
 
+# one shape for each tile of gemm_tile.hip (256 x 256, 128 x 128 twice, 64 x 128, 64 x 64, 32 x 64, 32 x 32), with rows and
+# columns past a tile's end and odd numbers of 64-wide K tiles.  fp32 sums of bf16 products: 1e-5; rounded to bf16: half a
+# unit in the last place of the largest value (2^-9) and the other side's sum
+@pytest.mark.parametrize("M,N,K", [(2100, 4100, 64), (4100, 4100, 192), (1030, 4000, 64), (1024, 3900, 320), (1000, 2000, 320), (257, 2020, 320),
+                                   (200, 2000, 1088), (65, 132, 448)])
+def test_matmul_tiles(ops, M, N, K):
+    H, R = ops
+    torch.manual_seed(M + N + K)
+    a = torch.randn(M, K + 8, device=DEV).bfloat16()[:, 8:]
+    w = (0.1 * torch.randn(N, K, device=DEV)).bfloat16()
+    b = torch.randn(N, device=DEV)
+    close(H.matmul_nt(a, w, b), R.matmul_nt(a, w, b), 1e-5)
+    close(H.matmul_nt(a, w, out_dtype=torch.bfloat16), R.matmul_nt(a, w, out_dtype=torch.bfloat16), 2 ** -8)
+    act = torch.tensor([0.4, -0.3], device=DEV)
+    close(H.matmul_nt(a, w, b, xielu=act), R.matmul_nt(a, w, b, xielu=act), 1e-5)
+    rates = torch.tensor([0.2, -0.5, 0.1, 0.3], device=DEV)
+    close(H.matmul_nt(a, w, b, decay=rates), R.matmul_nt(a, w, b, decay=rates), 1e-5)
+    E = 5                                                           # row groups, empty ones among them
+    offs = torch.tensor([0, 0, M // 2, M // 2 + 1, M, M], dtype=torch.int32, device=DEV)
+    wg = (0.1 * torch.randn(E, N, K, device=DEV)).bfloat16()
+    close(H.grouped_matmul_nt(a, wg, offs), R.grouped_matmul_nt(a, wg, offs), 1e-5)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_rows(ops, cdt, tol):
     H, R = ops
