@@ -1,5 +1,6 @@
 // C[M,N] fp32 = A[M,K] . W[N,K]^T (+ bias): the matrix product of the stateful models, for bf16 and
-// for true-fp32 operands, with fp32 accumulation on the matrix cores.
+// for true-fp32 operands, with fp32 accumulation on the matrix cores: the entry point, and the kernels for any size and
+// alignment (aligned rows go to gemm_rows.hip and gemm_tile.hip).
 //
 // A 64 x 64 block tile, four wavefronts in a 2 x 2 grid, one 32 x 32 MFMA accumulator each (16
 // fp32 per lane).  K advances 32 at a time through LDS: 256 threads stage 64 x 32 of A and of W
@@ -284,76 +285,6 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_nt_big(const TA* __restri
   }
 }
 
-// ------------------------------------------------------------------------- few rows (decoding)
-// M <= 32 rows against bf16 weights: the product is a stream of W through the chip once, so the
-// kernel is shaped for bandwidth.  A block owns 32 output columns; its four waves split K in chunks
-// of 64 taken in turn, each lane reading its own W row (and A row) 16 bytes at a time straight from
-// global memory -- a lane pair covers a whole 128-byte line of a row per chunk -- into one 32x32x16 MFMA
-// accumulator (rows beyond M are zero).  The four partial accumulators meet in LDS.
-template <typename TA>
-__device__ __forceinline__ bf16x8 load8(const TA* p) {
-  if constexpr (sizeof(TA) == 2) {
-    const uint4 v = *reinterpret_cast<const uint4*>(p);
-    return *reinterpret_cast<const bf16x8*>(&v);
-  } else {
-    const float4 a = *reinterpret_cast<const float4*>(p), b = *reinterpret_cast<const float4*>(p + 4);
-    bf16_t e[8] = {f_to_bf16(a.x), f_to_bf16(a.y), f_to_bf16(a.z), f_to_bf16(a.w),
-                   f_to_bf16(b.x), f_to_bf16(b.y), f_to_bf16(b.z), f_to_bf16(b.w)};
-    return *reinterpret_cast<const bf16x8*>(e);
-  }
-}
-
-template <typename TA>
-__global__ __launch_bounds__(256) void gemm_nt_skinny(const TA* __restrict__ A, const bf16_t* __restrict__ W, void* __restrict__ C,
-                                                      Epi epi, int M, int N, int K, int lda, int ldw, int ldc,
-                                                      const int* __restrict__ offs, long long w_gs) {
-  __shared__ float red[4][16][64];
-  if (offs != nullptr) {                   // row groups (experts): this block's group owns rows offs[g] .. offs[g+1]
-    const int g = blockIdx.y, r0 = offs[g];
-    M = offs[g + 1] - r0;
-    if (M <= 0) return;
-    A += (size_t)r0 * lda;
-    C = reinterpret_cast<char*>(C) + (size_t)r0 * ldc * (epi.tc == 1 ? 2 : 4);
-    W += (size_t)g * w_gs;
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int ql = lane & 31, h2 = lane >> 5;
-  const int col = blockIdx.x * 32 + ql;
-  const bool rowok = ql < M, colok = col < N;
-  const bf16_t* wp = W + (size_t)(colok ? col : 0) * ldw;
-  const TA* ap = A + (size_t)(rowok ? ql : 0) * lda;
-  floatx16 acc;
-#pragma unroll
-  for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-  const uint4 z4 = make_uint4(0, 0, 0, 0);
-  for (int kc = wave * 64; kc < K; kc += 256) {
-#pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) {
-      const int k = kc + 16 * s2 + 8 * h2;
-      bf16x8 a = *reinterpret_cast<const bf16x8*>(&z4), b = a;
-      if (k + 8 <= K) {
-        if (colok) b = load8<bf16_t>(wp + k);
-        if (rowok) a = load8<TA>(ap + k);
-      }
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 16; ++r) red[wave][r][lane] = acc[r];
-  __syncthreads();
-  if (colok) {
-    EpiRegs er = epi_regs(epi);
-    epi_column(epi, er, col);
-    const float bv = epi.bias != nullptr ? epi.bias[col] : 0.f;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) {
-      const int r = wave * 4 + x;
-      const int row = (r >> 2) * 8 + h2 * 4 + (r & 3);
-      if (row < M) emit(C, (size_t)row * ldc + col, red[0][r][lane] + red[1][r][lane] + red[2][r][lane] + red[3][r][lane] + bv, epi, er);
-    }
-  }
-}
-
 static bool aligned16(const void* p, long long ld_elems, int esize, int K) {
   return ((uintptr_t)p % 16 == 0) && ((ld_elems * esize) % 16 == 0) && (K % 8 == 0);
 }
@@ -384,20 +315,17 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
   const int vec_a = aligned16(A, lda, ea, K) && (a_gs * ea) % 16 == 0;
   const int vec_w = aligned16(W, ldw, ew, K) && (w_gs * ew) % 16 == 0;
-  hipStream_t st0 = (hipStream_t)s;
-  // (row groups: M bounds every group's rows, so M <= 32 means every group fits the kernel's 32 rows)
-  if ((groups == 1 || offs != nullptr) && tw == 1 && M <= 32 && vec_a && vec_w) {
-    dim3 g((N + 31) / 32, offs != nullptr ? groups : 1);
-    if (ta == 1) hipLaunchKernelGGL((gemm_nt_skinny<bf16_t>), g, dim3(256), 0, st0, (const bf16_t*)A, (const bf16_t*)W, C, bias, M, N, K, lda, ldw, ldc, offs, w_gs);
-    else hipLaunchKernelGGL((gemm_nt_skinny<float>), g, dim3(256), 0, st0, (const float*)A, (const bf16_t*)W, C, bias, M, N, K, lda, ldw, ldc, offs, w_gs);
-    SEQ_LAUNCH_CHECK();
-    return 0;
-  }
-  if (tw == 1 && ta == 1 && vec_a && vec_w) {
-    const int rc = seq_gemm_tile((const bf16_t*)A, (const bf16_t*)W, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_gs, a_mod, w_gs, c_gs, st0);
+  const hipStream_t st = (hipStream_t)s;
+  if (vec_a && vec_w) {
+    // Few rows (in all; for row groups 8 each on average, their sizes are on the device): bound by reading W, no tile to fill.
+    // 48 rows of 8 experts (4096 x 2048 each): 32 us, the best tile 36; 40 rows x 2048 x 2048: 12 us, the best tile 7.
+    int rc = 0;
+    if (offs != nullptr ? M <= 8 * groups : groups == 1 && M <= 32)
+      rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, w_gs, st);
+    if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_gs, a_mod, w_gs, c_gs, st);
     if (rc != 0) return rc == 1 ? 0 : rc;
   }
-  // what is left has fp32 rows, ragged K or N, or fp32 weights.  Tile side by the rows of a group (on average, for row
+  // what is left has a ragged K or N or unaligned rows.  Tile side by the rows of a group (on average, for row
   // groups): 64, 128, or 256 when the problem still gives the chip a few hundred blocks
   const int gm = offs != nullptr ? M / groups : M;
   int big = 0;
@@ -405,7 +333,6 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
   if (gm > 192 && N > 128 && (long long)((M + 255) / 256) * ((N + 255) / 256) * groups >= 256) big = 256;
   const int ts = big ? big : BM;
   dim3 grid((N + ts - 1) / ts, (M + ts - 1) / ts, groups);
-  hipStream_t st = (hipStream_t)s;
   if (a_mod < 1) a_mod = 1;
   if (tw == 1 && ta == 1) launch<bf16_t, bf16_t>(big, grid, st, A, W, C, bias, M, N, K, lda, ldw, ldc, offs, a_gs, a_mod, w_gs, c_gs, vec_a, vec_w);
   else if (tw == 1) launch<float, bf16_t>(big, grid, st, A, W, C, bias, M, N, K, lda, ldw, ldc, offs, a_gs, a_mod, w_gs, c_gs, vec_a, vec_w);

@@ -35,7 +35,12 @@ __device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e,
   else reinterpret_cast<float*>(C)[idx] = v;
 }
 
-// gemm_tile.hip: the product of bf16 rows and bf16 weights on LDS-DMA tiles.  1: launched; 0: not a shape it serves;
-// < 0: failed.
-int seq_gemm_tile(const bf16_t* A, const bf16_t* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
+// gemm_tile.hip: the product on LDS-DMA tiles; element types bf16 x bf16, fp32 x fp32, or fp32 rows against bf16 weights (rounded
+// to them).  Needs 16-byte-aligned rows of A and W.  1: launched; 0: not a shape it serves; < 0: failed.
+int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
                   const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s);
+
+// gemm_rows.hip: the same for few rows.  Needs
+// 16-byte-aligned rows of A and W.  1: launched; 0: not a shape it serves; < 0: failed.
+int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
+                  int groups, const int* offs, long long w_gs, hipStream_t s);

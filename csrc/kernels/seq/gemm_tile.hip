@@ -1,6 +1,6 @@
-// C[M,N] = epilogue(A[M,K] . W[N,K]^T), bf16 operands, fp32 accumulation: the prompt projections of the stateful models.
+// C[M,N] = epilogue(A[M,K] . W[N,K]^T), fp32 accumulation: the prompt projections of the stateful models.
 //
-// Both operands go from global memory to LDS by DMA (no registers in between), 64 columns of K at a time, 1 KiB pieces of
+// Both operands go from global memory to LDS by DMA (no registers in between), 128 bytes of a row at a time, 1 KiB pieces of
 // 8 rows x 128 bytes whose 16-byte chunks are XOR-swizzled by the row (chunk c of row r in slot c ^ (r & 7)), so that the
 // 16-byte fragment reads of 16x16x32 MFMAs have no bank conflicts.  Rows past M and columns past N re-read the last valid row
 // (never out of bounds) and are not stored.
@@ -15,14 +15,14 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 #define LDS_AS __attribute__((address_space(3)))
 
 struct Tile {
-  const bf16_t* A;
-  const bf16_t* W;
+  const char* A;
+  const char* W;
   void* C;
   Epi epi;
-  int M, N, K, lda, ldw, ldc;
+  int M, N, nk, lda, ldw, ldc;  // nk: K tiles; lda, ldw: bytes; ldc: elements
   const int* offs;          // row groups (experts): group g owns rows offs[g] .. offs[g + 1] and weight g
   int groups;
-  long long w_gs, a_gs, c_gs;   // strided batch (grid y): operand and column offsets of group g
+  long long w_gs, a_gs, c_gs;   // group g's operands (bytes); strided batch (grid y): its columns of C (elements)
   int a_mod;
   int tiles_m, tiles_n, order;
 };
@@ -42,7 +42,7 @@ __device__ __forceinline__ int2 place(int b, int tiles_m, int tiles_n, int order
 
 // This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
 template <int TM, int TN>
-__device__ __forceinline__ bool locate(const Tile& a, const bf16_t*& A, const bf16_t*& W, size_t& cbase, int& m0, int& mend, int& n0) {
+__device__ __forceinline__ bool locate(const Tile& a, const char*& A, const char*& W, size_t& cbase, int& m0, int& mend, int& n0) {
   const int nwg = gridDim.x;
   int bid = blockIdx.x;
   {                                      // blocks go to the 8 XCDs in turn: give each a run of consecutive ids
@@ -185,7 +185,7 @@ __device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], si
 // accumulation register the compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between
 // them; reads run one phase of 32 MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
 namespace t256 {
-constexpr int TM = 256, TN = 256, KT = 64, STG = 65536, WIMG = 32768, LDS_BYTES = 2 * STG;
+constexpr int TM = 256, TN = 256, KT = 128 /* bytes of a K tile's row */, STG = 65536, WIMG = 32768, LDS_BYTES = 2 * STG;
 }
 
 __device__ __forceinline__ void mfma_in_place(floatx4& c, const bf16x8& a, const bf16x8& b) {
@@ -195,7 +195,7 @@ __device__ __forceinline__ void mfma_in_place(floatx4& c, const bf16x8& a, const
 __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
   using namespace t256;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const bf16_t *A, *W;
+  const char *A, *W;
   size_t cbase;
   int m0, mend, n0;
   if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
@@ -212,15 +212,15 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
     prow[i] = (j >> 3) * 128 + (j & 7) * 8;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      xo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, mlast) * a.lda + lc * 8) * 2u;
-      wo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, nlast) * a.ldw + lc * 8) * 2u;
+      xo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, mlast) * a.lda + lc * 16);
+      wo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, nlast) * a.ldw + lc * 16);
     }
   }
-  const char* Ab = reinterpret_cast<const char*>(A + (size_t)m0 * a.lda);
-  const char* Wb = reinterpret_cast<const char*>(W + (size_t)n0 * a.ldw);
+  const char* Ab = A + (size_t)m0 * a.lda;
+  const char* Wb = W + (size_t)n0 * a.ldw;
   // (past the last K tile the DMAs go through a descriptor of no records: counted like the others, they write zeros)
   const __amdgpu_buffer_rsrc_t rA = rsrc_of(Ab, true), rW = rsrc_of(Wb, true), r0 = rsrc_of(Ab, false);
-#define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, (k0) * 2, 0, 0)
+#define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, k0, 0, 0)
 #define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[(h) * 4 + (i)], k0, smem + (buf) * STG + (prow[i] + (h) * 64) * 128)
 #define T_W(rs, buf, h, i, k0) T_DMA(rs, wo[(h) * 4 + (i)], k0, smem + (buf) * STG + WIMG + (prow[i] + (h) * 64) * 128)
   const int wm = wave >> 1, wn = wave & 1;
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
   T_PHASE(0, 0, 1, 1, 1, 0, rw, 1, 1, dk, 1)                                                       \
   T_PHASE(1, 0, 1, 0, 0, 0, rw, 1, 0, dk, 0)                                                       \
   T_PHASE(1, 1, 0, 0, 0, 1, rx, 1, 1, dk, 1)
-  const int nk = a.K / KT;
+  const int nk = a.nk;
   {
     const __amdgpu_buffer_rsrc_t rA1 = nk > 1 ? rA : r0, rW1 = nk > 1 ? rW : r0;
     const int k1 = nk > 1 ? KT : 0;
@@ -336,23 +336,41 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
 // while tile t is multiplied, one barrier per K tile.  What bounds them is the chain of one K tile (wait, barrier, LDS read,
 // MFMA), 0.5 us or more for one wave a SIMD whatever the tile: KG groups of four waves take every KG-th K tile each, so that a
 // SIMD has KG chains to run (256 x 2048 x 2048 in 64 x 64 tiles: 16 us with one group, 12 with two).
-template <int MI, int NJ>
-__device__ __forceinline__ void fill(const char* Ab, const char* Wb, int kt, int nk, int wave, const unsigned* xo, const unsigned* wo,
-                                     char* stg) {
-  const bool live = kt < nk;             // (past the last K tile: a descriptor of no records; counted like the others, nothing reads what they leave)
-  const __amdgpu_buffer_rsrc_t ra = rsrc_of(Ab, live), rw = rsrc_of(Wb, live);
-  const int k0 = live ? kt * 64 : 0;
+//
+// A K tile is a 128-byte row of W: 64 bf16 (two 16x16x32 MFMAs per fragment pair) or 32 fp32 (eight 16x16x4 MFMAs: lane group g
+// holds elements 4 g .. 4 g + 3 of 16, and MFMA i multiplies the i-th ones).  fp32 rows against bf16 weights come in as they
+// are, 256 bytes a row, and are rounded when a fragment is read.
+template <typename T> struct Frag;
+template <> struct Frag<bf16_t> { typedef bf16x8 V; };
+template <> struct Frag<float> { typedef floatx4 V; };
+__device__ __forceinline__ floatx4 mfma_frag(const bf16x8& w, const bf16x8& x, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, c, 0, 0, 0);
+}
+__device__ __forceinline__ floatx4 mfma_frag(const floatx4& w, const floatx4& x, floatx4 c) {
 #pragma unroll
-  for (int i = 0; i < MI; ++i) T_DMA(ra, xo[i], k0, stg + (MI * wave + i) * 1024);
-#pragma unroll
-  for (int i = 0; i < NJ; ++i) T_DMA(rw, wo[i], k0, stg + 32 * MI * 128 + (NJ * wave + i) * 1024);
+  for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[i], c, 0, 0, 0);
+  return c;
 }
 
-template <int MI, int NJ, int S, int OCC, int KG>
+// the DMAs of K tile kt: PX pieces of A (128 XS bytes a row), PW of W
+template <int PX, int PW, int XS, int XIMG>
+__device__ __forceinline__ void fill(const char* Ab, const char* Wb, int kt, int nk, int wave, const unsigned* xo, const unsigned* wo, char* stg) {
+  const bool live = kt < nk;             // (past the last K tile: a descriptor of no records, counted like the others; it leaves zeros)
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(Ab, live), rw = rsrc_of(Wb, live);
+  const int k0 = live ? kt * 128 : 0;
+#pragma unroll
+  for (int i = 0; i < PX; ++i) T_DMA(ra, xo[i], k0 * XS, stg + (PX * wave + i) * 1024);
+#pragma unroll
+  for (int i = 0; i < PW; ++i) T_DMA(rw, wo[i], k0, stg + XIMG + (PW * wave + i) * 1024);
+}
+
+template <typename TA, typename TW, int MI, int NJ, int S, int OCC, int KG>
 __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
-  constexpr int TM = 32 * MI, TN = 32 * NJ, STG = (TM + TN) * 128, WIMG = TM * 128;
+  typedef typename Frag<TW>::V V;
+  constexpr int XS = sizeof(TA) / sizeof(TW);               // 2: fp32 rows against bf16 weights
+  constexpr int TM = 32 * MI, TN = 32 * NJ, XIMG = TM * 128 * XS, STG = XIMG + TN * 128, PX = MI * XS, PW = NJ;
   extern __shared__ __attribute__((aligned(16))) char smem_all[];
-  const bf16_t *A, *W;
+  const char *A, *W;
   size_t cbase;
   int m0, mend, n0;
   if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
@@ -362,50 +380,66 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
   char* smem = smem_all + kg * (S * STG);
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
   const int mlast = mend - 1 - m0, nlast = a.N - 1 - n0;
-  unsigned xo[MI], wo[NJ];
+  unsigned xo[PX], wo[PW];
 #pragma unroll
-  for (int i = 0; i < MI; ++i) xo[i] = (unsigned)(min((MI * wave + i) * 8 + lr, mlast) * a.lda + lc * 8) * 2u;
+  for (int i = 0; i < PX; ++i) {
+    if constexpr (XS == 1) {
+      xo[i] = (unsigned)(min((PX * wave + i) * 8 + lr, mlast) * a.lda + lc * 16);
+    } else {                                                 // pieces of 4 rows x 256 bytes, chunk c of row r in slot c ^ (r & 15)
+      const int r = (PX * wave + i) * 4 + (lane >> 4);
+      xo[i] = (unsigned)(min(r, mlast) * a.lda + ((lane ^ r) & 15) * 16);
+    }
+  }
 #pragma unroll
-  for (int i = 0; i < NJ; ++i) wo[i] = (unsigned)(min((NJ * wave + i) * 8 + lr, nlast) * a.ldw + lc * 8) * 2u;
-  const char* Ab = reinterpret_cast<const char*>(A + (size_t)m0 * a.lda);
-  const char* Wb = reinterpret_cast<const char*>(W + (size_t)n0 * a.ldw);
-  const int nk = a.K / 64;
+  for (int i = 0; i < PW; ++i) wo[i] = (unsigned)(min((PW * wave + i) * 8 + lr, nlast) * a.ldw + lc * 16);
+  const char* Ab = A + (size_t)m0 * a.lda;
+  const char* Wb = W + (size_t)n0 * a.ldw;
+  const int nk = a.nk;
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
   const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
-  const int xrow = (wm * 16 * MI + fr) * 128, wrow = WIMG + (wn * 16 * NJ + fr) * 128;
+  const int xrow = (wm * 16 * MI + fr) * 128 * XS, wrow = XIMG + (wn * 16 * NJ + fr) * 128;
   floatx4 acc[MI][NJ];
 #pragma unroll
   for (int u = 0; u < MI; ++u)
 #pragma unroll
     for (int t = 0; t < NJ; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int s = 0; s < S - 1; ++s) fill<MI, NJ>(Ab, Wb, s * KG + kg, nk, wave, xo, wo, smem + s * STG);
+  for (int s = 0; s < S - 1; ++s) fill<PX, PW, XS, XIMG>(Ab, Wb, s * KG + kg, nk, wave, xo, wo, smem + s * STG);
   int cur = 0, nxt = S - 1;
-  for (int kt = kg; kt < nk + kg; kt += KG) {
+  for (int kt = kg; kt < nk + kg; kt += KG) {               // (every group as often as the first: they share the barriers)
     // this wave's pieces of tile kt have landed and its reads of the tile before are done; after the barrier, everyone's
     asm volatile("" ::: "memory");
-    constexpr int LEFT = (S - 2) * (MI + NJ);               // DMAs of later K tiles that may stay in flight
+    constexpr int LEFT = (S - 2) * (PX + PW);               // DMAs of later K tiles that may stay in flight
     __builtin_amdgcn_s_waitcnt((LEFT & 15) | (LEFT >> 4) << 14 | 0x70);       // vmcnt(LEFT) lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    fill<MI, NJ>(Ab, Wb, kt + (S - 1) * KG, nk, wave, xo, wo, smem + nxt * STG);
+    fill<PX, PW, XS, XIMG>(Ab, Wb, kt + (S - 1) * KG, nk, wave, xo, wo, smem + nxt * STG);
     const char* stg = smem + cur * STG;
-    bf16x8 x[2][MI], w[2][NJ];
+    V x[2][MI], w[2][NJ];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       const int c = k ? c1 : c0;
 #pragma unroll
-      for (int u = 0; u < MI; ++u) x[k][u] = *(const bf16x8*)(stg + xrow + u * 2048 + c);
+      for (int u = 0; u < MI; ++u) {
+        if constexpr (XS == 1) {
+          x[k][u] = *(const V*)(stg + xrow + u * 2048 + c);
+        } else {
+          typedef float floatx8 __attribute__((ext_vector_type(8)));
+          const char* row = stg + xrow + u * 4096;
+          const floatx4 lo = *(const floatx4*)(row + (((8 * k + 2 * grp) ^ fr) << 4)), hi = *(const floatx4*)(row + (((8 * k + 2 * grp + 1) ^ fr) << 4));
+          x[k][u] = __builtin_convertvector((floatx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), V);
+        }
+      }
 #pragma unroll
-      for (int t = 0; t < NJ; ++t) w[k][t] = *(const bf16x8*)(stg + wrow + t * 2048 + c);
+      for (int t = 0; t < NJ; ++t) w[k][t] = *(const V*)(stg + wrow + t * 2048 + c);
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k)
 #pragma unroll
       for (int u = 0; u < MI; ++u)
 #pragma unroll
-        for (int t = 0; t < NJ; ++t) acc[u][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k][t], x[k][u], acc[u][t], 0, 0, 0);
+        for (int t = 0; t < NJ; ++t) acc[u][t] = mfma_frag(w[k][t], x[k][u], acc[u][t]);
     cur = cur + 1 == S ? 0 : cur + 1;
     nxt = nxt + 1 == S ? 0 : nxt + 1;
   }
@@ -413,6 +447,7 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   constexpr int OUT = 16 * MI * 16 * NJ * 4;                // a wave's accumulators
+  static_assert(4 * OUT * (KG > 1 ? KG - 1 : 1) <= KG * S * STG, "the accumulators fit the stages");
   if constexpr (KG > 1) {                                    // the wave groups' partial sums meet in LDS, in the groups' order
     if (kg > 0) {
 #pragma unroll
@@ -430,6 +465,7 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
 #pragma unroll
         for (int t = 0; t < NJ; ++t)
           acc[u][t] += *reinterpret_cast<const floatx4*>(smem_all + ((g - 1) * 4 + wave) * OUT + ((u * NJ + t) * 64 + lane) * 16);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the same wave lays its rows down in the same place)
   }
   finish<MI, NJ, MI>(a, acc, cbase, m0 + wm * 16 * MI, n0 + wn * 16 * NJ, mend, smem_all + wave * OUT);
 }
@@ -460,31 +496,35 @@ int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
 
 }  // namespace
 
-// The tiles, and what a launch of each costs: rounds of `slots` blocks (what the chip holds at once), each K / 64 K tiles and
-// a start and a store.  us per K tile and per round, measured on full rounds at K = 2048 .. 8192 (one MI355X):
-//   256 x 256   1.35  12    least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
-//   128 x 128   1.0    9    two blocks a CU
-//   128 x 128   0.55   6    eight waves, two wave groups each taking every other K tile
-//    64 x 128   0.40   5    the same
-//    64 x 64    0.26   3    the same
-//    32 x 64    0.16   3.5  sixteen waves, four wave groups
-//    32 x 32    0.12   3.5  the same
-// A launch that leaves CUs idle in its last (or only) round wants smaller tiles, a long one the large tile; the cheapest sum
-// wins (1024 x 2048 x 2048: 64 x 128 at 18 us, the 256 tile 45; 256 x 2048 x 2048: 32 x 64 at 9 us, the 256 tile 45;
-// 16384 x 14336 x 4096: the 256 tile at 1.49 ms, 128 x 128 at 2.28).
+// The tiles, and what a launch of each costs: rounds of `slots` blocks (what the chip holds at once), each nk K tiles and
+// a start and a store.  us per K tile and per round, measured on full rounds at K = 128 .. 8192 (one MI355X).  A launch that leaves
+// CUs idle in its last (or only) round wants smaller tiles, a long one the large tile; the cheapest sum wins.
 struct TileCost { int tm, tn, slots; float k_us, round_us; };
-static const TileCost TILES[] = {{256, 256, 256, 1.35f, 12.f}, {128, 128, 512, 1.0f, 9.f}, {128, 128, 256, 0.55f, 6.f}, {64, 128, 256, 0.40f, 5.f},
-                                 {64, 64, 256, 0.26f, 3.f}, {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f}};
+// bf16 (16384 x 14336 x 4096: the 256 tile 1.49 ms, 128 x 128 2.28; 1024 x 2048 x 2048: 64 x 128 18 us, the 256 tile 45;
+// 256 x 2048 x 2048: 32 x 64 9 us, the 256 tile 45)
+static const TileCost TILES[] = {{256, 256, 256, 1.35f, 12.f},      // least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
+                                 {128, 128, 512, 1.0f, 9.f},        // two blocks a CU
+                                 {128, 128, 256, 0.55f, 6.f}, {64, 128, 256, 0.40f, 5.f}, {64, 64, 256, 0.26f, 3.f},      // two wave groups
+                                 {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f}};                                 // four
+// fp32 rows, bf16 weights (16384 rows x 32 blocks of 256 x 256: 128 x 128 432 us, 458 at 64 x 128, 615 before; 400 x 2048 x 2048:
+// 64 x 64 16 us, 128 x 128 39)
+static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f}, {64, 128, 256, 0.47f, 5.f}, {64, 64, 256, 0.37f, 4.2f},
+                                       {64, 64, 512, 0.6f, 4.f},    // two blocks a CU
+                                       {32, 32, 256, 0.16f, 3.5f}};
+// fp32 (bound by the fp32 MFMA's 150 TFLOP/s; 400 x 2048 x 8192: 64 x 64 165 us, 128 x 128 573; 3000 x 2048 x 2048: 64 x 128 224 us,
+// 128 x 128 269)
+static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f}, {128, 128, 256, 2.15f, 6.f}, {64, 128, 256, 1.1f, 6.f},
+                                     {64, 64, 256, 0.63f, 4.f}, {32, 64, 256, 0.33f, 4.f}, {32, 32, 256, 0.195f, 4.f}};
 
-static int pick_tile(int M, int N, int K, int groups, bool by_rows) {
+static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int groups, bool by_rows) {
   int best = 0;
   float least = 0.f;
-  for (int v = 0; v < (int)(sizeof(TILES) / sizeof(TILES[0])); ++v) {
-    const TileCost& t = TILES[v];
+  for (int v = 0; v < count; ++v) {
+    const TileCost& t = tiles[v];
     // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average)
     const long long rows = by_rows ? (long long)M / t.tm + (groups + 1) / 2 : (long long)((M + t.tm - 1) / t.tm) * groups;
-    const long long tiles = rows * ((N + t.tn - 1) / t.tn);
-    const float us = (float)((tiles + t.slots - 1) / t.slots) * ((float)(K / 64) * t.k_us + t.round_us);
+    const long long blocks = rows * ((N + t.tn - 1) / t.tn);
+    const float us = (float)((blocks + t.slots - 1) / t.slots) * ((float)nk * t.k_us + t.round_us);
     if (v == 0 || us < least) {
       least = us;
       best = v;
@@ -493,20 +533,43 @@ static int pick_tile(int M, int N, int K, int groups, bool by_rows) {
   return best;
 }
 
-int seq_gemm_tile(const bf16_t* A, const bf16_t* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
+int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
                   const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
+  const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
   // whole K tiles; stores of four columns; 32-bit offsets within a tile
-  if (K % 64 || N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16)) return 0;
-  if ((long long)lda * 512 + K * 2LL >= (1LL << 31) || (long long)ldw * 512 + K * 2LL >= (1LL << 31)) return 0;
+  if (K * ew % 128 || N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16)) return 0;
+  if (((long long)lda * 256 + K) * ea >= (1LL << 31) || ((long long)ldw * 256 + K) * ew >= (1LL << 31)) return 0;
   if (offs == nullptr && groups > 65535) return 0;
-  const Tile t = {A, W, C, epi, M, N, K, lda, ldw, ldc, offs, groups, w_gs, a_gs, c_gs, a_mod < 1 ? 1 : a_mod, 0, 0, 0};
-  switch (pick_tile(M, N, K, groups, offs != nullptr)) {
-    case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
-    case 1: return start<gemm_tile_mid<4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
-    case 2: return start<gemm_tile_mid<4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
-    case 3: return start<gemm_tile_mid<2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
-    case 4: return start<gemm_tile_mid<2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
-    case 5: return start<gemm_tile_mid<1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
-    default: return start<gemm_tile_mid<1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
+  const int nk = K * ew / 128;
+  const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, offs, groups, w_gs * ew, a_gs * ea, c_gs,
+                  a_mod < 1 ? 1 : a_mod, 0, 0, 0};
+  const bool by_rows = offs != nullptr;
+  if (ta == 1) {
+    switch (pick_tile(TILES, 7, M, N, nk, groups, by_rows)) {
+      case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
+      case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
+      case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
+      case 3: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
+      case 4: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
+      case 5: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
+      default: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
+    }
+  }
+  if (tw == 1) {
+    switch (pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows)) {
+      case 0: return start<gemm_tile_mid<float, bf16_t, 4, 4, 3, 1, 1>>(128, 128, 256, 3 * 49152, t, s);
+      case 1: return start<gemm_tile_mid<float, bf16_t, 2, 4, 2, 1, 2>>(64, 128, 512, 4 * 32768, t, s);
+      case 2: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 1, 2>>(64, 64, 512, 6 * 24576, t, s);
+      case 3: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 2, 1>>(64, 64, 256, 3 * 24576, t, s);
+      default: return start<gemm_tile_mid<float, bf16_t, 1, 1, 3, 1, 4>>(32, 32, 1024, 12 * 12288, t, s);
+    }
+  }
+  switch (pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows)) {
+    case 0: return start<gemm_tile_mid<float, float, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
+    case 1: return start<gemm_tile_mid<float, float, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
+    case 2: return start<gemm_tile_mid<float, float, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
+    case 3: return start<gemm_tile_mid<float, float, 2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
+    case 4: return start<gemm_tile_mid<float, float, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
+    default: return start<gemm_tile_mid<float, float, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
   }
 }

@@ -98,6 +98,34 @@ def test_matmul_tiles(ops, M, N, K):
     close(H.grouped_matmul_nt(a, wg, offs), R.grouped_matmul_nt(a, wg, offs), 1e-5)
 
 
+# the same for fp32 operands and for fp32 rows against bf16 weights: shapes for each of their tiles, blocks of a strided batch
+@pytest.mark.parametrize("M,N,K", [(4000, 2052, 96), (1300, 2500, 160), (520, 2052, 224), (260, 2052, 288), (130, 1028, 352), (40, 132, 416)])
+def test_matmul_tiles_fp32_rows(ops, M, N, K):
+    H, R = ops
+    torch.manual_seed(M + N + K)
+    a = torch.randn(M, K + 4, device=DEV)[:, 4:]
+    w = 0.1 * torch.randn(N, K, device=DEV)
+    b = torch.randn(N, device=DEV)
+    want = (a.double() @ w.double().t() + b.double()).float()
+    close(H.matmul_nt(a, w, b), want, 1e-5)
+    kt = -(-K // 64) * 64
+    a, w = torch.randn(M, kt, device=DEV), (0.1 * torch.randn(N, kt, device=DEV)).bfloat16()
+    close(H.matmul_nt(a, w, b), R.matmul_nt(a.bfloat16(), w, b), 1e-5)
+    u, wg, bg = torch.randn(M, 192, device=DEV), torch.randn(6, 64, 64, device=DEV).bfloat16(), torch.randn(6 * 64, device=DEV)
+    close(H.block_linear(u, wg, bg, 3, torch.bfloat16), R.block_linear(u, wg, bg, 3, torch.bfloat16), 1e-5)
+
+
+# few rows per group, one group of more than the 16 that a pass over its weights takes, empty groups, a K tail
+@pytest.mark.parametrize("cdt,tol", DTYPES)
+@pytest.mark.parametrize("K", [64, 200])
+def test_grouped_few_rows(ops, cdt, tol, K):
+    H, R = ops
+    torch.manual_seed(K)
+    offs = torch.tensor([0, 0, 30, 31, 37, 37], dtype=torch.int32, device=DEV)
+    a, w = torch.randn(37, K, device=DEV).to(cdt), torch.randn(5, 100, K, device=DEV).to(cdt)
+    close(H.grouped_matmul_nt(a, w, offs), R.grouped_matmul_nt(a, w, offs), 1e-5)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_rows(ops, cdt, tol):
     H, R = ops
