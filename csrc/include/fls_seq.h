@@ -16,11 +16,15 @@ int fls_seq_version(void);
 // offs != null: row groups: group g owns rows [offs[g], offs[g+1]) of A and C and weight W + g * w_gs;
 // M is then the total row count (the bound of every group's rows).
 // Epilogue: + bias, then an activation (act_kind 0: none; 1: xIELU, act = {p, q} on the device; 2: max(z, 0)^2;
-// 3: exp(-exp(act[n / act_n]) softplus(z)), a decay per column n; groups == 1), stored as type tc (fp32, or bf16 when the
-// consumer is the next product).
+// 3: exp(-exp(act[n / act_n]) softplus(z)), a decay per column n; groups == 1; 4: p tanh(z / p); 5: p z; 6, 7, 8: a gated product, W
+// = [gate rows; up rows] (N / 2 each), C has N / 2 columns: silu(g) u, gelu(g) u, or the clamped gate of fls_seq_gate_mul
+// with limit p and alpha q; no bias), stored as type tc (fp32, or bf16 when the consumer is the next product).
+// a_rows (with offs; nullable): row r of the product is made from row a_rows[r] of A, which has at most M rows.
+// FLS_SEQ_NOT_SERVED: nothing was done -- a gated product or a_rows, and rows whose alignment or size only the general kernels take.
+#define FLS_SEQ_NOT_SERVED (-100)
 int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias, const float* act,
-                 int act_kind, int act_n, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs, long long a_gs,
-                 int a_mod, long long w_gs, long long c_gs, fls_stream_t s);
+                 int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
+                 const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s);
 // y[r] = w * x[row] / sqrt(mean_g(x[row]^2) + eps) per group of D / groups columns, row = idx ? idx[r] : r.
 // add != 0: y (fp32) += instead (the residual update), ty ignored.  woff is added to the weight (1 for
 // weights stored around zero).  w_one != 0: w is one number for all columns.

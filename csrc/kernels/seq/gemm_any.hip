@@ -305,11 +305,13 @@ static void launch(int big, dim3 grid, hipStream_t st, const void* A, const void
 }
 
 extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias_p,
-                            const float* act, int act_kind, int act_n, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
-                            long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s) {
-  if (act_kind < 0 || act_kind > 3 || ((act_kind == 1 || act_kind == 3) && act == nullptr)) return -1;
-  if (act_kind == 3 && (act_n < 1 || groups != 1 || offs != nullptr)) return -1;
-  const Epi bias = {bias_p, act, act_kind, tc, act_n};
+                            const float* act, int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc,
+                            int groups, const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s) {
+  if (act_kind < 0 || act_kind > EPI_LAST || ((act_kind == EPI_XIELU || act_kind == EPI_DECAY) && act == nullptr)) return -1;
+  if (act_kind == EPI_DECAY && (act_n < 1 || groups != 1 || offs != nullptr)) return -1;
+  if (act_kind >= EPI_GATE && (N % 2 || bias_p != nullptr || (groups != 1 && offs == nullptr))) return -1;
+  if (a_rows != nullptr && offs == nullptr) return -1;
+  const Epi bias = {bias_p, act, act_kind, tc, act_n, act_p, act_q};
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || groups < 1 || (ta == 1 && tw == 0)) return -1;
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
@@ -321,10 +323,11 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
     // 48 rows of 8 experts (4096 x 2048 each): 32 us, the best tile 36; 40 rows x 2048 x 2048: 12 us, the best tile 7.
     int rc = 0;
     if (offs != nullptr ? M <= 8 * groups : groups == 1 && M <= 32)
-      rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, w_gs, st);
-    if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_gs, a_mod, w_gs, c_gs, st);
+      rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, st);
+    if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, a_gs, a_mod, w_gs, c_gs, st);
     if (rc != 0) return rc == 1 ? 0 : rc;
   }
+  if (act_kind >= EPI_GATE || a_rows != nullptr) return FLS_SEQ_NOT_SERVED;
   // what is left has a ragged K or N or unaligned rows.  Tile side by the rows of a group (on average, for row
   // groups): 64, 128, or 256 when the problem still gives the chip a few hundred blocks
   const int gm = offs != nullptr ? M / groups : M;

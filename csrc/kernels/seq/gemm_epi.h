@@ -2,32 +2,49 @@
 #pragma once
 #include "seq_common.h"
 
-// What a kernel does with a finished accumulator element: + bias, optionally an activation (kind 1, xIELU with
-// act = {p, q}: z > 0: softplus(p) z^2 + z/2, else (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2; kind 2: the square
-// of max(z, 0); kind 3, a decay: exp(-exp(act[column / act_n]) softplus(z))), then the store as fp32 or bf16 -- so a projection whose consumer is the next matrix product writes that
-// product's operand directly and the fp32 intermediate never reaches memory.
+// What a kernel does with a finished accumulator element: + bias, optionally an activation, then the store as fp32 or bf16 --
+// so a projection whose consumer is the next matrix product writes that product's operand directly and the fp32
+// intermediate never reaches memory.
+//   1  xIELU with act = {p, q}: z > 0: softplus(p) z^2 + z/2, else (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2
+//   2  the square of max(z, 0)
+//   3  a decay: exp(-exp(act[column / act_n]) softplus(z))
+//   4  p tanh(z / p)
+//   5  p z
+//   6, 7, 8  a gated product: W holds [gate rows; up rows], N / 2 of each, C has N / 2 columns: silu(g) u, gelu(g) u (tanh
+//      form), or g sigmoid(q g) (u + 1) with g = min(gate, p), u = clamp(up, -p, p)
+enum { EPI_XIELU = 1, EPI_RELU2 = 2, EPI_DECAY = 3, EPI_SOFTCAP = 4, EPI_SCALE = 5, EPI_GATE = 6, EPI_LAST = 8 };
 struct Epi {
   const float* bias;
   const float* act;      // the activation's numbers on the device, if it has any
-  int kind;              // 0 none, 1 xIELU, 2 squared ReLU, 3 decay
+  int kind;
   int tc;                // element type of C: 0 fp32, 1 bf16
   int act_n;             // kind 3: columns per number of act
+  float p, q;
 };
 struct EpiRegs { float ap, an; };
 __device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {
   EpiRegs r = {0.f, 0.f};
-  if (e.kind == 1) { r.ap = softplus_f(e.act[0]); r.an = 0.5f + softplus_f(e.act[1]); }
+  if (e.kind == EPI_XIELU) { r.ap = softplus_f(e.act[0]); r.an = 0.5f + softplus_f(e.act[1]); }
   return r;
 }
 // (kind 3: what a lane's column needs, before its elements are emitted)
 __device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
-  if (e.kind == 3) r.ap = -expf(e.act[col / e.act_n]);
+  if (e.kind == EPI_DECAY) r.ap = -expf(e.act[col / e.act_n]);
 }
 __device__ __forceinline__ float epi_value(float v, const Epi& e, const EpiRegs& r) {
-  if (e.kind == 2) { v = fmaxf(v, 0.f); v *= v; }
-  else if (e.kind == 3) v = expf(r.ap * softplus_f(v));
-  else if (e.kind == 1) v = v > 0.f ? r.ap * v * v + 0.5f * v : r.an * (expm1f(v) - v) + 0.5f * v;
+  if (e.kind == EPI_RELU2) { v = fmaxf(v, 0.f); v *= v; }
+  else if (e.kind == EPI_DECAY) v = expf(r.ap * softplus_f(v));
+  else if (e.kind == EPI_XIELU) v = v > 0.f ? r.ap * v * v + 0.5f * v : r.an * (expm1f(v) - v) + 0.5f * v;
+  else if (e.kind == EPI_SOFTCAP) v = e.p * tanhf(v / e.p);
+  else if (e.kind == EPI_SCALE) v *= e.p;
   return v;
+}
+__device__ __forceinline__ float epi_gate(float g, float u, const Epi& e) {
+  if (e.kind == EPI_GATE) return silu_f(g) * u;
+  if (e.kind == EPI_GATE + 1) return gelu_tanh_f(g) * u;
+  g = fminf(g, e.p);
+  u = fminf(fmaxf(u, -e.p), e.p);
+  return g / (1.f + expf(-e.q * g)) * (u + 1.f);
 }
 __device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e, const EpiRegs& r) {
   v = epi_value(v, e, r);
@@ -36,11 +53,11 @@ __device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e,
 }
 
 // gemm_tile.hip: the product on LDS-DMA tiles; element types bf16 x bf16, fp32 x fp32, or fp32 rows against bf16 weights (rounded
-// to them).  Needs 16-byte-aligned rows of A and W.  1: launched; 0: not a shape it serves; < 0: failed.
+// to them).  a_rows (nullable): row r of the product is made from row a_rows[r] of A.  Needs 16-byte-aligned rows of A and W.  1: launched; 0: not a shape it serves; < 0: failed.
 int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
-                  const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s);
+                  const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s);
 
 // gemm_rows.hip: the same for few rows.  Needs
 // 16-byte-aligned rows of A and W.  1: launched; 0: not a shape it serves; < 0: failed.
 int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
-                  int groups, const int* offs, long long w_gs, hipStream_t s);
+                  int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s);

@@ -38,17 +38,19 @@ __device__ __forceinline__ floatx4 mfma_step(const floatx4& w, const floatx4& x,
   return c;
 }
 
-template <typename TA, typename TW, int MG, int WV>
+template <typename TA, typename TW, int MG, int WV, bool GATED>
 __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, const TW* __restrict__ W, void* __restrict__ C, Epi epi,
-                                                     int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs, long long w_gs) {
+                                                     int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs,
+                                                     const int* __restrict__ a_rows, long long w_gs) {
   typedef typename Step<TW>::V V;
-  constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, U = 8;
-  __shared__ floatx4 red[WV][MG][64];
+  constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, U = GATED ? 4 : 8, HW = GATED ? 2 : 1;
+  __shared__ floatx4 red[WV][MG * HW][64];
   if (offs != nullptr) {                   // row groups (experts): this block's group owns rows offs[g] .. offs[g+1]
     const int g = blockIdx.y, r0 = offs[g];
     M = offs[g + 1] - r0;
     if (M <= 0) return;
-    A += (size_t)r0 * lda;
+    if (a_rows != nullptr) a_rows += r0;
+    else A += (size_t)r0 * lda;
     C = reinterpret_cast<char*>(C) + (size_t)r0 * ldc * (epi.tc == 1 ? 2 : 4);
     W += (size_t)g * w_gs;
   }
@@ -58,25 +60,33 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   const int n0 = blockIdx.x * 16;
   const int steps = (K + SK - 1) / SK, per = (steps + WV - 1) / WV;
   const int s0 = wave * per, s1 = min(steps, s0 + per);
-  const TW* wp = W + (size_t)min(n0 + fr, N - 1) * ldw + grp * LN;
+  // (a gated product: the columns' gate rows and, N rows on, their up rows)
+  const TW* wp[HW];
+#pragma unroll
+  for (int h = 0; h < HW; ++h) wp[h] = W + (size_t)(min(n0 + fr, N - 1) + h * N) * ldw + grp * LN;
   for (int m0 = 0; m0 < M; m0 += 16 * MG) {
-    floatx4 acc[MG];
+    floatx4 acc[HW][MG];
     bool ok[MG];
     const TA* xp[MG];
 #pragma unroll
     for (int u = 0; u < MG; ++u) {
-      acc[u] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int h = 0; h < HW; ++h) acc[h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+      const int r = min(m0 + u * 16 + fr, M - 1);
       ok[u] = m0 + u * 16 + fr < M;
-      xp[u] = A + (size_t)min(m0 + u * 16 + fr, M - 1) * lda + grp * LN;
+      xp[u] = A + (size_t)(a_rows != nullptr ? a_rows[r] : r) * lda + grp * LN;
     }
     for (int s = s0; s < s1; s += U) {
-      V w[U], x[MG][U];
+      V w[HW][U], x[MG][U];
       bool in[U];                          // (the last step may end short: K is a multiple of a lane's share)
 #pragma unroll
       for (int i = 0; i < U; ++i) {
-        w[i] = V{};
         in[i] = s + i < s1 && (s + i) * SK + grp * LN < K;
-        if (in[i]) load_step(wp + (size_t)(s + i) * SK, w[i]);
+#pragma unroll
+        for (int h = 0; h < HW; ++h) {
+          w[h][i] = V{};
+          if (in[i]) load_step(wp[h] + (size_t)(s + i) * SK, w[h][i]);
+        }
       }
 #pragma unroll
       for (int u = 0; u < MG; ++u)
@@ -88,24 +98,37 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
 #pragma unroll
       for (int i = 0; i < U; ++i)
 #pragma unroll
-        for (int u = 0; u < MG; ++u) acc[u] = mfma_step(w[i], x[u][i], acc[u]);
+        for (int u = 0; u < MG; ++u)
+#pragma unroll
+          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
     }
     if (m0 > 0) __syncthreads();
 #pragma unroll
-    for (int u = 0; u < MG; ++u) red[wave][u][lane] = acc[u];
+    for (int u = 0; u < MG; ++u)
+#pragma unroll
+      for (int h = 0; h < HW; ++h) red[wave][u * HW + h][lane] = acc[h][u];
     __syncthreads();
     for (int i = threadIdx.x; i < 64 * MG; i += 64 * WV) {
       const int u = i >> 6, l = i & 63;
       const int row = m0 + u * 16 + (l & 15), col0 = n0 + 4 * (l >> 4);
       if (row < M) {
-        floatx4 v = red[0][u][l];
+        floatx4 v = red[0][u * HW][l], v2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 1; w < WV; ++w) v += red[w][u][l];
+        for (int w = 1; w < WV; ++w) v += red[w][u * HW][l];
+        if constexpr (GATED) {
+#pragma unroll
+          for (int w = 0; w < WV; ++w) v2 += red[w][u * HW + 1][l];
+        }
         EpiRegs er = epi_regs(epi);
 #pragma unroll
         for (int x = 0; x < 4; ++x) {
           const int col = col0 + x;
-          if (col < N) {
+          if (col >= N) continue;
+          if constexpr (GATED) {
+            const float o = epi_gate(v[x], v2[x], epi);
+            if (epi.tc == 1) reinterpret_cast<bf16_t*>(C)[(size_t)row * ldc + col] = f_to_bf16(o);
+            else reinterpret_cast<float*>(C)[(size_t)row * ldc + col] = o;
+          } else {
             epi_column(epi, er, col);
             emit(C, (size_t)row * ldc + col, v[x] + (epi.bias != nullptr ? epi.bias[col] : 0.f), epi, er);
           }
@@ -115,11 +138,11 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   }
 }
 
-template <typename TA, typename TW, int MG, int WV>
+template <typename TA, typename TW, int MG, int WV, bool GATED>
 int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
-          long long w_gs, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_rows<TA, TW, MG, WV>), dim3((N + 15) / 16, offs != nullptr ? groups : 1), dim3(64 * WV), 0, s, (const TA*)A,
-                     (const TW*)W, C, epi, M, N, K, lda, ldw, ldc, offs, w_gs);
+          const int* a_rows, long long w_gs, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_rows<TA, TW, MG, WV, GATED>), dim3((N + 15) / 16, offs != nullptr ? groups : 1), dim3(64 * WV), 0, s, (const TA*)A,
+                     (const TW*)W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 1 : -(int)e;
 }
@@ -127,18 +150,22 @@ int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, i
 }  // namespace
 
 int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
-                  int groups, const int* offs, long long w_gs, hipStream_t s) {
+                  int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s) {
   // Row groups of 16 rows a pass over W, or 32 (17 .. 32 rows in one pass: 24 x 2048 x 2048 8.1 us, 10.3 in two).  Eight waves share
   // K where one block a CU or less has all the columns (2048 columns: 6.4 us, 6.8 with four), four where several blocks share a CU
   // anyway (32000 columns: 32 us, 41 with eight; floor 28).
+  const bool gated = epi.kind >= EPI_GATE;
+  if (gated) N >>= 1;                      // columns of C
   const bool two = offs == nullptr && M > 16;
   const bool many = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1) > 256;
-#define ROWS(TA, TW)                                                                                                      \
-  (two ? (many ? start<TA, TW, 2, 4>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, w_gs, s)                         \
-               : start<TA, TW, 2, 8>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, w_gs, s))                        \
-       : (many ? start<TA, TW, 1, 4>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, w_gs, s)                         \
-               : start<TA, TW, 1, 8>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, w_gs, s)))
+#define ROWS_AS(TA, TW, GATED)                                                                                            \
+  (two ? (many ? start<TA, TW, 2, 4, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)          \
+               : start<TA, TW, 2, 8, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s))         \
+       : (many ? start<TA, TW, 1, 4, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)          \
+               : start<TA, TW, 1, 8, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)))
+#define ROWS(TA, TW) (gated ? ROWS_AS(TA, TW, true) : ROWS_AS(TA, TW, false))
   if (tw == 0) return ROWS(float, float);
   return ta == 1 ? ROWS(bf16_t, bf16_t) : ROWS(float, bf16_t);
 #undef ROWS
+#undef ROWS_AS
 }

@@ -20,6 +20,7 @@ struct Tile {
   void* C;
   Epi epi;
   int M, N, nk, lda, ldw, ldc;  // nk: K tiles; lda, ldw: bytes; ldc: elements
+  const int* a_rows;        // row r of the product is made from row a_rows[r] of A (null: r)
   const int* offs;          // row groups (experts): group g owns rows offs[g] .. offs[g + 1] and weight g
   int groups;
   long long w_gs, a_gs, c_gs;   // group g's operands (bytes); strided batch (grid y): its columns of C (elements)
@@ -94,6 +95,23 @@ __device__ __forceinline__ bool locate(const Tile& a, const char*& A, const char
   return true;
 }
 
+// Byte offsets of a tile's row r of A (from row m0, or from the first row with a_rows) and of its row j of W.  Rows past
+// the end re-read the last one.  A gated product takes 16 gate rows, their 16 up rows, the next 16 gate rows, ..., so that a wave
+// has both halves of a column; its W is addressed from column n0 / 2 of the gate rows.
+__device__ __forceinline__ unsigned a_offset(const Tile& a, int m0, int mend, int r) {
+  r = min(r, mend - 1 - m0);
+  return (unsigned)((a.a_rows != nullptr ? a.a_rows[m0 + r] : r) * a.lda);
+}
+__device__ __forceinline__ unsigned w_offset(const Tile& a, int n0, int j) {
+  if (a.epi.kind < EPI_GATE) return (unsigned)(min(j, a.N - 1 - n0) * a.ldw);
+  const int half = a.N >> 1;
+  return (unsigned)((min((j >> 5) * 16 + (j & 15), half - 1 - (n0 >> 1)) + ((j >> 4) & 1) * half) * a.ldw);
+}
+__device__ __forceinline__ const char* a_base(const Tile& a, const char* A, int m0) { return a.a_rows != nullptr ? A : A + (size_t)m0 * a.lda; }
+__device__ __forceinline__ const char* w_base(const Tile& a, const char* W, int n0) {
+  return W + (size_t)(a.epi.kind < EPI_GATE ? n0 : n0 >> 1) * a.ldw;
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, bool live) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, live ? -1 : 0, 0x00020000);
 }
@@ -118,6 +136,21 @@ __device__ __forceinline__ void hold(floatx4& c) {
 // A wave's outputs: acc[u][t] = rows mw + 16 u + (lane & 15), columns nw + 16 t + 4 (lane >> 4) .. + 3.  Without an activation
 // they leave straight from the registers.  An activation runs in a short loop over rows that the wave first lays down in
 // its own piece of LDS (PU row groups at a time): unrolled over all accumulators its code would be larger than the cache.
+template <int MI, int NJ, int PU, bool ACC>
+__device__ __forceinline__ void lay_down(floatx4 (&acc)[MI][NJ], int p, char* lds) {
+  constexpr int CH = 4 * NJ;
+  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+#pragma unroll
+  for (int u = 0; u < PU; ++u)
+#pragma unroll
+    for (int t = 0; t < NJ; ++t) {
+      const int r = u * 16 + fr;
+      hold<ACC>(acc[p * PU + u][t]);
+      *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = acc[p * PU + u][t];
+    }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (the wave's own rows: no other wave reads them)
+}
+
 template <int MI, int NJ, int PU, bool ACC, int TC>
 __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
   const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
@@ -141,6 +174,27 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
     return;
   }
   constexpr int CH = 4 * NJ, RI = 64 / CH;          // 16-byte chunks of a row; rows per step of the loop
+  if (NJ >= 2 && e.kind >= EPI_GATE) {               // (no bias: the gated products have none)
+    const int c = lane % (CH / 2), cg = (c >> 2) * 8 + (c & 3);          // column chunk, its gate chunk (the up chunk: + 4)
+    const int n = (nw >> 1) + 4 * c;
+#pragma unroll
+    for (int p = 0; p < MI / PU; ++p) {
+      lay_down<MI, NJ, PU, ACC>(acc, p, lds);
+#pragma unroll 1
+      for (int i = 0; i < 16 * PU; i += 2 * RI) {
+        const int r = i + lane / (CH / 2);
+        const floatx4 g = *reinterpret_cast<const floatx4*>(lds + (r * CH + (cg ^ (r & (CH - 1)))) * 16);
+        const floatx4 u = *reinterpret_cast<const floatx4*>(lds + (r * CH + ((cg + 4) ^ (r & (CH - 1)))) * 16);
+        floatx4 v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = epi_gate(g[x], u[x], e);
+        const int m = mw + p * PU * 16 + r;
+        if (m < mend && n < (a.N >> 1)) store4<TC>(a.C, (size_t)m * a.ldc + n, v);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    return;
+  }
   const EpiRegs er0 = epi_regs(e);
   const int c = lane % CH, n = nw + 4 * c;
   EpiRegs er[4] = {er0, er0, er0, er0};
@@ -152,15 +206,7 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
   }
 #pragma unroll
   for (int p = 0; p < MI / PU; ++p) {
-#pragma unroll
-    for (int u = 0; u < PU; ++u)
-#pragma unroll
-      for (int t = 0; t < NJ; ++t) {
-        const int r = u * 16 + fr;
-        hold<ACC>(acc[p * PU + u][t]);
-        *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = acc[p * PU + u][t];
-      }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the wave's own rows: no other wave reads them)
+    lay_down<MI, NJ, PU, ACC>(acc, p, lds);
 #pragma unroll 1
     for (int i = 0; i < 16 * PU; i += RI) {
       const int r = i + lane / CH;
@@ -205,19 +251,18 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
   int prow[4];
   unsigned xo[8], wo[8];
-  const int mlast = mend - 1 - m0, nlast = a.N - 1 - n0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = 4 * wave + i;
     prow[i] = (j >> 3) * 128 + (j & 7) * 8;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      xo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, mlast) * a.lda + lc * 16);
-      wo[4 * h + i] = (unsigned)(min(prow[i] + 64 * h + lr, nlast) * a.ldw + lc * 16);
+      xo[4 * h + i] = a_offset(a, m0, mend, prow[i] + 64 * h + lr) + lc * 16;
+      wo[4 * h + i] = w_offset(a, n0, prow[i] + 64 * h + lr) + lc * 16;
     }
   }
-  const char* Ab = A + (size_t)m0 * a.lda;
-  const char* Wb = W + (size_t)n0 * a.ldw;
+  const char* Ab = a_base(a, A, m0);
+  const char* Wb = w_base(a, W, n0);
   // (past the last K tile the DMAs go through a descriptor of no records: counted like the others, they write zeros)
   const __amdgpu_buffer_rsrc_t rA = rsrc_of(Ab, true), rW = rsrc_of(Wb, true), r0 = rsrc_of(Ab, false);
 #define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, k0, 0, 0)
@@ -379,21 +424,20 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
   const int wave = wall & 3, kg = wall >> 2;
   char* smem = smem_all + kg * (S * STG);
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
-  const int mlast = mend - 1 - m0, nlast = a.N - 1 - n0;
   unsigned xo[PX], wo[PW];
 #pragma unroll
   for (int i = 0; i < PX; ++i) {
     if constexpr (XS == 1) {
-      xo[i] = (unsigned)(min((PX * wave + i) * 8 + lr, mlast) * a.lda + lc * 16);
+      xo[i] = a_offset(a, m0, mend, (PX * wave + i) * 8 + lr) + lc * 16;
     } else {                                                 // pieces of 4 rows x 256 bytes, chunk c of row r in slot c ^ (r & 15)
       const int r = (PX * wave + i) * 4 + (lane >> 4);
-      xo[i] = (unsigned)(min(r, mlast) * a.lda + ((lane ^ r) & 15) * 16);
+      xo[i] = a_offset(a, m0, mend, r) + ((lane ^ r) & 15) * 16;
     }
   }
 #pragma unroll
-  for (int i = 0; i < PW; ++i) wo[i] = (unsigned)(min((PW * wave + i) * 8 + lr, nlast) * a.ldw + lc * 16);
-  const char* Ab = A + (size_t)m0 * a.lda;
-  const char* Wb = W + (size_t)n0 * a.ldw;
+  for (int i = 0; i < PW; ++i) wo[i] = w_offset(a, n0, (PW * wave + i) * 8 + lr) + lc * 16;
+  const char* Ab = a_base(a, A, m0);
+  const char* Wb = w_base(a, W, n0);
   const int nk = a.nk;
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
@@ -516,11 +560,12 @@ static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f}, {64, 128, 25
 static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f}, {128, 128, 256, 2.15f, 6.f}, {64, 128, 256, 1.1f, 6.f},
                                      {64, 64, 256, 0.63f, 4.f}, {32, 64, 256, 0.33f, 4.f}, {32, 32, 256, 0.195f, 4.f}};
 
-static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int groups, bool by_rows) {
+static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int groups, bool by_rows, bool gated) {
   int best = 0;
   float least = 0.f;
   for (int v = 0; v < count; ++v) {
     const TileCost& t = tiles[v];
+    if (gated && t.tn < 64) continue;      // (a wave of the 32-column tile has one half of a gated column only)
     // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average)
     const long long rows = by_rows ? (long long)M / t.tm + (groups + 1) / 2 : (long long)((M + t.tm - 1) / t.tm) * groups;
     const long long blocks = rows * ((N + t.tn - 1) / t.tn);
@@ -534,18 +579,21 @@ static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int
 }
 
 int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
-                  const int* offs, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
+                  const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
   // whole K tiles; stores of four columns; 32-bit offsets within a tile
   if (K * ew % 128 || N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16)) return 0;
   if (((long long)lda * 256 + K) * ea >= (1LL << 31) || ((long long)ldw * 256 + K) * ew >= (1LL << 31)) return 0;
   if (offs == nullptr && groups > 65535) return 0;
+  const bool gated = epi.kind >= EPI_GATE;
+  if (gated && (N % 8 || (long long)N * ldw * ew >= (1LL << 31) || (offs == nullptr && groups > 1))) return 0;
+  if (a_rows != nullptr && (long long)M * lda * ea >= (1LL << 31)) return 0;      // (there are at most as many rows of A as of the product)
   const int nk = K * ew / 128;
-  const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, offs, groups, w_gs * ew, a_gs * ea, c_gs,
+  const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, a_rows, offs, groups, w_gs * ew, a_gs * ea, c_gs,
                   a_mod < 1 ? 1 : a_mod, 0, 0, 0};
   const bool by_rows = offs != nullptr;
   if (ta == 1) {
-    switch (pick_tile(TILES, 7, M, N, nk, groups, by_rows)) {
+    switch (pick_tile(TILES, 7, M, N, nk, groups, by_rows, gated)) {
       case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
       case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
       case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
@@ -556,7 +604,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
     }
   }
   if (tw == 1) {
-    switch (pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows)) {
+    switch (pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows, gated)) {
       case 0: return start<gemm_tile_mid<float, bf16_t, 4, 4, 3, 1, 1>>(128, 128, 256, 3 * 49152, t, s);
       case 1: return start<gemm_tile_mid<float, bf16_t, 2, 4, 2, 1, 2>>(64, 128, 512, 4 * 32768, t, s);
       case 2: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 1, 2>>(64, 64, 512, 6 * 24576, t, s);
@@ -564,7 +612,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
       default: return start<gemm_tile_mid<float, bf16_t, 1, 1, 3, 1, 4>>(32, 32, 1024, 12 * 12288, t, s);
     }
   }
-  switch (pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows)) {
+  switch (pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows, gated)) {
     case 0: return start<gemm_tile_mid<float, float, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
     case 1: return start<gemm_tile_mid<float, float, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
     case 2: return start<gemm_tile_mid<float, float, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);

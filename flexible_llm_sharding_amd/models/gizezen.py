@@ -169,9 +169,8 @@ def _moe(ctx, mlp: dict, W, h, x):
     E, top, fs = mlp["router"]["experts"], mlp["router"]["top"], _shared_ff(mlp)
     zr = ops.matmul_nt(h, W["wsr"])                                       # fp32 [T, shared gate | up | router | sg]
     route = ops.moe_route_topk(zr[:, 2 * fs:2 * fs + E], top)
-    hp = ops.gather_rows(h, route.rows)                                   # rows sorted by expert
-    gu = ops.grouped_matmul_nt(hp, W["wgu"], route.offs)                  # fp32 [T top, gate | up]
-    yo = ops.grouped_matmul_nt(ops.silu_mul(gu, out_dtype=cdt), W["wdown"], route.offs)
+    act = ops.gated_matmul_nt(h, W["wgu"], cdt, offs=route.offs, rows=route.rows)   # rows sorted by expert, silu(gate) up
+    yo = ops.grouped_matmul_nt(act, W["wdown"], route.offs)
     ys = gate = None
     if fs:
         ys = ops.matmul_nt(ops.silu_mul(zr[:, :2 * fs], out_dtype=cdt), W["wsdown"])

@@ -206,9 +206,7 @@ def _moe(ctx, mlp: dict, W, h):
     E, top = mlp["router"]["experts"], mlp["router"]["top"]
     logits = ops.matmul_nt(h, W["wrouter"])                               # fp32 accumulation of the rows
     route = ops.moe_route_corrected(logits, W["corr"], top)
-    hp = ops.gather_rows(h, route.rows)                                   # rows sorted by expert
-    gu = ops.grouped_matmul_nt(hp, W["wgu"], route.offs)                  # fp32 [T top, gate | up]
-    a = ops.silu_mul(gu, out_dtype=cdt)
+    a = ops.gated_matmul_nt(h, W["wgu"], cdt, offs=route.offs, rows=route.rows)     # rows sorted by expert, silu(gate) up
     yo = ops.grouped_matmul_nt(a, W["wdown"], route.offs)
     return ops.moe_weighted_sum(yo, route)                                # fp32 [T, D]
 
@@ -244,8 +242,7 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
     if kind == "norm":
         return ops.group_rmsnorm(state, W["norm"], cfg.norm_groups, cfg.norm_eps, out_dtype=ctx.compute_dtype,
                                  row_idx=meta["want_idx"])
-    z = ops.matmul_nt(state, W["head"])
-    return ops.softcap_(z, cfg.logit_softcap)
+    return ops.matmul_nt(state, W["head"], softcap=cfg.logit_softcap)
 
 
 def layer_flops(cfg, name: str, rows: int, ctx_keys: float = 0.0) -> float:

@@ -222,7 +222,7 @@ def _channel_delta(ctx, L, W, h, meta, name: str):
 
 def _dense(ctx, mlp: dict, W, h):
     ops, cdt = ctx.ops, ctx.compute_dtype
-    return ops.matmul_nt(ops.gate_mul(ops.matmul_nt(h, W["wgu"]), cdt, act="silu"), W["wdown"])
+    return ops.matmul_nt(ops.gated_matmul_nt(h, W["wgu"], cdt), W["wdown"])
 
 
 def _moe(ctx, mlp: dict, W, h):
@@ -234,9 +234,8 @@ def _moe(ctx, mlp: dict, W, h):
     route = ops.moe_route_softmax_grouped(logits, W["corr"], int(r["top"]), int(g.get("count", 0)), int(g.get("keep", 0)),
                                           float(r.get("scale", 1.0)))
     offs = route.offs[:E + 1]                                              # (rows of identity experts sort behind the experts')
-    hp = ops.gather_rows(h, route.rows)
-    gu = ops.grouped_matmul_nt(hp, W["wgu"], offs)                         # fp32 [T top, gate | up]
-    act = ops.gate_mul(gu, cdt, act="clamped", limit=float(mlp["expert"]["limit"]), alpha=EXPERT_ALPHA)
+    act = ops.gated_matmul_nt(h, W["wgu"], cdt, act="clamped", limit=float(mlp["expert"]["limit"]), alpha=EXPERT_ALPHA, offs=offs,
+                              rows=route.rows)
     return ops.grouped_matmul_nt(act, W["wdown"], offs), route, h, E
 
 
@@ -273,8 +272,7 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
         return run_block(ctx, W, state, meta, name)
     if kind == "norm":
         return ops.group_rmsnorm(state[:, :cfg.width], W["norm"], 1, cfg.norm_eps, out_dtype=ctx.compute_dtype, row_idx=meta["want_idx"])
-    z = ops.matmul_nt(state, W["head"])
-    return ops.scale_(z, cfg.logit_scale) if cfg.logit_scale != 1.0 else z
+    return ops.matmul_nt(state, W["head"], scale=cfg.logit_scale if cfg.logit_scale != 1.0 else None)
 
 
 def layer_flops(cfg, name: str, rows: int, ctx_keys: float = 0.0) -> float:

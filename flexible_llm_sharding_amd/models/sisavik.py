@@ -236,8 +236,7 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
     ops.add_group_rmsnorm_(x, y, W["norm1"], 1, eps, w_offset=1.0)
     if L.mlp is not None:
         h = ops.causal_conv(x, W["canon2"], None, st["canon2"], meta, residual=True, out_dtype=cdt)
-        gu = ops.matmul_nt(h, W["wgu"])                                   # fp32 [T, gate | up]
-        y = ops.matmul_nt(ops.gate_mul(gu, cdt, act="gelu_tanh"), W["wdown"])
+        y = ops.matmul_nt(ops.gated_matmul_nt(h, W["wgu"], cdt, act="gelu_tanh"), W["wdown"])
         ops.add_group_rmsnorm_(x, y, W["norm2"], 1, eps, w_offset=1.0)
     return x
 

@@ -471,17 +471,24 @@ class HipSeqOps:
             self.block_means(kc, vc, blocks, meta, G * d, Gv * dv)
         return q_out
 
-    def _gemm(self, a, w, c, bias, M, N, K, lda, ldw, ldc, groups=1, offs=None, a_gs=0, a_mod=1, w_gs=0, c_gs=0,
-              act=None, kind=0, act_n=0):
-        _chk(self.k.fls_seq_gemm(a.data_ptr(), _code(a, "a"), w.data_ptr(), _code(w, "w"), c.data_ptr(), _code(c, "c"),
-                                 bias.data_ptr() if bias is not None else None,
-                                 act.data_ptr() if act is not None else None, kind, act_n, M, N, K, lda, ldw, ldc, groups,
-                                 offs.data_ptr() if offs is not None else None, a_gs, a_mod, w_gs, c_gs, _stream()),
-             "fls_seq_gemm")
+    NOT_SERVED = -100          # fls_seq.h FLS_SEQ_NOT_SERVED
 
-    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None):
-        """a . w^T (+ bias); ``xielu`` ({p, q}), ``relu2`` (max(z, 0)^2) or ``decay`` (rates of equal runs of columns:
-        exp(-exp(rate) softplus(z))): that activation in the epilogue;
+    def _gemm(self, a, w, c, bias, M, N, K, lda, ldw, ldc, groups=1, offs=None, a_gs=0, a_mod=1, w_gs=0, c_gs=0,
+              act=None, kind=0, act_n=0, p=0.0, q=0.0, a_rows=None):
+        """-> False when only the general kernels take these rows and the call needs more than they do (nothing was done)."""
+        rc = self.k.fls_seq_gemm(a.data_ptr(), _code(a, "a"), w.data_ptr(), _code(w, "w"), c.data_ptr(), _code(c, "c"),
+                                 bias.data_ptr() if bias is not None else None,
+                                 act.data_ptr() if act is not None else None, kind, act_n, float(p), float(q), M, N, K, lda, ldw, ldc, groups,
+                                 offs.data_ptr() if offs is not None else None, a_rows.data_ptr() if a_rows is not None else None,
+                                 a_gs, a_mod, w_gs, c_gs, _stream())
+        if rc == self.NOT_SERVED:
+            return False
+        _chk(rc, "fls_seq_gemm")
+        return True
+
+    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None):
+        """a . w^T (+ bias); ``xielu`` ({p, q}), ``relu2`` (max(z, 0)^2), ``decay`` (rates of equal runs of columns:
+        exp(-exp(rate) softplus(z))), ``softcap`` (cap tanh(z / cap)) or ``scale``: that activation in the epilogue;
         ``out_dtype``: the accumulator as it is (fp32) or rounded for the next product (bf16)."""
         _rows(a, "a")
         _rows(w, "w")
@@ -497,15 +504,45 @@ class HipSeqOps:
             _vec(xielu, "xielu", 2)
         if decay is not None and (N % decay.numel() or not decay.numel()):
             raise ValueError("matmul_nt: decay rates do not divide the columns")
-        if (xielu is not None) + bool(relu2) + (decay is not None) > 1:
+        kinds = [k for k, on in ((1, xielu is not None), (2, bool(relu2)), (3, decay is not None), (4, softcap is not None),
+                                 (5, scale is not None)) if on]
+        if len(kinds) > 1:
             raise ValueError("matmul_nt: one activation at a time")
         if decay is not None:
             _vec(decay, "decay", decay.numel())
         c = torch.empty(M, N, dtype=out_dtype, device=a.device)
         self._gemm(a, w, c, bias, M, N, K, a.stride(0), w.stride(0), N, act=xielu if decay is None else decay,
-                   kind=1 if xielu is not None else (2 if relu2 else (3 if decay is not None else 0)),
-                   act_n=N // decay.numel() if decay is not None else 0)
+                   kind=kinds[0] if kinds else 0, act_n=N // decay.numel() if decay is not None else 0,
+                   p=softcap if softcap is not None else (scale if scale is not None else 0.0))
         return c
+
+    def gated_matmul_nt(self, a, w, out_dtype, act="silu", limit=0.0, alpha=1.702, offs=None, rows=None):
+        """``gate_mul`` of a . w^T, w = [gate rows; up rows], in the product's epilogue.  ``offs``: w [E, 2 ff, K], expert e's weights
+        make rows offs[e] .. offs[e + 1] of the result, row r from row ``rows[r]`` of a (no ``rows``: row r)."""
+        _rows(a, "a")
+        if w.dim() != (2 if offs is None else 3) or w.shape[-1] != a.shape[1] or w.shape[-2] % 2 or (offs is not None and not w.is_contiguous()):
+            raise ValueError(f"gated_matmul_nt: {tuple(a.shape)} against {tuple(w.shape)}")
+        if (rows is not None and offs is None) or (a.dtype == torch.bfloat16 and w.dtype == torch.float32):
+            raise ValueError("gated_matmul_nt: rows go with offs, bf16 rows with bf16 weights")
+        N, K = w.shape[-2:]
+        M = a.shape[0] if rows is None else rows.numel()
+        E = 1
+        if offs is not None:
+            E = w.shape[0]
+            _vec(offs, "offs", E + 1, torch.int32)
+        else:
+            _rows(w, "w")
+        if rows is not None:
+            _vec(rows, "rows", M, torch.int32)
+            if a.shape[0] > M:
+                raise ValueError("gated_matmul_nt: more rows than places for them")
+        y = torch.empty(M, N // 2, dtype=out_dtype, device=a.device)
+        if self._gemm(a, w, y, None, M, N, K, a.stride(0), w.stride(-2), N // 2, groups=E, offs=offs, w_gs=N * K if offs is not None else 0,
+                      kind=6 + self._ACT[act], p=limit, q=alpha, a_rows=rows):
+            return y
+        if rows is not None:
+            a = self.gather_rows(a, rows)
+        return self.gate_mul(self.matmul_nt(a, w) if offs is None else self.grouped_matmul_nt(a, w, offs), out_dtype, act, limit, alpha)
 
     def block_linear(self, u, w, b, blocks, cdt):
         _rows(u, "u", torch.float32)

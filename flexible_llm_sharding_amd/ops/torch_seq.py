@@ -158,8 +158,9 @@ class TorchSeqOps:
         """o * sigmoid(g), element by element."""
         return (o.float() * torch.sigmoid(g.float())).to(out_dtype)
 
-    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None):
-        """``decay`` (rates [R] of equal runs of output columns): exp(-exp(rate) softplus(y)) of the biased product."""
+    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None):
+        """``decay`` (rates [R] of equal runs of output columns): exp(-exp(rate) softplus(y)) of the biased product; ``softcap``:
+        cap tanh(y / cap); ``scale``: scale y."""
         if a.dtype != w.dtype:
             a = a.to(w.dtype)
         y = (a @ w.t()).float() if w.dtype == torch.float32 else (a.float() @ w.float().t())
@@ -171,7 +172,18 @@ class TorchSeqOps:
             y = torch.relu(y).square()
         if decay is not None:
             y = torch.exp(-torch.exp(decay.float()).repeat_interleave(y.shape[1] // decay.numel()) * F.softplus(y))
+        if softcap is not None:
+            y = softcap * torch.tanh(y / softcap)
+        if scale is not None:
+            y = y * scale
         return y.to(out_dtype)
+
+    def gated_matmul_nt(self, a, w, out_dtype, act="silu", limit=0.0, alpha=1.702, offs=None, rows=None):
+        """``gate_mul`` of a . w^T, w = [gate rows; up rows]; with ``offs`` per expert (grouped_matmul_nt), row r of the result from
+        row ``rows[r]`` of a."""
+        if rows is not None:
+            a = self.gather_rows(a, rows)
+        return self.gate_mul(self.matmul_nt(a, w) if offs is None else self.grouped_matmul_nt(a, w, offs), out_dtype, act, limit, alpha)
 
     def block_linear(self, u, w, b, blocks, cdt):
         """[T, blocks * bw] -> [T, G * bw]: column block g of the output is block g % blocks of

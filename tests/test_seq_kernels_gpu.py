@@ -115,6 +115,30 @@ def test_matmul_tiles_fp32_rows(ops, M, N, K):
     close(H.block_linear(u, wg, bg, 3, torch.bfloat16), R.block_linear(u, wg, bg, 3, torch.bfloat16), 1e-5)
 
 
+# gated products ([gate; up] rows of W, the gate in the epilogue): few rows, every tile from 32 x 64 up, experts with gathered rows,
+# and rows no tile takes (K = 100: the product and the gate as two kernels)
+@pytest.mark.parametrize("cdt,tol", DTYPES)
+@pytest.mark.parametrize("M,I,K", [(5, 40, 64), (23, 100, 200), (70, 1028, 192), (300, 1028, 64), (1030, 2052, 64), (2100, 2052, 64), (20, 24, 100)])
+def test_gated_matmul(ops, cdt, tol, M, I, K):
+    H, R = ops
+    torch.manual_seed(M + I + K)
+    a, w = torch.randn(M, K, device=DEV).to(cdt), (0.2 * torch.randn(2 * I, K, device=DEV)).to(cdt)
+    for act, lim in (("silu", 0.0), ("gelu_tanh", 0.0), ("clamped", 0.7)):
+        close(H.gated_matmul_nt(a, w, cdt, act, lim), R.gated_matmul_nt(a, w, cdt, act, lim), tol)
+        close(H.gated_matmul_nt(a, w, torch.float32, act, lim), R.gated_matmul_nt(a, w, torch.float32, act, lim), 2e-5)
+    E, n = 5, 2 * M                                                 # two places per row of a, the last ones in no expert's range
+    rows = torch.randperm(n, device=DEV).to(torch.int32) // 2
+    offs = torch.tensor([0, 0, M, M + 1, n - 2, n - 2], dtype=torch.int32, device=DEV)
+    wg = (0.2 * torch.randn(E, 2 * I, K, device=DEV)).to(cdt)
+    close(H.gated_matmul_nt(a, wg, cdt, offs=offs, rows=rows)[:n - 2], R.gated_matmul_nt(a, wg, cdt, offs=offs, rows=rows)[:n - 2], tol)
+    z = H.matmul_nt(a, w, softcap=3.0)
+    close(z, R.matmul_nt(a, w, softcap=3.0), 2e-5)
+    close(H.matmul_nt(a, w, scale=0.3), R.matmul_nt(a, w, scale=0.3), 1e-5)
+    wide = torch.cat([z, z[:, :1]], 1)[:, :2 * I]                   # (a row stride that is no multiple of four)
+    for t in (z, wide):
+        assert torch.equal(H.argmax_f32(t), t.argmax(1).to(torch.int32))
+
+
 # few rows per group, one group of more than the 16 that a pass over its weights takes, empty groups, a K tail
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("K", [64, 200])
