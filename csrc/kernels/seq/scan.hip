@@ -38,17 +38,19 @@ __global__ void causal_conv_kernel(const float* __restrict__ x, int ldx, const f
 // walks CONV_ROWS consecutive rows, keeping the last taps inputs in registers (xv[j] = the input j rows
 // back); only the first row of its run, or of a new request inside it, gathers its lags from memory or
 // from the carried state.  fuse_state (every request of the step has one row, so the thread that walks a
-// request's row has seen all its inputs): the thread also rewrites its channel of the carried state.
+// request's row has seen all its inputs): the thread also rewrites its channel of the carried state.  Such a step has few
+// rows, each with a chain of loads of its own (request, position, slot, inputs): a thread walks one row instead of 16
+// (ROWS; 24 rows x 6144 channels: 23 us walked).
 #define CONV_MAX_TAPS 8
 #define CONV_ROWS 16
-template <typename TO>
+template <typename TO, int ROWS>
 __global__ void causal_conv_rows_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w, const float* __restrict__ b,
                                         float* __restrict__ state, TO* __restrict__ out, int ldo,
                                         const int* __restrict__ tok_seq, const int* __restrict__ cu, const int* __restrict__ pos0,
                                         const int* __restrict__ slot, int T, int C, int taps, int act, int residual, int fuse_state) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= C) return;
-  const int t0 = blockIdx.y * CONV_ROWS, t1 = min(T, t0 + CONV_ROWS);
+  const int t0 = blockIdx.y * ROWS, t1 = min(T, t0 + ROWS);
   float wv[CONV_MAX_TAPS], xv[CONV_MAX_TAPS];
 #pragma unroll
   for (int j = 0; j < CONV_MAX_TAPS; ++j) {
@@ -56,14 +58,14 @@ __global__ void causal_conv_rows_kernel(const float* __restrict__ x, int ldx, co
     xv[j] = 0.f;
   }
   const float bias = b != nullptr ? b[c] : 0.f;
-  if (t1 - t0 == CONV_ROWS && !fuse_state && tok_seq[t0] == tok_seq[t1 - 1]) {
+  if (ROWS > 1 && t1 - t0 == ROWS && !fuse_state && tok_seq[t0] == tok_seq[t1 - 1]) {
     // a full run inside one request: all its loads are issued at once, the sums follow from registers
     const int s = tok_seq[t0], tl = t0 - cu[s];
     const bool carried = pos0[s] > 0;
     const float* hist = state + (size_t)slot[s] * (taps - 1) * C;
-    float xr[CONV_ROWS];
+    float xr[ROWS];
 #pragma unroll
-    for (int r = 0; r < CONV_ROWS; ++r) xr[r] = x[(size_t)(t0 + r) * ldx + c];
+    for (int r = 0; r < ROWS; ++r) xr[r] = x[(size_t)(t0 + r) * ldx + c];
 #pragma unroll
     for (int j = 1; j < CONV_MAX_TAPS; ++j)
       if (j < taps) {
@@ -71,7 +73,7 @@ __global__ void causal_conv_rows_kernel(const float* __restrict__ x, int ldx, co
         else if (carried) xv[j] = hist[(size_t)(taps - 1 + tl - j) * C + c];
       }
 #pragma unroll
-    for (int r = 0; r < CONV_ROWS; ++r) {
+    for (int r = 0; r < ROWS; ++r) {
       float acc = bias;
 #pragma unroll
       for (int j = 0; j < CONV_MAX_TAPS; ++j) acc += wv[j] * (r >= j ? xr[r >= j ? r - j : 0] : xv[r >= j ? 0 : j - r]);
@@ -144,10 +146,13 @@ extern "C" int fls_seq_causal_conv(const float* x, int ldx, const float* w, cons
   if (taps < 1) return -1;
   hipStream_t st = (hipStream_t)s;
   if (taps <= CONV_MAX_TAPS) {
-    dim3 grid((C + 255) / 256, (T + CONV_ROWS - 1) / CONV_ROWS);
     const int fuse = one_row_each && T == B;
-    if (to == 1) hipLaunchKernelGGL((causal_conv_rows_kernel<bf16_t>), grid, dim3(256), 0, st, x, ldx, w, b, state, (bf16_t*)out, ldo, tok_seq, cu, pos0, slot, T, C, taps, act, residual, fuse);
-    else hipLaunchKernelGGL((causal_conv_rows_kernel<float>), grid, dim3(256), 0, st, x, ldx, w, b, state, (float*)out, ldo, tok_seq, cu, pos0, slot, T, C, taps, act, residual, fuse);
+    const dim3 grid((C + 255) / 256, fuse ? T : (T + CONV_ROWS - 1) / CONV_ROWS);
+#define CONV(TO, ROWS) hipLaunchKernelGGL((causal_conv_rows_kernel<TO, ROWS>), grid, dim3(256), 0, st, x, ldx, w, b, state, (TO*)out, ldo, tok_seq, \
+                                          cu, pos0, slot, T, C, taps, act, residual, fuse)
+    if (to == 1) { if (fuse) CONV(bf16_t, 1); else CONV(bf16_t, CONV_ROWS); }
+    else { if (fuse) CONV(float, 1); else CONV(float, CONV_ROWS); }
+#undef CONV
     SEQ_LAUNCH_CHECK();
     if (fuse) return 0;
   } else if (to == 1) hipLaunchKernelGGL((causal_conv_kernel<bf16_t>), dim3((C + 255) / 256, T), dim3(256), 0, st, x, ldx, w, b, state, (bf16_t*)out, ldo, tok_seq, cu, pos0, slot, C, taps, act, residual);
