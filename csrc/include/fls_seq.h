@@ -164,6 +164,11 @@ int fls_seq_ssd_scan(const float* xbc, int ldx, const float* z, int ldz, const f
                      const float* dt_bias, const float* A_log, const float* Dskip, float* state, float* out, int ldo,
                      const int* cu, const int* pos0, const int* slot, int B, int nh, int P, int N, int G,
                      fls_stream_t s);
+// the same 64 rows at a time, for steps with many rows per request (max_rows: the most of one): N 64 or 128, P a multiple of 16,
+// xbc 16-byte aligned with ldx a multiple of 4; scratch: T G 64 floats, 16-byte aligned
+int fls_seq_ssd_scan_chunked(const float* xbc, int ldx, const float* z, int ldz, const float* dt, int lddt, const float* dt_bias,
+                             const float* A_log, const float* Dskip, float* state, float* out, int ldo, const int* cu,
+                             const int* pos0, const int* slot, int B, int max_rows, int nh, int P, int N, int G, float* scratch, fls_stream_t s);
 // softmax scores over E experts; the top largest of (score + corr) chosen (ties: the lower expert);
 // ids[T, top], w[T, top] = bare scores; hist[E] += number of entries per expert (hist zeroed by the caller).
 // corr == null: the top largest logits are chosen and w = the softmax over the chosen logits only

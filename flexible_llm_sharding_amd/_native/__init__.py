@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 13   # csrc/include/fls_seq.h
+SEQ_ABI = 14   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -169,6 +169,7 @@ def _load_seq():
     _bind(lib, "fls_seq_rglru_scan", i, p, i, p, i, p, p, i, p, p, i, i, p, p, p, i, i, f, p)
     _bind(lib, "fls_seq_rglru_scan_tiled", i, p, i, p, i, p, p, i, p, p, i, i, p, i, p, p, p, p, i, i, f, p)
     _bind(lib, "fls_seq_ssd_scan", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, p)
+    _bind(lib, "fls_seq_ssd_scan_chunked", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, p, p)
     _bind(lib, "fls_seq_moe_route", i, p, i, p, i, i, i, p, p, p, p)
     _bind(lib, "fls_seq_moe_scan", i, p, i, p, p, p)
     _bind(lib, "fls_seq_moe_place", i, p, i, i, p, p, p, p)

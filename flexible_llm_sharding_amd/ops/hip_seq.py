@@ -890,6 +890,8 @@ class HipSeqOps:
                                        meta["n_seqs"], Wd, float(c), _stream()), "fls_seq_rglru_scan")
         return out
 
+    SSD_CHUNK_ROWS = 24        # rows of one request from which the chunked scan is the faster one
+
     def ssd_scan(self, xbc, z, dt, dt_bias, A_log, Dskip, state, meta, nh, P, N, G):
         _rows(xbc, "xbc", torch.float32)
         _rows(z, "z", torch.float32)
@@ -901,6 +903,15 @@ class HipSeqOps:
         for n, t in (("dt_bias", dt_bias), ("A_log", A_log), ("D", Dskip)):
             _vec(t, n, nh)
         out = torch.empty(T, inner, dtype=torch.float32, device=xbc.device)
+        if (meta["max_rows"] >= self.SSD_CHUNK_ROWS and N in (64, 128) and P % 16 == 0 and xbc.stride(0) % 4 == 0
+                and xbc.data_ptr() % 16 == 0):
+            scores = torch.empty(T * G * 64, dtype=torch.float32, device=xbc.device)
+            _chk(self.k.fls_seq_ssd_scan_chunked(xbc.data_ptr(), xbc.stride(0), z.data_ptr(), z.stride(0), dt.data_ptr(), dt.stride(0),
+                                                 dt_bias.data_ptr(), A_log.data_ptr(), Dskip.data_ptr(), state.data_ptr(),
+                                                 out.data_ptr(), inner, meta["cu"].data_ptr(), meta["pos0"].data_ptr(),
+                                                 meta["slot"].data_ptr(), meta["n_seqs"], int(meta["max_rows"]), nh, P, N, G,
+                                                 scores.data_ptr(), _stream()), "fls_seq_ssd_scan_chunked")
+            return out
         _chk(self.k.fls_seq_ssd_scan(xbc.data_ptr(), xbc.stride(0), z.data_ptr(), z.stride(0), dt.data_ptr(), dt.stride(0),
                                      dt_bias.data_ptr(), A_log.data_ptr(), Dskip.data_ptr(), state.data_ptr(),
                                      out.data_ptr(), inner, meta["cu"].data_ptr(), meta["pos0"].data_ptr(),

@@ -232,6 +232,37 @@ def test_conv_and_scans_carry_state(ops, cdt, tol):
             close(s1, s2, 3e-5)
 
 
+# the chunked state-space scan: chunk ends, one row, a carried state, one and two column tiles a block, groups; the oracle in fp64 (a
+# decay as strong as exp(-30) a row: differences of running sums must not lose it)
+@pytest.mark.parametrize("lens,pos0,nh,P,N,G,strong", [((64, 1, 65), (0, 7, 0), 4, 16, 64, 2, 0.0), ((200,), (5,), 2, 48, 128, 1, 0.0),
+                                                       ((24, 128), (0, 0), 2, 32, 128, 1, 3.0), ((40, 90), (0, 3), 128, 32, 64, 1, 0.0)])
+def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
+    H, R = ops
+    torch.manual_seed(sum(lens))
+    md, _, nslots = meta_of(lens, pos0, DEV)
+    T, inner = sum(lens), nh * P
+    xbc = torch.randn(T, inner + 2 * G * N, device=DEV)
+    z, dt = torch.randn(T, inner, device=DEV), torch.randn(T, nh, device=DEV)
+    dtb, Al, Ds = torch.randn(nh, device=DEV), torch.randn(nh, device=DEV) * 0.5 + strong, torch.randn(nh, device=DEV)
+    s1 = torch.randn(nslots, nh, N, P, device=DEV)
+    s2 = s1.cpu().double()
+    got = H.ssd_scan(xbc, z, dt, dtb, Al, Ds, s1, md, nh, P, N, G)
+    x, B, C = (t.cpu().double() for t in torch.split(xbc, [inner, G * N, G * N], 1))
+    dtv = torch.nn.functional.softplus((dt + dtb).cpu().double())
+    dec = torch.exp(-torch.exp(Al.cpu().double()) * dtv)
+    want = torch.empty(T, inner, dtype=torch.float64)
+    for s, (n, p0) in enumerate(zip(lens, pos0)):
+        a0, slot = int(md["cu_host"][s]), int(md["slot"][s])
+        S = s2[slot] if p0 else torch.zeros(nh, N, P, dtype=torch.float64)
+        for t in range(a0, a0 + n):
+            Bt, Ct = (v[t].reshape(G, N).repeat_interleave(nh // G, 0) for v in (B, C))
+            S = dec[t][:, None, None] * S + dtv[t][:, None, None] * Bt[:, :, None] * x[t].reshape(nh, 1, P)
+            want[t] = ((S * Ct[:, :, None]).sum(1) + Ds.cpu().double()[:, None] * x[t].reshape(nh, P)).reshape(-1)
+        s2[slot] = S
+    close(got, want * torch.nn.functional.silu(z.cpu().double()), 3e-6)
+    close(s1, s2, 3e-6)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("T,E,top", [(33, 10, 3), (700, 8, 2), (5, 40, 9), (300, 3, 1), (4, 8, 2), (10, 6, 3), (1, 5, 5)])
 def test_routing_and_expert_products(ops, cdt, tol, T, E, top):
