@@ -20,8 +20,8 @@ int fls_seq_version(void);
 // = [gate rows; up rows] (N / 2 each), C has N / 2 columns: silu(g) u, gelu(g) u, or the clamped gate of fls_seq_gate_mul
 // with limit p and alpha q; no bias), stored as type tc (fp32, or bf16 when the consumer is the next product).
 // a_rows (with offs; nullable): row r of the product is made from row a_rows[r] of A, which has at most M rows.
-// FLS_SEQ_NOT_SERVED: nothing was done -- a gated product or a_rows, and rows whose alignment or size only the general kernels take.
-#define FLS_SEQ_NOT_SERVED (-100)
+// SEQ_NOT_SERVED: nothing was done -- a gated product or a_rows, and rows whose alignment or size only the general kernels take.
+#define SEQ_NOT_SERVED (-100)
 int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias, const float* act,
                  int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
                  const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s);

@@ -327,7 +327,7 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
     if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, a_gs, a_mod, w_gs, c_gs, st);
     if (rc != 0) return rc == 1 ? 0 : rc;
   }
-  if (act_kind >= EPI_GATE || a_rows != nullptr) return FLS_SEQ_NOT_SERVED;
+  if (act_kind >= EPI_GATE || a_rows != nullptr) return SEQ_NOT_SERVED;
   // what is left has a ragged K or N or unaligned rows.  Tile side by the rows of a group (on average, for row
   // groups): 64, 128, or 256 when the problem still gives the chip a few hundred blocks
   const int gm = offs != nullptr ? M / groups : M;

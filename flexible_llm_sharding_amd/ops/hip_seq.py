@@ -471,7 +471,7 @@ class HipSeqOps:
             self.block_means(kc, vc, blocks, meta, G * d, Gv * dv)
         return q_out
 
-    NOT_SERVED = -100          # fls_seq.h FLS_SEQ_NOT_SERVED
+    NOT_SERVED = -100          # fls_seq.h SEQ_NOT_SERVED
 
     def _gemm(self, a, w, c, bias, M, N, K, lda, ldw, ldc, groups=1, offs=None, a_gs=0, a_mod=1, w_gs=0, c_gs=0,
               act=None, kind=0, act_n=0, p=0.0, q=0.0, a_rows=None):
