@@ -565,7 +565,7 @@ class ShardedRunner:
         batch = pack_step(entries, self.seq_cache)
         logits, am = self._decode_graphs.run(batch, self.seq_cache.generation)
         if any(e.want for e in entries):
-            lh, ah = logits.cpu().numpy(), am.cpu().numpy()        # (synchronous: the static outputs are reused)
+            lh, ah = self._decode_graphs.read(logits, am)          # (synchronous: the static outputs are reused)
             for i, e in enumerate(entries):
                 if len(e.want):
                     out[i] = (lh[i:i + 1].copy(), ah[i:i + 1].copy())

@@ -505,6 +505,8 @@ class StepBatch:
 def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
     """Pack one micro-batch of a step and claim its rows' places in ``cache`` (a
     runtime.seq_state.SequenceStateCache): pages for the new tokens, a state slot for a new request."""
+    if entries and all(len(e.tokens) == 1 for e in entries):
+        return _pack_tokens(entries, cache)
     ids, want, wc, cu, pos0, slot, prev = [], [], [], [0], [], [], []
     ps = cache.page_size
     for e in entries:
@@ -544,6 +546,33 @@ def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
     return StepBatch(rids, i32(ids), i32(seq), i32(pos), i32(cu), i32(pos0), i32(slot), table,
                      i32(pages.astype(np.int64) * ps + pos_a % ps), i32(want), wc, len(ids), max_rows, q_tiles, tile_cu, local,
                      {P: cache.block_table(rids, P) for P in cache.block_sizes}, np.concatenate(prev) if prev else None)
+
+
+def _pack_tokens(entries: Sequence[StepEntry], cache) -> StepBatch:
+    """:func:`pack_step` of one token per request (a decode step): row i is request i."""
+    B, ps = len(entries), cache.page_size
+    ids, want, pos0, slot, prev = [], [], [], [], []
+    for i, e in enumerate(entries):
+        p0, s = cache.extend(e.rid, 1)
+        pos0.append(p0)
+        slot.append(s)
+        ids.append(e.tokens[0])
+        if cache.prev_token:
+            prev.append(cache.advance_token(e.rid, e.tokens[0]))
+        for w in e.want:
+            if w != 0:
+                raise ValueError(f"request {e.rid!r}: a wanted place lies outside its 1 tokens")
+            want.append(i)
+    rids = [e.rid for e in entries]
+    table = cache.page_table(rids)
+    seq, pos = np.arange(B, dtype=np.int32), np.asarray(pos0, dtype=np.int32)
+    pages = table[seq, pos // ps]
+    if (pages < 0).any():
+        raise RuntimeError("a new token's page is missing from the page table")
+    i32 = lambda a: np.asarray(a, dtype=np.int32)
+    return StepBatch(rids, i32(ids), seq, pos, np.arange(B + 1, dtype=np.int32), pos.copy(), i32(slot), table,
+                     i32(pages.astype(np.int64) * ps + pos % ps), i32(want), [len(e.want) for e in entries], B, 1, None, None, None,
+                     {P: cache.block_table(rids, P) for P in cache.block_sizes}, i32(prev) if prev else None)
 
 
 def split_step(entries: Sequence[StepEntry], token_budget: int) -> List[List[int]]:
