@@ -9,9 +9,9 @@
 // b < (i - window + 1) / ab.P.
 //
 // The host cuts every request's rows of the step into tiles of up to 128 consecutive rows; a block
-// serves one tile and one query head, its four waves 32 query rows each.  Keys are walked 32 at a
+// serves one tile and one query head, its four waves 32 query rows each.  Keys are walked 64 at a
 // time, from the first key the tile's first row may see to the tile's last row, gathered from the
-// request's pages into LDS: K as [key][d], V transposed as [column][key].  Per key tile and wave:
+// request's pages into LDS: K as [key][d], V transposed as [column][key].  Per half of a key tile and wave:
 //   S^T = K Q^T        one 32x32x16 MFMA per 16 of d (Q fragments stay in registers): a lane then
 //                      holds 16 keys' scores of ONE query (column = lane % 32), its partner lane ^ 32
 //                      the other 16, so the softmax statistics are per-lane scalars: one shuffle
@@ -22,6 +22,14 @@
 //                      together), so the value product loses nothing to a bf16 rounding of p;
 //   O^T += V^T P^T     MFMAs again; O^T has the same column = query layout, so the rescale is a
 //                      per-lane multiply.
+//
+// What bounds it is the vector work per score beside the matrix work (24 MFMAs, 768 cycles, per half tile and wave with heads of
+// 128).  So scores are in units of log 2: exp and log are one instruction each and the penalty needs no factor.  The cap's
+// quotient is a reciprocal, bf16 terms come from the conversion instruction, and a half tile that every row of the wave sees
+// has no mask.  The accumulators are rescaled only when a maximum has grown by more than 8: weights stay below 2^8, which fp32
+// sums and two-term weights hold as exactly.  Tiles of 64 keys halve the barriers, and two keys of V make one 4-byte LDS store.
+// Measured against tiles of 32 with a rescale and a mask for every score:
+//   cap and distance penalty, 48 heads of 128:   2033 -> 988 us      fp32 queries, 9 layers' mean:   426 -> 222 and 317 -> 156 us
 #include "seq_common.h"
 #include "fls_seq.h"
 
@@ -30,6 +38,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 #define KT 32             // keys per tile
 #define PLD (KT + 8)      // row stride (elements) of the transposed V tile and of the weight tiles
+#define PT 64             // keys per tile of the prompt kernel, worked on in halves of KT
+#define VLD (PT + 8)
+#define LOG2E 1.4426950408889634f
+
+__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
+__device__ __forceinline__ float log2_hw(float x) { return __builtin_amdgcn_logf(x); }
+__device__ __forceinline__ float rcp_hw(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // (two waves per SIMD: a few registers over 256 would halve that)
 template <int D, int DV, typename TQ, typename TO, bool POOL>
@@ -43,13 +58,14 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
                                                            const float* __restrict__ gate_bias, float out_scale, int page_size,
                                                            int has_sink, float sink, const float* __restrict__ sink_h,
                                                            const float* __restrict__ head_gate,
-                                                           int ldhg, int Gv, AttnBlocks ab) {
+                                                           int ldhg, int Gv, AttnBlocks ab, int page_shift) {
   constexpr int KLD = D + 8;
-  __shared__ __attribute__((aligned(16))) bf16_t Ks[KT * KLD];
-  __shared__ __attribute__((aligned(16))) bf16_t Vt[DV * PLD];
+  __shared__ __attribute__((aligned(16))) bf16_t Ks[PT * KLD];
+  __shared__ __attribute__((aligned(16))) bf16_t Vt[DV * VLD];
   __shared__ __attribute__((aligned(16))) bf16_t Ps[4][2][32 * PLD];
   const int h = blockIdx.x, g = h / (H / G);
-  const int row0 = tiles[2 * blockIdx.y], nrows = tiles[2 * blockIdx.y + 1];
+  const int tile = gridDim.y - 1 - blockIdx.y;                       // (the last tiles of a long prompt have the most keys: they go first)
+  const int row0 = tiles[2 * tile], nrows = tiles[2 * tile + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int ql = lane & 31, h2 = lane >> 5;
   const int* table = page_table + (size_t)tok_seq[row0] * pt_stride;
@@ -66,6 +82,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
   const int w_first = i_first + wave * 32, w_last = min(i_last, w_first + 31);
   int lo_w = chunk > 0 ? (w_first / chunk) * chunk : 0;
   if (window > 0 && w_first - window + 1 > lo_w) lo_w = w_first - window + 1;
+  int lo_wl = chunk > 0 ? (w_last / chunk) * chunk : 0;              // the first key that the wave's last row sees: the latest of its rows
+  if (window > 0 && w_last - window + 1 > lo_wl) lo_wl = w_last - window + 1;
   bf16x8 Qf[D / 16];
   {
     const TQ* qp = q + (size_t)(row0 + (qok ? qrow : 0)) * ldq + (size_t)h * D + h2 * 8;
@@ -91,11 +109,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
 #pragma unroll
     for (int r = 0; r < 16; ++r) O[c][r] = 0.f;
   // (the softmax's silent entry of score `sink` / sink_h[h], if any, is where every query's running maximum and sum start)
-  float m = has_sink ? (sink_h != nullptr ? sink_h[h] : sink) : -1e30f, l = has_sink ? 1.f : 0.f;
+  float m = has_sink ? (sink_h != nullptr ? sink_h[h] : sink) * LOG2E : -1e30f, l = has_sink ? 1.f : 0.f;
   const float a1 = r1 != nullptr ? r1[h] : 0.f, a2 = r2 != nullptr ? r2[h] : 0.f;
   const bool gated = gate_bias != nullptr;
-  const float gb = gated ? gate_bias[h] : 0.f;
-  const float inv_cap = softcap > 0.f ? 1.f / softcap : 0.f;
+  const float gb = gated ? gate_bias[h] * LOG2E : 0.f;
+  // scores in units of log 2; with a cap: cap (1 - 2 / (exp(2 s / cap) + 1)), the exponential's argument straight from the product
+  const float sc_mul = softcap > 0.f ? 2.f * LOG2E * scale / softcap : scale * LOG2E;
+  const float cap2 = softcap * LOG2E;
   // key tiles: nt_keep tiles over the kept first keys [0, nkeep) that lie before the block's window,
   // then the tiles from lo_blk to the block's last row
   // (POOL: instead nt_keep tiles over the blocks [0, nkeep) that the block's last row sees)
@@ -104,16 +124,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
   const int keep_q = POOL ? seen_blocks(iq) : keep_first;            // what of them this lane's query sees ...
   const int keep_w = POOL ? seen_blocks(w_last) : keep_first;        // ... and any of the wave's
   const int* btable = POOL ? ab.table + (size_t)tok_seq[row0] * ab.t_stride : nullptr;
-  const int nt_keep = (nkeep + KT - 1) / KT;
-  const int nt = nt_keep + (i_last - lo_blk) / KT + 1;
+  const int nt_keep = (nkeep + PT - 1) / PT;
+  const int nt = nt_keep + (i_last - lo_blk) / PT + 1;
   // K / V of a key tile travel global -> registers -> LDS; the next tile's loads are issued before this
   // tile's matrix work and land in LDS after it, so the page gather's latency hides under the MFMAs
-  constexpr int PK = KT * (D / 8), PV = KT * (DV / 8);               // 16-byte pieces of a tile
+  constexpr int PK = PT * (D / 8), PV = PT / 2 * (DV / 8);           // 16-byte pieces of K; pieces of two neighbouring keys of V
   constexpr int NK = (PK + 255) / 256, NV = (PV + 255) / 256;        // per thread (the last one of some threads may be none)
-  uint4 kreg[NK], vreg[NV];
+  uint4 kreg[NK], vreg[NV][2];
+  auto pool_row = [&](const int* tab, int j) {
+    const int pg = page_shift >= 0 ? j >> page_shift : j / page_size;
+    return (size_t)tab[pg] * page_size + (j - pg * page_size);
+  };
   auto fetch = [&](int ti) {
     const bool pre = ti < nt_keep;
-    const int j0 = pre ? ti * KT : lo_blk + (ti - nt_keep) * KT;
+    const int j0 = pre ? ti * PT : lo_blk + (ti - nt_keep) * PT;
     const int jend = pre ? nkeep : i_last + 1;
     const int* tab = POOL && pre ? btable : table;
     const bf16_t* kb = POOL && pre ? reinterpret_cast<const bf16_t*>(ab.kp) : kc;
@@ -122,30 +146,27 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
 #pragma unroll
     for (int x = 0; x < NK; ++x) {
       const int e = threadIdx.x + 256 * x;
-      const int kk = e / (D / 8), seg = e % (D / 8);
-      const int j = j0 + kk;
+      const int j = j0 + e / (D / 8), seg = e % (D / 8);
       kreg[x] = make_uint4(0, 0, 0, 0);
-      if (j < jend && (PK % 256 == 0 || e < PK)) {
-        const size_t row = (size_t)tab[j / page_size] * page_size + j % page_size;
-        kreg[x] = *reinterpret_cast<const uint4*>(kb + row * lk + (size_t)g * D + seg * 8);
-      }
+      if (j < jend && (PK % 256 == 0 || e < PK)) kreg[x] = *reinterpret_cast<const uint4*>(kb + pool_row(tab, j) * lk + (size_t)g * D + seg * 8);
     }
 #pragma unroll
     for (int x = 0; x < NV; ++x) {
       const int e = threadIdx.x + 256 * x;
-      const int kk = e % KT, seg = e / KT;
-      const int j = j0 + kk;
-      vreg[x] = make_uint4(0, 0, 0, 0);
-      if (j < jend && (PV % 256 == 0 || e < PV)) {
-        const size_t row = (size_t)tab[j / page_size] * page_size + j % page_size;
-        vreg[x] = *reinterpret_cast<const uint4*>(vb + row * lv + (size_t)(g % Gv) * DV + seg * 8);
+      const int seg = e / (PT / 2);
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        const int j = j0 + 2 * (e % (PT / 2)) + y;
+        vreg[x][y] = make_uint4(0, 0, 0, 0);
+        if (j < jend && (PV % 256 == 0 || e < PV))
+          vreg[x][y] = *reinterpret_cast<const uint4*>(vb + pool_row(tab, j) * lv + (size_t)(g % Gv) * DV + seg * 8);
       }
     }
   };
   fetch(0);
   for (int ti = 0; ti < nt; ++ti) {
     const bool kept = ti < nt_keep;
-    const int j0 = kept ? ti * KT : lo_blk + (ti - nt_keep) * KT;
+    const int jt = kept ? ti * PT : lo_blk + (ti - nt_keep) * PT;
     const int jend = kept ? nkeep : i_last + 1;      // keys from jend on are padding of this tile
     __syncthreads();                          // the previous tile's readers are done
 #pragma unroll
@@ -154,71 +175,100 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
       if (PK % 256 == 0 || e < PK) *reinterpret_cast<uint4*>(Ks + (e / (D / 8)) * KLD + (e % (D / 8)) * 8) = kreg[x];
     }
 #pragma unroll
-    for (int x = 0; x < NV; ++x) {
+    for (int x = 0; x < NV; ++x) {            // (two keys of a column make one 4-byte store)
       const int e = threadIdx.x + 256 * x;
-      const int kk = e % KT, seg = e / KT;
-      const bf16_t* ev = reinterpret_cast<const bf16_t*>(&vreg[x]);
       if (PV % 256 != 0 && e >= PV) continue;
+      uint32_t* dst = reinterpret_cast<uint32_t*>(Vt + (e / (PT / 2)) * 8 * VLD) + e % (PT / 2);
+      const uint32_t a[4] = {vreg[x][0].x, vreg[x][0].y, vreg[x][0].z, vreg[x][0].w}, b[4] = {vreg[x][1].x, vreg[x][1].y, vreg[x][1].z, vreg[x][1].w};
 #pragma unroll
-      for (int y = 0; y < 8; ++y) Vt[(seg * 8 + y) * PLD + kk] = ev[y];
+      for (int y = 0; y < 4; ++y) {
+        dst[2 * y * (VLD / 2)] = __builtin_amdgcn_perm(b[y], a[y], 0x05040100);
+        dst[(2 * y + 1) * (VLD / 2)] = __builtin_amdgcn_perm(b[y], a[y], 0x07060302);
+      }
     }
     __syncthreads();
     if (ti + 1 < nt) fetch(ti + 1);
-    if (wave * 32 >= nrows || (POOL && kept && j0 >= keep_w) ||
+#pragma unroll 1
+    for (int half = 0; half < 2; ++half) {
+    const int j0 = jt + half * KT;
+    if (j0 >= jend || wave * 32 >= nrows || (POOL && kept && j0 >= keep_w) ||
         (!kept && (j0 > w_last || (j0 + KT - 1 < lo_w && (POOL || j0 >= keep_first))))) continue;   // (wave-uniform)
+    // every row of the wave sees every key of this half (rows past the tile's end compute what nobody stores)
+    const bool full = !kept && j0 + KT - 1 <= w_first && j0 >= lo_wl;
     floatx16 S;
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[r] = 0.f;
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) {
-      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(Ks + ql * KLD + 16 * s + h2 * 8);
+      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(Ks + (half * KT + ql) * KLD + 16 * s + h2 * 8);
       S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, Qf[s], S, 0, 0, 0);
     }
     float p[16];
     float mt = -1e30f;
+    // (this kernel serves bf16 models only: the hardware exp / log / reciprocal are far inside their rounding)
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int j = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
-      // (this kernel serves bf16 models only: the hardware exp / log are far inside their rounding)
-      float sc = S[r] * scale;
-      if (softcap > 0.f) sc = softcap * (1.f - 2.f / (__expf(2.f * sc * inv_cap) + 1.f));
-      if (a1 != 0.f) sc -= a1 * __logf(1.f + a2 * (float)max(iq - j, 0));
-      const bool vis = POOL ? qok && (kept ? j < keep_q : j >= lo_q && j <= iq)
-                            : qok && j < jend && j <= iq && (j >= lo_q || j < keep_first);
-      if (gated) p[r] = vis ? 1.f / (1.f + __expf(-(sc + gb))) : 0.f;
-      else p[r] = vis ? sc : -1e30f;
-      mt = fmaxf(mt, p[r]);
+    for (int r = 0; r < 16; ++r) p[r] = S[r] * sc_mul;
+    if (softcap > 0.f) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = cap2 - 2.f * cap2 * rcp_hw(exp2_hw(p[r]) + 1.f);
     }
-    if (!gated) {
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      mt = fmaxf(mt, m);
-      float ps = 0.f;
+    if (a1 != 0.f) {
+      const float dist0 = (float)(iq - j0 - 4 * h2);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] -= a1 * log2_hw(1.f + a2 * fmaxf(dist0 - (float)(8 * (r >> 2) + (r & 3)), 0.f));
+    }
+    if (gated) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) p[r] = rcp_hw(1.f + exp2_hw(-(p[r] + gb)));
+    }
+    if (!full) {
+      // the row sees keys [mlo, mhi] and, of a window's tiles, those before keep_first (no key of a row past the tile's end)
+      const int jb = j0 + 4 * h2;
+      const int mlo = (kept ? 0 : lo_q) - jb, mkeep = (POOL ? 0 : keep_first) - jb;
+      const int mhi = (!qok ? -1 : POOL ? (kept ? keep_q - 1 : iq) : min(iq, jend - 1)) - jb;
+      const float hidden = gated ? 0.f : -1e30f;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        p[r] = p[r] > -1e29f ? __expf(p[r] - mt) : 0.f;
-        ps += p[r];
+        const int o = 8 * (r >> 2) + (r & 3);
+        const bool vis = (o <= mhi) & ((o >= mlo) | (o < mkeep));
+        p[r] = vis ? p[r] : hidden;
       }
-      ps += __shfl_xor(ps, 32, 64);
-      const float corr = __expf(m - mt);
-      l = l * corr + ps;
-      m = mt;
+    }
+    if (!gated) {
 #pragma unroll
-      for (int c = 0; c < DV / 32; ++c)
+      for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[r]);
+      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      if (__any(mt > m + 8.f)) {               // (wave-uniform)
+        mt = fmaxf(mt, m);
+        const float corr = exp2_hw(m - mt);
+        l *= corr;
+        m = mt;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) O[c][r] *= corr;
+        for (int c = 0; c < DV / 32; ++c)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) O[c][r] *= corr;
+      }
+      float ps = 0.f;
+      if (full) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { p[r] = exp2_hw(p[r] - m); ps += p[r]; }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) { p[r] = p[r] > -1e29f ? exp2_hw(p[r] - m) : 0.f; ps += p[r]; }
+      }
+      l += ps + __shfl_xor(ps, 32, 64);
     }
     bf16_t* ph = Ps[wave][0] + ql * PLD;
     bf16_t* pl = Ps[wave][1] + ql * PLD;
 #pragma unroll
     for (int rg = 0; rg < 4; ++rg) {
-      bf16_t hi[4], lo[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        hi[x] = f_to_bf16(p[4 * rg + x]);
-        lo[x] = f_to_bf16(p[4 * rg + x] - bf16_to_f(hi[x]));
-      }
-      *reinterpret_cast<uint2*>(ph + 8 * rg + 4 * h2) = *reinterpret_cast<const uint2*>(hi);
-      *reinterpret_cast<uint2*>(pl + 8 * rg + 4 * h2) = *reinterpret_cast<const uint2*>(lo);
+      typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+      typedef float floatx4 __attribute__((ext_vector_type(4)));
+      const floatx4 v = {p[4 * rg], p[4 * rg + 1], p[4 * rg + 2], p[4 * rg + 3]};
+      const bf16x4 hi = __builtin_convertvector(v, bf16x4);
+      const bf16x4 lo = __builtin_convertvector(v - __builtin_convertvector(hi, floatx4), bf16x4);
+      *reinterpret_cast<bf16x4*>(ph + 8 * rg + 4 * h2) = hi;
+      *reinterpret_cast<bf16x4*>(pl + 8 * rg + 4 * h2) = lo;
     }
     __builtin_amdgcn_wave_barrier();          // (a wave reads back its own lanes' writes: LDS is in order per wave)
 #pragma unroll
@@ -227,12 +277,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
       const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pl + 16 * ks + 8 * h2);
 #pragma unroll
       for (int c = 0; c < DV / 32; ++c) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(Vt + (32 * c + ql) * PLD + 16 * ks + 8 * h2);
+        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(Vt + (32 * c + ql) * VLD + half * KT + 16 * ks + 8 * h2);
         O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bh, O[c], 0, 0, 0);
         O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bl, O[c], 0, 0, 0);
       }
     }
     __builtin_amdgcn_wave_barrier();
+    }
   }
   if (qok && (gated || l > 0.f)) {
     float inv = gated ? out_scale : out_scale / l;
@@ -276,13 +327,14 @@ extern "C" int fls_seq_attn_prefill(const void* q, int ldq, int tq, const void* 
     return -1;                                          // (blocks go with a plain softmax over a window)
   if (pool_P > 0 && (tq != 0 || ldkp % 8 || ldvp % 8 || (uintptr_t)kp % 16 || (uintptr_t)vp % 16)) return -2;
   const AttnBlocks ab = {pool_P, kp, ldkp, vp, ldvp, block_table, bt_stride};
+  const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   dim3 grid(H, n_tiles);
   hipStream_t st = (hipStream_t)s;
 #define ATTN_PF_(DD, DDV, TQ_, TO_, PP)                                                                                   \
   hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, TQ_, TO_, PP>), grid, dim3(256), 0, st, (const TQ_*)q, ldq,            \
                      (const bf16_t*)kc, ldk, (const bf16_t*)vc, ldv, (TO_*)out, ldo, tiles, tok_seq, tok_pos,             \
                      page_table, pt_stride, H, G, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias,           \
-                     out_scale, page_size, has_sink, sink, sink_h, head_gate, ldhg, Gv, ab)
+                     out_scale, page_size, has_sink, sink, sink_h, head_gate, ldhg, Gv, ab, page_shift)
 #define ATTN_PF(DD, DDV)                                                                                                  \
   do {                                                                                                                    \
     if (tq == 1 && to == 1) ATTN_PF_(DD, DDV, bf16_t, bf16_t, false);                                                     \

@@ -201,6 +201,39 @@ def test_attention(ops, cdt, tol, Hh, G, d, dv):
         close(o1, o2, tol)
 
 
+# prompt attention over 64-key tiles in two halves: lengths about a half, a tile and a 128-row block, windows and chunks that end inside
+# a half, kept first keys, pages of 24 (no power of two); `grow`: scores that rise along the keys in small steps or in large ones
+# (the running maximum stays behind by up to 8 units of log 2), with a sink far below, near and far above them.  bf16 tolerance as above
+@pytest.mark.parametrize("lens,pos0", [([31, 33], [0, 0]), ([64, 65], [0, 7]), ([129], [0]), ([200], [333])])
+@pytest.mark.parametrize("d,dv,ps", [(64, 128, 24), (128, 128, 16)])
+def test_prompt_attention_tiles(ops, lens, pos0, d, dv, ps):
+    H, R = ops
+    Hh, G, T = 4, 2, sum(lens)
+    torch.manual_seed(T + d)
+    md, npages, _ = meta_of(lens, pos0, DEV, ps)
+    kc, vc = torch.randn(npages, ps, G * d, device=DEV).bfloat16(), torch.randn(npages, ps, G * dv, device=DEV).bfloat16()
+    q = torch.randn(T, Hh * d, device=DEV).bfloat16()
+    for chunk, window, keep in ((0, 0, 0), (45, 0, 0), (0, 37, 0), (0, 37, 5), (0, 100, 70)):
+        for qq in (q, q.float()):
+            o1, o2 = (o.attn_paged(qq, kc, vc, md, Hh, G, d, dv, d ** -0.5, 0.0, None, None, chunk, ps, torch.bfloat16, window=window,
+                                   keep_first=keep) for o in (H, R))
+            close(o1, o2, 2e-2)
+    for step in (0.02, 0.9):
+        order = torch.arange(max(p + n for p, n in zip(pos0, lens)), device=DEV, dtype=torch.float32)
+        kg = kc.clone().view(npages * ps, G, d)
+        for b in range(len(lens)):
+            j = torch.arange(pos0[b] + lens[b], device=DEV)
+            rows = md["page_table"][b].long()[j // ps] * ps + j % ps
+            kg[rows, :, 0] = (order[:len(j), None] * step).bfloat16()
+        qg = q.clone().view(T, Hh, d)
+        qg[:, :, 0] = 1.0
+        for sink in (None, -20.0, 5.0, 60.0):
+            kw = {} if sink is None else dict(sink=sink)
+            o1, o2 = (o.attn_paged(qg.view(T, -1), kg.view(npages, ps, G * d), vc, md, Hh, G, d, dv, 0.3, 0.0, None, None, 0, ps,
+                                   torch.bfloat16, **kw) for o in (H, R))
+            close(o1, o2, 2e-2)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_conv_and_scans_carry_state(ops, cdt, tol):
     H, R = ops
