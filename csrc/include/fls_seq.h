@@ -140,13 +140,15 @@ int fls_seq_block_means(const void* kc, int ldk, const void* vc, int ldv, int tc
 // w = exp(-decay_scale sigmoid(wz + w0)), a = sigmoid(az); out = out_scale o / rms_head(o; norm_eps) norm_w sigmoid(g).
 // r, k, v, az, wz, g: fp32 [T, H d] with their row strides; d <= 128.  col_splits > 1 (a divisor of d): the
 // columns of every state are cut over that many blocks (few heads x requests, many rows) and the outputs
-// are finished by a second kernel; raw: T H d floats of scratch
+// are finished by a second kernel; raw: T H d floats of scratch.  fac (nullable) with raw: requests of up to max_rows rows in chunks of
+// 16, seg chunks of every request at a time (delta_chunk.hip): B H seg (65 d + 768) floats, 16-byte aligned; head sizes and alignments
+// that form does not serve go row by row
 int fls_seq_delta_rule_scan(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* az,
                             int lda, const float* wz, int ldw, const float* g, int ldg, const float* w0,
                             const float* norm_w, float* state, void* out, int to, int ldo, const int* cu,
                             const int* pos0, const int* slot, int T, int B, int H, int d, float decay_scale,
                             float key_eps, float norm_eps, float out_scale, int col_splits, float* raw,
-                            fls_stream_t s);
+                            int max_rows, float* fac, int seg, fls_stream_t s);
 // S_t = a_t S_(t-1) + sqrt(1 - a_t^2) sigmoid(g[t, W + c]) u_t, a_t = exp(-c sigmoid(g[t, c]) softplus(lam));
 // out = S_t * gelu_tanh(y_t); state[slot][W]
 int fls_seq_rglru_scan(const float* u, int ldu, const float* g, int ldg, const float* lam, const float* y, int ldy,
@@ -244,11 +246,11 @@ int fls_seq_latent_rows(const float* z, int ldz, int qr, int r, int dr, const fl
 // state[slot][H][dv][d]: S <- diag(g) S; u = sigmoid(beta) (v - S^T k); S <- S + k u^T; o = S^T q.  qkv = fp32 rows
 // [q (G d) | k (G d) | v (H dv)], head h reads q / k head h / (H / G); q and k are divided by sqrt(sum(x^2) + unit_eps), q times
 // q_scale; decay: fp32 [T, H d] in (0, 1]; out = o / sqrt(mean_head(o^2) + norm_eps) norm_w sigmoid(gate).  d <= 256, dv <= 512.
-// raw: T H dv floats of scratch (16-byte aligned)
+// raw: T H dv floats of scratch (16-byte aligned).  fac (nullable): as above, B H seg (49 d + 512) floats
 int fls_seq_gated_delta_scan(const float* qkv, int ldq, const float* beta, int ldb, const float* decay, int ldd, const float* gate,
                              int ldg, const float* norm_w, float* state, float* raw, void* out, int to, int ldo, const int* cu,
                              const int* pos0, const int* slot, int T, int B, int one_row_each, int H, int G, int d, int dv,
-                             float q_scale, float unit_eps, float norm_eps, fls_stream_t s);
+                             float q_scale, float unit_eps, float norm_eps, int max_rows, float* fac, int seg, fls_stream_t s);
 #ifdef __cplusplus
 }
 #endif

@@ -24,6 +24,12 @@
 #include "seq_common.h"
 #include "fls_seq.h"
 
+// delta_chunk.hip
+int seq_delta_rule_chunked(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* az, int lda,
+                           const float* wz, int ldw, const float* w0, float* state, float* raw, const int* cu, const int* pos0,
+                           const int* slot, int B, int H, int d, float decay_scale, float key_eps, int max_rows, float* fac, int seg,
+                           fls_stream_t s);
+
 #define DR_MAX_D 128
 #define DR_ROWS 256          // LDS floats per staged vector: TP rows x d channels <= 256
 
@@ -207,9 +213,22 @@ extern "C" int fls_seq_delta_rule_scan(const float* r, int ldr, const float* k, 
                                        const float* norm_w, float* state, void* out, int to, int ldo, const int* cu,
                                        const int* pos0, const int* slot, int T, int B, int H, int d, float decay_scale,
                                        float key_eps, float norm_eps, float out_scale, int col_splits, float* raw,
-                                       fls_stream_t s) {
+                                       int max_rows, float* fac, int seg, fls_stream_t s) {
   if (B <= 0 || H <= 0) return 0;
   if (d < 1 || d > DR_MAX_D || col_splits < 1 || d % col_splits || (col_splits > 1 && raw == nullptr)) return -1;
+  auto finish = [&]() {
+    const int items = T * H;
+    if (items <= 0) return 0;
+    if (to == 1) hipLaunchKernelGGL((delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (bf16_t*)out, ldo, H, d, norm_eps, out_scale, items);
+    else hipLaunchKernelGGL((delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (float*)out, ldo, H, d, norm_eps, out_scale, items);
+    SEQ_LAUNCH_CHECK();
+    return 0;
+  };
+  if (fac != nullptr && raw != nullptr) {            // (the caller's rule: requests with many rows)
+    const int rc = seq_delta_rule_chunked(r, ldr, k, ldk, v, ldv, az, lda, wz, ldw, w0, state, raw, cu, pos0, slot, B, H, d, decay_scale,
+                                          key_eps, max_rows, fac, seg, s);
+    if (rc != -2) return rc != 0 ? rc : finish();
+  }
   // a wave owns cw = ceil(d / 4) columns, spanned by 1 << cwl lanes; the 64 >> cwl row groups of a wave hold
   // ceil(d / groups) rows each (rounded up to the next kernel instance)
   const int cw = (d / col_splits + 3) / 4;
@@ -233,11 +252,5 @@ extern "C" int fls_seq_delta_rule_scan(const float* r, int ldr, const float* k, 
   }
 #undef DR_ARGS
   SEQ_LAUNCH_CHECK();
-  if (col_splits > 1 && T > 0) {
-    const int items = T * H;
-    if (to == 1) hipLaunchKernelGGL((delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, st, raw, g, ldg, norm_w, (bf16_t*)out, ldo, H, d, norm_eps, out_scale, items);
-    else hipLaunchKernelGGL((delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, st, raw, g, ldg, norm_w, (float*)out, ldo, H, d, norm_eps, out_scale, items);
-    SEQ_LAUNCH_CHECK();
-  }
-  return 0;
+  return col_splits > 1 ? finish() : 0;
 }

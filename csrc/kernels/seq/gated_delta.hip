@@ -17,6 +17,11 @@
 #include "seq_common.h"
 #include "fls_seq.h"
 
+// delta_chunk.hip
+int seq_gated_delta_chunked(const float* qkv, int ldq, const float* beta, int ldb, const float* decay, int ldd, float* state, float* raw,
+                            const int* cu, const int* pos0, const int* slot, int B, int H, int G, int d, int dv, float q_scale,
+                            float unit_eps, int max_rows, float* fac, int seg, fls_stream_t s);
+
 template <int RPL, int CN, int WAVES, int TT, bool FUSED, typename TO>
 __global__ __launch_bounds__(64 * WAVES) void gated_delta_kernel(const float* __restrict__ qkv, int ldq, const float* __restrict__ beta,
                                                                  int ldb, const float* __restrict__ decay, int ldd,
@@ -222,7 +227,8 @@ __global__ __launch_bounds__(256) void gated_delta_out_kernel(const float* __res
 extern "C" int fls_seq_gated_delta_scan(const float* qkv, int ldq, const float* beta, int ldb, const float* decay, int ldd,
                                         const float* gate, int ldg, const float* norm_w, float* state, float* raw, void* out, int to,
                                         int ldo, const int* cu, const int* pos0, const int* slot, int T, int B, int one_row_each,
-                                        int H, int G, int d, int dv, float q_scale, float unit_eps, float norm_eps, fls_stream_t s) {
+                                        int H, int G, int d, int dv, float q_scale, float unit_eps, float norm_eps, int max_rows,
+                                        float* fac, int seg, fls_stream_t s) {
   if (T <= 0 || B <= 0) return 0;
   if (d < 1 || d > 256 || dv < 1 || dv > 512 || H < 1 || G < 1 || H % G) return -1;
   const int vec = d % 4 == 0 && ldq % 4 == 0 && ldd % 4 == 0 && (uintptr_t)qkv % 16 == 0 && (uintptr_t)decay % 16 == 0 &&
@@ -247,18 +253,26 @@ extern "C" int fls_seq_gated_delta_scan(const float* qkv, int ldq, const float* 
     }
   }
   if (raw == nullptr) return -1;
-  // as many columns a lane as still leave the chip two waves per SIMD: the factors read from LDS serve them all
-  int cn = rpl == 16 ? 2 : 4;
-  while (cn > 1 && (long long)H * B * ((dv + 16 * cn - 1) / (16 * cn)) * 4 < 2048) cn /= 2;
+  int rc = -2;
+  if (fac != nullptr) {                              // (the caller's rule: requests with many rows)
+    rc = seq_gated_delta_chunked(qkv, ldq, beta, ldb, decay, ldd, state, raw, cu, pos0, slot, B, H, G, d, dv, q_scale, unit_eps, max_rows,
+                                 fac, seg, s);
+    if (rc != 0 && rc != -2) return rc;
+  }
+  if (rc != 0) {
+    // as many columns a lane as still leave the chip two waves per SIMD: the factors read from LDS serve them all
+    int cn = rpl == 16 ? 2 : 4;
+    while (cn > 1 && (long long)H * B * ((dv + 16 * cn - 1) / (16 * cn)) * 4 < 2048) cn /= 2;
 #define GD_P(R, C) hipLaunchKernelGGL((gated_delta_kernel<R, C, 4, 16, false, float>), dim3((dv + 16 * C - 1) / (16 * C), H, B), dim3(256), 0, st, \
                                       GD_ARGS, raw, H * dv, GD_TAIL)
-  if (rpl == 4) { if (cn == 1) GD_P(4, 1); else if (cn == 2) GD_P(4, 2); else GD_P(4, 4); }
-  else if (rpl == 8) { if (cn == 1) GD_P(8, 1); else if (cn == 2) GD_P(8, 2); else GD_P(8, 4); }
-  else { if (cn == 1) GD_P(16, 1); else GD_P(16, 2); }
+    if (rpl == 4) { if (cn == 1) GD_P(4, 1); else if (cn == 2) GD_P(4, 2); else GD_P(4, 4); }
+    else if (rpl == 8) { if (cn == 1) GD_P(8, 1); else if (cn == 2) GD_P(8, 2); else GD_P(8, 4); }
+    else { if (cn == 1) GD_P(16, 1); else GD_P(16, 2); }
 #undef GD_P
+    SEQ_LAUNCH_CHECK();
+  }
 #undef GD_ARGS
 #undef GD_TAIL
-  SEQ_LAUNCH_CHECK();
   const int items = T * H;
   if (to == 1) hipLaunchKernelGGL((gated_delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (bf16_t*)out, ldo, H, dv, norm_eps, items);
   else hipLaunchKernelGGL((gated_delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (float*)out, ldo, H, dv, norm_eps, items);

@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 14   # csrc/include/fls_seq.h
+SEQ_ABI = 15   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -156,7 +156,7 @@ def _load_seq():
     _bind(lib, "fls_seq_gate_mul", i, p, i, p, i, i, i, i, i, f, f, p)
     _bind(lib, "fls_seq_unary", i, p, i, p, i, i, i, i, i, p)
     _bind(lib, "fls_seq_head_norm_rope", i, p, i, i, i, i, i, i, p, f, p, i, p, p, p, i, i, i, i, p, i, i, i, i, f, p)
-    _bind(lib, "fls_seq_delta_rule_scan", i, p, i, p, i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, f, f, f, f, i, p, p)
+    _bind(lib, "fls_seq_delta_rule_scan", i, p, i, p, i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, f, f, f, f, i, p, i, p, i, p)
     _bind(lib, "fls_seq_softcap", i, p, i, i, i, f, p)
     _bind(lib, "fls_seq_argmax", i, p, i, i, i, p, p)
     _bind(lib, "fls_seq_kv_store", i, p, i, p, f, p, i, p, p, i, p, i, i, i, p)
@@ -180,7 +180,7 @@ def _load_seq():
     _bind(lib, "fls_seq_rmsnorm_pair", i, p, i, p, i, p, p, i, p, p, i, i, i, i, f, p)
     _bind(lib, "fls_seq_parallel_update", i, p, i, p, i, p, p, i, p, p, i, p, p, p, i, i, p, i, i, i, i, p)
     _bind(lib, "fls_seq_latent_rows", i, p, i, i, i, i, p, p, f, p, i, p, p, p, i, p, i, i, i, p)
-    _bind(lib, "fls_seq_gated_delta_scan", i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, i, i, i, f, f, f, p)
+    _bind(lib, "fls_seq_gated_delta_scan", i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, i, i, i, f, f, f, i, p, i, p)
     _bind(lib, "fls_seq_streams_norm", i, p, i, p, p, p, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_streams_update", i, p, i, p, i, p, i, p, f, i, i, i, p, p, p, i, i, f, p)
     _bind(lib, "fls_seq_scale", i, p, i, i, i, f, p)

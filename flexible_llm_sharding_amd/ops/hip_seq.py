@@ -815,6 +815,25 @@ class HipSeqOps:
              "fls_seq_causal_conv")
         return out
 
+    # rows of one request from which the chunked delta rules are the faster ones.  1 request, 16 heads of 64, 16 / 24 / 64 rows: 21 / 25 /
+    # 57 us row by row, 22 / 23 / 25 in chunks; gated, 16 heads of 128: 1 request of 48 / 64 rows 21 / 25 and 24 / 26, 8 of 64: 46 and 36
+    DELTA_CHUNK_ROWS = 24
+    GATED_CHUNK_ROWS = 64
+    # 9 requests of 1500 rows (gated): 900 / 750 / 680 / 658 us with 32 / 64 / 128 / 256 MB, 1060 row by row
+    DELTA_FACTOR_BYTES = 128 << 20
+
+    def _delta_factors(self, meta, heads, dim, mats, least, device):
+        """Memory for the chunks' factors of the delta rules, ``mats`` matrices of 16 x dim and the small ones a chunk and head, for as many
+        chunks at a time as stay in the last-level cache; (None, 0) where a row-by-row walk serves: short requests, and so many that
+        less than four chunks of each fit (200 requests of 300 rows: 2.5 ms row by row, 4.6 ms a chunk at a time)."""
+        rows = int(meta.get("max_rows") or 0)
+        each = meta["n_seqs"] * heads * (16 * dim * mats + 256 * (mats - 1) + dim)
+        chunks = -(-rows // 16)
+        seg = min(chunks, self.DELTA_FACTOR_BYTES // (4 * each))
+        if rows < least or dim not in (64, 128) or seg < min(chunks, 4):
+            return None, 0
+        return torch.empty(seg * each, dtype=torch.float32, device=device), seg
+
     def delta_rule_scan(self, r, k, v, a, wz, g, w0, norm_w, state, meta, heads, dim, decay_scale, key_eps, norm_eps,
                         out_scale, out):
         T, hd = r.shape[0], heads * dim
@@ -834,14 +853,16 @@ class HipSeqOps:
         if meta.get("q_tiles") is not None:
             while heads * meta["n_seqs"] * splits < 512 and splits < 4 and dim % (2 * splits) == 0 and dim // (2 * splits) >= 8:
                 splits *= 2
-        raw = torch.empty(T * hd, dtype=torch.float32, device=r.device) if splits > 1 else None
+        fac, seg = self._delta_factors(meta, heads, dim, 4, self.DELTA_CHUNK_ROWS, r.device)
+        raw = torch.empty(T * hd, dtype=torch.float32, device=r.device) if splits > 1 or fac is not None else None
         _chk(self.k.fls_seq_delta_rule_scan(r.data_ptr(), r.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0),
                                             a.data_ptr(), a.stride(0), wz.data_ptr(), wz.stride(0), g.data_ptr(), g.stride(0),
                                             w0.data_ptr(), norm_w.data_ptr(), state.data_ptr(), out.data_ptr(),
                                             _code(out, "out"), out.stride(0), meta["cu"].data_ptr(), meta["pos0"].data_ptr(),
                                             meta["slot"].data_ptr(), T, meta["n_seqs"], heads, dim, float(decay_scale),
                                             float(key_eps), float(norm_eps), float(out_scale), splits,
-                                            raw.data_ptr() if raw is not None else None, _stream()),
+                                            raw.data_ptr() if raw is not None else None, int(meta.get("max_rows") or 0),
+                                            fac.data_ptr() if fac is not None else None, seg, _stream()),
              "fls_seq_delta_rule_scan")
         return out
 
@@ -857,11 +878,13 @@ class HipSeqOps:
         out = torch.empty(T, H * dv, dtype=out_dtype, device=qkv.device)
         one_each = meta.get("max_rows") == 1
         raw = torch.empty(T * H * dv, dtype=torch.float32, device=qkv.device)
+        fac, seg = self._delta_factors(meta, H, d, 3, self.GATED_CHUNK_ROWS, qkv.device) if dv % 16 == 0 else (None, 0)
         _chk(self.k.fls_seq_gated_delta_scan(qkv.data_ptr(), qkv.stride(0), beta.data_ptr(), beta.stride(0), decay.data_ptr(),
                                              decay.stride(0), gate.data_ptr(), gate.stride(0), norm_w.data_ptr(), state.data_ptr(),
                                              raw.data_ptr(), out.data_ptr(), _CODE[out_dtype], out.stride(0), meta["cu"].data_ptr(),
                                              meta["pos0"].data_ptr(), meta["slot"].data_ptr(), T, meta["n_seqs"],
-                                             1 if one_each else 0, H, G, d, dv, d ** -0.5, float(unit_eps), float(norm_eps), _stream()),
+                                             1 if one_each else 0, H, G, d, dv, d ** -0.5, float(unit_eps), float(norm_eps),
+                                             int(meta.get("max_rows") or 0), fac.data_ptr() if fac is not None else None, seg, _stream()),
              "fls_seq_gated_delta_scan")
         return out
 

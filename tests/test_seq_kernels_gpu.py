@@ -296,6 +296,59 @@ def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
     close(s1, s2, 3e-6)
 
 
+# the chunked delta rules: chunk ends, one row and none beside long requests, a carried state, shared keys, value columns that do not fill
+# four waves, decays from none to exact zeros, and (small memory) several launches that pass the state on; the oracle in fp64.  The
+# bound is that of fp32 sums over some 128 terms and 16-row chains; the row-by-row kernels have to meet it too
+@pytest.mark.parametrize("lens,pos0", [([24, 1, 15], [0, 3, 5]), ([16, 17, 33], [7, 0, 0]), ([150, 31], [0, 64])])
+@pytest.mark.parametrize("d,dv,heads,kv,small", [(64, 64, 3, 3, False), (128, 128, 2, 1, True), (128, 48, 4, 2, False), (64, 160, 2, 2, True)])
+def test_delta_chunks(ops, monkeypatch, lens, pos0, d, dv, heads, kv, small):
+    H, _ = ops
+    torch.manual_seed(sum(lens) + d)
+    md, _, nslots = meta_of(lens, pos0, DEV)
+    T, hd = sum(lens), heads * d
+    f64 = lambda t, *shape: t.cpu().double().reshape(T, *shape)
+    qkv, beta, gate = torch.randn(T, 2 * kv * d + heads * dv, device=DEV), torch.randn(T, heads, device=DEV), torch.randn(T, heads * dv, device=DEV)
+    dec, nw = torch.rand(T, hd, device=DEV) ** 3, torch.randn(dv, device=DEV)
+    dec[:, ::5], dec[:, 1::7] = 1.0, 0.0
+    st = torch.randn(nslots, heads, dv, d, device=DEV)
+    z, w0, nw2 = torch.randn(T, 6 * hd, device=DEV), torch.randn(hd, device=DEV) - 2.0, torch.randn(hd, device=DEV)
+    r, k, v, a, wz, g = (z[:, i * hd:(i + 1) * hd] for i in range(6))
+    st2 = torch.randn(nslots, heads, d, d, device=DEV)
+    # fp64: gated, then generalized
+    unit = lambda x, eps: x / (x.pow(2).sum(-1, keepdim=True) + eps).sqrt()
+    q6 = (unit(f64(qkv[:, :kv * d], kv, d), 1e-6) * d ** -0.5).repeat_interleave(heads // kv, 1)
+    k6 = unit(f64(qkv[:, kv * d:2 * kv * d], kv, d), 1e-6).repeat_interleave(heads // kv, 1)
+    v6, b6, g6 = f64(qkv[:, 2 * kv * d:], heads, dv), torch.sigmoid(f64(beta, heads)), f64(dec, heads, d)
+    r7, k7, v7, a7 = f64(r, heads, d), f64(k, heads, d), f64(v, heads, d), torch.sigmoid(f64(a, heads, d))
+    w7, u7 = torch.exp(-0.6065 * torch.sigmoid(f64(wz, heads, d) + w0.cpu().double().reshape(heads, d))), unit(f64(k, heads, d), 1e-6)
+    want, want2, o6, o7 = st.cpu().double(), st2.cpu().double(), torch.empty(T, heads, dv).double(), torch.empty(T, heads, d).double()
+    for s, (n, p0) in enumerate(zip(lens, pos0)):
+        a0, slot = int(md["cu_host"][s]), int(md["slot"][s])
+        S, S2 = want[slot] * bool(p0), want2[slot] * bool(p0)
+        for t in range(a0, a0 + n):
+            S = S * g6[t][:, None, :]
+            S = S + (b6[t][:, None] * (v6[t] - (S * k6[t][:, None, :]).sum(-1)))[:, :, None] * k6[t][:, None, :]
+            o6[t] = (S * q6[t][:, None, :]).sum(-1)
+            x = (S2 * u7[t][:, :, None]).sum(1)
+            S2 = w7[t][:, :, None] * S2 - (a7[t] * u7[t])[:, :, None] * x[:, None, :] + k7[t][:, :, None] * v7[t][:, None, :]
+            o7[t] = (S2 * r7[t][:, :, None]).sum(1)
+        want[slot], want2[slot] = S, S2
+    o6 = o6 / (o6.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt() * nw.cpu().double()
+    o6 = o6.reshape(T, -1) * torch.sigmoid(gate.cpu().double())
+    o7 = (o7 / (o7.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(T, -1) * nw2.cpu().double() * torch.sigmoid(g.cpu().double()) * 1.3
+    for rows in (1, 10 ** 9):
+        monkeypatch.setattr(H, "DELTA_CHUNK_ROWS", rows)
+        monkeypatch.setattr(H, "GATED_CHUNK_ROWS", rows)
+        if small:
+            monkeypatch.setattr(H, "DELTA_FACTOR_BYTES", 4 * 4 * len(lens) * heads * (65 * d + 768))
+        s1, s2 = st.clone(), st2.clone()
+        got = H.gated_delta_scan(qkv, beta, dec, gate, nw, s1, md, heads, kv, d, dv, 1e-6, 1e-5, torch.float32)
+        out = torch.empty(T, hd, device=DEV)
+        H.delta_rule_scan(r, k, v, a, wz, g, w0, nw2, s2, md, heads, d, decay_scale=0.6065, key_eps=1e-6, norm_eps=1e-5, out_scale=1.3, out=out)
+        for x, y in ((got, o6), (s1, want), (out, o7), (s2, want2)):
+            close(x, y, 1e-5)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("T,E,top", [(33, 10, 3), (700, 8, 2), (5, 40, 9), (300, 3, 1), (4, 8, 2), (10, 6, 3), (1, 5, 5)])
 def test_routing_and_expert_products(ops, cdt, tol, T, E, top):
