@@ -462,6 +462,27 @@ def test_gemm_row_exact_small_m_bitwise(ops, ref, hd):
     assert rel_err(full[2].cpu(), ref.swiglu_up((x.float() * rs[:, None]).cpu(), wgu.float().cpu())) < 3e-3
 
 
+@pytest.mark.parametrize("N,K", [(256, 512), (1024, 4096), (8064, 256)])
+def test_gemm_col16_bitwise(ops, N, K):
+    """Few rows and N below a round of 32-column blocks, row-exact: 16-column blocks (a K shorter and longer than their ring)
+    give the 32-column mid blocks' bits, plain and with residual, for row counts about a 16-row tile; N = 8064 is the last
+    width that takes them."""
+    x, w, r = rnd(64, K, seed=161), rnd(N, K, scale=0.03, seed=162), rnd(64, N, seed=163)
+    rs, b = (torch.rand(64, device=DEV) + 0.5).float(), rnd(N, scale=0.5, seed=164)
+    for m in (1, 15, 16, 17, 32, 33, 64):
+        run = lambda: (ops.gemm(x[:m], w, bias=b), ops.gemm(x[:m], w, EPI_RESID, out=r[:m].clone(), resid=r[:m].clone(), rscale=rs[:m]))
+        with ops.row_exact():
+            got = run()
+            old = ops.k.fls_gemm_set_mid_bn(32)
+            try:
+                want = run()
+            finally:
+                ops.k.fls_gemm_set_mid_bn(old)
+        for a, c in zip(got, want):
+            assert torch.equal(a, c), m
+    assert rel_err(got[0], x.float() @ w.float().t() + b.float()) < 2e-3
+
+
 def test_row_ss_matches_residual_epilogue(ops):
     """fls_row_ss on a hidden state == the partial sums of squares the residual GEMM epilogue wrote
     for the same rows (v10 / v11 tiles and the mid-M kernel + ss_partials), bit for bit, and the
@@ -1124,3 +1145,13 @@ def test_argmax_rows_first_index(ops):
     torch.cuda.synchronize()
     assert np.array_equal(got.cpu().numpy(), np.argmax(x.cpu().numpy(), axis=-1))
     assert got[3].item() == 100 and got[5].item() == 0
+
+
+@pytest.mark.parametrize("V", [1, 7, 1000, 8193, 32000, 32003])
+def test_argmax_rows_widths(ops, V):
+    """Widths about a block's 8,192 values, rows aligned and not (a row stride of V or of V + 3): the first index of the maximum."""
+    for ld in (V, V + 3, (V + 7) // 8 * 8):
+        x = (torch.rand(5, ld, generator=torch.Generator().manual_seed(V)) * 3).round().div(8).half().to(DEV)[:, :V]
+        x[1] = 0
+        x[2, V - 1] = 2.0
+        assert np.array_equal(ops.argmax_rows(x).cpu().numpy(), np.argmax(x.cpu().numpy(), axis=-1)), ld
