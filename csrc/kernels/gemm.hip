@@ -17,6 +17,7 @@
 //     half-tile super-phases in flight, one counted vmcnt + raw s_barrier per
 //     two phases, LDS fragment reads and DMA interleaved into the MFMA stream.
 //     XCD-aware bijective block remap + grouped tile order (guide T1).
+//   * gemm_nt_col16 — 16-column blocks, K-tiles of 256, for M <= 64 and narrow outputs;
 //   * gemm_nt_mid — 64 x 128 x 64 tiles, 3-deep LDS-DMA ring, for M too small
 //     to fill 256 CUs with 256 x 256 tiles, and for odd K-tile counts (v10's
 //     body is unrolled over two K-tiles); 4 waves, or 8 (two per SIMD) for
@@ -331,6 +332,81 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   }
 }
 
+// 16-column blocks for M <= 64 and N below a round of 32-column mid blocks (the O / down projections of a 7B-sized
+// generation step: N = 4,096, 128 blocks of 32): what bounds those is the bytes in flight, one block's ring on half the
+// CUs, with 64 rows of A staged whatever M is.  Here every CU streams 16 weight rows, K-tiles of 256 (two rows a DMA
+// instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile; only ceil(M / 16) row
+// tiles of A are staged, wave w multiplies row tile w, the others only move data.  Same fragments, MFMA and K order as
+// the mid blocks: bitwise equal rows.  M = 16, K = 4,096 and 11,008 in turn (124 MB in both): 35.8 -> 16.6 us on average, 13 at
+// the rate of a large copy.
+namespace col16 {
+constexpr int KT = 256;
+constexpr int stage_bytes(int rt) { return 16 * (1 + rt) * KT * 2; }
+constexpr int stages(int rt) { return rt == 1 ? 8 : rt == 2 ? 6 : 3; }      // 128 / 144 / 120 KB
+}  // namespace col16
+
+template <int EPI, int RT>
+__global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ A, const half_t* __restrict__ W,
+                                                   half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
+                                                   int ldc, Epi ep) {
+  constexpr int KT = col16::KT, NST = col16::stages(RT), STAGE = col16::stage_bytes(RT);
+  constexpr int PER_WAVE = 8 * (1 + RT) / 4;           // 1 KB DMA groups (two rows) of a stage, per wave
+  extern __shared__ __attribute__((aligned(16))) char lds_c16[];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int fr = lane & 15, grp = lane >> 4;
+  const int n0 = blockIdx.x * 16, nk = K / KT;
+  const half_t* src[PER_WAVE];                         // groups 0 .. 7: W rows, then A rows
+#pragma unroll
+  for (int i = 0; i < PER_WAVE; ++i) {
+    const int g = wave + 4 * i, row = (g & 7) * 2 + (lane >> 5);          // row inside its tile of 16
+    const int kc = ((lane & 31) ^ row) * 8;
+    src[i] = g < 8 ? W + (size_t)(n0 + row) * ldw + kc : A + (size_t)min((g / 8 - 1) * 16 + row, M - 1) * lda + kc;
+  }
+  auto stage = [&](int s, int kt) {
+    char* base = lds_c16 + (s % NST) * STAGE;
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) glds16(src[i] + (size_t)kt * KT, base + (wave + 4 * i) * 1024);
+  };
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int d = 0; d < NST - 1; ++d) stage(d, min(d, nk - 1));
+  for (int kt = 0; kt < nk; ++kt) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * PER_WAVE) : "memory");
+    __builtin_amdgcn_s_barrier();                      // every wave's part of tile kt landed; tile kt - 1 has been read
+    asm volatile("" ::: "memory");
+    stage(kt + NST - 1, min(kt + NST - 1, nk - 1));    // (past the end: the last tile again, into a stage nobody reads)
+    if (wave < RT) {
+      const char* Ws = lds_c16 + (kt % NST) * STAGE + fr * (KT * 2);
+      const char* Xs = Ws + (1 + wave) * 16 * KT * 2;
+      half8 wf[KT / 32], xf[KT / 32];
+#pragma unroll
+      for (int ks = 0; ks < KT / 32; ++ks) {
+        const int c = ((ks * 4 + grp) ^ fr) << 4;
+        wf[ks] = *(const half8*)(Ws + c);
+        xf[ks] = *(const half8*)(Xs + c);
+      }
+#pragma unroll
+      for (int ks = 0; ks < KT / 32; ++ks) acc = mfma16x16x32(wf[ks], xf[ks], acc);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int m = wave * 16 + fr;
+  if (wave < RT && m < M) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc, ep);
+}
+
+template <int EPI, int RT>
+void launch_col16(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
+                  const Epi& ep, hipStream_t s) {
+  constexpr int lds = col16::stages(RT) * col16::stage_bytes(RT);
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)gemm_nt_col16<EPI, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr = true;
+  }
+  hipLaunchKernelGGL((gemm_nt_col16<EPI, RT>), dim3(N / 16), dim3(256), lds, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
+}
+
 int g_order = 0;             // 0: by shape, else a fixed signed group size (fls_gemm_set_order)
 int g_mid = 1;               // mid-M kernel on (fls_gemm_set_mid)
 int g_mid_bn = 0;            // mid-M block columns: 0 auto, 64 / 128 forced where valid (fls_gemm_set_mid_bn)
@@ -606,6 +682,16 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     const bool bn32 = bn32_epi && N % 32 == 0 && g_mid_waves != 4 &&
                       (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
     if constexpr (bn32_epi) {
+      // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
+      if (bn32 && g_mid_bn == 0 && N / 32 < 256 && K % col16::KT == 0) {
+        if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        FLS_CHECK_LAUNCH();
+        ss_partials(C, ldc, M, N, ep, s);
+        FLS_CHECK_LAUNCH();
+        return 0;
+      }
       if (bn32) {
         launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         FLS_CHECK_LAUNCH();
