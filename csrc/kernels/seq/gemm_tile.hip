@@ -26,6 +26,7 @@ struct Tile {
   long long w_gs, a_gs, c_gs;   // group g's operands (bytes); strided batch (grid y): its columns of C (elements)
   int a_mod;
   int tiles_m, tiles_n, order;
+  int ragged;               // columns or rows of C that four-column stores don't fit
 };
 
 // Virtual tile id -> (tile row, tile column): groups of `order` tiles of one dimension (order < 0: of N) walked along the
@@ -155,6 +156,23 @@ template <int MI, int NJ, int PU, bool ACC, int TC>
 __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
   const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
   const Epi& e = a.epi;
+  if constexpr (!ACC) {
+    if (a.ragged) {                                         // (plain products of few columns: a column at a time)
+#pragma unroll
+      for (int t = 0; t < NJ; ++t)
+#pragma unroll
+        for (int u = 0; u < MI; ++u)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const int n = nw + t * 16 + 4 * grp + x, m = mw + u * 16 + fr;
+            const size_t at = cbase + (size_t)m * a.ldc + n;
+            if (n >= a.N || m >= mend) continue;
+            if constexpr (TC == 1) reinterpret_cast<bf16_t*>(a.C)[at] = f_to_bf16(acc[u][t][x]);
+            else reinterpret_cast<float*>(a.C)[at] = acc[u][t][x];
+          }
+      return;
+    }
+  }
   if (e.kind == 0) {
 #pragma unroll
     for (int t = 0; t < NJ; ++t) {
@@ -581,8 +599,10 @@ static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int
 int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
                   const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
-  // whole K tiles; stores of four columns; 32-bit offsets within a tile
-  if (K * ew % 128 || N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16)) return 0;
+  // Whole K tiles; stores of four columns, or of one for a plain product of up to 128 columns (a router of 10 outputs
+  // over the rows of 9 prompts of 1,500 tokens: 76 us from the kernel for any shape, 15 here); 32-bit offsets within a tile.
+  const bool ragged = N % 4 || ldc % 4 || (uintptr_t)C % 16 || (offs == nullptr && c_gs % 4) || (epi.bias != nullptr && (uintptr_t)epi.bias % 16);
+  if (K * ew % 128 || (ragged && (epi.kind != 0 || epi.bias != nullptr || offs != nullptr || groups != 1 || N > 128))) return 0;
   if (((long long)lda * 256 + K) * ea >= (1LL << 31) || ((long long)ldw * 256 + K) * ew >= (1LL << 31)) return 0;
   if (offs == nullptr && groups > 65535) return 0;
   const bool gated = epi.kind >= EPI_GATE;
@@ -590,10 +610,10 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
   if (a_rows != nullptr && (long long)M * lda * ea >= (1LL << 31)) return 0;      // (there are at most as many rows of A as of the product)
   const int nk = K * ew / 128;
   const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, a_rows, offs, groups, w_gs * ew, a_gs * ea, c_gs,
-                  a_mod < 1 ? 1 : a_mod, 0, 0, 0};
+                  a_mod < 1 ? 1 : a_mod, 0, 0, 0, ragged};
   const bool by_rows = offs != nullptr;
   if (ta == 1) {
-    switch (pick_tile(TILES, 7, M, N, nk, groups, by_rows, gated)) {
+    switch (ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 7, M, N, nk, groups, by_rows, gated)) {
       case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
       case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
       case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);

@@ -234,6 +234,45 @@ def test_prompt_attention_tiles(ops, lens, pos0, d, dv, ps):
             close(o1, o2, 2e-2)
 
 
+# norms with rows in registers: one to eight steps of 1024 columns a group, the last one partly filled, the widest and the first beyond it
+# (8192, 8196), odd widths and strides that go to the general kernel, one weight for all columns; the residual update with the
+# next norm against the two in turn.  fp32 outputs against fp64: sums of up to 8196 squares in a tree, 1e-6; bf16 rounding 2^-8
+@pytest.mark.parametrize("n,groups", [(4, 3), (1020, 1), (1024, 2), (1028, 2), (2052, 1), (4096, 1), (4100, 2), (8192, 1), (8196, 1), (30, 2)])
+def test_norm_widths(ops, n, groups):
+    H, _ = ops
+    torch.manual_seed(n)
+    D = n * groups
+    norm = lambda x, w: (x.reshape(-1, groups, n) / (x.reshape(-1, groups, n).pow(2).mean(-1, keepdim=True) + 1e-6).sqrt()).reshape(-1, D) * w
+    w, w2 = torch.randn(D, device=DEV), torch.randn(D, device=DEV)
+    for pad in (0, 4, 3):
+        x, y = (torch.randn(5, D + pad, device=DEV)[:, :D] for _ in range(2))
+        x6, y6, w6, v6 = (t.cpu().double() for t in (x, y, w, w2))
+        close(H.group_rmsnorm(x, w, groups, 1e-6, torch.float32, w_offset=1.0), norm(x6, w6 + 1), 1e-6)
+        close(H.group_rmsnorm(x, w, groups, 1e-6, torch.bfloat16), norm(x6, w6), 2 ** -8)
+        close(H.group_rmsnorm(x, w[:1], groups, 1e-6, torch.float32), norm(x6, w6[:1]), 1e-6)
+        for cdt, tol in ((torch.float32, 1e-6), (torch.bfloat16, 2 ** -8)):
+            x1 = torch.empty(5, D + pad, device=DEV)[:, :D].copy_(x)
+            h = H.add_group_rmsnorm_next_(x1, y, w, w2, groups, 1e-6, cdt)
+            new = x6 + norm(y6, w6)
+            close(x1, new, 1e-6)
+            close(h, norm(new, v6), tol)
+
+
+# plain products of few columns that four-column stores don't fit: one column at a time from the tiles, rows about a tile's, all three
+# operand types; sums of 256 products against fp64
+@pytest.mark.parametrize("N", [1, 3, 10, 33, 62, 127])
+@pytest.mark.parametrize("ta,tw,tol", [(torch.bfloat16, torch.bfloat16, 1e-6), (torch.float32, torch.bfloat16, 5e-3), (torch.float32, torch.float32, 1e-6)])
+def test_matmul_few_columns(ops, N, ta, tw, tol):
+    H, _ = ops
+    torch.manual_seed(N)
+    w = torch.randn(N, 256, device=DEV).to(tw)
+    for M in (33, 64, 129, 1000):
+        a = torch.randn(M, 256, device=DEV).to(ta)
+        want = a.cpu().double() @ w.cpu().double().t()
+        close(H.matmul_nt(a, w), want, tol)
+        close(H.matmul_nt(a, w, out_dtype=torch.bfloat16), want, max(tol, 2 ** -8))
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_conv_and_scans_carry_state(ops, cdt, tol):
     H, R = ops
