@@ -30,6 +30,9 @@ int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, 
 // weights stored around zero).  w_one != 0: w is one number for all columns.
 int fls_seq_group_rmsnorm(const float* x, int ldx, const int* idx, const float* w, void* y, int ty, int ldy,
                           int rows, int D, int groups, float eps, int add, float woff, int w_one, fls_stream_t s);
+// x += norm(y; w + woff), then h = norm(x; w2 + woff2) of the new x, both per group of D / groups columns; h of type th
+int fls_seq_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const float* w, float woff, const float* w2, float woff2,
+                                   void* h, int th, int ldh, int rows, int D, int groups, float eps, fls_stream_t s);
 // new = (keep ? x : 0) + coef (rms(a) wa + rms(b) wb) + f (all fp32 rows; a and b nullable together, f nullable), x <- new;
 // h != null: h = rms(new) hw as type th, hw a vector or (hw_one) one number
 int fls_seq_residual_branches(float* x, int ldx, int keep, const float* a, int lda, const float* wa, const float* b,

@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 15   # csrc/include/fls_seq.h
+SEQ_ABI = 16   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -141,6 +141,7 @@ def _load_seq():
         raise RuntimeError(f"{_SEQ} is a stale build; rebuild with python -m flexible_llm_sharding_amd._native.build")
     p, i, f, ll = c_void_p, c_int, c_float, ctypes.c_longlong
     _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p)
+    _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_group_rmsnorm", i, p, i, p, p, p, i, i, i, i, i, f, i, f, i, p)
     _bind(lib, "fls_seq_residual_branches", i, p, i, i, p, i, p, p, i, p, f, p, i, p, i, i, p, i, i, i, f, p)
     _bind(lib, "fls_seq_block_means", i, p, i, p, i, i, p, p, i, i, i, i, p, i, i, i, p, i, p, i, p, i, p)

@@ -217,9 +217,10 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
     ng, eps = cfg.norm_groups, cfg.norm_eps
     h = ops.group_rmsnorm(x, W["norm1"], ng, eps, out_dtype=cdt)
     y = {"attention": _attention, "rglru": _rglru, "mamba2": _mamba2}[L.type](ctx, L.mixer, W, h, meta, name)
-    ops.add_group_rmsnorm_(x, y, W["norm1b"], ng, eps)
-    if L.mlp is not None:
-        h = ops.group_rmsnorm(x, W["norm2"], ng, eps, out_dtype=cdt)
+    if L.mlp is None:
+        ops.add_group_rmsnorm_(x, y, W["norm1b"], ng, eps)
+    else:
+        h = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], W["norm2"], ng, eps, out_dtype=cdt)
         if L.mlp["kind"] == "dense":
             # (the activation and the rounding for the down projection happen in the up projection's epilogue)
             y = ops.matmul_nt(ops.matmul_nt(h, W["wup"], xielu=W["act"], out_dtype=cdt), W["wdown"])

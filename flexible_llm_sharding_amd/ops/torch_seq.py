@@ -60,6 +60,11 @@ class TorchSeqOps:
         p = p * torch.rsqrt(p.pow(2).mean(-1, keepdim=True) + eps)
         return (p.reshape(T, D) * (w.float() + w_offset)).to(out_dtype)
 
+    def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype):
+        """``add_group_rmsnorm_`` and the norm of the new rows by ``w2``, which it returns."""
+        self.add_group_rmsnorm_(x, y, w, groups, eps)
+        return self.group_rmsnorm(x, w2, groups, eps, out_dtype)
+
     def add_group_rmsnorm_(self, x, y, w, groups, eps, w_offset=0.0):
         x.add_(self.group_rmsnorm(y, w, groups, eps, torch.float32, w_offset=w_offset))
         return x
