@@ -30,6 +30,10 @@ int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, 
 // weights stored around zero).  w_one != 0: w is one number for all columns.
 int fls_seq_group_rmsnorm(const float* x, int ldx, const int* idx, const float* w, void* y, int ty, int ldy,
                           int rows, int D, int groups, float eps, int add, float woff, int w_one, fls_stream_t s);
+// x[r] += norm(sum_k mw[r, k] y[dest[r, k]]; w + woff), k < top, per group of D / groups columns; SEQ_NOT_SERVED: groups or alignments
+// that only fls_seq_moe_sum and fls_seq_group_rmsnorm take
+int fls_seq_moe_sum_add_group_rmsnorm(float* x, int ldx, const float* y, int ldy, const int* dest, const float* mw, int top, const float* w,
+                                      float woff, int rows, int D, int groups, float eps, fls_stream_t s);
 // x += norm(y; w + woff), then h = norm(x; w2 + woff2) of the new x, both per group of D / groups columns; h of type th
 int fls_seq_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const float* w, float woff, const float* w2, float woff2,
                                    void* h, int th, int ldh, int rows, int D, int groups, float eps, fls_stream_t s);
@@ -176,9 +180,10 @@ int fls_seq_ssd_scan_chunked(const float* xbc, int ldx, const float* z, int ldz,
                              const int* pos0, const int* slot, int B, int max_rows, int nh, int P, int N, int G, float* scratch, fls_stream_t s);
 // softmax scores over E experts; the top largest of (score + corr) chosen (ties: the lower expert);
 // ids[T, top], w[T, top] = bare scores; hist[E] += number of entries per expert (hist zeroed by the caller).
+// Up to FLS_SEQ_ROUTE_FUSED tokens, with corr: offs, dest and rows are filled in the same launch (no scan, no place; hist unused).
 // corr == null: the top largest logits are chosen and w = the softmax over the chosen logits only
 int fls_seq_moe_route(const float* logits, int ldl, const float* corr, int T, int E, int top, int* ids, float* w,
-                      int* hist, fls_stream_t s);
+                      int* hist, int* offs, int* dest, int* rows, fls_stream_t s);
 // scores sigmoid(logit); `groups` equal groups of neighbouring experts, each worth the sum of its two largest scores;
 // only experts of the `keep` best groups compete (groups <= 1: all); the top largest scores are chosen (ties: the
 // lower expert), w = score / (sum of the chosen + 1e-20) * scale; hist as above.  groups <= 64

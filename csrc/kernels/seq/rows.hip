@@ -30,27 +30,45 @@ __global__ __launch_bounds__(256) void group_rmsnorm_kernel(const float* __restr
 // reduction.  MODE 0: y = norm(x); 1: y += norm(x); 2: y += norm(x), then h = norm(y; w2) of the new row: a sublayer's
 // post-norm, the residual update and the next sublayer's norm in one pass.  Bound by its bytes from some hundred rows on
 // and by a launch and two memory latencies below.  16384 rows of 4096 in two groups, a column a thread before: norm 146 -> 82 us,
-// residual update 199 -> 140, update and next norm in turn 345, here 182.
-template <typename TO, int MODE, int NV>
+// residual update 199 -> 140, update and next norm in turn 345, here 182.  SUM: x is a mixture's rows, sorted by expert; row r of the sum is
+// sum_k mw[r, k] x[idx[r, k]], k < top, made on the way in (moe_sum_kernel's order).
+template <typename TO, int MODE, int NV, bool SUM = false>
 __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, const int* __restrict__ idx,
                                                                 const float* __restrict__ w, void* __restrict__ y, int ldy, int n,
                                                                 float eps, float woff, int w_one, const float* __restrict__ w2,
-                                                                TO* __restrict__ h, int ldh, float woff2) {
+                                                                TO* __restrict__ h, int ldh, float woff2,
+                                                                const float* __restrict__ mw, int top) {
   __shared__ float red[8];
   const int r = blockIdx.x, g = blockIdx.y;
-  const float* xr = x + (size_t)(idx != nullptr ? idx[r] : r) * ldx + (size_t)g * n;
+  const float* xr = x + (size_t)(!SUM && idx != nullptr ? idx[r] : r) * ldx + (size_t)g * n;
   float* yr = reinterpret_cast<float*>(y) + (size_t)r * ldy + (size_t)g * n;
   const float* wg = w + (size_t)g * n;
   float4 v[NV], u[NV], a[NV], b[NV];
   const float one = w_one ? w[0] : 0.f;
   float ss = 0.f;
+  if constexpr (SUM) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int k = 0; k < top; ++k) {
+      const float* row = x + (size_t)idx[(size_t)r * top + k] * ldx + (size_t)g * n;
+      const float f = mw[(size_t)r * top + k];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int c = (threadIdx.x + 256 * i) * 4;
+        if (c >= n) continue;
+        const float4 e = *reinterpret_cast<const float4*>(row + c);
+        v[i].x += f * e.x; v[i].y += f * e.y; v[i].z += f * e.z; v[i].w += f * e.w;
+      }
+    }
+  }
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + 256 * i) * 4;
-    v[i] = u[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    u[i] = b[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (!SUM) v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
     a[i] = make_float4(one, one, one, one);
     if (c < n) {
-      v[i] = *reinterpret_cast<const float4*>(xr + c);
+      if constexpr (!SUM) v[i] = *reinterpret_cast<const float4*>(xr + c);
       if constexpr (MODE != 0) u[i] = *reinterpret_cast<const float4*>(yr + c);
       if (!w_one) a[i] = *reinterpret_cast<const float4*>(wg + c);
       if constexpr (MODE == 2) b[i] = *reinterpret_cast<const float4*>(w2 + (size_t)g * n + c);
@@ -89,15 +107,16 @@ __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __r
 }
 
 // rows of up to 8,192 columns a group with 16-byte alignment throughout (8 bytes for bf16 outputs); false: the kernel above serves
-template <typename TO, int MODE>
+template <typename TO, int MODE, bool SUM = false>
 static bool group_rmsnorm_vec(const float* x, int ldx, const int* idx, const float* w, void* y, int ldy, int rows, int D, int groups,
-                              float eps, float woff, int w_one, const float* w2, TO* h, int ldh, float woff2, hipStream_t st) {
+                              float eps, float woff, int w_one, const float* w2, TO* h, int ldh, float woff2, hipStream_t st,
+                              const float* mw = nullptr, int top = 0) {
   const int n = D / groups, ya = MODE == 0 ? 4 * (int)sizeof(TO) : 16;
   if (n % 4 || n > 8192 || ldx % 4 || ldy % 4 || ldh % 4 || (uintptr_t)x % 16 || (uintptr_t)y % ya || (!w_one && (uintptr_t)w % 16) ||
       (uintptr_t)w2 % 16 || (uintptr_t)h % (4 * sizeof(TO)))
     return false;
   dim3 grid(rows, groups);
-#define GN_VEC(NV) hipLaunchKernelGGL((group_rmsnorm_vec_kernel<TO, MODE, NV>), grid, dim3(256), 0, st, x, ldx, idx, w, y, ldy, n, eps, woff, w_one, w2, h, ldh, woff2)
+#define GN_VEC(NV) hipLaunchKernelGGL((group_rmsnorm_vec_kernel<TO, MODE, NV, SUM>), grid, dim3(256), 0, st, x, ldx, idx, w, y, ldy, n, eps, woff, w_one, w2, h, ldh, woff2, mw, top)
   if (n <= 1024) GN_VEC(1);
   else if (n <= 2048) GN_VEC(2);
   else if (n <= 4096) GN_VEC(4);
@@ -121,6 +140,16 @@ extern "C" int fls_seq_group_rmsnorm(const float* x, int ldx, const int* idx, co
   if (add) hipLaunchKernelGGL((group_rmsnorm_kernel<float, 1>), grid, dim3(256), 0, st, x, ldx, idx, w, (float*)y, ldy, D, groups, eps, woff, w_one);
   else if (ty == 1) hipLaunchKernelGGL((group_rmsnorm_kernel<bf16_t, 0>), grid, dim3(256), 0, st, x, ldx, idx, w, (bf16_t*)y, ldy, D, groups, eps, woff, w_one);
   else hipLaunchKernelGGL((group_rmsnorm_kernel<float, 0>), grid, dim3(256), 0, st, x, ldx, idx, w, (float*)y, ldy, D, groups, eps, woff, w_one);
+  SEQ_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int fls_seq_moe_sum_add_group_rmsnorm(float* x, int ldx, const float* y, int ldy, const int* dest, const float* mw, int top,
+                                                 const float* w, float woff, int rows, int D, int groups, float eps, fls_stream_t s) {
+  if (rows <= 0) return 0;
+  if (groups < 1 || D % groups || top < 1) return -1;
+  if (!group_rmsnorm_vec<float, 1, true>(y, ldy, dest, w, x, ldx, rows, D, groups, eps, woff, 0, nullptr, nullptr, 0, 0.f, (hipStream_t)s, mw, top))
+    return SEQ_NOT_SERVED;
   SEQ_LAUNCH_CHECK();
   return 0;
 }
@@ -574,61 +603,36 @@ extern "C" int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col,
 }
 
 // ------------------------------------------------------------------------ mixture of experts
-// one thread per token: softmax statistics, then `top` passes each taking the best unchosen expert.
-// corr == null: the `top` largest logits are chosen (ties: the lower expert) and weighted by the softmax
-// over the chosen logits only
+// one thread per token: the `top` largest logits are chosen (ties: the lower expert) and weighted by the softmax over the chosen
+// logits only
 #define MOE_MAX_TOP 16
-__global__ void moe_route_kernel(const float* __restrict__ logits, int ldl, const float* __restrict__ corr, int T, int E, int top,
-                                 int* __restrict__ ids, float* __restrict__ w, int* __restrict__ hist) {
+__global__ void moe_route_kernel(const float* __restrict__ logits, int ldl, int T, int E, int top, int* __restrict__ ids,
+                                 float* __restrict__ w) {
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= T) return;
   const float* l = logits + (size_t)t * ldl;
-  if (corr == nullptr) {
-    int chosen[MOE_MAX_TOP];
-    float val[MOE_MAX_TOP];
-    for (int k = 0; k < top; ++k) {
-      float best = -INFINITY;
-      int be = -1;
-      for (int e = 0; e < E; ++e) {
-        bool used = false;
-        for (int j = 0; j < k; ++j) used |= (chosen[j] == e);
-        if (used) continue;
-        const float c = l[e];
-        if (be < 0 || c > best) { best = c; be = e; }
-      }
-      chosen[k] = be;
-      val[k] = best;
-    }
-    const float mx = val[0];                          // (the first choice is the largest)
-    float sum = 0.f;
-    for (int k = 0; k < top; ++k) { val[k] = expf(val[k] - mx); sum += val[k]; }
-    const float inv = 1.f / sum;
-    for (int k = 0; k < top; ++k) {
-      ids[(size_t)t * top + k] = chosen[k];
-      w[(size_t)t * top + k] = val[k] * inv;
-    }
-    return;
-  }
-  float mx = -INFINITY;
-  for (int e = 0; e < E; ++e) mx = fmaxf(mx, l[e]);
-  float sum = 0.f;
-  for (int e = 0; e < E; ++e) sum += expf(l[e] - mx);
-  const float inv = 1.f / sum;
   int chosen[MOE_MAX_TOP];
+  float val[MOE_MAX_TOP];
   for (int k = 0; k < top; ++k) {
-    float best = -INFINITY, bs = 0.f;
-    int be = 0;
+    float best = -INFINITY;
+    int be = -1;
     for (int e = 0; e < E; ++e) {
       bool used = false;
       for (int j = 0; j < k; ++j) used |= (chosen[j] == e);
       if (used) continue;
-      const float sc = expf(l[e] - mx) * inv;
-      const float c = sc + corr[e];
-      if (c > best) { best = c; be = e; bs = sc; }
+      const float c = l[e];
+      if (be < 0 || c > best) { best = c; be = e; }
     }
     chosen[k] = be;
-    ids[(size_t)t * top + k] = be;
-    w[(size_t)t * top + k] = bs;
+    val[k] = best;
+  }
+  const float mx = val[0];                          // (the first choice is the largest)
+  float sum = 0.f;
+  for (int k = 0; k < top; ++k) { val[k] = expf(val[k] - mx); sum += val[k]; }
+  const float inv = 1.f / sum;
+  for (int k = 0; k < top; ++k) {
+    ids[(size_t)t * top + k] = chosen[k];
+    w[(size_t)t * top + k] = val[k] * inv;
   }
 }
 
@@ -701,12 +705,13 @@ __global__ void moe_route_grouped_kernel(const float* __restrict__ logits, int l
 
 // Softmax scores with a correction for the choice, a wave per token: lane l holds experts l, l + 64, ...  Every choice is a
 // maximum over the wave (ties: the lower index).  FUSED (one block, few tokens): afterwards the block counts the entries
-// per expert in LDS, scans the counts and gives every entry its row, so that a decode step routes in one launch.
+// per expert in LDS, scans the counts and gives every entry its row, so that a decode step routes in one launch (8 rows:
+// 4.5 us, 22 in five launches).  bare: the weights are the scores as they are.
 #define RSG_FUSED_WAVES 16
 template <int NE, int NW, bool FUSED>
 __global__ __launch_bounds__(64 * NW) void moe_route_softmax_grouped_kernel(const float* __restrict__ logits, int ldl,
                                                                             const float* __restrict__ corr, int T, int E, int top,
-                                                                            int groups, int keep, float scale,
+                                                                            int groups, int keep, float scale, int bare,
                                                                             int* __restrict__ ids, float* __restrict__ w,
                                                                             int* __restrict__ offs, int* __restrict__ dest,
                                                                             int* __restrict__ rows) {
@@ -784,7 +789,7 @@ __global__ __launch_bounds__(64 * NW) void moe_route_softmax_grouped_kernel(cons
     }
     if (lane < top) {
       ids[(size_t)t * top + lane] = my_e;
-      w[(size_t)t * top + lane] = my_s * (scale / (total + 1e-20f));
+      w[(size_t)t * top + lane] = bare ? my_s : my_s * (scale / (total + 1e-20f));
       if constexpr (FUSED) atomicAdd(&cnt[my_e], 1);
     }
   }
@@ -813,20 +818,15 @@ __global__ __launch_bounds__(64 * NW) void moe_route_softmax_grouped_kernel(cons
   }
 }
 
-extern "C" int fls_seq_moe_route_softmax_grouped(const float* logits, int ldl, const float* corr, int T, int E, int top, int groups,
-                                                 int keep, float scale, int* ids, float* w, int* hist, int* offs, int* dest, int* rows,
-                                                 fls_stream_t s) {
-  if (T <= 0) return 0;
-  if (top < 1 || top > MOE_MAX_TOP || top > E || E > MOE_MAX_E || groups < 0 || groups > MOE_MAX_GROUPS) return -1;
-  if (groups > 1 && (E % groups || keep < 1 || keep > groups || keep * (E / groups) < top)) return -1;
-  hipStream_t st = (hipStream_t)s;
+static int moe_route_softmax(const float* logits, int ldl, const float* corr, int T, int E, int top, int groups, int keep, float scale,
+                             int bare, int* ids, float* w, int* hist, int* offs, int* dest, int* rows, hipStream_t st) {
   const bool fused = T <= FLS_SEQ_ROUTE_FUSED;
 #define RSG(NE)                                                                                                                     \
   do {                                                                                                                              \
     if (fused) hipLaunchKernelGGL((moe_route_softmax_grouped_kernel<NE, (NE > 4 ? 8 : RSG_FUSED_WAVES), true>), dim3(1),            \
-                                  dim3(64 * (NE > 4 ? 8 : RSG_FUSED_WAVES)), 0, st, logits, ldl, corr, T, E, top, groups, keep, scale, ids, w, offs, dest, rows); \
+                                  dim3(64 * (NE > 4 ? 8 : RSG_FUSED_WAVES)), 0, st, logits, ldl, corr, T, E, top, groups, keep, scale, bare, ids, w, offs, dest, rows); \
     else hipLaunchKernelGGL((moe_route_softmax_grouped_kernel<NE, 4, false>), dim3((T + 3) / 4), dim3(256), 0, st, logits, ldl, corr, T, E, top, groups,          \
-                            keep, scale, ids, w, offs, dest, rows);                                                                 \
+                            keep, scale, bare, ids, w, offs, dest, rows);                                                           \
   } while (0)
   if (E <= 64) RSG(1);
   else if (E <= 128) RSG(2);
@@ -839,6 +839,15 @@ extern "C" int fls_seq_moe_route_softmax_grouped(const float* logits, int ldl, c
     SEQ_LAUNCH_CHECK();
   }
   return 0;
+}
+
+extern "C" int fls_seq_moe_route_softmax_grouped(const float* logits, int ldl, const float* corr, int T, int E, int top, int groups,
+                                                 int keep, float scale, int* ids, float* w, int* hist, int* offs, int* dest, int* rows,
+                                                 fls_stream_t s) {
+  if (T <= 0) return 0;
+  if (top < 1 || top > MOE_MAX_TOP || top > E || E > MOE_MAX_E || groups < 0 || groups > MOE_MAX_GROUPS) return -1;
+  if (groups > 1 && (E % groups || keep < 1 || keep > groups || keep * (E / groups) < top)) return -1;
+  return moe_route_softmax(logits, ldl, corr, T, E, top, groups, keep, scale, 0, ids, w, hist, offs, dest, rows, (hipStream_t)s);
 }
 
 extern "C" int fls_seq_moe_route_grouped(const float* logits, int ldl, int T, int E, int top, int groups, int keep, float scale,
@@ -855,10 +864,11 @@ extern "C" int fls_seq_moe_route_grouped(const float* logits, int ldl, int T, in
 }
 
 extern "C" int fls_seq_moe_route(const float* logits, int ldl, const float* corr, int T, int E, int top, int* ids, float* w,
-                                 int* hist, fls_stream_t s) {
+                                 int* hist, int* offs, int* dest, int* rows, fls_stream_t s) {
   if (T <= 0) return 0;
   if (top < 1 || top > MOE_MAX_TOP || top > E || E > MOE_MAX_E) return -1;
-  hipLaunchKernelGGL(moe_route_kernel, dim3((T + 127) / 128), dim3(128), 0, (hipStream_t)s, logits, ldl, corr, T, E, top, ids, w, hist);
+  if (corr != nullptr) return moe_route_softmax(logits, ldl, corr, T, E, top, 0, 0, 1.f, 1, ids, w, hist, offs, dest, rows, (hipStream_t)s);
+  hipLaunchKernelGGL(moe_route_kernel, dim3((T + 127) / 128), dim3(128), 0, (hipStream_t)s, logits, ldl, T, E, top, ids, w);
   SEQ_LAUNCH_CHECK();
   hipLaunchKernelGGL(moe_hist_kernel, dim3((T * top + 4095) / 4096), dim3(256), 0, (hipStream_t)s, ids, T * top, E, hist);
   SEQ_LAUNCH_CHECK();
@@ -961,4 +971,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 16; }
+extern "C" int fls_seq_version(void) { return 17; }

@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 16   # csrc/include/fls_seq.h
+SEQ_ABI = 17   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -141,6 +141,7 @@ def _load_seq():
         raise RuntimeError(f"{_SEQ} is a stale build; rebuild with python -m flexible_llm_sharding_amd._native.build")
     p, i, f, ll = c_void_p, c_int, c_float, ctypes.c_longlong
     _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p)
+    _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm", i, p, i, p, i, p, p, i, p, f, i, i, i, f, p)
     _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_group_rmsnorm", i, p, i, p, p, p, i, i, i, i, i, f, i, f, i, p)
     _bind(lib, "fls_seq_residual_branches", i, p, i, i, p, i, p, p, i, p, f, p, i, p, i, i, p, i, i, i, f, p)
@@ -171,7 +172,7 @@ def _load_seq():
     _bind(lib, "fls_seq_rglru_scan_tiled", i, p, i, p, i, p, p, i, p, p, i, i, p, i, p, p, p, p, i, i, f, p)
     _bind(lib, "fls_seq_ssd_scan", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, p)
     _bind(lib, "fls_seq_ssd_scan_chunked", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, p, p)
-    _bind(lib, "fls_seq_moe_route", i, p, i, p, i, i, i, p, p, p, p)
+    _bind(lib, "fls_seq_moe_route", i, p, i, p, i, i, i, p, p, p, p, p, p, p)
     _bind(lib, "fls_seq_moe_scan", i, p, i, p, p, p)
     _bind(lib, "fls_seq_moe_place", i, p, i, i, p, p, p, p)
     _bind(lib, "fls_seq_moe_sum", i, p, i, p, p, p, i, i, i, i, p)

@@ -207,8 +207,7 @@ def _moe(ctx, mlp: dict, W, h):
     logits = ops.matmul_nt(h, W["wrouter"])                               # fp32 accumulation of the rows
     route = ops.moe_route_corrected(logits, W["corr"], top)
     a = ops.gated_matmul_nt(h, W["wgu"], cdt, offs=route.offs, rows=route.rows)     # rows sorted by expert, silu(gate) up
-    yo = ops.grouped_matmul_nt(a, W["wdown"], route.offs)
-    return ops.moe_weighted_sum(yo, route)                                # fp32 [T, D]
+    return ops.grouped_matmul_nt(a, W["wdown"], route.offs), route        # fp32 rows by expert
 
 
 def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
@@ -225,7 +224,8 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
             # (the activation and the rounding for the down projection happen in the up projection's epilogue)
             y = ops.matmul_nt(ops.matmul_nt(h, W["wup"], xielu=W["act"], out_dtype=cdt), W["wdown"])
         else:
-            y = _moe(ctx, L.mlp, W, h)
+            y, route = _moe(ctx, L.mlp, W, h)
+            return ops.add_group_rmsnorm_moe_(x, y, route, W["norm2b"], ng, eps)
         ops.add_group_rmsnorm_(x, y, W["norm2b"], ng, eps)
     return x
 

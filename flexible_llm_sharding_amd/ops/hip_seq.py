@@ -991,17 +991,34 @@ class HipSeqOps:
         dev = logits.device
         ids = torch.empty(T, top, dtype=torch.int32, device=dev)
         w = torch.empty(T, top, dtype=torch.float32, device=dev)
-        ints = torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)          # hist | cursor | offs
-        hist, cursor, offs = ints[:E], ints[E:2 * E], ints[2 * E:]
+        fused = corr is not None and T <= self.ROUTE_FUSED
+        ints = torch.empty(E + 1, dtype=torch.int32, device=dev) if fused else torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)
+        offs, hist, cursor = ints[:E + 1], ints[E + 1:2 * E + 1], ints[2 * E + 1:]
         dest = torch.empty(T, top, dtype=torch.int32, device=dev)
         rows = torch.empty(T * top, dtype=torch.int32, device=dev)
         s = _stream()
         _chk(self.k.fls_seq_moe_route(logits.data_ptr(), logits.stride(0), corr.data_ptr() if corr is not None else None, T, E, top, ids.data_ptr(),
-                                      w.data_ptr(), hist.data_ptr(), s), "fls_seq_moe_route")
+                                      w.data_ptr(), hist.data_ptr(), offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s), "fls_seq_moe_route")
+        if fused:
+            return SeqRoute(ids, w, offs, rows, dest, top)
         _chk(self.k.fls_seq_moe_scan(hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), s), "fls_seq_moe_scan")
         _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, cursor.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
              "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
+
+    def add_group_rmsnorm_moe_(self, x, y, route, w, groups, eps):
+        _rows(x, "x", torch.float32)
+        _rows(y, "y", torch.float32)
+        T, top = route.dest.shape
+        if x.shape != (T, y.shape[1]):
+            raise ValueError("add_group_rmsnorm_moe_: shapes differ")
+        _vec(w, "w", x.shape[1])
+        rc = self.k.fls_seq_moe_sum_add_group_rmsnorm(x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), route.dest.data_ptr(),
+                                                      route.w.data_ptr(), top, w.data_ptr(), 0.0, T, x.shape[1], groups, float(eps), _stream())
+        if rc == self.NOT_SERVED:
+            return self.add_group_rmsnorm_(x, self.moe_weighted_sum(y, route), w, groups, eps)
+        _chk(rc, "fls_seq_moe_sum_add_group_rmsnorm")
+        return x
 
     def moe_weighted_sum(self, y, route):
         _rows(y, "y", torch.float32)

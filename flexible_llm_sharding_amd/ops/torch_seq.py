@@ -60,6 +60,10 @@ class TorchSeqOps:
         p = p * torch.rsqrt(p.pow(2).mean(-1, keepdim=True) + eps)
         return (p.reshape(T, D) * (w.float() + w_offset)).to(out_dtype)
 
+    def add_group_rmsnorm_moe_(self, x, y, route, w, groups, eps):
+        """``add_group_rmsnorm_`` of a mixture's output: the weighted sum of its rows ``y``, which lie sorted by expert."""
+        return self.add_group_rmsnorm_(x, self.moe_weighted_sum(y, route), w, groups, eps)
+
     def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype):
         """``add_group_rmsnorm_`` and the norm of the new rows by ``w2``, which it returns."""
         self.add_group_rmsnorm_(x, y, w, groups, eps)

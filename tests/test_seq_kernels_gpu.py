@@ -258,6 +258,20 @@ def test_norm_widths(ops, n, groups):
             close(h, norm(new, v6), tol)
 
 
+# the residual update of a mixture: rows summed on the way into the norm, one to many choices, widths as above and one for the general
+# kernels, tokens on both sides of the one-launch routing; fp32 sums in the oracle's order
+@pytest.mark.parametrize("T", [3, 70])
+@pytest.mark.parametrize("D,groups,E,top", [(24, 3, 5, 1), (2048, 2, 20, 4), (4100, 1, 40, 16), (30, 2, 6, 3)])
+def test_mixture_into_norm(ops, T, D, groups, E, top):
+    H, R = ops
+    torch.manual_seed(D + T)
+    route = H.moe_route_corrected(torch.randn(T, E, device=DEV), torch.randn(E, device=DEV) * 0.1, top)
+    y, w, x = torch.randn(T * top, D, device=DEV), torch.randn(D, device=DEV), torch.randn(T, D, device=DEV)
+    y6 = (y.cpu().double()[route.dest.cpu().long()] * route.w.cpu().double()[:, :, None]).sum(1).reshape(T, groups, -1)
+    want = x.cpu().double() + (y6 / (y6.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt()).reshape(T, D) * w.cpu().double()
+    close(H.add_group_rmsnorm_moe_(x, y, route, w, groups, 1e-6), want, 1e-6)
+
+
 # plain products of few columns that four-column stores don't fit: one column at a time from the tiles, rows about a tile's, all three
 # operand types; sums of 256 products against fp64
 @pytest.mark.parametrize("N", [1, 3, 10, 33, 62, 127])
