@@ -272,6 +272,41 @@ def test_mixture_into_norm(ops, T, D, groups, E, top):
     close(H.add_group_rmsnorm_moe_(x, y, route, w, groups, 1e-6), want, 1e-6)
 
 
+# activations with bf16 results from the tiles' epilogues, element by element over the bf16 range (tiny, about the forms' seam at -1/2, large,
+# infinite): within a rounding of the fp64 value (2^-8 relative; a sigmoid
+# below 2^-126 may be flushed, and a result)
+@pytest.mark.parametrize("kind", ["xielu", "silu", "gelu_tanh", "clamped"])
+def test_epilogue_bf16_values(ops, kind):
+    H, _ = ops
+    g = torch.Generator().manual_seed(5)
+    z = torch.cat([torch.linspace(-1, 1, 300), torch.logspace(-30, 2, 300, base=2.0) * torch.where(torch.rand(300, generator=g) < 0.5, -1.0, 1.0),
+                   torch.linspace(-90, 90, 150), torch.tensor([0.0, -0.0, -0.5, 0.5, 3e4, -3e4])]).bfloat16()
+    M, N, K = z.numel(), 256, 64
+    a = torch.zeros(M, K, dtype=torch.bfloat16)
+    a[:, 0], a[:, 1] = z, z.flip(0)
+    z6, u6 = z.double(), z.flip(0).double()
+    if kind == "xielu":
+        act = torch.tensor([0.3, -0.2])
+        w = torch.zeros(N, K)
+        w[:, 0] = 1
+        got = H.matmul_nt(a.to(DEV), w.bfloat16().to(DEV), xielu=act.to(DEV), out_dtype=torch.bfloat16)
+        p, q = torch.nn.functional.softplus(act.double())
+        want = torch.where(z6 > 0, p * z6 * z6, (0.5 + q) * (torch.expm1(z6) - z6)) + 0.5 * z6
+    else:
+        w = torch.zeros(2 * N, K)
+        w[:N, 0], w[N:, 1] = 1, 1
+        got = H.gated_matmul_nt(a.to(DEV), w.bfloat16().to(DEV), torch.bfloat16, act=kind, limit=7.0, alpha=1.702)
+        if kind == "silu":
+            want = z6 * torch.sigmoid(z6) * u6
+        elif kind == "gelu_tanh":
+            want = z6 * torch.sigmoid(2 * (2 / torch.pi) ** 0.5 * (z6 + 0.044715 * z6 ** 3)) * u6
+        else:
+            zc = z6.clamp(max=7.0)
+            want = zc * torch.sigmoid(1.702 * zc) * (u6.clamp(-7.0, 7.0) + 1)
+    err = (got.cpu().double() - want[:, None]).abs()
+    assert bool((err <= want[:, None].abs() * 2 ** -8 + (1 + (z6 * (u6.abs() + 1)).abs())[:, None] * 2.0 ** -126).all())
+
+
 # plain products of few columns that four-column stores don't fit: one column at a time from the tiles, rows about a tile's, all three
 # operand types; sums of 256 products against fp64
 @pytest.mark.parametrize("N", [1, 3, 10, 33, 62, 127])
