@@ -243,21 +243,26 @@ __device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], si
   else finish_as<MI, NJ, PU, ACC, 0>(a, acc, cbase, mw, nw, mend, lds);
 }
 
-// ------------------------------------------------------------------------------------ 256 x 256
-// Four waves, one per SIMD, 128 x 128 outputs each: all 256 accumulation registers of a wave.  A fragment read from LDS
-// feeds 8 MFMAs.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
+// ------------------------------------------------------------------------------------ 256, 192 and 128 x 256
+// Four waves, one per SIMD, 32 HX x 128 outputs each.  HX = 4: 128 x 128, all 256 accumulation registers of a wave, a fragment
+// read from LDS feeds 8 MFMAs.  HX = 3, 2: 192 and 128 rows, for row counts that leave the chip idle in the last (or only) round of
+// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 2048 two thirds of
+// the 192-row tile's time.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
 // accumulation register the compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between
-// them; reads run one phase of 32 MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
+// them; reads run one phase of 8 HX MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
 namespace t256 {
-constexpr int TM = 256, TN = 256, KT = 128 /* bytes of a K tile's row */, STG = 65536, WIMG = 32768, LDS_BYTES = 2 * STG;
+constexpr int TN = 256, KT = 128 /* bytes of a K tile's row */;
+constexpr int lds_bytes(int hx) { return 2 * (64 * hx + TN) * KT; }
 }
 
 __device__ __forceinline__ void mfma_in_place(floatx4& c, const bf16x8& a, const bf16x8& b) {
   asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
 }
 
-__global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
+template <int HX>
+__device__ __forceinline__ void tile_256(const Tile& a) {
   using namespace t256;
+  constexpr int TM = 64 * HX, WIMG = TM * KT, STG = WIMG + TN * KT;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const char *A, *W;
   size_t cbase;
@@ -265,63 +270,69 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
   if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // DMA: a half-tile is 16 pieces, rows (j >> 3) 128 + (j & 7) 8 (+ 64: the second half); a wave moves pieces 4 wave .. + 3
+  // DMA: a half-tile is 16 pieces (A: 4 HX) of eight rows, half of them for either half of the waves: piece j of W is rows
+  // (j >> 3) 128 + (j & 7) 8 (+ 64: the second half); a wave moves pieces 4 wave .. + 3 (A: HX wave .. + HX - 1)
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
-  int prow[4];
-  unsigned xo[8], wo[8];
+  int xpr[HX], wpr[4];
+  unsigned xo[2 * HX], wo[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = 4 * wave + i;
-    prow[i] = (j >> 3) * 128 + (j & 7) * 8;
+    wpr[i] = (j >> 3) * 128 + (j & 7) * 8;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      xo[4 * h + i] = a_offset(a, m0, mend, prow[i] + 64 * h + lr) + lc * 16;
-      wo[4 * h + i] = w_offset(a, n0, prow[i] + 64 * h + lr) + lc * 16;
-    }
+    for (int h = 0; h < 2; ++h) wo[4 * h + i] = w_offset(a, n0, wpr[i] + 64 * h + lr) + lc * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < HX; ++i) {
+    const int j = HX * wave + i;
+    xpr[i] = j / (2 * HX) * (32 * HX) + j % (2 * HX) * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) xo[HX * h + i] = a_offset(a, m0, mend, xpr[i] + 16 * HX * h + lr) + lc * 16;
   }
   const char* Ab = a_base(a, A, m0);
   const char* Wb = w_base(a, W, n0);
   // (past the last K tile the DMAs go through a descriptor of no records: counted like the others, they write zeros)
   const __amdgpu_buffer_rsrc_t rA = rsrc_of(Ab, true), rW = rsrc_of(Wb, true), r0 = rsrc_of(Ab, false);
 #define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, k0, 0, 0)
-#define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[(h) * 4 + (i)], k0, smem + (buf) * STG + (prow[i] + (h) * 64) * 128)
-#define T_W(rs, buf, h, i, k0) T_DMA(rs, wo[(h) * 4 + (i)], k0, smem + (buf) * STG + WIMG + (prow[i] + (h) * 64) * 128)
+#define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[(h) * HX + (i)], k0, smem + (buf) * STG + (xpr[i] + (h) * 16 * HX) * 128)
+#define T_W(rs, buf, h, i, k0) T_DMA(rs, wo[(h) * 4 + (i)], k0, smem + (buf) * STG + WIMG + (wpr[i] + (h) * 64) * 128)
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
   const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
-  const int xrow = (wm * 128 + fr) * 128, wrow = WIMG + (wn * 128 + fr) * 128;
-  floatx4 acc[8][8];
+  const int xrow = (wm * 32 * HX + fr) * 128, wrow = WIMG + (wn * 128 + fr) * 128;
+  floatx4 acc[2 * HX][8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u)
+  for (int u = 0; u < 2 * HX; ++u)
 #pragma unroll
     for (int t = 0; t < 8; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 xf[8][2], wf[8][2];
+  bf16x8 xf[2 * HX][2], wf[8][2];
 #define T_HOLD()                                                                                   \
-  _Pragma("unroll") for (int u_ = 0; u_ < 8; ++u_)                                                 \
+  _Pragma("unroll") for (int u_ = 0; u_ < 2 * HX; ++u_)                                            \
   _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+a"(acc[u_][t_]));
   T_HOLD();
   asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");          // (the zeros are written before the first MFMA reads them)
 #define T_RX(buf, f, k) xf[f][k] = *(const bf16x8*)(smem + (buf) * STG + xrow + (f) * 2048 + ((k) ? c1 : c0))
 #define T_RW(buf, f, k) wf[f][k] = *(const bf16x8*)(smem + (buf) * STG + wrow + (f) * 2048 + ((k) ? c1 : c0))
-// 32 MFMAs of the quadrant (x half xh, w half wh); after the first even ones the 8 reads of the half needed next (RX: of x),
-// after four later ones the DMAs of a half-tile (DX: of x)
+// 8 HX MFMAs of the quadrant (x half xh, w half wh); after the first even ones the reads of the half needed next (RX: of x), 2 HX
+// or 8 of them, after later ones the DMAs of a half-tile (DX: of x), HX or 4
 #define T_PHASE(xh, wh, RX, rbuf, rh, DX, rs, dbuf, dh, dk, SYNC)                                  \
   {                                                                                                \
-    _Pragma("unroll") for (int i_ = 0; i_ < 32; ++i_) {                                            \
-      const int s_ = i_ >> 4, u_ = (xh) * 4 + ((i_ >> 2) & 3), t_ = (wh) * 4 + (i_ & 3);           \
+    _Pragma("unroll") for (int i_ = 0; i_ < 8 * HX; ++i_) {                                        \
+      const int s_ = i_ / (4 * HX), u_ = (xh) * HX + (i_ >> 2) % HX, t_ = (wh) * 4 + (i_ & 3);     \
       mfma_in_place(acc[u_][t_], wf[t_][s_], xf[u_][s_]);                                          \
-      if (i_ < 16 && (i_ & 1) == 0) {                                                              \
-        const int f_ = (rh) * 4 + (i_ >> 2), k_ = (i_ >> 1) & 1;                                   \
-        if (RX) T_RX(rbuf, f_, k_);                                                                \
-        else T_RW(rbuf, f_, k_);                                                                   \
+      if (i_ < (RX ? 4 * HX : 16) && (i_ & 1) == 0) {                                              \
+        const int f_ = i_ >> 2, k_ = (i_ >> 1) & 1;                                                \
+        if (RX) T_RX(rbuf, (rh) * HX + f_, k_);                                                    \
+        else T_RW(rbuf, (rh) * 4 + f_, k_);                                                        \
       }                                                                                            \
-      if (i_ >= 17 && i_ <= 26 && (i_ - 17) % 3 == 0) {                                            \
-        if (DX) T_X(rs, dbuf, dh, (i_ - 17) / 3, dk);                                              \
-        else T_W(rs, dbuf, dh, (i_ - 17) / 3, dk);                                                 \
+      constexpr int D0_ = HX == 4 ? 17 : HX == 3 ? 13 : 5, DN_ = DX ? HX : 4;                      \
+      if (i_ >= D0_ && i_ < D0_ + 3 * DN_ && (i_ - D0_) % 3 == 0) {                                \
+        if (DX) T_X(rs, dbuf, dh, (i_ - D0_) / 3, dk);                                             \
+        else T_W(rs, dbuf, dh, (i_ - D0_) / 3, dk);                                                \
       }                                                                                            \
     }                                                                                              \
     if (SYNC) {                                                                                    \
-      asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");                                 \
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * HX + 8) : "memory");                 \
       __builtin_amdgcn_s_barrier();                                                                \
     }                                                                                              \
   }
@@ -341,30 +352,30 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
     const __amdgpu_buffer_rsrc_t rA1 = nk > 1 ? rA : r0, rW1 = nk > 1 ? rW : r0;
     const int k1 = nk > 1 ? KT : 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) T_X(rA, 0, 0, i, 0);
+    for (int i = 0; i < HX; ++i) T_X(rA, 0, 0, i, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW, 0, 0, i, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW, 0, 1, i, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) T_X(rA, 0, 1, i, 0);
+    for (int i = 0; i < HX; ++i) T_X(rA, 0, 1, i, 0);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) T_X(rA1, 1, 0, i, k1);
+    for (int i = 0; i < HX; ++i) T_X(rA1, 1, 0, i, k1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW1, 1, 1, i, k1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW1, 1, 0, i, k1);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) T_X(rA1, 1, 1, i, k1);
+    for (int i = 0; i < HX; ++i) T_X(rA1, 1, 1, i, k1);
   }
-  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * HX + 12) : "memory");
   __builtin_amdgcn_s_barrier();
 #pragma unroll
   for (int f = 0; f < 4; ++f) {
-    T_RX(0, f, 0); T_RX(0, f, 1);
+    if (f < HX) { T_RX(0, f, 0); T_RX(0, f, 1); }
     T_RW(0, f, 0); T_RW(0, f, 1);
   }
-  asm volatile("s_waitcnt vmcnt(16) lgkmcnt(0)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * HX + 8) : "memory");
   __builtin_amdgcn_s_barrier();
   // (an odd last K tile is followed by one of zeros, which is what a DMA without records leaves in LDS: a loop exit in the
   // middle would have the compiler move accumulators between registers while asm MFMAs it cannot see are still writing them)
@@ -391,8 +402,12 @@ __global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) {
 #undef T_ODD
 #undef T_X
 #undef T_W
-  finish<8, 8, 4, true>(a, acc, cbase, m0 + wm * 128, n0 + wn * 128, mend, smem + wave * 32768);
+  finish<2 * HX, 8, HX, true>(a, acc, cbase, m0 + wm * 32 * HX, n0 + wn * 128, mend, smem + wave * (HX * 8192));
 }
+
+__global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) { tile_256<4>(a); }
+__global__ __launch_bounds__(256, 1) void gemm_tile_192(Tile a) { tile_256<3>(a); }
+__global__ __launch_bounds__(256, 1) void gemm_tile_128(Tile a) { tile_256<2>(a); }
 
 // ------------------------------------------------------------------------------------ smaller tiles
 // 32 MI x 32 NJ outputs, four waves in a 2 x 2 grid of 16 MI x 16 NJ, S stages of LDS: the DMAs of K tile t + S - 1 are issued
@@ -564,10 +579,11 @@ int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
 struct TileCost { int tm, tn, slots; float k_us, round_us; };
 // bf16 (16384 x 14336 x 4096: the 256 tile 1.49 ms, 128 x 128 2.28; 1024 x 2048 x 2048: 64 x 128 18 us, the 256 tile 45;
 // 256 x 2048 x 2048: 32 x 64 9 us, the 256 tile 45)
-static const TileCost TILES[] = {{256, 256, 256, 1.35f, 12.f},      // least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
-                                 {128, 128, 512, 1.0f, 9.f},        // two blocks a CU
+static const TileCost TILES[] = {{256, 256, 256, 1.42f, 11.f},     // least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
+                                 {128, 128, 512, 1.08f, 5.f},      // two blocks a CU
                                  {128, 128, 256, 0.55f, 6.f}, {64, 128, 256, 0.40f, 5.f}, {64, 64, 256, 0.26f, 3.f},      // two wave groups
-                                 {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f}};                                 // four
+                                 {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f},                                  // four
+                                 {192, 256, 256, 1.09f, 9.5f}, {128, 256, 256, 0.82f, 8.f}};
 // fp32 rows, bf16 weights (16384 rows x 32 blocks of 256 x 256: 128 x 128 432 us, 458 at 64 x 128, 615 before; 400 x 2048 x 2048:
 // 64 x 64 16 us, 128 x 128 39)
 static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f}, {64, 128, 256, 0.47f, 5.f}, {64, 64, 256, 0.37f, 4.2f},
@@ -584,10 +600,17 @@ static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int
   for (int v = 0; v < count; ++v) {
     const TileCost& t = tiles[v];
     if (gated && t.tn < 64) continue;      // (a wave of the 32-column tile has one half of a gated column only)
-    // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average)
-    const long long rows = by_rows ? (long long)M / t.tm + (groups + 1) / 2 : (long long)((M + t.tm - 1) / t.tm) * groups;
-    const long long blocks = rows * ((N + t.tn - 1) / t.tn);
-    const float us = (float)((blocks + t.slots - 1) / t.slots) * ((float)nk * t.k_us + t.round_us);
+    // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average, and how they fall on the
+    // CUs is chance: a launch that just fills the chip takes a second round, 2048 rows of 8 experts on 192-row tiles 80 us, 62 on 256)
+    const long long cols = (N + t.tn - 1) / t.tn;
+    float rounds;
+    if (by_rows) {
+      const float full = ((float)M / t.tm + 0.5f * groups) * cols / t.slots;
+      rounds = full <= 0.9f ? 1.f : full + 0.5f;
+    } else {
+      rounds = (float)(((long long)((M + t.tm - 1) / t.tm) * groups * cols + t.slots - 1) / t.slots);
+    }
+    const float us = rounds * ((float)nk * t.k_us + t.round_us);
     if (v == 0 || us < least) {
       least = us;
       best = v;
@@ -613,14 +636,16 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
                   a_mod < 1 ? 1 : a_mod, 0, 0, 0, ragged};
   const bool by_rows = offs != nullptr;
   if (ta == 1) {
-    switch (ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 7, M, N, nk, groups, by_rows, gated)) {
-      case 0: return start<gemm_tile_256>(256, 256, 256, t256::LDS_BYTES, t, s);
+    switch (ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 9, M, N, nk, groups, by_rows, gated)) {
+      case 0: return start<gemm_tile_256>(256, 256, 256, t256::lds_bytes(4), t, s);
       case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
       case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
       case 3: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
       case 4: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
       case 5: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
-      default: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
+      case 6: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
+      case 7: return start<gemm_tile_192>(192, 256, 256, t256::lds_bytes(3), t, s);
+      default: return start<gemm_tile_128>(128, 256, 256, t256::lds_bytes(2), t, s);
     }
   }
   if (tw == 1) {

@@ -75,11 +75,11 @@ def test_matmul(ops, cdt, tol, M, N, K):
     close(H.matmul_nt(af, w), R.matmul_nt(af.to(cdt), w), 1e-5)
 
 
-# one shape for each tile of gemm_tile.hip (256 x 256, 128 x 128 twice, 64 x 128, 64 x 64, 32 x 64, 32 x 32), with rows and
+# one shape for each tile of gemm_tile.hip (256 x 256, 128 x 128 twice, 64 x 128, 64 x 64, 32 x 64, 32 x 32, 192 and 128 x 256), with rows and
 # columns past a tile's end and odd numbers of 64-wide K tiles.  fp32 sums of bf16 products: 1e-5; rounded to bf16: half a
 # unit in the last place of the largest value (2^-9) and the other side's sum
 @pytest.mark.parametrize("M,N,K", [(2100, 4100, 64), (4100, 4100, 192), (1030, 4000, 64), (1024, 3900, 320), (1000, 2000, 320), (257, 2020, 320),
-                                   (200, 2000, 1088), (65, 132, 448)])
+                                   (200, 2000, 1088), (65, 132, 448), (4000, 4092, 320), (2500, 4100, 320), (3000, 4092, 256), (2000, 4000, 1984), (1025, 7000, 1088)])
 def test_matmul_tiles(ops, M, N, K):
     H, R = ops
     torch.manual_seed(M + N + K)
