@@ -327,7 +327,7 @@ int launch_grouped(const half_t* A, const half_t* W, half_t* C, int M_bound, int
     attr = true;
   }
   const int tiles_m = (M_bound + BM - 1) / BM, tiles_n = N / BN;
-  Epi ep{nullptr, 0, nullptr, nullptr, nullptr, 0, 0, nullptr, N / 2, auto_order(tiles_m, tiles_n),
+  Epi ep{nullptr, 0, nullptr, nullptr, nullptr, 0, 0, nullptr, N / 2, tiles_n <= 8 ? -tiles_n : -4,
          tiles, offs, rows, wstride, n_groups};
   hipLaunchKernelGGL((gemm_nt_v10<EPI, true>), dim3(tiles_m * tiles_n), dim3(256), 2 * BUF, s, A, W, C, M_bound, N,
                      K, lda, ldw, ldc, ep);

@@ -45,13 +45,25 @@ __device__ __forceinline__ int2 place(int b, int tiles_m, int tiles_n, int order
 // This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
 template <int TM, int TN>
 __device__ __forceinline__ bool locate(const Tile& a, const char*& A, const char*& W, size_t& cbase, int& m0, int& mend, int& n0) {
-  const int nwg = gridDim.x;
+  int nwg = gridDim.x, tiles_m = a.tiles_m;
   int bid = blockIdx.x;
+  // The launch covers the most tiles that row groups can have; only those there are take part, or whole XCDs get few or none (19384
+  // rows at most, 15500 in 8 groups, 2 x 2048 columns, 2048 terms: 333 -> 274 us).
+  if (a.offs != nullptr) {
+    const int lane = threadIdx.x & 63;
+    int cnt = 0;
+    for (int g = lane; g < a.groups; g += 64) cnt += (a.offs[g + 1] - a.offs[g] + TM - 1) / TM;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+    tiles_m = __builtin_amdgcn_readfirstlane(cnt);
+    nwg = tiles_m * a.tiles_n;
+    if (bid >= nwg) return false;
+  }
   {                                      // blocks go to the 8 XCDs in turn: give each a run of consecutive ids
     const int q = nwg >> 3, r = nwg & 7, xcd = bid & 7, loc = bid >> 3;
     bid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + loc;
   }
-  const int2 t = place(bid, a.tiles_m, a.tiles_n, a.order);
+  const int2 t = place(bid, tiles_m, a.tiles_n, a.order);
   int tm = t.x;
   A = a.A;
   W = a.W;
