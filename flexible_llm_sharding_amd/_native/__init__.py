@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 17   # csrc/include/fls_seq.h
+SEQ_ABI = 18   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -173,8 +173,7 @@ def _load_seq():
     _bind(lib, "fls_seq_ssd_scan", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, p)
     _bind(lib, "fls_seq_ssd_scan_chunked", i, p, i, p, i, p, i, p, p, p, p, p, i, p, p, p, i, i, i, i, i, i, p, p)
     _bind(lib, "fls_seq_moe_route", i, p, i, p, i, i, i, p, p, p, p, p, p, p)
-    _bind(lib, "fls_seq_moe_scan", i, p, i, p, p, p)
-    _bind(lib, "fls_seq_moe_place", i, p, i, i, p, p, p, p)
+    _bind(lib, "fls_seq_moe_place", i, p, i, i, p, i, p, p, p, p, p)
     _bind(lib, "fls_seq_moe_sum", i, p, i, p, p, p, i, i, i, i, p)
     _bind(lib, "fls_seq_moe_route_grouped", i, p, i, i, i, i, i, i, f, p, p, p, p)
     _bind(lib, "fls_seq_embed_pos", i, p, p, i, p, p, p, p, i, ll, ll, p, i, i, i, i, f, i, p)

@@ -370,9 +370,8 @@ class HipSeqOps:
         s = _stream()
         _chk(self.k.fls_seq_moe_route_grouped(logits.data_ptr(), logits.stride(0), T, E, top, int(groups or 0), int(keep or 0),
                                               float(scale), ids.data_ptr(), w.data_ptr(), hist.data_ptr(), s), "fls_seq_moe_route_grouped")
-        _chk(self.k.fls_seq_moe_scan(hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), s), "fls_seq_moe_scan")
-        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, cursor.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
-             "fls_seq_moe_place")
+        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+                                      rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 
     ROUTE_FUSED = 64          # (the limit in csrc/include/fls_seq.h) up to that many tokens one launch routes, counts and places
@@ -396,9 +395,8 @@ class HipSeqOps:
                                                       w.data_ptr(), hist.data_ptr(), offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
              "fls_seq_moe_route_softmax_grouped")
         if not fused:
-            _chk(self.k.fls_seq_moe_scan(hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), s), "fls_seq_moe_scan")
-            _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, cursor.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
-                 "fls_seq_moe_place")
+            _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+                                          rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 
     @staticmethod
@@ -991,7 +989,7 @@ class HipSeqOps:
         dev = logits.device
         ids = torch.empty(T, top, dtype=torch.int32, device=dev)
         w = torch.empty(T, top, dtype=torch.float32, device=dev)
-        fused = corr is not None and T <= self.ROUTE_FUSED
+        fused = corr is not None and 0 < T <= self.ROUTE_FUSED
         ints = torch.empty(E + 1, dtype=torch.int32, device=dev) if fused else torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)
         offs, hist, cursor = ints[:E + 1], ints[E + 1:2 * E + 1], ints[2 * E + 1:]
         dest = torch.empty(T, top, dtype=torch.int32, device=dev)
@@ -1001,9 +999,8 @@ class HipSeqOps:
                                       w.data_ptr(), hist.data_ptr(), offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s), "fls_seq_moe_route")
         if fused:
             return SeqRoute(ids, w, offs, rows, dest, top)
-        _chk(self.k.fls_seq_moe_scan(hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), s), "fls_seq_moe_scan")
-        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, cursor.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
-             "fls_seq_moe_place")
+        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+                                      rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 
     def add_group_rmsnorm_moe_(self, x, y, route, w, groups, eps):
