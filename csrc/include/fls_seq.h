@@ -167,6 +167,10 @@ int fls_seq_rglru_scan_tiled(const float* u, int ldu, const float* g, int ldg, c
                              int ldy, float* state, void* out, int to, int ldo, const int* tiles, int n_tiles,
                              const int* tile_cu, float* scratch, const int* pos0, const int* slot, int B, int W,
                              float c, fls_stream_t s);
+// the same in one pass over each request's rows (no scratch): requests that are not too long, or that fill the chip
+int fls_seq_rglru_scan_rows(const float* u, int ldu, const float* g, int ldg, const float* lam, const float* y, int ldy, float* state,
+                            void* out, int to, int ldo, const int* cu, const int* pos0, const int* slot, int B, int W, float c,
+                            fls_stream_t s);
 // S_t = exp(-exp(A_log) dt_t) S_(t-1) + dt_t B_t x_t^T, y_t = S_t^T C_t + D x_t, dt_t = softplus(dt + dt_bias);
 // out = y * silu(z) fp32; xbc = [x (nh P) | B (G N) | C (G N)] columns; state[slot][nh][N][P]
 int fls_seq_ssd_scan(const float* xbc, int ldx, const float* z, int ldz, const float* dt, int lddt,

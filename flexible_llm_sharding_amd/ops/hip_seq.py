@@ -899,6 +899,10 @@ class HipSeqOps:
              "fls_seq_gated_delta_scan")
         return out
 
+    # rows of the longest request up to which one pass over its rows beats three over tiles of all, where the channels of all requests do
+    # not fill the chip (2048 channels, 1 request of 2048 / 4096 / 16384 rows: 84 / 164 / 716 us, in three 116 / 149 / 327)
+    RGLRU_ROWS = 3072
+
     def rglru_scan(self, u, g, lam, y, state, meta, c, out_dtype):
         _rows(u, "u", torch.float32)
         _rows(g, "g", torch.float32)
@@ -909,8 +913,15 @@ class HipSeqOps:
         _vec(lam, "lam", Wd)
         out = torch.empty(T, Wd, dtype=out_dtype, device=u.device)
         tiles, tile_cu = meta.get("q_tiles"), meta.get("tile_cu")
+        rows = int(meta.get("max_rows") or 0)
+        if tiles is not None and (rows <= self.RGLRU_ROWS or -(-Wd // 64) * meta["n_seqs"] >= 256):
+            _chk(self.k.fls_seq_rglru_scan_rows(u.data_ptr(), u.stride(0), g.data_ptr(), g.stride(0), lam.data_ptr(), y.data_ptr(),
+                                                y.stride(0), state.data_ptr(), out.data_ptr(), _CODE[out_dtype], Wd, meta["cu"].data_ptr(),
+                                                meta["pos0"].data_ptr(), meta["slot"].data_ptr(), meta["n_seqs"], Wd, float(c), _stream()),
+                 "fls_seq_rglru_scan_rows")
+            return out
         if tiles is not None and tile_cu is not None:
-            # many rows per request: three passes over row tiles instead of one thread per prompt and channel
+            # few long requests: three passes over row tiles instead of one thread per prompt and channel
             scratch = torch.empty(2 * tiles.shape[0] * Wd, dtype=torch.float32, device=u.device)
             _chk(self.k.fls_seq_rglru_scan_tiled(u.data_ptr(), u.stride(0), g.data_ptr(), g.stride(0), lam.data_ptr(),
                                                  y.data_ptr(), y.stride(0), state.data_ptr(), out.data_ptr(),

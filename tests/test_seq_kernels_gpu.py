@@ -384,6 +384,34 @@ def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
     close(s1, s2, 3e-6)
 
 
+# the gated linear recurrence in one pass over the rows (32 channels a block, and 64 where the requests fill the chip) and in three over row
+# tiles: parts and rounds of 128 rows that end early, one-row requests beside long ones, carried states; the oracle in fp64
+@pytest.mark.parametrize("lens,W,limit", [([300, 1, 129, 16], 70, 10 ** 9), ([300, 1, 129, 16], 70, 0), ([1, 128, 3, 130] * 35, 130, 0)])
+def test_rglru_forms(ops, monkeypatch, lens, W, limit):
+    H, _ = ops
+    torch.manual_seed(W)
+    monkeypatch.setattr(H, "RGLRU_ROWS", limit)
+    pos0 = [5 * (i % 2) for i in range(len(lens))]
+    md, _, nslots = meta_of(lens, pos0, DEV)
+    T = sum(lens)
+    u, g, lam, y = torch.randn(T, W, device=DEV), torch.randn(T, 2 * W, device=DEV), torch.randn(W, device=DEV), torch.randn(T, W, device=DEV)
+    st = torch.randn(nslots, W, device=DEV)
+    want, out = st.cpu().double(), torch.empty(T, W, dtype=torch.float64)
+    u6, g6, l6, y6 = (t.cpu().double() for t in (u, g, lam, y))
+    la = -8.0 * torch.sigmoid(g6[:, :W]) * torch.nn.functional.softplus(l6)
+    a6, b6 = torch.exp(la), torch.sqrt(-torch.expm1(2 * la)) * torch.sigmoid(g6[:, W:]) * u6
+    for s, (n, p0) in enumerate(zip(lens, pos0)):
+        a0, slot = int(md["cu_host"][s]), int(md["slot"][s])
+        S = want[slot] * bool(p0)
+        for t in range(a0, a0 + n):
+            S = a6[t] * S + b6[t]
+            out[t] = S
+        want[slot] = S
+    got = H.rglru_scan(u, g, lam, y, st, md, 8.0, torch.float32)
+    close(got, out * torch.nn.functional.gelu(y6, approximate="tanh"), 2e-6)
+    close(st, want, 2e-6)
+
+
 # the chunked delta rules: chunk ends, one row and none beside long requests, a carried state, shared keys, value columns that do not fill
 # four waves, decays from none to exact zeros, and (small memory) several launches that pass the state on; the oracle in fp64.  The
 # bound is that of fp32 sums over some 128 terms and 16-row chains; the row-by-row kernels have to meet it too
