@@ -4,8 +4,9 @@
 //   y_i = exp(c_i) C_i . S + sum_{j <= i} exp(c_i - c_j) dt_j (C_i . B_j) x_j,    S' = exp(c_64) S + sum_j exp(c_64 - c_j) dt_j B_j x_j^T
 //
 // so a request of n rows is a chain of n / 64 chunks instead of n rows.  What bounds the row-by-row form is that chain (0.7 us a
-// row: 512 rows 359 us whatever the batch); here it is the products, 2.6 us of MFMAs a chunk and block, and the L2 reads of
-// B and C.  C_i . B_j is the same for all heads of a group: a first kernel leaves it in memory once ([T, groups, 64] fp32).  Exponents
+// row); here it is a chunk's chain of products and LDS reads, with C, the scores and z loaded while the chunk is laid down.  C_i . B_j
+// is the same for all heads of a group: a first kernel leaves it in memory once ([T, groups, 64] fp32).  Row by row against this, heads
+// of 64 x 128: 2 requests of 512 rows, 32 heads 352 -> 61 us; 8 of 2048 rows, 64 heads 1883 -> 652; 1 of 2048 1445 -> 193.  Exponents
 // are differences of running sums: the sums are fp64, so a difference is exact to fp32 however far a chunk has decayed.
 // All products are fp32 (16x16x4 MFMAs: lane group g holds elements 4 g .. 4 g + 3 of 16, MFMA r multiplies the r-th ones).
 #include "seq_common.h"
@@ -121,6 +122,28 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
   prefetch(a0);
   for (int r0 = a0; r0 < a1; r0 += CQ) {
     const int nt = min(CQ, a1 - r0);
+    // what this wave's rows of y need beside LDS travels while the chunk is laid down and its decays are summed
+    const int row = r0 + min(16 * w + fr, nt - 1);            // (rows past the end are computed from the last one and not stored)
+    constexpr bool AHEAD = PT * NW < 4;                       // (C's row too, where the registers are there: with 2 x 2 it spilled, 882 -> 1140 us)
+    floatx4 cr[AHEAD ? N / 16 : 1], sr[4];
+    float zr[PT][4];
+    const float* crow = a.xbc + (size_t)row * a.ldx + inner + (a.G + g) * N + 4 * grp;
+    if (16 * w < nt) {
+      const float* sc = a.scores + ((size_t)row * a.G + g) * CQ + 4 * grp;
+      if constexpr (AHEAD) {
+#pragma unroll
+        for (int n = 0; n < N / 16; ++n) cr[n] = *reinterpret_cast<const floatx4*>(crow + 16 * n);
+      }
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb)
+        if (jb <= w) sr[jb] = *reinterpret_cast<const floatx4*>(sc + 16 * jb);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = min(16 * w + 4 * grp + r, nt - 1);
+#pragma unroll
+        for (int p = 0; p < PT; ++p) zr[p][r] = a.z[(size_t)(r0 + t) * a.ldz + h * a.P + p0 + 16 * p + fr];
+      }
+    }
     __syncthreads();                                          // (the chunk before has been read)
 #pragma unroll
     for (int i = 0; i < NB4; ++i) {
@@ -154,18 +177,16 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
     __syncthreads();
     if (r0 + CQ < a1) prefetch(r0 + CQ);
     // y: the chunk's own rows, then the state before it
-    const int row = r0 + min(16 * w + fr, nt - 1);            // (rows past the end are computed from the last one and not stored)
     floatx4 own[PT], past[PT];
 #pragma unroll
     for (int p = 0; p < PT; ++p) own[p] = past[p] = floatx4{0.f, 0.f, 0.f, 0.f};
     if (16 * w < nt) {
       const int i = 16 * w + fr;
       const double ci = cs[i];
-      const float* sc = a.scores + ((size_t)row * a.G + g) * CQ + 4 * grp;
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb) {
         if (jb > w) continue;
-        const floatx4 m = *reinterpret_cast<const floatx4*>(sc + 16 * jb);
+        const floatx4 m = sr[jb];
         floatx4 l;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -180,10 +201,9 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
           own[p] = mfma16(l, x, own[p]);
         }
       }
-      const float* crow = a.xbc + (size_t)row * a.ldx + inner + (a.G + g) * N + 4 * grp;
 #pragma unroll
       for (int n = 0; n < N; n += 16) {
-        const floatx4 c = *reinterpret_cast<const floatx4*>(crow + n);
+        const floatx4 c = AHEAD ? cr[AHEAD ? n / 16 : 0] : *reinterpret_cast<const floatx4*>(crow + n);
 #pragma unroll
         for (int p = 0; p < PT; ++p) {
           floatx4 v;
@@ -201,7 +221,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
           for (int p = 0; p < PT; ++p) {
             const int col = h * a.P + p0 + 16 * p + fr;
             const float y = e * past[p][r] + own[p][r] + dsk * xs[t * LX + 16 * p + fr];
-            a.out[(size_t)(r0 + t) * a.ldo + col] = y * silu_f(a.z[(size_t)(r0 + t) * a.ldz + col]);
+            a.out[(size_t)(r0 + t) * a.ldo + col] = y * silu_f(zr[p][r]);
           }
         }
       }

@@ -935,7 +935,9 @@ class HipSeqOps:
                                        meta["n_seqs"], Wd, float(c), _stream()), "fls_seq_rglru_scan")
         return out
 
-    SSD_CHUNK_ROWS = 24        # rows of one request from which the chunked scan is the faster one
+    # rows of one request from which the chunked scan is the faster one (32 heads of 64 x 128, 1 request of 16 / 24 / 64 rows: 15.1 / 20.5 /
+    # 46 us row by row, 15.9 / 15.4 / 19 in chunks; 32 requests: 41 / 56 / 124 and 44 / 51 / 64)
+    SSD_CHUNK_ROWS = 24
 
     def ssd_scan(self, xbc, z, dt, dt_bias, A_log, Dskip, state, meta, nh, P, N, G):
         _rows(xbc, "xbc", torch.float32)
