@@ -838,10 +838,12 @@ class HipSeqOps:
         chunks at a time as stay in the last-level cache; (None, 0) where a row-by-row walk serves: short requests, and so many that
         less than four chunks of each fit (200 requests of 300 rows: 2.5 ms row by row, 4.6 ms a chunk at a time)."""
         rows = int(meta.get("max_rows") or 0)
+        if rows < least or dim not in (64, 128):
+            return None, 0
         each = meta["n_seqs"] * heads * (16 * dim * mats + 256 * (mats - 1) + dim)
         chunks = -(-rows // 16)
         seg = min(chunks, self.DELTA_FACTOR_BYTES // (4 * each))
-        if rows < least or dim not in (64, 128) or seg < min(chunks, 4):
+        if seg < min(chunks, 4):
             return None, 0
         return torch.empty(seg * each, dtype=torch.float32, device=device), seg
 
