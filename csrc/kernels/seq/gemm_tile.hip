@@ -258,8 +258,7 @@ __device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], si
 // ------------------------------------------------------------------------------------ 256, 192 and 128 x 256
 // Four waves, one per SIMD, 32 HX x 128 outputs each.  HX = 4: 128 x 128, all 256 accumulation registers of a wave, a fragment
 // read from LDS feeds 8 MFMAs.  HX = 3, 2: 192 and 128 rows, for row counts that leave the chip idle in the last (or only) round of
-// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 2048 two thirds of
-// the 192-row tile's time.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
+// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 1024 35, 29, 24.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
 // accumulation register the compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between
 // them; reads run one phase of 8 HX MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
 namespace t256 {
