@@ -6,7 +6,7 @@
 // so a request of n rows is a chain of n / 64 chunks instead of n rows.  What bounds the row-by-row form is that chain (0.7 us a
 // row); here it is a chunk's chain of products and LDS reads, with C, the scores and z loaded while the chunk is laid down.  C_i . B_j
 // is the same for all heads of a group: a first kernel leaves it in memory once ([T, groups, 64] fp32).  Row by row against this, heads
-// of 64 x 128: 2 requests of 512 rows, 32 heads 352 -> 61 us; 8 of 2048 rows, 64 heads 1883 -> 652; 1 of 2048 1445 -> 193.  Exponents
+// of 64 x 128: 2 requests of 512 rows, 32 heads 348 -> 62 us; 8 of 2048 rows, 64 heads 1880 -> 688; 1 of 2048 1443 -> 198.  Exponents
 // are differences of running sums: the sums are fp64, so a difference is exact to fp32 however far a chunk has decayed.
 // All products are fp32 (16x16x4 MFMAs: lane group g holds elements 4 g .. 4 g + 3 of 16, MFMA r multiplies the r-th ones).
 #include "seq_common.h"
@@ -183,6 +183,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
     if (16 * w < nt) {
       const int i = 16 * w + fr;
       const double ci = cs[i];
+      bool odd = false;                                       // inf or NaN among the wave's own rows
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb) {
         if (jb > w) continue;
@@ -198,7 +199,27 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
           floatx4 x;
 #pragma unroll
           for (int r = 0; r < 4; ++r) x[r] = xs[(16 * jb + 4 * grp + r) * LX + 16 * p + fr];
+          if (jb == w) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const bool f = __builtin_isfinite(x[r]);
+              odd |= !f;
+              x[r] = f ? x[r] : 0.f;
+            }
+          }
           own[p] = mfma16(l, x, own[p]);
+        }
+      }
+      // (a weight of 0 would spread such a value to the rows before it: it stayed out of the product and makes NaN of its own and
+      // later rows; row by row the signs of B and C make inf or NaN of them)
+      if (__any(odd)) {
+#pragma unroll
+        for (int p = 0; p < PT; ++p) {
+          int at = CQ;
+          for (int j = 15; j >= 0; --j)
+            if (!__builtin_isfinite(xs[(16 * w + j) * LX + 16 * p + fr])) at = j;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) own[p][r] = 4 * grp + r >= at ? __builtin_nanf("") : own[p][r];
         }
       }
 #pragma unroll

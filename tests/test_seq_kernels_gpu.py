@@ -384,6 +384,43 @@ def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
     close(s1, s2, 3e-6)
 
 
+# a value that is not finite stays where the recurrence puts it: rows before its own, other requests and (a value of x) other columns are
+# what they are without it, bit by bit.  Rows in the first, a middle and the last block of 16 of a chunk, and in the second chunk
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("nh,P,N", [(2, 16, 64), (2, 48, 128), (128, 32, 128)])
+def test_ssd_chunks_values_that_are_not_finite(ops, bad, nh, P, N):
+    H, _ = ops
+    torch.manual_seed(P + N)
+    lens, pos0, inner = (100, 70), (0, 3), nh * P
+    md, _, nslots = meta_of(lens, pos0, DEV)
+    T, a1 = sum(lens), int(md["cu_host"][1])
+    xbc, z, dt = torch.randn(T, inner + 2 * N, device=DEV), torch.randn(T, inner, device=DEV), torch.randn(T, nh, device=DEV)
+    dtb, Al, Ds = torch.randn(nh, device=DEV), torch.randn(nh, device=DEV) * 0.5, torch.randn(nh, device=DEV)
+    s0 = torch.randn(nslots, nh, N, P, device=DEV)
+    other = int(md["slot"][1])
+
+    def run(x, d):
+        st = s0.clone()
+        return H.ssd_scan(x, z, d, dtb, Al, Ds, st, md, nh, P, N, 1), st
+
+    clean, sclean = run(xbc, dt)
+    for t in (5, 44, 63, 90):
+        for col in (3, inner + 2, inner + N + 2):                       # of x, B and C
+            x = xbc.clone()
+            x[t, col] = bad
+            got, st = run(x, dt)
+            assert torch.equal(got[:t], clean[:t]) and torch.equal(got[a1:], clean[a1:]) and torch.equal(st[other], sclean[other])
+            assert not bool(got[t, :P].isfinite().all())
+            if col == 3:
+                keep = torch.arange(inner, device=DEV) != 3
+                assert torch.equal(got[:, keep], clean[:, keep]) and not bool(got[t, 3].isfinite())
+        d = dt.clone()
+        d[t, 0] = bad
+        got, st = run(xbc, d)                                           # (a step of -inf is one of size 0)
+        assert torch.equal(got[:t], clean[:t]) and torch.equal(got[a1:], clean[a1:]) and torch.equal(st[other], sclean[other])
+        assert torch.equal(got[:, P:], clean[:, P:]) and (bad < 0 or not bool(got[t, :P].isfinite().all()))
+
+
 # the gated linear recurrence in one pass over the rows (32 channels a block, and 64 where the requests fill the chip) and in three over row
 # tiles: parts and rounds of 128 rows that end early, one-row requests beside long ones, carried states; the oracle in fp64
 @pytest.mark.parametrize("lens,W,limit", [([300, 1, 129, 16], 70, 10 ** 9), ([300, 1, 129, 16], 70, 0), ([1, 128, 3, 130] * 35, 130, 0)])
