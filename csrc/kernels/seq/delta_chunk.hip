@@ -21,7 +21,7 @@
 // What bounds the row-by-row forms is a chain of LDS reads, sums over lanes and updates per row, 0.5 us (128 x 128) or 0.7 us (64 x 64); a
 // chunk's chain here is its MFMAs and the two kernels' traffic over the factors, which stay in the last-level cache for as many chunks
 // as are made at a time.  Row by row against this (16 heads; outputs' norm included), gated 128 x 128 and generalized 64 x 64:
-//   1 request of 2048 rows:  640 -> 373 us, 1590 -> 284 us       9 of 1500:  1060 -> 680 us, 1410 -> 394 us
+//   1 request of 2048 rows:  640 -> 376 us, 1590 -> 287 us       9 of 1500:  1060 -> 687 us, 1410 -> 400 us
 #include "seq_common.h"
 #include "fls_seq.h"
 
@@ -237,6 +237,29 @@ __global__ __launch_bounds__(256, GEN ? 2 : 3) void delta_factors_kernel(Delta a
   }
 }
 
+// A chunk's lower triangular matrix (m: where it lies in LDS, f: as a left operand) times 16 rows of which some are not finite: those
+// rows reach the rows after them (DIAG: and their own) only.
+template <bool DIAG>
+__device__ __forceinline__ floatx4 below(const float* m, const floatx4& f, const floatx4& v) {
+  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+  floatx4 c;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) c[r] = __builtin_isfinite(v[r]) ? v[r] : 0.f;
+  floatx4 acc = mfma16(f, c, floatx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll 1
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const float e = __shfl(v[x], g * 16 + fr, 64);          // row 4 g + x of this lane's column
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int t = 4 * grp + r, s = 4 * g + x;
+        if (!__builtin_isfinite(e) && (DIAG ? t >= s : t > s)) acc[r] += m[frag(t, s)] * e;
+      }
+    }
+  return acc;
+}
+
 // wave = 16 value columns of one head and request; the block's waves share the factors, which travel to LDS a chunk ahead
 template <int D, bool GEN>
 __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
@@ -321,8 +344,16 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
 #pragma unroll
       for (int j = 0; j < d; ++j) { x[j] += x[j + d]; o[j] += o[j + d]; }
     X += x[0];
-    if constexpr (GEN) o[0] += mfma16(bk, v, zero);
-    O = mfma16(b, X, zero) + o[0];
+    if constexpr (GEN) O = mfma16(b, X, zero) + (mfma16(bk, v, zero) + o[0]);
+    else O = mfma16(b, X, zero) + o[0];
+    bool odd = false;                                          // (zeros above the diagonals would spread a later row's inf or NaN)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) odd |= !__builtin_isfinite(v[r]) | !__builtin_isfinite(X[r]);
+    if (__any(odd)) {
+      X = below<!GEN>(fs[buf] + L::N1, n1, v) + x[0];
+      if constexpr (GEN) o[0] += below<true>(fs[buf] + L::BK, bk, v);
+      O = below<true>(fs[buf] + L::B, b, X) + o[0];
+    }
 #pragma unroll
     for (int j = 0; j < J; ++j) S[j] *= *reinterpret_cast<const floatx4*>(fs[buf] + L::P + 16 * j + 4 * grp);
     __builtin_amdgcn_sched_barrier(0);

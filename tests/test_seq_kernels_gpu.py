@@ -502,6 +502,55 @@ def test_delta_chunks(ops, monkeypatch, lens, pos0, d, dv, heads, kv, small):
             close(x, y, 1e-5)
 
 
+# the same of the chunked delta rules: a value that is not finite changes no row before its own, no other request and no other head
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("d,heads", [(64, 2), (128, 3)])
+def test_delta_chunks_values_that_are_not_finite(ops, monkeypatch, bad, d, heads):
+    H, _ = ops
+    torch.manual_seed(d)
+    monkeypatch.setattr(H, "DELTA_CHUNK_ROWS", 1)
+    monkeypatch.setattr(H, "GATED_CHUNK_ROWS", 1)
+    lens, pos0 = [40, 21], [0, 5]
+    md, _, nslots = meta_of(lens, pos0, DEV)
+    T, hd, a1, other = sum(lens), heads * d, int(md["cu_host"][1]), int(md["slot"][1])
+    qkv, beta, gate = torch.randn(T, 3 * hd, device=DEV), torch.randn(T, heads, device=DEV), torch.randn(T, hd, device=DEV)
+    dec, nw = torch.rand(T, hd, device=DEV), torch.randn(d, device=DEV)
+    z, w0, nw2 = torch.randn(T, 6 * hd, device=DEV), torch.randn(hd, device=DEV) - 2.0, torch.randn(hd, device=DEV)
+    s0 = torch.randn(nslots, heads, d, d, device=DEV)
+
+    def gated(qkv, beta, dec):
+        st = s0.clone()
+        return H.gated_delta_scan(qkv, beta, dec, gate, nw, st, md, heads, heads, d, d, 1e-6, 1e-5, torch.float32), st
+
+    def general(z):
+        st, out = s0.clone(), torch.empty(T, hd, device=DEV)
+        H.delta_rule_scan(*(z[:, i * hd:(i + 1) * hd] for i in range(6)), w0, nw2, st, md, heads, d, decay_scale=0.6065, key_eps=1e-6,
+                          norm_eps=1e-5, out_scale=1.3, out=out)
+        return out, st
+
+    def check(got, clean, t, row):
+        assert torch.equal(got[0][:t], clean[0][:t]) and torch.equal(got[0][a1:], clean[0][a1:])
+        assert torch.equal(got[0][:, d:], clean[0][:, d:])
+        assert torch.equal(got[1][other], clean[1][other])
+        assert not row or not bool(got[0][t, :d].isfinite().all())
+
+    cg, cz = gated(qkv, beta, dec), general(z)
+    for t in (4, 15, 20, 38):
+        for at in (1, hd + 1, 2 * hd + 1):                              # of q, k and v in head 0
+            x = qkv.clone()
+            x[t, at] = bad
+            check(gated(x, beta, dec), cg, t, True)
+        x, y = beta.clone(), dec.clone()
+        x[t, 0] = float("nan")
+        y[t, 1] = bad
+        check(gated(qkv, x, dec), cg, t, True)
+        check(gated(qkv, beta, y), cg, t, t > 15)                       # (before the first rows the state is zero: inf x 0 and NaN x 0 apart)
+        for i in range(6):                                              # of r, k, v, removal rate, decay and gate
+            x = z.clone()
+            x[t, i * hd + 1] = bad
+            check(general(x), cz, t, i in (0, 1, 2) or (bad != bad and i < 5))
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("T,E,top", [(33, 10, 3), (700, 8, 2), (5, 40, 9), (300, 3, 1), (4, 8, 2), (10, 6, 3), (1, 5, 5)])
 def test_routing_and_expert_products(ops, cdt, tol, T, E, top):
