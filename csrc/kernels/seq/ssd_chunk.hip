@@ -163,7 +163,8 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
         for (int r = 0; r < 4; ++r) Ss[(16 * (NW * w + k) + 4 * grp + r) * LX + 16 * p + fr] = S[k][p][r];
     if (w == 0) {                                             // a row a lane: step sizes and the running sums of the decays' logarithms
       const float dtv = lane < nt ? softplus_f(pdt + db) : 0.f;
-      double c = lane < nt ? (double)fmaxf(negA * dtv, -1e30f) : 0.0;       // (an infinite decay stays a number)
+      // (past -104 a row's decay is an exact 0: held at -200 it still is, and no huge or infinite one costs the sums the rows after it)
+      double c = lane < nt ? (double)fmaxf(negA * dtv, -200.f) : 0.0;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
         const double v = __shfl_up(c, o, 64);

@@ -384,6 +384,29 @@ def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
     close(s1, s2, 3e-6)
 
 
+# a step so large that its own decay is 0 and the sum of a chunk's exponents would lose those of the rows after it
+@pytest.mark.parametrize("step", [3e2, 1e12, 1e17, 1e25])
+def test_ssd_chunks_huge_step(ops, step):
+    H, _ = ops
+    torch.manual_seed(7)
+    n, P, N = 60, 16, 64
+    md, _, nslots = meta_of((n,), (4,), DEV)
+    xbc, z, dt = torch.randn(n, P + 2 * N, device=DEV), torch.randn(n, P, device=DEV), torch.randn(n, 1, device=DEV) - 2
+    dt[20, 0] = step
+    st, one = torch.randn(nslots, 1, N, P, device=DEV), torch.zeros(1, device=DEV)
+    S, slot = st[int(md["slot"][0]), 0].cpu().double(), int(md["slot"][0])
+    x, B, C = (t.cpu().double() for t in torch.split(xbc, [P, N, N], 1))
+    d, want = torch.nn.functional.softplus(dt.cpu().double())[:, 0], torch.empty(n, P, dtype=torch.float64)
+    for t in range(n):
+        S = torch.exp(-d[t]) * S + d[t] * B[t][:, None] * x[t]
+        want[t] = C[t] @ S
+    got = H.ssd_scan(xbc, z, dt, one, one, one, st, md, 1, P, N, 1)
+    want = want * torch.nn.functional.silu(z.cpu().double())
+    close(got[:20], want[:20], 3e-6)
+    close(got[20:], want[20:], 3e-6)
+    close(st[slot, 0], S, 3e-6)
+
+
 # a value that is not finite stays where the recurrence puts it: rows before its own, other requests and (a value of x) other columns are
 # what they are without it, bit by bit.  Rows in the first, a middle and the last block of 16 of a chunk, and in the second chunk
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
