@@ -12,7 +12,7 @@
 //   factors (independent of the state, a block per chunk and head)     M1 .. into memory.  Nothing divides by a decay: a pair (t, s)
 //     belongs to the one of four levels (8, 4, 2, 1) at which t is in the upper and s in the lower half of the same block of rows; left
 //     rows carry the decay from the middle to t, right rows from s to the middle, both at most 1, and one wave's MFMAs make a
-//     level's products.  The triangular system is solved by a thread per column.
+//     level's products.  The triangular system is solved by a thread per column.  Products of decays are made in fp64 and rounded once.
 //   walk (a wave per 16 value columns, head and request)     three products a chunk.  An accumulator's layout of the 16x16x4 MFMA is the
 //     layout of its right operand when lane group g holds elements 4 g .. 4 g + 3 of 16 and MFMA r multiplies the r-th ones: S and X go
 //     from product to product in registers, without LDS, barriers or shuffles.  The next chunk's factors are loaded as
@@ -21,7 +21,11 @@
 // What bounds the row-by-row forms is a chain of LDS reads, sums over lanes and updates per row, 0.5 us (128 x 128) or 0.7 us (64 x 64); a
 // chunk's chain here is its MFMAs and the two kernels' traffic over the factors, which stay in the last-level cache for as many chunks
 // as are made at a time.  Row by row against this (16 heads; outputs' norm included), gated 128 x 128 and generalized 64 x 64:
-//   1 request of 2048 rows:  640 -> 376 us, 1590 -> 287 us       9 of 1500:  1060 -> 687 us, 1410 -> 400 us
+//   1 request of 2048 rows:  640 -> 388 us, 1590 -> 290 us       9 of 1500:  1060 -> 702 us, 1410 -> 410 us
+// Error against 64 bits (2-norm; 1500 rows of 64 x 64, 700 of 128 x 128), row by row and here: gated outputs 1.13e-7 and 1.12e-7 with strong
+// decays, 1.67e-7 .. 1.69e-7 and 1.51e-7 .. 1.54e-7 with weak ones, generalized 1.83e-7 .. 1.88e-7 and 1.65e-7 .. 1.69e-7; states 0.58e-7 .. 1.66e-7
+// and 0.54e-7 .. 1.37e-7.  It takes sums of 16 terms joined by trees, decays rounded once, a state that is rounded once a chunk and
+// (gated) diagonals outside the MFMAs; without these it was up to 13% above the rows' (and 3% faster).
 #include "seq_common.h"
 #include "fls_seq.h"
 
@@ -141,31 +145,31 @@ __global__ __launch_bounds__(256, GEN ? 2 : 3) void delta_factors_kernel(Delta a
       const int b = 8 >> l;
 #pragma unroll
       for (int m0 = 0; m0 < CH; m0 += 2 * b) {
-        float z = 1.f;
+        double z = 1.0;
 #pragma unroll
-        for (int t = m0 + b; t < m0 + 2 * b; ++t) { z *= g[t]; Z[l][t * LD + ch] = z; }
-        z = 1.f;
+        for (int t = m0 + b; t < m0 + 2 * b; ++t) { z *= g[t]; Z[l][t * LD + ch] = (float)z; }
+        z = 1.0;
 #pragma unroll
-        for (int t = m0 + b - 1; t >= m0; --t) { Z[l][t * LD + ch] = z; z *= g[t]; }
+        for (int t = m0 + b - 1; t >= m0; --t) { Z[l][t * LD + ch] = (float)z; z *= g[t]; }
       }
     }
     if (part == PARTS - 1) {
-      float z = 1.f;
+      double z = 1.0;
 #pragma unroll
       for (int t = 0; t < CH; ++t) {
-        const float before = z;
+        const double before = z;
         z *= g[t];
-        kp[t] = K[t * LD + ch] * (GEN ? before : z);
-        fac[L::QP + (ch >> 4) * 256 + frag(t, ch & 15)] = Q[t * LD + ch] * z;
+        kp[t] = (float)(K[t * LD + ch] * (GEN ? before : z));
+        fac[L::QP + (ch >> 4) * 256 + frag(t, ch & 15)] = (float)(Q[t * LD + ch] * z);
       }
-      fac[L::P + ch] = z;
-      z = 1.f;
+      fac[L::P + ch] = (float)z;
+      z = 1.0;
       floatx4 l1[4], l2[4];
 #pragma unroll
       for (int t = CH - 1; t >= 0; --t) {
-        const float k = K[t * LD + ch] * z;
+        const float k = (float)(K[t * LD + ch] * z);
         l2[t >> 2][t & 3] = k;
-        if constexpr (GEN) l1[t >> 2][t & 3] = -R[t * LD + ch] * z;
+        if constexpr (GEN) l1[t >> 2][t & 3] = (float)(-R[t * LD + ch] * z);
         z *= g[t];
       }
 #pragma unroll
@@ -180,11 +184,14 @@ __global__ __launch_bounds__(256, GEN ? 2 : 3) void delta_factors_kernel(Delta a
     const int fr = lane & 15, grp = lane >> 4, b = 8 >> wave;
     const bool up = (fr & b) != 0, first = (fr & (b - 1)) == 0;
     const floatx4 zero = {0.f, 0.f, 0.f, 0.f}, one = {1.f, 1.f, 1.f, 1.f};
-    floatx4 sA[4] = {zero, zero, zero, zero}, sB[4] = {zero, zero, zero, zero}, sAk[4] = {zero, zero, zero, zero}, sBk[4] = {zero, zero, zero, zero};
-#pragma unroll 4
-    for (int j = 0; j < D / 16; ++j) {
+    constexpr int J = D / 16;
+    floatx4 sA[J], sB[J], sAk[J], sBk[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) sA[j] = sB[j] = sAk[j] = sBk[j] = zero;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
       const int e = fr * LD + 16 * j + 4 * grp;
-      floatx4 &accA = sA[j & 3], &accB = sB[j & 3], &accAk = sAk[j & 3], &accBk = sBk[j & 3];
+      floatx4 &accA = sA[j], &accB = sB[j], &accAk = sAk[j], &accBk = sBk[j];
       const floatx4 z = wave < 3 ? *reinterpret_cast<const floatx4*>(&Z[wave][e]) : up ? *reinterpret_cast<const floatx4*>(G + e) : one, k = *reinterpret_cast<const floatx4*>(K + e),
                     q = *reinterpret_cast<const floatx4*>(Q + e);
       if constexpr (GEN) {
@@ -201,8 +208,11 @@ __global__ __launch_bounds__(256, GEN ? 2 : 3) void delta_factors_kernel(Delta a
         accB = mfma16(lb, ra, accB);
       }
     }
-    const floatx4 accA = (sA[0] + sA[1]) + (sA[2] + sA[3]), accB = (sB[0] + sB[1]) + (sB[2] + sB[3]),
-                  accAk = (sAk[0] + sAk[1]) + (sAk[2] + sAk[3]), accBk = (sBk[0] + sBk[1]) + (sBk[2] + sBk[3]);
+#pragma unroll
+    for (int d = J / 2; d > 0; d /= 2)
+#pragma unroll
+      for (int j = 0; j < d; ++j) { sA[j] += sA[j + d]; sB[j] += sB[j + d]; sAk[j] += sAk[j + d]; sBk[j] += sBk[j + d]; }
+    const floatx4 accA = sA[0], accB = sB[0], accAk = sAk[0], accBk = sBk[0];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int t = 4 * grp + r;
@@ -321,13 +331,26 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
     const auto at = [&](int off) { return *reinterpret_cast<const floatx4*>(F + off); };
     // (each product's operands are read from LDS while the one before runs: the barriers keep the reads where they stand)
     floatx4 m1[J], qp[J], l1[J], l2[GEN ? J : 1];
-    const floatx4 n1 = at(L::N1), b = at(L::B), bk = GEN ? at(L::BK) : zero;
+    // (gated: N1 and B without their diagonals, which enter by a multiply-add of their own.  They are the largest terms where decays are
+    // strong, and a MFMA rounds each product)
+    const auto lower = [&](int off) {
+      floatx4 m = at(off);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) m[r] = 4 * grp + r == fr ? 0.f : m[r];
+      return m;
+    };
+    const auto add_diagonal = [&](int off, const floatx4& y, floatx4 c) {      // of this lane's rows 4 grp + r
+#pragma unroll
+      for (int r = 0; r < 4; ++r) c[r] = __builtin_fmaf(fs[buf][off + frag(4 * grp + r, 4 * grp + r)], y[r], c[r]);
+      return c;
+    };
+    const floatx4 n1 = GEN ? at(L::N1) : lower(L::N1), b = GEN ? at(L::B) : lower(L::B), bk = GEN ? at(L::BK) : zero;
 #pragma unroll
     for (int j = 0; j < J; ++j) m1[j] = at(256 * j);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < J; ++j) qp[j] = at(L::QP + 256 * j);
-    floatx4 X, x[J], o[J];                                     // (short sums, then a tree: as exact as the row-by-row kernels' sums over lanes)
+    floatx4 X, x[J], o[J];                                     // (short sums, then a tree, like the row-by-row kernels' sums over lanes)
 #pragma unroll
     for (int j = 0; j < J; ++j) x[j] = mfma16(m1[j], S[j], zero);
     X = mfma16(n1, v, zero);
@@ -344,23 +367,32 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
 #pragma unroll
       for (int j = 0; j < d; ++j) { x[j] += x[j + d]; o[j] += o[j + d]; }
     X += x[0];
-    if constexpr (GEN) O = mfma16(b, X, zero) + (mfma16(bk, v, zero) + o[0]);
-    else O = mfma16(b, X, zero) + o[0];
+    if constexpr (GEN) {
+      O = mfma16(b, X, zero) + (mfma16(bk, v, zero) + o[0]);
+    } else {
+      X = add_diagonal(L::N1, v, X);
+      O = add_diagonal(L::B, X, mfma16(b, X, zero) + o[0]);
+    }
     bool odd = false;                                          // (zeros above the diagonals would spread a later row's inf or NaN)
 #pragma unroll
     for (int r = 0; r < 4; ++r) odd |= !__builtin_isfinite(v[r]) | !__builtin_isfinite(X[r]);
     if (__any(odd)) {
-      X = below<!GEN>(fs[buf] + L::N1, n1, v) + x[0];
-      if constexpr (GEN) o[0] += below<true>(fs[buf] + L::BK, bk, v);
-      O = below<true>(fs[buf] + L::B, b, X) + o[0];
+      X = below<false>(fs[buf] + L::N1, n1, v) + x[0];         // (GEN: N1 has no diagonal)
+      if constexpr (GEN) {
+        O = below<true>(fs[buf] + L::B, b, X) + (below<true>(fs[buf] + L::BK, bk, v) + o[0]);
+      } else {
+        X = add_diagonal(L::N1, v, X);
+        O = add_diagonal(L::B, X, below<false>(fs[buf] + L::B, b, X) + o[0]);
+      }
     }
-#pragma unroll
-    for (int j = 0; j < J; ++j) S[j] *= *reinterpret_cast<const floatx4*>(fs[buf] + L::P + 16 * j + 4 * grp);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < J; ++j) {
-      S[j] = mfma16(l1[j], X, S[j]);
-      if constexpr (GEN) S[j] = mfma16(l2[j], v, S[j]);
+    for (int j = 0; j < J; ++j) {                              // (the chunk's sum first: one rounding at the state's size)
+      const floatx4 P = *reinterpret_cast<const floatx4*>(fs[buf] + L::P + 16 * j + 4 * grp);
+      floatx4 u = mfma16(l1[j], X, zero);
+      if constexpr (GEN) u = mfma16(l2[j], v, u);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[j][r] = __builtin_fmaf(S[j][r], P[r], u[r]);
     }
   }
   if (!live) return;

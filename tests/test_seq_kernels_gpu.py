@@ -525,6 +525,45 @@ def test_delta_chunks(ops, monkeypatch, lens, pos0, d, dv, heads, kv, small):
             close(x, y, 1e-5)
 
 
+# the chunked delta rules are no further from 64 bits than the row-by-row kernels (both repeat themselves exactly; 3% for another card's sums)
+@pytest.mark.parametrize("n,d", [(700, 128), (900, 64)])
+@pytest.mark.parametrize("power", [3.0, 0.05])
+def test_delta_chunks_are_as_exact_as_rows(ops, monkeypatch, n, d, power):
+    H, _ = ops
+    torch.manual_seed(n)
+    h = 2
+    hd, unit, f64 = h * d, lambda x: x / (x.pow(2).sum(-1, keepdim=True) + 1e-6).sqrt(), lambda t: t.double().reshape(n, h, -1)
+    md, _, nslots = meta_of([n], [0], DEV)
+    qkv, beta, gate = torch.randn(n, 3 * hd, device=DEV), torch.randn(n, h, device=DEV), torch.zeros(n, hd, device=DEV)
+    dec, nw = torch.rand(n, hd, device=DEV) ** power, torch.ones(d, device=DEV)
+    z, w0, nw2 = torch.randn(n, 6 * hd, device=DEV), torch.randn(hd, device=DEV) - 2, torch.ones(hd, device=DEV)
+    parts = [z[:, i * hd:(i + 1) * hd] for i in range(6)]
+    q6, k6, v6, b6, g6 = unit(f64(qkv[:, :hd])) * d ** -0.5, unit(f64(qkv[:, hd:2 * hd])), f64(qkv[:, 2 * hd:]), torch.sigmoid(beta.double()), f64(dec)
+    r7, k7, v7, a7 = f64(parts[0]), f64(parts[1]), f64(parts[2]), torch.sigmoid(f64(parts[3]))
+    w7, u7 = torch.exp(-0.6065 * torch.sigmoid(f64(parts[4]) + w0.double().reshape(h, d))), unit(k7)
+    S, S2 = torch.zeros(h, d, d, device=DEV).double(), torch.zeros(h, d, d, device=DEV).double()
+    o6, o7 = torch.empty(n, h, d, device=DEV).double(), torch.empty(n, h, d, device=DEV).double()
+    for t in range(n):
+        S = S * g6[t][:, None, :]
+        S = S + (b6[t][:, None] * (v6[t] - (S * k6[t][:, None, :]).sum(-1)))[:, :, None] * k6[t][:, None, :]
+        o6[t] = (S * q6[t][:, None, :]).sum(-1)
+        x = (S2 * u7[t][:, :, None]).sum(1)
+        S2 = w7[t][:, :, None] * S2 - (a7[t] * u7[t])[:, :, None] * x[:, None, :] + k7[t][:, :, None] * v7[t][:, None, :]
+        o7[t] = (S2 * r7[t][:, :, None]).sum(1)
+    norm = lambda o: (o / (o.pow(2).mean(-1, keepdim=True) + 1e-5).sqrt()).reshape(n, -1)
+    want = (norm(o6) * 0.5, S, norm(o7) * torch.sigmoid(parts[5].double()), S2)
+    err = []
+    for rows in (10 ** 9, 1):
+        monkeypatch.setattr(H, "DELTA_CHUNK_ROWS", rows)
+        monkeypatch.setattr(H, "GATED_CHUNK_ROWS", rows)
+        s1, s2, out = torch.zeros(nslots, h, d, d, device=DEV), torch.zeros(nslots, h, d, d, device=DEV), torch.empty(n, hd, device=DEV)
+        got = H.gated_delta_scan(qkv, beta, dec, gate, nw, s1, md, h, h, d, d, 1e-6, 1e-5, torch.float32)
+        H.delta_rule_scan(*parts, w0, nw2, s2, md, h, d, decay_scale=0.6065, key_eps=1e-6, norm_eps=1e-5, out_scale=1.0, out=out)
+        slot = int(md["slot"][0])
+        err.append([float((x.double() - y).norm() / y.norm()) for x, y in zip((got, s1[slot], out, s2[slot]), want)])
+    assert all(c <= 1.03 * r for r, c in zip(*err)), err
+
+
 # the same of the chunked delta rules: a value that is not finite changes no row before its own, no other request and no other head
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("d,heads", [(64, 2), (128, 3)])
