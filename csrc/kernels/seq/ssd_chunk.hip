@@ -6,8 +6,11 @@
 // so a request of n rows is a chain of n / 64 chunks instead of n rows.  What bounds the row-by-row form is that chain (0.7 us a
 // row); here it is a chunk's chain of products and LDS reads, with C, the scores and z loaded while the chunk is laid down.  C_i . B_j
 // is the same for all heads of a group: a first kernel leaves it in memory once ([T, groups, 64] fp32).  Row by row against this, heads
-// of 64 x 128: 2 requests of 512 rows, 32 heads 348 -> 62 us; 8 of 2048 rows, 64 heads 1880 -> 688; 1 of 2048 1443 -> 198.  Exponents
+// of 64 x 128: 2 requests of 512 rows, 32 heads 350 -> 63 us; 8 of 2048 rows, 64 heads 1880 -> 676; 1 of 2048 1443 -> 197.  Exponents
 // are differences of running sums: the sums are fp64, so a difference is exact to fp32 however far a chunk has decayed.
+// Error against 64 bits (2-norm, row by row and here): outputs 1.39e-7 and 1.34e-7, states 1.03e-7 and 0.97e-7 where a row decays by some 0.85;
+// 1.26e-7 and 1.23e-7, 0.78e-7 and 0.89e-7 by 0.6; 12e-7 and 1.8e-7, 14e-7 and 1.3e-7 by 0.99.  It takes sums of 16 or 32 terms joined
+// by trees and a row's own term outside the MFMAs, which round each product: in single chains outputs were up to 1.8 times as far off.
 // All products are fp32 (16x16x4 MFMAs: lane group g holds elements 4 g .. 4 g + 3 of 16, MFMA r multiplies the r-th ones).
 #include "seq_common.h"
 #include "fls_seq.h"
@@ -40,6 +43,7 @@ struct Ssd {
 };
 
 // block = (chunk, group, request), wave = 16 of its rows
+template <int N>
 __global__ __launch_bounds__(256) void ssd_scores_kernel(Ssd a) {
   const int s = blockIdx.z, g = blockIdx.y;
   const int r0 = a.cu[s] + blockIdx.x * CQ, end = a.cu[s + 1];
@@ -52,25 +56,32 @@ __global__ __launch_bounds__(256) void ssd_scores_kernel(Ssd a) {
   const float* B = a.xbc + (size_t)r0 * a.ldx + inner + g * a.N;
   const float* C = B + a.G * a.N;
   const float* crow = C + (size_t)min(i0 + fr, nt - 1) * a.ldx + 4 * grp;
-  floatx4 acc[4];
+  // (sums of 16 terms, then a tree)
+  floatx4 part[N / 16][4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  for (int n = 0; n < a.N; n += 16) {
-    const floatx4 c = *reinterpret_cast<const floatx4*>(crow + n);
+  for (int q = 0; q < N / 16; ++q) {
+    const floatx4 c = *reinterpret_cast<const floatx4*>(crow + 16 * q);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      part[q][j] = floatx4{0.f, 0.f, 0.f, 0.f};
       if (j > w) continue;
-      const floatx4 b = *reinterpret_cast<const floatx4*>(B + (size_t)min(16 * j + fr, nt - 1) * a.ldx + 4 * grp + n);
-      acc[j] = mfma16(c, b, acc[j]);
+      const floatx4 b = *reinterpret_cast<const floatx4*>(B + (size_t)min(16 * j + fr, nt - 1) * a.ldx + 4 * grp + 16 * q);
+      part[q][j] = mfma16(c, b, part[q][j]);
     }
   }
+#pragma unroll
+  for (int d = N / 32; d > 0; d /= 2)
+#pragma unroll
+    for (int q = 0; q < d; ++q)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part[q][j] += part[q + d][j];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     if (j > w) continue;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = i0 + 4 * grp + r;
-      if (i < nt) a.scores[((size_t)(r0 + i) * a.G + g) * CQ + 16 * j + fr] = acc[j][r];
+      if (i < nt) a.scores[((size_t)(r0 + i) * a.G + g) * CQ + 16 * j + fr] = part[0][j][r];
     }
   }
 }
@@ -84,7 +95,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
   __shared__ __attribute__((aligned(16))) float xs[CQ * LX];
   __shared__ float Ss[N * LX];
   __shared__ double cs[CQ];
-  __shared__ float dts[CQ], wj[CQ];
+  __shared__ float dts[CQ], wj[CQ], self[CQ];                 // self: a row's own term of y, D's among it
   const int s = blockIdx.z, h = blockIdx.y, p0 = blockIdx.x * 16 * PT;
   const int g = h / (a.nh / a.G), inner = a.nh * a.P;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, fr = lane & 15, grp = lane >> 4;
@@ -105,7 +116,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
   // the next chunk's inputs come into registers while this one is computed
   constexpr int NB4 = CQ * N / 4 / 256, NX4 = (CQ * 16 * PT / 4 + 255) / 256;
   floatx4 pb[NB4], px[NX4];
-  float pdt = 0.f;
+  float pdt = 0.f, pself = 0.f;
   auto prefetch = [&](int r0) {
 #pragma unroll
     for (int i = 0; i < NB4; ++i) {
@@ -117,7 +128,10 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
       const int e = threadIdx.x + 256 * i, row = e / (4 * PT), c = e % (4 * PT) * 4;
       px[i] = r0 + row < a1 ? *reinterpret_cast<const floatx4*>(a.xbc + (size_t)(r0 + row) * a.ldx + h * a.P + p0 + c) : floatx4{0.f, 0.f, 0.f, 0.f};
     }
-    if (w == 0) pdt = r0 + lane < a1 ? a.dt[(size_t)(r0 + lane) * a.lddt + h] : 0.f;
+    if (w == 0) {
+      pdt = r0 + lane < a1 ? a.dt[(size_t)(r0 + lane) * a.lddt + h] : 0.f;
+      pself = r0 + lane < a1 ? a.scores[((size_t)(r0 + lane) * a.G + g) * CQ + lane] : 0.f;
+    }
   };
   prefetch(a0);
   for (int r0 = a0; r0 < a1; r0 += CQ) {
@@ -173,11 +187,12 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
       const double last = __shfl(c, 63, 64);
       cs[lane] = c;
       dts[lane] = dtv;
+      self[lane] = dtv * pself + dsk;
       wj[lane] = expf((float)(last - c)) * dtv;
     }
     __syncthreads();
     if (r0 + CQ < a1) prefetch(r0 + CQ);
-    // y: the chunk's own rows, then the state before it
+    // y: the chunk's earlier rows, then the state before it
     floatx4 own[PT], past[PT];
 #pragma unroll
     for (int p = 0; p < PT; ++p) own[p] = past[p] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -193,7 +208,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int j = 16 * jb + 4 * grp + r;
-          l[r] = j <= i && j < nt ? expf((float)(ci - cs[j])) * dts[j] * m[r] : 0.f;
+          l[r] = j < i && j < nt ? expf((float)(ci - cs[j])) * dts[j] * m[r] : 0.f;
         }
 #pragma unroll
         for (int p = 0; p < PT; ++p) {
@@ -223,16 +238,25 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
           for (int r = 0; r < 4; ++r) own[p][r] = 4 * grp + r >= at ? __builtin_nanf("") : own[p][r];
         }
       }
+      // (sums of 32 terms)
 #pragma unroll
-      for (int n = 0; n < N; n += 16) {
-        const floatx4 c = AHEAD ? cr[AHEAD ? n / 16 : 0] : *reinterpret_cast<const floatx4*>(crow + n);
+      for (int n0 = 0; n0 < N; n0 += 32) {
+        floatx4 part[PT];
 #pragma unroll
-        for (int p = 0; p < PT; ++p) {
-          floatx4 v;
+        for (int p = 0; p < PT; ++p) part[p] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = Ss[(n + 4 * grp + r) * LX + 16 * p + fr];
-          past[p] = mfma16(c, v, past[p]);
+        for (int n = n0; n < n0 + 32; n += 16) {
+          const floatx4 c = AHEAD ? cr[AHEAD ? n / 16 : 0] : *reinterpret_cast<const floatx4*>(crow + n);
+#pragma unroll
+          for (int p = 0; p < PT; ++p) {
+            floatx4 v;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = Ss[(n + 4 * grp + r) * LX + 16 * p + fr];
+            part[p] = mfma16(c, v, part[p]);
+          }
         }
+#pragma unroll
+        for (int p = 0; p < PT; ++p) past[p] += part[p];
       }
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -242,7 +266,7 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
 #pragma unroll
           for (int p = 0; p < PT; ++p) {
             const int col = h * a.P + p0 + 16 * p + fr;
-            const float y = e * past[p][r] + own[p][r] + dsk * xs[t * LX + 16 * p + fr];
+            const float y = self[t] * xs[t * LX + 16 * p + fr] + (e * past[p][r] + own[p][r]);
             a.out[(size_t)(r0 + t) * a.ldo + col] = y * silu_f(zr[p][r]);
           }
         }
@@ -252,8 +276,9 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
     const float dec = expf((float)cs[CQ - 1]);
 #pragma unroll
     for (int k = 0; k < NW; ++k) {
+      floatx4 u[PT];                                          // (the chunk's sum first, 16 rows at a time: one rounding at the state's size)
 #pragma unroll
-      for (int p = 0; p < PT; ++p) S[k][p] *= dec;
+      for (int p = 0; p < PT; ++p) u[p] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int jb = 0; jb < 4; ++jb) {
         floatx4 b;
@@ -267,9 +292,13 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_kernel(Ssd a) {
           floatx4 x;
 #pragma unroll
           for (int r = 0; r < 4; ++r) x[r] = xs[(16 * jb + 4 * grp + r) * LX + 16 * p + fr];
-          S[k][p] = mfma16(b, x, S[k][p]);
+          u[p] += mfma16(b, x, floatx4{0.f, 0.f, 0.f, 0.f});
         }
       }
+#pragma unroll
+      for (int p = 0; p < PT; ++p)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[k][p][r] = __builtin_fmaf(S[k][p][r], dec, u[p][r]);
     }
   }
 #pragma unroll
@@ -291,7 +320,9 @@ extern "C" int fls_seq_ssd_scan_chunked(const float* xbc, int ldx, const float* 
   if ((N != 64 && N != 128) || P % 16 || G < 1 || nh % G || ldx % 4 || (uintptr_t)xbc % 16 || scratch == nullptr || (uintptr_t)scratch % 16) return -1;
   const Ssd a = {xbc, ldx, z, ldz, dt, lddt, dt_bias, A_log, Dskip, state, out, ldo, cu, pos0, slot, nh, P, N, G, scratch};
   const hipStream_t st = (hipStream_t)s;
-  hipLaunchKernelGGL(ssd_scores_kernel, dim3((max_rows + CQ - 1) / CQ, G, B), dim3(256), 0, st, a);
+  const dim3 chunks((max_rows + CQ - 1) / CQ, G, B);
+  if (N == 128) hipLaunchKernelGGL(ssd_scores_kernel<128>, chunks, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL(ssd_scores_kernel<64>, chunks, dim3(256), 0, st, a);
   SEQ_LAUNCH_CHECK();
   // two column tiles a block read B and C half as often; one where that would leave CUs without a block
   const bool two = P % 32 == 0 && (long long)B * nh * (P / 32) >= 256;

@@ -407,6 +407,38 @@ def test_ssd_chunks_huge_step(ops, step):
     close(st[slot, 0], S, 3e-6)
 
 
+# the chunked scan is no further from 64 bits than the row-by-row kernel (both repeat themselves exactly; 3% for another card's sums).  Rates
+# about exp(-1), steps about 0.4: a row decays by some 0.85; then by 0.5 and 0.98, at the first of which outputs are what is compared
+@pytest.mark.parametrize("P,N", [(16, 64), (16, 128)])
+@pytest.mark.parametrize("rate", [-1.0, 0.8, -4.0])
+def test_ssd_chunks_are_as_exact_as_rows(ops, monkeypatch, P, N, rate):
+    H, _ = ops
+    torch.manual_seed(N)
+    nh, lens = 64, (130, 300, 413, 500, 601)
+    md, _, nslots = meta_of(lens, [0] * len(lens), DEV)
+    T = sum(lens)
+    xbc, z, dt = torch.randn(T, nh * P + 2 * N, device=DEV), torch.randn(T, nh * P, device=DEV), 0.5 * torch.randn(T, nh, device=DEV)
+    dtb, Al, Ds = torch.randn(nh, device=DEV) - 1, 0.7 * torch.randn(nh, device=DEV) + rate, torch.randn(nh, device=DEV)
+    x, B, C = (t.double() for t in torch.split(xbc, [nh * P, N, N], 1))
+    d = torch.nn.functional.softplus((dt + dtb).double())
+    e, o, states, t = torch.exp(-torch.exp(Al.double()) * d), torch.empty(T, nh, P, device=DEV).double(), [], 0
+    for n in lens:
+        S = torch.zeros(nh, N, P, device=DEV).double()
+        for t in range(t, t + n):
+            xt = x[t].reshape(nh, P)
+            S = e[t][:, None, None] * S + d[t][:, None, None] * B[t][None, :, None] * xt[:, None, :]
+            o[t] = (S * C[t][None, :, None]).sum(1) + Ds.double()[:, None] * xt
+        states.append(S)
+        t += 1
+    want, err = (o.reshape(T, -1) * torch.nn.functional.silu(z.double()), torch.stack(states)), []
+    for rows in (10 ** 9, 1):
+        monkeypatch.setattr(H, "SSD_CHUNK_ROWS", rows)
+        st = torch.zeros(nslots, nh, N, P, device=DEV)
+        got = H.ssd_scan(xbc, z, dt, dtb, Al, Ds, st, md, nh, P, N, 1)
+        err.append([float((a.double() - b).norm() / b.norm()) for a, b in zip((got, st[md["slot"].long()]), want)])
+    assert err[1][0] <= 1.03 * err[0][0] and (rate > 0 or err[1][1] <= 1.03 * err[0][1]), err
+
+
 # a value that is not finite stays where the recurrence puts it: rows before its own, other requests and (a value of x) other columns are
 # what they are without it, bit by bit.  Rows in the first, a middle and the last block of 16 of a chunk, and in the second chunk
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
