@@ -46,28 +46,6 @@ __device__ __forceinline__ float epi_gate(float g, float u, const Epi& e) {
   u = fminf(fmaxf(u, -e.p), e.p);
   return g / (1.f + expf(-e.q * g)) * (u + 1.f);
 }
-// The same for results that are rounded to bf16 (2^-9): the hardware's exponential and reciprocal (1 ulp each, the exponent's product
-// with log2(e) adding |x| 2^-24 relative) stay far inside that rounding and take a quarter of the instructions.  xIELU's
-// exp(z) - 1 - z cancels near 0, where it is a polynomial (next term below 1e-9 of the result at -1/2).  256 x 256 tiles, one block a
-// CU, so nothing hides the epilogue: 7903 x 10880 x 2048 gelu gate 391 -> 356 us, 9692 x 10880 x 2048 silu gate 449 -> 396, 16384 x
-// 14336 x 4096 xIELU 1859 -> 1716.
-__device__ __forceinline__ float exp_hw(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
-__device__ __forceinline__ float sigmoid_hw(float x) { return __builtin_amdgcn_rcpf(1.f + exp_hw(-x)); }
-__device__ __forceinline__ float epi_value_bf16(float v, const Epi& e, const EpiRegs& r) {
-  if (e.kind == EPI_XIELU) {
-    const float poly = v * v * (0.5f + v * (1.f / 6 + v * (1.f / 24 + v * (1.f / 120 + v * (1.f / 720 + v * (1.f / 5040 + v * (1.f / 40320)))))));
-    const float low = v > -0.5f ? poly : exp_hw(v) - 1.f - v;
-    return (v > 0.f ? r.ap * v * v : r.an * low) + 0.5f * v;
-  }
-  return epi_value(v, e, r);
-}
-__device__ __forceinline__ float epi_gate_bf16(float g, float u, const Epi& e) {
-  if (e.kind == EPI_GATE) return g * sigmoid_hw(g) * u;
-  if (e.kind == EPI_GATE + 1) return g * sigmoid_hw(1.5957691216057308f * (g + 0.044715f * g * g * g)) * u;
-  g = fminf(g, e.p);
-  u = fminf(fmaxf(u, -e.p), e.p);
-  return g * sigmoid_hw(e.q * g) * (u + 1.f);
-}
 __device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e, const EpiRegs& r) {
   v = epi_value(v, e, r);
   if (e.tc == 1) reinterpret_cast<bf16_t*>(C)[idx] = f_to_bf16(v);

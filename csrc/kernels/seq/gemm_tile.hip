@@ -217,7 +217,7 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
         const floatx4 u = *reinterpret_cast<const floatx4*>(lds + (r * CH + ((cg + 4) ^ (r & (CH - 1)))) * 16);
         floatx4 v;
 #pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = TC == 1 ? epi_gate_bf16(g[x], u[x], e) : epi_gate(g[x], u[x], e);
+        for (int x = 0; x < 4; ++x) v[x] = epi_gate(g[x], u[x], e);
         const int m = mw + p * PU * 16 + r;
         if (m < mend && n < (a.N >> 1)) store4<TC>(a.C, (size_t)m * a.ldc + n, v);
       }
@@ -242,7 +242,7 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
       const int r = i + lane / CH;
       floatx4 v = *reinterpret_cast<const floatx4*>(lds + (r * CH + (c ^ (r & (CH - 1)))) * 16) + b;
 #pragma unroll
-      for (int x = 0; x < 4; ++x) v[x] = TC == 1 ? epi_value_bf16(v[x], e, er[x]) : epi_value(v[x], e, er[x]);
+      for (int x = 0; x < 4; ++x) v[x] = epi_value(v[x], e, er[x]);
       const int m = mw + p * PU * 16 + r;
       if (m < mend && n < a.N) store4<TC>(a.C, cbase + (size_t)m * a.ldc + n, v);
     }

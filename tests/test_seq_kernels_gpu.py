@@ -307,6 +307,29 @@ def test_epilogue_bf16_values(ops, kind):
     assert bool((err <= want[:, None].abs() * 2 ** -8 + (1 + (z6 * (u6.abs() + 1)).abs())[:, None] * 2.0 ** -126).all())
 
 
+# an activation of the same sum has the same bits from the few-row kernel, the tiles and the kernels for any size (every sum here is one
+# product, exact in any order)
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_epilogue_values_do_not_depend_on_the_rows(ops, out):
+    H, _ = ops
+    g = torch.Generator().manual_seed(6)
+    M, N, K = 2080, 256, 64
+    z, u = (3 * torch.randn(M, generator=g)).bfloat16(), torch.randn(N, generator=g).abs().bfloat16()
+    a, w = torch.zeros(M, K, dtype=torch.bfloat16), torch.zeros(2 * N, K, dtype=torch.bfloat16)
+    a[:, 0], a[:, 1], w[:N, 0], w[N:, 1] = z, z.flip(0), 1 + u / 8, u
+    a, w, act = a.to(DEV), w.to(DEV), torch.tensor([0.3, -0.2], device=DEV)
+    ragged = torch.zeros(M, K + 3, dtype=torch.bfloat16, device=DEV)[:, :K]
+    ragged.copy_(a)
+    for how in (dict(xielu=act), dict(relu2=True), dict(softcap=3.0), dict(scale=0.3), dict(decay=act)):
+        f = lambda x: H.matmul_nt(x, w, out_dtype=out, **how)
+        whole = f(a)
+        assert torch.equal(whole, torch.cat([f(a[i:i + 32]) for i in range(0, M, 32)])) and torch.equal(whole, f(ragged)), how
+    for kind in ("silu", "gelu_tanh", "clamped"):
+        f = lambda x: H.gated_matmul_nt(x, w, out, act=kind, limit=7.0)
+        whole = f(a)
+        assert torch.equal(whole, torch.cat([f(a[i:i + 32]) for i in range(0, M, 32)])) and torch.equal(whole, f(ragged)), kind
+
+
 # plain products of few columns that four-column stores don't fit: one column at a time from the tiles, rows about a tile's, all three
 # operand types; sums of 256 products against fp64
 @pytest.mark.parametrize("N", [1, 3, 10, 33, 62, 127])
