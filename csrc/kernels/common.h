@@ -52,8 +52,7 @@ __device__ __forceinline__ float warp_sum(float v) {
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
-// (every result is rounded to fp16: the hardware's reciprocal, 1 ulp, for the division's nine more instructions)
-__device__ __forceinline__ float silu(float x) { return x * __builtin_amdgcn_rcpf(1.0f + __expf(-x)); }
+__device__ __forceinline__ float silu(float x) { return x / (1.0f + __expf(-x)); }
 
 #define FLS_CHECK_LAUNCH()                                  \
   do {                                                      \

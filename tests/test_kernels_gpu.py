@@ -50,6 +50,21 @@ def test_gemm_plain(ops, M, N, K):
     assert rel_err(y, r) < 2e-3
 
 
+# SwiGLU bit for bit as x / (1 + exp(-x)) times up in fp32, rounded once: every sum here is one product, exact in fp32 (few rows, middle and
+# large tiles; exp as 2^(-x log2 e), which is what the hardware's exponential is)
+@pytest.mark.parametrize("M", [8, 100, 2048])
+def test_swiglu_divides(ops, M):
+    I, K = 2048, 64
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.zeros(M, K, dtype=torch.float16), torch.zeros(2 * I, K, dtype=torch.float16)
+    x[:, 0], x[:, 1] = torch.randn(M, generator=g).half() * 2, torch.randn(M, generator=g).half()
+    w[:I, 0], w[I:, 1] = torch.randn(I, generator=g).half(), torch.randn(I, generator=g).half()
+    x, w = x.to(DEV), w.to(DEV)
+    gate, up = x[:, :1].float() * w[:I, 0].float(), x[:, 1:2].float() * w[I:, 1].float()
+    want = gate / (1.0 + torch.exp2(-gate * 1.4426950408889634)) * up
+    assert torch.equal(ops.swiglu_up(x, w), want.half())
+
+
 def test_gemm_asymmetric_exact(ops):
     # A = identity-like, asymmetric B: catches transposed C writes (guide §3 check)
     M = N = K = 256
