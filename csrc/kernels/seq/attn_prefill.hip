@@ -24,12 +24,15 @@
 //                      per-lane multiply.
 //
 // What bounds it is the vector work per score beside the matrix work (24 MFMAs, 768 cycles, per half tile and wave with heads of
-// 128).  So scores are in units of log 2: exp and log are one instruction each and the penalty needs no factor.  The cap's
-// quotient is a reciprocal, bf16 terms come from the conversion instruction, and a half tile that every row of the wave sees
-// has no mask.  The accumulators are rescaled only when a maximum has grown by more than 8: weights stay below 2^8, which fp32
-// sums and two-term weights hold as exactly.  Tiles of 64 keys halve the barriers, and two keys of V make one 4-byte LDS store.
-// Measured against tiles of 32 with a rescale and a mask for every score:
-//   cap and distance penalty, 48 heads of 128:   2033 -> 988 us      fp32 queries, 9 layers' mean:   426 -> 222 and 317 -> 156 us
+// 128).  So scores are in units of log 2: exp and log are one instruction each and the penalty needs no factor.  The cap and the
+// sigmoid weights come from exp(-|x|) and a reciprocal of [1, 2] that one Newton step makes as exact as a division (divisions: 468 us where
+// this takes 446; 172 and 194 with heads of 64).  bf16 terms come from the conversion instruction, and a half tile that every row of the
+// wave sees has no mask.  The accumulators are rescaled when a maximum grows, and only then: a query's largest weight is exactly 1,
+// which two bf16 terms hold without error (left up to 2^8 behind the maximum, outputs were up to twice as far from 64 bits, for 4% of
+// the time).  Tiles of 64 keys halve the barriers, and two keys of V make one 4-byte LDS store.
+// Measured against tiles of 32 with a rescale and a mask for every score, 4 prompts of 1500, 48 heads of 128 on 8 keys' heads:
+//   plain 815 -> 415 us     cap 890 -> 446     cap and distance penalty 890 -> 461     sigmoid weights 825 -> 375
+// and 6 of 1500, 16 heads of 64 on 4:   300 -> 135, 355 -> 172, 356 -> 195, 319 -> 141 us
 #include "seq_common.h"
 #include "fls_seq.h"
 
@@ -44,7 +47,11 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ float log2_hw(float x) { return __builtin_amdgcn_logf(x); }
-__device__ __forceinline__ float rcp_hw(float x) { return __builtin_amdgcn_rcpf(x); }
+// 1 / x for x in [1, 2], as a division rounds it: the hardware's reciprocal and one Newton step
+__device__ __forceinline__ float rcp_near(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
+}
 
 // (two waves per SIMD: a few registers over 256 would halve that)
 template <int D, int DV, typename TQ, typename TO, bool POOL>
@@ -208,9 +215,12 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     // (this kernel serves bf16 models only: the hardware exp / log / reciprocal are far inside their rounding)
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = S[r] * sc_mul;
-    if (softcap > 0.f) {
+    if (softcap > 0.f) {                       // cap tanh: (1 - e) / (1 + e), e = exp(-2 |s| / cap), never overflows or cancels
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = cap2 - 2.f * cap2 * rcp_hw(exp2_hw(p[r]) + 1.f);
+      for (int r = 0; r < 16; ++r) {
+        const float e = exp2_hw(-fabsf(p[r]));
+        p[r] = copysignf(cap2 * (1.f - e) * rcp_near(1.f + e), p[r]);
+      }
     }
     if (a1 != 0.f) {
       const float dist0 = (float)(iq - j0 - 4 * h2);
@@ -219,7 +229,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     }
     if (gated) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] = rcp_hw(1.f + exp2_hw(-(p[r] + gb)));
+      for (int r = 0; r < 16; ++r) {
+        const float y = p[r] + gb, e = exp2_hw(-fabsf(y)), q = rcp_near(1.f + e);
+        p[r] = y < 0.f ? e * q : q;
+      }
     }
     if (!full) {
       // the row sees keys [mlo, mhi] and, of a window's tiles, those before keep_first (no key of a row past the tile's end)
@@ -238,7 +251,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[r]);
       mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-      if (__any(mt > m + 8.f)) {               // (wave-uniform)
+      if (__any(mt > m)) {               // (wave-uniform)
         mt = fmaxf(mt, m);
         const float corr = exp2_hw(m - mt);
         l *= corr;

@@ -4,6 +4,8 @@ GEMMs (64 / 128 / 256 tiles, the skinny decode kernel, K tails, column-slice ope
 row groups), group norm, activations, K/V store, both attention kernels over paged keys (chunks, windows,
 carried positions, head sizes on and off the matrix-core path), convolution and both scans with carried
 state in scattered slots, routing."""
+import math
+
 import numpy as np
 import pytest
 import torch
@@ -203,7 +205,7 @@ def test_attention(ops, cdt, tol, Hh, G, d, dv):
 
 # prompt attention over 64-key tiles in two halves: lengths about a half, a tile and a 128-row block, windows and chunks that end inside
 # a half, kept first keys, pages of 24 (no power of two); `grow`: scores that rise along the keys in small steps or in large ones
-# (the running maximum stays behind by up to 8 units of log 2), with a sink far below, near and far above them.  bf16 tolerance as above
+# (the running maximum grows key by key, or in jumps), with a sink far below, near and far above them.  bf16 tolerance as above
 @pytest.mark.parametrize("lens,pos0", [([31, 33], [0, 0]), ([64, 65], [0, 7]), ([129], [0]), ([200], [333])])
 @pytest.mark.parametrize("d,dv,ps", [(64, 128, 24), (128, 128, 16)])
 def test_prompt_attention_tiles(ops, lens, pos0, d, dv, ps):
@@ -232,6 +234,32 @@ def test_prompt_attention_tiles(ops, lens, pos0, d, dv, ps):
             o1, o2 = (o.attn_paged(qg.view(T, -1), kg.view(npages, ps, G * d), vc, md, Hh, G, d, dv, 0.3, 0.0, None, None, 0, ps,
                                    torch.bfloat16, **kw) for o in (H, R))
             close(o1, o2, 2e-2)
+
+
+# a query's largest weight is exactly 1 whatever came before it: every other key's value is 0, so the output is that key's value over the sum of
+# weights to fp32, at jumps of 0.1 to 6 over the keys before and with a sink and the cap (two bf16 terms of any other weight: 7.6e-6)
+@pytest.mark.parametrize("d,dv", [(64, 128), (128, 64)])
+@pytest.mark.parametrize("cap,sink", [(0.0, None), (0.0, 0.05), (30.0, None)])
+def test_prompt_attention_largest_weight(ops, d, dv, cap, sink):
+    H, _ = ops
+    Hh, n, at = 16, 100, 70
+    md, npages, _ = meta_of([n], [0], DEV)
+    jump = torch.linspace(0.1, 6.0, Hh).bfloat16()
+    q, k, v = torch.zeros(n, Hh, d), torch.zeros(n, d), torch.zeros(n, dv)
+    q[:, :, 0], k[at, 0], v[at] = jump.float(), 1.0, torch.randn(dv, generator=torch.Generator().manual_seed(d)).bfloat16().float()
+    kc, vc = torch.zeros(npages, 16, d).bfloat16(), torch.zeros(npages, 16, dv).bfloat16()
+    tab, j = md["page_table"][0].cpu().long(), torch.arange(n)
+    kc.view(-1, d)[tab[j // 16] * 16 + j % 16], vc.view(-1, dv)[tab[j // 16] * 16 + j % 16] = k.bfloat16(), v.bfloat16()
+    out = torch.empty(n, Hh * dv, device=DEV)
+    H.attn_paged(q.bfloat16().view(n, -1).to(DEV), kc.to(DEV), vc.to(DEV), md, Hh, 1, d, dv, 1.0, cap, None, None, 0, 16, torch.bfloat16, out=out,
+                 **({} if sink is None else dict(sink=sink)))
+    s = jump.double()
+    s = cap * torch.tanh(s / cap) if cap else s
+    for i in range(at, n):
+        w = torch.exp(s) / (torch.exp(s) + i + (0.0 if sink is None else math.exp(sink)))
+        want = w[:, None] * v[at].double()
+        assert float(((out[i].cpu().double().view(Hh, dv) - want).abs() / want.abs().clamp(min=1e-30)).max()) < 1e-6
+    assert not bool(out[:at].any())
 
 
 # norms with rows in registers: one to eight steps of 1024 columns a group, the last one partly filled, the widest and the first beyond it
