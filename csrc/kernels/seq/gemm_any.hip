@@ -319,10 +319,12 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
   const int vec_w = aligned16(W, ldw, ew, K) && (w_gs * ew) % 16 == 0;
   const hipStream_t st = (hipStream_t)s;
   if (vec_a && vec_w) {
-    // Few rows (in all; for row groups 8 each on average, their sizes are on the device): bound by reading W, no tile to fill.
-    // 48 rows of 8 experts (4096 x 2048 each): 32 us, the best tile 36; 40 rows x 2048 x 2048: 12 us, the best tile 7.
+    // Few rows: bound by reading W, no tile to fill.  40 rows x 2048 x 2048: 12 us, the best tile 7.  Row groups: 8 rows each on average, and
+    // 128 in all (64 in fp32), because their sizes are on the device and a router may send most rows to one: a block then reads its weight
+    // panel once per 16 rows.  128 groups (1536 x 2048, bf16), rows spread or all in one: 64 rows 68 and 18 us, tiles 76 and 13; 128 rows 102
+    // and 34, 110 and 14; 1024 rows 171 and 264, 154 and 29.  fp32: 64 rows 161 and 39, 165 and 26; 1024 rows 391 and 616, 337 and 83.
     int rc = 0;
-    if (offs != nullptr ? M <= 8 * groups : groups == 1 && M <= 32)
+    if (offs != nullptr ? M <= 8 * groups && M <= (tw == 1 ? 128 : 64) : groups == 1 && M <= 32)
       rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, st);
     if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, a_gs, a_mod, w_gs, c_gs, st);
     if (rc != 0) return rc == 1 ? 0 : rc;

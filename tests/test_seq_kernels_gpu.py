@@ -152,6 +152,19 @@ def test_grouped_few_rows(ops, cdt, tol, K):
     close(H.grouped_matmul_nt(a, w, offs), R.grouped_matmul_nt(a, w, offs), 1e-5)
 
 
+# about the rows up to which row groups take the few-row kernel, spread over the groups and nearly all in one
+@pytest.mark.parametrize("cdt,tol", DTYPES)
+@pytest.mark.parametrize("M", [64, 65, 128, 129])
+def test_grouped_rows_in_one_group(ops, cdt, tol, M):
+    H, R = ops
+    torch.manual_seed(M)
+    E, N, K = 20, 72, 192
+    a, w = torch.randn(M, K, device=DEV).to(cdt), torch.randn(E, N, K, device=DEV).to(cdt)
+    for sizes in ([M // E] * (E - 1) + [M - M // E * (E - 1)], [0, 1] + [0] * (E - 4) + [M - 2, 1]):
+        offs = torch.tensor(np.cumsum([0] + sizes), dtype=torch.int32, device=DEV)
+        close(H.grouped_matmul_nt(a, w, offs), R.grouped_matmul_nt(a, w, offs), 1e-5)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_rows(ops, cdt, tol):
     H, R = ops
