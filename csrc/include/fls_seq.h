@@ -71,7 +71,6 @@ int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col, int x_hs, 
                            const float* freqs, int rot, const int* tok_pos, const int* row_map, void* out, int to,
                            int ldo, int out_col, int out_hs, void* raw, int ldr, int rows, int unit_after, int half, float amp,
                            fls_stream_t s);
-int fls_seq_softcap(float* z, int ldz, int rows, int cols, float cap, fls_stream_t s);
 int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, fls_stream_t s);
 // k rows RMS-normed over all kcols (times kn), k and v rows written at row kv_slot[r] of the pools
 int fls_seq_kv_store(const float* k, int ldk, const float* kn, float eps, const float* v, int ldv, void* kc, void* vc,
@@ -223,7 +222,6 @@ int fls_seq_streams_norm(const float* xs, int ldx, const int* idx, const float* 
 int fls_seq_streams_update(float* xs, int ldx, const float* y, int ldy, const float* gate, int ldg, const float* hc, float mult,
                            int rows, int D, int S, const float* ncoef, const float* nw, void* h, int th, int ldh, float eps,
                            fls_stream_t s);
-int fls_seq_scale(float* z, int ldz, int rows, int cols, float alpha, fls_stream_t s);
 // y = o * sigmoid(g); o of type to_, y of type ty
 int fls_seq_sigmoid_gate(const void* o, int to_, int ldo, const float* g, int ldg, void* y, int ty, int ldy, int rows, int cols,
                          fls_stream_t s);

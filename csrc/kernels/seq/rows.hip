@@ -422,18 +422,6 @@ extern "C" int fls_seq_unary(const float* z, int ldz, void* y, int ty, int ldy, 
   return 0;
 }
 
-__global__ void softcap_kernel(float* __restrict__ z, int ldz, int cols, float cap) {
-  float* zr = z + (size_t)blockIdx.x * ldz;
-  for (int c = threadIdx.x; c < cols; c += blockDim.x) zr[c] = cap * tanhf(zr[c] / cap);
-}
-
-extern "C" int fls_seq_softcap(float* z, int ldz, int rows, int cols, float cap, fls_stream_t s) {
-  if (rows <= 0) return 0;
-  hipLaunchKernelGGL(softcap_kernel, dim3(rows), dim3(256), 0, (hipStream_t)s, z, ldz, cols, cap);
-  SEQ_LAUNCH_CHECK();
-  return 0;
-}
-
 // first index of the row maximum.  Few rows (decoding): a block per row, so what bounds it is one block's chain of loads: 1024
 // threads with 16-byte loads (32000 columns: 8 loads deep, 6 us; 256 threads of single loads 21)
 #define ARGMAX_THREADS 1024
@@ -985,4 +973,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 19; }
+extern "C" int fls_seq_version(void) { return 20; }

@@ -206,18 +206,6 @@ extern "C" int fls_seq_streams_update(float* xs, int ldx, const float* y, int ld
 }
 
 // ------------------------------------------------------------------------------- small row kernels
-__global__ void scale_kernel(float* __restrict__ z, int ldz, int cols, float alpha) {
-  float* zr = z + (size_t)blockIdx.x * ldz;
-  for (int c = threadIdx.x; c < cols; c += blockDim.x) zr[c] *= alpha;
-}
-
-extern "C" int fls_seq_scale(float* z, int ldz, int rows, int cols, float alpha, fls_stream_t s) {
-  if (rows <= 0) return 0;
-  hipLaunchKernelGGL(scale_kernel, dim3(rows), dim3(256), 0, (hipStream_t)s, z, ldz, cols, alpha);
-  SEQ_LAUNCH_CHECK();
-  return 0;
-}
-
 template <typename TI, typename TO>
 __global__ void sigmoid_gate_kernel(const TI* __restrict__ o, int ldo, const float* __restrict__ g, int ldg, TO* __restrict__ y,
                                     int ldy, int cols) {

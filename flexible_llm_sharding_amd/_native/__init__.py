@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     return lib
 
 
-SEQ_ABI = 19   # csrc/include/fls_seq.h
+SEQ_ABI = 20   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -159,7 +159,6 @@ def _load_seq():
     _bind(lib, "fls_seq_unary", i, p, i, p, i, i, i, i, i, p)
     _bind(lib, "fls_seq_head_norm_rope", i, p, i, i, i, i, i, i, p, f, p, i, p, p, p, i, i, i, i, p, i, i, i, i, f, p)
     _bind(lib, "fls_seq_delta_rule_scan", i, p, i, p, i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, f, f, f, f, i, p, i, p, i, p)
-    _bind(lib, "fls_seq_softcap", i, p, i, i, i, f, p)
     _bind(lib, "fls_seq_argmax", i, p, i, i, i, p, p)
     _bind(lib, "fls_seq_kv_store", i, p, i, p, f, p, i, p, p, i, p, i, i, i, p)
     _bind(lib, "fls_seq_attn_paged", i, p, i, i, p, i, p, i, i, p, i, i, p, p, p, i, i, i, i, i, i, f, f, p, p, i, i, i, p, f, i, i, p,
@@ -185,7 +184,6 @@ def _load_seq():
     _bind(lib, "fls_seq_gated_delta_scan", i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, i, i, i, f, f, f, i, p, i, p)
     _bind(lib, "fls_seq_streams_norm", i, p, i, p, p, p, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_streams_update", i, p, i, p, i, p, i, p, f, i, i, i, p, p, p, i, i, f, p)
-    _bind(lib, "fls_seq_scale", i, p, i, i, i, f, p)
     _bind(lib, "fls_seq_sigmoid_gate", i, p, i, i, p, i, p, i, i, i, i, p)
     _bind(lib, "fls_seq_diff_combine", i, p, i, p, i, f, i, i, f, p, i, i, i, p)
     _bind(lib, "fls_seq_hgrn2_scan", i, p, i, p, i, p, i, p, p, p, p, i, p, p, p, i, i, i, i, p)

@@ -311,11 +311,6 @@ class HipSeqOps:
     def streams_update_norm_(self, xs, y, gate, hc, mult, streams, coef, w, eps, out_dtype):
         return self._streams_update(xs, y, gate, hc, mult, streams, coef, w, eps, out_dtype)
 
-    def scale_(self, z, alpha):
-        _rows(z, "z", torch.float32)
-        _chk(self.k.fls_seq_scale(z.data_ptr(), z.stride(0), z.shape[0], z.shape[1], float(alpha), _stream()), "fls_seq_scale")
-        return z
-
     def sigmoid_gate(self, o, g, out_dtype):
         _rows(o, "o")
         _rows(g, "g", torch.float32)
@@ -674,12 +669,6 @@ class HipSeqOps:
                                            1 if half else 0, float(amp), _stream()),
              "fls_seq_head_norm_rope")
         return out
-
-    def softcap_(self, z, cap):
-        _rows(z, "z", torch.float32)
-        _chk(self.k.fls_seq_softcap(z.data_ptr(), z.stride(0), z.shape[0], z.shape[1], float(cap), _stream()),
-             "fls_seq_softcap")
-        return z
 
     def argmax_f32(self, z):
         _rows(z, "z", torch.float32)

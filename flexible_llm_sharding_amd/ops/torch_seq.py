@@ -159,10 +159,6 @@ class TorchSeqOps:
         self.streams_update_(xs, y, gate, hc, mult, streams)
         return self.streams_norm(xs, coef, w, eps, out_dtype, streams)
 
-    def scale_(self, z, alpha):
-        z.mul_(float(alpha))
-        return z
-
     def sigmoid_gate(self, o, g, out_dtype):
         """o * sigmoid(g), element by element."""
         return (o.float() * torch.sigmoid(g.float())).to(out_dtype)
@@ -380,10 +376,6 @@ class TorchSeqOps:
             if blocks is not None:
                 self.block_means(kc, vc, blocks, meta, G * d, Gv * dv)
         return q_out
-
-    def softcap_(self, z, cap):
-        z.copy_(cap * torch.tanh(z / cap))
-        return z
 
     def gather_rows(self, x, idx, out=None):
         return x.index_select(0, idx.long())
