@@ -25,6 +25,9 @@ int fls_seq_version(void);
 int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias, const float* act,
                  int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
                  const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s);
+// the tile that such a product of aligned rows takes, as its index in the table of these types (gemm_tile.hip); by_rows: row groups.  On the host
+// alone, for the tests that hold every tile
+int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated);
 // y[r] = w * x[row] / sqrt(mean_g(x[row]^2) + eps) per group of D / groups columns, row = idx ? idx[r] : r.
 // add != 0: y (fp32) += instead (the residual update), ty ignored.  woff is added to the weight (1 for
 // weights stored around zero).  w_one != 0: w is one number for all columns.

@@ -258,9 +258,10 @@ __device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], si
 // ------------------------------------------------------------------------------------ 256, 192 and 128 x 256
 // Four waves, one per SIMD, 32 HX x 128 outputs each.  HX = 4: 128 x 128, all 256 accumulation registers of a wave, a fragment
 // read from LDS feeds 8 MFMAs.  HX = 3, 2: 192 and 128 rows, for row counts that leave the chip idle in the last (or only) round of
-// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 1024 35, 29, 24.  The products are written as in-place asm so that the accumulators stay where they are (with no spare
-// accumulation register the compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between
-// them; reads run one phase of 8 HX MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
+// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 1024 35, 29, 24.
+// The products are written as in-place asm so that the accumulators stay where they are (with no spare accumulation register the
+// compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between them; reads run one phase of 8 HX
+// MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
 namespace t256 {
 constexpr int TN = 256, KT = 128 /* bytes of a K tile's row */;
 constexpr int lds_bytes(int hx) { return 2 * (64 * hx + TN) * KT; }
@@ -630,6 +631,16 @@ static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int
   return best;
 }
 
+// the index of the tile in its table
+static int choose(int ta, int tw, bool ragged, int M, int N, int nk, int groups, bool by_rows, bool gated) {
+  if (ta == 1) return ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 9, M, N, nk, groups, by_rows, gated);
+  return tw == 1 ? pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows, gated);
+}
+
+extern "C" int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated) {
+  return choose(ta, tw, false, M, N, K * (tw == 1 ? 2 : 4) / 128, groups, by_rows != 0, gated != 0);
+}
+
 int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
                   const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, hipStream_t s) {
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
@@ -645,9 +656,9 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
   const int nk = K * ew / 128;
   const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, a_rows, offs, groups, w_gs * ew, a_gs * ea, c_gs,
                   a_mod < 1 ? 1 : a_mod, 0, 0, 0, ragged};
-  const bool by_rows = offs != nullptr;
+  const int tile = choose(ta, tw, ragged, M, N, nk, groups, offs != nullptr, gated);
   if (ta == 1) {
-    switch (ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 9, M, N, nk, groups, by_rows, gated)) {
+    switch (tile) {
       case 0: return start<gemm_tile_256>(256, 256, 256, t256::lds_bytes(4), t, s);
       case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
       case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
@@ -660,7 +671,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
     }
   }
   if (tw == 1) {
-    switch (pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows, gated)) {
+    switch (tile) {
       case 0: return start<gemm_tile_mid<float, bf16_t, 4, 4, 3, 1, 1>>(128, 128, 256, 3 * 49152, t, s);
       case 1: return start<gemm_tile_mid<float, bf16_t, 2, 4, 2, 1, 2>>(64, 128, 512, 4 * 32768, t, s);
       case 2: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 1, 2>>(64, 64, 512, 6 * 24576, t, s);
@@ -668,7 +679,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
       default: return start<gemm_tile_mid<float, bf16_t, 1, 1, 3, 1, 4>>(32, 32, 1024, 12 * 12288, t, s);
     }
   }
-  switch (pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows, gated)) {
+  switch (tile) {
     case 0: return start<gemm_tile_mid<float, float, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
     case 1: return start<gemm_tile_mid<float, float, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
     case 2: return start<gemm_tile_mid<float, float, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);

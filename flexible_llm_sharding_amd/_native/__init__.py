@@ -141,6 +141,7 @@ def _load_seq():
         raise RuntimeError(f"{_SEQ} is a stale build; rebuild with python -m flexible_llm_sharding_amd._native.build")
     p, i, f, ll = c_void_p, c_int, c_float, ctypes.c_longlong
     _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p)
+    _bind(lib, "fls_seq_gemm_tile_of", i, i, i, i, i, i, i, i, i)
     _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm", i, p, i, p, i, p, p, i, p, f, i, i, i, f, p)
     _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_group_rmsnorm", i, p, i, p, p, p, i, i, i, i, i, f, i, f, i, p)

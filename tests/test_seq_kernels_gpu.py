@@ -77,8 +77,8 @@ def test_matmul(ops, cdt, tol, M, N, K):
     close(H.matmul_nt(af, w), R.matmul_nt(af.to(cdt), w), 1e-5)
 
 
-# one shape for each tile of gemm_tile.hip (256 x 256, 128 x 128 twice, 64 x 128, 64 x 64, 32 x 64, 32 x 32, 192 and 128 x 256), with rows and
-# columns past a tile's end and odd numbers of 64-wide K tiles.  fp32 sums of bf16 products: 1e-5; rounded to bf16: half a
+# sizes that take each bf16 tile of gemm_tile.hip (256 x 256, 128 x 128 twice, 64 x 128, 64 x 64, 32 x 64, 32 x 32, 192 and 128 x 256) for the plain
+# product, with rows and columns past a tile's end and odd numbers of 64-wide K tiles (which tile is asserted in test_every_tile).  fp32 sums of bf16 products: 1e-5; rounded to bf16: half a
 # unit in the last place of the largest value (2^-9) and the other side's sum
 @pytest.mark.parametrize("M,N,K", [(2100, 4100, 64), (4100, 4100, 192), (1030, 4000, 64), (1024, 3900, 320), (1000, 2000, 320), (257, 2020, 320),
                                    (200, 2000, 1088), (65, 132, 448), (4000, 4092, 320), (2500, 4100, 320), (3000, 4092, 256), (2000, 4000, 1984), (1025, 7000, 1088)])
@@ -100,7 +100,7 @@ def test_matmul_tiles(ops, M, N, K):
     close(H.grouped_matmul_nt(a, wg, offs), R.grouped_matmul_nt(a, wg, offs), 1e-5)
 
 
-# the same for fp32 operands and for fp32 rows against bf16 weights: shapes for each of their tiles, blocks of a strided batch
+# the same for fp32 operands and for fp32 rows against bf16 weights, blocks of a strided batch (their tiles one by one: test_every_tile)
 @pytest.mark.parametrize("M,N,K", [(4000, 2052, 96), (1300, 2500, 160), (520, 2052, 224), (260, 2052, 288), (130, 1028, 352), (40, 132, 416)])
 def test_matmul_tiles_fp32_rows(ops, M, N, K):
     H, R = ops
@@ -117,8 +117,8 @@ def test_matmul_tiles_fp32_rows(ops, M, N, K):
     close(H.block_linear(u, wg, bg, 3, torch.bfloat16), R.block_linear(u, wg, bg, 3, torch.bfloat16), 1e-5)
 
 
-# gated products ([gate; up] rows of W, the gate in the epilogue): few rows, every tile from 32 x 64 up, experts with gathered rows,
-# and rows no tile takes (K = 100: the product and the gate as two kernels)
+# gated products ([gate; up] rows of W, the gate in the epilogue): few rows, some of the tiles (each of them: test_every_tile), experts with
+# gathered rows, and rows no tile takes (K = 100: the product and the gate as two kernels)
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("M,I,K", [(5, 40, 64), (23, 100, 200), (70, 1028, 192), (300, 1028, 64), (1030, 2052, 64), (2100, 2052, 64), (20, 24, 100)])
 def test_gated_matmul(ops, cdt, tol, M, I, K):
@@ -139,6 +139,53 @@ def test_gated_matmul(ops, cdt, tol, M, I, K):
     wide = torch.cat([z, z[:, :1]], 1)[:, :2 * I]                   # (a row stride that is no multiple of four)
     for t in (z, wide):
         assert torch.equal(H.argmax_f32(t), t.argmax(1).to(torch.int32))
+
+
+# every tile of gemm_tile.hip by the index in its table (the library says which one a product takes, so a changed rule shows here): plain with a
+# bias, an activation and bf16 results; gated; row groups, empty and of one row among them; gated row groups from gathered rows.  Rows and
+# columns past a tile's end, odd numbers of K tiles.  Sums as in test_matmul_tiles, bf16 operands against fp64 of their products
+EVERY_TILE = [("bf16", v, p, g) for v, (p, g) in enumerate([
+    ((8200, 1304, 192), (2500, 4104, 192)), ((390, 8200, 192), (130, 8200, 192)), ((200, 8200, 192), (200, 5128, 192)), ((65, 8200, 192), (130, 4104, 192)),
+    ((65, 72, 192), (130, 72, 192)), ((65, 3080, 448), (130, 1032, 448)), ((65, 72, 320), (130, 72, 320)), ((900, 8200, 192), (700, 8200, 192)),
+    ((390, 8200, 1088), (200, 8200, 1088))])]
+EVERY_TILE += [("mixed", v, p, g) for v, (p, g) in enumerate([
+    ((200, 8200, 192), (1700, 1544, 192)), ((65, 8200, 1088), (130, 3080, 1088)), ((65, 3080, 192), (130, 1032, 192)), ((65, 8200, 192), (130, 3080, 192)),
+    ((65, 72, 192), (130, 72, 192))])]
+EVERY_TILE += [("fp32", v, p, g) for v, (p, g) in enumerate([
+    ((8200, 392, 96), (257, 8200, 96)), ((8200, 136, 64), (200, 5128, 96)), ((65, 8200, 96), (130, 4104, 96)), ((4100, 72, 96), (130, 2056, 96)),
+    ((65, 3080, 96), (130, 1032, 96)), ((65, 72, 96), (130, 72, 96))])]
+
+
+@pytest.mark.parametrize("types,tile,plain,grouped", EVERY_TILE)
+def test_every_tile(ops, types, tile, plain, grouped):
+    H, _ = ops
+    ta, tw = {"bf16": (torch.bfloat16, torch.bfloat16), "mixed": (torch.float32, torch.bfloat16), "fp32": (torch.float32, torch.float32)}[types]
+    code, E = lambda t: int(t == torch.bfloat16), 6
+    gated = (types, tile) not in (("bf16", 6), ("mixed", 4), ("fp32", 5))           # (32-column tiles hold one half of a gated column)
+    for (M, N, K), groups in ((plain, 1), (grouped, E)):
+        for g in (0, 1)[:1 + gated]:
+            assert H.k.fls_seq_gemm_tile_of(code(ta), code(tw), M, N, K, groups, int(groups > 1), g) == tile
+    f64 = lambda t: (t.to(tw) if types == "mixed" else t).double()                  # (fp32 rows are rounded to bf16 weights)
+    M, N, K = plain
+    torch.manual_seed(M + N + K)
+    a, w, b = torch.randn(M, K, device=DEV).to(ta), (0.1 * torch.randn(N, K, device=DEV)).to(tw), torch.randn(N, device=DEV)
+    z = f64(a) @ w.double().t()
+    close(H.matmul_nt(a, w, b), z + b, 1e-5)
+    close(H.matmul_nt(a, w, b, relu2=True, out_dtype=torch.bfloat16), torch.relu(z + b).square(), 2 ** -8)
+    silu = lambda y: torch.nn.functional.silu(y[..., :y.shape[-1] // 2]) * y[..., y.shape[-1] // 2:]
+    if gated:
+        close(H.gated_matmul_nt(a, w, torch.float32), silu(z), 2e-5)
+        close(H.gated_matmul_nt(a, w, torch.bfloat16), silu(z), 2 ** -8)
+    M, N, K = grouped
+    sizes = [0, M // 2, 1, M - M // 2 - 1 - 3, 0, 3]
+    offs = torch.tensor(np.cumsum([0] + sizes), dtype=torch.int32, device=DEV)
+    a, w = torch.randn(M, K, device=DEV).to(ta), (0.1 * torch.randn(E, N, K, device=DEV)).to(tw)
+    y = lambda x: torch.cat([f64(x[offs[e]:offs[e + 1]]) @ w[e].double().t() for e in range(E)])
+    close(H.grouped_matmul_nt(a, w, offs), y(a), 1e-5)
+    if gated:
+        rows, few = torch.randperm(M, device=DEV).to(torch.int32) // 2, a[:(M + 1) // 2]        # (two places per row)
+        for out, tol in ((torch.float32, 2e-5), (torch.bfloat16, 2 ** -8)):
+            close(H.gated_matmul_nt(few, w, out, offs=offs, rows=rows), silu(y(few[rows.long()])), tol)
 
 
 # few rows per group, one group of more than the 16 that a pass over its weights takes, empty groups, a K tail
