@@ -6,8 +6,8 @@
 //   gated:        X = the updates u;                M1 = -(I + b A)^-1 b K+,   N1 = (I + b A)^-1 b
 //   generalized:  X = k^T S before each row;        M1 = (I + A)^-1 K+,        N1 = (I + A)^-1 Ak
 //
-// (in brackets the generalized rule's) where K+, Q+ are rows times the decay since the chunk's start, and A, B, .. hold sum_i left_t,i right_s,i prod(decays between s and t)
-// for s < t (B: and s = t).  Two kernels:
+// (in brackets the generalized rule's) where K+, Q+ are rows times the decay since the chunk's start, and A, B, .. hold
+// sum_i left_t,i right_s,i prod(decays between s and t) for s < t (B: and s = t).  Two kernels:
 //
 //   factors (independent of the state, a block per chunk and head)     M1 .. into memory.  Nothing divides by a decay: a pair (t, s)
 //     belongs to the one of four levels (8, 4, 2, 1) at which t is in the upper and s in the lower half of the same block of rows; left

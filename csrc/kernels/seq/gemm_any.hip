@@ -6,9 +6,8 @@
 // fp32 per lane).  K advances 32 at a time through LDS: 256 threads stage 64 x 32 of A and of W
 // (rounding A to the weight's type on the way in when the producer left fp32), then every wave
 // issues 4 (bf16, 32x32x8) or 16 (fp32, 32x32x2) MFMAs per stage.  Rows, columns and K tails are
-// zero-filled, so any shape runs.  A row's result depends only on that row of A and on W (the
-// K order is fixed and no other row enters its accumulator), so it does not depend on what else is
-// in the batch.
+// zero-filled, so any shape runs.  No other row enters a row's accumulator: beside other rows its result is the same to rounding (which
+// kernel and tile a product takes, and so how K is summed, goes by the number of rows).
 //
 // Two batch forms share the kernel: a strided batch (block-diagonal gates: group g multiplies
 // column block g % a_mod of A by its own square matrix into column block g of C) and row groups

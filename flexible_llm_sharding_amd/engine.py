@@ -511,8 +511,10 @@ class ShardedRunner:
         the state earlier steps left (``self.seq_cache``); requests named in ``end`` give their pages
         and slots back afterwards.  -> per entry (logits [len(want), vocab] fp32, their argmax) or
         None when it wants nothing.  Entries are cut into micro-batches of whole requests under the
-        token budget and scheduled over the shards like a scoring call's micro-batches; a row's
-        result does not depend on which other requests share its micro-batch."""
+        token budget and scheduled over the shards like a scoring call's micro-batches.  No row's result
+        contains another request's; how its sums are split (the products' tiles by the micro-batch's rows,
+        recurrences row by row or in chunks by its longest request) follows the micro-batch, so with other
+        requests beside it a row is the same to rounding."""
         if not self.hybrid:
             raise RuntimeError("step() serves hybrid stacks; Llama-structured models score (prefix, suffixes) prompts")
         t_start = time.perf_counter()

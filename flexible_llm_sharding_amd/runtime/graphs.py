@@ -246,9 +246,9 @@ class StepGraphs:
     graphs are dropped.  Every row's logits are computed (``want_idx`` = all rows); the caller picks
     the wanted ones.
 
-    A step's index arrays are segments of one int32 buffer that goes up in one copy from pinned memory, and its
-    logits come down into pinned memory (:meth:`read`): one copy each way (nine pageable ones up were 145 us of a
-    950 us step of 8 requests, the pageable 1 MB down another 100)."""
+    A step's index arrays are segments of one int32 buffer that goes up in one copy from pinned memory (nine
+    pageable ones were 145 us of a 950 us step of 8 requests); its logits and their argmax come down into pinned
+    memory, a copy each and one wait for both (:meth:`read`; pageable, the 1 MB of logits took another 100)."""
 
     TABLE_BUCKET = 16
     KEYS = ("ids", "tok_seq", "tok_pos", "cu", "pos0", "slot", "page_table", "kv_slot", "want_idx")
