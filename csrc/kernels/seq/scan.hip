@@ -739,7 +739,6 @@ extern "C" int fls_seq_rglru_scan_rows(const float* u, int ldu, const float* g, 
                                        float* state, void* out, int to, int ldo, const int* cu, const int* pos0, const int* slot,
                                        int B, int W, float c, fls_stream_t s) {
   if (B <= 0 || W <= 0) return 0;
-  if (B > 65535) return -1;
 #define RG_ROWS(CB, TO) hipLaunchKernelGGL((rglru_rows_kernel<CB, TO>), dim3((W + CB - 1) / CB, B), dim3(1024), 0, (hipStream_t)s, u, ldu, \
                                            g, ldg, lam, y, ldy, state, (TO*)out, ldo, cu, pos0, slot, W, c)
   // (32 channels a block where 64 leave CUs idle)

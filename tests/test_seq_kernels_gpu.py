@@ -616,6 +616,21 @@ def test_rglru_forms(ops, monkeypatch, lens, W, limit):
     close(st, want, 2e-6)
 
 
+# more requests in a step than 16 bits count: the same rows from the one pass as row by row
+def test_rglru_many_requests(ops):
+    H, _ = ops
+    torch.manual_seed(9)
+    lens, W = [1] * 65540 + [40], 8
+    md, _, nslots = meta_of(lens, [0] * len(lens), DEV)
+    T = sum(lens)
+    u, g, lam, y = torch.randn(T, W, device=DEV), torch.randn(T, 2 * W, device=DEV), torch.randn(W, device=DEV), torch.randn(T, W, device=DEV)
+    st, st2 = torch.zeros(nslots, W, device=DEV), torch.zeros(nslots, W, device=DEV)
+    got = H.rglru_scan(u, g, lam, y, st, md, 8.0, torch.float32)
+    want = H.rglru_scan(u, g, lam, y, st2, dict(md, q_tiles=None), 8.0, torch.float32)
+    close(got, want, 2e-6)
+    close(st, st2, 2e-6)
+
+
 # the chunked delta rules: chunk ends, one row and none beside long requests, a carried state, shared keys, value columns that do not fill
 # four waves, decays from none to exact zeros, and (small memory) several launches that pass the state on; the oracle in fp64.  The
 # bound is that of fp32 sums over some 128 terms and 16-row chains; the row-by-row kernels have to meet it too
