@@ -676,8 +676,10 @@ extern "C" int fls_seq_rglru_scan_tiled(const float* u, int ldu, const float* g,
 // request 128 rows at a time.  A thread takes 128 CB / 1024 consecutive rows of a channel, keeps their a and b in registers, leaves
 // their product and their state from zero in LDS, joins those of the rows before its own and replays its rows: every input is read
 // once and every a and b, which is what this scan costs (an exponential, an expm1, a root and two sigmoids a row), is made once.
-// The next 128 rows' inputs are loaded before these are worked on.  Against the three passes: 2 requests of 512 rows x 2048 channels 106
-// -> 25 us, 8 of 2048 x 4096 516 -> 368, one of 2048 x 2048 116 -> 84; of 4096 149 -> 164, of 16384 327 -> 716.
+// The next 128 rows' inputs are loaded before these are worked on.  Products and states of parts are fp64 and joined in fp64: rounded
+// to fp32 they put outputs and last states up to 0.6% and 6% further from 64 bits than row by row (for 6% of the time), so they are up to 7%
+// nearer.  Against the three passes: 2 requests of 512 rows x 2048 channels 104 -> 26 us, 8 of 2048 x 4096 516 -> 367, one of
+// 2048 x 2048 115 -> 87, of 3000 143 -> 129; of 4096 146 -> 175, of 16384 294 -> 754.
 template <int CB, typename TO>
 __global__ __launch_bounds__(1024) void rglru_rows_kernel(const float* __restrict__ u, int ldu, const float* __restrict__ g, int ldg,
                                                           const float* __restrict__ lam, const float* __restrict__ y, int ldy,
@@ -685,7 +687,8 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(const float* __restric
                                                           const int* __restrict__ cu, const int* __restrict__ pos0,
                                                           const int* __restrict__ slot, int W, float cdecay) {
   constexpr int PARTS = 1024 / CB, R = 128 / PARTS;
-  __shared__ float sA[2][PARTS][CB], sL[2][PARTS][CB], sS[2][CB];
+  __shared__ double sA[2][PARTS][CB], sL[2][PARTS][CB];
+  __shared__ float sS[2][CB];
   const int s = blockIdx.y, lc = threadIdx.x % CB, part = threadIdx.x / CB;
   const int c = blockIdx.x * CB + lc;
   const bool ok = c < W;
@@ -709,7 +712,8 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(const float* __restric
   int buf = 0;
   for (int t0 = a0; t0 < a1; t0 += 128, buf ^= 1) {
     const int tr = t0 + part * R;
-    float a[R], b[R], yv[R], A = 1.f, L = 0.f;
+    float a[R], b[R], yv[R];
+    double A = 1.0, L = 0.0;
 #pragma unroll
     for (int j = 0; j < R; ++j) yv[j] = ok && tr + j < a1 ? y[(size_t)(tr + j) * ldy + c] : 0.f;
 #pragma unroll
@@ -723,8 +727,9 @@ __global__ __launch_bounds__(1024) void rglru_rows_kernel(const float* __restric
     sL[buf][part][lc] = L;
     __syncthreads();
     if (t0 + 128 < a1) load(t0 + 128);
-    float S = sS[buf][lc];
-    for (int p = 0; p < part; ++p) S = sA[buf][p][lc] * S + sL[buf][p][lc];
+    double S0 = sS[buf][lc];
+    for (int p = 0; p < part; ++p) S0 = sA[buf][p][lc] * S0 + sL[buf][p][lc];
+    float S = (float)S0;
 #pragma unroll
     for (int j = 0; j < R; ++j) {
       S = a[j] * S + b[j];

@@ -891,7 +891,7 @@ class HipSeqOps:
         return out
 
     # rows of the longest request up to which one pass over its rows beats three over tiles of all, where the channels of all requests do
-    # not fill the chip (2048 channels, 1 request of 2048 / 4096 / 16384 rows: 84 / 164 / 716 us, in three 116 / 149 / 327)
+    # not fill the chip (2048 channels, 1 request of 2048 / 3000 / 4096 / 16384 rows: 87 / 129 / 175 / 754 us, in three 115 / 143 / 146 / 294)
     RGLRU_ROWS = 3072
 
     def rglru_scan(self, u, g, lam, y, state, meta, c, out_dtype):

@@ -616,6 +616,36 @@ def test_rglru_forms(ops, monkeypatch, lens, W, limit):
     close(st, want, 2e-6)
 
 
+# the one pass over the rows is no further from 64 bits than the row-by-row kernel (both repeat themselves exactly): rounds of 128 rows
+# that end in mid-part, gates that keep little of a row's state and nearly all of it
+@pytest.mark.parametrize("bias", [0.0, -2.0, -4.0])
+def test_rglru_rows_are_as_exact_as_row_by_row(ops, monkeypatch, bias):
+    H, _ = ops
+    torch.manual_seed(5)
+    lens, W = (100, 300, 413, 500, 601), 2048
+    md, _, nslots = meta_of(lens, [0] * len(lens), DEV)
+    T = sum(lens)
+    u, g, lam, y = torch.randn(T, W, device=DEV), torch.randn(T, 2 * W, device=DEV) + bias, torch.randn(W, device=DEV), torch.randn(T, W, device=DEV)
+    g6 = g.double()
+    la = -8.0 * torch.sigmoid(g6[:, :W]) * torch.nn.functional.softplus(lam.double())
+    a6, b6 = torch.exp(la), torch.sqrt(-torch.expm1(2 * la)) * torch.sigmoid(g6[:, W:]) * u.double()
+    out, states, r = torch.empty(T, W, device=DEV).double(), [], 0
+    for n in lens:
+        S = torch.zeros(W, device=DEV).double()
+        for t in range(r, r + n):
+            S = a6[t] * S + b6[t]
+            out[t] = S
+        states.append(S)
+        r += n
+    want, err = (out * torch.nn.functional.gelu(y.double(), approximate="tanh"), torch.stack(states)), []
+    monkeypatch.setattr(H, "RGLRU_ROWS", 10 ** 9)
+    for m in (dict(md, q_tiles=None), md):
+        st = torch.zeros(nslots, W, device=DEV)
+        got = H.rglru_scan(u, g, lam, y, st, m, 8.0, torch.float32)
+        err.append([float((a.double() - b).norm() / b.norm()) for a, b in zip((got, st[md["slot"].long()]), want)])
+    assert err[1][0] <= 1.005 * err[0][0] and err[1][1] <= 1.01 * err[0][1], err
+
+
 # more requests in a step than 16 bits count: the same rows from the one pass as row by row
 def test_rglru_many_requests(ops):
     H, _ = ops
