@@ -905,7 +905,7 @@ class HipSeqOps:
         out = torch.empty(T, Wd, dtype=out_dtype, device=u.device)
         tiles, tile_cu = meta.get("q_tiles"), meta.get("tile_cu")
         rows = int(meta.get("max_rows") or 0)
-        if tiles is not None and (rows <= self.RGLRU_ROWS or -(-Wd // 64) * meta["n_seqs"] >= 256):
+        if tiles is not None and (0 < rows <= self.RGLRU_ROWS or -(-Wd // 64) * meta["n_seqs"] >= 256):
             _chk(self.k.fls_seq_rglru_scan_rows(u.data_ptr(), u.stride(0), g.data_ptr(), g.stride(0), lam.data_ptr(), y.data_ptr(),
                                                 y.stride(0), state.data_ptr(), out.data_ptr(), _CODE[out_dtype], Wd, meta["cu"].data_ptr(),
                                                 meta["pos0"].data_ptr(), meta["slot"].data_ptr(), meta["n_seqs"], Wd, float(c), _stream()),
@@ -941,13 +941,14 @@ class HipSeqOps:
         for n, t in (("dt_bias", dt_bias), ("A_log", A_log), ("D", Dskip)):
             _vec(t, n, nh)
         out = torch.empty(T, inner, dtype=torch.float32, device=xbc.device)
-        if (meta["max_rows"] >= self.SSD_CHUNK_ROWS and N in (64, 128) and P % 16 == 0 and xbc.stride(0) % 4 == 0
+        rows = int(meta.get("max_rows") or 0)
+        if (rows >= self.SSD_CHUNK_ROWS and N in (64, 128) and P % 16 == 0 and xbc.stride(0) % 4 == 0
                 and xbc.data_ptr() % 16 == 0):
             scores = torch.empty(T * G * 64, dtype=torch.float32, device=xbc.device)
             _chk(self.k.fls_seq_ssd_scan_chunked(xbc.data_ptr(), xbc.stride(0), z.data_ptr(), z.stride(0), dt.data_ptr(), dt.stride(0),
                                                  dt_bias.data_ptr(), A_log.data_ptr(), Dskip.data_ptr(), state.data_ptr(),
                                                  out.data_ptr(), inner, meta["cu"].data_ptr(), meta["pos0"].data_ptr(),
-                                                 meta["slot"].data_ptr(), meta["n_seqs"], int(meta["max_rows"]), nh, P, N, G,
+                                                 meta["slot"].data_ptr(), meta["n_seqs"], rows, nh, P, N, G,
                                                  scores.data_ptr(), _stream()), "fls_seq_ssd_scan_chunked")
             return out
         _chk(self.k.fls_seq_ssd_scan(xbc.data_ptr(), xbc.stride(0), z.data_ptr(), z.stride(0), dt.data_ptr(), dt.stride(0),

@@ -496,6 +496,20 @@ def test_ssd_chunks(ops, lens, pos0, nh, P, N, G, strong):
     close(s1, s2, 3e-6)
 
 
+# a step described without its longest request is walked row by row
+def test_ssd_scan_without_the_longest_request(ops):
+    H, R = ops
+    torch.manual_seed(8)
+    nh, P, N = 2, 16, 64
+    md, _, nslots = meta_of([40, 3], [0, 5], DEV)
+    args = [torch.randn(43, n, device=DEV) for n in (nh * P + 2 * N, nh * P, nh)] + [torch.randn(nh, device=DEV) for _ in range(3)]
+    s1 = torch.randn(nslots, nh, N, P, device=DEV)
+    s2 = s1.clone()
+    got = H.ssd_scan(*args, s1, {k: v for k, v in md.items() if k != "max_rows"}, nh, P, N, 1)
+    close(got, R.ssd_scan(*args, s2, md, nh, P, N, 1), 3e-5)
+    close(s1, s2, 3e-5)
+
+
 # a step so large that its own decay is 0 and the sum of a chunk's exponents would lose those of the rows after it
 @pytest.mark.parametrize("step", [3e2, 1e12, 1e17, 1e25])
 def test_ssd_chunks_huge_step(ops, step):
