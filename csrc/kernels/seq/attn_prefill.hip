@@ -212,7 +212,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     }
     float p[16];
     float mt = -1e30f;
-    // (this kernel serves bf16 models only: the hardware exp / log / reciprocal are far inside their rounding)
+    // (this kernel serves bf16 models only: the hardware exp / log are far inside their rounding)
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = S[r] * sc_mul;
     if (softcap > 0.f) {                       // cap tanh: (1 - e) / (1 + e), e = exp(-2 |s| / cap), never overflows or cancels
