@@ -980,3 +980,41 @@ def test_gemm_v11_round_rule():
     assert pays(14784, H) == 1
     # 16,128 rows: v11 needs 6 rounds, v10 8: 6 x 1.45 > 8
     assert pays(16128, H) == 0
+
+
+@pytest.mark.parametrize("family", ["numolorn", "nudadra"])        # (previous tokens; blocks of keys; looped layers in both)
+def test_one_token_steps_pack_like_portions(tmp_path, family):
+    """A step of one token per request packs by itself; beside a two-token request the same rows go through the general
+    packing.  Over many steps both give every request the same arrays, and refuse the same wanted places."""
+    import importlib
+    from flexible_llm_sharding_amd.config import load_config
+    from flexible_llm_sharding_amd.runtime.batch import StepEntry, pack_step
+    from flexible_llm_sharding_amd.runtime.seq_state import SequenceStateCache
+    t, u = importlib.import_module(f"test_{family}"), importlib.import_module(f"{family}_util")
+    d = u.config(t.STACK, loop=t.LOOP)
+    cfg = load_config(u.write_model(str(tmp_path / "m"), d, u.random_weights(d)))
+    alone, beside = (SequenceStateCache(cfg, "cpu", torch.float32, 64, 8) for _ in range(2))
+    rng = np.random.default_rng(3)
+    for step in range(40):
+        rids = rng.permutation(5)[:1 + step % 5].tolist()
+        entries = [StepEntry(r, [int(rng.integers(50))], [0] * int(rng.integers(2))) for r in rids]
+        a = pack_step(entries, alone)
+        b = pack_step(entries + [StepEntry("more", [1, 2])], beside)
+        n = len(rids)
+        assert a.max_rows == 1 and a.num_tokens == n and b.num_tokens == n + 2
+        for k in ("ids", "tok_seq", "tok_pos", "pos0", "want_idx", "prev_ids"):
+            x, y = getattr(a, k), getattr(b, k)
+            assert (x is None and y is None) or (x.dtype == y.dtype == np.int32 and np.array_equal(x, y[:len(x)])), k
+        assert a.rids == rids and a.want_count == b.want_count[:n] and np.array_equal(a.cu, b.cu[:n + 1])
+        assert len(a.want_idx) == len(b.want_idx) == sum(a.want_count)
+        # (pages and slots are handed out in another order: they have to lead to the same places of each request's own)
+        for c, p in ((alone, a), (beside, b)):
+            table = c.page_table(p.rids)
+            want = table[p.tok_seq, p.tok_pos // c.page_size].astype(np.int64) * c.page_size + p.tok_pos % c.page_size
+            assert np.array_equal(p.kv_slot, want) and np.array_equal(p.page_table, table) and len(set(p.slot.tolist())) == len(p.rids)
+            assert sorted(p.block_tables) == c.block_sizes and all(np.array_equal(v, c.block_table(p.rids, P)) for P, v in p.block_tables.items())
+    assert a.q_tiles is None and a.tile_cu is None and a.local_table is None
+    for bad in (1, -1):
+        for more in ([], [StepEntry("other", [1, 2])]):
+            with pytest.raises(ValueError, match="lies outside its 1 tokens"):
+                pack_step([StepEntry("x", [3], [bad])] + more, alone)
