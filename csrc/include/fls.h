@@ -103,6 +103,7 @@ int fls_copy_rows(const void* x, int ldx, const int* src_idx, void* y, int ldy, 
                   fls_stream_t s);
 int fls_gemm_set_splitk(int on);
 int fls_gemm_set_row_chunk(int rows);   // rows per main-path GEMM launch (default 16384; 0 = unlimited)
+int fls_gemm_set_v10_rows(int rows);    // rows of a 256-column main-path tile: 0 by shape, 128, 192 or 256 forced (tests / A-B)
 // mixture-of-experts FFN (csrc/kernels/moe.hip): routing, stable expert sort, grouped v10 GEMM
 // (every expert of a layer in one launch, optional row gather), fp16-ordered weighted combine
 int fls_moe_route(const void* logits, int ldl, int T, int E, int k, int norm, int round16, int* ids, float* w,

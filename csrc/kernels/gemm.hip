@@ -428,15 +428,29 @@ void launch_mid(const half_t* A, const half_t* W, half_t* C, int M, int N, int K
                      lda, ldw, ldc, ep);
 }
 
-template <int EPI>
-void launch_main(int tiles, const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw,
-                 int ldc, const Epi& ep, hipStream_t s) {
+template <int EPI, int HX>
+void launch_rows(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc, Epi ep,
+                 hipStream_t s) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm_nt_v10<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, 2 * BUF);
+    (void)hipFuncSetAttribute((const void*)gemm_nt_v10<EPI, false, HX>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              2 * v10_stage(HX));
     attr = true;
   }
-  hipLaunchKernelGGL((gemm_nt_v10<EPI>), dim3(tiles), dim3(256), 2 * BUF, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
+  const int tiles_m = (M + 64 * HX - 1) / (64 * HX), tiles_n = N / BN;
+  ep.order = g_order ? g_order : auto_order(tiles_m, tiles_n);
+  hipLaunchKernelGGL((gemm_nt_v10<EPI, false, HX>), dim3(tiles_m * tiles_n), dim3(256), 2 * v10_stage(HX), s, A, W, C,
+                     M, N, K, lda, ldw, ldc, ep);
+}
+
+int g_v10_rows = 0;          // rows of a v10 tile: 0 by shape (v10_rows), 128, 192 or 256 forced (fls_gemm_set_v10_rows)
+
+template <int EPI>
+void launch_main(int rows, const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw,
+                 int ldc, const Epi& ep, hipStream_t s) {
+  if (rows == 128) launch_rows<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+  else if (rows == 192) launch_rows<EPI, 3>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+  else launch_rows<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
 }
 
 
@@ -603,9 +617,68 @@ int splitk_slices(int M, int N, int K, size_t tiles, size_t ws_bytes) {
   return best;
 }
 
+// Which path takes a product of more than 64 rows that all of them could: the least estimated time.  A tile launch is
+// whole rounds of 256 blocks and a last one; a round of blocks takes a start and a store and nk K tiles, more per K tile when all CUs pull
+// on memory and power than when few do (full / part below, us, measured at K = 2,048 .. 28,672).  Rounds are why no one tile
+// serves a range: 600 x 12,288 x 4,096 on 256-row tiles is 144 blocks of 79 us, on 128-row ones 240 of 62; 600 x 22,016 258 blocks
+// (two rounds, 168 us) or 430 (117); 1,700 x 4,096 x 4,096 91 us on 64-row blocks, 57 here; 600 x 10,240 x 8,192 161 and 111.
+enum Route { ROUTE_NONE, ROUTE_SKINNY, ROUTE_SPLIT, ROUTE_MID, ROUTE_128, ROUTE_192, ROUTE_256, ROUTE_V11 };
+
+struct RoundCost { int rows; float full_k, full, part_k, part; };
+const RoundCost ROUNDS[4] = {{128, 0.92f, 4.f, 0.733f, 3.f}, {192, 1.14f, 8.f, 0.82f, 5.5f}, {256, 1.45f, 15.f, 1.f, 9.f},
+                             {384, 2.19f, 11.f, 1.6f, 10.f}};
+
+float rounds_us(const RoundCost& c, long blocks, int nk) {
+  const float full = c.full_k * nk + c.full, part = c.part_k * nk + c.part;
+  const float fill = (float)(blocks % 256) / 256.f;
+  return (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * fill * fill : 0.f);
+}
+
+// ws: scratch for split-K partials (0 bytes: none).  Above four rounds of 256-row tiles the forms are within 3% of each other:
+// ROUTE_NONE (v11 or v10 by whole rounds, v11_pays)
+Route route_of(int M, int N, int K, bool row_exact, size_t ws_bytes) {
+  const int nk = K / BK;
+  const long cols = N / BN;
+  const long tiles256 = (long)((M + 255) / 256) * cols;
+  if (M <= 64 || M > ROW_CHUNK || tiles256 > 1024 || g_v10_rows || g_mid_bn || g_mid_waves || g_mid_rows || g_skinny > 1) return ROUTE_NONE;
+  Route best = ROUTE_NONE;
+  float least = 0.f;
+  auto offer = [&](Route r, float us) {
+    if (best == ROUTE_NONE || us < least) {
+      best = r;
+      least = us;
+    }
+  };
+  for (int i = 0; i < 3; ++i) offer((Route)(ROUTE_128 + i), rounds_us(ROUNDS[i], (long)((M + ROUNDS[i].rows - 1) / ROUNDS[i].rows) * cols, nk));
+  if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], (long)((M + 383) / 384) * cols, nk));
+  const float bytes = (float)N * K * 2.f;                      // the weight, once
+  if (g_mid) {               // 64 x 128 blocks: two share a CU, and from the third round on the weights' re-reads take over
+    const long blocks = (long)((M + 63) / 64) * (N / 128), r = (blocks + 255) / 256;
+    const float fill = bytes > 64e6f ? 1.f : 0.35f + 0.65f * (float)(blocks - 256) / 256.f;
+    offer(ROUTE_MID, r <= 1   ? (M > 128 ? 0.43f : blocks <= 128 ? 0.32f : 0.48f) * nk + 2.5f
+                     : r == 2 ? 0.43f * nk + 2.5f + fill * (0.31f * nk + 2.5f)
+                     : r == 3 ? 1.1f * nk + 5.f
+                              : (0.28f * nk + 1.5f) * r);
+  }
+  if (!row_exact && ws_bytes) {
+    const float slab = (float)M * N * 8.f / 4e6f;              // a slice's partials written and read, us
+    if (g_splitk && M <= SPLITK_MAX_M) {
+      const int S = splitk_slices(M, N, K, (size_t)tiles256, ws_bytes);
+      if (S >= 2) offer(ROUTE_SPLIT, fmaxf(16.f + bytes / 4.8e6f, 0.75f * (rounds_us(ROUNDS[2], tiles256 * S, nk / S) + 5.f + S * slab)));
+    }
+    if (g_skinny && M <= 256) {
+      const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
+      const long r = ((long)(N / bn) * S + 255) / 256;         // (its K tile: all of the rows go through LDS)
+      if (S == 1 || (size_t)S * M * N * 4 <= ws_bytes)
+        offer(ROUTE_SKINNY, 7.f + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * r * nk / S) + (S > 1 ? 0.5f * S * slab : 0.f));
+    }
+  }
+  return best;
+}
+
 template <int EPI>
 int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
-           const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes) {
+           const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes, Route route) {
   const bool mid_ok = N % mid::BNm == 0 && K % mid::BKm == 0 && lda % 8 == 0 && ldw % 8 == 0;
   const size_t tiles256 = (size_t)((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   // 32-bit per-lane DMA offsets (X rows; SWIGLU up-block rows)
@@ -625,12 +698,15 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
                         ldw % 8 == 0 && (size_t)M * lda * 2 < (1ull << 32) && ldc % 4 == 0 &&
                         ((uintptr_t)C & 7) == 0 && ((uintptr_t)ws & 15) == 0 &&
                         (EPI != FLS_EPI_RESID || (ep.ldr % 4 == 0 && ((uintptr_t)ep.R & 7) == 0));
-  if (!ep.row_exact) {
-    const int rc = try_skinny<EPI>(A, W, C, M, N, K, lda, ldw, ldc, ep, s, ws, ws_bytes);
+  if (!main_ok) route = ROUTE_NONE;
+  if (!ep.row_exact && (route == ROUTE_NONE || route == ROUTE_SKINNY)) {
+    const int rc = try_skinny<EPI>(A, W, C, M, N, K, lda, ldw, ldc, ep, s, ws, ws_bytes, route == ROUTE_SKINNY);
     if (rc > 0) ss_partials(C, ldc, M, N, ep, s);
     if (rc) return rc > 0 ? 0 : rc;
   }
-  const int S = split_ok && !ep.row_exact ? splitk_slices(M, N, K, tiles256, ws_bytes) : 0;
+  if (route == ROUTE_SKINNY) route = ROUTE_NONE;             // (its operands' alignment did not allow it)
+  const int S = split_ok && !ep.row_exact && (route == ROUTE_NONE || route == ROUTE_SPLIT)
+                    ? splitk_slices(M, N, K, tiles256, ws_bytes) : 0;
   if (S >= 2 && (M > 64 || tiles256 * S >= 128)) {
     static bool attr_f32 = false;
     if (!attr_f32) {
@@ -656,7 +732,9 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     FLS_CHECK_LAUNCH();
     return 0;
   }
-  if (mid_ok && (!main_ok || (g_mid && (tiles256 < 128 || (M <= 64 && tiles256 < 512))))) {
+  if (route == ROUTE_SPLIT) route = ROUTE_NONE;
+  if (mid_ok && (!main_ok || route == ROUTE_MID ||
+                 (route == ROUTE_NONE && g_mid && (tiles256 < 128 || (M <= 64 && tiles256 < 512))))) {
     // 64-column blocks for a single row tile whose 128-column grid fills less than one round of the
     // 256 CUs: 70B generation steps with 8 prompts (M = 40) 39.7 vs 46.7 ms per step; with 32 prompts
     // (M = 160, three row tiles) the 128-column blocks are faster, 53 vs 55.5 ms (profiles/r6_decode/
@@ -730,7 +808,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   // Only when every chunk still fills the chip (>= 256 tiles), so each piece stays on this path.
   const int n_chunks = (M + ROW_CHUNK - 1) / ROW_CHUNK;
   const int step = ((M + n_chunks - 1) / n_chunks + BM - 1) / BM * BM;
-  if (M > ROW_CHUNK && (size_t)(step / BM) * (N / BN) >= 256) {
+  if (route <= ROUTE_MID && M > ROW_CHUNK && (size_t)(step / BM) * (N / BN) >= 256) {
     for (int r0 = 0; r0 < M; r0 += step) {
       Epi e = ep;
       if (e.pos) e.pos += r0;
@@ -738,7 +816,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
       if (e.ss) e.ss += (size_t)r0 * e.ss_ld;
       if (e.rs) e.rs += r0;                  // (the fused norm's per-row statistic follows its rows)
       const int rc = launch<EPI>(A + (size_t)r0 * lda, W, C + (size_t)r0 * ldc, min(step, M - r0), N, K, lda, ldw,
-                                 ldc, e, s, ws, ws_bytes);
+                                 ldc, e, s, ws, ws_bytes, ROUTE_NONE);
       if (rc) return rc;
     }
     return 0;
@@ -746,13 +824,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   // One block per tile, dispatched by the hardware as CUs free up.  A persistent form (one block
   // per CU walking its tiles, the next tile's prologue DMA under this tile's epilogue) measured
   // 1.1-3.9% slower on every 70B / 7B shape once the tile order was XCD-aware (profiles/r2_gemm).
-  const int tiles = (int)tiles256;
-  const int tiles_m = (M + BM - 1) / BM, tiles_n = N / BN;
-  int order = g_order;
-  if (order == 0) order = auto_order(tiles_m, tiles_n);
-  Epi e = ep;
-  e.order = order;
-  launch_main<EPI>(tiles, A, W, C, M, N, K, lda, ldw, ldc, e, s);
+  launch_main<EPI>(g_v10_rows ? g_v10_rows : route == ROUTE_128 ? 128 : route == ROUTE_192 ? 192 : 256, A, W, C, M, N, K, lda, ldw, ldc, ep, s);
   FLS_CHECK_LAUNCH();
   return 0;
 }
@@ -788,6 +860,13 @@ extern "C" int fls_gemm_set_skinny_bn(int bn) {
 extern "C" int fls_gemm_set_splitk(int on) {
   const int old = g_splitk;
   g_splitk = on ? 1 : 0;
+  return old;
+}
+
+// rows of a v10 tile: 0 by shape (default), 128, 192 or 256 forced (tests / A-B); returns the previous
+extern "C" int fls_gemm_set_v10_rows(int rows) {
+  const int old = g_v10_rows;
+  g_v10_rows = rows == 128 || rows == 192 || rows == 256 ? rows : 0;
   return old;
 }
 
@@ -854,7 +933,7 @@ extern "C" int fls_gemm_set_mid(int on) {
 extern "C" int fls_gemm_v11_try(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda,
                                 int ldw, int ldc, int ldr, int epi, const int* pos, const float* cos_t,
                                 const float* sin_t, int rope_cols, int head_dim, const void* bias,
-                                const float* rscale, float alpha, float* ss, int ss_ld, fls_stream_t s);
+                                const float* rscale, float alpha, float* ss, int ss_ld, int want, fls_stream_t s);
 
 extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
                         int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
@@ -869,10 +948,13 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
   if ((epi == FLS_EPI_SWIGLU || epi == FLS_EPI_ROPE) && (N % 32)) return -2;
   if (epi == FLS_EPI_ROPE && ((head_dim != 64 && head_dim != 128) || rope_cols % head_dim || N % head_dim))
     return -3;
+  Route route = N % BN == 0 && K % (2 * BK) == 0 ? route_of(M, N, K, row_exact != 0, ws ? ws_bytes : 0) : ROUTE_NONE;
   {
     const int rc = fls_gemm_v11_try(A, W, C, R, M, N, K, lda, ldw, ldc, ldr, epi, pos, cos_t, sin_t, rope_cols,
-                                    head_dim, bias, rscale, alpha, ss, ss_ld, s);
+                                    head_dim, bias, rscale, alpha, ss, ss_ld,
+                                    route == ROUTE_NONE ? 0 : route == ROUTE_V11 ? 1 : -1, s);
     if (rc) return rc > 0 ? 0 : rc;
+    if (route == ROUTE_V11) route = ROUTE_NONE;
   }
   Epi ep{(const half_t*)R, ldr, pos, cos_t, sin_t, rope_cols, head_dim, (const half_t*)bias, N / 2, 0,
          nullptr, nullptr, nullptr, 0, 0};
@@ -886,12 +968,12 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
   auto c = (half_t*)C;
   auto st = (hipStream_t)s;
   switch (epi) {
-    case FLS_EPI_NONE: return launch<FLS_EPI_NONE>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes);
-    case FLS_EPI_RESID: return launch<FLS_EPI_RESID>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes);
-    case FLS_EPI_SWIGLU: return launch<FLS_EPI_SWIGLU>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes);
+    case FLS_EPI_NONE: return launch<FLS_EPI_NONE>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route);
+    case FLS_EPI_RESID: return launch<FLS_EPI_RESID>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route);
+    case FLS_EPI_SWIGLU: return launch<FLS_EPI_SWIGLU>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route);
     case FLS_EPI_ROPE:
-      return head_dim == 128 ? launch<FLS_EPI_ROPE>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes)
-                             : launch<EPI_ROPE64>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes);
+      return head_dim == 128 ? launch<FLS_EPI_ROPE>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route)
+                             : launch<EPI_ROPE64>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route);
   }
   return -1;
 }

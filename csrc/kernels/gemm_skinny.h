@@ -242,53 +242,57 @@ int launch_skinny_epi(int rs, int bn, const half_t* A, const half_t* W, half_t* 
   }
 }
 
-// -> 1 when the skinny path took the GEMM, 0 when it does not apply, < 0 on a launch error
+// The block width and K slices of a skinny launch.
+// K slices.  BN = 128: else the fewest powers of two that give whole 256-CU rounds or at least
+// two rounds (one block per CU: a fractional single round leaves a tail of full-K blocks).  BN = 256: the fewest that give 192 blocks (3/4 of
+// the CUs; its deeper DMA queue keeps HBM busy from fewer CUs).  g_skinny_blocks > 0 (A/B) sets
+// a block target instead.
+// BN = 128 first tries one round of 7/8 to all of the CUs with uneven slices (70B QKV at M = 160:
+// 80 blocks x 3 = 240 instead of 80 x 8 = 640, 2.5 rounds, and 8 slabs of fp32 partials).
+int skinny_slices(int N, int K, int bn) {
+  const long nblk = N / bn;
+  const int nkt = K / sk::KT;
+  if (bn == 128 && g_skinny_blocks == 0) {
+    for (int s = 2; s <= 16 && nblk * s <= 256; ++s)
+      if (nblk * s >= 224 && nkt / s >= 8) return s;
+  }
+  auto good = [&](int s) {
+    const long b = nblk * s;
+    if (g_skinny_blocks > 0) return b >= g_skinny_blocks;
+    return bn == 256 ? b >= 192 : (b % 256 == 0 || b >= 512);
+  };
+  int s = 1;
+  while (!good(s) && s < 16 && nkt % (2 * s) == 0 && nkt / (2 * s) >= 8) s *= 2;
+  return s;
+}
+
+// BN = 256 (auto) where its split gives whole 256-CU rounds: the 70B O and down projections
+// (32 x 8 blocks), 4% faster on down at M = 160 and equal on O; QKV (40 x 8) and gate/up (224 x 1)
+// run slower with it (profiles/r4_gen/bn256/skinny_ab.log)
+// auto: the wide gate/up GEMM (N / 128 >= 256 blocks, 224 main-path tiles) runs faster on the main
+// path at M = 64 / 160 / 256 (175 / 209 / 221 us vs 195 / 246 / 332 with 128-row blocks), but at
+// 65..144 rows the 256-row block without a K split beats it (same box, M = 96 / 112 / 128 / 144:
+// 180 / 182 / 184 / 199 us vs 216 / 205 / 199 / 206; profiles/r4_gen/gateup_mid_m)
+bool skinny_wide(int N) { return N / 128 >= 256; }
+bool skinny_wide_bn256(int M, int N) { return skinny_wide(N) && M > 64 && M <= 144 && N % 256 == 0; }
+int skinny_bn(int M, int N, int K) {
+  const bool ok = N % 256 == 0 && (M + 31) / 32 * 2 <= SK_BN256_MAX_RS;
+  return ok && (g_skinny_bn == 256 || (g_skinny_bn == 0 && (skinny_wide_bn256(M, N) || (long)(N / 256) * skinny_slices(N, K, 256) % 256 == 0)))
+             ? 256 : 128;
+}
+
+// -> 1 when the skinny path took the GEMM, 0 when it does not apply, < 0 on a launch error.  chosen: the launcher's estimate
+// (route_of) picked it; otherwise only M 17..192 on the narrow projections (the range measured in profiles/r4_gen, 70B shapes)
 template <int EPI>
 int try_skinny(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
-               const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes) {
+               const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes, bool chosen) {
   if (!g_skinny || M > 256 || N % 128 || K % sk::KT || lda % 8 || ldw % 8 || ((uintptr_t)A & 15) ||
       ((uintptr_t)W & 15))
     return 0;
   const int rs = ((M + 31) / 32) * 2;
-  const int nkt = K / sk::KT;
-  // auto: the measured range (profiles/r4_gen, 70B shapes): M 17..192 on the narrow projections;
-  // the wide gate/up GEMM (N / 128 >= 256 blocks, 224 main-path tiles) runs faster on the main
-  // path at M = 64 / 160 / 256 (175 / 209 / 221 us vs 195 / 246 / 332 with 128-row blocks), but at
-  // 65..144 rows the 256-row block without a K split beats it (same box, M = 96 / 112 / 128 / 144:
-  // 180 / 182 / 184 / 199 us vs 216 / 205 / 199 / 206; profiles/r4_gen/gateup_mid_m)
-  const bool wide = N / 128 >= 256;
-  const bool wide_bn256 = wide && M > 64 && M <= 144 && N % 256 == 0;
-  if (g_skinny == 1 && (M < 17 || M > 192 || (wide && !wide_bn256))) return 0;
-  // K slices.  BN = 128: else the fewest powers of two that give whole 256-CU rounds or at least
-  // two rounds (one block per CU: a fractional single round leaves a tail of full-K blocks).  BN = 256: the fewest that give 192 blocks (3/4 of
-  // the CUs; its deeper DMA queue keeps HBM busy from fewer CUs).  g_skinny_blocks > 0 (A/B) sets
-  // a block target instead.
-  // BN = 128 first tries one round of 7/8 to all of the CUs with uneven slices (70B QKV at M = 160:
-  // 80 blocks x 3 = 240 instead of 80 x 8 = 640, 2.5 rounds, and 8 slabs of fp32 partials).
-  auto slices = [&](int bn) {
-    const long nblk = N / bn;
-    if (bn == 128 && g_skinny_blocks == 0) {
-      for (int s = 2; s <= 16 && nblk * s <= 256; ++s)
-        if (nblk * s >= 224 && nkt / s >= 8) return s;
-    }
-    auto good = [&](int s) {
-      const long b = nblk * s;
-      if (g_skinny_blocks > 0) return b >= g_skinny_blocks;
-      return bn == 256 ? b >= 192 : (b % 256 == 0 || b >= 512);
-    };
-    int s = 1;
-    while (!good(s) && s < 16 && nkt % (2 * s) == 0 && nkt / (2 * s) >= 8) s *= 2;
-    return s;
-  };
-  // BN = 256 (auto) where its split gives whole 256-CU rounds: the 70B O and down projections
-  // (32 x 8 blocks), 4% faster on down at M = 160 and equal on O; QKV (40 x 8) and gate/up (224 x 1)
-  // run slower with it (profiles/r4_gen/bn256/skinny_ab.log)
-  const bool bn256_ok = N % 256 == 0 && rs <= SK_BN256_MAX_RS;
-  int bn = 128;
-  if (bn256_ok && (g_skinny_bn == 256 ||
-                   (g_skinny_bn == 0 && (wide_bn256 || (long)(N / 256) * slices(256) % 256 == 0))))
-    bn = 256;
-  const int S = slices(bn);
+  if (g_skinny == 1 && !chosen && (M < 17 || M > 192 || (skinny_wide(N) && !skinny_wide_bn256(M, N)))) return 0;
+  const int bn = skinny_bn(M, N, K);
+  const int S = skinny_slices(N, K, bn);
   const bool direct_epi = EPI == FLS_EPI_NONE || EPI == FLS_EPI_RESID || EPI == FLS_EPI_SWIGLU;
   const bool direct = S == 1 && direct_epi;
   if (direct) {

@@ -20,8 +20,9 @@ constexpr int EPI_ROPE64 = 4;
 // epilogue runs in splitk_reduce_kernel, gemm.hip)
 constexpr int EPI_F32 = 6;
 constexpr bool is_rope(int epi) { return epi == FLS_EPI_ROPE || epi == EPI_ROPE64; }
-constexpr int BUF = 65536;    // one K-tile stage: X image (32 KiB) then W image (32 KiB)
-constexpr int WIMG = 32768;
+// one K-tile stage of v10 with 64 HX rows: X image (8 HX KiB) then W image (32 KiB)
+constexpr int v10_stage(int hx) { return 8192 * hx + 32768; }
+constexpr int BUF = v10_stage(4);
 
 struct Epi {
   const half_t* R;
@@ -437,6 +438,21 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, -1, 0x00020000);
 }
 
+// at most N of the wave's LDS-DMAs still in flight
+template <int N>
+__device__ __forceinline__ void wait_dmas() {
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
+// every accumulator stays in its accumulation register up to here
+template <int U>
+__device__ __forceinline__ void fence_acc(floatx4 (&acc)[U][8]) {
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int t = 0; t < 8; ++t) asm volatile("" : "+a"(acc[u][t]));
+}
+
 // Grouped (mixture-of-experts) form of v10 (GRP): G row groups (experts) share one launch.  Group e
 // owns rows [g_offs[e], g_offs[e+1]) of C, its M tiles are virtual tiles [g_tiles[e], g_tiles[e+1])
 // (ceil of its rows / BM), its weight is W + e * g_wstride, and its A rows are either contiguous from
@@ -446,16 +462,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base) {
 // block -> tile mapping and the others exit before touching LDS: mapped over the bound, whole XCDs got few or no
 // tiles (128 experts, 48,608 rows, 2048 -> 2 x 768: 452 -> 345 us; 768 -> 2048: 335 -> 283).  The N tiles of an M tile go one
 // after the other where there are at most eight: an expert's A rows are read once (342 and 261; 384 rows: 226 -> 197).
-template <int EPI, bool GRP = false>
-__global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__ A, const half_t* __restrict__ W,
-                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
-                                                    int ldc, Epi ep) {
+template <int EPI, bool GRP, int HX>
+__device__ __forceinline__ void tile_v10(const half_t* __restrict__ A, const half_t* __restrict__ W,
+                                         half_t* __restrict__ C, int M, int N, int K, int lda, int ldw, int ldc,
+                                         const Epi& ep) {
+  constexpr int TM = 64 * HX, WOFF = TM * 128, STG = v10_stage(HX);
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-  int tiles_m = (M + BM - 1) / BM;
+  int tiles_m = (M + TM - 1) / TM;
   const int tiles_n = N / BN;
   int nwg = gridDim.x;
   int bid = blockIdx.x;
@@ -496,36 +513,39 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__
     Wg += (size_t)ks * ep.kslice;
     Cg = (half_t*)((float*)C + (size_t)ks * ep.part_stride);
   }
-  const int m0 = tm * BM, n0 = tn * BN;
+  const int m0 = tm * TM, n0 = tn * BN;
 
-  // staging: a half-tile = 16 pieces of 8 rows x 128 B, rows {(j>>3)*128 + (j&7)*8} (+64 for the B half);
-  // wave w moves pieces 4w .. 4w+3
+  // staging: a half-tile = 16 pieces (of X: 4 HX) of 8 rows x 128 B, W rows {(j>>3)*128 + (j&7)*8} (+64 for the B half), X
+  // rows {j / (2 HX) * 32 HX + j % (2 HX) * 8} (+ 16 HX); wave w moves W pieces 4w .. 4w+3, X pieces HX w .. HX w + HX - 1
   const int lr = lane >> 3;
   const int lc = (lane & 7) ^ lr;
-  int prow[4];
+  int prow[4], xprow[HX];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = 4 * wave + i;
     prow[i] = (j >> 3) * 128 + (j & 7) * 8;
   }
+#pragma unroll
+  for (int i = 0; i < HX; ++i) {
+    const int j = HX * wave + i;
+    xprow[i] = j / (2 * HX) * (32 * HX) + j % (2 * HX) * 8;
+  }
   // per-lane 32-bit byte offsets; the K offset goes into the (scalar) base pointer so every
   // LDS-DMA is the saddr + voffset form (no per-lane 64-bit address registers)
-  unsigned xo[8], wo[8];
+  unsigned xo[2 * HX], wo[8];
   const size_t wb_off = (size_t)64 * ldw * 2;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (GRP) {
-      int ra = min(m0 + prow[i] + lr, M - 1), rb = min(m0 + prow[i] + 64 + lr, M - 1);
-      if (rows) {
-        ra = rows[ra];
-        rb = rows[rb];
+  for (int i = 0; i < HX; ++i)
+#pragma unroll
+    for (int hb = 0; hb < 2; ++hb) {
+      int r = min(m0 + xprow[i] + hb * 16 * HX + lr, M - 1);
+      if constexpr (GRP) {
+        if (rows) r = rows[r];
       }
-      xo[i] = (unsigned)(ra * lda + lc * 8) * 2u;
-      xo[4 + i] = (unsigned)(rb * lda + lc * 8) * 2u;
-    } else {
-      xo[i] = (unsigned)(min(m0 + prow[i] + lr, M - 1) * lda + lc * 8) * 2u;
-      xo[4 + i] = (unsigned)(min(m0 + prow[i] + 64 + lr, M - 1) * lda + lc * 8) * 2u;
+      xo[hb * HX + i] = (unsigned)(r * lda + lc * 8) * 2u;
     }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
     if constexpr (EPI == FLS_EPI_SWIGLU) {
 #pragma unroll
       for (int hb = 0; hb < 2; ++hb) {
@@ -543,78 +563,63 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__
   const __amdgpu_buffer_rsrc_t rZ = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(Ab), (short)0, 0, 0x00020000);
 // LDS-DMA of one 1 KiB piece: buffer_load ... lds with the per-lane 32-bit offset and the K (and
 // half-tile) step in soffset (0.5-1% over the global_load_lds form, profiles/r2_gemm)
-#define V10_DMA_X(rs, k0, idx, dst)                                                                \
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, xo[idx], (k0) * 2, 0, 0)
+#define V10_DMA_X(rs, k0, buf, hb, i)                                                              \
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(                                                        \
+      rs, (LDS_AS void*)(smem + (buf) * STG + (xprow[i] + (hb) * 16 * HX) * 128), 16, xo[(hb) * HX + (i)], (k0) * 2, 0, 0)
 #define V10_DMA_W(rs, hb, i, k0, dst)                                                              \
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16,                             \
       EPI == FLS_EPI_SWIGLU ? wo[(hb) * 4 + (i)] : wo[(i)],                                         \
       (EPI == FLS_EPI_SWIGLU ? 0u : (unsigned)((hb) * wb_off)) + (k0) * 2, 0, 0)
 #define V10_X(buf, hb, k0)                                                                         \
-  _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_)                                                \
-    V10_DMA_X(rA, k0, (hb) * 4 + i_, smem + (buf) * BUF + (prow[i_] + (hb) * 64) * 128);
+  _Pragma("unroll") for (int i_ = 0; i_ < HX; ++i_) V10_DMA_X(rA, k0, buf, hb, i_);
 #define V10_W(buf, hb, k0)                                                                         \
   _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_)                                                \
-    V10_DMA_W(rW, hb, i_, k0, smem + (buf) * BUF + WIMG + (prow[i_] + (hb) * 64) * 128);
+    V10_DMA_W(rW, hb, i_, k0, smem + (buf) * STG + WOFF + (prow[i_] + (hb) * 64) * 128);
 
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4;
   const int sw = fr & 7;
   const int c0 = ((0 + grp) ^ sw) << 4;
   const int c1 = ((4 + grp) ^ sw) << 4;
-  const int xrow = (wm * 128 + fr) * 128;
-  const int wrow = WIMG + (wn * 128 + fr) * 128;
+  const int xrow = (wm * 32 * HX + fr) * 128;
+  const int wrow = WOFF + (wn * 128 + fr) * 128;
 
-  floatx4 acc[8][8];
+  floatx4 acc[2 * HX][8];
 #pragma unroll
-  for (int u = 0; u < 8; ++u)
+  for (int u = 0; u < 2 * HX; ++u)
 #pragma unroll
     for (int t = 0; t < 8; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  half8 xf[8][2], wf[8][2];
-#define V10_FENCE_ACC()                                                                            \
-  _Pragma("unroll") for (int u_ = 0; u_ < 8; ++u_)                                                \
-  _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+a"(acc[u_][t_]));
+  half8 xf[2 * HX][2], wf[8][2];
   // zero-init (VALU AGPR writes) must not sit right before the first asm MFMA reading them
-  V10_FENCE_ACC();
+  fence_acc(acc);
   asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");
 
-#define V10_RX(buf, h)                                                                             \
-  _Pragma("unroll") for (int u_ = (h) * 4; u_ < (h) * 4 + 4; ++u_) {                              \
-    xf[u_][0] = *(const half8*)(smem + (buf) * BUF + xrow + u_ * 2048 + c0);                      \
-    xf[u_][1] = *(const half8*)(smem + (buf) * BUF + xrow + u_ * 2048 + c1);                      \
-  }
-#define V10_RW(buf, h)                                                                             \
-  _Pragma("unroll") for (int t_ = (h) * 4; t_ < (h) * 4 + 4; ++t_) {                              \
-    wf[t_][0] = *(const half8*)(smem + (buf) * BUF + wrow + t_ * 2048 + c0);                      \
-    wf[t_][1] = *(const half8*)(smem + (buf) * BUF + wrow + t_ * 2048 + c1);                      \
-  }
-// one phase: 32 MFMAs (k-step outer, 4x4 tiles of the quadrant) with, in issue order,
-// one ds_read after each of the first 16 even-numbered MFMAs and the half-tile's 4
-// LDS-DMA ops after MFMAs 17, 20, 23, 26; then lgkmcnt(0) + counted vmcnt + barrier.
-// RX: 1 = read an X half, 0 = a W half.
+#define V10_RX(buf, f, k) xf[f][k] = *(const half8*)(smem + (buf) * STG + xrow + (f) * 2048 + ((k) ? c1 : c0))
+#define V10_RW(buf, f, k) wf[f][k] = *(const half8*)(smem + (buf) * STG + wrow + (f) * 2048 + ((k) ? c1 : c0))
+// one phase: 8 HX MFMAs (k-step outer, HX x 4 tiles of the quadrant) with, in issue order, one ds_read
+// after each of the first even-numbered MFMAs (2 HX for an X half, 8 for a W half) and the half-tile's
+// HX or 4 LDS-DMA ops after every third later MFMA; SYNC: then lgkmcnt(0) + counted vmcnt + barrier.
+// RX, DX: 1 = an X half, 0 = a W half.
 #define V10_PHASE(xh, wh, RX, rbuf, rh, DX, dbuf, dhb, dk0, SYNC)                                  \
   {                                                                                               \
-    _Pragma("unroll") for (int i_ = 0; i_ < 32; ++i_) {                                           \
-      const int s_ = i_ >> 4, u_ = (xh) * 4 + ((i_ >> 2) & 3), t_ = (wh) * 4 + (i_ & 3);          \
+    _Pragma("unroll") for (int i_ = 0; i_ < 8 * HX; ++i_) {                                       \
+      const int s_ = i_ / (4 * HX), u_ = (xh) * HX + (i_ >> 2) % HX, t_ = (wh) * 4 + (i_ & 3);    \
       mfma_acc_inplace_ordered(acc[u_][t_], wf[t_][s_], xf[u_][s_]);                              \
-      if (i_ < 16 && (i_ & 1) == 0) {                                                             \
-        const int rj_ = i_ >> 1;                                                                  \
-        const int f_ = (rh) * 4 + (rj_ >> 1), k_ = rj_ & 1;                                       \
-        if (RX)                                                                                   \
-          xf[f_][k_] = *(const half8*)(smem + (rbuf) * BUF + xrow + f_ * 2048 + (k_ ? c1 : c0));  \
-        else                                                                                      \
-          wf[f_][k_] = *(const half8*)(smem + (rbuf) * BUF + wrow + f_ * 2048 + (k_ ? c1 : c0));  \
+      if (i_ < (RX ? 4 * HX : 16) && (i_ & 1) == 0) {                                             \
+        const int f_ = i_ >> 2, k_ = (i_ >> 1) & 1;                                               \
+        if (RX) V10_RX(rbuf, (rh) * HX + f_, k_);                                                 \
+        else V10_RW(rbuf, (rh) * 4 + f_, k_);                                                     \
       }                                                                                           \
-      if (i_ >= 17 && i_ <= 26 && (i_ - 17) % 3 == 0) {                                           \
-        const int p_ = (i_ - 17) / 3;                                                             \
-        if (DX)                                                                                   \
-          V10_DMA_X(rX##dk0, dk0, (dhb) * 4 + p_, smem + (dbuf) * BUF + (prow[p_] + (dhb) * 64) * 128); \
-        else                                                                                      \
-          V10_DMA_W(rW##dk0, dhb, p_, dk0, smem + (dbuf) * BUF + WIMG + (prow[p_] + (dhb) * 64) * 128); \
+      constexpr int D0_ = HX == 4 ? 17 : HX == 3 ? 13 : 5, DN_ = DX ? HX : 4;                     \
+      if (i_ >= D0_ && i_ < D0_ + 3 * DN_ && (i_ - D0_) % 3 == 0) {                               \
+        const int p_ = (i_ - D0_) / 3;                                                            \
+        if (DX) V10_DMA_X(rX##dk0, dk0, dbuf, dhb, p_);                                           \
+        else V10_DMA_W(rW##dk0, dhb, p_, dk0, smem + (dbuf) * STG + WOFF + (prow[p_] + (dhb) * 64) * 128); \
       }                                                                                           \
     }                                                                                             \
     if (SYNC) {                                                                                   \
       __builtin_amdgcn_s_waitcnt(0xC07F);                 /* lgkmcnt(0) */                        \
-      asm volatile("s_waitcnt vmcnt(16)" ::: "memory");                                           \
+      wait_dmas<2 * HX + 8>();                                                                    \
       __builtin_amdgcn_s_barrier();                                                               \
     }                                                                                             \
   }
@@ -624,11 +629,15 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__
   // prologue = virtual SPs -4..-1: [XA0 WA0] [WB0 XB0] [XA1 WB1] [WA1 XB1]
   V10_X(0, 0, 0); V10_W(0, 0, 0); V10_W(0, 1, 0); V10_X(0, 1, 0);
   V10_X(1, 0, kc1); V10_W(1, 1, kc1); V10_W(1, 0, kc1); V10_X(1, 1, kc1);
-  asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+  wait_dmas<3 * HX + 12>();
   __builtin_amdgcn_s_barrier();
-  V10_RX(0, 0); V10_RW(0, 0);                  // SP -1's reads: x0(0), w0(0)
+#pragma unroll
+  for (int f = 0; f < 4; ++f) {                // SP -1's reads: x0(0), w0(0)
+    if (f < HX) { V10_RX(0, f, 0); V10_RX(0, f, 1); }
+    V10_RW(0, f, 0); V10_RW(0, f, 1);
+  }
   __builtin_amdgcn_s_waitcnt(0xC07F);
-  asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+  wait_dmas<2 * HX + 8>();
   __builtin_amdgcn_s_barrier();
   for (int kt = 0; kt < nk; kt += 2) {
     const int ka = min(kt + 2, nk - 1) * BK;   // tile kt+2 -> buf 0
@@ -653,8 +662,7 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__
   // the nops give the last ones their passes, and the tied empty asms (ordered after the
   // nops, being volatile too) make every later AGPR read depend on them
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
-  V10_FENCE_ACC();
-#undef V10_FENCE_ACC
+  fence_acc(acc);
 #undef V10_RW
 #undef V10_RX
 #undef V10_W
@@ -662,10 +670,17 @@ __global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__
 #undef V10_DMA_X
 #undef V10_DMA_W
 
-  epilogue_quadrant<EPI>(Cg, ldc, M, m0 + wm * 128 + fr, n0 + wn * 128, grp, acc, ep);
+  epilogue_quadrant<EPI, 2 * HX>(Cg, ldc, M, m0 + wm * 32 * HX + fr, n0 + wn * 128, grp, acc, ep);
 }
 
 #undef V10_PHASE
+
+template <int EPI, bool GRP = false, int HX = 4>
+__global__ __launch_bounds__(256, 1) void gemm_nt_v10(const half_t* __restrict__ A, const half_t* __restrict__ W,
+                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
+                                                    int ldc, Epi ep) {
+  tile_v10<EPI, GRP, HX>(A, W, C, M, N, K, lda, ldw, ldc, ep);
+}
 
 // Default tile order (profiles/r2_gemm/README.md).  Groups of g tiles of one dimension are walked
 // along the other; the XCD remap gives XCD x the virtual ids [x*q, (x+1)*q), q = tiles / 8.

@@ -366,14 +366,16 @@ extern "C" int fls_gemm_set_v11_cost(int cost) {
 
 // Applicability of v11 for a launch; the shape rules of gemm.hip's v10 main path plus M >= 384.
 // Called from fls_gemm (gemm.hip) before its own dispatch.  Returns 1 and launches when v11 takes
-// the GEMM, 0 when it does not apply, < 0 on a launch error.
+// the GEMM, 0 when it does not apply, < 0 on a launch error.  want (auto mode): 1 the caller's estimate
+// picked it, -1 another path, 0 decide here.
 extern "C" int fls_gemm_v11_try(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda,
                                 int ldw, int ldc, int ldr, int epi, const int* pos, const float* cos_t,
                                 const float* sin_t, int rope_cols, int head_dim, const void* bias,
-                                const float* rscale, float alpha, float* ss, int ss_ld, fls_stream_t s) {
+                                const float* rscale, float alpha, float* ss, int ss_ld, int want, fls_stream_t s) {
   using namespace v11;
   if (!g_v11 || M < TM || N % TN || K % TK || (K / TK) % 2 || lda % 8 || ldw % 8) return 0;
-  if (g_v11 == 1) {
+  if (g_v11 == 1 && want < 0) return 0;
+  if (g_v11 == 1 && want == 0) {
     // fills the chip (at least one tile per CU per launch) and takes no longer in whole tile rounds
     if ((size_t)((M + TM - 1) / TM) * (N / TN) < 256 || !v11_pays(M, N)) return 0;
   }

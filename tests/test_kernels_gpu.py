@@ -418,6 +418,66 @@ def test_gemm_main_all_epilogues(ops, ref):
         ops.k.fls_gemm_set_mid(1)
 
 
+# 128- and 192-row forms of the 256-column tile: bit for bit the 256-row form (the same MFMAs in the same order per output), which
+# test_gemm_main_all_epilogues holds to fp32; rows at the edges of every form's tiles, two K tiles (the least) and more
+@pytest.mark.parametrize("epi", ["none", "resid", "swiglu", "rope128", "rope64"])
+def test_gemm_tile_rows_bitwise(ops, epi):
+    from flexible_llm_sharding_amd.config import ModelConfig
+    from flexible_llm_sharding_amd.models.llama import rope_tables
+    k = ops.k
+    old = (k.fls_gemm_set_v11(0), k.fls_gemm_set_mid(0), k.fls_gemm_set_skinny(0, 0), k.fls_gemm_set_splitk(0))
+    try:
+        for M, N, K in ((1, 256, 128), (64, 512, 128), (65, 512, 256), (127, 256, 384), (129, 512, 256), (192, 256, 128), (193, 512, 256),
+                        (255, 256, 256), (385, 512, 512), (641, 768, 256)):
+            x, w, b = rnd(M, K, seed=M), rnd(N, K, scale=0.05, seed=N + M), rnd(N, seed=3)
+            rs = torch.rand(M, device=DEV) + 0.5
+            r0 = rnd(M, N, seed=5)
+            outs = []
+            for rows in (256, 192, 128):
+                assert k.fls_gemm_set_v10_rows(rows) in (0, 128, 192, 256)
+                if epi == "none":
+                    outs.append((ops.gemm(x, w, bias=b, rscale=rs),))
+                elif epi == "resid":
+                    ss = torch.full((M, N // 128), -1.0, device=DEV)
+                    outs.append((ops.gemm(x, w, EPI_RESID, out=r0.clone(), resid=r0, bias=b, alpha=0.7, rscale=rs, ss=ss), ss))
+                elif epi == "swiglu":
+                    outs.append((ops.gemm(x, w, EPI_SWIGLU, rscale=rs),))
+                else:
+                    hd = int(epi[4:])
+                    cfg = ModelConfig(hidden_size=N, num_attention_heads=N // hd, num_key_value_heads=N // hd)
+                    cos, sin = rope_tables(cfg, 1024)
+                    pos = torch.arange(M, dtype=torch.int32, device=DEV) % 1000
+                    outs.append((ops.gemm(x, w, EPI_ROPE, positions=pos, cos=cos.to(DEV), sin=sin.to(DEV), rope_cols=128, head_dim=hd,
+                                          bias=b, rscale=rs),))
+            for o in outs[1:]:
+                assert all(torch.equal(p, q) for p, q in zip(o, outs[0])), (M, N, K)
+            if epi == "none":
+                assert rel_err(outs[0][0], rs[:, None] * (x.float() @ w.float().t()) + b.float()) < 2e-3
+    finally:
+        k.fls_gemm_set_v10_rows(0)
+        k.fls_gemm_set_v11(old[0])
+        k.fls_gemm_set_mid(old[1])
+        k.fls_gemm_set_skinny(old[2], 0)
+        k.fls_gemm_set_splitk(old[3])
+    torch.cuda.synchronize()
+
+
+# whichever path the estimate picks (65 rows on): against fp32 (fp16 result: 2e-3 as above), with scratch and without (rows that share no
+# product with others: the row-exact form, bit for bit the same rows of a larger call)
+@pytest.mark.parametrize("N,K", [(512, 2048), (5120, 2048), (12288, 1024), (2048, 8192), (1024, 256)])
+def test_gemm_route_by_estimate(ops, N, K):
+    w = rnd(N, K, scale=0.05, seed=7)
+    big = rnd(1300, K, seed=8)
+    with ops.row_exact():
+        whole = ops.gemm(big, w)
+    for M in (65, 100, 161, 200, 256, 257, 300, 385, 512, 513, 640, 1025, 1300):
+        x = big[:M]
+        assert rel_err(ops.gemm(x, w), x.float() @ w.float().t()) < 2e-3
+        with ops.row_exact():
+            assert torch.equal(ops.gemm(x, w), whole[:M])
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("hd", [128, 64])
 def test_gemm_row_exact_small_m_bitwise(ops, ref, hd):
     """Row-exact small-M GEMMs (generation steps): every row of M = 1 / 17 / 64 / 160 / 320 equals,
