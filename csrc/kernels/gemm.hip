@@ -634,13 +634,29 @@ float rounds_us(const RoundCost& c, long blocks, int nk) {
   return (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * fill * fill : 0.f);
 }
 
+// Up to 64 rows one row tile covers them all and a product is a stream of its weight: the choice is between blocks of 16, 32 or
+// 64 columns over the whole K (ROUTE_MID; bound by a K tile's chain of wait, read and MFMA where K is long) and the K-split skinny
+// blocks with their partial sums (8 rows: 12,288 x 4,096 25 and 29 us, 4,096 x 11,008 22 and 23, 8,192 x 28,672 137 and 85; on
+// split 256-row tiles, where up to 16 rows went before, 39, 23 and 111).
+//
 // ws: scratch for split-K partials (0 bytes: none).  Above four rounds of 256-row tiles the forms are within 3% of each other:
 // ROUTE_NONE (v11 or v10 by whole rounds, v11_pays)
-Route route_of(int M, int N, int K, bool row_exact, size_t ws_bytes) {
+Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
   const int nk = K / BK;
+  const float bytes = (float)N * K * 2.f;                      // the weight, once
   const long cols = N / BN;
   const long tiles256 = (long)((M + 255) / 256) * cols;
-  if (M <= 64 || M > ROW_CHUNK || tiles256 > 1024 || g_v10_rows || g_mid_bn || g_mid_waves || g_mid_rows || g_skinny > 1) return ROUTE_NONE;
+  if (M > ROW_CHUNK || tiles256 > 1024 || g_v10_rows || g_mid_bn || g_mid_waves || g_mid_rows || g_skinny > 1) return ROUTE_NONE;
+  if (M <= 64) {
+    if (row_exact || !g_mid || !g_skinny) return ROUTE_NONE;
+    const bool narrow = (epi == FLS_EPI_NONE || epi == FLS_EPI_RESID) && N / 32 < 256;       // (16-column blocks)
+    const float mid = narrow ? (N / 16 > 256 ? 6.5f : 4.f) + fmaxf(bytes / 4.8e6f, 0.08f * nk) + (M <= 16 ? 0.f : M <= 32 ? 0.03f : 0.062f) * nk
+                             : fmaxf(bytes / 5.8e6f + 7.f, 0.33f * nk + 3.f) + 0.05f * M;
+    const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
+    if ((S > 1 && (size_t)S * M * N * 4 > ws_bytes) || (skinny_wide(N) && M > 32)) return ROUTE_MID;
+    const float skinny = 7.f + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * nk / S) + (S > 1 ? S * (float)M * N * 1e-6f : 0.f);
+    return mid <= skinny ? ROUTE_MID : ROUTE_SKINNY;
+  }
   Route best = ROUTE_NONE;
   float least = 0.f;
   auto offer = [&](Route r, float us) {
@@ -651,7 +667,6 @@ Route route_of(int M, int N, int K, bool row_exact, size_t ws_bytes) {
   };
   for (int i = 0; i < 3; ++i) offer((Route)(ROUTE_128 + i), rounds_us(ROUNDS[i], (long)((M + ROUNDS[i].rows - 1) / ROUNDS[i].rows) * cols, nk));
   if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], (long)((M + 383) / 384) * cols, nk));
-  const float bytes = (float)N * K * 2.f;                      // the weight, once
   if (g_mid) {               // 64 x 128 blocks: two share a CU, and from the third round on the weights' re-reads take over
     const long blocks = (long)((M + 63) / 64) * (N / 128), r = (blocks + 255) / 256;
     const float fill = bytes > 64e6f ? 1.f : 0.35f + 0.65f * (float)(blocks - 256) / 256.f;
@@ -670,7 +685,7 @@ Route route_of(int M, int N, int K, bool row_exact, size_t ws_bytes) {
       const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
       const long r = ((long)(N / bn) * S + 255) / 256;         // (its K tile: all of the rows go through LDS)
       if (S == 1 || (size_t)S * M * N * 4 <= ws_bytes)
-        offer(ROUTE_SKINNY, 7.f + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * r * nk / S) + (S > 1 ? 0.5f * S * slab : 0.f));
+        offer(ROUTE_SKINNY, (r > 2 ? 10.f : 7.f) + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * r * nk / S) + (S > 1 ? 0.5f * S * slab : 0.f));
     }
   }
   return best;
@@ -948,7 +963,7 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
   if ((epi == FLS_EPI_SWIGLU || epi == FLS_EPI_ROPE) && (N % 32)) return -2;
   if (epi == FLS_EPI_ROPE && ((head_dim != 64 && head_dim != 128) || rope_cols % head_dim || N % head_dim))
     return -3;
-  Route route = N % BN == 0 && K % (2 * BK) == 0 ? route_of(M, N, K, row_exact != 0, ws ? ws_bytes : 0) : ROUTE_NONE;
+  Route route = N % BN == 0 && K % (2 * BK) == 0 ? route_of(M, N, K, epi, row_exact != 0, ws ? ws_bytes : 0) : ROUTE_NONE;
   {
     const int rc = fls_gemm_v11_try(A, W, C, R, M, N, K, lda, ldw, ldc, ldr, epi, pos, cos_t, sin_t, rope_cols,
                                     head_dim, bias, rscale, alpha, ss, ss_ld,

@@ -462,7 +462,7 @@ def test_gemm_tile_rows_bitwise(ops, epi):
     torch.cuda.synchronize()
 
 
-# whichever path the estimate picks (65 rows on): against fp32 (fp16 result: 2e-3 as above), with scratch and without (rows that share no
+# whichever path the estimate picks: against fp32 (fp16 result: 2e-3 as above), with scratch and without (rows that share no
 # product with others: the row-exact form, bit for bit the same rows of a larger call)
 @pytest.mark.parametrize("N,K", [(512, 2048), (5120, 2048), (12288, 1024), (2048, 8192), (1024, 256)])
 def test_gemm_route_by_estimate(ops, N, K):
@@ -470,9 +470,11 @@ def test_gemm_route_by_estimate(ops, N, K):
     big = rnd(1300, K, seed=8)
     with ops.row_exact():
         whole = ops.gemm(big, w)
-    for M in (65, 100, 161, 200, 256, 257, 300, 385, 512, 513, 640, 1025, 1300):
+    for M in (1, 2, 15, 16, 17, 31, 33, 64, 65, 100, 161, 200, 256, 257, 300, 385, 512, 513, 640, 1025, 1300):
         x = big[:M]
         assert rel_err(ops.gemm(x, w), x.float() @ w.float().t()) < 2e-3
+        r0 = rnd(M, N, seed=9)
+        assert rel_err(ops.gemm(x, w, EPI_RESID, out=r0.clone(), resid=r0), r0.float() + x.float() @ w.float().t()) < 2e-3
         with ops.row_exact():
             assert torch.equal(ops.gemm(x, w), whole[:M])
     torch.cuda.synchronize()
