@@ -7,7 +7,10 @@ call ``runtime_or_none()``.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
+import sysconfig
 import threading
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -15,6 +18,7 @@ _KERNELS = os.path.join(HERE, "libfls_kernels.so")
 _RUNTIME = os.path.join(HERE, "libfls_runtime.so")
 _COMM = os.path.join(HERE, "libfls_comm.so")
 _SEQ = os.path.join(HERE, "libfls_seq.so")
+_FASTCALL = os.path.join(HERE, "fls_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 _lock = threading.Lock()
 _libs = {}
@@ -27,6 +31,29 @@ def _bind(lib, name, restype, *argtypes):
     f = getattr(lib, name)
     f.restype = restype
     f.argtypes = list(argtypes)
+
+
+def _fastcall():
+    if not os.path.exists(_FASTCALL):
+        raise RuntimeError(f"native extension {_FASTCALL} is missing — build it with "
+                           f"`python -m flexible_llm_sharding_amd._native.build`")
+    loader = importlib.machinery.ExtensionFileLoader("fls_fastcall", _FASTCALL)
+    mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("fls_fastcall", loader))
+    loader.exec_module(mod)
+    return mod
+
+
+class _Quick:
+    """A library whose bound functions are called through ``fls_fastcall`` (csrc/python/fastcall.c) instead of ctypes, which
+    remains for the arguments that one does not take."""
+
+    def __init__(self, lib: ctypes.CDLL):
+        self._lib, self._name = lib, lib._name
+        function = _fastcall().function
+        kinds = {c_void_p: "p", c_int: "i", ctypes.c_longlong: "l", c_int64: "l", c_uint64: "l", c_float: "f"}
+        for name, f in list(vars(lib).items()):
+            if isinstance(f, lib._FuncPtr) and f.argtypes is not None and f.restype is c_int:
+                setattr(self, name, function(ctypes.cast(f, c_void_p).value, "".join(kinds[t] for t in f.argtypes), f))
 
 
 def _load_runtime():
@@ -128,7 +155,7 @@ def _load_kernels(path: str = _KERNELS):
     _bind(lib, "fls_gemv_skinny", c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
           c_void_p)
     _bind(lib, "fls_fill_random", c_int, c_void_p, c_uint64, c_uint64, c_float, c_float, c_void_p)
-    return lib
+    return _Quick(lib)
 
 
 SEQ_ABI = 20   # csrc/include/fls_seq.h
@@ -189,7 +216,7 @@ def _load_seq():
     _bind(lib, "fls_seq_sigmoid_gate", i, p, i, i, p, i, p, i, i, i, i, p)
     _bind(lib, "fls_seq_diff_combine", i, p, i, p, i, f, i, i, f, p, i, i, i, p)
     _bind(lib, "fls_seq_hgrn2_scan", i, p, i, p, i, p, i, p, p, p, p, i, p, p, p, i, i, i, i, p)
-    return lib
+    return _Quick(lib)
 
 
 def _load_comm():

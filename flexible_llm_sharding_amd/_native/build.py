@@ -3,7 +3,9 @@
 * ``libfls_kernels.so`` — every ``csrc/kernels/*.hip`` compiled by
   ``hipcc --offload-arch=gfx950`` (CDNA4 only) and linked into one library;
 * ``libfls_runtime.so`` — ``csrc/runtime/*.cpp`` host runtime (g++ against
-  libamdhip64).
+  libamdhip64);
+* ``fls_fastcall.<interpreter>.so`` — the Python extension the kernel libraries are called through (gcc against
+  this interpreter's headers).
 
 Objects are rebuilt only when a source or header is newer.  Usage::
 
@@ -17,6 +19,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -32,6 +35,7 @@ SEQ_SO = os.path.join(HERE, "libfls_seq.so")
 NO_PK_F32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 RUNTIME_SO = os.path.join(HERE, "libfls_runtime.so")
 COMM_SO = os.path.join(HERE, "libfls_comm.so")
+FASTCALL_SO = os.path.join(HERE, "fls_fastcall" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
 def _hipcc() -> str:
@@ -141,12 +145,23 @@ def build_comm(force=False, verbose=False):
     return COMM_SO
 
 
+def build_fastcall(force=False, verbose=False):
+    """fls_fastcall: the Python extension the kernel libraries are called through (csrc/python)."""
+    src = os.path.join(CSRC, "python", "fastcall.c")
+    if not (force or _stale(FASTCALL_SO, [src])):
+        return FASTCALL_SO
+    _run([shutil.which("gcc") or "gcc", "-O2", "-fPIC", "-shared", "-Wall", "-I", sysconfig.get_paths()["include"], src, "-o", FASTCALL_SO],
+         verbose)
+    return FASTCALL_SO
+
+
 def build_all(force=False, jobs=8, verbose=False):
     rt = build_runtime(force=force, verbose=verbose)
     k = build_kernels(force=force, jobs=jobs, verbose=verbose)
     c = build_comm(force=force, verbose=verbose)
     q = build_seq_kernels(force=force, jobs=jobs, verbose=verbose)
-    return rt, k, c, q
+    f = build_fastcall(force=force, verbose=verbose)
+    return rt, k, c, q, f
 
 
 def main(argv=None):

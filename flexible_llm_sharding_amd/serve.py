@@ -23,12 +23,13 @@ from .runtime.weights import CheckpointSource, HostStore
 
 def ensure_built(device: torch.device) -> None:
     """Build what serving a hybrid model on a GPU loads, if it is not there: the host runtime (pinned
-    memory) and the stateful-model kernels.  Nothing of the scoring kernels is compiled."""
+    memory), the stateful-model kernels and the extension that calls them.  Nothing of the scoring kernels is compiled."""
     if device.type != "cuda":
         return
     from ._native import build
     build.build_runtime()
     build.build_seq_kernels()
+    build.build_fastcall()
 
 
 def load_runner(model_path: str, dtype: torch.dtype, device=None, max_tokens: int = 4096, max_seqs: int = 8,

@@ -1,0 +1,60 @@
+"""The extension that the kernel libraries are called through (csrc/python/fastcall.c) against ctypes: the same C functions, the same
+arguments, each signature length that it passes in another way (up to 16, 32 and 64 integers), floats between the integers."""
+import ctypes
+import random
+import shutil
+import subprocess
+
+import pytest
+
+from flexible_llm_sharding_amd import _native
+
+TYPES = {"p": ctypes.c_void_p, "i": ctypes.c_int, "l": ctypes.c_longlong, "f": ctypes.c_float}
+SIGS = ["i", "p", "fi", "pipipippiiffiiiiiiippliillp"[:26] + "p", "f" * 8 + "i" * 16, "if" * 8 + "p" * 9, "pl" * 16, "ppi" * 21 + "f", "l" * 64]
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    if shutil.which("gcc") is None:
+        pytest.skip("no gcc")
+    c = {"p": "const void*", "i": "int", "l": "long long", "f": "float"}
+    src = "#include <stdio.h>\nstatic char out[8192];\nconst char* seen(void) { return out; }\n"
+    for n, sig in enumerate(SIGS):
+        put = "".join(f"n += sprintf(out + n, \"{'%a' if k == 'f' else '%lld'} \", {'(double)a' if k == 'f' else '(long long)a'}{i});" for i, k in enumerate(sig))
+        src += f"int f{n}({', '.join(f'{c[k]} a{i}' for i, k in enumerate(sig))}) {{ int n = 0; {put} return -n; }}\n"
+    d = tmp_path_factory.mktemp("fastcall")
+    (d / "f.c").write_text(src)
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-w", str(d / "f.c"), "-o", str(d / "f.so")], check=True)
+    lib = ctypes.CDLL(str(d / "f.so"))
+    lib.seen.restype = ctypes.c_char_p
+    for n, sig in enumerate(SIGS):
+        _native._bind(lib, f"f{n}", ctypes.c_int, *(TYPES[k] for k in sig))
+    return lib
+
+
+def test_same_arguments_as_ctypes(lib):
+    quick, rng = _native._Quick(lib), random.Random(0)
+    for n, sig in enumerate(SIGS):
+        for _ in range(20):
+            args = [rng.choice((None, 0, rng.getrandbits(47))) if k == "p" else rng.randint(-2 ** 31, 2 ** 31 - 1) if k == "i"
+                    else rng.randint(-2 ** 63, 2 ** 63 - 1) if k == "l" else rng.choice((rng.uniform(-1e3, 1e3), 3, float("inf"))) for k in sig]
+            want = (getattr(lib, f"f{n}")(*args), lib.seen())
+            assert (getattr(quick, f"f{n}")(*args), lib.seen()) == want
+
+
+def test_other_arguments_go_to_ctypes(lib):
+    quick = _native._Quick(lib)
+    buf = ctypes.create_string_buffer(8)
+    assert quick.f1(buf) == lib.f1(buf)                              # (an address that only ctypes knows how to take)
+    for call in ((quick.f0, "x"), (quick.f0, None), (quick.f0, 1.5), (quick.f2, "x", 1), (quick.f0,), (quick.f2, 1.0)):
+        with pytest.raises((ctypes.ArgumentError, TypeError)):
+            call[0](*call[1:])
+
+
+def test_refuses_what_it_cannot_pass():
+    f = _native._fastcall().function
+    for sig in ("d", "f" * 9, "i" * 65):
+        with pytest.raises(ValueError):
+            f(1, sig, None)
+    with pytest.raises(ValueError):
+        f(0, "i", None)
