@@ -31,20 +31,38 @@ __device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {
 __device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
   if (e.kind == EPI_DECAY) r.ap = -expf(e.act[col / e.act_n]);
 }
-__device__ __forceinline__ float epi_value(float v, const Epi& e, const EpiRegs& r) {
-  if (e.kind == EPI_RELU2) { v = fmaxf(v, 0.f); v *= v; }
-  else if (e.kind == EPI_DECAY) v = expf(r.ap * softplus_f(v));
-  else if (e.kind == EPI_XIELU) v = v > 0.f ? r.ap * v * v + 0.5f * v : r.an * (expm1f(v) - v) + 0.5f * v;
-  else if (e.kind == EPI_SOFTCAP) v = e.p * tanhf(v / e.p);
-  else if (e.kind == EPI_SCALE) v *= e.p;
-  return v;
+template <int KIND>
+__device__ __forceinline__ float epi_value_of(float v, const Epi& e, const EpiRegs& r) {
+  if constexpr (KIND == EPI_RELU2) { v = fmaxf(v, 0.f); return v * v; }
+  else if constexpr (KIND == EPI_DECAY) return expf(r.ap * softplus_f(v));
+  else if constexpr (KIND == EPI_XIELU) {
+    const float low = both_sides(r.an * expm1_less_z(v));
+    return (v > 0.f ? r.ap * v * v : low) + 0.5f * v;
+  }
+  else if constexpr (KIND == EPI_SOFTCAP) return e.p * tanhf(v / e.p);
+  else if constexpr (KIND == EPI_SCALE) return v * e.p;
+  else return v;
 }
-__device__ __forceinline__ float epi_gate(float g, float u, const Epi& e) {
-  if (e.kind == EPI_GATE) return silu_f(g) * u;
-  if (e.kind == EPI_GATE + 1) return gelu_tanh_f(g) * u;
+template <int KIND>
+__device__ __forceinline__ float epi_gate_of(float g, float u, const Epi& e) {
+  if constexpr (KIND == EPI_GATE) return silu_f(g) * u;
+  else if constexpr (KIND == EPI_GATE + 1) return gelu_tanh_f(g) * u;
   g = fminf(g, e.p);
   u = fminf(fmaxf(u, -e.p), e.p);
   return g / (1.f + expf(-e.q * g)) * (u + 1.f);
+}
+__device__ __forceinline__ float epi_value(float v, const Epi& e, const EpiRegs& r) {
+  if (e.kind == EPI_RELU2) return epi_value_of<EPI_RELU2>(v, e, r);
+  if (e.kind == EPI_DECAY) return epi_value_of<EPI_DECAY>(v, e, r);
+  if (e.kind == EPI_XIELU) return epi_value_of<EPI_XIELU>(v, e, r);
+  if (e.kind == EPI_SOFTCAP) return epi_value_of<EPI_SOFTCAP>(v, e, r);
+  if (e.kind == EPI_SCALE) return epi_value_of<EPI_SCALE>(v, e, r);
+  return v;
+}
+__device__ __forceinline__ float epi_gate(float g, float u, const Epi& e) {
+  if (e.kind == EPI_GATE) return epi_gate_of<EPI_GATE>(g, u, e);
+  if (e.kind == EPI_GATE + 1) return epi_gate_of<EPI_GATE + 1>(g, u, e);
+  return epi_gate_of<EPI_GATE + 2>(g, u, e);
 }
 __device__ __forceinline__ void emit(void* C, size_t idx, float v, const Epi& e, const EpiRegs& r) {
   v = epi_value(v, e, r);

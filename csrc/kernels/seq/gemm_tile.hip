@@ -146,9 +146,10 @@ __device__ __forceinline__ void hold(floatx4& c) {
   if constexpr (ACC) asm volatile("" : "+a"(c));
 }
 
-// A wave's outputs: acc[u][t] = rows mw + 16 u + (lane & 15), columns nw + 16 t + 4 (lane >> 4) .. + 3.  Without an activation
-// they leave straight from the registers.  An activation runs in a short loop over rows that the wave first lays down in
-// its own piece of LDS (PU row groups at a time): unrolled over all accumulators its code would be larger than the cache.
+// A wave's outputs: acc[u][t] = rows mw + 16 u + (lane & 15), columns nw + 16 t + 4 (lane >> 4) .. + 3.  The wave lays them down in its
+// own piece of LDS (PU row groups at a time) and takes them up row by row, so that a store covers whole rows of the tile (straight from the
+// registers it was pieces of 32 or 64 bytes of 16 rows: 16384 x 4096 x 4096 404 -> 392 us, 9692 x 10880 x 2048 390 -> 340) and an
+// activation is a short loop: unrolled over all accumulators its code would be larger than the cache.
 template <int MI, int NJ, int PU, bool ACC>
 __device__ __forceinline__ void lay_down(floatx4 (&acc)[MI][NJ], int p, char* lds) {
   constexpr int CH = 4 * NJ;
@@ -162,6 +163,39 @@ __device__ __forceinline__ void lay_down(floatx4 (&acc)[MI][NJ], int p, char* ld
       *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = acc[p * PU + u][t];
     }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (the wave's own rows: no other wave reads them)
+}
+
+// The rows that a wave laid down: a loop for each kind of epilogue.  With the kind asked for at each value the loop was a chain of
+// branches over the other kinds' code, and a wave that has its SIMD to itself waits for the instructions after each: 16384 x 14336 x
+// 4096 with xIELU 1827 us, 1523 so (branches in xIELU itself: 1572); 9692 x 10880 x 2048 silu gates 469 and 362.
+template <int NJ, int PU, int TC, int KIND>
+__device__ __forceinline__ void value_rows(const Tile& a, const EpiRegs (&er)[4], floatx4 b, size_t cbase, int m0, int n, int mend, const char* lds) {
+  constexpr int CH = 4 * NJ, RI = 64 / CH;          // 16-byte chunks of a row; rows per step of the loop
+  const int lane = threadIdx.x & 63, c = lane % CH;
+#pragma unroll 2
+  for (int i = 0; i < 16 * PU; i += RI) {
+    const int r = i + lane / CH;
+    floatx4 v = *reinterpret_cast<const floatx4*>(lds + (r * CH + (c ^ (r & (CH - 1)))) * 16) + b;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = epi_value_of<KIND>(v[x], a.epi, er[x]);
+    if (m0 + r < mend && n < a.N) store4<TC>(a.C, cbase + (size_t)(m0 + r) * a.ldc + n, v);
+  }
+}
+template <int NJ, int PU, int TC, int KIND>
+__device__ __forceinline__ void gate_rows(const Tile& a, int m0, int nw, int mend, const char* lds) {
+  constexpr int CH = 4 * NJ, RI = 64 / CH;
+  const int lane = threadIdx.x & 63, c = lane % (CH / 2), cg = (c >> 2) * 8 + (c & 3);      // column chunk, its gate chunk (the up chunk: + 4)
+  const int n = (nw >> 1) + 4 * c;
+#pragma unroll 2
+  for (int i = 0; i < 16 * PU; i += 2 * RI) {
+    const int r = i + lane / (CH / 2);
+    const floatx4 g = *reinterpret_cast<const floatx4*>(lds + (r * CH + (cg ^ (r & (CH - 1)))) * 16);
+    const floatx4 u = *reinterpret_cast<const floatx4*>(lds + (r * CH + ((cg + 4) ^ (r & (CH - 1)))) * 16);
+    floatx4 v;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = epi_gate_of<KIND>(g[x], u[x], a.epi);
+    if (m0 + r < mend && n < (a.N >> 1)) store4<TC>(a.C, (size_t)(m0 + r) * a.ldc + n, v);
+  }
 }
 
 template <int MI, int NJ, int PU, bool ACC, int TC>
@@ -185,48 +219,21 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
       return;
     }
   }
-  if (e.kind == 0) {
-#pragma unroll
-    for (int t = 0; t < NJ; ++t) {
-      asm volatile("" ::: "memory");                        // (one column group at a time: fewer live registers)
-      const int n = nw + t * 16 + 4 * grp;
-      if (n < a.N) {
-        floatx4 b = {0.f, 0.f, 0.f, 0.f};
-        if (e.bias != nullptr) b = *reinterpret_cast<const floatx4*>(e.bias + cbase + n);
-        const size_t at = cbase + (size_t)(mw + fr) * a.ldc + n;
-#pragma unroll
-        for (int u = 0; u < MI; ++u) {
-          hold<ACC>(acc[u][t]);
-          if (mw + u * 16 + fr < mend) store4<TC>(a.C, at + (size_t)(u * 16) * a.ldc, acc[u][t] + b);
-        }
-      }
-    }
-    return;
-  }
-  constexpr int CH = 4 * NJ, RI = 64 / CH;          // 16-byte chunks of a row; rows per step of the loop
+  constexpr int CH = 4 * NJ;                         // 16-byte chunks of a row
   if (NJ >= 2 && e.kind >= EPI_GATE) {               // (no bias: the gated products have none)
-    const int c = lane % (CH / 2), cg = (c >> 2) * 8 + (c & 3);          // column chunk, its gate chunk (the up chunk: + 4)
-    const int n = (nw >> 1) + 4 * c;
 #pragma unroll
     for (int p = 0; p < MI / PU; ++p) {
       lay_down<MI, NJ, PU, ACC>(acc, p, lds);
-#pragma unroll 1
-      for (int i = 0; i < 16 * PU; i += 2 * RI) {
-        const int r = i + lane / (CH / 2);
-        const floatx4 g = *reinterpret_cast<const floatx4*>(lds + (r * CH + (cg ^ (r & (CH - 1)))) * 16);
-        const floatx4 u = *reinterpret_cast<const floatx4*>(lds + (r * CH + ((cg + 4) ^ (r & (CH - 1)))) * 16);
-        floatx4 v;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) v[x] = epi_gate(g[x], u[x], e);
-        const int m = mw + p * PU * 16 + r;
-        if (m < mend && n < (a.N >> 1)) store4<TC>(a.C, (size_t)m * a.ldc + n, v);
-      }
+      const int m0 = mw + p * PU * 16;
+      if (e.kind == EPI_GATE) gate_rows<NJ, PU, TC, EPI_GATE>(a, m0, nw, mend, lds);
+      else if (e.kind == EPI_GATE + 1) gate_rows<NJ, PU, TC, EPI_GATE + 1>(a, m0, nw, mend, lds);
+      else gate_rows<NJ, PU, TC, EPI_GATE + 2>(a, m0, nw, mend, lds);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     return;
   }
   const EpiRegs er0 = epi_regs(e);
-  const int c = lane % CH, n = nw + 4 * c;
+  const int n = nw + 4 * (lane % CH);
   EpiRegs er[4] = {er0, er0, er0, er0};
   floatx4 b = {0.f, 0.f, 0.f, 0.f};
   if (n < a.N) {
@@ -237,14 +244,14 @@ __device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ],
 #pragma unroll
   for (int p = 0; p < MI / PU; ++p) {
     lay_down<MI, NJ, PU, ACC>(acc, p, lds);
-#pragma unroll 1
-    for (int i = 0; i < 16 * PU; i += RI) {
-      const int r = i + lane / CH;
-      floatx4 v = *reinterpret_cast<const floatx4*>(lds + (r * CH + (c ^ (r & (CH - 1)))) * 16) + b;
-#pragma unroll
-      for (int x = 0; x < 4; ++x) v[x] = epi_value(v[x], e, er[x]);
-      const int m = mw + p * PU * 16 + r;
-      if (m < mend && n < a.N) store4<TC>(a.C, cbase + (size_t)m * a.ldc + n, v);
+    const int m0 = mw + p * PU * 16;
+    switch (e.kind) {
+      case EPI_XIELU: value_rows<NJ, PU, TC, EPI_XIELU>(a, er, b, cbase, m0, n, mend, lds); break;
+      case EPI_RELU2: value_rows<NJ, PU, TC, EPI_RELU2>(a, er, b, cbase, m0, n, mend, lds); break;
+      case EPI_DECAY: value_rows<NJ, PU, TC, EPI_DECAY>(a, er, b, cbase, m0, n, mend, lds); break;
+      case EPI_SOFTCAP: value_rows<NJ, PU, TC, EPI_SOFTCAP>(a, er, b, cbase, m0, n, mend, lds); break;
+      case EPI_SCALE: value_rows<NJ, PU, TC, EPI_SCALE>(a, er, b, cbase, m0, n, mend, lds); break;
+      default: value_rows<NJ, PU, TC, 0>(a, er, b, cbase, m0, n, mend, lds);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }

@@ -332,7 +332,7 @@ __global__ void xielu_kernel(const float* __restrict__ z, int ldz, const float* 
   TO* yr = y + (size_t)blockIdx.x * ldy;
   for (int c = threadIdx.x; c < cols; c += blockDim.x) {
     const float v = zr[c];
-    stf(yr, c, v > 0.f ? ap * v * v + 0.5f * v : an * (expm1f(v) - v) + 0.5f * v);
+    stf(yr, c, v > 0.f ? ap * v * v + 0.5f * v : an * expm1_less_z(v) + 0.5f * v);
   }
 }
 

@@ -48,6 +48,25 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
+// x, computed here and not in a branch of what chooses it: a lane's short alternatives side by side are cheaper than a wave's turns
+__device__ __forceinline__ float both_sides(float x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+// exp(z) - 1 - z for z <= 0, the negative side of xIELU, without branches and no further from it than expm1f(z) - z: down to -1, where
+// that difference cancels, z^2 times the polynomial that interpolates (exp(z) - 1 - z) / z^2 at seven Chebyshev nodes (6e-10
+// relative); below, exp(z) - (1 + z) with exp(z) = 2^h (1 + l ln 2), h + l = z log2(e) to twice fp32's digits.  xIELU with it against
+// 64 bits, root mean square of the relative error over z in [-1, 0] 1.1e-7 (1.5e-7 with expm1f), [-0.01, 0] 2.6e-8 (6.2e-8), [-100, -5]
+// 1.1e-7 (the same).
+__device__ __forceinline__ float expm1_less_z(float z) {
+  const float p = z * z * (0.5f + z * (0.166666643f + z * (0.0416662902f + z * (0.00833105026f + z * (0.00138224157f + z * (0.000188324755f +
+                  z * 1.69281272e-5f))))));
+  const float t = fmaxf(z, -128.f);                          // (2^h is 0 long before; NaN stays in 1 + z)
+  const float h = t * 1.44269502f, l = fmaf(t, 1.92596303e-8f, fmaf(t, 1.44269502f, -h));
+  const float e = __builtin_amdgcn_exp2f(h);
+  const float far = both_sides(fmaf(e, l * 0.693147182f, e) - (1.f + z));
+  return z > -1.f ? both_sides(p) : far;
+}
 __device__ __forceinline__ float sigmoid_f(float z) { return 1.f / (1.f + expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.f + expf(-z)); }
 // gelu, tanh form: 0.5 z (1 + tanh(u)) with u = sqrt(2/pi) (z + 0.044715 z^3), written as z sigmoid(2u):

@@ -396,6 +396,24 @@ def test_epilogue_bf16_values(ops, kind):
     assert bool((err <= want[:, None].abs() * 2 ** -8 + (1 + (z6 * (u6.abs() + 1)).abs())[:, None] * 2.0 ** -126).all())
 
 
+# xIELU's negative side on both sides of its seam at -1, near 0 (where exp(z) - 1 cancels) and far out, against fp64: 3 ulp of
+# (exp(z) - 1 - z) (1/2 + softplus(q)) and one of each of the sums' terms
+def test_xielu_against_fp64(ops):
+    H, _ = ops
+    act = torch.tensor([0.3, -0.2])
+    p, q = torch.nn.functional.softplus(act.double())
+    ap, an = p, 0.5 + q
+    z = torch.cat([torch.linspace(a, b, 4096) for a, b in ((-100, -20), (-20, -1), (-1.01, -0.99), (-1, 0), (-1e-2, 0), (-1e-4, 0), (0, 5))]
+                  + [torch.tensor([-1.0, -0.99999994, -1.0000001, -0.0, 0.0, -200.0, -1e30, 1e-30, -1e-30])])
+    d = z.double()
+    low = torch.where(d > -1e-2, d * d * (0.5 + d * (1 / 6 + d * (1 / 24 + d / 120))), torch.expm1(d) - d)
+    want = torch.where(d > 0, ap * d * d, an * low) + 0.5 * d
+    got = H.xielu(z[None].to(DEV), act.to(DEV), torch.float32).cpu().double()[0]
+    ulp = 2.0 ** -23
+    assert bool(((got - want).abs() <= ulp * (3 * torch.where(d > 0, ap * d * d, an * low) + 0.5 * d.abs() + want.abs()) + 1e-44).all())
+    assert torch.isnan(H.xielu(torch.tensor([[float("nan")]], device=DEV), act.to(DEV), torch.float32)).all()
+
+
 # an activation of the same sum has the same bits from the few-row kernel, the tiles and the kernels for any size (every sum here is one
 # product, exact in any order)
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
