@@ -20,11 +20,13 @@ int fls_seq_version(void);
 // = [gate rows; up rows] (N / 2 each), C has N / 2 columns: silu(g) u, gelu(g) u, or the clamped gate of fls_seq_gate_mul
 // with limit p and alpha q; no bias), stored as type tc (fp32, or bf16 when the consumer is the next product).
 // a_rows (with offs; nullable): row r of the product is made from row a_rows[r] of A, which has at most M rows.
-// SEQ_NOT_SERVED: nothing was done -- a gated product or a_rows, and rows whose alignment or size only the general kernels take.
+// mirror (nullable): a cell on the device that holds an address the device can write (pinned host memory, say): the results, fp32 rows of
+// N, go there too.
+// SEQ_NOT_SERVED: nothing was done -- a mirror of anything but a plain product of up to 32 rows; a gated product or a_rows, and rows whose alignment or size only the general kernels take.
 #define SEQ_NOT_SERVED (-100)
 int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias, const float* act,
                  int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
-                 const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s);
+                 const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, float* const* mirror, fls_stream_t s);
 // the tile that such a product of aligned rows takes, as its index in the table of these types (gemm_tile.hip); by_rows: row groups.  On the host
 // alone, for the tests that hold every tile
 int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated);
@@ -74,7 +76,10 @@ int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col, int x_hs, 
                            const float* freqs, int rot, const int* tok_pos, const int* row_map, void* out, int to,
                            int ldo, int out_col, int out_hs, void* raw, int ldr, int rows, int unit_after, int half, float amp,
                            fls_stream_t s);
-int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, fls_stream_t s);
+// (host, nullable: a cell as fls_seq_gemm's mirror; the indexes go behind rows x cols floats there as well, and with_rows the rows before them)
+int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, void* const* host, int with_rows, fls_stream_t s);
+// dst[0 .. n) = src[0 .. n): index arrays of a step from pinned host memory, as a kernel of the step's own graph
+int fls_seq_copy_words(const int* src, int* dst, int n, fls_stream_t s);
 // k rows RMS-normed over all kcols (times kn), k and v rows written at row kv_slot[r] of the pools
 int fls_seq_kv_store(const float* k, int ldk, const float* kn, float eps, const float* v, int ldv, void* kc, void* vc,
                      int tc, const int* kv_slot, int rows, int kcols, int vcols, fls_stream_t s);

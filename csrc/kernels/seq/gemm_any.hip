@@ -305,18 +305,21 @@ static void launch(int big, dim3 grid, hipStream_t st, const void* A, const void
 
 extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias_p,
                             const float* act, int act_kind, int act_n, float act_p, float act_q, int M, int N, int K, int lda, int ldw, int ldc,
-                            int groups, const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, fls_stream_t s) {
+                            int groups, const int* offs, const int* a_rows, long long a_gs, int a_mod, long long w_gs, long long c_gs, float* const* mirror,
+                            fls_stream_t s) {
   if (act_kind < 0 || act_kind > EPI_LAST || ((act_kind == EPI_XIELU || act_kind == EPI_DECAY) && act == nullptr)) return -1;
   if (act_kind == EPI_DECAY && (act_n < 1 || groups != 1 || offs != nullptr)) return -1;
   if (act_kind >= EPI_GATE && (N % 2 || bias_p != nullptr || (groups != 1 && offs == nullptr))) return -1;
   if (a_rows != nullptr && offs == nullptr) return -1;
-  const Epi bias = {bias_p, act, act_kind, tc, act_n, act_p, act_q};
+  const Epi bias = {bias_p, act, act_kind, tc, act_n, act_p, act_q, mirror};
   if (M <= 0 || N <= 0) return 0;
   if (K <= 0 || groups < 1 || (ta == 1 && tw == 0)) return -1;
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
   const int vec_a = aligned16(A, lda, ea, K) && (a_gs * ea) % 16 == 0;
   const int vec_w = aligned16(W, ldw, ew, K) && (w_gs * ew) % 16 == 0;
   const hipStream_t st = (hipStream_t)s;
+  if (mirror != nullptr && (tc != 0 || act_kind >= EPI_GATE || offs != nullptr || groups != 1 || M > 32 || N % 4 || !vec_a || !vec_w))
+    return SEQ_NOT_SERVED;                 // (only the few-row kernel writes twice)
   if (vec_a && vec_w) {
     // Few rows: bound by reading W, no tile to fill.  40 rows x 2048 x 2048: 12 us, the best tile 7.  Row groups: 8 rows each on average, and
     // 128 in all (64 in fp32), because their sizes are on the device and a router may send most rows to one: a block then reads its weight

@@ -120,18 +120,27 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
           for (int w = 0; w < WV; ++w) v2 += red[w][u * HW + 1][l];
         }
         EpiRegs er = epi_regs(epi);
+        if constexpr (GATED) {
 #pragma unroll
-        for (int x = 0; x < 4; ++x) {
-          const int col = col0 + x;
-          if (col >= N) continue;
-          if constexpr (GATED) {
+          for (int x = 0; x < 4; ++x) {
+            const int col = col0 + x;
+            if (col >= N) continue;
             const float o = epi_gate(v[x], v2[x], epi);
             if (epi.tc == 1) reinterpret_cast<bf16_t*>(C)[(size_t)row * ldc + col] = f_to_bf16(o);
             else reinterpret_cast<float*>(C)[(size_t)row * ldc + col] = o;
-          } else {
-            epi_column(epi, er, col);
-            emit(C, (size_t)row * ldc + col, v[x] + (epi.bias != nullptr ? epi.bias[col] : 0.f), epi, er);
           }
+        } else {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            const int col = col0 + x;
+            if (col >= N) continue;
+            epi_column(epi, er, col);
+            v[x] = epi_value(v[x] + (epi.bias != nullptr ? epi.bias[col] : 0.f), epi, er);
+            if (epi.tc == 1) reinterpret_cast<bf16_t*>(C)[(size_t)row * ldc + col] = f_to_bf16(v[x]);
+            else reinterpret_cast<float*>(C)[(size_t)row * ldc + col] = v[x];
+          }
+          // (N is a multiple of 4 then: rows of N, 64 bytes of one a store)
+          if (epi.mirror != nullptr && col0 < N) *reinterpret_cast<floatx4*>(*epi.mirror + (size_t)row * N + col0) = v;
         }
       }
     }

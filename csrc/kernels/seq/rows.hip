@@ -425,22 +425,31 @@ extern "C" int fls_seq_unary(const float* z, int ldz, void* y, int ty, int ldy, 
 // first index of the row maximum.  Few rows (decoding): a block per row, so what bounds it is one block's chain of loads: 1024
 // threads with 16-byte loads (32000 columns: 8 loads deep, 6 us; 256 threads of single loads 21)
 #define ARGMAX_THREADS 1024
-__global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __restrict__ z, int ldz, int cols, int vec, int* __restrict__ out) {
+__global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __restrict__ z, int ldz, int cols, int vec, int* __restrict__ out,
+                                                               void* const* __restrict__ host, int with_rows) {
   __shared__ float bv[ARGMAX_THREADS];
   __shared__ int bi[ARGMAX_THREADS];
   const float* zr = z + (size_t)blockIdx.x * ldz;
+  float* const hr = host != nullptr && with_rows ? reinterpret_cast<float*>(*host) + (size_t)blockIdx.x * cols : nullptr;
   float best = -INFINITY;
   int at = 0x7fffffff;
   const int c4 = vec ? cols & ~3 : 0;
   for (int c = 4 * threadIdx.x; c < c4; c += 4 * ARGMAX_THREADS) {
     const float4 q = *reinterpret_cast<const float4*>(zr + c);
     const float v[4] = {q.x, q.y, q.z, q.w};
+    if (hr != nullptr) {
+      if (cols % 4 == 0) *reinterpret_cast<float4*>(hr + c) = q;
+      else
+#pragma unroll
+        for (int i = 0; i < 4; ++i) hr[c + i] = v[i];
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       if (v[i] > best || (v[i] == best && c + i < at)) { best = v[i]; at = c + i; }
   }
   for (int c = c4 + threadIdx.x; c < cols; c += ARGMAX_THREADS) {
     const float v = zr[c];
+    if (hr != nullptr) hr[c] = v;
     if (v > best || (v == best && c < at)) { best = v; at = c; }
   }
   bv[threadIdx.x] = best;
@@ -454,12 +463,34 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __r
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[blockIdx.x] = bi[0] == 0x7fffffff ? 0 : bi[0];
+  if (threadIdx.x == 0) {
+    const int best_at = bi[0] == 0x7fffffff ? 0 : bi[0];
+    out[blockIdx.x] = best_at;
+    if (host != nullptr) reinterpret_cast<int*>(*host)[(size_t)gridDim.x * cols + blockIdx.x] = best_at;
+  }
 }
 
-extern "C" int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, fls_stream_t s) {
+extern "C" int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, void* const* host, int with_rows, fls_stream_t s) {
   if (rows <= 0) return 0;
-  hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(ARGMAX_THREADS), 0, (hipStream_t)s, z, ldz, cols, (uintptr_t)z % 16 == 0 && ldz % 4 == 0, out);
+  hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(ARGMAX_THREADS), 0, (hipStream_t)s, z, ldz, cols, (uintptr_t)z % 16 == 0 && ldz % 4 == 0, out,
+                     host, with_rows);
+  SEQ_LAUNCH_CHECK();
+  return 0;
+}
+
+__global__ __launch_bounds__(1024) void copy_words_kernel(const int* __restrict__ src, int* __restrict__ dst, int n) {
+  const int i = 4 * (blockIdx.x * 1024 + threadIdx.x);
+  if (i + 4 <= n) *reinterpret_cast<int4*>(dst + i) = *reinterpret_cast<const int4*>(src + i);
+  else
+    for (int j = i; j < n; ++j) dst[j] = src[j];
+}
+
+// A decode step's index arrays (some KB) over the host link by a kernel of the step's graph: 4 us, where a copy before the graph took 5
+// and left 20 of idle GPU between the two (8 requests, one step of 650 us).
+extern "C" int fls_seq_copy_words(const int* src, int* dst, int n, fls_stream_t s) {
+  if (n <= 0) return 0;
+  if ((uintptr_t)src % 16 || (uintptr_t)dst % 16) return -1;
+  hipLaunchKernelGGL(copy_words_kernel, dim3((n + 4095) / 4096), dim3(1024), 0, (hipStream_t)s, src, dst, n);
   SEQ_LAUNCH_CHECK();
   return 0;
 }
@@ -973,4 +1004,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 20; }
+extern "C" int fls_seq_version(void) { return 21; }

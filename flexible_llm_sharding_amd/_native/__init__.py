@@ -158,7 +158,7 @@ def _load_kernels(path: str = _KERNELS):
     return _Quick(lib)
 
 
-SEQ_ABI = 20   # csrc/include/fls_seq.h
+SEQ_ABI = 21   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -168,7 +168,7 @@ def _load_seq():
     if lib.fls_seq_version() != SEQ_ABI:
         raise RuntimeError(f"{_SEQ} is a stale build; rebuild with python -m flexible_llm_sharding_amd._native.build")
     p, i, f, ll = c_void_p, c_int, c_float, ctypes.c_longlong
-    _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p)
+    _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p, p)
     _bind(lib, "fls_seq_gemm_tile_of", i, i, i, i, i, i, i, i, i)
     _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm", i, p, i, p, i, p, p, i, p, f, i, i, i, f, p)
     _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
@@ -188,7 +188,8 @@ def _load_seq():
     _bind(lib, "fls_seq_unary", i, p, i, p, i, i, i, i, i, p)
     _bind(lib, "fls_seq_head_norm_rope", i, p, i, i, i, i, i, i, p, f, p, i, p, p, p, i, i, i, i, p, i, i, i, i, f, p)
     _bind(lib, "fls_seq_delta_rule_scan", i, p, i, p, i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, f, f, f, f, i, p, i, p, i, p)
-    _bind(lib, "fls_seq_argmax", i, p, i, i, i, p, p)
+    _bind(lib, "fls_seq_argmax", i, p, i, i, i, p, p, i, p)
+    _bind(lib, "fls_seq_copy_words", i, p, p, i, p)
     _bind(lib, "fls_seq_kv_store", i, p, i, p, f, p, i, p, p, i, p, i, i, i, p)
     _bind(lib, "fls_seq_attn_paged", i, p, i, i, p, i, p, i, i, p, i, i, p, p, p, i, i, i, i, i, i, f, f, p, p, i, i, i, p, f, i, i, p,
           i, f, p, p, i, i, i, p, i, p, i, p, i, p)

@@ -562,17 +562,14 @@ class ShardedRunner:
                 state = None
                 for name in self.names:
                     state = self._run_layer(self.ctx, name, self._W_all[name], state, None, meta)
-                return state, self.ops.argmax_f32(state)
-            self._decode_graphs = StepGraphs(self.dev, forward)
+                return state, self.ops.argmax_f32(state, meta["mirror"])
+            self._decode_graphs = StepGraphs(self.dev, forward, self.ops, self.cfg.vocab_size)
         batch = pack_step(entries, self.seq_cache)
-        logits, am = self._decode_graphs.run(batch, self.seq_cache.generation)
-        if any(e.want for e in entries):
-            lh, ah = self._decode_graphs.read(logits, am)          # (synchronous: the static outputs are reused)
+        got = self._decode_graphs.run(batch, self.seq_cache.generation, any(len(e.want) for e in entries))
+        if got is not None:
             for i, e in enumerate(entries):
                 if len(e.want):
-                    out[i] = (lh[i:i + 1].copy(), ah[i:i + 1].copy())
-        else:
-            torch.cuda.current_stream(self.dev).synchronize()
+                    out[i] = (got[0][i:i + 1], got[1][i:i + 1])
         for e in entries:
             self.seq_cache.trim(e.rid)
         self.stats = {"tokens": float(len(entries)), "graph_replays": float(self._decode_graphs.replays),

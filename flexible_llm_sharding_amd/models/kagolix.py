@@ -243,7 +243,7 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
     if kind == "norm":
         return ops.group_rmsnorm(state, W["norm"], cfg.norm_groups, cfg.norm_eps, out_dtype=ctx.compute_dtype,
                                  row_idx=meta["want_idx"])
-    return ops.matmul_nt(state, W["head"], softcap=cfg.logit_softcap)
+    return ops.matmul_nt(state, W["head"], softcap=cfg.logit_softcap, mirror=meta.get("mirror"))
 
 
 def layer_flops(cfg, name: str, rows: int, ctx_keys: float = 0.0) -> float:

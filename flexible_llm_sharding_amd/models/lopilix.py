@@ -319,7 +319,7 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
         return run_block(ctx, W, state, meta, name)
     if kind == "norm":
         return ops.streams_norm(state, None, W["norm"], cfg.norm_eps, ctx.compute_dtype, cfg.streams, row_idx=meta["want_idx"])
-    return ops.matmul_nt(state, W["head"], scale=cfg.logit_scale if cfg.logit_scale != 1.0 else None)
+    return ops.matmul_nt(state, W["head"], scale=cfg.logit_scale if cfg.logit_scale != 1.0 else None, mirror=meta.get("mirror"))
 
 
 def layer_flops(cfg, name: str, rows: int, ctx_keys: float = 0.0) -> float:

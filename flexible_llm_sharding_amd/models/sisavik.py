@@ -254,7 +254,7 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
     if kind == "norm":
         return ops.group_rmsnorm(state, W["norm"], 1, cfg.norm_eps, out_dtype=ctx.compute_dtype,
                                  row_idx=meta["want_idx"], w_offset=1.0)
-    return ops.matmul_nt(state, W["head"])
+    return ops.matmul_nt(state, W["head"], mirror=meta.get("mirror"))
 
 
 def layer_flops(cfg, name: str, rows: int, ctx_keys: float = 0.0) -> float:

@@ -46,6 +46,14 @@ def _vec(t: torch.Tensor, name: str, n: int, dtype=torch.float32):
     return t
 
 
+class HostRows:
+    """Where a step's logits and their argmax go on the host: ``cell`` (one int64 on the device) holds the address of rows x vocab
+    floats and, behind them, the rows' argmax; ``rows_there``: the logits are written already."""
+
+    def __init__(self, cell: torch.Tensor):
+        self.cell, self.rows_there = cell, False
+
+
 class HipSeqOps:
     name = "hip-seq"
     fused_norm = False
@@ -480,22 +488,24 @@ class HipSeqOps:
     NOT_SERVED = -100          # fls_seq.h SEQ_NOT_SERVED
 
     def _gemm(self, a, w, c, bias, M, N, K, lda, ldw, ldc, groups=1, offs=None, a_gs=0, a_mod=1, w_gs=0, c_gs=0,
-              act=None, kind=0, act_n=0, p=0.0, q=0.0, a_rows=None):
+              act=None, kind=0, act_n=0, p=0.0, q=0.0, a_rows=None, mirror=None):
         """-> False when only the general kernels take these rows and the call needs more than they do (nothing was done)."""
         rc = self.k.fls_seq_gemm(a.data_ptr(), _code(a, "a"), w.data_ptr(), _code(w, "w"), c.data_ptr(), _code(c, "c"),
                                  bias.data_ptr() if bias is not None else None,
                                  act.data_ptr() if act is not None else None, kind, act_n, float(p), float(q), M, N, K, lda, ldw, ldc, groups,
                                  offs.data_ptr() if offs is not None else None, a_rows.data_ptr() if a_rows is not None else None,
-                                 a_gs, a_mod, w_gs, c_gs, _stream())
+                                 a_gs, a_mod, w_gs, c_gs, mirror, _stream())
         if rc == self.NOT_SERVED:
             return False
         _chk(rc, "fls_seq_gemm")
         return True
 
-    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None):
+    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None,
+                  mirror=None):
         """a . w^T (+ bias); ``xielu`` ({p, q}), ``relu2`` (max(z, 0)^2), ``decay`` (rates of equal runs of columns:
         exp(-exp(rate) softplus(z))), ``softcap`` (cap tanh(z / cap)) or ``scale``: that activation in the epilogue;
-        ``out_dtype``: the accumulator as it is (fp32) or rounded for the next product (bf16)."""
+        ``out_dtype``: the accumulator as it is (fp32) or rounded for the next product (bf16); ``mirror`` (HostRows): the rows go
+        there as well where the product's kernel can (``mirror.rows_there``; else argmax_f32 takes them)."""
         _rows(a, "a")
         _rows(w, "w")
         M, K = a.shape
@@ -517,9 +527,13 @@ class HipSeqOps:
         if decay is not None:
             _vec(decay, "decay", decay.numel())
         c = torch.empty(M, N, dtype=out_dtype, device=a.device)
-        self._gemm(a, w, c, bias, M, N, K, a.stride(0), w.stride(0), N, act=xielu if decay is None else decay,
-                   kind=kinds[0] if kinds else 0, act_n=N // decay.numel() if decay is not None else 0,
-                   p=softcap if softcap is not None else (scale if scale is not None else 0.0))
+        more = dict(act=xielu if decay is None else decay, kind=kinds[0] if kinds else 0, act_n=N // decay.numel() if decay is not None else 0,
+                    p=softcap if softcap is not None else (scale if scale is not None else 0.0))
+        if mirror is not None:
+            mirror.rows_there = self._gemm(a, w, c, bias, M, N, K, a.stride(0), w.stride(0), N, mirror=mirror.cell.data_ptr(), **more)
+            if mirror.rows_there:
+                return c
+        self._gemm(a, w, c, bias, M, N, K, a.stride(0), w.stride(0), N, **more)
         return c
 
     def gated_matmul_nt(self, a, w, out_dtype, act="silu", limit=0.0, alpha=1.702, offs=None, rows=None):
@@ -670,12 +684,24 @@ class HipSeqOps:
              "fls_seq_head_norm_rope")
         return out
 
-    def argmax_f32(self, z):
+    def argmax_f32(self, z, mirror=None):
+        """The rows' argmax; with ``mirror`` (HostRows) it also goes behind the rows there, and the rows if they are not there yet."""
         _rows(z, "z", torch.float32)
         out = torch.empty(z.shape[0], dtype=torch.int32, device=z.device)
-        _chk(self.k.fls_seq_argmax(z.data_ptr(), z.stride(0), z.shape[0], z.shape[1], out.data_ptr(), _stream()),
-             "fls_seq_argmax")
+        _chk(self.k.fls_seq_argmax(z.data_ptr(), z.stride(0), z.shape[0], z.shape[1], out.data_ptr(),
+                                   mirror.cell.data_ptr() if mirror is not None else None,
+                                   int(mirror is not None and not mirror.rows_there), _stream()), "fls_seq_argmax")
         return out
+
+    def host_rows(self, cell):
+        return HostRows(_vec(cell, "cell", 1, torch.int64))
+
+    def copy_words(self, src, dst):
+        """dst = src, int32, by a kernel that reads ``src`` (pinned host memory) itself."""
+        if src.dtype != torch.int32 or dst.dtype != torch.int32 or not src.is_pinned() or not src.is_contiguous() or src.numel() < dst.numel():
+            raise TypeError("copy_words: contiguous int32, from pinned host memory")
+        _vec(dst, "dst", dst.numel(), torch.int32)
+        _chk(self.k.fls_seq_copy_words(src.data_ptr(), dst.data_ptr(), dst.numel(), _stream()), "fls_seq_copy_words")
 
     def gather_rows(self, x, idx, out=None):
         _rows(x, "x")

@@ -163,7 +163,8 @@ class TorchSeqOps:
         """o * sigmoid(g), element by element."""
         return (o.float() * torch.sigmoid(g.float())).to(out_dtype)
 
-    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None):
+    def matmul_nt(self, a, w, bias=None, xielu=None, out_dtype=torch.float32, relu2=False, decay=None, softcap=None, scale=None,
+                  mirror=None):
         """``decay`` (rates [R] of equal runs of output columns): exp(-exp(rate) softplus(y)) of the biased product; ``softcap``:
         cap tanh(y / cap); ``scale``: scale y."""
         if a.dtype != w.dtype:

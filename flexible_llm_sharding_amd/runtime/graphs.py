@@ -35,6 +35,7 @@ import numpy as np
 import torch
 
 from .batch import WORK_ITEM_FIELDS, PackedBatch
+from .hostmem import alloc_host
 
 TOKEN_BUCKET = 256
 WORK_BUCKET = 32
@@ -234,6 +235,29 @@ class DecodeGraphs:
         return g.out
 
 
+class _StepInputs:
+    """A decode shape's index arrays: ``up`` (pinned) and ``flat`` (device), each array from a 64-byte boundary behind the first
+    ``head`` entries, and ``meta``, the device arrays by name."""
+
+    def __init__(self, host: Dict[str, np.ndarray], B: int, head: int, dev):
+        at = [head]
+        for v in host.values():
+            at.append(at[-1] + _ceil(v.size, 16))
+        self.up = torch.empty(at[-1], dtype=torch.int32, pin_memory=True)
+        self.flat = torch.empty(at[-1], dtype=torch.int32, device=dev)
+        words = self.up.numpy()
+        self.address = words[:2].view(np.int64)
+        self.views = [words[o:o + v.size].reshape(v.shape) for v, o in zip(host.values(), at)]
+        self.meta = {k: self.flat[o:o + v.size].view(v.shape) for (k, v), o in zip(host.items(), at)}
+        self.meta.update(n_seqs=B, max_rows=1)
+
+    def fill(self, host: Dict[str, np.ndarray], down: torch.Tensor) -> None:
+        """(the step that last read ``up`` has been waited for)"""
+        self.address[0] = down.data_ptr()
+        for dst, v in zip(self.views, host.values()):
+            dst[...] = v
+
+
 class StepGraphs:
     """Captured decode steps of a stateful (hybrid) model: one token per request, resident weights.
 
@@ -246,55 +270,34 @@ class StepGraphs:
     graphs are dropped.  Every row's logits are computed (``want_idx`` = all rows); the caller picks
     the wanted ones.
 
-    A step's index arrays are segments of one int32 buffer that goes up in one copy from pinned memory (nine
-    pageable ones were 145 us of a 950 us step of 8 requests); its logits and their argmax come down into pinned
-    memory, a copy each and one wait for both (:meth:`read`; pageable, the 1 MB of logits took another 100)."""
+    A step's index arrays are segments of one int32 buffer that the graph's first kernel fetches from pinned memory, and its
+    logits and their argmax go straight to pinned memory, by the kernels that make them, at the address the buffer begins with:
+    a step is one launch and one wait (with a copy before the graph and two behind it the GPU idled 60 of 650 us of a step of 8
+    requests)."""
 
     TABLE_BUCKET = 16
     KEYS = ("ids", "tok_seq", "tok_pos", "cu", "pos0", "slot", "page_table", "kv_slot", "want_idx")
+    MAX_SEEN = 128
+    ADDRESS = 16                # entries of the buffer before its first array; the results' address is in two of them
 
-    def __init__(self, device, forward: Callable, max_graphs: int = 8):
+    def __init__(self, device, forward: Callable, ops, vocab: int, max_graphs: int = 8):
         self.dev = torch.device(device)
-        self.forward = forward              # forward(meta) -> (logits [B, V] fp32, argmax [B] int32)
+        self.forward = forward              # forward(meta) -> (logits [B, V] fp32, argmax [B] int32), written to meta["mirror"] too
+        self.ops = ops
+        self.vocab = int(vocab)
         self.max_graphs = max_graphs
         self.pool = torch.cuda.graph_pool_handle()
         self.graphs: "OrderedDict[tuple, _Graph]" = OrderedDict()
-        self.seen: set = set()
+        self.seen: "OrderedDict[tuple, _StepInputs]" = OrderedDict()      # shapes a step of which has run
         self.captures = self.replays = self.eager = 0
         self.generation = -1
-        self._up: Optional[torch.Tensor] = None        # pinned images of the index arrays and of the results
-        self._down: Optional[torch.Tensor] = None
-        self._up_read: Optional[torch.cuda.Event] = None
+        self._down: Optional[torch.Tensor] = None      # pinned: where a step's results go
 
-    def _pack(self, host: Dict[str, np.ndarray]) -> Tuple[torch.Tensor, List[int]]:
-        """The arrays back to back in pinned memory, each from a 64-byte boundary -> (that memory, their offsets)."""
-        offs = [0]
-        for v in host.values():
-            offs.append(offs[-1] + _ceil(v.size, 16))
-        if self._up is None or self._up.numel() < offs[-1]:
-            self._up = torch.empty(2 * offs[-1], dtype=torch.int32, pin_memory=True)
-        elif self._up_read is not None:
-            self._up_read.synchronize()                # the copy that last read it has run
-        flat = self._up.numpy()
-        for o, v in zip(offs, host.values()):
-            flat[o:o + v.size] = v.reshape(-1)
-        return self._up[:offs[-1]], offs
-
-    def _send(self, up: torch.Tensor, dev: torch.Tensor) -> None:
-        dev.copy_(up, non_blocking=True)
-        self._up_read = torch.cuda.Event()
-        self._up_read.record(torch.cuda.current_stream(self.dev))
-
-    def read(self, logits: torch.Tensor, am: torch.Tensor) -> Tuple[np.ndarray, np.ndarray]:
-        """The step's logits and argmax on the host, in memory that the next call reuses."""
-        n, B = logits.numel(), am.numel()
-        if self._down is None or self._down.numel() < n + B:
-            self._down = torch.empty(n + B, dtype=torch.float32, pin_memory=True)
-        lh, ah = self._down[:n].view(logits.shape), self._down[n:n + B].view(torch.int32)
-        lh.copy_(logits, non_blocking=True)
-        ah.copy_(am, non_blocking=True)
-        torch.cuda.current_stream(self.dev).synchronize()
-        return lh.numpy(), ah.numpy()
+    def _step(self, inputs: "_StepInputs"):
+        """The step's launches, its index arrays' arrival first."""
+        self.ops.copy_words(inputs.up, inputs.flat)
+        inputs.meta["mirror"] = self.ops.host_rows(inputs.flat[:2].view(torch.int64))
+        return self.forward(inputs.meta)
 
     @classmethod
     def _widened(cls, t: np.ndarray) -> np.ndarray:
@@ -313,8 +316,8 @@ class StepGraphs:
         m["want_idx"] = np.arange(B, dtype=np.int32)
         return m
 
-    def run(self, batch, generation: int):
-        """-> (logits, argmax) static device tensors of the step (valid until the next run)."""
+    def run(self, batch, generation: int, want: bool):
+        """One step, waited for -> (logits [B, V] fp32, argmax [B] int32) on the host, the caller's own; None without ``want``."""
         if generation != self.generation:
             self.graphs.clear()
             self.seen.clear()
@@ -322,33 +325,47 @@ class StepGraphs:
         B = len(batch.rids)
         host = self.host_meta(batch)
         key = (B,) + tuple(v.shape[1] for v in host.values() if v.ndim == 2)
+        n = 4 * B * (self.vocab + 1)
+        if self._down is None or self._down.numel() < n:
+            self._down = alloc_host(n)
+        try:
+            self._replay(key, host, B)
+        finally:                                       # (pinned memory of the step is not touched before its kernels are done)
+            torch.cuda.current_stream(self.dev).synchronize()
+        if not want:
+            return None
+        raw = self._down.numpy()[:n].copy()
+        return raw[:-4 * B].view(np.float32).reshape(B, self.vocab), raw[-4 * B:].view(np.int32)
+
+    def _replay(self, key, host, B: int) -> None:
         g = self.graphs.get(key)
-        up, offs = self._pack(host)
-        if g is None:
-            flat = torch.empty(up.numel(), dtype=torch.int32, device=self.dev)
-            self._send(up, flat)
-            meta = {k: flat[o:o + v.size].view(v.shape) for (k, v), o in zip(host.items(), offs)}
-            meta.update(n_seqs=B, max_rows=1)
-            if key not in self.seen:
-                self.seen.add(key)
+        if g is not None:
+            self.graphs.move_to_end(key)
+            g.inputs.fill(host, self._down)
+        else:
+            first = key not in self.seen
+            if first:
+                if len(self.seen) >= self.MAX_SEEN:
+                    self.seen.popitem(last=False)
+                self.seen[key] = _StepInputs(host, B, self.ADDRESS, self.dev)
+            inputs = self.seen[key]
+            inputs.fill(host, self._down)
+            if first:
                 self.eager += 1
-                return self.forward(meta)
+                self._step(inputs)
+                return
             if len(self.graphs) >= self.max_graphs:
                 self.graphs.popitem(last=False)
-            g = _Graph(meta)
-            g.flat = flat
+            g = _Graph(inputs.meta)
+            g.inputs = inputs
             s = torch.cuda.Stream(self.dev)
             s.wait_stream(torch.cuda.current_stream(self.dev))
             torch.cuda.synchronize(self.dev)
             with torch.cuda.graph(g.graph, pool=self.pool, stream=s):
-                g.out = self.forward(meta)
+                g.out = self._step(inputs)
             torch.cuda.synchronize(self.dev)
             self.graphs[key] = g
             self.captures += 1
-        else:
-            self.graphs.move_to_end(key)
-            self._send(up, g.flat)
         g.graph.replay()
         g.replays += 1
         self.replays += 1
-        return g.out

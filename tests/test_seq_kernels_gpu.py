@@ -396,6 +396,38 @@ def test_epilogue_bf16_values(ops, kind):
     assert bool((err <= want[:, None].abs() * 2 ** -8 + (1 + (z6 * (u6.abs() + 1)).abs())[:, None] * 2.0 ** -126).all())
 
 
+# results that go to pinned host memory by the kernels that make them: the few-row product's rows bit for bit (32 rows are its most), or,
+# where another kernel takes the product (more rows, columns that are no multiple of 4), the rows by the argmax; the argmax behind them
+@pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33])
+@pytest.mark.parametrize("N", [4, 20, 1000, 4100, 510, 1023])
+@pytest.mark.parametrize("cdt", [torch.bfloat16, torch.float32])
+def test_rows_written_to_the_host(ops, M, N, cdt):
+    H, _ = ops
+    g = torch.Generator().manual_seed(M + N)
+    a, w = torch.randn(M, 256, generator=g).to(cdt).to(DEV), torch.randn(N, 256, generator=g).to(cdt).to(DEV)
+    down = torch.full((M * N + M + 4,), -7.0, pin_memory=True)
+    cell = torch.tensor([down.data_ptr()], dtype=torch.int64, device=DEV)
+    for how in ({}, dict(softcap=5.0)):
+        down.fill_(-7.0)
+        mirror = H.host_rows(cell)
+        c = H.matmul_nt(a, w, mirror=mirror, **how)
+        assert mirror.rows_there == (M <= 32 and N % 4 == 0)
+        am = H.argmax_f32(c, mirror)
+        torch.cuda.synchronize()
+        assert torch.equal(c, H.matmul_nt(a, w, **how)) and torch.equal(am.cpu().long(), c.argmax(1).cpu())
+        assert torch.equal(down[:M * N].view(M, N), c.cpu()) and torch.equal(down[M * N:M * N + M].view(torch.int32), am.cpu())
+        assert bool((down[M * N + M:] == -7.0).all())
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 64, 4095, 4096, 4097, 9001])
+def test_copy_words_from_the_host(ops, n):
+    H, _ = ops
+    src = torch.randint(-2 ** 31, 2 ** 31 - 1, (n,), dtype=torch.int32).pin_memory()
+    dst = torch.full((n + 8,), 5, dtype=torch.int32, device=DEV)
+    H.copy_words(src, dst[:n])
+    assert torch.equal(dst[:n].cpu(), src) and bool((dst[n:] == 5).all())
+
+
 # xIELU's negative side on both sides of its seam at -1, near 0 (where exp(z) - 1 cancels) and far out, against fp64: 3 ulp of
 # (exp(z) - 1 - z) (1/2 + softplus(q)) and one of each of the sums' terms
 def test_xielu_against_fp64(ops):
