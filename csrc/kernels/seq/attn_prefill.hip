@@ -18,26 +18,34 @@
 //                      per reduction, and the running maximum, sum and rescale factor live in the
 //                      lane that owns the query;
 //   scores             scale, cap, distance penalty, mask (chunk / window / causal) in fp32;
-//   weights            exp in fp32, written to LDS as two bf16 terms (p = hi + lo, 16 mantissa bits
-//                      together), so the value product loses nothing to a bf16 rounding of p;
+//   weights            exp in fp32, then two bf16 terms (p = hi + lo, 16 mantissa bits together), so the
+//                      value product loses nothing to a bf16 rounding of p;
 //   O^T += V^T P^T     MFMAs again; O^T has the same column = query layout, so the rescale is a
-//                      per-lane multiply.
+//                      per-lane multiply.  The keys of V's rows stand in the order in which a lane holds
+//                      its scores, so the weights are the operand as they are.
 //
 // What bounds it is the vector work per score beside the matrix work (24 MFMAs, 768 cycles, per half tile and wave with heads of
-// 128).  So scores are in units of log 2: exp and log are one instruction each and the penalty needs no factor.  The cap and the
-// sigmoid weights come from exp(-|x|) and a reciprocal of [1, 2] that one Newton step makes as exact as a division (divisions: 468 us where
-// this takes 446; 172 and 194 with heads of 64).  bf16 terms come from the conversion instruction, and a half tile that every row of the
-// wave sees has no mask.  The accumulators are rescaled when a maximum grows, and only then: a query's largest weight is exactly 1,
-// which two bf16 terms hold without error (left up to 2^8 behind the maximum, outputs were up to twice as far from 64 bits, for 4% of
-// the time).  Tiles of 64 keys halve the barriers, and two keys of V make one 4-byte LDS store.
-// Measured against tiles of 32 with a rescale and a mask for every score, 4 prompts of 1500, 48 heads of 128 on 8 keys' heads:
-//   plain 815 -> 415 us     cap 890 -> 446     cap and distance penalty 890 -> 461     sigmoid weights 825 -> 375
-// and 6 of 1500, 16 heads of 64 on 4:   300 -> 135, 355 -> 172, 356 -> 195, 319 -> 141 us
+// 128), with two waves a SIMD to overlap them.  So scores are in units of log 2: exp and log are one instruction each and the penalty
+// needs no factor.  The cap and the sigmoid weights come from exp(-|x|) and a reciprocal of [1, 2] that one Newton step makes as exact
+// as a division.  bf16 terms come from the conversion instruction, and a half tile that every row of the wave sees has no mask.  The
+// accumulators are rescaled when a maximum grows, and only then: a query's largest weight is exactly 1, which two bf16 terms hold without
+// error (left up to 2^8 behind the maximum, outputs were up to twice as far from 64 bits, for 4% of the time).  A half tile has 63
+// different distances: a lane works out the penalty of one and reads its 16 from LDS.  The pool row of every key is found once, a tile
+// ahead, by one thread (every 16-byte piece used to look its page up, 12 a thread and tile).  Weights pass to the value product in
+// registers (through LDS before), maxima cross lanes without LDS, sums meet at the end, and a kernel for each kind of weight
+// leaves no branch in a score's way.  All heads of a group run on one XCD, whose L2 then holds the group's keys once (fetched from
+// memory, 8 prompts of 2048 with 32 heads on 8: 250 MB -> 105).  Before and after these:
+//   8 of 2048, 32 heads of 128 on 8, cap and penalty   988 -> 663 us      4 of 1500, 48 on 8, plain             379 -> 230 us
+//   9 of 510 .. 1501, 16 on 16, plain, fp32 queries    250 -> 140         the same with a window of 1024        221 -> 129
+//   6 of 610 .. 1800, 16 on 4, sigmoid, window 512     137 -> 92          2 x 512 rows at 512, 16 on 4, penalty 88 -> 60
+//   6 of 1500, 16 heads of 64 on 4, cap and penalty    195 -> 135         3 of 37 .. 120                        17.3 -> 14.0
+// (both halves of a tile at once spill: 718 us in the first, 136 in the windowed one.)
 #include "seq_common.h"
 #include "fls_seq.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 #define KT 32             // keys per tile
 #define PLD (KT + 8)      // row stride (elements) of the transposed V tile and of the weight tiles
@@ -53,8 +61,19 @@ __device__ __forceinline__ float rcp_near(float x) {
   return __builtin_fmaf(__builtin_fmaf(-x, r, 1.f), r, r);
 }
 
+// maximum / sum over lanes l and l ^ 32, in both
+__device__ __forceinline__ float halves_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // (two waves per SIMD: a few registers over 256 would halve that)
-template <int D, int DV, typename TQ, typename TO, bool POOL>
+// KIND: 0 softmax of the scaled scores, 1 with a cap and / or a distance penalty, 2 sigmoid weights
+template <int D, int DV, typename TQ, typename TO, bool POOL, int KIND>
 __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restrict__ q, int ldq, const bf16_t* __restrict__ kc, int ldk,
                                                            const bf16_t* __restrict__ vc, int ldv, TO* __restrict__ out, int ldo,
                                                            const int* __restrict__ tiles, const int* __restrict__ tok_seq,
@@ -69,8 +88,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
   constexpr int KLD = D + 8;
   __shared__ __attribute__((aligned(16))) bf16_t Ks[PT * KLD];
   __shared__ __attribute__((aligned(16))) bf16_t Vt[DV * VLD];
-  __shared__ __attribute__((aligned(16))) bf16_t Ps[4][2][32 * PLD];
-  const int h = blockIdx.x, g = h / (H / G);
+  __shared__ __attribute__((aligned(8))) int rows[PT];               // pool rows of the tile that is fetched next
+  __shared__ float pen[4][64];                                       // a wave's distance penalties of a half tile
+  // (blocks go to the XCDs in turn: a group's heads onto one of them)
+  const int h = H % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (H / 8) + (int)blockIdx.x / 8, g = h / (H / G);
   const int tile = gridDim.y - 1 - blockIdx.y;                       // (the last tiles of a long prompt have the most keys: they go first)
   const int row0 = tiles[2 * tile], nrows = tiles[2 * tile + 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -116,9 +137,10 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
 #pragma unroll
     for (int r = 0; r < 16; ++r) O[c][r] = 0.f;
   // (the softmax's silent entry of score `sink` / sink_h[h], if any, is where every query's running maximum and sum start)
-  float m = has_sink ? (sink_h != nullptr ? sink_h[h] : sink) * LOG2E : -1e30f, l = has_sink ? 1.f : 0.f;
+  // (a lane sums its own keys: the two sums of a query meet at the end)
+  float m = has_sink ? (sink_h != nullptr ? sink_h[h] : sink) * LOG2E : -1e30f, l = has_sink && h2 == 0 ? 1.f : 0.f;
   const float a1 = r1 != nullptr ? r1[h] : 0.f, a2 = r2 != nullptr ? r2[h] : 0.f;
-  const bool gated = gate_bias != nullptr;
+  constexpr bool gated = KIND == 2;
   const float gb = gated ? gate_bias[h] * LOG2E : 0.f;
   // scores in units of log 2; with a cap: cap (1 - 2 / (exp(2 s / cap) + 1)), the exponential's argument straight from the product
   const float sc_mul = softcap > 0.f ? 2.f * LOG2E * scale / softcap : scale * LOG2E;
@@ -137,55 +159,69 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
   // tile's matrix work and land in LDS after it, so the page gather's latency hides under the MFMAs
   constexpr int PK = PT * (D / 8), PV = PT / 2 * (DV / 8);           // 16-byte pieces of K; pieces of two neighbouring keys of V
   constexpr int NK = (PK + 255) / 256, NV = (PV + 255) / 256;        // per thread (the last one of some threads may be none)
-  uint4 kreg[NK], vreg[NV][2];
-  auto pool_row = [&](const int* tab, int j) {
-    const int pg = page_shift >= 0 ? j >> page_shift : j / page_size;
-    return (size_t)tab[pg] * page_size + (j - pg * page_size);
-  };
-  auto fetch = [&](int ti) {
+  u32x4 kreg[NK], vreg[NV][2];
+  // rows of the pools that hold a tile's keys: one thread a key, kept in LDS a tile ahead of the loads that use them (keys behind
+  // the tile's last are that one again: every row masks them)
+  auto find_row = [&](int ti) {
     const bool pre = ti < nt_keep;
     const int j0 = pre ? ti * PT : lo_blk + (ti - nt_keep) * PT;
-    const int jend = pre ? nkeep : i_last + 1;
+    const int j = min(j0 + (int)threadIdx.x, (pre ? nkeep : i_last + 1) - 1);
     const int* tab = POOL && pre ? btable : table;
-    const bf16_t* kb = POOL && pre ? reinterpret_cast<const bf16_t*>(ab.kp) : kc;
-    const bf16_t* vb = POOL && pre ? reinterpret_cast<const bf16_t*>(ab.vp) : vc;
-    const int lk = POOL && pre ? ab.ldk : ldk, lv = POOL && pre ? ab.ldv : ldv;
+    const int pg = page_shift >= 0 ? j >> page_shift : j / page_size;
+    return int2{tab[pg], j - pg * page_size};
+  };
+  const int vpair = threadIdx.x % (PT / 2);
+  auto fetch = [&](int ti) {
+    const bool pre = POOL && ti < nt_keep;
+    const bf16_t* kb = pre ? reinterpret_cast<const bf16_t*>(ab.kp) : kc;
+    const bf16_t* vb = pre ? reinterpret_cast<const bf16_t*>(ab.vp) : vc;
+    const int lk = pre ? ab.ldk : ldk, lv = pre ? ab.ldv : ldv;
+    kb += (size_t)g * D;
+    vb += (size_t)(g % Gv) * DV;
 #pragma unroll
     for (int x = 0; x < NK; ++x) {
       const int e = threadIdx.x + 256 * x;
-      const int j = j0 + e / (D / 8), seg = e % (D / 8);
-      kreg[x] = make_uint4(0, 0, 0, 0);
-      if (j < jend && (PK % 256 == 0 || e < PK)) kreg[x] = *reinterpret_cast<const uint4*>(kb + pool_row(tab, j) * lk + (size_t)g * D + seg * 8);
+      if (PK % 256 == 0 || e < PK) kreg[x] = *reinterpret_cast<const u32x4*>(kb + (size_t)rows[e / (D / 8)] * lk + e % (D / 8) * 8);
     }
+    const int2 vr = *reinterpret_cast<const int2*>(rows + 2 * vpair);
+    const bf16_t* v0 = vb + (size_t)vr.x * lv;
+    const bf16_t* v1 = vb + (size_t)vr.y * lv;
 #pragma unroll
     for (int x = 0; x < NV; ++x) {
       const int e = threadIdx.x + 256 * x;
-      const int seg = e / (PT / 2);
-#pragma unroll
-      for (int y = 0; y < 2; ++y) {
-        const int j = j0 + 2 * (e % (PT / 2)) + y;
-        vreg[x][y] = make_uint4(0, 0, 0, 0);
-        if (j < jend && (PV % 256 == 0 || e < PV))
-          vreg[x][y] = *reinterpret_cast<const uint4*>(vb + pool_row(tab, j) * lv + (size_t)(g % Gv) * DV + seg * 8);
+      if (PV % 256 == 0 || e < PV) {
+        vreg[x][0] = *reinterpret_cast<const u32x4*>(v0 + e / (PT / 2) * 8);
+        vreg[x][1] = *reinterpret_cast<const u32x4*>(v1 + e / (PT / 2) * 8);
       }
     }
   };
+  // (a key's place in a row of the transposed V: keys 4 .. 7 and 8 .. 11 of every 16 change places, so that the weights a lane
+  // holds are the values' operand as they stand)
+  const int vplace = (vpair & ~6) | (vpair & 2) << 1 | (vpair & 4) >> 1;
+  int2 next_row = {0, 0};
+  if (threadIdx.x < PT) {
+    const int2 r = find_row(0);
+    rows[threadIdx.x] = r.x * page_size + r.y;
+    if (nt > 1) next_row = find_row(1);
+  }
+  __syncthreads();
   fetch(0);
   for (int ti = 0; ti < nt; ++ti) {
     const bool kept = ti < nt_keep;
     const int jt = kept ? ti * PT : lo_blk + (ti - nt_keep) * PT;
     const int jend = kept ? nkeep : i_last + 1;      // keys from jend on are padding of this tile
     __syncthreads();                          // the previous tile's readers are done
+    if (threadIdx.x < PT) rows[threadIdx.x] = next_row.x * page_size + next_row.y;
 #pragma unroll
     for (int x = 0; x < NK; ++x) {
       const int e = threadIdx.x + 256 * x;
-      if (PK % 256 == 0 || e < PK) *reinterpret_cast<uint4*>(Ks + (e / (D / 8)) * KLD + (e % (D / 8)) * 8) = kreg[x];
+      if (PK % 256 == 0 || e < PK) *reinterpret_cast<u32x4*>(Ks + (e / (D / 8)) * KLD + (e % (D / 8)) * 8) = kreg[x];
     }
 #pragma unroll
     for (int x = 0; x < NV; ++x) {            // (two keys of a column make one 4-byte store)
       const int e = threadIdx.x + 256 * x;
       if (PV % 256 != 0 && e >= PV) continue;
-      uint32_t* dst = reinterpret_cast<uint32_t*>(Vt + (e / (PT / 2)) * 8 * VLD) + e % (PT / 2);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(Vt + (e / (PT / 2)) * 8 * VLD) + vplace;
       const uint32_t a[4] = {vreg[x][0].x, vreg[x][0].y, vreg[x][0].z, vreg[x][0].w}, b[4] = {vreg[x][1].x, vreg[x][1].y, vreg[x][1].z, vreg[x][1].w};
 #pragma unroll
       for (int y = 0; y < 4; ++y) {
@@ -195,13 +231,16 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     }
     __syncthreads();
     if (ti + 1 < nt) fetch(ti + 1);
-#pragma unroll 1
+    if (ti + 2 < nt && threadIdx.x < PT) next_row = find_row(ti + 2);
+#pragma unroll
     for (int half = 0; half < 2; ++half) {
     const int j0 = jt + half * KT;
     if (j0 >= jend || wave * 32 >= nrows || (POOL && kept && j0 >= keep_w) ||
         (!kept && (j0 > w_last || (j0 + KT - 1 < lo_w && (POOL || j0 >= keep_first))))) continue;   // (wave-uniform)
     // every row of the wave sees every key of this half (rows past the tile's end compute what nobody stores)
     const bool full = !kept && j0 + KT - 1 <= w_first && j0 >= lo_wl;
+    // a distance penalty depends on query - key alone, 63 of them a half tile: a lane works out one
+    if (KIND != 0 && a1 != 0.f) pen[wave][lane] = log2_hw(1.f + a2 * fmaxf((float)(w_first - j0 + 31 - lane), 0.f));
     floatx16 S;
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[r] = 0.f;
@@ -215,17 +254,17 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     // (this kernel serves bf16 models only: the hardware exp / log are far inside their rounding)
 #pragma unroll
     for (int r = 0; r < 16; ++r) p[r] = S[r] * sc_mul;
-    if (softcap > 0.f) {                       // cap tanh: (1 - e) / (1 + e), e = exp(-2 |s| / cap), never overflows or cancels
+    if (KIND != 0 && softcap > 0.f) {          // cap tanh: (1 - e) / (1 + e), e = exp(-2 |s| / cap), never overflows or cancels
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float e = exp2_hw(-fabsf(p[r]));
-        p[r] = copysignf(cap2 * (1.f - e) * rcp_near(1.f + e), p[r]);
+        p[r] = copysignf(__builtin_fmaf(-cap2, e, cap2) * rcp_near(1.f + e), p[r]);
       }
     }
-    if (a1 != 0.f) {
-      const float dist0 = (float)(iq - j0 - 4 * h2);
+    if (KIND != 0 && a1 != 0.f) {
+      const float* pq = pen[wave] + 31 - ql + 4 * h2;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) p[r] -= a1 * log2_hw(1.f + a2 * fmaxf(dist0 - (float)(8 * (r >> 2) + (r & 3)), 0.f));
+      for (int r = 0; r < 16; ++r) p[r] -= a1 * pq[8 * (r >> 2) + (r & 3)];
     }
     if (gated) {
 #pragma unroll
@@ -250,7 +289,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     if (!gated) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, p[r]);
-      mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+      mt = halves_max(mt);
       if (__any(mt > m)) {               // (wave-uniform)
         mt = fmaxf(mt, m);
         const float corr = exp2_hw(m - mt);
@@ -269,35 +308,31 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
 #pragma unroll
         for (int r = 0; r < 16; ++r) { p[r] = p[r] > -1e29f ? exp2_hw(p[r] - m) : 0.f; ps += p[r]; }
       }
-      l += ps + __shfl_xor(ps, 32, 64);
+      l += ps;
     }
-    bf16_t* ph = Ps[wave][0] + ql * PLD;
-    bf16_t* pl = Ps[wave][1] + ql * PLD;
-#pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-      typedef float floatx4 __attribute__((ext_vector_type(4)));
-      const floatx4 v = {p[4 * rg], p[4 * rg + 1], p[4 * rg + 2], p[4 * rg + 3]};
-      const bf16x4 hi = __builtin_convertvector(v, bf16x4);
-      const bf16x4 lo = __builtin_convertvector(v - __builtin_convertvector(hi, floatx4), bf16x4);
-      *reinterpret_cast<bf16x4*>(ph + 8 * rg + 4 * h2) = hi;
-      *reinterpret_cast<bf16x4*>(pl + 8 * rg + 4 * h2) = lo;
-    }
-    __builtin_amdgcn_wave_barrier();          // (a wave reads back its own lanes' writes: LDS is in order per wave)
+    // two bf16 terms of each weight, in the order of the keys of a row of V
+    bf16x8 ph[KT / 16], pl[KT / 16];
 #pragma unroll
     for (int ks = 0; ks < KT / 16; ++ks) {
-      const bf16x8 bh = *reinterpret_cast<const bf16x8*>(ph + 16 * ks + 8 * h2);
-      const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pl + 16 * ks + 8 * h2);
+      typedef float floatx8 __attribute__((ext_vector_type(8)));
+      floatx8 v;
+#pragma unroll
+      for (int x = 0; x < 8; ++x) v[x] = p[8 * ks + x];
+      ph[ks] = __builtin_convertvector(v, bf16x8);
+      pl[ks] = __builtin_convertvector(v - __builtin_convertvector(ph[ks], floatx8), bf16x8);
+    }
+#pragma unroll
+    for (int ks = 0; ks < KT / 16; ++ks) {
 #pragma unroll
       for (int c = 0; c < DV / 32; ++c) {
         const bf16x8 vf = *reinterpret_cast<const bf16x8*>(Vt + (32 * c + ql) * VLD + half * KT + 16 * ks + 8 * h2);
-        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bh, O[c], 0, 0, 0);
-        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bl, O[c], 0, 0, 0);
+        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph[ks], O[c], 0, 0, 0);
+        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl[ks], O[c], 0, 0, 0);
       }
     }
-    __builtin_amdgcn_wave_barrier();
     }
   }
+  l = halves_sum(l);
   if (qok && (gated || l > 0.f)) {
     float inv = gated ? out_scale : out_scale / l;
     if (head_gate != nullptr) inv *= sigmoid_f(head_gate[(size_t)(row0 + qrow) * ldhg + h]);
@@ -343,22 +378,31 @@ extern "C" int fls_seq_attn_prefill(const void* q, int ldq, int tq, const void* 
   const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   dim3 grid(H, n_tiles);
   hipStream_t st = (hipStream_t)s;
-#define ATTN_PF_(DD, DDV, TQ_, TO_, PP)                                                                                   \
-  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, TQ_, TO_, PP>), grid, dim3(256), 0, st, (const TQ_*)q, ldq,            \
+#define ATTN_PF_(DD, DDV, TQ_, TO_, PP, KK)                                                                                   \
+  hipLaunchKernelGGL((attn_prefill_kernel<DD, DDV, TQ_, TO_, PP, KK>), grid, dim3(256), 0, st, (const TQ_*)q, ldq,            \
                      (const bf16_t*)kc, ldk, (const bf16_t*)vc, ldv, (TO_*)out, ldo, tiles, tok_seq, tok_pos,             \
                      page_table, pt_stride, H, G, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias,           \
                      out_scale, page_size, has_sink, sink, sink_h, head_gate, ldhg, Gv, ab, page_shift)
+#define ATTN_PF_KIND(DD, DDV, TQ_, TO_)                                                                                   \
+  do {                                                                                                                    \
+    if (gate_bias != nullptr) ATTN_PF_(DD, DDV, TQ_, TO_, false, 2);                                                      \
+    else if (softcap > 0.f || r1 != nullptr) ATTN_PF_(DD, DDV, TQ_, TO_, false, 1);                                       \
+    else ATTN_PF_(DD, DDV, TQ_, TO_, false, 0);                                                                           \
+  } while (0)
 #define ATTN_PF(DD, DDV)                                                                                                  \
   do {                                                                                                                    \
-    if (tq == 1 && to == 1) ATTN_PF_(DD, DDV, bf16_t, bf16_t, false);                                                     \
-    else if (tq == 1) ATTN_PF_(DD, DDV, bf16_t, float, false);                                                            \
-    else if (to == 1) ATTN_PF_(DD, DDV, float, bf16_t, false);                                                            \
-    else ATTN_PF_(DD, DDV, float, float, false);                                                                          \
+    if (tq == 1 && to == 1) ATTN_PF_KIND(DD, DDV, bf16_t, bf16_t);                                                        \
+    else if (tq == 1) ATTN_PF_KIND(DD, DDV, bf16_t, float);                                                               \
+    else if (to == 1) ATTN_PF_KIND(DD, DDV, float, bf16_t);                                                               \
+    else ATTN_PF_KIND(DD, DDV, float, float);                                                                             \
   } while (0)
 #define ATTN_PF_POOL(DD, DDV)                                                                                             \
   do {                                                                                                                    \
-    if (to == 1) ATTN_PF_(DD, DDV, float, bf16_t, true);                                                                  \
-    else ATTN_PF_(DD, DDV, float, float, true);                                                                           \
+    if (softcap > 0.f) {                                                                                                  \
+      if (to == 1) ATTN_PF_(DD, DDV, float, bf16_t, true, 1);                                                             \
+      else ATTN_PF_(DD, DDV, float, float, true, 1);                                                                      \
+    } else if (to == 1) ATTN_PF_(DD, DDV, float, bf16_t, true, 0);                                                        \
+    else ATTN_PF_(DD, DDV, float, float, true, 0);                                                                        \
   } while (0)
   if (pool_P > 0) {
     if (d == 128 && dv == 128) ATTN_PF_POOL(128, 128);
@@ -375,6 +419,7 @@ extern "C" int fls_seq_attn_prefill(const void* q, int ldq, int tq, const void* 
   else return -2;
 #undef ATTN_PF_POOL
 #undef ATTN_PF
+#undef ATTN_PF_KIND
 #undef ATTN_PF_
   SEQ_LAUNCH_CHECK();
   return 0;

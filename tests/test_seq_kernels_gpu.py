@@ -323,6 +323,29 @@ def test_prompt_attention_largest_weight(ops, d, dv, cap, sink):
     assert not bool(out[:at].any())
 
 
+# every kind of weight (softmax, cap, penalty, both, sigmoid) with heads that go to the XCDs by groups (8, 16) and as they come (6), lengths
+# about a half, a tile and a block, pages no tile fits, carried positions.  fp32 results: weights of two bf16 terms (2^-17), scores of up to
+# 30 in units of log 2 to fp32 (2e-6 each side, and 2e-6 for exp's own): 3e-5
+@pytest.mark.parametrize("Hh,G", [(8, 2), (16, 16), (6, 3)])
+@pytest.mark.parametrize("lens,pos0", [([32, 1, 63], [0, 300, 1]), ([128, 33], [0, 95]), ([257], [64])])
+@pytest.mark.parametrize("kind", ["plain", "cap", "penalty", "both", "sigmoid"])
+def test_prompt_attention_kinds(ops, Hh, G, lens, pos0, kind):
+    H, R = ops
+    T, d, ps = sum(lens), 128, 24
+    torch.manual_seed(T + Hh)
+    md, npages, _ = meta_of(lens, pos0, DEV, ps)
+    kc, vc = torch.randn(npages, ps, G * d, device=DEV).bfloat16(), torch.randn(npages, ps, G * d, device=DEV).bfloat16()
+    q = torch.randn(T, Hh * d, device=DEV).bfloat16()
+    r1, r2 = (torch.rand(Hh, device=DEV), torch.rand(Hh, device=DEV)) if kind in ("penalty", "both") else (None, None)
+    cap = 8.0 if kind in ("cap", "both") else 0.0
+    kw = dict(gate_bias=torch.randn(Hh, device=DEV) - 2) if kind == "sigmoid" else {}
+    for chunk, window, keep in ((0, 0, 0), (100, 0, 0), (0, 70, 0), (0, 70, 40)):
+        o1, o2 = torch.empty(T, Hh * d, device=DEV), torch.empty(T, Hh * d, device=DEV)
+        for o, out in ((H, o1), (R, o2)):
+            o.attn_paged(q, kc, vc, md, Hh, G, d, d, d ** -0.5, cap, r1, r2, chunk, ps, torch.bfloat16, window=window, keep_first=keep, out=out, **kw)
+        close(o1, o2, 3e-5)
+
+
 # norms with rows in registers: one to eight steps of 1024 columns a group, the last one partly filled, the widest and the first beyond it
 # (8192, 8196), odd widths and strides that go to the general kernel, one weight for all columns; the residual update with the
 # next norm against the two in turn.  fp32 outputs against fp64: sums of up to 8196 squares in a tree, 1e-6; bf16 rounding 2^-8
