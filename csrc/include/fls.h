@@ -113,8 +113,8 @@ int fls_moe_router_route(const void* h, int ldh, const void* wr, int ldw, int T,
 int fls_moe_plan_scratch(int n, int E);   // ints of the bhist scratch fls_moe_plan needs
 int fls_moe_plan(const int* ids, int n, int k, int E, int* offs, int* tiles, int* rows, int* dest, int* bhist,
                  fls_stream_t s);
-int fls_moe_gemm(const void* A, const void* W, void* C, int M_bound, int N, int K, int lda, int ldw, int ldc, int epi,
-                 const int* tiles, const int* offs, const int* rows, int n_groups, long long wstride, int a_rows,
+int fls_moe_gemm(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int epi,
+                 const int* offs, const int* rows, int n_groups, long long wstride, int a_rows,
                  fls_stream_t s);
 int fls_moe_combine(const void* y, int ldy, const int* ids, const int* dest, const float* w, void* x, int ldx, int T,
                     int k, int H, const void* sh, int ldsh, fls_stream_t s);   // sh: optional shared-expert term

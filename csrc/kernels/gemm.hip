@@ -972,7 +972,7 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
     if (route == ROUTE_V11) route = ROUTE_NONE;
   }
   Epi ep{(const half_t*)R, ldr, pos, cos_t, sin_t, rope_cols, head_dim, (const half_t*)bias, N / 2, 0,
-         nullptr, nullptr, nullptr, 0, 0};
+         nullptr, nullptr, 0, 0};
   ep.rs = rscale;
   ep.alpha = alpha;
   ep.ss = ss;

@@ -36,7 +36,6 @@ struct Epi {
   int gu_rows;          // SWIGLU: I (rows of gate = rows of up)
   int order;            // v10 tile order (tile_of), set by the launcher
   // grouped v10 (mixture-of-experts; moe.hip): see gemm_nt_v10<EPI, true>
-  const int* g_tiles;
   const int* g_offs;
   const int* g_rows;
   long long g_wstride;
@@ -453,12 +452,51 @@ __device__ __forceinline__ void fence_acc(floatx4 (&acc)[U][8]) {
     for (int t = 0; t < 8; ++t) asm volatile("" : "+a"(acc[u][t]));
 }
 
+// The M tiles of up to 256 row groups, one group's after the other's (TM rows each, the last of a group partly filled; empty groups
+// own none): lane l holds groups 4 l .. 4 l + 3.  A wave counts and finds them with two loads and a scan over its lanes; walked group by
+// group, a block of the 128th paid 128 dependent scalar loads before its first DMA.
+template <int TM>
+struct Groups {
+  int row[5], tiles[4], upto;                 // first rows, M tiles; tiles of the groups up to and with this lane's
+  __device__ __forceinline__ int count(const int* __restrict__ offs, int n, int lane) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) row[q] = offs[min(4 * lane + q, n)];
+    upto = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) upto += tiles[q] = (row[q + 1] - row[q] + TM - 1) / TM;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, 64);
+      upto += lane >= o ? v : 0;
+    }
+    return __builtin_amdgcn_readlane(upto, 63);
+  }
+  // the group of tile tm, which becomes the tile's number in it; its first row and how many it has
+  __device__ __forceinline__ int find(int& tm, int& first, int& rows) const {
+    const int l = __builtin_ctzll(__ballot(upto > tm));
+    int e = 4 * l, at = __builtin_amdgcn_readlane(row[0], l), end = __builtin_amdgcn_readlane(row[1], l);
+    tm -= __builtin_amdgcn_readlane(upto - tiles[0] - tiles[1] - tiles[2] - tiles[3], l);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int t = __builtin_amdgcn_readlane(tiles[q], l);
+      if (e == 4 * l + q && tm >= t) {
+        tm -= t;
+        ++e;
+        at = end;
+        end = __builtin_amdgcn_readlane(row[q + 2], l);
+      }
+    }
+    first = at;
+    rows = end - at;
+    return e;
+  }
+};
+
 // Grouped (mixture-of-experts) form of v10 (GRP): G row groups (experts) share one launch.  Group e
-// owns rows [g_offs[e], g_offs[e+1]) of C, its M tiles are virtual tiles [g_tiles[e], g_tiles[e+1])
-// (ceil of its rows / BM), its weight is W + e * g_wstride, and its A rows are either contiguous from
-// row g_offs[e] of A or gathered: A row g_rows[g_offs[e] + i] (the token a routed entry came from, so
+// owns rows [g_offs[e], g_offs[e+1]) of C and the M tiles these make, its weight is W + e * g_wstride, and its A rows are either
+// contiguous from row g_offs[e] of A or gathered: A row g_rows[g_offs[e] + i] (the token a routed entry came from, so
 // the activations are never permuted in memory; one index load per staged row, at block start).  M is
-// a bound on the rows (the launch covers ceil(M / BM) M tiles).  Only the g_tiles[G] M tiles there are take part in the
+// all groups' rows (the launch covers the most M tiles they can make).  Only the M tiles there are take part in the
 // block -> tile mapping and the others exit before touching LDS: mapped over the bound, whole XCDs got few or no
 // tiles (128 experts, 48,608 rows, 2048 -> 2 x 768: 452 -> 345 us; 768 -> 2048: 335 -> 283).  The N tiles of an M tile go one
 // after the other where there are at most eight: an expert's A rows are read once (342 and 261; 384 rows: 226 -> 197).
@@ -476,8 +514,9 @@ __device__ __forceinline__ void tile_v10(const half_t* __restrict__ A, const hal
   const int tiles_n = N / BN;
   int nwg = gridDim.x;
   int bid = blockIdx.x;
+  [[maybe_unused]] Groups<TM> gr;
   if constexpr (GRP) {
-    tiles_m = ep.g_tiles[ep.g_n];
+    tiles_m = gr.count(ep.g_offs, ep.g_n, lane);
     nwg = tiles_m * tiles_n;
     if (bid >= nwg) return;                          // past the last group's tiles: whole block exits
   }
@@ -498,11 +537,8 @@ __device__ __forceinline__ void tile_v10(const half_t* __restrict__ A, const hal
   half_t* Cg = C;
   const int* rows = nullptr;
   if constexpr (GRP) {
-    int e = 0;
-    while (ep.g_tiles[e + 1] <= tm) ++e;             // wave-uniform scan (empty groups own no tiles)
-    const int r0 = ep.g_offs[e];
-    M = ep.g_offs[e + 1] - r0;
-    tm -= ep.g_tiles[e];
+    int r0;
+    const int e = gr.find(tm, r0, M);                // (tm: from here the tile within its group)
     Wg = W + (size_t)e * ep.g_wstride;
     Cg = C + (size_t)r0 * ldc;
     if (ep.g_rows) rows = ep.g_rows + r0;

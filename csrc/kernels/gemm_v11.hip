@@ -387,7 +387,7 @@ extern "C" int fls_gemm_v11_try(const void* A, const void* W, void* C, const voi
   if (ldc % 8 || ((uintptr_t)C & 15)) return 0;
   if (epi == FLS_EPI_RESID && (ldr % 8 || ((uintptr_t)R & 15))) return 0;
   Epi ep{(const half_t*)R, ldr, pos, cos_t, sin_t, rope_cols, head_dim, (const half_t*)bias, N / 2, 0,
-         nullptr, nullptr, nullptr, 0, 0};
+         nullptr, nullptr, 0, 0};
   ep.rs = rscale;
   ep.alpha = alpha;
   ep.ss = ss;

@@ -10,8 +10,8 @@
 //                      256-row GEMM tiles, prefix), rows [T*k] (permuted row -> token), dest [T*k]
 //                      (entry -> permuted row).  Deterministic: entries keep token order inside an
 //                      expert, so a run is bitwise reproducible.
-//   4. fls_moe_gemm    the v10 MFMA GEMM in grouped form (gemm_v10.h): every expert's rows in ONE
-//                      launch, no host round trip for the counts.  gate/up + SwiGLU gathers its A rows
+//   4. fls_moe_gemm    the v10 MFMA GEMM in grouped form (gemm_v10.h) on M tiles of 128, 192 or 256 rows: every expert's rows
+//                      in ONE launch, no host round trip for the counts.  gate/up + SwiGLU gathers its A rows
 //                      straight from h through `rows` (the LDS-DMA source offsets are per row, fixed
 //                      for the whole K loop, so the gather costs one index load per staged row); down
 //                      reads the permuted SwiGLU output contiguously.
@@ -161,8 +161,8 @@ __global__ __launch_bounds__(ROUTE_WAVES * 64) void moe_router_route_kernel(
 // Stable counting sort of the n routed entries by expert, in three launches over blocks of
 // PB_ENTRIES consecutive entries (entry i = token i / k, slot i % k): per-block histograms, one scan
 // block (per-expert offsets, tile prefix, each block's base per expert), then placement: every wave
-// keeps its 16 x 64 entries in registers, ranks each 64-entry group by shuffles (rank = earlier
-// lanes with the same expert) and advances its per-expert base in LDS.  Entries of an expert keep
+// keeps its 16 x 64 entries in registers, ranks each 64-entry group by ballots (rank = earlier
+// lanes with the same expert; the plan of 45,900 entries 53 -> 20 us against a shuffle for every pair) and advances its per-expert base in LDS.  Entries of an expert keep
 // token order, so the plan — and every result computed from it — is deterministic.
 constexpr int PB_THREADS = 256;
 constexpr int PB_GROUPS = 16;                                  // 64-entry groups per wave
@@ -251,12 +251,14 @@ __global__ __launch_bounds__(PB_THREADS) void moe_place_kernel(const int* __rest
 #pragma unroll
   for (int g = 0; g < PB_GROUPS; ++g) {
     const int id = v[g];
-    int before = 0, after = 0;
-    for (int j = 0; j < 64; ++j) {
-      const int o = __shfl(id, j, 64);
-      before += (j < lane && o == id) ? 1 : 0;
-      after += (j > lane && o == id) ? 1 : 0;
+    unsigned long long same = __ballot(id >= 0);              // the lanes with this lane's expert, a bit of its number at a time
+#pragma unroll
+    for (int bit = 1; bit < MAX_E; bit <<= 1) {
+      const unsigned long long set = __ballot((id & bit) != 0);
+      same &= (id & bit) != 0 ? set : ~set;
     }
+    const int before = __builtin_popcountll(same & ((1ull << lane) - 1));
+    const bool last = (same >> lane) == 1;
     if (id >= 0) {
       const int i = wbeg + g * 64 + lane;
       const int pos = wbase[wave][id] + before;
@@ -264,7 +266,7 @@ __global__ __launch_bounds__(PB_THREADS) void moe_place_kernel(const int* __rest
       rows[pos] = i / k;
     }
     __builtin_amdgcn_wave_barrier();
-    if (id >= 0 && after == 0) wbase[wave][id] += before + 1;
+    if (id >= 0 && last) wbase[wave][id] += before + 1;
     __builtin_amdgcn_wave_barrier();
   }
 }
@@ -316,23 +318,56 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const half_t* __restri
   }
 }
 
-template <int EPI>
-int launch_grouped(const half_t* A, const half_t* W, half_t* C, int M_bound, int N, int K, int lda, int ldw,
-                   int ldc, const int* tiles, const int* offs, const int* rows, int n_groups, long long wstride,
-                   hipStream_t s) {
+template <int EPI, int HX>
+int launch_grouped(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw,
+                   int ldc, const int* offs, const int* rows, int n_groups, long long wstride, hipStream_t s) {
+  constexpr int TM = 64 * HX, LDS = 2 * v10_stage(HX);
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm_nt_v10<EPI, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              2 * BUF);
+    (void)hipFuncSetAttribute((const void*)gemm_nt_v10<EPI, true, HX>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS);
     attr = true;
   }
-  const int tiles_m = (M_bound + BM - 1) / BM, tiles_n = N / BN;
+  const long long tiles_m = ((long long)M + (long long)(TM - 1) * min(n_groups, M)) / TM;      // (each group with rows may end in a part of one)
+  const int tiles_n = N / BN;
   Epi ep{nullptr, 0, nullptr, nullptr, nullptr, 0, 0, nullptr, N / 2, tiles_n <= 8 ? -tiles_n : -4,
-         tiles, offs, rows, wstride, n_groups};
-  hipLaunchKernelGGL((gemm_nt_v10<EPI, true>), dim3(tiles_m * tiles_n), dim3(256), 2 * BUF, s, A, W, C, M_bound, N,
+         offs, rows, wstride, n_groups};
+  hipLaunchKernelGGL((gemm_nt_v10<EPI, true, HX>), dim3((unsigned)(tiles_m * tiles_n)), dim3(256), LDS, s, A, W, C, M, N,
                      K, lda, ldw, ldc, ep);
   FLS_CHECK_LAUNCH();
   return 0;
+}
+
+// Rows of the M tiles (64 HX; every form gives the same bits): the least estimated time.  The groups' sizes are on the device: each is
+// taken to have its share of the rows and half a tile of padding, one tile at least.  A launch is rounds of 256 blocks, each nk
+// K tiles and a start and a store (us, fitted to 8, 60 and 128 groups of 3 .. 1500 rows, K = 768 .. 14336), a last round of few blocks three
+// quarters of one.  Few rows a group want small tiles, as their padding costs matrix work that the stream of weights does not hide: gate / up of
+// 128 x (2 x 768 x 2048) with 3 rows each 175 us on 256-row tiles, 138 on 128; down 101 and 67; with 94 each 228 and 187, 134 and 114.
+// Many want large ones: 750 each 643 us (the group found by a walk), 609 on 256, 648 on 128.  8 x (4096 x 14336), 600 each: 582, 539 on 192.
+int grouped_hx(int M, int N, int K, int n_groups) {
+  static const struct { float k_us, us; } COST[3] = {{0.85f, 7.f}, {1.13f, 9.5f}, {1.42f, 11.f}};
+  const float share = (float)M / (float)min(M, n_groups);
+  int best = 2;
+  float least = 0.f;
+  for (int i = 0; i < 3; ++i) {
+    const float tiles = (float)min(M, n_groups) * fmaxf(1.f, share / (float)(128 + 64 * i) + 0.5f);
+    const float rounds = tiles * (float)(N / BN) / 256.f, whole = floorf(rounds), rest = rounds - whole;
+    const float t = (whole + (rest > 0.f ? 0.75f + 0.25f * rest * rest : 0.f)) * (COST[i].k_us * (float)(K / BK) + COST[i].us);
+    if (i == 0 || t < least) {
+      least = t;
+      best = i + 2;
+    }
+  }
+  return best;
+}
+
+template <int EPI>
+int launch_grouped(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw,
+                   int ldc, const int* offs, const int* rows, int n_groups, long long wstride, hipStream_t s) {
+  switch (grouped_hx(M, N, K, n_groups)) {
+    case 2: return launch_grouped<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, offs, rows, n_groups, wstride, s);
+    case 3: return launch_grouped<EPI, 3>(A, W, C, M, N, K, lda, ldw, ldc, offs, rows, n_groups, wstride, s);
+    default: return launch_grouped<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, offs, rows, n_groups, wstride, s);
+  }
 }
 
 }  // namespace
@@ -393,12 +428,12 @@ extern "C" int fls_moe_combine(const void* y, int ldy, const int* ids, const int
 
 // Grouped expert GEMM (v10 grouped form).  epi: FLS_EPI_SWIGLU (W per group = [gate; up], C has N/2
 // columns) or FLS_EPI_NONE.  rows: optional gather (A row of each permuted row), else A is permuted.
-// M_bound >= sum over groups of their rows rounded up to 256 (T*k + 255*G suffices).  Returns -5 when
+// M: the groups' rows, all together.  Returns -5 when
 // the shape is outside the kernel's contract (caller falls back to per-group fls_gemm).
-extern "C" int fls_moe_gemm(const void* A, const void* W, void* C, int M_bound, int N, int K, int lda, int ldw,
-                            int ldc, int epi, const int* tiles, const int* offs, const int* rows, int n_groups,
+extern "C" int fls_moe_gemm(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw,
+                            int ldc, int epi, const int* offs, const int* rows, int n_groups,
                             long long wstride, int a_rows, fls_stream_t s) {
-  if (M_bound <= 0) return 0;
+  if (M <= 0) return 0;
   const bool ok = N % BN == 0 && K % BK == 0 && (K / BK) % 2 == 0 && lda % 8 == 0 && ldw % 8 == 0 && ldc % 8 == 0 &&
                   ((uintptr_t)C & 15) == 0 && n_groups >= 1 && n_groups <= MAX_E &&
                   (size_t)a_rows * lda * 2 < (1ull << 32) &&
@@ -410,7 +445,6 @@ extern "C" int fls_moe_gemm(const void* A, const void* W, void* C, int M_bound, 
   auto c = (half_t*)C;
   auto st = (hipStream_t)s;
   if (epi == FLS_EPI_SWIGLU)
-    return launch_grouped<FLS_EPI_SWIGLU>(a, w, c, M_bound, N, K, lda, ldw, ldc, tiles, offs, rows, n_groups, wstride,
-                                          st);
-  return launch_grouped<FLS_EPI_NONE>(a, w, c, M_bound, N, K, lda, ldw, ldc, tiles, offs, rows, n_groups, wstride, st);
+    return launch_grouped<FLS_EPI_SWIGLU>(a, w, c, M, N, K, lda, ldw, ldc, offs, rows, n_groups, wstride, st);
+  return launch_grouped<FLS_EPI_NONE>(a, w, c, M, N, K, lda, ldw, ldc, offs, rows, n_groups, wstride, st);
 }

@@ -130,7 +130,7 @@ def _load_kernels(path: str = _KERNELS):
     _bind(lib, "fls_moe_plan", c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
           c_void_p)
     _bind(lib, "fls_moe_gemm", c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
-          c_void_p, c_void_p, c_void_p, c_int, ctypes.c_longlong, c_int, c_void_p)
+          c_void_p, c_void_p, c_int, ctypes.c_longlong, c_int, c_void_p)
     _bind(lib, "fls_moe_combine", c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int,
           c_int, c_int, c_void_p, c_int, c_void_p)
     _bind(lib, "fls_gemm_set_order", c_int, c_int)

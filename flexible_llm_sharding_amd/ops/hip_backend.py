@@ -380,17 +380,16 @@ class HipOps:
         dev, st = h.device, _stream()
         m = m_out if m_out is not None else torch.empty(n, I, dtype=torch.float16, device=dev)
         y = y_out if y_out is not None else torch.empty(n, H, dtype=torch.float16, device=dev)
-        bound = n + 255 * E                       # >= sum over experts of their rows rounded up to 256
-        rc = self.k.fls_moe_gemm(h.data_ptr(), wgu.data_ptr(), m.data_ptr(), bound, I2, H, h.stride(0),
-                                 wgu.stride(1), m.stride(0), EPI_SWIGLU, route.tiles.data_ptr(),
-                                 route.offs.data_ptr(), route.rows.data_ptr(), E, wgu.stride(0), T, st)
+        rc = self.k.fls_moe_gemm(h.data_ptr(), wgu.data_ptr(), m.data_ptr(), n, I2, H, h.stride(0),
+                                 wgu.stride(1), m.stride(0), EPI_SWIGLU, route.offs.data_ptr(), route.rows.data_ptr(),
+                                 E, wgu.stride(0), T, st)
         if rc == -5:                              # shape outside the grouped kernel: per-expert GEMMs
             self._moe_per_expert(h, wgu, wdown, route, m, y)
         else:
             _chk(rc, "fls_moe_gemm(gate/up)")
-            _chk(self.k.fls_moe_gemm(m.data_ptr(), wdown.data_ptr(), y.data_ptr(), bound, H, I, m.stride(0),
-                                     wdown.stride(1), y.stride(0), EPI_NONE, route.tiles.data_ptr(),
-                                     route.offs.data_ptr(), None, E, wdown.stride(0), n, st), "fls_moe_gemm(down)")
+            _chk(self.k.fls_moe_gemm(m.data_ptr(), wdown.data_ptr(), y.data_ptr(), n, H, I, m.stride(0),
+                                     wdown.stride(1), y.stride(0), EPI_NONE, route.offs.data_ptr(), None, E,
+                                     wdown.stride(0), n, st), "fls_moe_gemm(down)")
         if shared is not None:
             _f16(shared, "shared")
             if tuple(shared.shape) != (T, H) or shared.stride(1) != 1:

@@ -98,6 +98,33 @@ def _torch_experts(h, x, wgu, wdown, ids, w, k):
     return (x.float() + acc.float()).half()
 
 
+# row groups about the edges of 128-, 192- and 256-row tiles (the launcher takes them in this order), empty ones among them, first, last and
+# 256 of them, gathered and not.  fp16 results of fp32 sums: 2^-11 of the largest, and as much for torch's own order
+@pytest.mark.parametrize("sizes,N", [([0, 1, 127, 128, 129, 0, 300, 0], 256), ([3, 0, 1, 130] * 64, 256), ([0] * 255 + [5], 256),
+                                     ([0, 191, 192, 193, 1, 1600, 1536, 1700, 1900, 687], 4096),
+                                     ([255, 256, 257, 1, 3000, 0, 3072, 3100, 3300, 1759], 4096)])
+def test_grouped_tiles(ops, sizes, N):
+    G, K, M = len(sizes), 128, sum(sizes)
+    a, w = rnd(M, K, seed=M), rnd(G, N, K, scale=K ** -0.5, seed=G)
+    offs = torch.tensor([0] + sizes).cumsum(0).int().to(DEV)
+    src = torch.randperm(M, generator=torch.Generator().manual_seed(1)).int().to(DEV)
+    group = torch.repeat_interleave(torch.arange(G), torch.tensor(sizes)).tolist()
+    for rows in (None, src):
+        x = a if rows is None else a[rows.long()]
+        got, act = (torch.full((M + 1, n), 7.0, dtype=torch.float16, device=DEV) for n in (N, N // 2))
+        for c, epi in ((got, 0), (act, 2)):
+            rc = ops.k.fls_moe_gemm(a.data_ptr(), w.data_ptr(), c.data_ptr(), M, N, K, K, K, c.stride(0), epi, offs.data_ptr(),
+                                    None if rows is None else rows.data_ptr(), G, w.stride(0), M, torch.cuda.current_stream().cuda_stream)
+            assert rc == 0
+        for e in sorted(set(group)):
+            b0, b1 = int(offs[e]), int(offs[e + 1])
+            p = x[b0:b1].float() @ w[e].float().t()
+            assert float((got[b0:b1].float() - p).abs().max()) < 1e-3 * float(p.abs().max())
+            p = torch.nn.functional.silu(p[:, :N // 2]) * p[:, N // 2:]
+            assert float((act[b0:b1].float() - p).abs().max()) < 2e-3 * float(p.abs().max())
+        assert bool((got[M] == 7).all()) and bool((act[M] == 7).all())
+
+
 @pytest.mark.parametrize("T,H,I,E,k", [(200, 256, 256, 4, 2),          # tiny-Mixtral geometry
                                        (1500, 512, 512, 8, 2),         # several 256-row tiles per expert
                                        (300, 256, 128, 128, 8),        # Qwen3-MoE-like: many empty experts
