@@ -85,6 +85,7 @@ int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N,
 // rstd[r] = rsqrt(sum_j ss[r * ss_ld + j] / H + eps) for j < nparts, summed in a fixed order
 int fls_row_stat(const void* x, int ldx, int rows, int H, float eps, float* rstd, fls_stream_t s);  // row_ss + rstd_from_ss, fused
 int fls_row_ss(const void* x, int ldx, int rows, int H, float* ss, int ss_ld, fls_stream_t s);  // residual-epilogue partials of x
+int fls_gemm_leaves_ss(int M, int N, int K, uint64_t ws_bytes);   // the RESID product's own epilogue writes ss
 int fls_rstd_from_ss(const float* ss, int ss_ld, int nparts, int rows, int H, float eps, float* rstd,
                      fls_stream_t s);
 // out[r] = first index of the maximum of row r of non-negative fp16 values (greedy decoding)

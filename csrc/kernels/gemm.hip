@@ -950,6 +950,15 @@ extern "C" int fls_gemm_v11_try(const void* A, const void* W, void* C, const voi
                                 const float* sin_t, int rope_cols, int head_dim, const void* bias,
                                 const float* rscale, float alpha, float* ss, int ss_ld, int want, fls_stream_t s);
 
+// Does a residual product of M x N x K write its rows' partial sums of squares in its epilogue (v10 and v11 tiles)?  On the other paths
+// they are a launch of their own behind it and a second one sums them; fls_row_stat gives the same bits in one (79 rows x 4,096:
+// 3.5 + 2.7 us and a launch more, 4.6 here).
+extern "C" int fls_gemm_leaves_ss(int M, int N, int K, uint64_t ws_bytes) {
+  if (M <= 64 || N % BN || K % (2 * BK)) return 0;
+  const Route route = route_of(M, N, K, FLS_EPI_RESID, false, ws_bytes);
+  return route == ROUTE_NONE ? (long)((M + 255) / 256) * (N / BN) >= 128 : route >= ROUTE_128;
+}
+
 extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
                         int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
                         int rope_cols, int head_dim, const void* bias, const float* rscale, float alpha, float* ss,

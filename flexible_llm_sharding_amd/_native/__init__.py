@@ -107,6 +107,7 @@ def _load_kernels(path: str = _KERNELS):
     _bind(lib, "fls_gemm", c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
           c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p,
           c_float, c_void_p, c_int, c_void_p, c_uint64, c_void_p)
+    _bind(lib, "fls_gemm_leaves_ss", c_int, c_int, c_int, c_int, ctypes.c_uint64)
     _bind(lib, "fls_rstd_from_ss", c_int, c_void_p, c_int, c_int, c_int, c_int, c_float, c_void_p, c_void_p)
     _bind(lib, "fls_row_ss", c_int, c_void_p, c_int, c_int, c_int, c_void_p, c_int, c_void_p)
     _bind(lib, "fls_row_stat", c_int, c_void_p, c_int, c_int, c_int, c_float, c_void_p, c_void_p)

@@ -212,14 +212,18 @@ class ExecContext:
         t = self.scratch(1, 2 * n)
         return t.view(torch.float32).view(n) if t is not None else None
 
-    def ss_take(self, rows: int, key: Optional[tuple] = None) -> Optional[torch.Tensor]:
-        """The [rows, H/128] partial-sums buffer the next residual GEMM writes (None when the path
-        is off: unfused norm, MoE, or a hidden size the 128-column partials do not divide).  With
+    def ss_take(self, rows: int, K: int, key: Optional[tuple] = None, chunk: int = 0) -> Optional[torch.Tensor]:
+        """The [rows, H/128] partial-sums buffer the next residual GEMM (of ``K`` terms, ``chunk`` rows at a time if
+        given) writes (None when the path is off: unfused norm, MoE, a hidden size the 128-column partials do not divide,
+        or a GEMM that would need a pass over its rows for them: the next norm makes that pass itself).  With
         ``key`` holding (the partials about to be read), that same buffer.  Eagerly, one buffer
         grown to the largest micro-batch (like the workspace); without a workspace (graph capture)
         a fresh one per forward from the graph's own pool, never a buffer that eager code frees."""
         H = self.cfg.hidden_size
         if not self.fused_norm or self.cfg.is_moe or H % 128 or self.row_exact:
+            return None
+        leaves = getattr(self.ops, "leaves_ss", None)
+        if leaves is not None and H <= 16384 and not leaves(min(rows, chunk) if chunk else rows, H, K):
             return None
         if key is not None and self.ss_key == key and self.ss_cur is not None:
             return self.ss_cur[:rows]
@@ -444,7 +448,7 @@ def _attention_whole(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tens
         idx = meta["last_idx"]
         a = ops.gather_rows(a, idx)
         x = ops.gather_rows(x, idx)
-    ss = ctx.ss_take(x.shape[0])
+    ss = ctx.ss_take(x.shape[0], W["wo"].shape[1])
     y = _resid(ctx, a, W["wo"], x, bias=W.get("bo"), ss=ss)
     ctx.ss_key = (id(batch), li, "attn", x.shape[0]) if ss is not None else None
     return y
@@ -532,7 +536,7 @@ def run_decoder(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, b
         # partials, which its gate/up has already read.
         li = _decoder_index(layer_name)
         key = (id(batch), li, "attn", T)
-        ss_all = ctx.ss_take(T, key)          # (the O projection's buffer when the key matches)
+        ss_all = ctx.ss_take(T, I, key, step)  # (the O projection's buffer when the key matches)
         for s in range(0, T, step):
             xs = x[s:s + step]
             n = xs.shape[0]

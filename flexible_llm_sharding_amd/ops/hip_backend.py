@@ -194,6 +194,10 @@ class HipOps:
         _f16(resid, "resid")
         return self.gemm(x, w, EPI_RESID, out=resid, resid=resid, bias=bias, alpha=alpha, ss=ss)
 
+    def leaves_ss(self, M: int, N: int, K: int) -> bool:
+        """Does :meth:`linear_residual` of [M, K] rows into N columns write ``ss`` without a pass of its own?"""
+        return bool(self.k.fls_gemm_leaves_ss(M, N, K, SPLITK_WS_BYTES if M <= SPLITK_MAX_M else 0))
+
     def rstd_from_ss(self, ss, H: int, eps, out=None):
         """[rows] fp32 rsqrt(sum of the row's ss partials / H + eps): the RMSNorm statistic of the rows
         a residual GEMM just wrote (:meth:`linear_residual` ``ss``), without reading them again."""

@@ -1232,3 +1232,17 @@ def test_argmax_rows_widths(ops, V):
         x[1] = 0
         x[2, V - 1] = 2.0
         assert np.array_equal(ops.argmax_rows(x).cpu().numpy(), np.argmax(x.cpu().numpy(), axis=-1)), ld
+
+
+# the statistic of a residual product's rows has the same bits from the partials it leaves and from its rows, on every path by rows (skinny,
+# blocks of 64 rows, split, tiles), and the product does not depend on which of the two is asked for
+@pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 79, 128, 129, 300, 1000, 4100])
+@pytest.mark.parametrize("N,K", [(4096, 4096), (4096, 11008), (2048, 768)])
+def test_residual_statistic_from_partials_or_rows(ops, M, N, K):
+    g = torch.Generator().manual_seed(M + N)
+    x, w, r = ((torch.randn(*s, generator=g) * f).half().to(DEV) for s, f in (((M, K), 1.0), ((N, K), K ** -0.5), ((M, N), 1.0)))
+    ss = torch.empty(M, N // 128, dtype=torch.float32, device=DEV)
+    a, b = ops.linear_residual(x, w, r.clone(), ss=ss), ops.linear_residual(x, w, r.clone())
+    assert torch.equal(a, b)
+    assert torch.equal(ops.rstd_from_ss(ss, N, 1e-5), ops.row_stat(b, 1e-5))
+    assert ops.leaves_ss(M, N, K) in (False, M > 64)
