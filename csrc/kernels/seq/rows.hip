@@ -3,6 +3,7 @@
 // norm, and the routing of a mixture of experts.  All statistics and sums are fp32.
 #include "seq_common.h"
 #include "fls_seq.h"
+#include "row_vec.h"
 
 // ------------------------------------------------------------------------- group RMS norm
 // one block per (row, group): sum of squares of D / groups columns, then the scaled row part
@@ -601,6 +602,122 @@ __global__ __launch_bounds__(256) void head_norm_rope_kernel(const TI* x, int ld
   }
 }
 
+// The same for heads of whole vectors of four entries, n <= 256 EV (four or eight entries a lane): a head takes 2^shift lanes, a block
+// `rb` rows with all their heads.  The general kernel above works every head's angles out anew, sine and cosine of each entry of each
+// pair, and that, not memory, bounds it; here a block makes a row's table once, in LDS, and its loads and stores are 16 bytes a lane.
+// 6,700 rows of 16 heads of 128, all turned, fp32 in place 64 -> 22 us (110 MB: 23 at the rate of a copy), of 64 42 -> 12; 9,700 of 16 x 128
+// in bf16 79 -> 23; 6,700 of one head of 512, normed, 9.3 -> 7.9.
+template <typename TI, typename TO, int EV>
+__global__ __launch_bounds__(256) void head_norm_rope_rows(const TI* x, int ldx, int x_col, int x_hs, int heads, int n,
+                                                           const float* __restrict__ w, float eps, const float* __restrict__ freqs, int rot,
+                                                           const int* __restrict__ tok_pos, const int* __restrict__ row_map, TO* out, int ldo,
+                                                           int out_col, int out_hs, TO* raw, int ldr, int rows, int unit_after, int half,
+                                                           float amp, int shift, int rb) {
+  __shared__ float2 turn[1024];                              // (rb rows of rot / 2 angles: 128 n / 2^shift at most)
+  const int t0 = blockIdx.x * rb, hr = rot >> 1;
+  if (rot > 0) {
+    for (int i = threadIdx.x; i < rb * hr; i += 256) {
+      const int r = i / hr;
+      if (t0 + r < rows) {
+        const float ang = (float)tok_pos[t0 + r] * freqs[i - r * hr];
+        turn[i] = make_float2(amp * cosf(ang), amp * sinf(ang));
+      }
+    }
+    __syncthreads();
+  }
+  const int lanes = 1 << shift, sub = threadIdx.x & (lanes - 1), base = (threadIdx.x & 63) - sub;
+  for (int it = threadIdx.x >> shift; it < rb * heads; it += 256 >> shift) {          // (a head's lanes together)
+    const int r = it / heads, h = it - r * heads, t = t0 + r;
+    if (t >= rows) break;
+    const TI* xr = x + (size_t)t * ldx + x_col + (size_t)h * x_hs;
+    RowVec<4> v[EV];
+    float ss = 0.f;
+#pragma unroll
+    for (int e = 0; e < EV; ++e) {
+      const int c = 4 * (sub + (e << shift));
+      v[e] = c < n ? row_load<4>(xr + c) : RowVec<4>{};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss += v[e].v[j] * v[e].v[j];
+    }
+    const size_t row = row_map != nullptr ? (size_t)row_map[t] : (size_t)t;
+    if (raw != nullptr) {
+      TO* rr = raw + row * ldr + out_col + (size_t)h * out_hs;
+#pragma unroll
+      for (int e = 0; e < EV; ++e) { const int c = 4 * (sub + (e << shift)); if (c < n) row_store<4>(rr + c, v[e]); }
+    }
+    if (w != nullptr) {
+      for (int o = 1; o < lanes; o <<= 1) ss += __shfl_xor(ss, o, 64);
+      const float rs = 1.f / sqrtf(ss / (float)n + eps);
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const int c = 4 * (sub + (e << shift));
+        if (c < n) {
+          const float4 wc = *reinterpret_cast<const float4*>(w + c);
+          v[e].v[0] *= rs * wc.x; v[e].v[1] *= rs * wc.y; v[e].v[2] *= rs * wc.z; v[e].v[3] *= rs * wc.w;
+        }
+      }
+    }
+    if (rot > 0) {
+      const float2* tr = turn + r * hr;
+      float oth[EV][4];
+      if (half) {                                            // the pair's other entry: another lane's, of whichever of its vectors
+#pragma unroll
+        for (int e = 0; e < EV; ++e) {
+          const int c = 4 * (sub + (e << shift)), pc = c >= rot ? c : c >= hr ? c - hr : c + hr, q = pc >> 2;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            oth[e][j] = __shfl(v[0].v[j], base + (q & (lanes - 1)), 64);
+            if constexpr (EV == 2) {
+              const float far = __shfl(v[1].v[j], base + (q & (lanes - 1)), 64);
+              if (q >> shift) oth[e][j] = far;
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < EV; ++e) {
+        const int c = 4 * (sub + (e << shift));
+        if (c >= rot) continue;
+        if (half) {
+          const bool second = c >= hr;
+          const float2* f = tr + (second ? c - hr : c);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[e].v[j] = second ? v[e].v[j] * f[j].x + oth[e][j] * f[j].y : v[e].v[j] * f[j].x - oth[e][j] * f[j].y;
+        } else {
+          const float2* f = tr + (c >> 1);
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            const float a = v[e].v[2 * j], b = v[e].v[2 * j + 1];
+            v[e].v[2 * j] = a * f[j].x - b * f[j].y;
+            v[e].v[2 * j + 1] = b * f[j].x + a * f[j].y;
+          }
+        }
+      }
+    }
+    if (unit_after) {
+      float s2 = 0.f;
+#pragma unroll
+      for (int e = 0; e < EV; ++e)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s2 += v[e].v[j] * v[e].v[j];
+      for (int o = 1; o < lanes; o <<= 1) s2 += __shfl_xor(s2, o, 64);
+      const float rs = 1.f / sqrtf(s2 / (float)n + eps);
+#pragma unroll
+      for (int e = 0; e < EV; ++e)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[e].v[j] *= rs;
+    }
+    TO* orow = out + row * ldo + out_col + (size_t)h * out_hs;
+#pragma unroll
+    for (int e = 0; e < EV; ++e) { const int c = 4 * (sub + (e << shift)); if (c < n) row_store<4>(orow + c, v[e]); }
+  }
+}
+
+// rows of elements of `size` bytes, heads `hs` apart from column `col` on: vectors of four all aligned?
+static bool vectors_of_four(const void* p, int size, int ld, int col, int hs, int heads) {
+  return (uintptr_t)p % (4 * size) == 0 && ld % 4 == 0 && col % 4 == 0 && (heads == 1 || hs % 4 == 0);
+}
+
 extern "C" int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col, int x_hs, int heads, int n, const float* w,
                                       float eps, const float* freqs, int rot, const int* tok_pos, const int* row_map, void* out,
                                       int to, int ldo, int out_col, int out_hs, void* raw, int ldr, int rows, int unit_after,
@@ -610,6 +727,31 @@ extern "C" int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col,
   const int items = rows * heads;
   dim3 grid((items + 3) / 4);
   hipStream_t st = (hipStream_t)s;
+  const int si = tx == 1 ? 2 : 4, so = to == 1 ? 2 : 4;
+  if (n % 4 == 0 && rot % (half ? 8 : 4) == 0 && vectors_of_four(x, si, ldx, x_col, x_hs, heads) &&
+      vectors_of_four(out, so, ldo, out_col, out_hs, heads) && (raw == nullptr || vectors_of_four(raw, so, ldr, out_col, out_hs, heads)) &&
+      (w == nullptr || (uintptr_t)w % 16 == 0)) {
+    int shift = 0;
+    while ((4 << shift) < n && shift < 6) ++shift;
+    const int per = heads << shift, rb = per >= 256 ? 1 : 256 / per;
+    const dim3 blocks((rows + rb - 1) / rb);
+#define HNR_(TI, TO, EV) hipLaunchKernelGGL((head_norm_rope_rows<TI, TO, EV>), blocks, dim3(256), 0, st, (const TI*)x, ldx, x_col, x_hs, heads, n, w,  \
+                                            eps, freqs, rot, tok_pos, row_map, (TO*)out, ldo, out_col, out_hs, (TO*)raw, ldr, rows, unit_after, half,  \
+                                            amp, shift, rb)
+#define HNR(TI, TO)                  \
+  do {                               \
+    if (n <= 256) HNR_(TI, TO, 1);   \
+    else HNR_(TI, TO, 2);            \
+  } while (0)
+    if (tx == 1 && to == 1) HNR(bf16_t, bf16_t);
+    else if (tx == 1) HNR(bf16_t, float);
+    else if (to == 1) HNR(float, bf16_t);
+    else HNR(float, float);
+#undef HNR
+#undef HNR_
+    SEQ_LAUNCH_CHECK();
+    return 0;
+  }
 #define HNR(TI, TO) hipLaunchKernelGGL((head_norm_rope_kernel<TI, TO>), grid, dim3(256), 0, st, (const TI*)x, ldx, x_col, x_hs, heads, \
                                        n, w, eps, freqs, rot, tok_pos, row_map, (TO*)out, ldo, out_col, out_hs, (TO*)raw, ldr, items, unit_after, half, amp)
   if (tx == 1 && to == 1) HNR(bf16_t, bf16_t);

@@ -966,6 +966,43 @@ def test_head_norm_rope(ops, cdt, tol):
             close(outs[0][1], outs[1][1], tol)
 
 
+# heads of whole vectors (rows with all their heads in a block, angles from a table): one lane a head and all of a wave's, several rows a
+# block with the last block's partly there, two vectors a lane, parts not turned, both kinds of pairs, in place, into pages, from columns
+# that vectors fit (4) and do not (5: the kernel for any head).  fp32 against fp32: sums of up to 512 squares and angles of up to 6,000
+# radians as products of fp32 (2^-12 of a radian at worst): 3e-4, as above; bf16 results 2^-8
+@pytest.mark.parametrize("n,rot", [(4, 4), (8, 8), (20, 8), (64, 64), (64, 0), (128, 64), (132, 40), (256, 256), (260, 256), (512, 512), (512, 264)])
+@pytest.mark.parametrize("heads", [1, 3, 16])
+@pytest.mark.parametrize("half", [False, True])
+def test_head_norm_rope_vectors(ops, n, rot, heads, half):
+    H, R = ops
+    torch.manual_seed(n + rot + heads)
+    lens, pos0 = [1, 40, 3, 33], [900, 0, 17, 5000]
+    md, n_pages, _ = meta_of(lens, pos0, DEV)
+    T = sum(lens)
+    for ti, to in ((torch.float32, torch.float32), (torch.float32, torch.bfloat16), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)):
+        tol = 3e-4 if to == torch.float32 else 2 ** -8
+        for col, w, unit, paged, raw in ((4, True, False, False, True), (4, False, True, True, False), (5, True, True, False, False)):
+            x = torch.randn(T, col + heads * (n + 8) + 3 + (5 - col) + (4 - heads * n % 4) % 4, device=DEV).to(ti)
+            x = x if x.shape[1] % 4 == 0 else torch.cat([x, x[:, :4 - x.shape[1] % 4]], 1)
+            wt = torch.rand(n, device=DEV) + 0.5 if w else None
+            got = []
+            for O in (H, R):
+                out = torch.full((n_pages * 16 if paged else T, 8 + heads * (n + 4)), 3.0, device=DEV, dtype=to)
+                rw = torch.zeros_like(out) if raw else None
+                O.head_norm_rope(x, heads, n, col, n + 8, out, 4, n + 4, md, w=wt, eps=1e-5, rot=(rot, 5000.0) if rot else None,
+                                 row_map=md["kv_slot"] if paged else None, unit_after=unit, half=half, raw=rw)
+                got.append((out, rw))
+            close(got[0][0], got[1][0], tol)
+            assert bool((got[0][0][:, :4] == 3).all()) and bool((got[0][0][:, 4 + heads * (n + 4):] == 3).all())
+            if raw:
+                assert torch.equal(got[0][1], got[1][1])
+            if ti == to:                                              # in place
+                a, b = x.clone(), x.clone()
+                for O, y in ((H, a), (R, b)):
+                    O.head_norm_rope(y, heads, n, col, n + 8, y, col, n + 8, md, w=wt, eps=1e-5, rot=(rot, 5000.0) if rot else None, half=half)
+                close(a, b, tol)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("Hh,G,d,dv,ldk,ldv,shared", [(6, 2, 24, 24, 48, 48, False), (3, 1, 20, 14, 20, 20, True),
                                                       (5, 1, 72, 56, 72, 72, True), (4, 4, 64, 64, 256, 256, False)])
