@@ -46,9 +46,11 @@
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 #define KT 32             // keys per tile
-#define PLD (KT + 8)      // row stride (elements) of the transposed V tile and of the weight tiles
+#define PLD (KT + 8)      // row stride (elements) of the transposed V tile of 32 keys
 #define PT 64             // keys per tile of the prompt kernel, worked on in halves of KT
 #define VLD (PT + 8)
 #define LOG2E 1.4426950408889634f
@@ -69,6 +71,16 @@ __device__ __forceinline__ float halves_max(float v) {
 __device__ __forceinline__ float halves_sum(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// eight weights as two bf16 terms each
+__device__ __forceinline__ void two_terms(const float* p, bf16x8& hi, bf16x8& lo) {
+  typedef float floatx8 __attribute__((ext_vector_type(8)));
+  floatx8 v;
+#pragma unroll
+  for (int x = 0; x < 8; ++x) v[x] = p[x];
+  hi = __builtin_convertvector(v, bf16x8);
+  lo = __builtin_convertvector(v - __builtin_convertvector(hi, floatx8), bf16x8);
 }
 
 // (two waves per SIMD: a few registers over 256 would halve that)
@@ -313,14 +325,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
     // two bf16 terms of each weight, in the order of the keys of a row of V
     bf16x8 ph[KT / 16], pl[KT / 16];
 #pragma unroll
-    for (int ks = 0; ks < KT / 16; ++ks) {
-      typedef float floatx8 __attribute__((ext_vector_type(8)));
-      floatx8 v;
-#pragma unroll
-      for (int x = 0; x < 8; ++x) v[x] = p[8 * ks + x];
-      ph[ks] = __builtin_convertvector(v, bf16x8);
-      pl[ks] = __builtin_convertvector(v - __builtin_convertvector(ph[ks], floatx8), bf16x8);
-    }
+    for (int ks = 0; ks < KT / 16; ++ks) two_terms(p + 8 * ks, ph[ks], pl[ks]);
 #pragma unroll
     for (int ks = 0; ks < KT / 16; ++ks) {
 #pragma unroll
@@ -432,8 +437,12 @@ extern "C" int fls_seq_attn_prefill(const void* q, int ldq, int tq, const void* 
 // key/value head, range of key tiles), stages each tile of 32 rows once in LDS for all heads, and its four
 // waves share the score product's operands but own a quarter of the value columns each, so every wave
 // keeps DV / 4 accumulator columns.  All waves compute the same scores and softmax statistics (no exchange
-// between them); the weights go to LDS as bf16 pairs as above.  A block whose range is one of several
-// leaves (maximum, sum, weighted values) in `part` for attn_merge_kernel.
+// between them) and pass the weights on in registers, as above.  A block whose range is one of several
+// leaves (maximum, sum, weighted values) in `part` for attn_merge_kernel.  A block mostly walks a tile or two, so what bounds it is
+// the chain up to its first product and the code it fetches for it: keys' rows are found by a thread a key (each 16-byte piece divided
+// by the page size and read the table before), queries past the last head are not laid down, two keys of V make one store.  Merge
+// included, 24 tokens of 16 heads on rows of 576, 130 keys in 8 ranges 22.0 -> 15.2 us; of 512, 1,024 keys 44.6 -> 25.5; 5 of 256,
+// 90 keys in one 16.0 -> 9.3.
 template <int D, int DV>
 __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict__ q, int ldq, const bf16_t* kc, int ldk,
                                                          const bf16_t* vc, int ldv, bf16_t* __restrict__ out, int ldo,
@@ -441,12 +450,12 @@ __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict
                                                          const int* __restrict__ page_table, int pt_stride, int H, int G,
                                                          float scale, int window, int keep_first, float out_scale,
                                                          int page_size, float* __restrict__ part, const float* __restrict__ sink_h,
-                                                         const float* __restrict__ head_gate, int ldhg) {
+                                                         const float* __restrict__ head_gate, int ldhg, int page_shift) {
   constexpr int KLD = D + 8;
   constexpr int CPW = DV / 128;               // 32-column blocks of the values per wave
   __shared__ __attribute__((aligned(16))) bf16_t Ks[KT * KLD];
   __shared__ __attribute__((aligned(16))) bf16_t Vt[DV * PLD];
-  __shared__ __attribute__((aligned(16))) bf16_t Ps[4][2][32 * PLD];
+  __shared__ __attribute__((aligned(8))) int rows[KT];               // pool rows of the tile that is fetched next
   const int t = blockIdx.x, g = blockIdx.y, nsplit = gridDim.z;
   const int nh = H / G;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -461,18 +470,30 @@ __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict
   const int ti_lo = blockIdx.z * tps, ti_hi = min(nt, ti_lo + tps);
   const bool qok = ql < nh;
   const int head = g * nh + (qok ? ql : 0);
+  // rows of the pools that hold a tile's keys, one thread a key (keys behind the tile's last are that one again, and masked)
+  auto find_row = [&](int ti) {
+    const bool kept = ti < nt_keep;
+    const int j0 = kept ? ti * KT : lo + (ti - nt_keep) * KT;
+    const int j = min(j0 + (int)threadIdx.x, (kept ? nkeep : i + 1) - 1);
+    const int pg = page_shift >= 0 ? j >> page_shift : j / page_size;
+    return int2{table[pg], j - pg * page_size};
+  };
+  const bool any = ti_lo < ti_hi;
+  int2 next_row = {0, 0};
+  if (any && threadIdx.x < KT) next_row = find_row(ti_lo);
   // the token's queries: read once by the whole block (16-byte loads over the heads' contiguous rows),
-  // rounded to bf16 into the key tile's LDS, and from there into every wave's fragments
+  // rounded to bf16 into the key tile's LDS, and from there into every wave's fragments (what stands there for heads past the last
+  // makes scores that are masked)
   bf16x8 Qf[D / 16];
   {
     const float* qb = q + (size_t)t * ldq + (size_t)g * nh * D;
-    for (int e = threadIdx.x; e < 32 * (D / 4); e += 256) {
+#pragma unroll 3
+    for (int e = threadIdx.x; e < (any ? nh * (D / 4) : 0); e += 256) {
       const int hh = e / (D / 4), c4 = e % (D / 4);
-      float4 f = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (hh < nh) f = *reinterpret_cast<const float4*>(qb + (size_t)hh * D + c4 * 4);
-      bf16_t e4[4] = {f_to_bf16(f.x), f_to_bf16(f.y), f_to_bf16(f.z), f_to_bf16(f.w)};
-      *reinterpret_cast<uint2*>(Ks + hh * KLD + c4 * 4) = *reinterpret_cast<const uint2*>(e4);
+      const floatx4 f = *reinterpret_cast<const floatx4*>(qb + (size_t)hh * D + c4 * 4);
+      *reinterpret_cast<bf16x4*>(Ks + hh * KLD + c4 * 4) = __builtin_convertvector(f, bf16x4);
     }
+    if (any && threadIdx.x < KT) rows[threadIdx.x] = next_row.x * page_size + next_row.y;
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < D / 16; ++s) Qf[s] = *reinterpret_cast<const bf16x8*>(Ks + ql * KLD + 16 * s + h2 * 8);
@@ -485,54 +506,53 @@ __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict
   // (a silent softmax entry of score sink_h[head] is where the running maximum and sum start; with ranges the merge adds it)
   const bool snk = sink_h != nullptr && nsplit == 1;
   float m = snk ? sink_h[head] : -1e30f, l = snk ? 1.f : 0.f;
-  constexpr int NK = KT * (D / 8) / 256, NV = KT * (DV / 8) / 256;
-  static_assert(NK >= 1 && NV >= 1 && KT * (D / 8) % 256 == 0 && KT * (DV / 8) % 256 == 0 && CPW >= 1, "tile pieces per thread");
-  uint4 kreg[NK], vreg[NV];
-  auto fetch = [&](int ti) {
-    const int j0 = ti < nt_keep ? ti * KT : lo + (ti - nt_keep) * KT;
-    const int jend = ti < nt_keep ? nkeep : i + 1;
+  constexpr int NK = KT * (D / 8) / 256, NV = KT / 2 * (DV / 8) / 256;       // pieces of K; pieces of two neighbouring keys of V
+  static_assert(NK >= 1 && NV >= 1 && KT * (D / 8) % 256 == 0 && KT / 2 * (DV / 8) % 256 == 0 && CPW >= 1, "tile pieces per thread");
+  const int vpair = threadIdx.x % (KT / 2);
+  const int vplace = (vpair & ~6) | (vpair & 2) << 1 | (vpair & 4) >> 1;     // (as in the prompt kernel)
+  u32x4 kreg[NK], vreg[NV][2];
+  auto fetch = [&]() {
+    const bf16_t* kb = kc + (size_t)g * D;
 #pragma unroll
     for (int x = 0; x < NK; ++x) {
       const int e = threadIdx.x + 256 * x;
-      const int j = j0 + e / (D / 8), seg = e % (D / 8);
-      kreg[x] = make_uint4(0, 0, 0, 0);
-      if (j < jend) {
-        const size_t row = (size_t)table[j / page_size] * page_size + j % page_size;
-        kreg[x] = *reinterpret_cast<const uint4*>(kc + row * ldk + (size_t)g * D + seg * 8);
-      }
+      kreg[x] = *reinterpret_cast<const u32x4*>(kb + (size_t)rows[e / (D / 8)] * ldk + e % (D / 8) * 8);
     }
+    const int2 vr = *reinterpret_cast<const int2*>(rows + 2 * vpair);
+    const bf16_t* v0 = vc + (size_t)vr.x * ldv + (size_t)g * DV;
+    const bf16_t* v1 = vc + (size_t)vr.y * ldv + (size_t)g * DV;
 #pragma unroll
     for (int x = 0; x < NV; ++x) {
-      const int e = threadIdx.x + 256 * x;
-      const int j = j0 + e % KT, seg = e / KT;
-      vreg[x] = make_uint4(0, 0, 0, 0);
-      if (j < jend) {
-        const size_t row = (size_t)table[j / page_size] * page_size + j % page_size;
-        vreg[x] = *reinterpret_cast<const uint4*>(vc + row * ldv + (size_t)g * DV + seg * 8);
-      }
+      const int seg = (threadIdx.x + 256 * x) / (KT / 2);
+      vreg[x][0] = *reinterpret_cast<const u32x4*>(v0 + seg * 8);
+      vreg[x][1] = *reinterpret_cast<const u32x4*>(v1 + seg * 8);
     }
   };
-  if (ti_lo < ti_hi) fetch(ti_lo);
+  if (any) fetch();
+  if (ti_lo + 1 < ti_hi && threadIdx.x < KT) next_row = find_row(ti_lo + 1);
   for (int ti = ti_lo; ti < ti_hi; ++ti) {
     const bool kept = ti < nt_keep;
     const int j0 = kept ? ti * KT : lo + (ti - nt_keep) * KT;
     const int jend = kept ? nkeep : i + 1;
     __syncthreads();
+    if (threadIdx.x < KT) rows[threadIdx.x] = next_row.x * page_size + next_row.y;
 #pragma unroll
     for (int x = 0; x < NK; ++x) {
       const int e = threadIdx.x + 256 * x;
-      *reinterpret_cast<uint4*>(Ks + (e / (D / 8)) * KLD + (e % (D / 8)) * 8) = kreg[x];
+      *reinterpret_cast<u32x4*>(Ks + (e / (D / 8)) * KLD + (e % (D / 8)) * 8) = kreg[x];
     }
 #pragma unroll
     for (int x = 0; x < NV; ++x) {
-      const int e = threadIdx.x + 256 * x;
-      const int kk = e % KT, seg = e / KT;
-      const bf16_t* ev = reinterpret_cast<const bf16_t*>(&vreg[x]);
+      uint32_t* dst = reinterpret_cast<uint32_t*>(Vt + (threadIdx.x + 256 * x) / (KT / 2) * 8 * PLD) + vplace;
 #pragma unroll
-      for (int y = 0; y < 8; ++y) Vt[(seg * 8 + y) * PLD + kk] = ev[y];
+      for (int y = 0; y < 4; ++y) {
+        dst[2 * y * (PLD / 2)] = __builtin_amdgcn_perm(vreg[x][1][y], vreg[x][0][y], 0x05040100);
+        dst[(2 * y + 1) * (PLD / 2)] = __builtin_amdgcn_perm(vreg[x][1][y], vreg[x][0][y], 0x07060302);
+      }
     }
     __syncthreads();
-    if (ti + 1 < ti_hi) fetch(ti + 1);
+    if (ti + 1 < ti_hi) fetch();
+    if (ti + 2 < ti_hi && threadIdx.x < KT) next_row = find_row(ti + 2);
     floatx16 S;
 #pragma unroll
     for (int r = 0; r < 16; ++r) S[r] = 0.f;
@@ -550,15 +570,14 @@ __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict
       p[r] = vis ? S[r] * scale : -1e30f;
       mt = fmaxf(mt, p[r]);
     }
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    mt = fmaxf(mt, m);
+    mt = fmaxf(halves_max(mt), m);
     float ps = 0.f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       p[r] = p[r] > -1e29f ? __expf(p[r] - mt) : 0.f;
       ps += p[r];
     }
-    ps += __shfl_xor(ps, 32, 64);
+    ps = halves_sum(ps);
     const float corr = __expf(m - mt);
     l = l * corr + ps;
     m = mt;
@@ -566,32 +585,17 @@ __global__ __launch_bounds__(256) void attn_heads_kernel(const float* __restrict
     for (int c = 0; c < CPW; ++c)
 #pragma unroll
       for (int r = 0; r < 16; ++r) O[c][r] *= corr;
-    bf16_t* ph = Ps[wave][0] + ql * PLD;
-    bf16_t* pl = Ps[wave][1] + ql * PLD;
-#pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      bf16_t hi[4], lw[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) {
-        hi[x] = f_to_bf16(p[4 * rg + x]);
-        lw[x] = f_to_bf16(p[4 * rg + x] - bf16_to_f(hi[x]));
-      }
-      *reinterpret_cast<uint2*>(ph + 8 * rg + 4 * h2) = *reinterpret_cast<const uint2*>(hi);
-      *reinterpret_cast<uint2*>(pl + 8 * rg + 4 * h2) = *reinterpret_cast<const uint2*>(lw);
-    }
-    __builtin_amdgcn_wave_barrier();
 #pragma unroll
     for (int ks = 0; ks < KT / 16; ++ks) {
-      const bf16x8 bh = *reinterpret_cast<const bf16x8*>(ph + 16 * ks + 8 * h2);
-      const bf16x8 bl = *reinterpret_cast<const bf16x8*>(pl + 16 * ks + 8 * h2);
+      bf16x8 ph, pl;
+      two_terms(p + 8 * ks, ph, pl);
 #pragma unroll
       for (int c = 0; c < CPW; ++c) {
         const bf16x8 vf = *reinterpret_cast<const bf16x8*>(Vt + (32 * (wave * CPW + c) + ql) * PLD + 16 * ks + 8 * h2);
-        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bh, O[c], 0, 0, 0);
-        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, bl, O[c], 0, 0, 0);
+        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, ph, O[c], 0, 0, 0);
+        O[c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pl, O[c], 0, 0, 0);
       }
     }
-    __builtin_amdgcn_wave_barrier();
   }
   if (!qok) return;
   if (nsplit == 1) {
@@ -629,12 +633,13 @@ extern "C" int fls_seq_attn_heads(const void* q, int ldq, const void* kc, int ld
       ldk % 8 || ldv % 8 || G * d > ldk || G * dv > ldv || (uintptr_t)q % 16 || (uintptr_t)kc % 16 || (uintptr_t)vc % 16 ||
       (uintptr_t)out % 8 || keep_first < 0)
     return -2;
+  const int page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   dim3 grid(T, G, nsplit);
   hipStream_t st = (hipStream_t)s;
 #define ATTN_HEADS(DD, DDV)                                                                                                \
   hipLaunchKernelGGL((attn_heads_kernel<DD, DDV>), grid, dim3(256), 0, st, (const float*)q, ldq, (const bf16_t*)kc, ldk,    \
                      (const bf16_t*)vc, ldv, (bf16_t*)out, ldo, tok_seq, tok_pos, page_table, pt_stride, H, G, scale, window, \
-                     keep_first, out_scale, page_size, part, sink_h, head_gate, ldhg)
+                     keep_first, out_scale, page_size, part, sink_h, head_gate, ldhg, page_shift)
   if (d == 576 && dv == 512) ATTN_HEADS(576, 512);
   else if (d == 512 && dv == 512) ATTN_HEADS(512, 512);
   else if (d == 256 && dv == 256) ATTN_HEADS(256, 256);
