@@ -16,14 +16,19 @@
 //            (16-byte loads when the head size allows) against the query in LDS, scales, caps
 //            (cap * tanh(s / cap)) and subtracts the distance penalty r1 * log(1 + r2 * (i - j));
 //   softmax: running maximum and sum per wave (online), weights to LDS;
-//   values : lane = value column.  Every lane walks the tile's keys, reading the value rows
-//            coalesced, and accumulates its columns in registers (up to 8 x 64 columns).
+//   values : heads of 32, 64, 128 or 256 aligned values: a lane has four columns of every 64 >> vsh-th key, eight of them in
+//            flight; any other: lane = value column, the lane walks the tile's keys (up to 8 x 64 columns).
 // The four waves' (maximum, sum, accumulator) are merged through LDS at the end.  All of it is fp32;
 // only the stored keys / values and the output have the model's element type.  A decoded token is
 // one row, so its block walks the (bounded) chunk or window with four waves; a prompt has one block
 // per row and head, which fills the chip without a second kernel.
+//
+// What bounds a decoded row is latency: a key's 16-byte loads came in two or three at a time, a value's columns 2 or 4 bytes a lane.  With a
+// key's 128 bytes and eight keys' values in flight: 16 requests of 1,000 keys, 32 heads of 128 on 8, 61.7 -> 45.6 us; 8 of 90 .. 240, 16 heads
+// 10.3 -> 9.4; in fp32 prompts of 400, 300 and 210 rows 217 -> 200.
 #include "seq_common.h"
 #include "fls_seq.h"
+#include "row_vec.h"
 
 #define MAX_DV_PER_LANE 8      // value columns per lane: head value size <= 512 (a latent row)
 #define MAX_D 1024
@@ -33,14 +38,34 @@ __device__ __forceinline__ float dot_row(const T* __restrict__ k, const float* _
   float acc = 0.f;
   if (vec) {
     if constexpr (sizeof(T) == 2) {
-      for (int c = 0; c < d; c += 8) {
+      int c = 0;
+      for (; c + 64 <= d; c += 64) {                // (128 bytes of the row in flight, the sum in the same order)
+        uint4 v[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) v[x] = *reinterpret_cast<const uint4*>(k + c + 8 * x);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          const bf16_t* e = reinterpret_cast<const bf16_t*>(&v[x]);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) acc += bf16_to_f(e[i]) * q[c + 8 * x + i];
+        }
+      }
+      for (; c < d; c += 8) {
         const uint4 v = *reinterpret_cast<const uint4*>(k + c);
         const bf16_t* e = reinterpret_cast<const bf16_t*>(&v);
 #pragma unroll
         for (int i = 0; i < 8; ++i) acc += bf16_to_f(e[i]) * q[c + i];
       }
     } else {
-      for (int c = 0; c < d; c += 4) {
+      int c = 0;
+      for (; c + 32 <= d; c += 32) {
+        float4 v[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) v[x] = *reinterpret_cast<const float4*>(k + c + 4 * x);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) acc += v[x].x * q[c + 4 * x] + v[x].y * q[c + 4 * x + 1] + v[x].z * q[c + 4 * x + 2] + v[x].w * q[c + 4 * x + 3];
+      }
+      for (; c < d; c += 4) {
         const float4 v = *reinterpret_cast<const float4*>(k + c);
         acc += v.x * q[c] + v.y * q[c + 1] + v.z * q[c + 2] + v.w * q[c + 3];
       }
@@ -60,7 +85,7 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
                                                          const float* __restrict__ r1, const float* __restrict__ r2,
                                                          int chunk, int window, int keep_first,
                                                          const float* __restrict__ gate_bias, float out_scale,
-                                                         int page_size, int vec, float* __restrict__ part, int has_sink,
+                                                         int page_size, int vec, int vsh, float* __restrict__ part, int has_sink,
                                                          float sink, const float* __restrict__ sink_h,
                                                          const float* __restrict__ head_gate, int ldhg, int Gv,
                                                          AttnBlocks ab) {
@@ -68,7 +93,7 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
   __shared__ float pw[4][64];
   __shared__ int prow[4][64];
   __shared__ float mm[4], ll[4];
-  __shared__ float accs[4][MAX_DV_PER_LANE * 64];
+  __shared__ __attribute__((aligned(16))) float accs[4][MAX_DV_PER_LANE * 64];
   const int t = blockIdx.y, h = blockIdx.x;
   const int g = h / (H / G);
   const int gv = g % Gv;                          // (several score maps over the same values: Gv < G value heads)
@@ -134,6 +159,27 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const int nk = min(64, tkeys - (n - lane));
+    if (vsh >= 0) {                                // (block-uniform) four columns a lane, 64 >> vsh keys side by side, eight of these in flight
+      const int at = 64 >> vsh, sub = lane >> vsh, col = 4 * (lane & ((1 << vsh) - 1));
+#pragma unroll
+      for (int x = 0; x < 4; ++x) acc[x] *= corr;
+      for (int j0 = sub; j0 - sub < nk; j0 += 8 * at) {
+        RowVec<4> v[8];
+        float pj[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+          const int jj = min(j0 + x * at, nk - 1);
+          pj[x] = pw[wave][jj];
+          v[x] = row_load<4>(vb + (size_t)prow[wave][jj] * lv + col);
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          if (j0 + x * at < nk) {
+#pragma unroll
+            for (int y = 0; y < 4; ++y) acc[y] += pj[x] * v[x].v[y];
+          }
+      }
+    } else
 #pragma unroll
     for (int c = 0; c < MAX_DV_PER_LANE; ++c) {
       const int e = lane + 64 * c;
@@ -154,8 +200,15 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
     __builtin_amdgcn_wave_barrier();
   }
   if (lane == 0) { mm[wave] = m; ll[wave] = l; }
+  if (vsh >= 0) {
+    for (int o = 1 << vsh; o < 64; o <<= 1)
 #pragma unroll
-  for (int c = 0; c < MAX_DV_PER_LANE; ++c) accs[wave][lane + 64 * c] = acc[c];
+      for (int x = 0; x < 4; ++x) acc[x] += __shfl_xor(acc[x], o, 64);
+    if (lane >> vsh == 0) *reinterpret_cast<float4*>(&accs[wave][4 * lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  } else {
+#pragma unroll
+    for (int c = 0; c < MAX_DV_PER_LANE; ++c) accs[wave][lane + 64 * c] = acc[c];
+  }
   __syncthreads();
   if (wave == 0) {
     float f[4], inv = out_scale, mx = 0.f, lt = 0.f;
@@ -257,8 +310,12 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   const AttnBlocks ab = {pool_P, kp, ldkp, vp, ldvp, block_table, bt_stride};
   dim3 grid(H, T, nsplit);
   hipStream_t st = (hipStream_t)s;
+  // lanes (a power of two, as an exponent) that share a row of values, four columns each; -1: not so many columns or not so aligned
+  const int es = tc == 1 ? 2 : 4;
+  const bool by4 = (uintptr_t)vc % (4 * es) == 0 && ldv % 4 == 0 && (pool_P == 0 || ((uintptr_t)vp % (4 * es) == 0 && ldvp % 4 == 0));
+  const int vsh = !by4 ? -1 : dv == 32 ? 3 : dv == 64 ? 4 : dv == 128 ? 5 : dv == 256 ? 6 : -1;
 #define ATTN_PAGED_ARGS ldq, (const TC*)kc, ldk, (const TC*)vc, ldv, (TOUT*)out, ldo, tok_seq, tok_pos, page_table, pt_stride, H, G, \
-                        d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, vec, part, has_sink, sink, sink_h, \
+                        d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, vec, vsh, part, has_sink, sink, sink_h, \
                         nsplit > 1 ? nullptr : head_gate, ldhg, Gv, ab
 #define ATTN_PAGED_GO(TQ)                                                                                                   \
   do {                                                                                                                      \
