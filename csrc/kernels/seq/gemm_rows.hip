@@ -1,12 +1,14 @@
 // C[M,N] = epilogue(A[M,K] . W[N,K]^T) for few rows (decoding, small expert groups): a stream of W through the chip once.
 //
-// A block owns 16 output columns and its WV waves cut K between them, so that the loads of a whole column panel are in flight
-// at once: a wave issues 16-byte loads of its 16 weight rows (and of the rows of A, which the caches hold) for eight K steps
-// before the first of their MFMAs, straight from global memory -- nothing is read twice, LDS would only add a wait.  A K step
-// is 32 elements of bf16 (one 16x16x32 MFMA) or 16 of fp32 (four 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).
-// The waves' partial sums meet in LDS, in the order of the waves.  Bound by HBM: 8 rows against 32000 x 2048 bf16 take 32 us (4.1
-// TB/s; 41 before), 2048 x 8192 16 us (43 before, four waves with two loads in flight each), in fp32 76 and 34 us (144 and 407
-// on 64 x 64 tiles).
+// A block owns 16 output columns (or 32: NB = 2) and its WV waves cut K between them in chunks of U steps: a wave issues a chunk's
+// 16-byte loads of its weight rows, and of the rows of A that there are (the caches hold them), before the first of their MFMAs, straight
+// from global memory -- nothing of W is read twice, LDS would only add a wait.  A K step is 32 elements of bf16 (one 16x16x32 MFMA) or 16
+// of fp32 (four 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  The waves' partial sums meet in LDS, in the order of the waves.
+// What bounds it is HBM where the weight is large, else the chain of a launch, a load's latency and the sums (2048 x 2048: 6.3 us); what
+// keeps the loads in flight is many waves with few registers each, not long chunks: with four steps a chunk, no masks on whole chunks
+// and 32-bit offsets a wave takes 60 to 105 registers (eight steps: 114 to 250).  Cold weights, eight steps and here: 8 rows x 8192 x 2048
+// 12.6 -> 10.0 us, 6416 x 2048 13.5 -> 9.9, 32000 x 2048 32 -> 30.7 (floor 28); 24 rows x 6416 x 2048 14.7 -> 12.1, gated 5440 x 2048 20.2 -> 18.1;
+// fp32, 3 rows x 2048 x 8192 29.9 -> 27.3, 32000 x 2048 59.6 -> 51.4.  A second chunk's registers, loaded ahead, were slower everywhere.
 #include "seq_common.h"
 #include "fls_seq.h"
 #include "gemm_epi.h"
@@ -38,12 +40,12 @@ __device__ __forceinline__ floatx4 mfma_step(const floatx4& w, const floatx4& x,
   return c;
 }
 
-template <typename TA, typename TW, int MG, int WV, bool GATED>
+template <typename TA, typename TW, int MG, int WV, int U, int NB, bool GATED>
 __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, const TW* __restrict__ W, void* __restrict__ C, Epi epi,
                                                      int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs,
                                                      const int* __restrict__ a_rows, long long w_gs) {
   typedef typename Step<TW>::V V;
-  constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, U = GATED ? 4 : 8, HW = GATED ? 2 : 1;
+  constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, HW = GATED ? 2 * NB : NB;
   __shared__ floatx4 red[WV][MG * HW][64];
   if (offs != nullptr) {                   // row groups (experts): this block's group owns rows offs[g] .. offs[g+1]
     const int g = blockIdx.y, r0 = offs[g];
@@ -57,43 +59,45 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int steps = (K + SK - 1) / SK, per = (steps + WV - 1) / WV;
+  const int n0 = blockIdx.x * 16 * NB;
+  const int steps = (K + SK - 1) / SK, chunks = (steps + U - 1) / U, per = (chunks + WV - 1) / WV * U;
   const int s0 = wave * per, s1 = min(steps, s0 + per);
   // (a gated product: the columns' gate rows and, N rows on, their up rows)
-  const TW* wp[HW];
+  const TW* wb[HW];
+  unsigned wo[HW];
 #pragma unroll
-  for (int h = 0; h < HW; ++h) wp[h] = W + (size_t)(min(n0 + fr, N - 1) + h * N) * ldw + grp * LN;
+  for (int h = 0; h < HW; ++h) {
+    const int b = GATED ? h >> 1 : h, n1 = min(n0 + 16 * b, N - 1);
+    wb[h] = W + (size_t)(n1 + (GATED && (h & 1) ? N : 0)) * ldw;
+    wo[h] = (unsigned)(min(fr, N - 1 - n1) * ldw + grp * LN);
+  }
   for (int m0 = 0; m0 < M; m0 += 16 * MG) {
     floatx4 acc[HW][MG];
     bool ok[MG];
     const TA* xp[MG];
+    V x[MG][U];
 #pragma unroll
     for (int u = 0; u < MG; ++u) {
 #pragma unroll
       for (int h = 0; h < HW; ++h) acc[h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < U; ++i) x[u][i] = V{};             // (rows past M stay zero: no loads for them)
       const int r = min(m0 + u * 16 + fr, M - 1);
       ok[u] = m0 + u * 16 + fr < M;
       xp[u] = A + (size_t)(a_rows != nullptr ? a_rows[r] : r) * lda + grp * LN;
     }
-    for (int s = s0; s < s1; s += U) {
-      V w[HW][U], x[MG][U];
-      bool in[U];                          // (the last step may end short: K is a multiple of a lane's share)
+    int s = s0;
+    for (; s + U <= s1 && (s + U) * SK <= K; s += U) {
+      V w[HW][U];
 #pragma unroll
-      for (int i = 0; i < U; ++i) {
-        in[i] = s + i < s1 && (s + i) * SK + grp * LN < K;
+      for (int i = 0; i < U; ++i)
 #pragma unroll
-        for (int h = 0; h < HW; ++h) {
-          w[h][i] = V{};
-          if (in[i]) load_step(wp[h] + (size_t)(s + i) * SK, w[h][i]);
-        }
-      }
+        for (int h = 0; h < HW; ++h) load_step(wb[h] + s * SK + (wo[h] + i * SK), w[h][i]);
 #pragma unroll
       for (int u = 0; u < MG; ++u)
+        if (ok[u]) {
 #pragma unroll
-        for (int i = 0; i < U; ++i) {
-          x[u][i] = V{};
-          if (in[i] && ok[u]) load_step(xp[u] + (size_t)(s + i) * SK, x[u][i]);
+          for (int i = 0; i < U; ++i) load_step(xp[u] + (size_t)(s + i) * SK, x[u][i]);
         }
 #pragma unroll
       for (int i = 0; i < U; ++i)
@@ -102,22 +106,43 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
 #pragma unroll
           for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
     }
+    for (; s < s1; ++s) {                  // (the last chunk may end short, and its last step: K is a multiple of a lane's share)
+      const bool in = s * SK + grp * LN < K;
+      V w[HW], xs[MG];
+#pragma unroll
+      for (int h = 0; h < HW; ++h) {
+        w[h] = V{};
+        if (in) load_step(wb[h] + s * SK + wo[h], w[h]);
+      }
+#pragma unroll
+      for (int u = 0; u < MG; ++u) {
+        xs[u] = V{};
+        if (in && ok[u]) load_step(xp[u] + (size_t)s * SK, xs[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < MG; ++u)
+#pragma unroll
+        for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h], xs[u], acc[h][u]);
+    }
     if (m0 > 0) __syncthreads();
 #pragma unroll
     for (int u = 0; u < MG; ++u)
 #pragma unroll
       for (int h = 0; h < HW; ++h) red[wave][u * HW + h][lane] = acc[h][u];
     __syncthreads();
-    for (int i = threadIdx.x; i < 64 * MG; i += 64 * WV) {
-      const int u = i >> 6, l = i & 63;
-      const int row = m0 + u * 16 + (l & 15), col0 = n0 + 4 * (l >> 4);
+    for (int i = threadIdx.x; i < 64 * MG * NB; i += 64 * WV) {
+      // (results that go to the host as well: neighbouring lanes write a row's columns, 64 NB bytes)
+      const bool by_rows = !GATED && epi.mirror != nullptr;
+      const int l = by_rows ? (i / (4 * NB) & 15) | (i & 3) << 4 : i & 63;
+      const int b = by_rows ? (i >> 2) % NB : (i >> 6) % NB, u = (i >> 6) / NB, at = u * HW + (GATED ? 2 * b : b);
+      const int row = m0 + u * 16 + (l & 15), col0 = n0 + 16 * b + 4 * (l >> 4);
       if (row < M) {
-        floatx4 v = red[0][u * HW][l], v2 = {0.f, 0.f, 0.f, 0.f};
+        floatx4 v = red[0][at][l], v2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 1; w < WV; ++w) v += red[w][u * HW][l];
+        for (int w = 1; w < WV; ++w) v += red[w][at][l];
         if constexpr (GATED) {
 #pragma unroll
-          for (int w = 0; w < WV; ++w) v2 += red[w][u * HW + 1][l];
+          for (int w = 0; w < WV; ++w) v2 += red[w][at + 1][l];
         }
         EpiRegs er = epi_regs(epi);
         if constexpr (GATED) {
@@ -147,11 +172,12 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   }
 }
 
-template <typename TA, typename TW, int MG, int WV, bool GATED>
+
+template <typename TA, typename TW, int MG, int WV, int U, int NB, bool GATED>
 int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
           const int* a_rows, long long w_gs, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_rows<TA, TW, MG, WV, GATED>), dim3((N + 15) / 16, offs != nullptr ? groups : 1), dim3(64 * WV), 0, s, (const TA*)A,
-                     (const TW*)W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs);
+  hipLaunchKernelGGL((gemm_rows<TA, TW, MG, WV, U, NB, GATED>), dim3((N + 16 * NB - 1) / (16 * NB), offs != nullptr ? groups : 1), dim3(64 * WV), 0, s,
+                     (const TA*)A, (const TW*)W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 1 : -(int)e;
 }
@@ -161,20 +187,23 @@ int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, i
 int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
                   int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s) {
   // Row groups of 16 rows a pass over W, or 32 (17 .. 32 rows in one pass: 24 x 2048 x 2048 8.1 us, 10.3 in two).  Eight waves share
-  // K where one block a CU or less has all the columns (2048 columns: 6.4 us, 6.8 with four), four where several blocks share a CU
-  // anyway (32000 columns: 32 us, 41 with eight; floor 28).
+  // K where one block a CU or less has all the columns (2048 x 8192: 15.4 us, 17.2 with four), four where several blocks share a CU
+  // anyway (8192 x 2048: 10.0, 10.8 with eight).  With two row groups a block of 16 columns reads twice as much of A as of W: 32 where
+  // 200 blocks are left then (24 rows x 6416 x 2048: 14.1 us -> 12.1, x 32000 44.7 -> 37.9; 4096 x 14336 38.6, 50 on 128 blocks).
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
+  if ((long long)ldw * 16 + 8 >= (1LL << 31)) return 0;      // (32-bit offsets within a panel)
   const bool two = offs == nullptr && M > 16;
   const bool many = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1) > 256;
-#define ROWS_AS(TA, TW, GATED)                                                                                            \
-  (two ? (many ? start<TA, TW, 2, 4, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)          \
-               : start<TA, TW, 2, 8, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s))         \
-       : (many ? start<TA, TW, 1, 4, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)          \
-               : start<TA, TW, 1, 8, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)))
-#define ROWS(TA, TW) (gated ? ROWS_AS(TA, TW, true) : ROWS_AS(TA, TW, false))
+#define START(TA, TW, MG, WV, U, NB, GATED) start<TA, TW, MG, WV, U, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
+#define ROWS(TA, TW)                                                                                                       \
+  (gated ? (two ? (many ? START(TA, TW, 2, 4, 2, 1, true) : START(TA, TW, 2, 8, 2, 1, true))                               \
+                : (many ? START(TA, TW, 1, 4, 2, 1, true) : START(TA, TW, 1, 8, 4, 1, true)))                              \
+         : (two ? (N >= 6400 ? START(TA, TW, 2, 4, 4, 2, false)                                                            \
+                             : many ? START(TA, TW, 2, 4, 4, 1, false) : START(TA, TW, 2, 8, 4, 1, false))                 \
+                : (many ? START(TA, TW, 1, 4, 4, 1, false) : START(TA, TW, 1, 8, 4, 1, false))))
   if (tw == 0) return ROWS(float, float);
   return ta == 1 ? ROWS(bf16_t, bf16_t) : ROWS(float, bf16_t);
 #undef ROWS
-#undef ROWS_AS
+#undef START
 }
