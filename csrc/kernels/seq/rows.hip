@@ -931,18 +931,20 @@ __global__ __launch_bounds__(64 * NW) void moe_route_softmax_grouped_kernel(cons
     float my_s = 0.f, total = 0.f;
     for (int k = 0; k < top; ++k) {
       float best = -INFINITY;
-      int be = 0x7fffffff;
 #pragma unroll
-      for (int i = 0; i < NE; ++i)
-        if (ch[i] > best) { best = ch[i]; be = lane + 64 * i; }
+      for (int i = 0; i < NE; ++i) best = fmaxf(best, ch[i]);
       const float bw = wave_max(best);
-      int e = best == bw ? be : 0x7fffffff;
-      for (int o = 32; o > 0; o >>= 1) e = min(e, __shfl_xor(e, o, 64));
+      int e = 0x7fffffff;                                    // the lowest of the largest
+#pragma unroll
+      for (int i = NE - 1; i >= 0; --i) {
+        const unsigned long long at = __ballot(ch[i] == bw && bw > -INFINITY);
+        if (at != 0) e = 64 * i + __ffsll((long long)at) - 1;
+      }
       float s = 0.f;
 #pragma unroll
       for (int i = 0; i < NE; ++i)
         if (lane + 64 * i == e) { s = sc[i]; ch[i] = -INFINITY; }
-      s = __shfl(s, e & 63, 64);
+      s = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), e & 63));
       total += s;
       if (lane == k) { my_e = e; my_s = s; }
     }

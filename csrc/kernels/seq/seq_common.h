@@ -18,22 +18,6 @@ __device__ __forceinline__ float ldf(const bf16_t* p, size_t i) { return bf16_to
 __device__ __forceinline__ void stf(float* p, size_t i, float v) { p[i] = v; }
 __device__ __forceinline__ void stf(bf16_t* p, size_t i, float v) { p[i] = f_to_bf16(v); }
 
-__device__ __forceinline__ float wave_max(float v) {
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
-}
-__device__ __forceinline__ float wave_sum(float v) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-// sum over the 256 threads of a block (red: 4 floats of LDS); every thread gets the result
-__device__ __forceinline__ float block_sum_256(float v, float* red) {
-  v = wave_sum(v);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
-}
 // v of another lane of this lane's row of 16, by a DPP control (no LDS)
 template <int CTRL>
 __device__ __forceinline__ float row_dpp(float v) {
@@ -46,6 +30,34 @@ __device__ __forceinline__ float row16_sum(float v) {
   v += row_dpp<0x141>(v);          // mirrored within 8
   v += row_dpp<0x140>(v);          // mirrored within 16
   return v;
+}
+// maximum / sum over the wave, every lane gets it: the four steps within a row of 16 by DPP, the two across rows by lane swaps.  Six
+// shuffles through LDS took some 400 cycles in a kernel's chain, these 60 (24 tokens routed over 10 outputs
+// in 5 groups 7.9 -> 5.4 us, 64 over 64 in 8 28 -> 18)
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, row_dpp<0xB1>(v));
+  v = fmaxf(v, row_dpp<0x4E>(v));
+  v = fmaxf(v, row_dpp<0x141>(v));
+  v = fmaxf(v, row_dpp<0x140>(v));
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row16_sum(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+// sum over the 256 threads of a block (red: 4 floats of LDS); every thread gets the result
+__device__ __forceinline__ float block_sum_256(float v, float* red) {
+  v = wave_sum(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return red[0] + red[1] + red[2] + red[3];
 }
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.f ? z : log1pf(expf(z)); }
 // x, computed here and not in a branch of what chooses it: a lane's short alternatives side by side are cheaper than a wave's turns
