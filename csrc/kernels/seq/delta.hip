@@ -23,6 +23,7 @@
 // A request whose step starts at position 0 starts from zeros without reading its slot.
 #include "seq_common.h"
 #include "fls_seq.h"
+#include "head_out.h"
 
 // delta_chunk.hip
 int seq_delta_rule_chunked(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* az, int lda,
@@ -219,8 +220,12 @@ extern "C" int fls_seq_delta_rule_scan(const float* r, int ldr, const float* k, 
   auto finish = [&]() {
     const int items = T * H;
     if (items <= 0) return 0;
-    if (to == 1) hipLaunchKernelGGL((delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (bf16_t*)out, ldo, H, d, norm_eps, out_scale, items);
-    else hipLaunchKernelGGL((delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (float*)out, ldo, H, d, norm_eps, out_scale, items);
+    const bool done = to == 1 ? head_out(raw, g, ldg, norm_w, d, (bf16_t*)out, ldo, H, d, norm_eps, out_scale, items, (hipStream_t)s)
+                              : head_out(raw, g, ldg, norm_w, d, (float*)out, ldo, H, d, norm_eps, out_scale, items, (hipStream_t)s);
+    if (!done) {
+      if (to == 1) hipLaunchKernelGGL((delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (bf16_t*)out, ldo, H, d, norm_eps, out_scale, items);
+      else hipLaunchKernelGGL((delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, (hipStream_t)s, raw, g, ldg, norm_w, (float*)out, ldo, H, d, norm_eps, out_scale, items);
+    }
     SEQ_LAUNCH_CHECK();
     return 0;
   };

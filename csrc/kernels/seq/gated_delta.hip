@@ -16,6 +16,7 @@
 // A request whose step starts at position 0 starts from zeros without reading its slot.
 #include "seq_common.h"
 #include "fls_seq.h"
+#include "head_out.h"
 
 // delta_chunk.hip
 int seq_gated_delta_chunked(const float* qkv, int ldq, const float* beta, int ldb, const float* decay, int ldd, float* state, float* raw,
@@ -203,7 +204,7 @@ __global__ __launch_bounds__(64 * WAVES) void gated_delta_kernel(const float* __
   }
 }
 
-// one wave per (row, head): o over its root mean square in the head, weight, gate
+// one wave per (row, head): o over its root mean square in the head, weight, gate (heads that head_out does not serve)
 template <typename TO>
 __global__ __launch_bounds__(256) void gated_delta_out_kernel(const float* __restrict__ raw, const float* __restrict__ gate, int ldg,
                                                               const float* __restrict__ norm_w, TO* __restrict__ out, int ldo, int H,
@@ -274,8 +275,12 @@ extern "C" int fls_seq_gated_delta_scan(const float* qkv, int ldq, const float* 
 #undef GD_ARGS
 #undef GD_TAIL
   const int items = T * H;
-  if (to == 1) hipLaunchKernelGGL((gated_delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (bf16_t*)out, ldo, H, dv, norm_eps, items);
-  else hipLaunchKernelGGL((gated_delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (float*)out, ldo, H, dv, norm_eps, items);
+  const bool done = to == 1 ? head_out(raw, gate, ldg, norm_w, 0, (bf16_t*)out, ldo, H, dv, norm_eps, 1.f, items, st)
+                            : head_out(raw, gate, ldg, norm_w, 0, (float*)out, ldo, H, dv, norm_eps, 1.f, items, st);
+  if (!done) {
+    if (to == 1) hipLaunchKernelGGL((gated_delta_out_kernel<bf16_t>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (bf16_t*)out, ldo, H, dv, norm_eps, items);
+    else hipLaunchKernelGGL((gated_delta_out_kernel<float>), dim3((items + 3) / 4), dim3(256), 0, st, raw, gate, ldg, norm_w, (float*)out, ldo, H, dv, norm_eps, items);
+  }
   SEQ_LAUNCH_CHECK();
   return 0;
 }
