@@ -274,9 +274,15 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_kernel(const TQ* __restri
       }
     }
     if (KIND != 0 && a1 != 0.f) {
+      // (other lanes' entries: LDS is in order per wave, but the compiler must neither move these loads above the stores nor the next
+      // half's stores above these loads)
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
       const float* pq = pen[wave] + 31 - ql + 4 * h2;
 #pragma unroll
       for (int r = 0; r < 16; ++r) p[r] -= a1 * pq[8 * (r >> 2) + (r & 3)];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
     if (gated) {
 #pragma unroll

@@ -346,6 +346,32 @@ def test_prompt_attention_kinds(ops, Hh, G, lens, pos0, kind):
         close(o1, o2, 3e-5)
 
 
+# every distance's penalty at its place: queries of zeros, so that a weight is (1 + r2 distance)^-r1 alone, and values that are the key's
+# unit vector, so that each output is one weight.  Two bf16 terms of a weight (2^-17) and fp32 logarithms of up to 10 times r1 <= 3: 3e-5
+# of the weight; none for a key behind the query
+@pytest.mark.parametrize("n,pos0", [(128, 0), (97, 31), (33, 95), (32, 64), (70, 1)])
+@pytest.mark.parametrize("sigmoid", [False, True])
+def test_prompt_attention_penalty_of_every_distance(ops, n, pos0, sigmoid):
+    H, _ = ops
+    Hh, G, d, keys = 8, 2, 128, pos0 + n
+    md, npages, _ = meta_of([n], [pos0], DEV)
+    kc, vc = torch.randn(npages, 16, G * d, device=DEV).bfloat16(), torch.zeros(npages, 16, G, d, device=DEV).bfloat16()
+    j = torch.arange(keys, device=DEV)
+    vc.view(-1, G, d)[md["page_table"][0].long()[j // 16] * 16 + j % 16, :, j] = 1.0
+    r1, r2 = torch.linspace(0.1, 3.0, Hh, device=DEV), torch.linspace(2.0, 0.01, Hh, device=DEV)
+    bias = torch.linspace(-2, 1, Hh, device=DEV)
+    out = torch.empty(n, Hh * d, device=DEV)
+    H.attn_paged(torch.zeros(n, Hh * d, device=DEV).bfloat16(), kc, vc.view(npages, 16, G * d), md, Hh, G, d, d, 0.1, 0.0, r1, r2, 0, 16,
+                 torch.bfloat16, out=out, **(dict(gate_bias=bias) if sigmoid else {}))
+    dist = (torch.arange(pos0, keys)[:, None] - torch.arange(keys)[None, :]).double()
+    s = -r1.cpu().double()[:, None, None] * torch.log1p(r2.cpu().double()[:, None, None] * dist.clamp(min=0))
+    s = torch.where(dist >= 0, s, -torch.inf)
+    want = torch.sigmoid(s + bias.cpu().double()[:, None, None]) if sigmoid else torch.softmax(s, -1)
+    got = out.cpu().double().view(n, Hh, d)[:, :, :keys].permute(1, 0, 2)
+    assert bool(((got - want).abs() <= 3e-5 * want).all())
+    assert not bool(out.view(n, Hh, d)[:, :, keys:].any())
+
+
 # norms with rows in registers: one to eight steps of 1024 columns a group, the last one partly filled, the widest and the first beyond it
 # (8192, 8196), odd widths and strides that go to the general kernel, one weight for all columns; the residual update with the
 # next norm against the two in turn.  fp32 outputs against fp64: sums of up to 8196 squares in a tree, 1e-6; bf16 rounding 2^-8
