@@ -328,6 +328,7 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
     int rc = 0;
     if (offs != nullptr ? M <= 8 * groups && M <= (tw == 1 ? 128 : 64) : groups == 1 && M <= 32)
       rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, st);
+    if (rc == 0 && mirror != nullptr) return SEQ_NOT_SERVED;
     if (rc == 0) rc = seq_gemm_tile(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, a_gs, a_mod, w_gs, c_gs, st);
     if (rc != 0) return rc == 1 ? 0 : rc;
   }

@@ -466,6 +466,28 @@ def test_rows_written_to_the_host(ops, M, N, cdt):
         assert torch.equal(c, H.matmul_nt(a, w, **how)) and torch.equal(am.cpu().long(), c.argmax(1).cpu())
         assert torch.equal(down[:M * N].view(M, N), c.cpu()) and torch.equal(down[M * N:M * N + M].view(torch.int32), am.cpu())
         assert bool((down[M * N + M:] == -7.0).all())
+        down.fill_(-7.0)
+        nowhere = H.host_rows(torch.zeros(1, dtype=torch.int64, device=DEV))
+        assert torch.equal(c, H.matmul_nt(a, w, mirror=nowhere, **how)) and torch.equal(am, H.argmax_f32(c, nowhere))
+        torch.cuda.synchronize()
+        assert bool((down == -7.0).all())
+
+
+# weight rows so far apart (2^27 elements: past the few-row kernel's 32-bit offsets) that another kernel takes the product: the argmax then
+# writes the rows
+def test_rows_written_to_the_host_of_far_weight_rows(ops):
+    H, _ = ops
+    M, N, K = 3, 4, 64
+    w = torch.empty_strided((N, K), (2 ** 27, 1), dtype=torch.bfloat16, device=DEV).copy_(torch.randn(N, K))
+    a = torch.randn(M, K, device=DEV).bfloat16()
+    down = torch.full((M * N + M,), -7.0, pin_memory=True)
+    mirror = H.host_rows(torch.tensor([down.data_ptr()], dtype=torch.int64, device=DEV))
+    c = H.matmul_nt(a, w, mirror=mirror)
+    am = H.argmax_f32(c, mirror)
+    torch.cuda.synchronize()
+    close(c, a.float() @ w.float().t(), 1e-5)
+    assert not mirror.rows_there
+    assert torch.equal(down[:M * N].view(M, N), c.cpu()) and torch.equal(down[M * N:].view(torch.int32), am.cpu())
 
 
 @pytest.mark.parametrize("n", [1, 3, 4, 64, 4095, 4096, 4097, 9001])
