@@ -20,8 +20,8 @@ int fls_seq_version(void);
 // = [gate rows; up rows] (N / 2 each), C has N / 2 columns: silu(g) u, gelu(g) u, or the clamped gate of fls_seq_gate_mul
 // with limit p and alpha q; no bias), stored as type tc (fp32, or bf16 when the consumer is the next product).
 // a_rows (with offs; nullable): row r of the product is made from row a_rows[r] of A, which has at most M rows.
-// mirror (nullable): a cell on the device that holds an address the device can write (pinned host memory, say): the results, fp32 rows of
-// N, go there too.
+// mirror (nullable): a cell on the device that holds an address the device can write (pinned host memory, say), or null: the results, fp32
+// rows of N, go there too, or nowhere else.
 // SEQ_NOT_SERVED: nothing was done -- a mirror of anything but a plain product of up to 32 rows; a gated product or a_rows, and rows whose alignment or size only the general kernels take.
 #define SEQ_NOT_SERVED (-100)
 int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* C, int tc, const float* bias, const float* act,

@@ -20,7 +20,7 @@ struct Epi {
   int tc;                // element type of C: 0 fp32, 1 bf16
   int act_n;             // kind 3: columns per number of act
   float p, q;
-  float* const* mirror;  // where the fp32 results go as well (the cell, on the device, holds an address the device can write; null: nowhere)
+  float* const* mirror;  // where the fp32 results go as well (the cell, on the device, holds an address the device can write; null, here or there: nowhere)
 };
 struct EpiRegs { float ap, an; };
 __device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {

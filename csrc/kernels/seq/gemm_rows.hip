@@ -47,6 +47,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   typedef typename Step<TW>::V V;
   constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, HW = GATED ? 2 * NB : NB;
   __shared__ floatx4 red[WV][MG * HW][64];
+  float* const host = !GATED && epi.mirror != nullptr ? *epi.mirror : nullptr;
   if (offs != nullptr) {                   // row groups (experts): this block's group owns rows offs[g] .. offs[g+1]
     const int g = blockIdx.y, r0 = offs[g];
     M = offs[g + 1] - r0;
@@ -132,7 +133,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
     __syncthreads();
     for (int i = threadIdx.x; i < 64 * MG * NB; i += 64 * WV) {
       // (results that go to the host as well: neighbouring lanes write a row's columns, 64 NB bytes)
-      const bool by_rows = !GATED && epi.mirror != nullptr;
+      const bool by_rows = host != nullptr;
       const int l = by_rows ? (i / (4 * NB) & 15) | (i & 3) << 4 : i & 63;
       const int b = by_rows ? (i >> 2) % NB : (i >> 6) % NB, u = (i >> 6) / NB, at = u * HW + (GATED ? 2 * b : b);
       const int row = m0 + u * 16 + (l & 15), col0 = n0 + 16 * b + 4 * (l >> 4);
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
             else reinterpret_cast<float*>(C)[(size_t)row * ldc + col] = v[x];
           }
           // (N is a multiple of 4 then: rows of N, 64 bytes of one a store)
-          if (epi.mirror != nullptr && col0 < N) *reinterpret_cast<floatx4*>(*epi.mirror + (size_t)row * N + col0) = v;
+          if (host != nullptr && col0 < N) *reinterpret_cast<floatx4*>(host + (size_t)row * N + col0) = v;
         }
       }
     }

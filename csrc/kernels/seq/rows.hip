@@ -427,11 +427,12 @@ extern "C" int fls_seq_unary(const float* z, int ldz, void* y, int ty, int ldy, 
 // threads with 16-byte loads (32000 columns: 8 loads deep, 6 us; 256 threads of single loads 21)
 #define ARGMAX_THREADS 1024
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __restrict__ z, int ldz, int cols, int vec, int* __restrict__ out,
-                                                               void* const* __restrict__ host, int with_rows) {
+                                                               void* const* __restrict__ cell, int with_rows) {
   __shared__ float bv[ARGMAX_THREADS];
   __shared__ int bi[ARGMAX_THREADS];
   const float* zr = z + (size_t)blockIdx.x * ldz;
-  float* const hr = host != nullptr && with_rows ? reinterpret_cast<float*>(*host) + (size_t)blockIdx.x * cols : nullptr;
+  void* const host = cell != nullptr ? *cell : nullptr;
+  float* const hr = host != nullptr && with_rows ? reinterpret_cast<float*>(host) + (size_t)blockIdx.x * cols : nullptr;
   float best = -INFINITY;
   int at = 0x7fffffff;
   const int c4 = vec ? cols & ~3 : 0;
@@ -467,7 +468,7 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __r
   if (threadIdx.x == 0) {
     const int best_at = bi[0] == 0x7fffffff ? 0 : bi[0];
     out[blockIdx.x] = best_at;
-    if (host != nullptr) reinterpret_cast<int*>(*host)[(size_t)gridDim.x * cols + blockIdx.x] = best_at;
+    if (host != nullptr) reinterpret_cast<int*>(host)[(size_t)gridDim.x * cols + blockIdx.x] = best_at;
   }
 }
 

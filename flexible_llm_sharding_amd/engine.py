@@ -565,11 +565,9 @@ class ShardedRunner:
                 return state, self.ops.argmax_f32(state, meta["mirror"])
             self._decode_graphs = StepGraphs(self.dev, forward, self.ops, self.cfg.vocab_size)
         batch = pack_step(entries, self.seq_cache)
-        got = self._decode_graphs.run(batch, self.seq_cache.generation, any(len(e.want) for e in entries))
-        if got is not None:
-            for i, e in enumerate(entries):
-                if len(e.want):
-                    out[i] = (got[0][i:i + 1], got[1][i:i + 1])
+        wanted = [i for i, e in enumerate(entries) if len(e.want)]
+        for i, row in zip(wanted, self._decode_graphs.run(batch, self.seq_cache.generation, wanted)):
+            out[i] = row
         for e in entries:
             self.seq_cache.trim(e.rid)
         self.stats = {"tokens": float(len(entries)), "graph_replays": float(self._decode_graphs.replays),

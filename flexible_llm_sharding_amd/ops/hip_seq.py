@@ -48,7 +48,7 @@ def _vec(t: torch.Tensor, name: str, n: int, dtype=torch.float32):
 
 class HostRows:
     """Where a step's logits and their argmax go on the host: ``cell`` (one int64 on the device) holds the address of rows x vocab
-    floats and, behind them, the rows' argmax; ``rows_there``: the logits are written already."""
+    floats and, behind them, the rows' argmax, or 0: nowhere; ``rows_there``: the logits are written already."""
 
     def __init__(self, cell: torch.Tensor):
         self.cell, self.rows_there = cell, False

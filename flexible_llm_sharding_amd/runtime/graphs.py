@@ -277,9 +277,9 @@ class _StepInputs:
         self.meta = arrays.views(self.flat)
         self.meta.update(n_seqs=B, max_rows=1)
 
-    def fill(self, host: Dict[str, np.ndarray], down: torch.Tensor) -> None:
+    def fill(self, host: Dict[str, np.ndarray], address: int) -> None:
         """(the step that last read ``up`` has been waited for)"""
-        self.address[0] = down.data_ptr()
+        self.address[0] = address
         for dst, v in zip(self.views, host.values()):
             dst[...] = v
 
@@ -297,8 +297,8 @@ class StepGraphs:
     the wanted ones.
 
     A step's index arrays are segments of one int32 buffer that the graph's first kernel fetches from pinned memory, and its
-    logits and their argmax go straight to pinned memory, by the kernels that make them, at the address the buffer begins with:
-    a step is one launch and one wait (with a copy before the graph and two behind it the GPU idled 60 of 650 us of a step of 8
+    logits and their argmax go straight to pinned memory, by the kernels that make them, at the address the buffer begins with (0, where
+    no row is wanted: nowhere): a step is one launch and one wait (with a copy before the graph and two behind it the GPU idled 60 of 650 us of a step of 8
     requests)."""
 
     TABLE_BUCKET = 16
@@ -342,8 +342,8 @@ class StepGraphs:
         m["want_idx"] = np.arange(B, dtype=np.int32)
         return m
 
-    def run(self, batch, generation: int, want: bool):
-        """One step, waited for -> (logits [B, V] fp32, argmax [B] int32) on the host, the caller's own; None without ``want``."""
+    def run(self, batch, generation: int, want: List[int]) -> List[Tuple[np.ndarray, np.ndarray]]:
+        """One step, waited for -> (logits [1, V] fp32, argmax [1] int32) of each row of ``want`` on the host, the caller's own."""
         if generation != self.generation:
             self.graphs.clear()
             self.seen.clear()
@@ -351,23 +351,24 @@ class StepGraphs:
         B = len(batch.rids)
         host = self.host_meta(batch)
         key = (B,) + tuple(v.shape[1] for v in host.values() if v.ndim == 2)
-        n = 4 * B * (self.vocab + 1)
-        if self._down is None or self._down.numel() < n:
-            self._down = alloc_host(n)
+        n = B * (self.vocab + 1)
+        if want and (self._down is None or self._down.numel() < 4 * n):
+            self._down = alloc_host(4 * n)
         try:
-            self._replay(key, host, B)
+            self._replay(key, host, B, self._down.data_ptr() if want else 0)
         finally:                                       # (pinned memory of the step is not touched before its kernels are done)
             torch.cuda.current_stream(self.dev).synchronize()
         if not want:
-            return None
-        raw = self._down.numpy()[:n].copy()
-        return raw[:-4 * B].view(np.float32).reshape(B, self.vocab), raw[-4 * B:].view(np.int32)
+            return []
+        words = self._down.numpy()[:4 * n].view(np.int32)
+        logits, am = words[:-B].view(np.float32).reshape(B, self.vocab), words[-B:]
+        return [(logits[i:i + 1].copy(), am[i:i + 1].copy()) for i in want]
 
-    def _replay(self, key, host, B: int) -> None:
+    def _replay(self, key, host, B: int, address: int) -> None:
         g = self.graphs.get(key)
         if g is not None:
             self.graphs.move_to_end(key)
-            g.inputs.fill(host, self._down)
+            g.inputs.fill(host, address)
         else:
             first = key not in self.seen
             if first:
@@ -375,7 +376,7 @@ class StepGraphs:
                     self.seen.popitem(last=False)
                 self.seen[key] = _StepInputs(host, B, self.ADDRESS, self.dev)
             inputs = self.seen[key]
-            inputs.fill(host, self._down)
+            inputs.fill(host, address)
             if first:
                 self.eager += 1
                 self._step(inputs)

@@ -611,6 +611,41 @@ def test_captured_decode_steps_equal_eager(tmp_path, monkeypatch):
     assert np.array_equal(eager, graphed)
 
 
+@pytest.mark.gpu
+def test_captured_decode_steps_bring_down_the_wanted_rows(tmp_path, monkeypatch):
+    """Steps that want every row, one, or none, through the eager step, the capture and the replays: the wanted rows equal the eager
+    ones, each in memory of its own, and a step that wants none writes nothing to the host."""
+    if not gpu_available():
+        pytest.skip("no GPU")
+
+    def run(graphs: bool):
+        monkeypatch.setenv("FLS_DECODE_GRAPHS", "1" if graphs else "0")
+        cfg, sd, runner, _ = build(tmp_path, STACK, seed=21, device="cuda:0", dtype=torch.bfloat16, max_tokens=256, max_seqs=4, loop=LOOP)
+        a, b = (nu.tokens(n, cfg["vocab"], 60 + n) for n in (40, 33))
+        outs = []
+        runner.step([StepEntry("a", a[:10], [9]), StepEntry("b", b[:12], [11])])
+        for t in range(16):
+            wants = (([], []), ([0], [0]), ([], [0]), ([0], []))[t % 4]
+            down = runner._decode_graphs._down if runner._decode_graphs is not None else None
+            if down is not None:
+                down.fill_(0x5a)
+            r = runner.step([StepEntry("a", [a[10 + t]], wants[0]), StepEntry("b", [b[12 + t]], wants[1])])
+            for x, want in zip(r, wants):
+                if want:
+                    outs += [x[0], x[1].reshape(1, 1).astype(np.float32)]
+                    assert not graphs or (x[0].flags.owndata and x[1].flags.owndata)
+            if down is not None:
+                assert bool((down == 0x5a).all()) == (t % 4 == 0)
+        replays = runner._decode_graphs.replays if runner._decode_graphs is not None else 0
+        runner.close()
+        return np.concatenate(outs, 1), replays
+
+    eager, n0 = run(False)
+    graphed, n1 = run(True)
+    assert n0 == 0 and n1 >= 14
+    assert np.array_equal(eager, graphed)
+
+
 def test_trace_run_program_replays_steps(tmp_path):
     """bin/trace_run as a process on a two-request schedule: prompts of unequal length in one step, then one token each; a
     flushed 'done <step>' after each step, logits files for the steps that want some, exit code 0 at end of input."""

@@ -445,10 +445,11 @@ def test_epilogue_bf16_values(ops, kind):
     assert bool((err <= want[:, None].abs() * 2 ** -8 + (1 + (z6 * (u6.abs() + 1)).abs())[:, None] * 2.0 ** -126).all())
 
 
-# results that go to pinned host memory by the kernels that make them: the few-row product's rows bit for bit (32 rows are its most), or,
-# where another kernel takes the product (more rows, columns that are no multiple of 4), the rows by the argmax; the argmax behind them
+# results that go to pinned host memory by the kernels that make them: the few-row product's rows bit for bit (32 rows are its most, blocks of 32
+# columns from 6,400 on), or, where another kernel takes the product (more rows, columns that are no multiple of 4), the rows by the
+# argmax; the argmax behind them; a cell of 0: nowhere
 @pytest.mark.parametrize("M", [1, 3, 16, 17, 32, 33])
-@pytest.mark.parametrize("N", [4, 20, 1000, 4100, 510, 1023])
+@pytest.mark.parametrize("N", [4, 20, 1000, 4100, 6400, 6404, 510, 1023])
 @pytest.mark.parametrize("cdt", [torch.bfloat16, torch.float32])
 def test_rows_written_to_the_host(ops, M, N, cdt):
     H, _ = ops
