@@ -58,3 +58,13 @@ def test_refuses_what_it_cannot_pass():
             f(1, sig, None)
     with pytest.raises(ValueError):
         f(0, "i", None)
+
+
+def test_a_library_of_other_signatures_is_refused(tmp_path):
+    """A kernel library built before fls_moe_gemm lost an argument says so by its version, and is refused with what to do about it."""
+    if shutil.which("gcc") is None:
+        pytest.skip("no gcc")
+    (tmp_path / "old.c").write_text("int fls_kernels_version(void) { return 33; }")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", str(tmp_path / "old.so")], check=True)
+    with pytest.raises(RuntimeError, match="stale build"):
+        _native._load_kernels(str(tmp_path / "old.so"))
