@@ -426,20 +426,23 @@ extern "C" int fls_seq_unary(const float* z, int ldz, void* y, int ty, int ldy, 
 // first index of the row maximum.  Few rows (decoding): a block per row, so what bounds it is one block's chain of loads: 1024
 // threads with 16-byte loads (32000 columns: 8 loads deep, 6 us; 256 threads of single loads 21)
 #define ARGMAX_THREADS 1024
+// (HOST 1: the indexes go to the address in `cell` too, 2: the rows before them as well; kernels of their own, because the question in the
+// loop cost 1.6 of 15 us at 151,936 columns)
+template <int HOST>
 __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __restrict__ z, int ldz, int cols, int vec, int* __restrict__ out,
-                                                               void* const* __restrict__ cell, int with_rows) {
+                                                               void* const* __restrict__ cell) {
   __shared__ float bv[ARGMAX_THREADS];
   __shared__ int bi[ARGMAX_THREADS];
   const float* zr = z + (size_t)blockIdx.x * ldz;
-  void* const host = cell != nullptr ? *cell : nullptr;
-  float* const hr = host != nullptr && with_rows ? reinterpret_cast<float*>(host) + (size_t)blockIdx.x * cols : nullptr;
+  void* const host = HOST ? *cell : nullptr;
+  float* const hr = HOST == 2 && host != nullptr ? reinterpret_cast<float*>(host) + (size_t)blockIdx.x * cols : nullptr;
   float best = -INFINITY;
   int at = 0x7fffffff;
   const int c4 = vec ? cols & ~3 : 0;
   for (int c = 4 * threadIdx.x; c < c4; c += 4 * ARGMAX_THREADS) {
     const float4 q = *reinterpret_cast<const float4*>(zr + c);
     const float v[4] = {q.x, q.y, q.z, q.w};
-    if (hr != nullptr) {
+    if (HOST == 2 && hr != nullptr) {
       if (cols % 4 == 0) *reinterpret_cast<float4*>(hr + c) = q;
       else
 #pragma unroll
@@ -451,7 +454,7 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __r
   }
   for (int c = c4 + threadIdx.x; c < cols; c += ARGMAX_THREADS) {
     const float v = zr[c];
-    if (hr != nullptr) hr[c] = v;
+    if (HOST == 2 && hr != nullptr) hr[c] = v;
     if (v > best || (v == best && c < at)) { best = v; at = c; }
   }
   bv[threadIdx.x] = best;
@@ -468,14 +471,15 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_kernel(const float* __r
   if (threadIdx.x == 0) {
     const int best_at = bi[0] == 0x7fffffff ? 0 : bi[0];
     out[blockIdx.x] = best_at;
-    if (host != nullptr) reinterpret_cast<int*>(host)[(size_t)gridDim.x * cols + blockIdx.x] = best_at;
+    if (HOST && host != nullptr) reinterpret_cast<int*>(host)[(size_t)gridDim.x * cols + blockIdx.x] = best_at;
   }
 }
 
 extern "C" int fls_seq_argmax(const float* z, int ldz, int rows, int cols, int* out, void* const* host, int with_rows, fls_stream_t s) {
   if (rows <= 0) return 0;
-  hipLaunchKernelGGL(argmax_kernel, dim3(rows), dim3(ARGMAX_THREADS), 0, (hipStream_t)s, z, ldz, cols, (uintptr_t)z % 16 == 0 && ldz % 4 == 0, out,
-                     host, with_rows);
+  const int vec = (uintptr_t)z % 16 == 0 && ldz % 4 == 0;
+  const auto kernel = host == nullptr ? argmax_kernel<0> : with_rows ? argmax_kernel<2> : argmax_kernel<1>;
+  hipLaunchKernelGGL(kernel, dim3(rows), dim3(ARGMAX_THREADS), 0, (hipStream_t)s, z, ldz, cols, vec, out, host);
   SEQ_LAUNCH_CHECK();
   return 0;
 }
