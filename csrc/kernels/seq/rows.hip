@@ -608,8 +608,9 @@ __global__ __launch_bounds__(256) void head_norm_rope_kernel(const TI* x, int ld
 }
 
 // The same for heads of whole vectors of four entries, n <= 256 EV (four or eight entries a lane): a head takes 2^shift lanes, a block
-// `rb` rows with all their heads.  The general kernel above works every head's angles out anew, sine and cosine of each entry of each
-// pair, and that, not memory, bounds it; here a block makes a row's table once, in LDS, and its loads and stores are 16 bytes a lane.
+// `rb` rows with all their heads, or, where that would be few blocks, hb heads of a row.  The general kernel above works every head's
+// angles out anew, sine and cosine of each entry of each pair, and that, not memory, bounds it; here a block makes a row's table once,
+// in LDS, and its loads and stores are 16 bytes a lane.
 // 6,700 rows of 16 heads of 128, all turned, fp32 in place 64 -> 22 us (110 MB: 23 at the rate of a copy), of 64 42 -> 12; 9,700 of 16 x 128
 // in bf16 79 -> 23; 6,700 of one head of 512, normed, 9.3 -> 7.9.
 template <typename TI, typename TO, int EV>
@@ -617,9 +618,9 @@ __global__ __launch_bounds__(256) void head_norm_rope_rows(const TI* x, int ldx,
                                                            const float* __restrict__ w, float eps, const float* __restrict__ freqs, int rot,
                                                            const int* __restrict__ tok_pos, const int* __restrict__ row_map, TO* out, int ldo,
                                                            int out_col, int out_hs, TO* raw, int ldr, int rows, int unit_after, int half,
-                                                           float amp, int shift, int rb) {
+                                                           float amp, int shift, int rb, int hb) {
   __shared__ float2 turn[1024];                              // (rb rows of rot / 2 angles: 128 n / 2^shift at most)
-  const int t0 = blockIdx.x * rb, hr = rot >> 1;
+  const int t0 = blockIdx.x * rb, hr = rot >> 1, h0 = blockIdx.y * hb, nh = min(hb, heads - h0);
   if (rot > 0) {
     for (int i = threadIdx.x; i < rb * hr; i += 256) {
       const int r = i / hr;
@@ -631,8 +632,8 @@ __global__ __launch_bounds__(256) void head_norm_rope_rows(const TI* x, int ldx,
     __syncthreads();
   }
   const int lanes = 1 << shift, sub = threadIdx.x & (lanes - 1), base = (threadIdx.x & 63) - sub;
-  for (int it = threadIdx.x >> shift; it < rb * heads; it += 256 >> shift) {          // (a head's lanes together)
-    const int r = it / heads, h = it - r * heads, t = t0 + r;
+  for (int it = threadIdx.x >> shift; it < rb * nh; it += 256 >> shift) {          // (a head's lanes together)
+    const int r = it / nh, h = h0 + it - r * nh, t = t0 + r;
     if (t >= rows) break;
     const TI* xr = x + (size_t)t * ldx + x_col + (size_t)h * x_hs;
     RowVec<4> v[EV];
@@ -738,11 +739,12 @@ extern "C" int fls_seq_head_norm_rope(const void* x, int tx, int ldx, int x_col,
       (w == nullptr || (uintptr_t)w % 16 == 0)) {
     int shift = 0;
     while ((4 << shift) < n && shift < 6) ++shift;
-    const int per = heads << shift, rb = per >= 256 ? 1 : 256 / per;
-    const dim3 blocks((rows + rb - 1) / rb);
+    const int per = heads << shift, rb = per >= 256 ? 1 : 256 / per, side = 256 >> shift;       // (heads that a block has side by side)
+    const int parts = per <= 256 || rows >= 1024 ? 1 : min((heads + side - 1) / side, (1024 + rows - 1) / rows), hb = (heads + parts - 1) / parts;
+    const dim3 blocks((rows + rb - 1) / rb, (heads + hb - 1) / hb);
 #define HNR_(TI, TO, EV) hipLaunchKernelGGL((head_norm_rope_rows<TI, TO, EV>), blocks, dim3(256), 0, st, (const TI*)x, ldx, x_col, x_hs, heads, n, w,  \
                                             eps, freqs, rot, tok_pos, row_map, (TO*)out, ldo, out_col, out_hs, (TO*)raw, ldr, rows, unit_after, half,  \
-                                            amp, shift, rb)
+                                            amp, shift, rb, hb)
 #define HNR(TI, TO)                  \
   do {                               \
     if (n <= 256) HNR_(TI, TO, 1);   \

@@ -1052,6 +1052,23 @@ def test_head_norm_rope_vectors(ops, n, rot, heads, half):
                 close(a, b, tol)
 
 
+# a row's heads over several blocks (fewer than 1,024 rows of more heads than a block has side by side), the last block's heads fewer, a block
+# that walks its heads, and rows enough for a block each; tolerance as above
+@pytest.mark.parametrize("T,heads,n", [(1, 32, 512), (3, 33, 64), (300, 20, 128), (700, 48, 132), (1023, 9, 256), (1024, 9, 256)])
+@pytest.mark.parametrize("half", [False, True])
+def test_head_norm_rope_heads_over_blocks(ops, T, heads, n, half):
+    H, R = ops
+    torch.manual_seed(T + heads)
+    md, _, _ = meta_of([T], [7], DEV)
+    x, w = torch.randn(T, heads * n, device=DEV), torch.rand(n, device=DEV) + 0.5
+    got = []
+    for O in (H, R):
+        out = torch.full((T, heads * n + 4), 3.0, device=DEV)
+        O.head_norm_rope(x, heads, n, 0, n, out, 0, n, md, w=w, eps=1e-5, rot=(n // 16 * 8, 5000.0), half=half)
+        got.append(out)
+    close(got[0], got[1], 3e-4)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("Hh,G,d,dv,ldk,ldv,shared", [(6, 2, 24, 24, 48, 48, False), (3, 1, 20, 14, 20, 20, True),
                                                       (5, 1, 72, 56, 72, 72, True), (4, 4, 64, 64, 256, 256, False)])
