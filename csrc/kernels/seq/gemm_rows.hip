@@ -107,23 +107,28 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
 #pragma unroll
           for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
     }
-    for (; s < s1; ++s) {                  // (the last chunk may end short, and its last step: K is a multiple of a lane's share)
-      const bool in = s * SK + grp * LN < K;
-      V w[HW], xs[MG];
+    if (s < s1) {                          // (the last chunk may end short, and its last step: K is a multiple of a lane's share)
+      V w[HW][U];
 #pragma unroll
-      for (int h = 0; h < HW; ++h) {
-        w[h] = V{};
-        if (in) load_step(wb[h] + s * SK + wo[h], w[h]);
+      for (int i = 0; i < U; ++i) {
+        const bool in = s + i < s1 && (s + i) * SK + grp * LN < K;
+#pragma unroll
+        for (int h = 0; h < HW; ++h) {
+          w[h][i] = V{};
+          if (in) load_step(wb[h] + s * SK + (wo[h] + i * SK), w[h][i]);
+        }
+#pragma unroll
+        for (int u = 0; u < MG; ++u) {
+          x[u][i] = V{};
+          if (in && ok[u]) load_step(xp[u] + (size_t)(s + i) * SK, x[u][i]);
+        }
       }
 #pragma unroll
-      for (int u = 0; u < MG; ++u) {
-        xs[u] = V{};
-        if (in && ok[u]) load_step(xp[u] + (size_t)s * SK, xs[u]);
-      }
+      for (int i = 0; i < U; ++i)
 #pragma unroll
-      for (int u = 0; u < MG; ++u)
+        for (int u = 0; u < MG; ++u)
 #pragma unroll
-        for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h], xs[u], acc[h][u]);
+          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
     }
     if (m0 > 0) __syncthreads();
 #pragma unroll
