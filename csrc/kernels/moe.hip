@@ -6,9 +6,8 @@
 //                      optional renormalisation, -> ids [T*k], weights [T*k] (fp32; Qwen3-MoE rounds
 //                      them to fp16 like HF)
 //   3. fls_moe_plan    stable counting sort of the T*k (token, slot) entries by expert (3 launches)
-//                      -> offs [E+1] (rows of each expert in the permuted order), tiles [E+1] (their
-//                      256-row GEMM tiles, prefix), rows [T*k] (permuted row -> token), dest [T*k]
-//                      (entry -> permuted row).  Deterministic: entries keep token order inside an
+//                      -> offs [E+1] (rows of each expert in the permuted order), rows [T*k] (permuted row
+//                      -> token), dest [T*k] (entry -> permuted row).  Deterministic: entries keep token order inside an
 //                      expert, so a run is bitwise reproducible.
 //   4. fls_moe_gemm    the v10 MFMA GEMM in grouped form (gemm_v10.h) on M tiles of 128, 192 or 256 rows: every expert's rows
 //                      in ONE launch, no host round trip for the counts.  gate/up + SwiGLU gathers its A rows
@@ -187,9 +186,9 @@ __global__ __launch_bounds__(PB_THREADS) void moe_hist_kernel(const int* __restr
   for (int e = threadIdx.x; e < E; e += PB_THREADS) bhist[(size_t)blockIdx.x * E + e] = hist[e];
 }
 
-// one block: bhist [B][E] counts -> per-block bases (in place), offs [E+1], tiles [E+1]
+// one block: bhist [B][E] counts -> per-block bases (in place), offs [E+1]
 __global__ __launch_bounds__(MAX_E) void moe_scan_kernel(int* __restrict__ bhist, int nb, int E,
-                                                         int* __restrict__ offs, int* __restrict__ tiles) {
+                                                         int* __restrict__ offs) {
   __shared__ int cnt[MAX_E], off[MAX_E + 1];
   const int e = threadIdx.x;
   if (e < E) {
@@ -199,15 +198,12 @@ __global__ __launch_bounds__(MAX_E) void moe_scan_kernel(int* __restrict__ bhist
   }
   __syncthreads();
   if (e == 0) {
-    int o = 0, t = 0;
+    int o = 0;
     offs[0] = 0;
-    tiles[0] = 0;
     for (int j = 0; j < E; ++j) {
       off[j] = o;
       o += cnt[j];
-      t += (cnt[j] + BM - 1) / BM;
       offs[j + 1] = o;
-      tiles[j + 1] = t;
     }
   }
   __syncthreads();
@@ -404,13 +400,13 @@ extern "C" int fls_moe_router_route(const void* h, int ldh, const void* wr, int 
 // bhist: scratch of plan_scratch_ints(n, E) ints
 extern "C" int fls_moe_plan_scratch(int n, int E) { return ((n + PB_ENTRIES - 1) / PB_ENTRIES) * E; }
 
-extern "C" int fls_moe_plan(const int* ids, int n, int k, int E, int* offs, int* tiles, int* rows, int* dest,
-                            int* bhist, fls_stream_t s) {
+extern "C" int fls_moe_plan(const int* ids, int n, int k, int E, int* offs, int* rows, int* dest, int* bhist,
+                            fls_stream_t s) {
   if (E < 1 || E > MAX_E || k < 1 || n < 0) return -2;
   auto st = (hipStream_t)s;
   const int nb = max(1, (n + PB_ENTRIES - 1) / PB_ENTRIES);
   hipLaunchKernelGGL(moe_hist_kernel, dim3(nb), dim3(PB_THREADS), 0, st, ids, n, E, bhist);
-  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(MAX_E), 0, st, bhist, nb, E, offs, tiles);
+  hipLaunchKernelGGL(moe_scan_kernel, dim3(1), dim3(MAX_E), 0, st, bhist, nb, E, offs);
   hipLaunchKernelGGL(moe_place_kernel, dim3(nb), dim3(PB_THREADS), 0, st, ids, n, k, E, bhist, rows, dest);
   FLS_CHECK_LAUNCH();
   return 0;

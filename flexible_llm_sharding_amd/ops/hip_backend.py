@@ -49,12 +49,11 @@ def _f16(t: torch.Tensor, name: str):
 @dataclass
 class MoeRoute:
     """Device-side routing of one MoE call (csrc/kernels/moe.hip): per (token, slot) entry the
-    expert id and weight; per expert its permuted-row offsets and 256-row tile prefix; permuted
-    row -> token (``rows``) and entry -> permuted row (``dest``)."""
+    expert id and weight; per expert its permuted-row offsets; permuted row -> token (``rows``) and
+    entry -> permuted row (``dest``)."""
     ids: torch.Tensor
     w: torch.Tensor
     offs: torch.Tensor
-    tiles: torch.Tensor
     rows: torch.Tensor
     dest: torch.Tensor
     k: int
@@ -352,7 +351,7 @@ class HipOps:
 
     def moe_route_logits(self, logits, top_k: int, norm_topk: bool, round_w16: bool = False) -> "MoeRoute":
         """Routing from fp16 router logits [T, E]: top-k ids / weights per token and the stable
-        expert sort (offsets, 256-row tile prefix, permuted row -> token, entry -> permuted row)."""
+        expert sort (offsets, permuted row -> token, entry -> permuted row)."""
         _f16(logits, "logits")
         T, E = logits.shape
         k, n, dev = int(top_k), T * int(top_k), logits.device
@@ -366,11 +365,11 @@ class HipOps:
     def _moe_plan(self, ids, w, E: int, k: int) -> "MoeRoute":
         n, dev = ids.numel(), ids.device
         scratch = self.k.fls_moe_plan_scratch(n, E)
-        meta = torch.empty(2 * (E + 1) + 2 * n + scratch, dtype=torch.int32, device=dev)
-        o = 2 * (E + 1)
-        r = MoeRoute(ids, w, meta[:E + 1], meta[E + 1:o], meta[o:o + n], meta[o + n:o + 2 * n], k)
-        _chk(self.k.fls_moe_plan(ids.data_ptr(), n, k, E, r.offs.data_ptr(), r.tiles.data_ptr(), r.rows.data_ptr(),
-                                 r.dest.data_ptr(), meta[o + 2 * n:].data_ptr(), _stream()), "fls_moe_plan")
+        meta = torch.empty(E + 1 + 2 * n + scratch, dtype=torch.int32, device=dev)
+        o = E + 1
+        r = MoeRoute(ids, w, meta[:o], meta[o:o + n], meta[o + n:o + 2 * n], k)
+        _chk(self.k.fls_moe_plan(ids.data_ptr(), n, k, E, r.offs.data_ptr(), r.rows.data_ptr(), r.dest.data_ptr(),
+                                 meta[o + 2 * n:].data_ptr(), _stream()), "fls_moe_plan")
         return r
 
     def moe_experts(self, h, x, wgu, wdown, route: "MoeRoute", m_out=None, y_out=None, shared=None):
