@@ -32,12 +32,12 @@ __device__ __forceinline__ EpiRegs epi_regs(const Epi& e) {
 __device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
   if (e.kind == EPI_DECAY) r.ap = -expf(e.act[col / e.act_n]);
 }
-template <int KIND>
+template <int KIND, bool SIDES = true>
 __device__ __forceinline__ float epi_value_of(float v, const Epi& e, const EpiRegs& r) {
   if constexpr (KIND == EPI_RELU2) { v = fmaxf(v, 0.f); return v * v; }
   else if constexpr (KIND == EPI_DECAY) return expf(r.ap * softplus_f(v));
   else if constexpr (KIND == EPI_XIELU) {
-    const float low = both_sides(r.an * expm1_less_z(v));
+    const float low = both_sides<SIDES>(r.an * expm1_less_z<SIDES>(v));
     return (v > 0.f ? r.ap * v * v : low) + 0.5f * v;
   }
   else if constexpr (KIND == EPI_SOFTCAP) return e.p * tanhf(v / e.p);
@@ -55,7 +55,7 @@ __device__ __forceinline__ float epi_gate_of(float g, float u, const Epi& e) {
 __device__ __forceinline__ float epi_value(float v, const Epi& e, const EpiRegs& r) {
   if (e.kind == EPI_RELU2) return epi_value_of<EPI_RELU2>(v, e, r);
   if (e.kind == EPI_DECAY) return epi_value_of<EPI_DECAY>(v, e, r);
-  if (e.kind == EPI_XIELU) return epi_value_of<EPI_XIELU>(v, e, r);
+  if (e.kind == EPI_XIELU) return epi_value_of<EPI_XIELU, false>(v, e, r);
   if (e.kind == EPI_SOFTCAP) return epi_value_of<EPI_SOFTCAP>(v, e, r);
   if (e.kind == EPI_SCALE) return epi_value_of<EPI_SCALE>(v, e, r);
   return v;
