@@ -16,16 +16,20 @@
 //            (16-byte loads when the head size allows) against the query in LDS, scales, caps
 //            (cap * tanh(s / cap)) and subtracts the distance penalty r1 * log(1 + r2 * (i - j));
 //   softmax: running maximum and sum per wave (online), weights to LDS;
-//   values : heads of 32, 64, 128 or 256 aligned values: a lane has four columns of every 64 >> vsh-th key, eight of them in
+//   values : heads of 32, 64, 128 or 256 aligned values (FOUR): a lane has four columns of every 64 >> vsh-th key, eight of them in
 //            flight; any other: lane = value column, the lane walks the tile's keys (up to 8 x 64 columns).
 // The four waves' (maximum, sum, accumulator) are merged through LDS at the end.  All of it is fp32;
 // only the stored keys / values and the output have the model's element type.  A decoded token is
 // one row, so its block walks the (bounded) chunk or window with four waves; a prompt has one block
 // per row and head, which fills the chip without a second kernel.
 //
-// What bounds a decoded row is latency: a key's 16-byte loads came in two or three at a time, a value's columns 2 or 4 bytes a lane.  With a
-// key's 128 bytes and eight keys' values in flight: 16 requests of 1,000 keys, 32 heads of 128 on 8, 61.7 -> 45.6 us; 8 of 90 .. 240, 16 heads
-// 10.3 -> 9.4; in fp32 prompts of 400, 300 and 210 rows 217 -> 200.
+// What bounds a decoded row is latency: a key's 16-byte loads came in two or three at a time, a value's columns 2 or 4 bytes a lane.  With KU
+// of a key's 16-byte pieces and eight keys' values in flight: 16 requests of 1,000 keys, 32 heads of 128 on 8, 61.7 -> 45.6 us; 8 of 90 .. 240,
+// 16 heads 10.3 -> 9.4; in fp32 prompts of 400, 300 and 210 rows 217 -> 200.  What bounds many rows is how many waves a SIMD holds, so each form is a
+// kernel of its own (bf16: 64 registers a lane without FOUR, 94 with KU = 4, 87 with 8; both in one 136, and prompts of heads of 96 took 1.4 to
+// 1.8 times as long).  6,500 random calls, mean over the lane = column kernel by heads of values: 32 (KU = 4) 0.64 .. 0.82, with KU = 8 0.73 .. 1.02
+// and up to 1.2; 64 .. 256 (KU = 8) 0.57 .. 0.86, with KU = 4 0 to 3 hundredths more; any other (KU = 1) the same, with KU = 8 up to 1.3.  With blocks
+// (POOL, 4,300 calls) 32 .. 128 (KU = 4) 0.70 .. 0.89, with KU = 8 0.71 .. 0.89 and up to 1.2; 256 (KU = 1) 0.74 .. 0.89, with KU = 8 up to 1.3.
 #include "seq_common.h"
 #include "fls_seq.h"
 #include "row_vec.h"
@@ -33,18 +37,19 @@
 #define MAX_DV_PER_LANE 8      // value columns per lane: head value size <= 512 (a latent row)
 #define MAX_D 1024
 
-template <typename T>
+// KU pieces of 16 bytes of the row in flight, the sum in the same order
+template <typename T, int KU>
 __device__ __forceinline__ float dot_row(const T* __restrict__ k, const float* __restrict__ q, int d, int vec) {
   float acc = 0.f;
   if (vec) {
     if constexpr (sizeof(T) == 2) {
       int c = 0;
-      for (; c + 64 <= d; c += 64) {                // (128 bytes of the row in flight, the sum in the same order)
-        uint4 v[8];
+      for (; KU > 1 && c + 8 * KU <= d; c += 8 * KU) {
+        uint4 v[KU];
 #pragma unroll
-        for (int x = 0; x < 8; ++x) v[x] = *reinterpret_cast<const uint4*>(k + c + 8 * x);
+        for (int x = 0; x < KU; ++x) v[x] = *reinterpret_cast<const uint4*>(k + c + 8 * x);
 #pragma unroll
-        for (int x = 0; x < 8; ++x) {
+        for (int x = 0; x < KU; ++x) {
           const bf16_t* e = reinterpret_cast<const bf16_t*>(&v[x]);
 #pragma unroll
           for (int i = 0; i < 8; ++i) acc += bf16_to_f(e[i]) * q[c + 8 * x + i];
@@ -58,12 +63,12 @@ __device__ __forceinline__ float dot_row(const T* __restrict__ k, const float* _
       }
     } else {
       int c = 0;
-      for (; c + 32 <= d; c += 32) {
-        float4 v[8];
+      for (; KU > 1 && c + 4 * KU <= d; c += 4 * KU) {
+        float4 v[KU];
 #pragma unroll
-        for (int x = 0; x < 8; ++x) v[x] = *reinterpret_cast<const float4*>(k + c + 4 * x);
+        for (int x = 0; x < KU; ++x) v[x] = *reinterpret_cast<const float4*>(k + c + 4 * x);
 #pragma unroll
-        for (int x = 0; x < 8; ++x) acc += v[x].x * q[c + 4 * x] + v[x].y * q[c + 4 * x + 1] + v[x].z * q[c + 4 * x + 2] + v[x].w * q[c + 4 * x + 3];
+        for (int x = 0; x < KU; ++x) acc += v[x].x * q[c + 4 * x] + v[x].y * q[c + 4 * x + 1] + v[x].z * q[c + 4 * x + 2] + v[x].w * q[c + 4 * x + 3];
       }
       for (; c < d; c += 4) {
         const float4 v = *reinterpret_cast<const float4*>(k + c);
@@ -76,7 +81,7 @@ __device__ __forceinline__ float dot_row(const T* __restrict__ k, const float* _
   return acc;
 }
 
-template <typename TQ, typename T, typename TO, bool POOL>
+template <typename TQ, typename T, typename TO, bool POOL, bool FOUR, int KU>
 __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ q, int ldq, const T* kc, int ldk,
                                                          const T* vc, int ldv, TO* __restrict__ out, int ldo,
                                                          const int* __restrict__ tok_seq, const int* __restrict__ tok_pos,
@@ -116,9 +121,10 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
   const float gb = gated ? gate_bias[h] : 0.f;
   const float snk = has_sink && sink_h != nullptr ? sink_h[h] : sink;
   float m = -1e30f, l = 0.f;
-  float acc[MAX_DV_PER_LANE];
+  constexpr int NA = FOUR ? 4 : MAX_DV_PER_LANE;
+  float acc[NA];
 #pragma unroll
-  for (int c = 0; c < MAX_DV_PER_LANE; ++c) acc[c] = 0.f;
+  for (int c = 0; c < NA; ++c) acc[c] = 0.f;
   // gridDim.z > 1: the key tiles are cut into gridDim.z ranges, one block each, whose (maximum, sum,
   // weighted values) go to `part` and are merged by attn_merge_kernel
   const int nsplit = gridDim.z;
@@ -138,7 +144,7 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
     int row = 0;
     if (valid) {
       row = tab[j / page_size] * page_size + j % page_size;
-      sc = dot_row<T>(kb + (size_t)row * lk + (size_t)g * d, qs, d, vec) * scale;
+      sc = dot_row<T, KU>(kb + (size_t)row * lk + (size_t)g * d, qs, d, vec) * scale;
       if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
       if (a1 != 0.f) sc -= a1 * log1pf(a2 * (float)(i - j));
     }
@@ -159,7 +165,7 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const int nk = min(64, tkeys - (n - lane));
-    if (vsh >= 0) {                                // (block-uniform) four columns a lane, 64 >> vsh keys side by side, eight of these in flight
+    if constexpr (FOUR) {                          // 64 >> vsh keys side by side, eight of these in flight
       const int at = 64 >> vsh, sub = lane >> vsh, col = 4 * (lane & ((1 << vsh) - 1));
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc[x] *= corr;
@@ -179,28 +185,29 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
             for (int y = 0; y < 4; ++y) acc[y] += pj[x] * v[x].v[y];
           }
       }
-    } else
+    } else {
 #pragma unroll
-    for (int c = 0; c < MAX_DV_PER_LANE; ++c) {
-      const int e = lane + 64 * c;
-      if (e < dv) {
-        float a = acc[c] * corr;
-        int jj = 0;
-        for (; jj + 8 <= nk; jj += 8) {            // eight independent value loads in flight
-          float v[8];
+      for (int c = 0; c < MAX_DV_PER_LANE; ++c) {
+        const int e = lane + 64 * c;
+        if (e < dv) {
+          float a = acc[c] * corr;
+          int jj = 0;
+          for (; jj + 8 <= nk; jj += 8) {          // eight independent value loads in flight
+            float v[8];
 #pragma unroll
-          for (int x = 0; x < 8; ++x) v[x] = ldf(vb + (size_t)prow[wave][jj + x] * lv, e);
+            for (int x = 0; x < 8; ++x) v[x] = ldf(vb + (size_t)prow[wave][jj + x] * lv, e);
 #pragma unroll
-          for (int x = 0; x < 8; ++x) a += pw[wave][jj + x] * v[x];
+            for (int x = 0; x < 8; ++x) a += pw[wave][jj + x] * v[x];
+          }
+          for (; jj < nk; ++jj) a += pw[wave][jj] * ldf(vb + (size_t)prow[wave][jj] * lv, e);
+          acc[c] = a;
         }
-        for (; jj < nk; ++jj) a += pw[wave][jj] * ldf(vb + (size_t)prow[wave][jj] * lv, e);
-        acc[c] = a;
       }
     }
     __builtin_amdgcn_wave_barrier();
   }
   if (lane == 0) { mm[wave] = m; ll[wave] = l; }
-  if (vsh >= 0) {
+  if constexpr (FOUR) {
     for (int o = 1 << vsh; o < 64; o <<= 1)
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc[x] += __shfl_xor(acc[x], o, 64);
@@ -317,10 +324,17 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
 #define ATTN_PAGED_ARGS ldq, (const TC*)kc, ldk, (const TC*)vc, ldv, (TOUT*)out, ldo, tok_seq, tok_pos, page_table, pt_stride, H, G, \
                         d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, vec, vsh, part, has_sink, sink, sink_h, \
                         nsplit > 1 ? nullptr : head_gate, ldhg, Gv, ab
-#define ATTN_PAGED_GO(TQ)                                                                                                   \
-  do {                                                                                                                      \
-    if (pool_P > 0) hipLaunchKernelGGL((attn_paged_kernel<TQ, TC, TOUT, true>), grid, dim3(256), 0, st, (const TQ*)q, ATTN_PAGED_ARGS); \
-    else hipLaunchKernelGGL((attn_paged_kernel<TQ, TC, TOUT, false>), grid, dim3(256), 0, st, (const TQ*)q, ATTN_PAGED_ARGS);           \
+#define ATTN_PAGED_FORM(TQ, POOL, FOUR, KU) \
+  hipLaunchKernelGGL((attn_paged_kernel<TQ, TC, TOUT, POOL, FOUR, KU>), grid, dim3(256), 0, st, (const TQ*)q, ATTN_PAGED_ARGS)
+#define ATTN_PAGED_GO(TQ)                                         \
+  do {                                                            \
+    if (pool_P > 0) {                                             \
+      if (vsh < 0) ATTN_PAGED_FORM(TQ, true, false, 1);           \
+      else if (dv == 256) ATTN_PAGED_FORM(TQ, true, true, 1);     \
+      else ATTN_PAGED_FORM(TQ, true, true, 4);                    \
+    } else if (vsh < 0) ATTN_PAGED_FORM(TQ, false, false, 1);     \
+    else if (dv == 32) ATTN_PAGED_FORM(TQ, false, true, 4);       \
+    else ATTN_PAGED_FORM(TQ, false, true, 8);                     \
   } while (0)
   if (tc == 1) {
     using TC = bf16_t;
@@ -341,6 +355,7 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
     ATTN_PAGED_GO(float);
   }
 #undef ATTN_PAGED_GO
+#undef ATTN_PAGED_FORM
 #undef ATTN_PAGED_ARGS
   SEQ_LAUNCH_CHECK();
   if (nsplit > 1) return seq_attn_merge(part, out, to, ldo, T, H, dv, nsplit, gate_bias != nullptr, out_scale, has_sink, sink, sink_h, head_gate, ldhg, s);

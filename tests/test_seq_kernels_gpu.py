@@ -264,6 +264,33 @@ def test_attention(ops, cdt, tol, Hh, G, d, dv):
         close(o1, o2, tol)
 
 
+# values by four columns a lane (heads of 32, 64, 128 and 256) and by one (any other, or rows that vectors do not fit): keys about what a wave has
+# side by side, has in flight, and about its tiles of 64, with windows, kept first keys and a second range.  fp32 pools against fp64: sums of up to
+# 700 terms of either sign in fp32, 2e-5 of the largest
+@pytest.mark.parametrize("dv", [32, 64, 128, 256, 36])
+@pytest.mark.parametrize("d,pad", [(32, 0), (36, 0), (96, 0), (96, 2), (160, 4)])
+def test_attention_values_by_columns(ops, dv, d, pad):
+    H, _ = ops
+    Hh, G = 4, 2
+    pos0 = [0, 1, 6, 7, 8, 9, 14, 15, 16, 31, 32, 62, 63, 64, 65, 127, 128, 129, 255, 700]
+    md, npages, _ = meta_of([1] * len(pos0), pos0, DEV)
+    torch.manual_seed(dv + d)
+    kc, vc = torch.randn(npages, 16, G * d, device=DEV), torch.randn(npages, 16, G * dv + pad, device=DEV)
+    q = torch.randn(len(pos0), Hh * d, device=DEV)
+    table, k64, v64 = md["page_table"].cpu().long(), kc.cpu().double().view(-1, G, d), vc.cpu().double().view(-1, G * dv + pad)[:, :G * dv]
+    q64 = q.cpu().double().view(-1, Hh, d)
+    for window, keep in ((0, 0), (20, 0), (70, 5)):
+        got = H.attn_paged(q, kc, vc, md, Hh, G, d, dv, d ** -0.5, 0.0, None, None, 0, 16, torch.float32, window=window, keep_first=keep).cpu().double()
+        for t, i in enumerate(pos0):
+            lo = max(0, i - window + 1) if window else 0
+            j = torch.tensor(list(range(min(keep, lo))) + list(range(lo, i + 1)))
+            rows = table[t][j // 16] * 16 + j % 16
+            kk, vv = k64[rows].repeat_interleave(Hh // G, 1), v64[rows].view(-1, G, dv).repeat_interleave(Hh // G, 1)
+            p = torch.softmax(torch.einsum("hd,nhd->hn", q64[t], kk) * d ** -0.5, -1)
+            want = torch.einsum("hn,nhv->hv", p, vv).reshape(-1)
+            assert float((got[t] - want).abs().max()) < 2e-5 * float(want.abs().max()), (i, window)
+
+
 # prompt attention over 64-key tiles in two halves: lengths about a half, a tile and a 128-row block, windows and chunks that end inside
 # a half, kept first keys, pages of 24 (no power of two); `grow`: scores that rise along the keys in small steps or in large ones
 # (the running maximum grows key by key, or in jumps), with a sink far below, near and far above them.  bf16 tolerance as above
@@ -1736,7 +1763,7 @@ def test_latent_rows(ops, cdt, tol, qr, r, dr, rot):
 
 
 @pytest.mark.parametrize("heads,kv,d,dv", [(4, 2, 7, 9), (3, 3, 1, 1), (2, 1, 64, 64), (3, 3, 48, 130), (2, 2, 128, 128), (6, 2, 130, 20),
-                                           (1, 1, 256, 300), (2, 1, 100, 512), (2, 2, 256, 128), (16, 8, 64, 64)])
+                                           (1, 1, 256, 300), (2, 1, 100, 512), (2, 2, 256, 128), (16, 8, 64, 64), (2, 2, 32, 32), (3, 1, 64, 256)])
 def test_gated_delta_scan_carries_state(ops, heads, kv, d, dv):
     """The gated delta rule over unequal requests, some continuing from states in scattered slots: portions longer and shorter
     than a staged round, one row each (the fused form), strong and weak decays; outputs and states."""
