@@ -40,6 +40,8 @@
 //           in the same lane; fp32 cos/sin tables [maxpos, hd/2], pos[m].
 #include "gemm_v10.h"
 
+extern "C" int fls_gemm_v11_pays(int M, int N);      // gemm_v11.hip
+
 namespace {
 
 // ------------------------------------------------------------- generic
@@ -617,76 +619,140 @@ int splitk_slices(int M, int N, int K, size_t tiles, size_t ws_bytes) {
   return best;
 }
 
-// Which path takes a product of more than 64 rows that all of them could: the least estimated time.  A tile launch is
-// whole rounds of 256 blocks and a last one; a round of blocks takes a start and a store and nk K tiles, more per K tile when all CUs pull
-// on memory and power than when few do (full / part below, us, measured at K = 2,048 .. 28,672).  Rounds are why no one tile
-// serves a range: 600 x 12,288 x 4,096 on 256-row tiles is 144 blocks of 79 us, on 128-row ones 240 of 62; 600 x 22,016 258 blocks
-// (two rounds, 168 us) or 430 (117); 1,700 x 4,096 x 4,096 91 us on 64-row blocks, 57 here; 600 x 10,240 x 8,192 161 and 111.
+// ---- Which path takes a product that all of them could: the least estimated time.
 enum Route { ROUTE_NONE, ROUTE_SKINNY, ROUTE_SPLIT, ROUTE_MID, ROUTE_128, ROUTE_192, ROUTE_256, ROUTE_V11 };
 
-struct RoundCost { int rows; float full_k, full, part_k, part; };
-const RoundCost ROUNDS[4] = {{128, 0.92f, 4.f, 0.733f, 3.f}, {192, 1.14f, 8.f, 0.82f, 5.5f}, {256, 1.45f, 15.f, 1.f, 9.f},
-                             {384, 2.19f, 11.f, 1.6f, 10.f}};
-
-float rounds_us(const RoundCost& c, long blocks, int nk) {
-  const float full = c.full_k * nk + c.full, part = c.part_k * nk + c.part;
-  const float fill = (float)(blocks % 256) / 256.f;
-  return (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * fill * fill : 0.f);
+// The blocks that the mid-M path takes.
+enum MidForm { MID_16, MID_32, MID_64, MID_64_W4, MID_128R, MID_128, MID_128_W4 };
+// pairs: an epilogue that joins columns (SwiGLU, RoPE).  K % 128 == 0
+MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
+  // 64-column blocks for a single row tile whose 128-column grid fills less than one round of the
+  // 256 CUs: 70B generation steps with 8 prompts (M = 40) 39.7 vs 46.7 ms per step; with 32 prompts
+  // (M = 160, three row tiles) the 128-column blocks are faster, 53 vs 55.5 ms (profiles/r6_decode/
+  // mid_bn: in-graph steps, cold weights; a same-weights GEMM loop favoured 64 there too)
+  const int tiles_m = (M + mid::BMm - 1) / mid::BMm;
+  const int blocks128 = tiles_m * (N / mid::BNm);
+  // (and, since the 8-wave blocks, for two row tiles of at most ~1.25 rounds: 70B at M = 96, down
+  // 193 -> 147 us, O 49 -> 36 us; profiles/r6_decode/mid8/bn64_m96_gemm_bench.log)
+  const int blocks64 = tiles_m * (N / 64);
+  const bool bn64 = bn64_ok && (g_mid_bn == 64 || (g_mid_bn == 0 && ((blocks128 < 256 && M <= mid::BMm) ||
+                                                                     (M <= 2 * mid::BMm && blocks64 <= 320))));
+  // 8 waves for grids of < 2 rounds of 64-row blocks; 128-row blocks when 64-row ones take more than
+  // one round, 128-row ones fit in one and K is long (profiles/r6_decode/mid8, 70B at M = 320: down
+  // 343 -> 276 us; the K = 8,192 projections ran 5-10% slower with 128 rows)
+  const bool w8 = g_mid_waves == 8 || (g_mid_waves == 0 && blocks128 < 512);
+  const int rows128 = (M + 127) / 128 * (N / mid::BNm);
+  const bool r128 = g_mid_rows == 128 || (g_mid_rows == 0 && blocks128 > 256 && rows128 <= 256 && K >= 16384);
+  const bool w8_64 = g_mid_waves == 8 || (g_mid_waves == 0 && blocks64 < 512);
+  // 32-column blocks (NONE / RESID epilogues) when even 64-column ones leave CUs idle: the 70B O and
+  // down projections of generation steps with <= 12 prompts (M <= 64: 128 -> 256 blocks)
+  const bool bn32 = !pairs && N % 32 == 0 && g_mid_waves != 4 &&
+                    (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
+  // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
+  if (bn32 && g_mid_bn == 0 && N / 32 < 256 && K % col16::KT == 0) return MID_16;
+  if (bn32) return MID_32;
+  if (bn64) return w8_64 ? MID_64 : MID_64_W4;
+  if (w8) return r128 ? MID_128R : MID_128;
+  return MID_128_W4;
 }
 
-// Up to 64 rows one row tile covers them all and a product is a stream of its weight: the choice is between blocks of 16, 32 or
-// 64 columns over the whole K (ROUTE_MID; bound by a K tile's chain of wait, read and MFMA where K is long) and the K-split skinny
-// blocks with their partial sums (8 rows: 12,288 x 4,096 25 and 29 us, 4,096 x 11,008 22 and 23, 8,192 x 28,672 137 and 85; on
-// split 256-row tiles, where up to 16 rows went before, 39, 23 and 111).
-//
+// The estimates (us).  Fitted to 15,400 random products of 1 .. 3,000 rows, 512 .. 29,440 columns (and a gate / up of 57,344) and 256 .. 28,928 terms,
+// each timed on every path that it can take, with weights that no cache holds; profiles/cases/gemm_routes.txt has the errors of the fits, 5 to 9%
+// each, and what the choice makes of them.  The shortest form that tells the paths apart: a start, and the larger of the weight's stream
+// and the K tiles of 64 terms (nk), which take longer the more blocks pull on memory and power at once.
+struct MidCost { float start, k_few, k_full, start2, k2, k2_more, tb; };       // tb: bytes of weight a us, in millions
+const MidCost MID_16_COST[3] = {{4.7f, 0.05f, 0.152f, 7.4f, 0.199f, 0.f, 4.76f}, {5.f, 0.092f, 0.165f, 7.8f, 0.247f, 0.f, 4.97f},
+                                {4.7f, 0.147f, 0.207f, 6.8f, 0.33f, 0.f, 4.99f}};        // up to 16, 32 and 64 rows
+const MidCost MID_32_COST = {4.4f, 0.269f, 0.337f, 6.f, 0.415f, 0.f, 4.2f};
+const MidCost MID_64_COST[2] = {{4.8f, 0.279f, 0.452f, 6.7f, 0.658f, 0.f, 4.8f}, {4.9f, 0.288f, 0.366f, 5.9f, 0.524f, 0.f, 5.f}};      // up to 64, 128 rows
+const MidCost MID_128_COST[2] = {{7.f, 0.38f, 0.543f, 8.9f, 0.833f, 0.173f, 5.6f}, {5.5f, 0.387f, 0.476f, 7.8f, 0.65f, 0.235f, 5.f}};
+const MidCost MID_128R_COST = {-14.f, 0.514f, 0.7f, 18.f, 0.6f, 0.3f, 3.8f};
+float mid_us(int M, int N, int K, bool pairs) {
+  const MidForm form = mid_form(M, N, K, pairs, true);
+  const int tiles_m = (M + 63) / 64;
+  const float nk = (float)(K / BK), bytes = (float)N * K * 2.f;
+  const MidCost& c = form == MID_16 ? MID_16_COST[M <= 16 ? 0 : M <= 32 ? 1 : 2]
+                     : form == MID_32 ? MID_32_COST
+                     : form == MID_64 || form == MID_64_W4 ? MID_64_COST[M > 64]
+                     : form == MID_128R ? MID_128R_COST : MID_128_COST[M > 128];
+  const int width = form == MID_16 ? 16 : form == MID_32 ? 32 : form == MID_64 || form == MID_64_W4 ? 64 : 128;
+  const float rounds = (float)((form == MID_128R ? (M + 127) / 128 : tiles_m) * (N / width)) / 256.f;
+  if (form == MID_128_W4) return (4.f + 0.532f * nk) * powf(rounds, 0.842f);
+  if (rounds <= 1.f) return c.start + fmaxf(bytes / (c.tb * 1e6f), (c.k_few + (c.k_full - c.k_few) * rounds) * nk);
+  return c.start2 + fmaxf(bytes / (c.tb * 1e6f), (c.k2 + c.k2_more * (rounds - 1.f)) * nk);
+}
+
+// Tiles of `rows` x 256: whole rounds of 256 blocks and a last one.  A weight that one or two row tiles read comes from memory and not from
+// another block's read (alone).  Rounds are why no one tile serves a range: 600 x 12,288 x 4,096 on 256-row tiles is 144 blocks of 79 us, on
+// 128-row ones 240 of 62; 600 x 22,016 258 blocks (two rounds, 168 us) or 430 (117).
+struct RoundCost { int rows; float full_k, full, part_k, part, fill, alone; };
+const RoundCost ROUNDS[4] = {{128, 0.798f, 9.3f, 0.406f, 5.8f, 0.148f, 0.305f}, {192, 1.006f, 12.2f, 0.704f, 9.4f, 0.609f, 0.18f},
+                             {256, 1.311f, 14.1f, 0.91f, 11.5f, 0.979f, 0.074f}, {384, 1.907f, 17.7f, 1.458f, 14.7f, 1.17f, 0.119f}};
+float rounds_us(const RoundCost& c, int M, int N, int K) {
+  const int tiles_m = (M + c.rows - 1) / c.rows;
+  const long blocks = (long)tiles_m * (N / BN);
+  const float nk = (float)(K / BK) * (1.f + c.alone / (float)tiles_m);
+  const float full = c.full_k * nk + c.full, part = c.part_k * nk + c.part, fill = (float)(blocks % 256) / 256.f;
+  return (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * powf(fill, c.fill) : 0.f);
+}
+// The same cut along K into S slices, and their sum
+float split_us(int M, int N, int K, int S) {
+  const int tiles_m = (M + 255) / 256;
+  const long blocks = (long)tiles_m * (N / BN) * S;
+  const float nk = (float)(K / BK) / S;
+  const float full = 1.365f * nk + 3.2f, part = 0.822f * nk, fill = (float)(blocks % 256) / 256.f;
+  const float tiles = (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * powf(fill, 0.349f) : 0.f);
+  return 12.2f + fmaxf((float)N * K * 2.f / 4.04e6f, tiles) + S * ((float)M * N * 1.314e-6f + 0.094f);
+}
+// K-split blocks of all rows (gemm_skinny.h): up to 64 rows, more without a split, more
+struct SkinnyCost { float start, tb, k, k_rows, k_fill, over, slab, slice, sum; };
+const SkinnyCost SKINNY_COST[3] = {{4.9f, 4.48f, 0.2f, 0.1115f, 0.408f, 1.097f, 2.19f, 0.41f, 2.4f}, {7.f, 4.94f, -0.15f, 0.167f, 0.785f, 1.f, 0.f, 0.f, 0.f},
+                                   {0.f, 4.55f, 0.194f, 0.0955f, 0.231f, 1.167f, 1.73f, 0.17f, 9.5f}};
+float skinny_us(int M, int N, int K, int bn, int S) {
+  const SkinnyCost& c = SKINNY_COST[M <= 64 ? 0 : S == 1 ? 1 : 2];
+  const float rounds = (float)(N / bn) * S / 256.f;
+  const float k = (c.k + c.k_rows * ((M + 31) / 32) + c.k_fill * fminf(rounds, 1.f)) * powf(fmaxf(rounds, 1.f), c.over);
+  return c.start + fmaxf((float)N * K * 2.f / (c.tb * 1e6f), k * (float)(K / BK) / S) +
+         (S > 1 ? c.sum + S * (c.slab * (float)M * N * 1e-6f + c.slice) : 0.f);
+}
+
+// The rules by shape alone, for what the estimates do not serve (launch, ROUTE_NONE)
+bool split_rule(int M, size_t tiles256, int S) { return S >= 2 && (M > 64 || tiles256 * S >= 128); }
+bool mid_rule(int M, size_t tiles256) { return tiles256 < 128 || (M <= 64 && tiles256 < 512); }
+
 // ws: scratch for split-K partials (0 bytes: none).  Above four rounds of 256-row tiles the forms are within 3% of each other:
-// ROUTE_NONE (v11 or v10 by whole rounds, v11_pays)
+// ROUTE_NONE (v11 or v10 by whole rounds, v11_pays).  A path that the rules by shape take keeps the product unless another is estimated more
+// than 6% faster, which is how far off the estimates are: of 13,900 products 0.5% are then more than 6% slower than by the rules, and all
+// take 0.86 of their time by the rules, 1.005 of the best path's.
 Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
-  const int nk = K / BK;
-  const float bytes = (float)N * K * 2.f;                      // the weight, once
-  const long cols = N / BN;
-  const long tiles256 = (long)((M + 255) / 256) * cols;
+  const long tiles256 = (long)((M + 255) / 256) * (N / BN);
   if (M > ROW_CHUNK || tiles256 > 1024 || g_v10_rows || g_mid_bn || g_mid_waves || g_mid_rows || g_skinny > 1) return ROUTE_NONE;
-  if (M <= 64) {
-    if (row_exact || !g_mid || !g_skinny) return ROUTE_NONE;
-    const bool narrow = (epi == FLS_EPI_NONE || epi == FLS_EPI_RESID) && N / 32 < 256;       // (16-column blocks)
-    const float mid = narrow ? (N / 16 > 256 ? 6.5f : 4.f) + fmaxf(bytes / 4.8e6f, 0.08f * nk) + (M <= 16 ? 0.f : M <= 32 ? 0.03f : 0.062f) * nk
-                             : fmaxf(bytes / 5.8e6f + 7.f, 0.33f * nk + 3.f) + 0.05f * M;
-    const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
-    if ((S > 1 && (size_t)S * M * N * 4 > ws_bytes) || (skinny_wide(N) && M > 32)) return ROUTE_MID;
-    const float skinny = 7.f + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * nk / S) + (S > 1 ? S * (float)M * N * 1e-6f : 0.f);
-    return mid <= skinny ? ROUTE_MID : ROUTE_SKINNY;
-  }
+  if (M <= 64 && (row_exact || !g_mid || !g_skinny)) return ROUTE_NONE;
+  const bool pairs = epi == FLS_EPI_SWIGLU || is_rope(epi);
+  const bool scratch = !row_exact && ws_bytes > 0;
+  const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
+  const bool skinny = !row_exact && g_skinny && M <= 256 && (S == 1 || (size_t)S * M * N * 4 <= ws_bytes) && (M > 32 ? M > 64 || !skinny_wide(N) : true);
+  const int S2 = scratch && g_splitk && M > 64 && M <= SPLITK_MAX_M ? splitk_slices(M, N, K, (size_t)tiles256, ws_bytes) : 0;
+  const bool split = split_rule(M, (size_t)tiles256, S2);
+  const Route rules = skinny && skinny_range(M, N) ? ROUTE_SKINNY
+                      : split ? ROUTE_SPLIT
+                      : g_mid && mid_rule(M, (size_t)tiles256) ? ROUTE_MID
+                      : M >= 384 && (long)((M + 383) / 384) * (N / BN) >= 256 && fls_gemm_v11_pays(M, N) ? ROUTE_V11 : ROUTE_256;
   Route best = ROUTE_NONE;
   float least = 0.f;
   auto offer = [&](Route r, float us) {
+    if (r == rules) us *= 0.94f;
     if (best == ROUTE_NONE || us < least) {
       best = r;
       least = us;
     }
   };
-  for (int i = 0; i < 3; ++i) offer((Route)(ROUTE_128 + i), rounds_us(ROUNDS[i], (long)((M + ROUNDS[i].rows - 1) / ROUNDS[i].rows) * cols, nk));
-  if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], (long)((M + 383) / 384) * cols, nk));
-  if (g_mid) {               // 64 x 128 blocks: two share a CU, and from the third round on the weights' re-reads take over
-    const long blocks = (long)((M + 63) / 64) * (N / 128), r = (blocks + 255) / 256;
-    const float fill = bytes > 64e6f ? 1.f : 0.35f + 0.65f * (float)(blocks - 256) / 256.f;
-    offer(ROUTE_MID, r <= 1   ? (M > 128 ? 0.43f : blocks <= 128 ? 0.32f : 0.48f) * nk + 2.5f
-                     : r == 2 ? 0.43f * nk + 2.5f + fill * (0.31f * nk + 2.5f)
-                     : r == 3 ? 1.1f * nk + 5.f
-                              : (0.28f * nk + 1.5f) * r);
-  }
-  if (!row_exact && ws_bytes) {
-    const float slab = (float)M * N * 8.f / 4e6f;              // a slice's partials written and read, us
-    if (g_splitk && M <= SPLITK_MAX_M) {
-      const int S = splitk_slices(M, N, K, (size_t)tiles256, ws_bytes);
-      if (S >= 2) offer(ROUTE_SPLIT, fmaxf(16.f + bytes / 4.8e6f, 0.75f * (rounds_us(ROUNDS[2], tiles256 * S, nk / S) + 5.f + S * slab)));
-    }
-    if (g_skinny && M <= 256) {
-      const int bn = skinny_bn(M, N, K), S = skinny_slices(N, K, bn);
-      const long r = ((long)(N / bn) * S + 255) / 256;         // (its K tile: all of the rows go through LDS)
-      if (S == 1 || (size_t)S * M * N * 4 <= ws_bytes)
-        offer(ROUTE_SKINNY, (r > 2 ? 10.f : 7.f) + fmaxf(bytes / 5.2e6f, (0.35f + 0.004f * M) * r * nk / S) + (S > 1 ? 0.5f * S * slab : 0.f));
-    }
+  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs));
+  if (skinny) offer(ROUTE_SKINNY, skinny_us(M, N, K, bn, S));
+  if (split) offer(ROUTE_SPLIT, split_us(M, N, K, S2));
+  if (M > 64) {              // (up to 64 rows one row tile covers them all, and three quarters of a 256-row one are padding)
+    for (int i = 0; i < 3; ++i) offer((Route)(ROUTE_128 + i), rounds_us(ROUNDS[i], M, N, K));
+    if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], M, N, K));
   }
   return best;
 }
@@ -722,7 +788,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   if (route == ROUTE_SKINNY) route = ROUTE_NONE;             // (its operands' alignment did not allow it)
   const int S = split_ok && !ep.row_exact && (route == ROUTE_NONE || route == ROUTE_SPLIT)
                     ? splitk_slices(M, N, K, tiles256, ws_bytes) : 0;
-  if (S >= 2 && (M > 64 || tiles256 * S >= 128)) {
+  if (split_rule(M, tiles256, S)) {
     static bool attr_f32 = false;
     if (!attr_f32) {
       (void)hipFuncSetAttribute((const void*)gemm_nt_v10<EPI_F32>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -749,60 +815,25 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   }
   if (route == ROUTE_SPLIT) route = ROUTE_NONE;
   if (mid_ok && (!main_ok || route == ROUTE_MID ||
-                 (route == ROUTE_NONE && g_mid && (tiles256 < 128 || (M <= 64 && tiles256 < 512))))) {
-    // 64-column blocks for a single row tile whose 128-column grid fills less than one round of the
-    // 256 CUs: 70B generation steps with 8 prompts (M = 40) 39.7 vs 46.7 ms per step; with 32 prompts
-    // (M = 160, three row tiles) the 128-column blocks are faster, 53 vs 55.5 ms (profiles/r6_decode/
-    // mid_bn: in-graph steps, cold weights; a same-weights GEMM loop favoured 64 there too)
-    const int blocks128 = ((M + mid::BMm - 1) / mid::BMm) * (N / mid::BNm);
-    const bool bn64_ok = N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0);
-    // (and, since the 8-wave blocks, for two row tiles of at most ~1.25 rounds: 70B at M = 96, down
-    // 193 -> 147 us, O 49 -> 36 us; profiles/r6_decode/mid8/bn64_m96_gemm_bench.log)
-    const int blocks64_ = ((M + mid::BMm - 1) / mid::BMm) * (N / 64);
-    const bool bn64 = bn64_ok && (g_mid_bn == 64 || (g_mid_bn == 0 && ((blocks128 < 256 && M <= mid::BMm) ||
-                                                                       (M <= 2 * mid::BMm && blocks64_ <= 320))));
-    // 8 waves for grids of < 2 rounds of 64-row blocks; 128-row blocks when 64-row ones take more than
-    // one round, 128-row ones fit in one and K is long (profiles/r6_decode/mid8, 70B at M = 320: down
-    // 343 -> 276 us; the K = 8,192 projections ran 5-10% slower with 128 rows)
-    const bool w8 = g_mid_waves == 8 || (g_mid_waves == 0 && blocks128 < 512);
-    const int rows128 = (M + 127) / 128 * (N / mid::BNm);
-    const bool r128 = g_mid_rows == 128 || (g_mid_rows == 0 && blocks128 > 256 && rows128 <= 256 && K >= 16384);
-    const int blocks64 = ((M + mid::BMm - 1) / mid::BMm) * (N / 64);
-    const bool w8_64 = g_mid_waves == 8 || (g_mid_waves == 0 && blocks64 < 512);
-    // 32-column blocks (NONE / RESID epilogues) when even 64-column ones leave CUs idle: the 70B O and
-    // down projections of generation steps with <= 12 prompts (M <= 64: 128 -> 256 blocks)
-    constexpr bool bn32_epi = EPI == FLS_EPI_NONE || EPI == FLS_EPI_RESID;
-    const bool bn32 = bn32_epi && N % 32 == 0 && g_mid_waves != 4 &&
-                      (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
-    if constexpr (bn32_epi) {
-      // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
-      if (bn32 && g_mid_bn == 0 && N / 32 < 256 && K % col16::KT == 0) {
-        if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        FLS_CHECK_LAUNCH();
-        ss_partials(C, ldc, M, N, ep, s);
-        FLS_CHECK_LAUNCH();
-        return 0;
-      }
-      if (bn32) {
-        launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        FLS_CHECK_LAUNCH();
-        ss_partials(C, ldc, M, N, ep, s);
-        FLS_CHECK_LAUNCH();
-        return 0;
-      }
+                 (route == ROUTE_NONE && g_mid && mid_rule(M, tiles256)))) {
+    constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
+    switch (mid_form(M, N, K, pairs, N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0))) {
+      case MID_16:
+        if constexpr (!pairs) {
+          if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+          else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+          else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        }
+        break;
+      case MID_32:
+        if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        break;
+      case MID_64: launch_mid<EPI, mid::NSTAGE, 64, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_64_W4: launch_mid<EPI, mid::NSTAGE, 64>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_128R: launch_mid<EPI, mid::NSTAGE, 128, 8, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_128: launch_mid<EPI, mid::NSTAGE, 128, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_128_W4: launch_mid<EPI, mid::NSTAGE, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
     }
-    if (bn64 && w8_64)
-      launch_mid<EPI, mid::NSTAGE, 64, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-    else if (bn64)
-      launch_mid<EPI, mid::NSTAGE, 64>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-    else if (w8 && r128)
-      launch_mid<EPI, mid::NSTAGE, 128, 8, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-    else if (w8)
-      launch_mid<EPI, mid::NSTAGE, 128, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-    else
-      launch_mid<EPI, mid::NSTAGE, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
     FLS_CHECK_LAUNCH();
     ss_partials(C, ldc, M, N, ep, s);
     FLS_CHECK_LAUNCH();

@@ -281,8 +281,11 @@ int skinny_bn(int M, int N, int K) {
              ? 256 : 128;
 }
 
+// M 17..192 on the narrow projections: the range measured in profiles/r4_gen (70B shapes)
+bool skinny_range(int M, int N) { return M >= 17 && M <= 192 && (!skinny_wide(N) || skinny_wide_bn256(M, N)); }
+
 // -> 1 when the skinny path took the GEMM, 0 when it does not apply, < 0 on a launch error.  chosen: the launcher's estimate
-// (route_of) picked it; otherwise only M 17..192 on the narrow projections (the range measured in profiles/r4_gen, 70B shapes)
+// (route_of) picked it; otherwise only in skinny_range
 template <int EPI>
 int try_skinny(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
                const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes, bool chosen) {
@@ -290,7 +293,7 @@ int try_skinny(const half_t* A, const half_t* W, half_t* C, int M, int N, int K,
       ((uintptr_t)W & 15))
     return 0;
   const int rs = ((M + 31) / 32) * 2;
-  if (g_skinny == 1 && !chosen && (M < 17 || M > 192 || (skinny_wide(N) && !skinny_wide_bn256(M, N)))) return 0;
+  if (g_skinny == 1 && !chosen && !skinny_range(M, N)) return 0;
   const int bn = skinny_bn(M, N, K);
   const int S = skinny_slices(N, K, bn);
   const bool direct_epi = EPI == FLS_EPI_NONE || EPI == FLS_EPI_RESID || EPI == FLS_EPI_SWIGLU;

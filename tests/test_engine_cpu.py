@@ -982,6 +982,21 @@ def test_gemm_v11_round_rule():
     assert pays(16128, H) == 0
 
 
+def test_residual_products_that_leave_their_rows_statistic():
+    """fls_gemm_leaves_ss (a host-side rule): the tiles of 128 rows and more write a residual product's partial sums of squares, the
+    blocks of up to 64 rows, the K-split ones and shapes that no tile takes do not."""
+    from flexible_llm_sharding_amd import _native
+    try:
+        k = _native.kernels()
+    except Exception as e:  # noqa: BLE001 (library not built in this checkout)
+        pytest.skip(f"kernel library unavailable: {e}")
+    ws = 64 << 20
+    for M, N, K, want in ((16384, 4096, 4096, 1), (4100, 4096, 4096, 1), (4100, 2048, 768, 1), (1000, 4096, 11008, 1), (43008, 8192, 8192, 1),
+                          (300, 4096, 4096, 0), (79, 4096, 4096, 0), (65, 2048, 768, 0), (64, 4096, 4096, 0), (1, 4096, 4096, 0),
+                          (4100, 4096, 4160, 0), (4100, 4224, 4096, 0)):
+        assert k.fls_gemm_leaves_ss(M, N, K, ws if M <= 512 else 0) == want, (M, N, K)
+
+
 @pytest.mark.parametrize("family", ["numolorn", "nudadra"])        # (previous tokens; blocks of keys; looped layers in both)
 def test_one_token_steps_pack_like_portions(tmp_path, family):
     """A step of one token per request packs by itself; beside a two-token request the same rows go through the general

@@ -1245,4 +1245,4 @@ def test_residual_statistic_from_partials_or_rows(ops, M, N, K):
     a, b = ops.linear_residual(x, w, r.clone(), ss=ss), ops.linear_residual(x, w, r.clone())
     assert torch.equal(a, b)
     assert torch.equal(ops.rstd_from_ss(ss, N, 1e-5), ops.row_stat(b, 1e-5))
-    assert ops.leaves_ss(M, N, K) in (False, M > 64)
+    assert ops.leaves_ss(M, N, K) == (M == 4100 or (M == 1000 and N == 4096))      # (the tiles' epilogue leaves them)
