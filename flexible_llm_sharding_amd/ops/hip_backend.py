@@ -167,8 +167,12 @@ class HipOps:
         return out
 
     def linear(self, x, w):
-        # (widths that the tiled products take are faster there even for one row: 151,936 x 2,048 104 us, 134 with the GEMV)
-        if x.shape[0] <= 16 and x.shape[1] % 32 == 0 and (w.shape[0] % 128 or x.shape[1] % 128) and not getattr(self._tl, "row_exact", False):
+        # Widths that the tiled products take are faster there even for one row (151,936 x 2,048 104 us, 134 with the GEMV; 4,096 x 4,096
+        # 0.3 of its time), except wide ones of few terms, where a tile's start and store are most of it: 32,000 x 2,048 39 us, 32 with the GEMV;
+        # 62,976 x 384 17.9 and 13.7; 98,176 x 256 20.0 and 13.2 (6,000 random widths, 1 .. 16 rows: profiles/cases/gemm_routes.txt).
+        N, K = w.shape
+        tiled = N % 128 == 0 and K % 128 == 0 and (N <= 16384 or K > (2048 if N <= 32768 else 768 if N <= 65536 else 512))
+        if x.shape[0] <= 16 and K % 32 == 0 and not tiled and not getattr(self._tl, "row_exact", False):
             return self.gemv_skinny(x, w)
         return self.gemm(x, w)
 
