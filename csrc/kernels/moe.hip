@@ -339,6 +339,10 @@ int launch_grouped(const half_t* A, const half_t* W, half_t* C, int M, int N, in
 // quarters of one.  Few rows a group want small tiles, as their padding costs matrix work that the stream of weights does not hide: gate / up of
 // 128 x (2 x 768 x 2048) with 3 rows each 175 us on 256-row tiles, 138 on 128; down 101 and 67; with 94 each 228 and 187, 134 and 114.
 // Many want large ones: 750 each 643 us (the group found by a walk), 609 on 256, 648 on 128.  8 x (4096 x 14336), 600 each: 582, 539 on 192.
+// Whether a launch ends in one more round depends on the sizes, which are not known here, so 256-row tiles stay unless others are
+// estimated 7% faster: of 11,600 random products (4 .. 256 groups, even and skewed, cold weights; profiles/cases/experts_tiles.txt) 1.4% are
+// more than 5% slower than on 256-row tiles (2.1% without that), the worst 1.5 times (192 blocks in one round, 272 in two), and all take
+// 0.86 of their time; the best of the three for each 0.85.
 int grouped_hx(int M, int N, int K, int n_groups) {
   static const struct { float k_us, us; } COST[3] = {{0.85f, 7.f}, {1.13f, 9.5f}, {1.42f, 11.f}};
   const float share = (float)M / (float)min(M, n_groups);
@@ -347,7 +351,8 @@ int grouped_hx(int M, int N, int K, int n_groups) {
   for (int i = 0; i < 3; ++i) {
     const float tiles = (float)min(M, n_groups) * fmaxf(1.f, share / (float)(128 + 64 * i) + 0.5f);
     const float rounds = tiles * (float)(N / BN) / 256.f, whole = floorf(rounds), rest = rounds - whole;
-    const float t = (whole + (rest > 0.f ? 0.75f + 0.25f * rest * rest : 0.f)) * (COST[i].k_us * (float)(K / BK) + COST[i].us);
+    const float t = (whole + (rest > 0.f ? 0.75f + 0.25f * rest * rest : 0.f)) * (COST[i].k_us * (float)(K / BK) + COST[i].us) *
+                    (i == 2 ? 0.93f : 1.f);
     if (i == 0 || t < least) {
       least = t;
       best = i + 2;
