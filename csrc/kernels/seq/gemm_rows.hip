@@ -5,10 +5,11 @@
 // from global memory -- nothing of W is read twice, LDS would only add a wait.  A K step is 32 elements of bf16 (one 16x16x32 MFMA) or 16
 // of fp32 (four 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  The waves' partial sums meet in LDS, in the order of the waves.
 // What bounds it is HBM where the weight is large, else the chain of a launch, a load's latency and the sums (2048 x 2048: 6.3 us); what
-// keeps the loads in flight is many waves with few registers each, not long chunks: with four steps a chunk, no masks on whole chunks
-// and 32-bit offsets a wave takes 60 to 105 registers (eight steps: 114 to 250).  Cold weights, eight steps and here: 8 rows x 8192 x 2048
+// keeps the loads in flight is many waves with few registers each, not long chunks: with two or four steps a chunk, no masks on whole chunks
+// and 32-bit offsets a wave takes 58 to 116 registers (blocks of 32 columns 130 to 148; eight steps: 98 to 156).  Cold weights, eight steps and here: 8 rows x 8192 x 2048
 // 12.6 -> 10.0 us, 6416 x 2048 13.5 -> 9.9, 32000 x 2048 32 -> 30.7 (floor 28); 24 rows x 6416 x 2048 14.7 -> 12.1, gated 5440 x 2048 20.2 -> 18.1;
-// fp32, 3 rows x 2048 x 8192 29.9 -> 27.3, 32000 x 2048 59.6 -> 51.4.  A second chunk's registers, loaded ahead, were slower everywhere.
+// fp32, 3 rows x 2048 x 8192 29.9 -> 27.3, 32000 x 2048 59.6 -> 51.4.  A second chunk's registers, loaded ahead, were slower everywhere.  What is
+// left of K behind the whole chunks is one chunk with masks (step by step, each waiting for its loads: 21 rows x 6416 x 736 8.7 us, 7.1 so).
 #include "seq_common.h"
 #include "fls_seq.h"
 #include "gemm_epi.h"
@@ -194,8 +195,9 @@ int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const E
                   int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s) {
   // Row groups of 16 rows a pass over W, or 32 (17 .. 32 rows in one pass: 24 x 2048 x 2048 8.1 us, 10.3 in two).  Eight waves share
   // K where one block a CU or less has all the columns (2048 x 8192: 15.4 us, 17.2 with four), four where several blocks share a CU
-  // anyway (8192 x 2048: 10.0, 10.8 with eight).  With two row groups a block of 16 columns reads twice as much of A as of W: 32 where
-  // 200 blocks are left then (24 rows x 6416 x 2048: 14.1 us -> 12.1, x 32000 44.7 -> 37.9; 4096 x 14336 38.6, 50 on 128 blocks).
+  // anyway (8192 x 2048: 10.0, 10.8 with eight).  With two row groups a block of 16 columns reads twice as much of A as of W: 32 from 6,400
+  // columns on (24 rows x 6416 x 2048: 14.1 us -> 12.1, x 32000 44.7 -> 37.9; 4096 x 14336 38.6, 50 on 128 blocks).  9,700 random products
+  // (profiles/cases/few_rows_columns.txt): 1.2 to 1.3 of the time up to 4,096 columns, 0.8 to 0.96 from there to 8,176, 0.9 to 1.15 above.
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
   if ((long long)ldw * 16 + 8 >= (1LL << 31)) return 0;      // (32-bit offsets within a panel)
