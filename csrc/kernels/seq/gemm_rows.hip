@@ -5,7 +5,7 @@
 // from global memory -- nothing of W is read twice, LDS would only add a wait.  A K step is 32 elements of bf16 (one 16x16x32 MFMA) or 16
 // of fp32 (four 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  The waves' partial sums meet in LDS, in the order of the waves.
 // What bounds it is HBM where the weight is large, else the chain of a launch, a load's latency and the sums (2048 x 2048: 6.3 us); what
-// keeps the loads in flight is many waves with few registers each, not long chunks: with two or four steps a chunk, no masks on whole chunks
+// keeps the loads in flight is many waves with few registers each, not long chunks: with two or four steps a chunk (row groups: twice), no masks on whole chunks
 // and 32-bit offsets a wave takes 58 to 116 registers (blocks of 32 columns 130 to 148; eight steps: 98 to 156).  Cold weights, eight steps and here: 8 rows x 8192 x 2048
 // 12.6 -> 10.0 us, 6416 x 2048 13.5 -> 9.9, 32000 x 2048 32 -> 30.7 (floor 28); 24 rows x 6416 x 2048 14.7 -> 12.1, gated 5440 x 2048 20.2 -> 18.1;
 // fp32, 3 rows x 2048 x 8192 29.9 -> 27.3, 32000 x 2048 59.6 -> 51.4.  A second chunk's registers, loaded ahead, were slower everywhere.  What is
@@ -198,6 +198,8 @@ int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const E
   // anyway (8192 x 2048: 10.0, 10.8 with eight).  With two row groups a block of 16 columns reads twice as much of A as of W: 32 from 6,400
   // columns on (24 rows x 6416 x 2048: 14.1 us -> 12.1, x 32000 44.7 -> 37.9; 4096 x 14336 38.6, 50 on 128 blocks).  9,700 random products
   // (profiles/cases/few_rows_columns.txt): 1.2 to 1.3 of the time up to 4,096 columns, 0.8 to 0.96 from there to 8,176, 0.9 to 1.15 above.
+  // Row groups: most of a launch's blocks may belong to empty groups, and the others have their CU to themselves: twice the steps in flight (of
+  // 10,200 random products 0.7% are more than 6% slower than on eight steps, gated four; with the short chunks 12%, up to 1.5 times).
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
   if ((long long)ldw * 16 + 8 >= (1LL << 31)) return 0;      // (32-bit offsets within a panel)
@@ -206,10 +208,12 @@ int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const E
 #define START(TA, TW, MG, WV, U, NB, GATED) start<TA, TW, MG, WV, U, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
 #define ROWS(TA, TW)                                                                                                       \
   (gated ? (two ? (many ? START(TA, TW, 2, 4, 2, 1, true) : START(TA, TW, 2, 8, 2, 1, true))                               \
-                : (many ? START(TA, TW, 1, 4, 2, 1, true) : START(TA, TW, 1, 8, 4, 1, true)))                              \
+                : (many ? (offs != nullptr ? START(TA, TW, 1, 4, 4, 1, true) : START(TA, TW, 1, 4, 2, 1, true))            \
+                        : START(TA, TW, 1, 8, 4, 1, true)))                                                                \
          : (two ? (N >= 6400 ? START(TA, TW, 2, 4, 4, 2, false)                                                            \
                              : many ? START(TA, TW, 2, 4, 4, 1, false) : START(TA, TW, 2, 8, 4, 1, false))                 \
-                : (many ? START(TA, TW, 1, 4, 4, 1, false) : START(TA, TW, 1, 8, 4, 1, false))))
+                : (many ? (offs != nullptr ? START(TA, TW, 1, 4, 8, 1, false) : START(TA, TW, 1, 4, 4, 1, false))          \
+                        : START(TA, TW, 1, 8, 4, 1, false))))
   if (tw == 0) return ROWS(float, float);
   return ta == 1 ? ROWS(bf16_t, bf16_t) : ROWS(float, bf16_t);
 #undef ROWS

@@ -199,6 +199,23 @@ def test_grouped_few_rows(ops, cdt, tol, K):
     close(H.grouped_matmul_nt(a, w, offs), R.grouped_matmul_nt(a, w, offs), 1e-5)
 
 
+# more column blocks than the chip has CUs over all groups (four waves a block, twice the steps in flight): whole chunks of them, what is left
+# and a K tail, plain and gated, rows as they are and gathered
+@pytest.mark.parametrize("cdt,tol", DTYPES)
+@pytest.mark.parametrize("K", [64, 200, 1024, 1096])
+def test_grouped_few_rows_many_blocks(ops, cdt, tol, K):
+    H, R = ops
+    torch.manual_seed(K)
+    sizes = [0, 1, 0, 17, 2] + [0, 1] * 18 + [3]
+    M, E, N = sum(sizes), len(sizes), 112
+    offs = torch.tensor([0] + sizes).cumsum(0).int().to(DEV)
+    a, w = torch.randn(M, K, device=DEV).to(cdt), torch.randn(E, 2 * N, K, device=DEV).to(cdt)
+    close(H.grouped_matmul_nt(a, w, offs), R.grouped_matmul_nt(a, w, offs), 1e-5)
+    close(H.grouped_matmul_nt(a, w[:, :N].contiguous(), offs), R.grouped_matmul_nt(a, w[:, :N].contiguous(), offs), 1e-5)
+    for rows in (None, torch.randperm(M).int().to(DEV)):
+        close(H.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), R.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), 1e-5)
+
+
 # about the rows up to which row groups take the few-row kernel, spread over the groups and nearly all in one
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("M", [64, 65, 128, 129])
