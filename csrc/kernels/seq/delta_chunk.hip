@@ -277,9 +277,9 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
   constexpr int J = D / 16, NL = (L::SIZE + 1023) / 1024, BUF = NL * 1024;       // 4 KB (16 bytes a thread) at a time
   __shared__ __attribute__((aligned(16))) float fs[2][BUF];
   const int h = blockIdx.x, s = blockIdx.y;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, fr = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fr = lane & 15, grp = lane >> 4;
   const int col = (blockIdx.z * 4 + wave) * 16 + fr;
-  const bool live = col < a.dv;                               // (dv is a multiple of 16: whole waves; the others only help to load)
+  const bool live = (int)(blockIdx.z * 4 + wave) * 16 < a.dv;  // (dv is a multiple of 16: whole waves; the others only help to load)
   const int start = a.cu[s], end = a.cu[s + 1];
   const int first = start + a.c0 * CH;
   if (first >= end) return;

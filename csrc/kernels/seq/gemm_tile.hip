@@ -43,6 +43,10 @@ __device__ __forceinline__ int2 place(int b, int tiles_m, int tiles_n, int order
 }
 
 // This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
+__device__ __forceinline__ const char* uniform(const char* p) {
+  const unsigned long long v = (unsigned long long)p;
+  return (const char*)((unsigned long long)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
+}
 template <int TM, int TN>
 __device__ __forceinline__ bool locate(const Tile& a, const char*& A, const char*& W, size_t& cbase, int& m0, int& mend, int& n0) {
   int nwg = gridDim.x, tiles_m = a.tiles_m;
@@ -126,7 +130,7 @@ __device__ __forceinline__ const char* w_base(const Tile& a, const char* W, int 
 }
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, bool live) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, live ? -1 : 0, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, live ? 0x7fffffff : 0, 0x00020000);
 }
 
 // four consecutive columns as fp32, or rounded to nearest even as bf16
@@ -488,8 +492,8 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
   }
 #pragma unroll
   for (int i = 0; i < PW; ++i) wo[i] = w_offset(a, n0, (PW * wave + i) * 8 + lr) + lc * 16;
-  const char* Ab = a_base(a, A, m0);
-  const char* Wb = w_base(a, W, n0);
+  const char* Ab = uniform(a_base(a, A, m0));
+  const char* Wb = uniform(w_base(a, W, n0));
   const int nk = a.nk;
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
