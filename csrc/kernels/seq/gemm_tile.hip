@@ -42,11 +42,15 @@ __device__ __forceinline__ int2 place(int b, int tiles_m, int tiles_n, int order
   return by_m ? int2{grouped, walked} : int2{walked, grouped};
 }
 
-// This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
+// An address that is the same in every lane, for a descriptor in scalar registers.  (Descriptors must be scalar: from a vector register each
+// DMA is a loop over the lanes' descriptors.  So is one whose record count is a choice between -1 and 0, which is made as a vector sign
+// extension; 1024 x 2048 x 2048 on 64 x 128 tiles 18.4 us with such loops, 15.5 without, 8448 x 2048 x 2048 on 128 x 128 97 and 81.)
 __device__ __forceinline__ const char* uniform(const char* p) {
   const unsigned long long v = (unsigned long long)p;
   return (const char*)((unsigned long long)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)v));
 }
+
+// This block's tile: rows [m0, mend) and first column of C, operands moved to its group; false: nothing to do.
 template <int TM, int TN>
 __device__ __forceinline__ bool locate(const Tile& a, const char*& A, const char*& W, size_t& cbase, int& m0, int& mend, int& n0) {
   int nwg = gridDim.x, tiles_m = a.tiles_m;
@@ -129,6 +133,7 @@ __device__ __forceinline__ const char* w_base(const Tile& a, const char* W, int 
   return W + (size_t)(a.epi.kind < EPI_GATE ? n0 : n0 >> 1) * a.ldw;
 }
 
+// (offsets of a tile stay below 2^31: the host checks)
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base, bool live) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, live ? 0x7fffffff : 0, 0x00020000);
 }
@@ -597,44 +602,56 @@ int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
 }  // namespace
 
 // The tiles, and what a launch of each costs: rounds of `slots` blocks (what the chip holds at once), each nk K tiles and
-// a start and a store.  us per K tile and per round, measured on full rounds at K = 128 .. 8192 (one MI355X).  A launch that leaves
-// CUs idle in its last (or only) round wants smaller tiles, a long one the large tile; the cheapest sum wins.
-struct TileCost { int tm, tn, slots; float k_us, round_us; };
-// bf16 (16384 x 14336 x 4096: the 256 tile 1.49 ms, 128 x 128 2.28; 1024 x 2048 x 2048: 64 x 128 18 us, the 256 tile 45;
-// 256 x 2048 x 2048: 32 x 64 9 us, the 256 tile 45)
-static const TileCost TILES[] = {{256, 256, 256, 1.42f, 11.f},     // least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows (0.63 before)
-                                 {128, 128, 512, 1.08f, 5.f},      // two blocks a CU
-                                 {128, 128, 256, 0.55f, 6.f}, {64, 128, 256, 0.40f, 5.f}, {64, 64, 256, 0.26f, 3.f},      // two wave groups
-                                 {32, 64, 256, 0.16f, 3.5f}, {32, 32, 256, 0.12f, 3.5f},                                  // four
-                                 {192, 256, 256, 1.09f, 9.5f}, {128, 256, 256, 0.82f, 8.f}};
-// fp32 rows, bf16 weights (16384 rows x 32 blocks of 256 x 256: 128 x 128 432 us, 458 at 64 x 128, 615 before; 400 x 2048 x 2048:
-// 64 x 64 16 us, 128 x 128 39)
-static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f}, {64, 128, 256, 0.47f, 5.f}, {64, 64, 256, 0.37f, 4.2f},
-                                       {64, 64, 512, 0.6f, 4.f},    // two blocks a CU
-                                       {32, 32, 256, 0.16f, 3.5f}};
-// fp32 (bound by the fp32 MFMA's 150 TFLOP/s; 400 x 2048 x 8192: 64 x 64 165 us, 128 x 128 573; 3000 x 2048 x 2048: 64 x 128 224 us,
-// 128 x 128 269)
-static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f}, {128, 128, 256, 2.15f, 6.f}, {64, 128, 256, 1.1f, 6.f},
-                                     {64, 64, 256, 0.63f, 4.f}, {32, 64, 256, 0.33f, 4.f}, {32, 32, 256, 0.195f, 4.f}};
+// a start and a store.  A launch that leaves CUs idle in its last (or only) round wants smaller tiles, a long one the large tile; the
+// cheapest sum wins.  us per K tile and per round for products of few K tiles, measured on full rounds at K = 128 .. 8192, and for those of
+// at least LONG (least squares of the relative error over 400, 120 and 100 random products of 64 .. 20,000 rows with cold weights), where a round
+// that fills a part of the chip takes PART of a full one's time a K tile and more by its share (the clock rises).  The second kind of
+// product takes 1.014 of the best tile's time on average (1.026 by the first figures; fp32 rows on bf16 weights 1.017 and 1.057, fp32 1.008
+// and 1.012); below LONG they are no better than the first.  Row groups stay with the first: their sizes and the blocks' share of a cold W
+// decide, and of 400 random ones 31 were more than 4% slower by the second (and 1% faster on average).
+struct TileCost { int tm, tn, slots; float k_us, round_us, k_long, round_long; };
+static const int LONG = 18;
+static const float PART = 0.8f;
+// bf16 (16384 x 14336 x 4096: the 256 tile 1.49 ms, 128 x 128 2.05; 1024 x 2048 x 2048: 64 x 128 14 us, the 256 tile 42;
+// 256 x 2048 x 2048: 32 x 64 8 us, the 256 tile 41)
+static const TileCost TILES[] = {{256, 256, 256, 1.42f, 11.f, 1.263f, 11.816f},     // least LDS and L2 traffic per product: 1.24 - 1.45 PFLOP/s at 16384 rows
+                                 {128, 128, 512, 1.08f, 5.f, 0.818f, 5.367f},       // two blocks a CU
+                                 {128, 128, 256, 0.55f, 6.f, 0.552f, 5.788f}, {64, 128, 256, 0.40f, 5.f, 0.315f, 4.453f},      // two wave groups
+                                 {64, 64, 256, 0.26f, 3.f, 0.2f, 3.425f},
+                                 {32, 64, 256, 0.16f, 3.5f, 0.137f, 3.665f}, {32, 32, 256, 0.12f, 3.5f, 0.089f, 3.092f},       // four
+                                 {192, 256, 256, 1.09f, 9.5f, 0.945f, 9.866f}, {128, 256, 256, 0.82f, 8.f, 0.733f, 7.441f},
+                                 {64, 128, 512, 0.f, 0.f, 0.455f, 4.821f}};         // two blocks a CU, which stand at barriers of their own: 1024 x 4096 x 2048
+                                                                                    // 23.6 us, 24.6 on 128 x 128, 28.2 on two wave groups (long products only)
+// fp32 rows, bf16 weights (2048 x 2048 x 2048: 128 x 128 36 us, 64 x 128 38, 64 x 64 45)
+static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f, 0.945f, 5.724f}, {64, 128, 256, 0.47f, 5.f, 0.561f, 3.771f}, {64, 64, 256, 0.37f, 4.2f, 0.313f, 3.17f},
+                                       {64, 64, 512, 0.6f, 4.f, 0.476f, 3.454f},    // two blocks a CU
+                                       {32, 32, 256, 0.16f, 3.5f, 0.137f, 3.025f}};
+// fp32 (bound by the fp32 MFMA's 150 TFLOP/s; 400 x 2048 x 8192: 64 x 64 165 us, 128 x 128 573; 1000 x 2048 x 2048: 64 x 128 71 us,
+// 128 x 128 129)
+static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f, 3.7f, 8.f}, {128, 128, 256, 2.15f, 6.f, 1.934f, 6.092f}, {64, 128, 256, 1.1f, 6.f, 1.05f, 4.441f},
+                                     {64, 64, 256, 0.63f, 4.f, 0.573f, 3.127f}, {32, 64, 256, 0.33f, 4.f, 0.294f, 3.226f}, {32, 32, 256, 0.195f, 4.f, 0.166f, 2.685f}};
 
-static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int groups, bool by_rows, bool gated) {
-  int best = 0;
+static int pick_tile(const TileCost* tiles, int count, float part, int M, int N, int nk, int groups, bool by_rows, bool gated) {
+  int best = -1;
   float least = 0.f;
   for (int v = 0; v < count; ++v) {
     const TileCost& t = tiles[v];
-    if (gated && t.tn < 64) continue;      // (a wave of the 32-column tile has one half of a gated column only)
+    const bool lng = nk >= LONG && !by_rows;
+    if ((gated && t.tn < 64) || (t.k_us == 0.f && !lng)) continue;      // (a wave of the 32-column tile has one half of a gated column only)
+    const float k = (float)nk * (lng ? t.k_long : t.k_us), round = lng ? t.round_long : t.round_us;
     // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average, and how they fall on the
     // CUs is chance: a launch that just fills the chip takes a second round, 2048 rows of 8 experts on 192-row tiles 80 us, 62 on 256)
     const long long cols = (N + t.tn - 1) / t.tn;
-    float rounds;
+    float us;
     if (by_rows) {
       const float full = ((float)M / t.tm + 0.5f * groups) * cols / t.slots;
-      rounds = full <= 0.9f ? 1.f : full + 0.5f;
+      us = (full <= 0.9f ? 1.f : full + 0.5f) * (k + round);
     } else {
-      rounds = (float)(((long long)((M + t.tm - 1) / t.tm) * groups * cols + t.slots - 1) / t.slots);
+      const long long blocks = (long long)((M + t.tm - 1) / t.tm) * groups * cols, rest = blocks % t.slots;
+      us = (float)(blocks / t.slots) * (k + round);
+      if (rest) us += k * (lng ? part + (1.f - part) * (float)rest / t.slots : 1.f) + round;
     }
-    const float us = rounds * ((float)nk * t.k_us + t.round_us);
-    if (v == 0 || us < least) {
+    if (best < 0 || us < least) {
       least = us;
       best = v;
     }
@@ -644,8 +661,9 @@ static int pick_tile(const TileCost* tiles, int count, int M, int N, int nk, int
 
 // the index of the tile in its table
 static int choose(int ta, int tw, bool ragged, int M, int N, int nk, int groups, bool by_rows, bool gated) {
-  if (ta == 1) return ragged ? 1 + pick_tile(TILES + 1, 6, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 9, M, N, nk, groups, by_rows, gated);
-  return tw == 1 ? pick_tile(TILES_MIXED, 5, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 6, M, N, nk, groups, by_rows, gated);
+  if (ta == 1)
+    return ragged ? 1 + pick_tile(TILES + 1, 6, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 10, PART, M, N, nk, groups, by_rows, gated);
+  return tw == 1 ? pick_tile(TILES_MIXED, 5, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 6, 1.f, M, N, nk, groups, by_rows, gated);
 }
 
 extern "C" int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated) {
@@ -678,7 +696,8 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
       case 5: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
       case 6: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
       case 7: return start<gemm_tile_192>(192, 256, 256, t256::lds_bytes(3), t, s);
-      default: return start<gemm_tile_128>(128, 256, 256, t256::lds_bytes(2), t, s);
+      case 8: return start<gemm_tile_128>(128, 256, 256, t256::lds_bytes(2), t, s);
+      default: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 4, 3, 2, 1>>(64, 128, 256, 3 * 24576, t, s);
     }
   }
   if (tw == 1) {

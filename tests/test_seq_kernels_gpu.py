@@ -188,6 +188,19 @@ def test_every_tile(ops, types, tile, plain, grouped):
             close(H.gated_matmul_nt(few, w, out, offs=offs, rows=rows), silu(y(few[rows.long()])), tol)
 
 
+# 64 x 128 tiles, two blocks a CU: long plain and gated products, rows and columns past the last tile's end, an odd number of K tiles.
+# fp32 sums of up to 2,048 products of the same bf16 operands: 1e-5 as in test_matmul_tiles
+@pytest.mark.parametrize("M,N,K", [(1000, 4040, 1216), (1024, 4096, 2048), (511, 7688, 1152)])
+def test_two_blocks_a_unit(ops, M, N, K):
+    H, _ = ops
+    assert [H.k.fls_seq_gemm_tile_of(1, 1, M, N, K, 1, 0, g) for g in (0, 1)] == [9, 9]
+    torch.manual_seed(M + N + K)
+    a, w = torch.randn(M, K, device=DEV).bfloat16(), (0.1 * torch.randn(N, K, device=DEV)).bfloat16()
+    z = a.double() @ w.double().t()
+    close(H.matmul_nt(a, w), z, 1e-5)
+    close(H.gated_matmul_nt(a, w, torch.float32), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
+
+
 # few rows per group, one group of more than the 16 that a pass over its weights takes, empty groups, a K tail
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("K", [64, 200])
