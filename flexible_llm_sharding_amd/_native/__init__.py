@@ -43,6 +43,17 @@ def _fastcall():
     return mod
 
 
+_host = None
+
+
+def host():
+    """``fls_fastcall``'s functions for the host's own arrays (``int32s``, ``step_rows``)."""
+    global _host
+    if _host is None:
+        _host = _fastcall()
+    return _host
+
+
 class _Quick:
     """A library whose bound functions are called through ``fls_fastcall`` (csrc/python/fastcall.c) instead of ctypes, which
     remains for the arguments that one does not take."""

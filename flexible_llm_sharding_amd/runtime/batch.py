@@ -27,18 +27,58 @@ causal mask they cannot influence it.
 """
 from __future__ import annotations
 
+import bisect
 import dataclasses
+import itertools
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence
 
 import numpy as np
 import torch
 
+from .. import _native
 from ..utils.tokenizer import TokenizedPrompt
 
 Q_BLOCK = 64            # query rows per attention work item (kernel tile)
 Q_BLOCK_MHA = 128       # multi-head models: 4 waves of one query head share each staged K/V tile
 WORK_ITEM_FIELDS = 8    # q_start q_len q_off r0_start r0_len r0_causal r1_start r1_len
+
+
+def _token_ids(parts: Sequence[Sequence[int]]) -> np.ndarray:
+    """The parts' token ids one after the other, int32."""
+    lens = [len(p) for p in parts]
+    out, at, int32s = np.empty(sum(lens), dtype=np.int32), 0, _native.host().int32s
+    for p, n in zip(parts, lens):
+        part = out[at:at + n]
+        if not int32s(part, p):
+            part[...] = np.asarray(p, dtype=np.int32)
+        at += n
+    return out
+
+
+def _table(rows: Sequence[Sequence[int]], width: int) -> np.ndarray:
+    """Rows of ``width`` numbers as an int32 array (numpy takes 0.1 us a number to find out what a list of tuples holds)."""
+    return _token_ids([list(itertools.chain.from_iterable(rows))]).reshape(-1, width)
+
+
+def _upload(arrays: dict, device) -> dict:
+    """int32 arrays on ``device``.  A GPU gets them by one copy from pinned memory, in stream order, as views of one buffer, each from a
+    64-byte boundary on (seven copies of a scoring call from pageable memory kept the host 54 us, one from there 81 to 145)."""
+    d = torch.device(device)
+    arrays = {k: np.ascontiguousarray(v, dtype=np.int32) for k, v in arrays.items()}
+    if d.type == "cpu":
+        return {k: torch.from_numpy(v).clone() for k, v in arrays.items()}
+    offs = [0]
+    for a in arrays.values():
+        offs.append(offs[-1] + -(-a.size // 16) * 16)
+    up = torch.empty(offs[-1] + 16, dtype=torch.int32, pin_memory=True)
+    flat = up.numpy()
+    flat[...] = 0
+    for a, o in zip(arrays.values(), offs):
+        flat[o:o + a.size] = a.reshape(-1)
+    dev = torch.empty_like(up, device=d, pin_memory=False)
+    dev.copy_(up, non_blocking=True)                        # (torch keeps the pinned memory until the copy has run)
+    return {k: dev[o:o + a.size].view(a.shape) for (k, a), o in zip(arrays.items(), offs)}
 
 
 @dataclass
@@ -194,10 +234,7 @@ class PackedBatch:
         """int32 metadata on ``device`` (cached; uploaded once, reused by all layers)."""
         key = str(device)
         if key not in self._dev:
-            d = torch.device(device)
-            nb = d.type != "cpu"
-            self._dev[key] = {k: torch.from_numpy(np.ascontiguousarray(v)).to(d, non_blocking=nb)
-                              for k, v in self.host_meta().items()}
+            self._dev[key] = _upload(self.host_meta(), device)
         return self._dev[key]
 
 
@@ -230,9 +267,16 @@ def pack_prompts(tps: Sequence[TokenizedPrompt], prompt_ids: Sequence[int],
     if kv_cached and prefix_offsets is None:
         raise ValueError("kv_cached needs prefix_offsets")
     pcausal = 1 if prefix_attention == "causal" else 0
-    # per-row arrays are gathered as numpy parts (one per prefix / suffix) and concatenated once:
+    # per-row arrays are made at the end from each prefix's and suffix's tokens, row count, first position and first row:
     # Python lists of 43k ints cost the host ~10 ms per call (the GPU idles at the call boundary)
-    ids, pos, seg_lo, segs, last, nsuf, lsegs = [], [], [], [], [], [], []
+    parts, lens, pos0, lo0, segs, last, nsuf, lsegs = [], [], [], [], [], [], [], []
+
+    def add_rows(tokens, n, first_pos, first_row):
+        parts.append(tokens)
+        lens.append(n)
+        pos0.append(first_pos)
+        lo0.append(first_row)
+
     if suffix_keep is not None and not kv_cached:
         raise ValueError("suffix K/V reuse needs the prefix K/V cache (kv_cached)")
     if suffix_keep is not None and any(r < 0 for rows in suffix_rows for r in rows):
@@ -250,10 +294,8 @@ def pack_prompts(tps: Sequence[TokenizedPrompt], prompt_ids: Sequence[int],
             p0 = prefix_offsets[j]
         else:
             p0 = t
-            ids.append(np.asarray(tp.prefix, dtype=np.int32))
-            pos.append(np.arange(Lp, dtype=np.int32))
+            add_rows(tp.prefix, Lp, 0, p0)
             segs.append(Segment(p0, Lp, p0, Lp, pcausal, 0, 0))
-            seg_lo.append(np.full(Lp, p0, dtype=np.int32))
             work.extend(_items(segs[-1], q_block))
             work2.extend([(0, 0)] * (len(work) - len(work2)))
             if prefix_offsets is not None:
@@ -261,17 +303,15 @@ def pack_prompts(tps: Sequence[TokenizedPrompt], prompt_ids: Sequence[int],
                 dst.append(np.arange(prefix_offsets[j], prefix_offsets[j] + Lp, dtype=np.int32))
             t += Lp
         sfx0 = t
-        sfx_lo = []                    # seg_lo of this prompt's suffix rows (row - sfx0)
+        sfx_starts = []                # first rows of this prompt's suffixes
         keep = suffix_keep[j] if suffix_keep is not None else None
         for si, s in enumerate(tp.suffixes):
             c = keep[si] if keep is not None else 0
             c0_row = suffix_rows[j][si] if suffix_rows is not None else -1
             n = len(s) - c
             s0 = t
-            ids.append(np.asarray(s[c:], dtype=np.int32))
-            pos.append(np.arange(Lp + c, Lp + c + n, dtype=np.int32))
-            seg_lo.append(np.full(n, s0, dtype=np.int32))
-            sfx_lo.extend([s0] * n)
+            add_rows(s[c:] if c else s, n, Lp + c, s0)
+            sfx_starts.append(s0)
             r2s, r2l = (c0_row, c) if c else (0, 0)
             segs.append(Segment(s0, n, p0, Lp, 0, s0, n, r2_start=r2s, r2_len=r2l))
             last.append(s0 + n - 1)
@@ -305,7 +345,7 @@ def pack_prompts(tps: Sequence[TokenizedPrompt], prompt_ids: Sequence[int],
                 work.append((c0, c1 - c0, 0, p0, Lp, 0, 0, 0))
                 work2.append((lo, hi - lo))
             else:
-                r1 = sfx_lo[c0 - sfx0]
+                r1 = sfx_starts[bisect.bisect_right(sfx_starts, c0) - 1]        # (the suffix that holds row c0)
                 work.append((c0, c1 - c0, c0 - r1, p0, Lp, 0, r1, c1 - r1))
                 work2.append((0, 0))
         max_pos = max(max_pos, Lp + max([len(s) for s in tp.suffixes] or [0]))
@@ -314,27 +354,28 @@ def pack_prompts(tps: Sequence[TokenizedPrompt], prompt_ids: Sequence[int],
         p_scored.append((sc0, len(last)))
         nsuf.append(tp.n_suffix)
         padded += tp.padded_tokens
-    work = np.asarray(work, dtype=np.int32).reshape(-1, WORK_ITEM_FIELDS)
+    work = _table(work, WORK_ITEM_FIELDS)
     reuse = suffix_keep is not None
+    lens = np.asarray(lens, dtype=np.int64)
+    per_row = lambda v: np.repeat(np.asarray(v, dtype=np.int32), lens)
 
     def cat(parts):
         return np.concatenate(parts) if parts else np.zeros(0, dtype=np.int32)
     return PackedBatch(
         prompt_ids=list(prompt_ids), n_suffix=nsuf,
-        ids=cat(ids), positions=cat(pos),
-        segments=segs, work=work, seg_lo=cat(seg_lo),
+        ids=_token_ids(parts), positions=np.arange(t, dtype=np.int32) + per_row(np.asarray(pos0, dtype=np.int64) - (np.cumsum(lens) - lens)),
+        segments=segs, work=work, seg_lo=per_row(lo0),
         last_idx=np.asarray(last, dtype=np.int32), last_segments=lsegs,
-        work_last=(np.asarray(lwork, dtype=np.int32).reshape(-1, WORK_ITEM_FIELDS) if reuse
-                   else _work_items(lsegs)), num_tokens=t, padded_tokens=padded,
+        work_last=_table(lwork, WORK_ITEM_FIELDS) if reuse else _work_items(lsegs), num_tokens=t, padded_tokens=padded,
         max_pos=max_pos, kv_cached=kv_cached, q_block=q_block,
         pfx_src=cat(src) if (prefix_offsets is not None and not kv_cached) else None,
         pfx_dst=cat(dst) if (prefix_offsets is not None and not kv_cached) else None,
         prompt_rows=np.asarray(p_rows, dtype=np.int64).reshape(-1, 2),
         prompt_items=np.asarray(p_items, dtype=np.int64).reshape(-1, 2),
         prompt_scored=np.asarray(p_scored, dtype=np.int64).reshape(-1, 2),
-        work2=np.asarray(work2, dtype=np.int32).reshape(-1, 2) if reuse else None,
-        r2win=np.asarray(r2win, dtype=np.int32).reshape(-1, 2) if reuse else None,
-        work2_last=np.asarray(lwork2, dtype=np.int32).reshape(-1, 2) if reuse else None,
+        work2=_table(work2, 2) if reuse else None,
+        r2win=_table(r2win, 2) if reuse else None,
+        work2_last=_table(lwork2, 2) if reuse else None,
         sfx_src=cat(sfx_src) if sfx_src else None,
         sfx_dst=cat(sfx_dst) if sfx_dst else None)
 
@@ -349,7 +390,7 @@ def _items(sg: Segment, q_block: int = Q_BLOCK) -> List[tuple]:
 def _work_items(segs: Sequence[Segment], q_block: int = Q_BLOCK) -> np.ndarray:
     """Segments -> [n_items, 8] int32 work items of at most ``q_block`` queries (one segment each)."""
     work = [it for sg in segs for it in _items(sg, q_block)]
-    return np.asarray(work, dtype=np.int32).reshape(-1, WORK_ITEM_FIELDS)
+    return _table(work, WORK_ITEM_FIELDS)
 
 
 def visible_keys(work: np.ndarray, seg_lo: Optional[np.ndarray], row: int,
@@ -477,8 +518,6 @@ class StepBatch:
     def device_tensors(self, device) -> dict:
         key = str(device)
         if key not in self._dev:
-            # one host-to-device copy for all the index arrays: each becomes a view of one int32 buffer
-            # (segments padded to 16 entries, so every view starts 64-byte aligned)
             names = ["ids", "tok_seq", "tok_pos", "cu", "pos0", "slot", "page_table", "kv_slot", "want_idx"]
             if self.prev_ids is not None:
                 names.append("prev_ids")
@@ -486,16 +525,9 @@ class StepBatch:
                 names += ["q_tiles", "tile_cu"]
             if self.local_table is not None:
                 names.append("local_table")
-            arrs = [np.ascontiguousarray(getattr(self, k), dtype=np.int32) for k in names]
-            for P, t in self.block_tables.items():
-                names.append(f"block_table_{P}")
-                arrs.append(np.ascontiguousarray(t, dtype=np.int32))
-            offs = np.cumsum([0] + [-(-a.size // 16) * 16 for a in arrs])
-            flat = np.zeros(int(offs[-1]) + 16, dtype=np.int32)
-            for a, o in zip(arrs, offs[:-1]):
-                flat[o:o + a.size] = a.reshape(-1)
-            dev_flat = torch.from_numpy(flat).to(device)
-            m = {k: dev_flat[o:o + a.size].view(a.shape) for k, a, o in zip(names, arrs, offs[:-1])}
+            arrays = {k: getattr(self, k) for k in names}
+            arrays.update((f"block_table_{P}", t) for P, t in self.block_tables.items())
+            m = _upload(arrays, device)
             m.update(n_seqs=len(self.rids), max_rows=self.max_rows, rows_host=np.diff(self.cu),
                      pos0_host=self.pos0, cu_host=self.cu)
             self._dev[key] = m
@@ -507,8 +539,8 @@ def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
     runtime.seq_state.SequenceStateCache): pages for the new tokens, a state slot for a new request."""
     if entries and all(len(e.tokens) == 1 for e in entries):
         return _pack_tokens(entries, cache)
-    ids, want, wc, cu, pos0, slot, prev = [], [], [], [0], [], [], []
-    ps = cache.page_size
+    ids = _token_ids([e.tokens for e in entries])
+    want, wc, cu, pos0, slot, before = [], [], [0], [], [], []
     for e in entries:
         n = len(e.tokens)
         if n == 0:
@@ -516,9 +548,8 @@ def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
         p0, s = cache.extend(e.rid, n)
         pos0.append(p0)
         slot.append(s)
-        ids.append(np.asarray(e.tokens, dtype=np.int32))
         if cache.prev_token:
-            prev += [np.asarray([cache.advance_token(e.rid, e.tokens[-1])], dtype=np.int32), ids[-1][:-1]]
+            before.append(cache.advance_token(e.rid, e.tokens[-1]))
         w = np.asarray(list(e.want), dtype=np.int64)
         if w.size and (w.min() < 0 or w.max() >= n):
             raise ValueError(f"request {e.rid!r}: a wanted place lies outside its {n} tokens")
@@ -527,25 +558,27 @@ def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
         cu.append(cu[-1] + n)
     rids = [e.rid for e in entries]
     table = cache.page_table(rids)
-    lens = np.diff(np.asarray(cu, dtype=np.int64))
-    seq_a = np.repeat(np.arange(len(entries), dtype=np.int64), lens)
-    pos_a = np.arange(cu[-1], dtype=np.int64) - np.repeat(np.asarray(cu[:-1], dtype=np.int64) - np.asarray(pos0, dtype=np.int64), lens)
-    ids, want, seq, pos = np.concatenate(ids), np.concatenate(want), seq_a, pos_a
-    pages = table[seq_a, pos_a // ps]
-    if (pages < 0).any():
-        raise RuntimeError("a new token's page is missing from the page table")
+    T = cu[-1]
     i32 = lambda a: np.asarray(a, dtype=np.int32)
+    cu_a, pos0_a = i32(cu), i32(pos0)
+    seq, pos, kv_slot = (np.empty(T, dtype=np.int32) for _ in range(3))
+    if not _native.host().step_rows(cu_a, pos0_a, table, cache.page_size, seq, pos, kv_slot):
+        raise RuntimeError("a new token's page is missing from the page table")
+    prev = None
+    if before:                                              # (each row's token before it: the row above, a request's first row its last one)
+        prev = np.empty(T, dtype=np.int32)
+        prev[1:] = ids[:-1]
+        prev[cu_a[:-1]] = before
     max_rows = max(len(e.tokens) for e in entries)
     q_tiles = tile_cu = local = None
     if max_rows >= Q_TILE_MIN_ROWS and not any(pos0):
-        local = i32(np.asarray(cu[:-1], dtype=np.int64)[:, None] + np.arange(max_rows, dtype=np.int64)[None, :])
+        local = cu_a[:-1, None] + np.arange(max_rows, dtype=np.int32)[None, :]
     if max_rows >= Q_TILE_MIN_ROWS:
-        q_tiles = i32([(a + o, min(Q_TILE_ROWS, b - a - o)) for a, b in zip(cu[:-1], cu[1:])
-                       for o in range(0, b - a, Q_TILE_ROWS)])
+        q_tiles = _table([(a + o, min(Q_TILE_ROWS, b - a - o)) for a, b in zip(cu[:-1], cu[1:])
+                          for o in range(0, b - a, Q_TILE_ROWS)], 2)
         tile_cu = i32(np.concatenate([[0], np.cumsum([-(-(b - a) // Q_TILE_ROWS) for a, b in zip(cu[:-1], cu[1:])])]))
-    return StepBatch(rids, i32(ids), i32(seq), i32(pos), i32(cu), i32(pos0), i32(slot), table,
-                     i32(pages.astype(np.int64) * ps + pos_a % ps), i32(want), wc, len(ids), max_rows, q_tiles, tile_cu, local,
-                     {P: cache.block_table(rids, P) for P in cache.block_sizes}, np.concatenate(prev) if prev else None)
+    return StepBatch(rids, ids, seq, pos, cu_a, pos0_a, i32(slot), table, kv_slot, i32(np.concatenate(want)), wc, T, max_rows, q_tiles, tile_cu,
+                     local, {P: cache.block_table(rids, P) for P in cache.block_sizes}, prev)
 
 
 def _pack_tokens(entries: Sequence[StepEntry], cache) -> StepBatch:

@@ -5,6 +5,7 @@ import random
 import shutil
 import subprocess
 
+import numpy as np
 import pytest
 
 from flexible_llm_sharding_amd import _native
@@ -68,3 +69,41 @@ def test_a_library_of_other_signatures_is_refused(tmp_path):
     subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", str(tmp_path / "old.so")], check=True)
     with pytest.raises(RuntimeError, match="stale build"):
         _native._load_kernels(str(tmp_path / "old.so"))
+
+
+def test_token_lists_to_int32():
+    int32s, rng = _native.host().int32s, random.Random(1)
+    for n in (0, 1, 7, 1000):
+        v = [rng.randint(-2 ** 31, 2 ** 31 - 1) for _ in range(n)]
+        for seq in (v, tuple(v)):
+            out = np.full(n + 2, 5, np.int32)
+            assert int32s(out[1:n + 1], seq) is True
+            assert out.tolist() == [5] + v + [5]
+    out = np.zeros(2, np.int32)
+    for seq in ([1, 2 ** 31], [1, -2 ** 31 - 1], [1, 2.0], [1, True], [1, np.int32(2)], [1], [1, 2, 3], np.array([1, 2]), range(2), "12", [1, 10 ** 30]):
+        assert int32s(out, seq) is False                             # (left to numpy, which takes or refuses them)
+    with pytest.raises((ValueError, BufferError)):
+        int32s(np.zeros(4, np.int32)[::2], [1, 2])
+
+
+@pytest.mark.parametrize("lens,pos0,ps", [([1], [0], 16), ([3, 40, 1], [0, 7, 100], 16), ([64, 64], [0, 64], 64), ([500, 33, 2], [1, 0, 30], 7)])
+def test_step_rows(lens, pos0, ps):
+    B, cu = len(lens), np.cumsum([0] + lens).astype(np.int32)
+    T, p0 = int(cu[-1]), np.asarray(pos0, np.int32)
+    P = max((a + n - 1) // ps for a, n in zip(pos0, lens)) + 1
+    table = np.random.default_rng(0).permutation(4 * B * P)[:B * P].reshape(B, P).astype(np.int32)
+    seq, pos, slot = (np.zeros(T, np.int32) for _ in range(3))
+    rows = _native.host().step_rows
+    assert rows(cu, p0, table, ps, seq, pos, slot) is True
+    b = np.repeat(np.arange(B), lens)
+    at = np.arange(T) - cu[b] + p0[b]
+    assert (seq == b).all() and (pos == at).all() and (slot == table[b, at // ps] * ps + at % ps).all()
+    for hole in ((0, 0 if pos0[0] < ps else pos0[0] // ps), (B - 1, (pos0[-1] + lens[-1] - 1) // ps)):
+        bad = table.copy()
+        bad[hole] = -1
+        assert rows(cu, p0, bad, ps, seq, pos, slot) is False
+    assert rows(cu, p0 + P * ps, table, ps, seq, pos, slot) is False     # (past the table)
+    for args in ((cu[:-1], p0, table, ps, seq, pos, slot), (cu, p0, table, 0, seq, pos, slot), (cu, p0, table, ps, seq[1:], pos, slot),
+                 (cu, p0, table, ps, seq, pos, slot.astype(np.int64)), (cu[::-1].copy(), p0, table, ps, seq, pos, slot), (cu, p0 - 200, table, ps, seq, pos, slot)):
+        with pytest.raises(ValueError):
+            rows(*args)
