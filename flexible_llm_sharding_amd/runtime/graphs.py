@@ -27,6 +27,8 @@ intermediates are shared between them.
 """
 from __future__ import annotations
 
+import contextlib
+import gc
 import weakref
 from collections import OrderedDict
 from typing import Callable, Dict, List, Optional, Tuple
@@ -90,6 +92,20 @@ class _Arrays:
         return out
 
 
+@contextlib.contextmanager
+def _capturing(graph: torch.cuda.CUDAGraph, pool, stream):
+    """Capture into ``graph`` without Python's automatic collections: one could free what a runner left in a cycle (pinned memory, events, graphs),
+    which is an error while a stream captures."""
+    collects = gc.isenabled()
+    gc.disable()
+    try:
+        with torch.cuda.graph(graph, pool=pool, stream=stream):
+            yield
+    finally:
+        if collects:
+            gc.enable()
+
+
 class _Graph:
     def __init__(self, meta: Dict[str, torch.Tensor]):
         self.meta = meta                     # static device inputs
@@ -130,7 +146,7 @@ class GraphedForward:
             self.forward(meta, batch)                       # warm-up (lazy inits, autotune)
         torch.cuda.current_stream(self.dev).wait_stream(s)
         torch.cuda.synchronize(self.dev)
-        with torch.cuda.graph(g.graph, pool=self.pool, stream=s):
+        with _capturing(g.graph, self.pool, s):
             g.out = self.forward(meta, batch)
         torch.cuda.synchronize(self.dev)
         self.captures += 1
@@ -247,7 +263,7 @@ class DecodeGraphs:
                 eager = self.forward(meta, batch)            # this step's result (+ lazy inits)
             torch.cuda.current_stream(self.dev).wait_stream(s)
             torch.cuda.synchronize(self.dev)
-            with torch.cuda.graph(g.graph, pool=self.pool, stream=s):
+            with _capturing(g.graph, self.pool, s):
                 g.out = self.forward(meta, batch)            # captured, not run: the eager pass computed
             torch.cuda.synchronize(self.dev)                 # this step (its cache writes are idempotent)
             self.captures += 1
@@ -388,7 +404,7 @@ class StepGraphs:
             s = torch.cuda.Stream(self.dev)
             s.wait_stream(torch.cuda.current_stream(self.dev))
             torch.cuda.synchronize(self.dev)
-            with torch.cuda.graph(g.graph, pool=self.pool, stream=s):
+            with _capturing(g.graph, self.pool, s):
                 g.out = self._step(inputs)
             torch.cuda.synchronize(self.dev)
             self.graphs[key] = g

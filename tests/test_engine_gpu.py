@@ -443,6 +443,36 @@ def test_decode_graphs_match_eager(setup, weights):
             assert np.array_equal(a, b)
 
 
+def test_capture_beside_garbage(setup):
+    """Captures while dead cycles hold pinned memory and Python would collect them at any allocation: the steps run, bitwise as without."""
+    import gc
+    from flexible_llm_sharding_amd.runtime.hostmem import alloc_host
+    path, cfg, tok, prompts, ref = setup
+    src = HostStore.from_model_path(cfg, path)
+    outs, limits = [], gc.get_threshold()
+    for often in (False, True):
+        r = ShardedRunner(cfg, src, "cuda:0", tok, layer_num_per_shard=1, prefix_kv_cache=True, suffix_kv_cache=True, resident=True)
+        word = prompts[0][0].split()[0]
+        outs.append([r(prompts)])
+        for step in (1, 2, 3):
+            class Dead:
+                pass
+            for _ in range(20):
+                d = Dead()
+                d.me, d.memory = d, alloc_host(1 << 16)
+            del d
+            try:
+                if often:
+                    gc.set_threshold(60, 1, 1)
+                outs[-1].append(r([(pre, tuple(sf + (" " + word) * step for sf in sufs)) for pre, sufs in prompts]))
+            finally:
+                gc.set_threshold(*limits)
+        assert r.stats["graph_captures"] >= 1 and gc.isenabled()
+        r.close()
+    for a, b in zip(*outs):
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
 def test_decode_graphs_survive_entry_eviction(setup):
     """A decode graph bakes in its cache entry's K/V addresses.  With one prefix-cache entry, a
     second prompt set of the same shapes evicts the first entry (its K/V freed; a new entry may get
