@@ -29,7 +29,6 @@ from __future__ import annotations
 
 import contextlib
 import gc
-import weakref
 from collections import OrderedDict
 from typing import Callable, Dict, List, Optional, Tuple
 
@@ -112,7 +111,7 @@ class _Graph:
         self.graph = torch.cuda.CUDAGraph()
         self.out: torch.Tensor = None        # static device output [S, V]
         self.replays = 0
-        self.entry_ref = None                # DecodeGraphs: the cache entry whose K/V the graph baked in
+        self.kv: frozenset = frozenset()     # DecodeGraphs: the addresses of the K/V buffers that the graph reads and writes
         self.arrays: Optional[_Arrays] = None      # DecodeGraphs: ``meta``'s places in ``flat``
         self.flat: Optional[torch.Tensor] = None
         self.staging: List[Tuple[Dict[str, np.ndarray], torch.Tensor, Optional[torch.cuda.Event]]] = []
@@ -179,9 +178,10 @@ class DecodeGraphs:
     each; one graph replays them all.
 
     Unlike :class:`GraphedForward` the shapes are EXACT (no bucket padding: a padded row would
-    also be captured into the suffix K/V cache), keyed by the batch's array shapes and the cache
-    entry, whose per-layer K/V buffers the graph reads and writes in place; consecutive steps of
-    one generation have the same shapes, so one capture serves them all.  The metadata of each
+    also be captured into the suffix K/V cache), keyed by the batch's array shapes and the addresses of the cache
+    entry's per-layer K/V buffers, which the graph reads and writes in place; consecutive steps of
+    one generation have the same shapes, so one capture serves them all, and the steps of a later entry in the same buffers
+    (``PrefixKVCache.begin``): nothing else of an entry is in a graph, its rows come with each step's metadata.  The metadata of each
     step (new token ids, positions, work items, cache rows and windows) is copied into the
     graph's static inputs before the replay."""
 
@@ -196,17 +196,16 @@ class DecodeGraphs:
 
     @staticmethod
     def key(batch: PackedBatch, entry) -> tuple:
-        """The entry's identity is its fingerprint plus the device address of every per-layer K/V
-        buffer the graph reads and writes (an evicted entry's id() and even its addresses can be
-        reused by a new one: ``run`` also checks the graph's weak reference to the entry)."""
+        """The device address of every per-layer K/V buffer that the graph reads and writes, and the step's shapes."""
         ptrs = tuple((n, t.data_ptr()) for n, t in sorted(entry.layers.items()))
-        return (entry.key, ptrs, batch.r2_q_block, batch.q_block) + tuple(
+        return (ptrs, batch.r2_q_block, batch.q_block) + tuple(
             (k, v.shape) for k, v in sorted(batch.host_meta().items()))
 
     def forget(self, entry) -> None:
-        """Drop every graph captured on ``entry`` (called when the prefix cache evicts or drops it:
-        its K/V buffers are about to be freed, and a replay would read / write freed HBM)."""
-        for k in [k for k, g in self.graphs.items() if g.entry_ref is None or g.entry_ref() in (None, entry)]:
+        """Drop every graph captured on ``entry``'s buffers (called when the prefix cache frees them: a replay would read / write
+        freed HBM)."""
+        freed = {t.data_ptr() for held in (entry.memory, entry.spare) for t in held.values()}
+        for k in [k for k, g in self.graphs.items() if g.kv & freed]:
             del self.graphs[k]
 
     # pinned staging sets per graph: a replay may be enqueued while the previous one (and its
@@ -240,9 +239,6 @@ class DecodeGraphs:
         key = self.key(batch, entry)
         host = batch.host_meta()
         g = self.graphs.get(key)
-        if g is not None and (g.entry_ref is None or g.entry_ref() is not entry):
-            del self.graphs[key]                             # captured on another (dead) entry
-            g = None
         if g is None:
             if len(self.graphs) >= self.max_graphs:
                 self.graphs.popitem(last=False)
@@ -256,7 +252,7 @@ class DecodeGraphs:
                 meta["ids"].copy_(ids_dev)
             g = _Graph(meta)
             g.arrays, g.flat = arrays, flat
-            g.entry_ref = weakref.ref(entry)
+            g.kv = frozenset(p for _, p in key[0])
             s = torch.cuda.Stream(self.dev)
             s.wait_stream(torch.cuda.current_stream(self.dev))
             with torch.cuda.stream(s):

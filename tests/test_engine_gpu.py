@@ -473,6 +473,34 @@ def test_capture_beside_garbage(setup):
         assert all(np.array_equal(x, y) for x, y in zip(a, b))
 
 
+def test_decode_graphs_serve_the_next_entry(setup):
+    """With one prefix-cache entry, a second prompt set of other lengths but the same step shapes takes over the first one's K/V buffers:
+    its decode steps replay the graph captured for the first, and every score == the eager runner's bitwise."""
+    path, cfg, tok, prompts, ref = setup
+    src = HostStore.from_model_path(cfg, path)
+    words = prompts[0][0].split()
+    other = [(" ".join(pre.split()[3:]), sufs) for pre, sufs in prompts]
+    outs, captures = {}, []
+    for graphs in ("1", "0"):
+        os.environ["FLS_DECODE_GRAPHS"] = graphs
+        try:
+            r = ShardedRunner(cfg, src, "cuda:0", tok, layer_num_per_shard=1, prefix_kv_cache=True, suffix_kv_cache=True, resident=True,
+                              prefix_cache_entries=1)
+            steps = []
+            for base in (prompts, other, prompts):
+                for step in range(4):
+                    steps.append(r([(pre, tuple(sf + (" " + " ".join(words[:step]) if step else "") for sf in sufs)) for pre, sufs in base]))
+                captures.append(r.stats.get("graph_captures", 0))
+            outs[graphs] = steps
+            r.close()
+        finally:
+            os.environ.pop("FLS_DECODE_GRAPHS", None)
+    assert captures[0] >= 1 and captures[1] == captures[2] == captures[0]
+    for sg, se in zip(outs["1"], outs["0"]):
+        for a, b in zip(sg, se):
+            assert np.array_equal(a, b)
+
+
 def test_decode_graphs_survive_entry_eviction(setup):
     """A decode graph bakes in its cache entry's K/V addresses.  With one prefix-cache entry, a
     second prompt set of the same shapes evicts the first entry (its K/V freed; a new entry may get
