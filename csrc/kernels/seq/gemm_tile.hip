@@ -159,30 +159,26 @@ __device__ __forceinline__ void hold(floatx4& c) {
 // own piece of LDS (PU row groups at a time) and takes them up row by row, so that a store covers whole rows of the tile (straight from the
 // registers it was pieces of 32 or 64 bytes of 16 rows: 16384 x 4096 x 4096 404 -> 392 us, 9692 x 10880 x 2048 390 -> 340) and an
 // activation is a short loop: unrolled over all accumulators its code would be larger than the cache.
-template <int MI, int NJ, int PU, bool ACC>
-__device__ __forceinline__ void lay_down(floatx4 (&acc)[MI][NJ], int p, char* lds) {
+template <int NJ, bool ACC>
+__device__ __forceinline__ void lay_down(floatx4 (&row)[NJ], int u, char* lds) {
   constexpr int CH = 4 * NJ;
-  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4, r = u * 16 + fr;
 #pragma unroll
-  for (int u = 0; u < PU; ++u)
-#pragma unroll
-    for (int t = 0; t < NJ; ++t) {
-      const int r = u * 16 + fr;
-      hold<ACC>(acc[p * PU + u][t]);
-      *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = acc[p * PU + u][t];
-    }
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (the wave's own rows: no other wave reads them)
+  for (int t = 0; t < NJ; ++t) {
+    hold<ACC>(row[t]);
+    *reinterpret_cast<floatx4*>(lds + (r * CH + ((4 * t + grp) ^ (r & (CH - 1)))) * 16) = row[t];
+  }
 }
 
 // The rows that a wave laid down: a loop for each kind of epilogue.  With the kind asked for at each value the loop was a chain of
 // branches over the other kinds' code, and a wave that has its SIMD to itself waits for the instructions after each: 16384 x 14336 x
 // 4096 with xIELU 1827 us, 1523 so (branches in xIELU itself: 1572); 9692 x 10880 x 2048 silu gates 469 and 362.
-template <int NJ, int PU, int TC, int KIND>
-__device__ __forceinline__ void value_rows(const Tile& a, const EpiRegs (&er)[4], floatx4 b, size_t cbase, int m0, int n, int mend, const char* lds) {
+template <int NJ, int TC, int KIND>
+__device__ __forceinline__ void value_rows(const Tile& a, const EpiRegs (&er)[4], floatx4 b, size_t cbase, int m0, int rows, int n, int mend, const char* lds) {
   constexpr int CH = 4 * NJ, RI = 64 / CH;          // 16-byte chunks of a row; rows per step of the loop
   const int lane = threadIdx.x & 63, c = lane % CH;
 #pragma unroll 2
-  for (int i = 0; i < 16 * PU; i += RI) {
+  for (int i = 0; i < rows; i += RI) {
     const int r = i + lane / CH;
     floatx4 v = *reinterpret_cast<const floatx4*>(lds + (r * CH + (c ^ (r & (CH - 1)))) * 16) + b;
 #pragma unroll
@@ -190,13 +186,13 @@ __device__ __forceinline__ void value_rows(const Tile& a, const EpiRegs (&er)[4]
     if (m0 + r < mend && n < a.N) store4<TC>(a.C, cbase + (size_t)(m0 + r) * a.ldc + n, v);
   }
 }
-template <int NJ, int PU, int TC, int KIND>
-__device__ __forceinline__ void gate_rows(const Tile& a, int m0, int nw, int mend, const char* lds) {
+template <int NJ, int TC, int KIND>
+__device__ __forceinline__ void gate_rows(const Tile& a, int m0, int rows, int nw, int mend, const char* lds) {
   constexpr int CH = 4 * NJ, RI = 64 / CH;
   const int lane = threadIdx.x & 63, c = lane % (CH / 2), cg = (c >> 2) * 8 + (c & 3);      // column chunk, its gate chunk (the up chunk: + 4)
   const int n = (nw >> 1) + 4 * c;
 #pragma unroll 2
-  for (int i = 0; i < 16 * PU; i += 2 * RI) {
+  for (int i = 0; i < rows; i += 2 * RI) {
     const int r = i + lane / (CH / 2);
     const floatx4 g = *reinterpret_cast<const floatx4*>(lds + (r * CH + (cg ^ (r & (CH - 1)))) * 16);
     const floatx4 u = *reinterpret_cast<const floatx4*>(lds + (r * CH + ((cg + 4) ^ (r & (CH - 1)))) * 16);
@@ -207,90 +203,113 @@ __device__ __forceinline__ void gate_rows(const Tile& a, int m0, int nw, int men
   }
 }
 
-template <int MI, int NJ, int PU, bool ACC, int TC>
-__device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
-  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+// One pass: the wave's rows m0 .. m0 + rows - 1, which it has laid down.
+template <int NJ, int TC>
+__device__ __forceinline__ void rows_out(const Tile& a, const EpiRegs (&er)[4], floatx4 b, size_t cbase, int m0, int rows, int nw, int mend, const char* lds) {
   const Epi& e = a.epi;
-  if constexpr (!ACC) {
-    if (a.ragged) {                                         // (plain products of few columns: a column at a time)
-#pragma unroll
-      for (int t = 0; t < NJ; ++t)
-#pragma unroll
-        for (int u = 0; u < MI; ++u)
-#pragma unroll
-          for (int x = 0; x < 4; ++x) {
-            const int n = nw + t * 16 + 4 * grp + x, m = mw + u * 16 + fr;
-            const size_t at = cbase + (size_t)m * a.ldc + n;
-            if (n >= a.N || m >= mend) continue;
-            if constexpr (TC == 1) reinterpret_cast<bf16_t*>(a.C)[at] = f_to_bf16(acc[u][t][x]);
-            else reinterpret_cast<float*>(a.C)[at] = acc[u][t][x];
-          }
-      return;
-    }
-  }
-  constexpr int CH = 4 * NJ;                         // 16-byte chunks of a row
+  const int n = nw + 4 * ((int)(threadIdx.x & 63) % (4 * NJ));
   if (NJ >= 2 && e.kind >= EPI_GATE) {               // (no bias: the gated products have none)
-#pragma unroll
-    for (int p = 0; p < MI / PU; ++p) {
-      lay_down<MI, NJ, PU, ACC>(acc, p, lds);
-      const int m0 = mw + p * PU * 16;
-      if (e.kind == EPI_GATE) gate_rows<NJ, PU, TC, EPI_GATE>(a, m0, nw, mend, lds);
-      else if (e.kind == EPI_GATE + 1) gate_rows<NJ, PU, TC, EPI_GATE + 1>(a, m0, nw, mend, lds);
-      else gate_rows<NJ, PU, TC, EPI_GATE + 2>(a, m0, nw, mend, lds);
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
+    if (e.kind == EPI_GATE) gate_rows<NJ, TC, EPI_GATE>(a, m0, rows, nw, mend, lds);
+    else if (e.kind == EPI_GATE + 1) gate_rows<NJ, TC, EPI_GATE + 1>(a, m0, rows, nw, mend, lds);
+    else gate_rows<NJ, TC, EPI_GATE + 2>(a, m0, rows, nw, mend, lds);
     return;
   }
+  switch (e.kind) {
+    case EPI_XIELU: value_rows<NJ, TC, EPI_XIELU>(a, er, b, cbase, m0, rows, n, mend, lds); break;
+    case EPI_RELU2: value_rows<NJ, TC, EPI_RELU2>(a, er, b, cbase, m0, rows, n, mend, lds); break;
+    case EPI_DECAY: value_rows<NJ, TC, EPI_DECAY>(a, er, b, cbase, m0, rows, n, mend, lds); break;
+    case EPI_SOFTCAP: value_rows<NJ, TC, EPI_SOFTCAP>(a, er, b, cbase, m0, rows, n, mend, lds); break;
+    case EPI_SCALE: value_rows<NJ, TC, EPI_SCALE>(a, er, b, cbase, m0, rows, n, mend, lds); break;
+    default: value_rows<NJ, TC, 0>(a, er, b, cbase, m0, rows, n, mend, lds);
+  }
+}
+// What a wave's columns need besides (lane: four columns from n on).
+__device__ __forceinline__ floatx4 column_terms(const Tile& a, EpiRegs (&er)[4], size_t cbase, int n) {
+  const Epi& e = a.epi;
   const EpiRegs er0 = epi_regs(e);
-  const int n = nw + 4 * (lane % CH);
-  EpiRegs er[4] = {er0, er0, er0, er0};
   floatx4 b = {0.f, 0.f, 0.f, 0.f};
-  if (n < a.N) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) er[i] = er0;
+  if (e.kind < EPI_GATE && n < a.N) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) epi_column(e, er[i], n + i);
     if (e.bias != nullptr) b = *reinterpret_cast<const floatx4*>(e.bias + cbase + n);
   }
-#pragma unroll
-  for (int p = 0; p < MI / PU; ++p) {
-    lay_down<MI, NJ, PU, ACC>(acc, p, lds);
-    const int m0 = mw + p * PU * 16;
-    switch (e.kind) {
-      case EPI_XIELU: value_rows<NJ, PU, TC, EPI_XIELU>(a, er, b, cbase, m0, n, mend, lds); break;
-      case EPI_RELU2: value_rows<NJ, PU, TC, EPI_RELU2>(a, er, b, cbase, m0, n, mend, lds); break;
-      case EPI_DECAY: value_rows<NJ, PU, TC, EPI_DECAY>(a, er, b, cbase, m0, n, mend, lds); break;
-      case EPI_SOFTCAP: value_rows<NJ, PU, TC, EPI_SOFTCAP>(a, er, b, cbase, m0, n, mend, lds); break;
-      case EPI_SCALE: value_rows<NJ, PU, TC, EPI_SCALE>(a, er, b, cbase, m0, n, mend, lds); break;
-      default: value_rows<NJ, PU, TC, 0>(a, er, b, cbase, m0, n, mend, lds);
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  }
-}
-template <int MI, int NJ, int PU, bool ACC = false>
-__device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
-  if (a.epi.tc == 1) finish_as<MI, NJ, PU, ACC, 1>(a, acc, cbase, mw, nw, mend, lds);
-  else finish_as<MI, NJ, PU, ACC, 0>(a, acc, cbase, mw, nw, mend, lds);
+  return b;
 }
 
-// ------------------------------------------------------------------------------------ 256, 192 and 128 x 256
-// Four waves, one per SIMD, 32 HX x 128 outputs each.  HX = 4: 128 x 128, all 256 accumulation registers of a wave, a fragment
-// read from LDS feeds 8 MFMAs.  HX = 3, 2: 192 and 128 rows, for row counts that leave the chip idle in the last (or only) round of
-// 256-row tiles: 9692 x 2048 x 2048 107, 88, 95 us; x 5440 229, 186, 204; 5120 x 4096 x 4096 173, 143; 2048 x 4096 x 1024 35, 29, 24.
+template <int MI, int NJ, int TC>
+__device__ __forceinline__ void finish_as(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
+  const int lane = threadIdx.x & 63, fr = lane & 15, grp = lane >> 4;
+  if (a.ragged) {                                           // (plain products of few columns: a column at a time)
+#pragma unroll
+    for (int t = 0; t < NJ; ++t)
+#pragma unroll
+      for (int u = 0; u < MI; ++u)
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          const int n = nw + t * 16 + 4 * grp + x, m = mw + u * 16 + fr;
+          const size_t at = cbase + (size_t)m * a.ldc + n;
+          if (n >= a.N || m >= mend) continue;
+          if constexpr (TC == 1) reinterpret_cast<bf16_t*>(a.C)[at] = f_to_bf16(acc[u][t][x]);
+          else reinterpret_cast<float*>(a.C)[at] = acc[u][t][x];
+        }
+    return;
+  }
+  EpiRegs er[4];
+  const floatx4 b = column_terms(a, er, cbase, nw + 4 * (lane % (4 * NJ)));
+#pragma unroll
+  for (int u = 0; u < MI; ++u) lay_down<NJ, false>(acc[u], u, lds);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (the wave's own rows: no other wave reads them)
+  rows_out<NJ, TC>(a, er, b, cbase, mw, 16 * MI, nw, mend, lds);
+}
+template <int MI, int NJ>
+__device__ __forceinline__ void finish(const Tile& a, floatx4 (&acc)[MI][NJ], size_t cbase, int mw, int nw, int mend, char* lds) {
+  if (a.epi.tc == 1) finish_as<MI, NJ, 1>(a, acc, cbase, mw, nw, mend, lds);
+  else finish_as<MI, NJ, 0>(a, acc, cbase, mw, nw, mend, lds);
+}
+
+// The same for the large tiles' U x 8 accumulators, PU row groups a pass; those past the eighth group are in vector registers.
+template <int U, int PU, int TC, int P = 0>
+__device__ __forceinline__ void finish_big(const Tile& a, floatx4 (&acc)[U < 8 ? U : 8][8], floatx4 (&more)[U > 8 ? U - 8 : 1][8], const EpiRegs (&er)[4],
+                                           floatx4 b, size_t cbase, int mw, int nw, int mend, char* lds) {
+  constexpr int N = U - P < PU ? U - P : PU;
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    if (P + u < 8) lay_down<8, true>(acc[P + u < 8 ? P + u : 0], u, lds);
+    else lay_down<8, false>(more[P + u < 8 ? 0 : P + u - 8], u, lds);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  rows_out<8, TC>(a, er, b, cbase, mw + 16 * P, 16 * N, nw, mend, lds);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if constexpr (P + PU < U) finish_big<U, PU, TC, P + PU>(a, acc, more, er, b, cbase, mw, nw, mend, lds);
+}
+
+// ------------------------------------------------------------------------------------ 32 U x 256: 128, 160 .. 320 rows
+// Four waves, one per SIMD, 16 U x 128 outputs each.  U = 8: 128 x 128, all 256 accumulation registers of a wave, a fragment
+// read from LDS feeds 8 MFMAs; U = 9 and 10 hold their last row groups in vector registers and all of LDS.  Heights other than 256 are for row
+// counts that leave the chip idle in the last (or only) round of 256-row tiles: 8536 x 2048 x 2048 takes 272 tiles of 256 rows, 77 us, and 240
+// of 288 rows, 60 us (320: 65, 160: 72); x 5440 192 rows 178, 288 147; 6722 x 2048 x 2048 192 rows 54, 224 50 - 53.  Over 500 random long
+// products of up to 20,000 rows the four heights beside 128, 192 and 256 give 3% on average.
 // The products are written as in-place asm so that the accumulators stay where they are (with no spare accumulation register the
-// compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between them; reads run one phase of 8 HX
-// MFMAs ahead, DMAs three half-tiles, one barrier per two phases.
+// compiler would otherwise copy them) and so that LDS reads and DMAs keep their places between them; reads run one phase of 8 MFMAs
+// a row group ahead, DMAs three half-tiles, one barrier per two phases.
 namespace t256 {
 constexpr int TN = 256, KT = 128 /* bytes of a K tile's row */;
-constexpr int lds_bytes(int hx) { return 2 * (64 * hx + TN) * KT; }
+constexpr int lds_bytes(int u) { return 2 * (32 * u + TN) * KT; }
 }
 
+template <bool ACC>
 __device__ __forceinline__ void mfma_in_place(floatx4& c, const bf16x8& a, const bf16x8& b) {
-  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
+  if constexpr (ACC) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b) : "memory");
+  else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b) : "memory");
 }
 
-template <int HX>
+// U: 16-row groups of a wave; they are taken in two halves, the first of H0, the second of U - H0.
+template <int U>
 __device__ __forceinline__ void tile_256(const Tile& a) {
   using namespace t256;
-  constexpr int TM = 64 * HX, WIMG = TM * KT, STG = WIMG + TN * KT;
+  constexpr int H0 = (U + 1) / 2, H1 = U / 2, TM = 32 * U, WIMG = TM * KT, STG = WIMG + TN * KT;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const char *A, *W;
   size_t cbase;
@@ -298,11 +317,11 @@ __device__ __forceinline__ void tile_256(const Tile& a) {
   if (!locate<TM, TN>(a, A, W, cbase, m0, mend, n0)) return;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // DMA: a half-tile is 16 pieces (A: 4 HX) of eight rows, half of them for either half of the waves: piece j of W is rows
-  // (j >> 3) 128 + (j & 7) 8 (+ 64: the second half); a wave moves pieces 4 wave .. + 3 (A: HX wave .. + HX - 1)
+  // DMA: a half-tile is 16 pieces (A: 4 H0 or 4 H1) of eight rows, half of them for either half of the waves: piece j of W is rows
+  // (j >> 3) 128 + (j & 7) 8 (+ 64: the second half); a wave moves pieces 4 wave .. + 3 (A: H0 or H1)
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
-  int xpr[HX], wpr[4];
-  unsigned xo[2 * HX], wo[8];
+  int xpr[2][H0], wpr[4];
+  unsigned xo[2][H0], wo[8];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int j = 4 * wave + i;
@@ -311,56 +330,61 @@ __device__ __forceinline__ void tile_256(const Tile& a) {
     for (int h = 0; h < 2; ++h) wo[4 * h + i] = w_offset(a, n0, wpr[i] + 64 * h + lr) + lc * 16;
   }
 #pragma unroll
-  for (int i = 0; i < HX; ++i) {
-    const int j = HX * wave + i;
-    xpr[i] = j / (2 * HX) * (32 * HX) + j % (2 * HX) * 8;
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) xo[HX * h + i] = a_offset(a, m0, mend, xpr[i] + 16 * HX * h + lr) + lc * 16;
-  }
+    for (int i = 0; i < (h ? H1 : H0); ++i) {
+      const int n = h ? H1 : H0, j = n * wave + i;
+      xpr[h][i] = j / (2 * n) * (16 * U) + h * 16 * H0 + j % (2 * n) * 8;
+      xo[h][i] = a_offset(a, m0, mend, xpr[h][i] + lr) + lc * 16;
+    }
   const char* Ab = a_base(a, A, m0);
   const char* Wb = w_base(a, W, n0);
   // (past the last K tile the DMAs go through a descriptor of no records: counted like the others, they write zeros)
   const __amdgpu_buffer_rsrc_t rA = rsrc_of(Ab, true), rW = rsrc_of(Wb, true), r0 = rsrc_of(Ab, false);
 #define T_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, k0, 0, 0)
-#define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[(h) * HX + (i)], k0, smem + (buf) * STG + (xpr[i] + (h) * 16 * HX) * 128)
+#define T_X(rs, buf, h, i, k0) T_DMA(rs, xo[h][i], k0, smem + (buf) * STG + xpr[h][i] * 128)
 #define T_W(rs, buf, h, i, k0) T_DMA(rs, wo[(h) * 4 + (i)], k0, smem + (buf) * STG + WIMG + (wpr[i] + (h) * 64) * 128)
   const int wm = wave >> 1, wn = wave & 1;
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
   const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
-  const int xrow = (wm * 32 * HX + fr) * 128, wrow = WIMG + (wn * 128 + fr) * 128;
-  floatx4 acc[2 * HX][8];
+  const int xrow = (wm * 16 * U + fr) * 128, wrow = WIMG + (wn * 128 + fr) * 128;
+  floatx4 acc[U < 8 ? U : 8][8], more[U > 8 ? U - 8 : 1][8];
 #pragma unroll
-  for (int u = 0; u < 2 * HX; ++u)
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int t = 0; t < 8; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 xf[2 * HX][2], wf[8][2];
+    for (int t = 0; t < 8; ++t) (u < 8 ? acc[u < 8 ? u : 0] : more[u < 8 ? 0 : u - 8])[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 xf[U][2], wf[8][2];
 #define T_HOLD()                                                                                   \
-  _Pragma("unroll") for (int u_ = 0; u_ < 2 * HX; ++u_)                                            \
-  _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+a"(acc[u_][t_]));
+  _Pragma("unroll") for (int u_ = 0; u_ < (U < 8 ? U : 8); ++u_)                                   \
+  _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+a"(acc[u_][t_]));           \
+  _Pragma("unroll") for (int u_ = 8; u_ < U; ++u_)                                                 \
+  _Pragma("unroll") for (int t_ = 0; t_ < 8; ++t_) asm volatile("" : "+v"(more[u_ < 8 ? 0 : u_ - 8][t_]));
   T_HOLD();
   asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");          // (the zeros are written before the first MFMA reads them)
 #define T_RX(buf, f, k) xf[f][k] = *(const bf16x8*)(smem + (buf) * STG + xrow + (f) * 2048 + ((k) ? c1 : c0))
 #define T_RW(buf, f, k) wf[f][k] = *(const bf16x8*)(smem + (buf) * STG + wrow + (f) * 2048 + ((k) ? c1 : c0))
-// 8 HX MFMAs of the quadrant (x half xh, w half wh); after the first even ones the reads of the half needed next (RX: of x), 2 HX
-// or 8 of them, after later ones the DMAs of a half-tile (DX: of x), HX or 4
+// 8 MFMAs a row group of the quadrant (x half xh, w half wh); after the first even ones the reads of the half needed next (RX: of x), two a row
+// group or 8 of them, after later ones the DMAs of a half-tile (DX: of x)
 #define T_PHASE(xh, wh, RX, rbuf, rh, DX, rs, dbuf, dh, dk, SYNC)                                  \
   {                                                                                                \
-    _Pragma("unroll") for (int i_ = 0; i_ < 8 * HX; ++i_) {                                        \
-      const int s_ = i_ / (4 * HX), u_ = (xh) * HX + (i_ >> 2) % HX, t_ = (wh) * 4 + (i_ & 3);     \
-      mfma_in_place(acc[u_][t_], wf[t_][s_], xf[u_][s_]);                                          \
-      if (i_ < (RX ? 4 * HX : 16) && (i_ & 1) == 0) {                                              \
+    constexpr int HN_ = (xh) ? H1 : H0, RN_ = (rh) ? H1 : H0, DN_ = DX ? ((dh) ? H1 : H0) : 4;     \
+    constexpr int D0_ = HN_ == 5 ? 25 : HN_ == 4 ? 17 : HN_ == 3 ? 13 : 5;                         \
+    _Pragma("unroll") for (int i_ = 0; i_ < 8 * HN_; ++i_) {                                       \
+      const int s_ = i_ / (4 * HN_), u_ = (xh) * H0 + (i_ >> 2) % HN_, t_ = (wh) * 4 + (i_ & 3);   \
+      if (u_ < 8) mfma_in_place<true>(acc[u_ < 8 ? u_ : 0][t_], wf[t_][s_], xf[u_][s_]);           \
+      else mfma_in_place<false>(more[u_ < 8 ? 0 : u_ - 8][t_], wf[t_][s_], xf[u_][s_]);            \
+      if (i_ < (RX ? 4 * RN_ : 16) && (i_ & 1) == 0) {                                             \
         const int f_ = i_ >> 2, k_ = (i_ >> 1) & 1;                                                \
-        if (RX) T_RX(rbuf, (rh) * HX + f_, k_);                                                    \
+        if (RX) T_RX(rbuf, (rh) * H0 + f_, k_);                                                    \
         else T_RW(rbuf, (rh) * 4 + f_, k_);                                                        \
       }                                                                                            \
-      constexpr int D0_ = HX == 4 ? 17 : HX == 3 ? 13 : 5, DN_ = DX ? HX : 4;                      \
       if (i_ >= D0_ && i_ < D0_ + 3 * DN_ && (i_ - D0_) % 3 == 0) {                                \
         if (DX) T_X(rs, dbuf, dh, (i_ - D0_) / 3, dk);                                             \
         else T_W(rs, dbuf, dh, (i_ - D0_) / 3, dk);                                                \
       }                                                                                            \
     }                                                                                              \
     if (SYNC) {                                                                                    \
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * HX + 8) : "memory");                 \
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(U + 8) : "memory");                      \
       __builtin_amdgcn_s_barrier();                                                                \
     }                                                                                              \
   }
@@ -380,30 +404,30 @@ __device__ __forceinline__ void tile_256(const Tile& a) {
     const __amdgpu_buffer_rsrc_t rA1 = nk > 1 ? rA : r0, rW1 = nk > 1 ? rW : r0;
     const int k1 = nk > 1 ? KT : 0;
 #pragma unroll
-    for (int i = 0; i < HX; ++i) T_X(rA, 0, 0, i, 0);
+    for (int i = 0; i < H0; ++i) T_X(rA, 0, 0, i, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW, 0, 0, i, 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW, 0, 1, i, 0);
 #pragma unroll
-    for (int i = 0; i < HX; ++i) T_X(rA, 0, 1, i, 0);
+    for (int i = 0; i < H1; ++i) T_X(rA, 0, 1, i, 0);
 #pragma unroll
-    for (int i = 0; i < HX; ++i) T_X(rA1, 1, 0, i, k1);
+    for (int i = 0; i < H0; ++i) T_X(rA1, 1, 0, i, k1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW1, 1, 1, i, k1);
 #pragma unroll
     for (int i = 0; i < 4; ++i) T_W(rW1, 1, 0, i, k1);
 #pragma unroll
-    for (int i = 0; i < HX; ++i) T_X(rA1, 1, 1, i, k1);
+    for (int i = 0; i < H1; ++i) T_X(rA1, 1, 1, i, k1);
   }
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * HX + 12) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(U + H1 + 12) : "memory");
   __builtin_amdgcn_s_barrier();
 #pragma unroll
-  for (int f = 0; f < 4; ++f) {
-    if (f < HX) { T_RX(0, f, 0); T_RX(0, f, 1); }
-    T_RW(0, f, 0); T_RW(0, f, 1);
+  for (int f = 0; f < H0 || f < 4; ++f) {
+    if (f < H0) { T_RX(0, f, 0); T_RX(0, f, 1); }
+    if (f < 4) { T_RW(0, f, 0); T_RW(0, f, 1); }
   }
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * HX + 8) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(U + 8) : "memory");
   __builtin_amdgcn_s_barrier();
   // (an odd last K tile is followed by one of zeros, which is what a DMA without records leaves in LDS: a loop exit in the
   // middle would have the compiler move accumulators between registers while asm MFMAs it cannot see are still writing them)
@@ -430,12 +454,17 @@ __device__ __forceinline__ void tile_256(const Tile& a) {
 #undef T_ODD
 #undef T_X
 #undef T_W
-  finish<2 * HX, 8, HX, true>(a, acc, cbase, m0 + wm * 32 * HX, n0 + wn * 128, mend, smem + wave * (HX * 8192));
+  constexpr int FIT = 2 * STG / (4 * 8192), PASSES = (U + FIT - 1) / FIT, PU = (U + PASSES - 1) / PASSES;      // row groups that a wave's share of LDS holds
+  char* const mine = smem + wave * (PU * 8192);
+  const int mw = m0 + wm * 16 * U, nw = n0 + wn * 128;
+  EpiRegs er[4];
+  const floatx4 b = column_terms(a, er, cbase, nw + 4 * (lane % 32));
+  if (a.epi.tc == 1) finish_big<U, PU, 1>(a, acc, more, er, b, cbase, mw, nw, mend, mine);
+  else finish_big<U, PU, 0>(a, acc, more, er, b, cbase, mw, nw, mend, mine);
 }
 
-__global__ __launch_bounds__(256, 1) void gemm_tile_256(Tile a) { tile_256<4>(a); }
-__global__ __launch_bounds__(256, 1) void gemm_tile_192(Tile a) { tile_256<3>(a); }
-__global__ __launch_bounds__(256, 1) void gemm_tile_128(Tile a) { tile_256<2>(a); }
+template <int U>
+__global__ __launch_bounds__(256, 1) void gemm_tile_big(Tile a) { tile_256<U>(a); }
 
 // ------------------------------------------------------------------------------------ smaller tiles
 // 32 MI x 32 NJ outputs, four waves in a 2 x 2 grid of 16 MI x 16 NJ, S stages of LDS: the DMAs of K tile t + S - 1 are issued
@@ -572,7 +601,7 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
           acc[u][t] += *reinterpret_cast<const floatx4*>(smem_all + ((g - 1) * 4 + wave) * OUT + ((u * NJ + t) * 64 + lane) * 16);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the same wave lays its rows down in the same place)
   }
-  finish<MI, NJ, MI>(a, acc, cbase, m0 + wm * 16 * MI, n0 + wn * 16 * NJ, mend, smem_all + wave * OUT);
+  finish<MI, NJ>(a, acc, cbase, m0 + wm * 16 * MI, n0 + wn * 16 * NJ, mend, smem_all + wave * OUT);
 }
 #undef T_DMA
 
@@ -606,7 +635,7 @@ int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
 // cheapest sum wins.  us per K tile and per round for products of few K tiles, measured on full rounds at K = 128 .. 8192, and for those of
 // at least LONG (least squares of the relative error over 400, 120 and 100 random products of 64 .. 20,000 rows with cold weights), where a round
 // that fills a part of the chip takes PART of a full one's time a K tile and more by its share (the clock rises).  The second kind of
-// product takes 1.014 of the best tile's time on average (1.026 by the first figures; fp32 rows on bf16 weights 1.017 and 1.057, fp32 1.008
+// product takes 1.009 of the best tile's time on average (1.026 by the first figures; fp32 rows on bf16 weights 1.017 and 1.057, fp32 1.008
 // and 1.012); below LONG they are no better than the first.  Row groups stay with the first: their sizes and the blocks' share of a cold W
 // decide, and of 400 random ones 31 were more than 4% slower by the second (and 1% faster on average).
 struct TileCost { int tm, tn, slots; float k_us, round_us, k_long, round_long; };
@@ -620,8 +649,10 @@ static const TileCost TILES[] = {{256, 256, 256, 1.42f, 11.f, 1.263f, 11.816f}, 
                                  {64, 64, 256, 0.26f, 3.f, 0.2f, 3.425f},
                                  {32, 64, 256, 0.16f, 3.5f, 0.137f, 3.665f}, {32, 32, 256, 0.12f, 3.5f, 0.089f, 3.092f},       // four
                                  {192, 256, 256, 1.09f, 9.5f, 0.945f, 9.866f}, {128, 256, 256, 0.82f, 8.f, 0.733f, 7.441f},
-                                 {64, 128, 512, 0.f, 0.f, 0.455f, 4.821f}};         // two blocks a CU, which stand at barriers of their own: 1024 x 4096 x 2048
-                                                                                    // 23.6 us, 24.6 on 128 x 128, 28.2 on two wave groups (long products only)
+                                 // long products only: two blocks a CU, which stand at barriers of their own (1024 x 4096 x 2048 23.6 us, 24.6 on
+                                 // 128 x 128, 28.2 on two wave groups), and the heights between and above those of 256 columns (above: 8536 x 2048 x 2048)
+                                 {64, 128, 512, 0.f, 0.f, 0.455f, 4.821f}, {160, 256, 256, 0.f, 0.f, 0.859f, 8.671f}, {224, 256, 256, 0.f, 0.f, 1.09f, 11.562f},
+                                 {288, 256, 256, 0.f, 0.f, 1.335f, 14.185f}, {320, 256, 256, 0.f, 0.f, 1.459f, 15.46f}};
 // fp32 rows, bf16 weights (2048 x 2048 x 2048: 128 x 128 36 us, 64 x 128 38, 64 x 64 45)
 static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f, 0.945f, 5.724f}, {64, 128, 256, 0.47f, 5.f, 0.561f, 3.771f}, {64, 64, 256, 0.37f, 4.2f, 0.313f, 3.17f},
                                        {64, 64, 512, 0.6f, 4.f, 0.476f, 3.454f},    // two blocks a CU
@@ -659,15 +690,15 @@ static int pick_tile(const TileCost* tiles, int count, float part, int M, int N,
   return best;
 }
 
-// the index of the tile in its table
-static int choose(int ta, int tw, bool ragged, int M, int N, int nk, int groups, bool by_rows, bool gated) {
+// the index of the tile in its table (tall: rows of A lie so that 320 of them are within 32-bit offsets)
+static int choose(int ta, int tw, bool ragged, bool tall, int M, int N, int nk, int groups, bool by_rows, bool gated) {
   if (ta == 1)
-    return ragged ? 1 + pick_tile(TILES + 1, 6, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, 10, PART, M, N, nk, groups, by_rows, gated);
+    return ragged ? 1 + pick_tile(TILES + 1, 6, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, tall ? 14 : 12, PART, M, N, nk, groups, by_rows, gated);
   return tw == 1 ? pick_tile(TILES_MIXED, 5, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 6, 1.f, M, N, nk, groups, by_rows, gated);
 }
 
 extern "C" int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated) {
-  return choose(ta, tw, false, M, N, K * (tw == 1 ? 2 : 4) / 128, groups, by_rows != 0, gated != 0);
+  return choose(ta, tw, false, true, M, N, K * (tw == 1 ? 2 : 4) / 128, groups, by_rows != 0, gated != 0);
 }
 
 int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups,
@@ -685,18 +716,22 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
   const int nk = K * ew / 128;
   const Tile t = {(const char*)A, (const char*)W, C, epi, M, N, nk, lda * ea, ldw * ew, ldc, a_rows, offs, groups, w_gs * ew, a_gs * ea, c_gs,
                   a_mod < 1 ? 1 : a_mod, 0, 0, 0, ragged};
-  const int tile = choose(ta, tw, ragged, M, N, nk, groups, offs != nullptr, gated);
+  const int tile = choose(ta, tw, ragged, ((long long)lda * 320 + K) * ea < (1LL << 31), M, N, nk, groups, offs != nullptr, gated);
   if (ta == 1) {
     switch (tile) {
-      case 0: return start<gemm_tile_256>(256, 256, 256, t256::lds_bytes(4), t, s);
+      case 0: return start<gemm_tile_big<8>>(256, 256, 256, t256::lds_bytes(8), t, s);
       case 1: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 2, 1>>(128, 128, 256, 2 * 32768, t, s);
       case 2: return start<gemm_tile_mid<bf16_t, bf16_t, 4, 4, 2, 1, 2>>(128, 128, 512, 4 * 32768, t, s);
       case 3: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
       case 4: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
       case 5: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
       case 6: return start<gemm_tile_mid<bf16_t, bf16_t, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
-      case 7: return start<gemm_tile_192>(192, 256, 256, t256::lds_bytes(3), t, s);
-      case 8: return start<gemm_tile_128>(128, 256, 256, t256::lds_bytes(2), t, s);
+      case 7: return start<gemm_tile_big<6>>(192, 256, 256, t256::lds_bytes(6), t, s);
+      case 8: return start<gemm_tile_big<4>>(128, 256, 256, t256::lds_bytes(4), t, s);
+      case 10: return start<gemm_tile_big<5>>(160, 256, 256, t256::lds_bytes(5), t, s);
+      case 11: return start<gemm_tile_big<7>>(224, 256, 256, t256::lds_bytes(7), t, s);
+      case 12: return start<gemm_tile_big<9>>(288, 256, 256, t256::lds_bytes(9), t, s);
+      case 13: return start<gemm_tile_big<10>>(320, 256, 256, t256::lds_bytes(10), t, s);
       default: return start<gemm_tile_mid<bf16_t, bf16_t, 2, 4, 3, 2, 1>>(64, 128, 256, 3 * 24576, t, s);
     }
   }

@@ -201,6 +201,22 @@ def test_two_blocks_a_unit(ops, M, N, K):
     close(H.gated_matmul_nt(a, w, torch.float32), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
 
 
+# 256-column tiles of 160, 224, 288 and 320 rows, whose row groups leave an odd one over and, in the two tallest, are partly held apart from the rest:
+# long plain and gated products, both result types, rows and columns past the last tile's end, an odd number of K tiles; tolerances as above
+@pytest.mark.parametrize("tile,M,N,K", [(10, 776, 9352, 1216), (11, 1169, 9264, 1216), (12, 1540, 9416, 1216), (13, 1731, 9360, 1216), (13, 2560, 8192, 1152)])
+def test_tile_heights(ops, tile, M, N, K):
+    H, _ = ops
+    assert [H.k.fls_seq_gemm_tile_of(1, 1, M, N, K, 1, 0, g) for g in (0, 1)] == [tile, tile]
+    torch.manual_seed(M + N + K)
+    a, w, b = torch.randn(M, K, device=DEV).bfloat16(), (0.1 * torch.randn(N, K, device=DEV)).bfloat16(), torch.randn(N, device=DEV)
+    z = a.double() @ w.double().t()
+    close(H.matmul_nt(a, w, b), z + b, 1e-5)
+    close(H.matmul_nt(a, w, b, relu2=True, out_dtype=torch.bfloat16), torch.relu(z + b).square(), 2 ** -8)
+    gate = torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:]
+    close(H.gated_matmul_nt(a, w, torch.float32), gate, 2e-5)
+    close(H.gated_matmul_nt(a, w, torch.bfloat16), gate, 2 ** -8)
+
+
 # few rows per group, one group of more than the 16 that a pass over its weights takes, empty groups, a K tail
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("K", [64, 200])
