@@ -1,15 +1,15 @@
 // C[M,N] = epilogue(A[M,K] . W[N,K]^T) for few rows (decoding, small expert groups): a stream of W through the chip once.
 //
-// A block owns 16 output columns (or 32: NB = 2) and its WV waves cut K between them in chunks of U steps: a wave issues a chunk's
-// 16-byte loads of its weight rows, and of the rows of A that there are (the caches hold them), before the first of their MFMAs, straight
-// from global memory -- nothing of W is read twice, LDS would only add a wait.  A K step is 32 elements of bf16 (one 16x16x32 MFMA) or 16
-// of fp32 (four 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  The waves' partial sums meet in LDS, in the order of the waves.
-// What bounds it is HBM where the weight is large, else the chain of a launch, a load's latency and the sums (2048 x 2048: 6.3 us); what
-// keeps the loads in flight is many waves with few registers each, not long chunks: with two or four steps a chunk (row groups: twice), no masks on whole chunks
-// and 32-bit offsets a wave takes 58 to 116 registers (blocks of 32 columns 130 to 148; eight steps: 98 to 156).  Cold weights, eight steps and here: 8 rows x 8192 x 2048
-// 12.6 -> 10.0 us, 6416 x 2048 13.5 -> 9.9, 32000 x 2048 32 -> 30.7 (floor 28); 24 rows x 6416 x 2048 14.7 -> 12.1, gated 5440 x 2048 20.2 -> 18.1;
-// fp32, 3 rows x 2048 x 8192 29.9 -> 27.3, 32000 x 2048 59.6 -> 51.4.  A second chunk's registers, loaded ahead, were slower everywhere.  What is
-// left of K behind the whole chunks is one chunk with masks (step by step, each waiting for its loads: 21 rows x 6416 x 736 8.7 us, 7.1 so).
+// A block owns 16 output columns (or 32: NB = 2); its WV waves take the K tiles (128 bytes of a row) by turns, each with a ring of its own
+// in LDS that DMAs fill, whole 128-byte lines of W's rows and of the rows of A that there are: no wave waits for another before the
+// sums, which meet in LDS in the order of the waves.  A tile is two steps of 32 elements of bf16 (a 16x16x32 MFMA each) or 16 of fp32 (four
+// 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  Why not straight to registers: what a lane needs for an MFMA is 16 bytes of its own
+// row, so that neighbouring lanes' loads are rows apart, and a CU takes such loads at 16 bytes a cycle, 54 by DMA; with the loads of A, as many for 16
+// rows as for 16 columns, that was the bound.  Cold weights, before and so (us): 8 rows x 2048 x 2048 6.3, 5.1; x 2048 x 8192 15.6, 13.1; x 32000 x 2048
+// 31.5, 27.2 (the rate of a copy: 27.8); 24 rows x 2048 x 2048 8.2, 5.5; x 2048 x 8192 23.2, 15.0; x 32000 x 2048 37.5, 29.3; gated 5440 x 2048 18.3, 13.2;
+// fp32 8 rows x 2048 x 8192 28.3, 21.9, 24 rows 49.4, 30; 16 rows in 8 groups, gated 2048 x 2048 29.4, 29.1, 2048 x 2048 16.5, 14.6.
+#include <algorithm>
+
 #include "seq_common.h"
 #include "fls_seq.h"
 #include "gemm_epi.h"
@@ -21,17 +21,9 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 // what a lane holds of one K step: 8 bf16 or 4 fp32
 template <typename TW> struct Step;
-template <> struct Step<bf16_t> { typedef bf16x8 V; static constexpr int K = 32, LANE = 8; };
-template <> struct Step<float> { typedef floatx4 V; static constexpr int K = 16, LANE = 4; };
+template <> struct Step<bf16_t> { typedef bf16x8 V; };
+template <> struct Step<float> { typedef floatx4 V; };
 
-__device__ __forceinline__ void load_step(const bf16_t* p, bf16x8& v) { v = *reinterpret_cast<const bf16x8*>(p); }
-__device__ __forceinline__ void load_step(const float* p, floatx4& v) { v = *reinterpret_cast<const floatx4*>(p); }
-__device__ __forceinline__ void load_step(const float* p, bf16x8& v) {        // fp32 rows against bf16 weights: rounded on the way in
-  typedef float floatx8 __attribute__((ext_vector_type(8)));
-  const floatx4 a = *reinterpret_cast<const floatx4*>(p), b = *reinterpret_cast<const floatx4*>(p + 4);
-  const floatx8 f = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-  v = __builtin_convertvector(f, bf16x8);
-}
 __device__ __forceinline__ floatx4 mfma_step(const bf16x8& w, const bf16x8& x, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x, c, 0, 0, 0);
 }
@@ -41,13 +33,30 @@ __device__ __forceinline__ floatx4 mfma_step(const floatx4& w, const floatx4& x,
   return c;
 }
 
-template <typename TA, typename TW, int MG, int WV, int U, int NB, bool GATED>
-__global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, const TW* __restrict__ W, void* __restrict__ C, Epi epi,
-                                                     int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs,
-                                                     const int* __restrict__ a_rows, long long w_gs) {
+#define LDS_AS __attribute__((address_space(3)))
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
+}
+#define R_DMA(rs, off, k0, dst) __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (LDS_AS void*)(dst), 16, off, k0, 0, 0)
+
+// A wave's ring: stages of a K tile of HW 16-row panels of W and of XR rows of A, 20 KB of them (eight waves on a CU, 64 KB of W and more in
+// flight) for up to two rounds of blocks (one in fp32), else 10 KB and twice the blocks on a CU: 150 random products by row groups, many of them empty, took
+// 0.93 (bf16), 0.87 (fp32 on bf16) and 0.86 (fp32) of their time before with 20 KB, 0.90, 0.85 and 0.82 with 10; 24 rows x 2048 x 8192 14.8 and 15.5 us,
+// 48 rows of 10 groups x 2048 x 2048 20.0 and 20.6, 6 of 8 in fp32 21.3 and 20.0.
+constexpr int stages_in(int bytes, int stage) { return bytes / stage < 2 ? 2 : bytes / stage > 6 ? 6 : bytes / stage; }
+template <typename TA, typename TW, int XR, int HW> struct Ring {
+  static constexpr int XS = sizeof(TA) / sizeof(TW), XA = XR * XS / 8, SW = HW * 2048, STAGE = SW + XA * 1024, CNT = 2 * HW + XA;
+  static constexpr int NST = stages_in(20480, STAGE), FEW = stages_in(10240, STAGE);
+};
+
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
+__device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
+                                        const int* offs, const int* a_rows, long long w_gs, int nst) {
   typedef typename Step<TW>::V V;
-  constexpr int SK = Step<TW>::K, LN = Step<TW>::LANE, HW = GATED ? 2 * NB : NB;
-  __shared__ floatx4 red[WV][MG * HW][64];
+  constexpr int HW = GATED ? 2 * NB : NB, MG = (XR + 15) / 16;
+  typedef Ring<TA, TW, XR, HW> R;
+  constexpr int XS = R::XS, XA = R::XA, STAGE = R::STAGE, NST = R::NST, CNT = R::CNT;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   float* const host = !GATED && epi.mirror != nullptr ? *epi.mirror : nullptr;
   if (offs != nullptr) {                   // row groups (experts): this block's group owns rows offs[g] .. offs[g+1]
     const int g = blockIdx.y, r0 = offs[g];
@@ -62,80 +71,107 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
   const int n0 = blockIdx.x * 16 * NB;
-  const int steps = (K + SK - 1) / SK, chunks = (steps + U - 1) / U, per = (chunks + WV - 1) / WV * U;
-  const int s0 = wave * per, s1 = min(steps, s0 + per);
-  // (a gated product: the columns' gate rows and, N rows on, their up rows)
-  const TW* wb[HW];
-  unsigned wo[HW];
+  // DMA pieces of 1 KB: 8 rows of 128 bytes, 16-byte chunk c of row r in place c ^ (r & 7) (rows of A of twice the size: 4 rows, c ^ (r & 15))
+  const int lr = lane >> 3, lc = (lane & 7) ^ lr;
+  const int kb = K * (int)sizeof(TW), stages = (kb + 127) / 128, mine = (stages - wave + WV - 1) / WV;
+  char* const ring = smem + wave * (nst * STAGE);
+  __amdgpu_buffer_rsrc_t rw[HW];
+  unsigned wo[HW][2];
 #pragma unroll
-  for (int h = 0; h < HW; ++h) {
+  for (int h = 0; h < HW; ++h) {           // (a gated product: the columns' gate rows and, N rows on, their up rows)
     const int b = GATED ? h >> 1 : h, n1 = min(n0 + 16 * b, N - 1);
-    wb[h] = W + (size_t)(n1 + (GATED && (h & 1) ? N : 0)) * ldw;
-    wo[h] = (unsigned)(min(fr, N - 1 - n1) * ldw + grp * LN);
+    const TW* p = W + (size_t)(n1 + (GATED && (h & 1) ? N : 0)) * ldw;
+    rw[h] = rsrc_of(p);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) wo[h][j] = (unsigned)min(8 * j + lr, N - 1 - n1) * ldw * (unsigned)sizeof(TW) + lc * 16;
   }
+  const __amdgpu_buffer_rsrc_t ra = rsrc_of(A);
+  const bool few = XR == 16 && M <= 8;                     // (a row group: half of its stages' pieces of A)
+  auto red = [&](int w, int at, int l) -> floatx4& { return *reinterpret_cast<floatx4*>(smem + w * (nst * STAGE) + (at * 64 + l) * 16); };
+  static_assert(MG * HW * 1024 <= STAGE, "a wave's sums fit its ring");
   for (int m0 = 0; m0 < M; m0 += 16 * MG) {
+    unsigned xo[XA];
+#pragma unroll
+    for (int i = 0; i < XA; ++i) {
+      const int row = XS == 1 ? 8 * i + lr : 4 * i + (lane >> 4), r = min(m0 + row, M - 1);
+      xo[i] = (unsigned)(a_rows != nullptr ? a_rows[r] : r) * lda * (unsigned)sizeof(TA) + (XS == 1 ? lc * 16 : ((lane ^ row) & 15) * 16);
+    }
     floatx4 acc[HW][MG];
-    bool ok[MG];
-    const TA* xp[MG];
-    V x[MG][U];
-#pragma unroll
-    for (int u = 0; u < MG; ++u) {
-#pragma unroll
-      for (int h = 0; h < HW; ++h) acc[h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int i = 0; i < U; ++i) x[u][i] = V{};             // (rows past M stay zero: no loads for them)
-      const int r = min(m0 + u * 16 + fr, M - 1);
-      ok[u] = m0 + u * 16 + fr < M;
-      xp[u] = A + (size_t)(a_rows != nullptr ? a_rows[r] : r) * lda + grp * LN;
-    }
-    int s = s0;
-    for (; s + U <= s1 && (s + U) * SK <= K; s += U) {
-      V w[HW][U];
-#pragma unroll
-      for (int i = 0; i < U; ++i)
-#pragma unroll
-        for (int h = 0; h < HW; ++h) load_step(wb[h] + s * SK + (wo[h] + i * SK), w[h][i]);
-#pragma unroll
-      for (int u = 0; u < MG; ++u)
-        if (ok[u]) {
-#pragma unroll
-          for (int i = 0; i < U; ++i) load_step(xp[u] + (size_t)(s + i) * SK, x[u][i]);
-        }
-#pragma unroll
-      for (int i = 0; i < U; ++i)
-#pragma unroll
-        for (int u = 0; u < MG; ++u)
-#pragma unroll
-          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
-    }
-    if (s < s1) {                          // (the last chunk may end short, and its last step: K is a multiple of a lane's share)
-      V w[HW][U];
-#pragma unroll
-      for (int i = 0; i < U; ++i) {
-        const bool in = s + i < s1 && (s + i) * SK + grp * LN < K;
-#pragma unroll
-        for (int h = 0; h < HW; ++h) {
-          w[h][i] = V{};
-          if (in) load_step(wb[h] + s * SK + (wo[h] + i * SK), w[h][i]);
-        }
-#pragma unroll
-        for (int u = 0; u < MG; ++u) {
-          x[u][i] = V{};
-          if (in && ok[u]) load_step(xp[u] + (size_t)(s + i) * SK, x[u][i]);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < U; ++i)
-#pragma unroll
-        for (int u = 0; u < MG; ++u)
-#pragma unroll
-          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][i], x[u][i], acc[h][u]);
-    }
-    if (m0 > 0) __syncthreads();
 #pragma unroll
     for (int u = 0; u < MG; ++u)
 #pragma unroll
-      for (int h = 0; h < HW; ++h) red[wave][u * HW + h][lane] = acc[h][u];
+      for (int h = 0; h < HW; ++h) acc[h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto fill = [&](int t, char* stg) {    // the wave's t-th stage (chunks past K: zeros)
+      const int k0 = (wave + t * WV) * 128;
+      const bool cut = k0 + 128 > kb;
+      const unsigned none = cut && k0 + lc * 16 >= kb ? 0x80000000u : 0u;
+#pragma unroll
+      for (int h = 0; h < HW; ++h)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) R_DMA(rw[h], wo[h][j] | none, k0, stg + (2 * h + j) * 1024);
+#pragma unroll
+      for (int i = 0; i < XA; ++i) {
+        unsigned no = none;
+        if (XS == 2) no = cut && k0 * 2 + (((lane ^ (4 * i + (lane >> 4))) & 15) * 16) >= kb * 2 ? 0x80000000u : 0u;
+        if (!(few && i >= XA / 2)) R_DMA(ra, xo[i] | no, k0 * XS, stg + R::SW + i * 1024);
+      }
+    };
+#pragma unroll
+    for (int t = 0; t < NST; ++t)
+      if (t < min(nst, mine)) fill(t, ring + t * STAGE);
+    char* stg = ring;
+    for (int t = 0; t < mine; ++t) {
+      const int after = min(nst - 1, mine - 1 - t);        // stages that may stay in flight
+      asm volatile("" ::: "memory");
+#define R_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | ((n) >> 4) << 14 | 0x0f70)
+      if (after == 0) R_VM(0);
+#define R_WAIT(n)                            \
+  else if (NST > n && after == n) {          \
+    if (few) R_VM(n * (CNT - XA / 2));       \
+    else R_VM(n * CNT);                      \
+  }
+      R_WAIT(1)
+      R_WAIT(2)
+      R_WAIT(3)
+      R_WAIT(4)
+      R_WAIT(5)
+#undef R_WAIT
+#undef R_VM
+      asm volatile("" ::: "memory");
+      V w[HW][2], x[MG][2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int c = ((4 * k + grp) ^ (fr & 7)) << 4;
+#pragma unroll
+        for (int h = 0; h < HW; ++h) w[h][k] = *reinterpret_cast<const V*>(stg + h * 2048 + fr * 128 + c);
+#pragma unroll
+        for (int u = 0; u < MG; ++u) {
+          const int r = min(u * 16 + fr, XR - 1);         // (rows past M: columns that are not stored)
+          if constexpr (XS == 1) {
+            x[u][k] = *reinterpret_cast<const V*>(stg + R::SW + r * 128 + (((4 * k + grp) ^ (r & 7)) << 4));
+          } else {
+            typedef float floatx8 __attribute__((ext_vector_type(8)));
+            const char* row = stg + R::SW + r * 256;
+            const int a = 8 * k + 2 * grp, sw = r & 15;
+            const floatx4 lo = *(const floatx4*)(row + ((a ^ sw) << 4)), hi = *(const floatx4*)(row + (((a + 1) ^ sw) << 4));
+            x[u][k] = __builtin_convertvector((floatx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), V);
+          }
+        }
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      if (t + nst < mine) fill(t + nst, stg);
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int u = 0; u < MG; ++u)
+#pragma unroll
+          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][k], x[u][k], acc[h][u]);
+      stg = stg + STAGE == ring + nst * STAGE ? ring : stg + STAGE;
+    }
+#pragma unroll
+    for (int u = 0; u < MG; ++u)
+#pragma unroll
+      for (int h = 0; h < HW; ++h) red(wave, u * HW + h, lane) = acc[h][u];
     __syncthreads();
     for (int i = threadIdx.x; i < 64 * MG * NB; i += 64 * WV) {
       // (results that go to the host as well: neighbouring lanes write a row's columns, 64 NB bytes)
@@ -144,12 +180,12 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
       const int b = by_rows ? (i >> 2) % NB : (i >> 6) % NB, u = (i >> 6) / NB, at = u * HW + (GATED ? 2 * b : b);
       const int row = m0 + u * 16 + (l & 15), col0 = n0 + 16 * b + 4 * (l >> 4);
       if (row < M) {
-        floatx4 v = red[0][at][l], v2 = {0.f, 0.f, 0.f, 0.f};
+        floatx4 v = red(0, at, l), v2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 1; w < WV; ++w) v += red[w][at][l];
+        for (int w = 1; w < WV; ++w) v += red(w, at, l);
         if constexpr (GATED) {
 #pragma unroll
-          for (int w = 0; w < WV; ++w) v2 += red[w][at + 1][l];
+          for (int w = 0; w < WV; ++w) v2 += red(w, at + 1, l);
         }
         EpiRegs er = epi_regs(epi);
         if constexpr (GATED) {
@@ -176,15 +212,28 @@ __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, c
         }
       }
     }
+    if (m0 + 16 * MG < M) __syncthreads();               // (the sums lie in the rings)
   }
 }
 
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
+__global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, const TW* __restrict__ W, void* __restrict__ C, Epi epi,
+                                                     int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs,
+                                                     const int* __restrict__ a_rows, long long w_gs, int nst) {
+  rows_of<TA, TW, XR, WV, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs, nst);
+}
 
-template <typename TA, typename TW, int MG, int WV, int U, int NB, bool GATED>
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
 int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
           const int* a_rows, long long w_gs, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_rows<TA, TW, MG, WV, U, NB, GATED>), dim3((N + 16 * NB - 1) / (16 * NB), offs != nullptr ? groups : 1), dim3(64 * WV), 0, s,
-                     (const TA*)A, (const TW*)W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs);
+  typedef Ring<TA, TW, XR, GATED ? 2 * NB : NB> R;
+  static const hipError_t a = hipFuncSetAttribute((const void*)gemm_rows<TA, TW, XR, WV, NB, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, WV * R::NST * R::STAGE);
+  if (a != hipSuccess) return -(int)a;
+  const int cols = (N + 16 * NB - 1) / (16 * NB), gs = offs != nullptr ? groups : 1, stages = (K * (int)sizeof(TW) + 127) / 128;
+  const bool deep = (long long)cols * gs <= (sizeof(TW) == 2 ? 1024 : 512);
+  const int nst = std::min((int)(deep ? R::NST : R::FEW), (stages + WV - 1) / WV);       // (a short K needs less)
+  hipLaunchKernelGGL((gemm_rows<TA, TW, XR, WV, NB, GATED>), dim3(cols, gs), dim3(64 * WV), WV * nst * R::STAGE, s, (const TA*)A, (const TW*)W, C, epi, M, N, K,
+                     lda, ldw, ldc, offs, a_rows, w_gs, nst);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 1 : -(int)e;
 }
@@ -193,29 +242,28 @@ int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, i
 
 int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
                   int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s) {
-  // Row groups of 16 rows a pass over W, or 32 (17 .. 32 rows in one pass: 24 x 2048 x 2048 8.1 us, 10.3 in two).  Eight waves share
-  // K where one block a CU or less has all the columns (2048 x 8192: 15.4 us, 17.2 with four), four where several blocks share a CU
-  // anyway (8192 x 2048: 10.0, 10.8 with eight).  With two row groups a block of 16 columns reads twice as much of A as of W: 32 from 6,400
-  // columns on (24 rows x 6416 x 2048: 14.1 us -> 12.1, x 32000 44.7 -> 37.9; 4096 x 14336 38.6, 50 on 128 blocks).  9,700 random products
-  // (profiles/cases/few_rows_columns.txt): 1.2 to 1.3 of the time up to 4,096 columns, 0.8 to 0.96 from there to 8,176, 0.9 to 1.15 above.
-  // Row groups: most of a launch's blocks may belong to empty groups, and the others have their CU to themselves: twice the steps in flight (of
-  // 10,200 random products 0.7% are more than 6% slower than on eight steps, gated four; with the short chunks 12%, up to 1.5 times).
+  // 16 rows a pass over W (8 if there are no more in all), without row groups up to 32 in one.  Eight waves share K where one block a CU or less
+  // has all the columns and K is more than a tile for each (8 rows x 2048 x 2048 5.1 us, 5.4 with four; 24 rows 5.8 and 5.6, gated 8.1 and 7.8),
+  // else four, two blocks a CU or more.  Blocks of 32 columns read half as much of A and leave no half-empty second round: from one round of
+  // 16-column blocks to 448 (8 rows x 6416 x 2048 9.3 -> 8.8 us; 8192, two full blocks a CU, 9.7 and 10.3), above 16 rows always (24 rows x 8192 x
+  // 2048 10.8 -> 10.4, x 32000 33.7 -> 29.3), plain bf16 products above 1024 blocks (8 rows x 32000 28.6 -> 27.2; fp32 49.5 and 55.4), and plain bf16 row
+  // groups of a row each or more (48 rows of 10 x 2048 x 2048 21.3 -> 19.9; 4 rows of 8 10.2 and 11.3).
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
-  if ((long long)ldw * 16 + 8 >= (1LL << 31)) return 0;      // (32-bit offsets within a panel)
+  const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
+  if (((long long)ldw * 16 + 8) * ew >= (1LL << 31) || (long long)lda * M * ea >= (1LL << 31)) return 0;      // (32-bit offsets within a panel, among the rows)
   const bool two = offs == nullptr && M > 16;
-  const bool many = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1) > 256;
-#define START(TA, TW, MG, WV, U, NB, GATED) start<TA, TW, MG, WV, U, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
-#define ROWS(TA, TW)                                                                                                       \
-  (gated ? (two ? (many ? START(TA, TW, 2, 4, 2, 1, true) : START(TA, TW, 2, 8, 2, 1, true))                               \
-                : (many ? (offs != nullptr ? START(TA, TW, 1, 4, 4, 1, true) : START(TA, TW, 1, 4, 2, 1, true))            \
-                        : START(TA, TW, 1, 8, 4, 1, true)))                                                                \
-         : (two ? (N >= 6400 ? START(TA, TW, 2, 4, 4, 2, false)                                                            \
-                             : many ? START(TA, TW, 2, 4, 4, 1, false) : START(TA, TW, 2, 8, 4, 1, false))                 \
-                : (many ? (offs != nullptr ? START(TA, TW, 1, 4, 8, 1, false) : START(TA, TW, 1, 4, 4, 1, false))          \
-                        : START(TA, TW, 1, 8, 4, 1, false))))
+  const long long blocks = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1);
+  const bool wide = offs != nullptr ? !gated && tw == 1 && M >= groups : blocks > 256 && (blocks <= 448 || (!gated && (two || (tw == 1 && blocks > 1024))));
+  const bool eight = !two && !gated && blocks <= 256 && K * ew > 512;
+#define START(TA, TW, XR, WV, NB, GATED) start<TA, TW, XR, WV, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
+#define PANELS(TA, TW, XR)                                                                                                 \
+  (gated ? (wide ? START(TA, TW, XR, 4, 2, true) : START(TA, TW, XR, 4, 1, true))                                          \
+         : wide ? START(TA, TW, XR, 4, 2, false) : eight ? START(TA, TW, XR <= 16 ? XR : 16, 8, 1, false) : START(TA, TW, XR, 4, 1, false))
+#define ROWS(TA, TW) (two ? (M <= 24 ? PANELS(TA, TW, 24) : PANELS(TA, TW, 32)) : M <= 8 ? PANELS(TA, TW, 8) : PANELS(TA, TW, 16))
   if (tw == 0) return ROWS(float, float);
   return ta == 1 ? ROWS(bf16_t, bf16_t) : ROWS(float, bf16_t);
 #undef ROWS
+#undef PANELS
 #undef START
 }

@@ -245,6 +245,27 @@ def test_grouped_few_rows_many_blocks(ops, cdt, tol, K):
         close(H.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), R.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), 1e-5)
 
 
+# few rows at the edges of what a pass takes; K of one lane's share, less than a K tile, a tile and a tail, more tiles than the waves' rings hold; columns
+# past a block's end, one and several rounds of blocks.  Rows of infinities and NaN leave the others alone.  fp32 sums of up to 4,168 products: 1e-5 as above
+@pytest.mark.parametrize("types", ["bf16", "mixed", "fp32"])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 24, 25, 32])
+def test_few_rows_edges(ops, types, M):
+    H, _ = ops
+    ta, tw = {"bf16": (torch.bfloat16, torch.bfloat16), "mixed": (torch.float32, torch.bfloat16), "fp32": (torch.float32, torch.float32)}[types]
+    f64 = lambda t: (t.to(tw) if types == "mixed" else t).double()
+    torch.manual_seed(M)
+    for N, K in ((20, 8), (268, 72), (4124, 200), (6440, 1032), (136, 4168)):
+        a, w = torch.randn(M, K, device=DEV).to(ta), (0.1 * torch.randn(N, K, device=DEV)).to(tw)
+        z = f64(a) @ w.double().t()
+        close(H.matmul_nt(a, w), z, 1e-5)
+        close(H.gated_matmul_nt(a, w, torch.float32), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
+        if M > 1:
+            b = a.clone()
+            b[M - 1, K // 2], b[M // 2 - 1, K - 1] = float("inf"), float("nan")
+            y, rest = H.matmul_nt(b, w), [r for r in range(M) if r not in (M - 1, M // 2 - 1)]
+            assert torch.equal(y[rest], H.matmul_nt(a, w)[rest]) and not y[[M - 1, M // 2 - 1]].isfinite().any()
+
+
 # about the rows up to which row groups take the few-row kernel, spread over the groups and nearly all in one
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("M", [64, 65, 128, 129])
