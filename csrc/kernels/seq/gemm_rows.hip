@@ -96,11 +96,11 @@ __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const
       const int row = XS == 1 ? 8 * i + lr : 4 * i + (lane >> 4), r = min(m0 + row, M - 1);
       xo[i] = (unsigned)(a_rows != nullptr ? a_rows[r] : r) * lda * (unsigned)sizeof(TA) + (XS == 1 ? lc * 16 : ((lane ^ row) & 15) * 16);
     }
-    floatx4 acc[HW][MG];
+    floatx4 acc[2][HW][MG];                // (the two steps of a tile in sums of their own, which rounds less)
 #pragma unroll
     for (int u = 0; u < MG; ++u)
 #pragma unroll
-      for (int h = 0; h < HW; ++h) acc[h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
+      for (int h = 0; h < HW; ++h) acc[0][h][u] = acc[1][h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
     auto fill = [&](int t, char* stg) {    // the wave's t-th stage (chunks past K: zeros)
       const int k0 = (wave + t * WV) * 128;
       const bool cut = k0 + 128 > kb;
@@ -165,13 +165,13 @@ __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const
 #pragma unroll
         for (int u = 0; u < MG; ++u)
 #pragma unroll
-          for (int h = 0; h < HW; ++h) acc[h][u] = mfma_step(w[h][k], x[u][k], acc[h][u]);
+          for (int h = 0; h < HW; ++h) acc[k][h][u] = mfma_step(w[h][k], x[u][k], acc[k][h][u]);
       stg = stg + STAGE == ring + nst * STAGE ? ring : stg + STAGE;
     }
 #pragma unroll
     for (int u = 0; u < MG; ++u)
 #pragma unroll
-      for (int h = 0; h < HW; ++h) red(wave, u * HW + h, lane) = acc[h][u];
+      for (int h = 0; h < HW; ++h) red(wave, u * HW + h, lane) = acc[0][h][u] + acc[1][h][u];
     __syncthreads();
     for (int i = threadIdx.x; i < 64 * MG * NB; i += 64 * WV) {
       // (results that go to the host as well: neighbouring lanes write a row's columns, 64 NB bytes)
