@@ -487,6 +487,15 @@ __device__ __forceinline__ floatx4 mfma_frag(const floatx4& w, const floatx4& x,
   return c;
 }
 
+// (even and odd terms of four in sums of their own)
+__device__ __forceinline__ void mfma_frag(const floatx4& w, const floatx4& x, floatx4& c, floatx4& odd) {
+#pragma unroll
+  for (int i = 0; i < 4; i += 2) {
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i], x[i], c, 0, 0, 0);
+    odd = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i + 1], x[i + 1], odd, 0, 0, 0);
+  }
+}
+
 // the DMAs of K tile kt: PX pieces of A (128 XS bytes a row), PW of W
 template <int PX, int PW, int XS, int XIMG>
 __device__ __forceinline__ void fill(const char* Ab, const char* Wb, int kt, int nk, int wave, const unsigned* xo, const unsigned* wo, char* stg) {
@@ -533,11 +542,16 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
   const int fr = lane & 15, grp = lane >> 4, sw = fr & 7;
   const int c0 = (grp ^ sw) << 4, c1 = ((4 + grp) ^ sw) << 4;
   const int xrow = (wm * 16 * MI + fr) * 128 * XS, wrow = XIMG + (wn * 16 * NJ + fr) * 128;
-  floatx4 acc[MI][NJ];
+  // (small tiles of one wave group: sums of a part of the terms each, as several groups have them.  One of all in a row is further from 64
+  // bits: fp32, 2048 terms 8.1e-7, 5.8e-7 in two sums and 4.1e-7 in four, for the same time)
+  constexpr int SUMS = KG > 1 || MI * NJ > 8 ? 1 : sizeof(TW) == 4 && MI * NJ <= 4 ? 4 : 2;
+  floatx4 sums[SUMS][MI][NJ], (&acc)[MI][NJ] = sums[0];
 #pragma unroll
-  for (int u = 0; u < MI; ++u)
+  for (int i = 0; i < SUMS; ++i)
 #pragma unroll
-    for (int t = 0; t < NJ; ++t) acc[u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < MI; ++u)
+#pragma unroll
+      for (int t = 0; t < NJ; ++t) sums[i][u][t] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int s = 0; s < S - 1; ++s) fill<PX, PW, XS, XIMG>(Ab, Wb, s * KG + kg, nk, wave, xo, wo, smem + s * STG);
   int cur = 0, nxt = S - 1;
@@ -573,10 +587,20 @@ __global__ __launch_bounds__(256 * KG, OCC * KG) void gemm_tile_mid(Tile a) {
 #pragma unroll
       for (int u = 0; u < MI; ++u)
 #pragma unroll
-        for (int t = 0; t < NJ; ++t) acc[u][t] = mfma_frag(w[k][t], x[k][u], acc[u][t]);
+        for (int t = 0; t < NJ; ++t) {
+          if constexpr (SUMS == 4) mfma_frag(w[k][t], x[k][u], sums[2 * k][u][t], sums[2 * k + 1][u][t]);
+          else sums[k % SUMS][u][t] = mfma_frag(w[k][t], x[k][u], sums[k % SUMS][u][t]);
+        }
     cur = cur + 1 == S ? 0 : cur + 1;
     nxt = nxt + 1 == S ? 0 : nxt + 1;
   }
+#pragma unroll
+  for (int u = 0; u < MI; ++u)
+#pragma unroll
+    for (int t = 0; t < NJ; ++t) {
+      if constexpr (SUMS == 4) acc[u][t] = (acc[u][t] + sums[SUMS - 3][u][t]) + (sums[SUMS - 2][u][t] + sums[SUMS - 1][u][t]);
+      else if constexpr (SUMS == 2) acc[u][t] += sums[1][u][t];
+    }
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -635,10 +659,10 @@ int start(int tm, int tn, int threads, int lds, Tile t, hipStream_t s) {
 // cheapest sum wins.  us per K tile and per round for products of few K tiles, measured on full rounds at K = 128 .. 8192, and for those of
 // at least LONG (least squares of the relative error over 400, 120 and 100 random products of 64 .. 20,000 rows with cold weights), where a round
 // that fills a part of the chip takes PART of a full one's time a K tile and more by its share (the clock rises).  The second kind of
-// product takes 1.009 of the best tile's time on average (1.026 by the first figures; fp32 rows on bf16 weights 1.017 and 1.057, fp32 1.008
-// and 1.012); below LONG they are no better than the first.  Row groups stay with the first: their sizes and the blocks' share of a cold W
-// decide, and of 400 random ones 31 were more than 4% slower by the second (and 1% faster on average).
-struct TileCost { int tm, tn, slots; float k_us, round_us, k_long, round_long; };
+// product takes 1.009 of the best tile's time on average (1.026 by the first figures); below LONG they are no better than the first.  Row groups
+// stay with the first: their sizes and the blocks' share of a cold W decide, and of 400 random ones 31 were more than 4% slower by the
+// second (and 1% faster on average).
+struct TileCost { int tm, tn, slots; float k_us, round_us, k_long, round_long; bool shared = false; };      // shared: only where a CU gets several blocks
 static const int LONG = 18;
 static const float PART = 0.8f;
 // bf16 (16384 x 14336 x 4096: the 256 tile 1.49 ms, 128 x 128 2.05; 1024 x 2048 x 2048: 64 x 128 14 us, the 256 tile 42;
@@ -654,14 +678,18 @@ static const TileCost TILES[] = {{256, 256, 256, 1.42f, 11.f, 1.263f, 11.816f}, 
                                  // 2048), at 1.02 of what was fitted: products of many rounds are within 2% of each other on tiles of 256 rows and more, and bound by power
                                  {64, 128, 512, 0.f, 0.f, 0.455f, 4.821f}, {160, 256, 256, 0.f, 0.f, 0.876f, 8.85f}, {224, 256, 256, 0.f, 0.f, 1.112f, 11.8f},
                                  {288, 256, 256, 0.f, 0.f, 1.362f, 14.47f}, {320, 256, 256, 0.f, 0.f, 1.488f, 15.77f}};
-// fp32 rows, bf16 weights (2048 x 2048 x 2048: 128 x 128 36 us, 64 x 128 38, 64 x 64 45)
-static const TileCost TILES_MIXED[] = {{128, 128, 256, 1.02f, 8.f, 0.945f, 5.724f}, {64, 128, 256, 0.47f, 5.f, 0.561f, 3.771f}, {64, 64, 256, 0.37f, 4.2f, 0.313f, 3.17f},
+// fp32 rows, bf16 weights.  64 x 128 on two blocks a CU with two stages each, whose loads, products and stores run beside one another's (before, 128 x 128
+// on one block with three: 2048 x 2048 x 2048 38 us, so 29; 8192 rows 141, 114; 9692 x 2048 x 128 35, 25; 16384 rows of 16 blocks x 256, two sets of weights 384, 321)
+static const TileCost TILES_MIXED[] = {{64, 128, 512, 0.66f, 4.5f, 0.66f, 7.2f}, {64, 128, 256, 0.47f, 5.f, 0.561f, 3.771f}, {64, 64, 256, 0.37f, 4.2f, 0.313f, 3.17f},
                                        {64, 64, 512, 0.6f, 4.f, 0.476f, 3.454f},    // two blocks a CU
                                        {32, 32, 256, 0.16f, 3.5f, 0.137f, 3.025f}};
 // fp32 (bound by the fp32 MFMA's 150 TFLOP/s; 400 x 2048 x 8192: 64 x 64 165 us, 128 x 128 573; 1000 x 2048 x 2048: 64 x 128 71 us,
 // 128 x 128 129)
 static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f, 3.7f, 8.f}, {128, 128, 256, 2.15f, 6.f, 1.934f, 6.092f}, {64, 128, 256, 1.1f, 6.f, 1.05f, 4.441f},
-                                     {64, 64, 256, 0.63f, 4.f, 0.573f, 3.127f}, {32, 64, 256, 0.33f, 4.f, 0.294f, 3.226f}, {32, 32, 256, 0.195f, 4.f, 0.166f, 2.685f}};
+                                     {64, 64, 256, 0.63f, 4.f, 0.573f, 3.127f}, {32, 64, 256, 0.33f, 4.f, 0.294f, 3.226f}, {32, 32, 256, 0.195f, 4.f, 0.166f, 2.685f},
+                                     // long products only: three blocks a CU keep its matrix units busy between them, so that a round is of 256 (1200 x 8192 x
+                                     // 2048 306 us, 343 on 64 x 128; x 4384 185, 205; x 2048 95, 101; one block a CU alone is slower: 400 x 2048 x 8192 156, 143)
+                                     {64, 64, 256, 0.f, 0.f, 0.475f, 0.5f, true}};
 
 static int pick_tile(const TileCost* tiles, int count, float part, int M, int N, int nk, int groups, bool by_rows, bool gated) {
   int best = -1;
@@ -680,6 +708,7 @@ static int pick_tile(const TileCost* tiles, int count, float part, int M, int N,
       us = (full <= 0.9f ? 1.f : full + 0.5f) * (k + round);
     } else {
       const long long blocks = (long long)((M + t.tm - 1) / t.tm) * groups * cols, rest = blocks % t.slots;
+      if (t.shared && blocks <= t.slots) continue;
       us = (float)(blocks / t.slots) * (k + round);
       if (rest) us += k * (lng ? part + (1.f - part) * (float)rest / t.slots : 1.f) + round;
     }
@@ -695,7 +724,7 @@ static int pick_tile(const TileCost* tiles, int count, float part, int M, int N,
 static int choose(int ta, int tw, bool ragged, bool tall, int M, int N, int nk, int groups, bool by_rows, bool gated) {
   if (ta == 1)
     return ragged ? 1 + pick_tile(TILES + 1, 6, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES, tall ? 14 : 12, PART, M, N, nk, groups, by_rows, gated);
-  return tw == 1 ? pick_tile(TILES_MIXED, 5, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 6, 1.f, M, N, nk, groups, by_rows, gated);
+  return tw == 1 ? pick_tile(TILES_MIXED, 5, PART, M, N, nk, groups, by_rows, gated) : pick_tile(TILES_F32, 7, 1.f, M, N, nk, groups, by_rows, gated);
 }
 
 extern "C" int fls_seq_gemm_tile_of(int ta, int tw, int M, int N, int K, int groups, int by_rows, int gated) {
@@ -738,7 +767,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
   }
   if (tw == 1) {
     switch (tile) {
-      case 0: return start<gemm_tile_mid<float, bf16_t, 4, 4, 3, 1, 1>>(128, 128, 256, 3 * 49152, t, s);
+      case 0: return start<gemm_tile_mid<float, bf16_t, 2, 4, 2, 2, 1>>(64, 128, 256, 2 * 32768, t, s);
       case 1: return start<gemm_tile_mid<float, bf16_t, 2, 4, 2, 1, 2>>(64, 128, 512, 4 * 32768, t, s);
       case 2: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 1, 2>>(64, 64, 512, 6 * 24576, t, s);
       case 3: return start<gemm_tile_mid<float, bf16_t, 2, 2, 3, 2, 1>>(64, 64, 256, 3 * 24576, t, s);
@@ -751,6 +780,7 @@ int seq_gemm_tile(const void* A, int ta, const void* W, int tw, void* C, const E
     case 2: return start<gemm_tile_mid<float, float, 2, 4, 3, 1, 2>>(64, 128, 512, 6 * 24576, t, s);
     case 3: return start<gemm_tile_mid<float, float, 2, 2, 4, 1, 2>>(64, 64, 512, 8 * 16384, t, s);
     case 4: return start<gemm_tile_mid<float, float, 1, 2, 3, 1, 4>>(32, 64, 1024, 12 * 12288, t, s);
+    case 6: return start<gemm_tile_mid<float, float, 2, 2, 3, 3, 1>>(64, 64, 256, 3 * 16384, t, s);
     default: return start<gemm_tile_mid<float, float, 1, 1, 4, 1, 4>>(32, 32, 1024, 16 * 8192, t, s);
   }
 }

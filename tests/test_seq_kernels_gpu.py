@@ -245,6 +245,20 @@ def test_grouped_few_rows_many_blocks(ops, cdt, tol, K):
         close(H.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), R.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), 1e-5)
 
 
+# fp32 on 64 x 64 tiles of three blocks a CU: long plain and gated products of more than a round, rows and columns past the last tile's end, an odd number
+# of K tiles; sums of 608 products in fp32: 1e-5 as above
+@pytest.mark.parametrize("M,N", [(1100, 2056), (1037, 2056), (641, 4104)])
+def test_three_blocks_a_unit(ops, M, N):
+    H, _ = ops
+    K = 608
+    assert [H.k.fls_seq_gemm_tile_of(0, 0, M, N, K, 1, 0, g) for g in (0, 1)] == [6, 6]
+    torch.manual_seed(M + N)
+    a, w = torch.randn(M, K, device=DEV), 0.1 * torch.randn(N, K, device=DEV)
+    z = a.double() @ w.double().t()
+    close(H.matmul_nt(a, w), z, 1e-5)
+    close(H.gated_matmul_nt(a, w, torch.float32), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
+
+
 # few rows at the edges of what a pass takes; K of one lane's share, less than a K tile, a tile and a tail, more tiles than the waves' rings hold; columns
 # past a block's end, one and several rounds of blocks.  Rows of infinities and NaN leave the others alone.  fp32 sums of up to 4,168 products: 1e-5 as above
 @pytest.mark.parametrize("types", ["bf16", "mixed", "fp32"])
