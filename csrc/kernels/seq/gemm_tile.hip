@@ -688,7 +688,8 @@ static const TileCost TILES_MIXED[] = {{64, 128, 512, 0.66f, 4.5f, 0.66f, 7.2f},
 static const TileCost TILES_F32[] = {{128, 128, 512, 4.0f, 8.f, 3.7f, 8.f}, {128, 128, 256, 2.15f, 6.f, 1.934f, 6.092f}, {64, 128, 256, 1.1f, 6.f, 1.05f, 4.441f},
                                      {64, 64, 256, 0.63f, 4.f, 0.573f, 3.127f}, {32, 64, 256, 0.33f, 4.f, 0.294f, 3.226f}, {32, 32, 256, 0.195f, 4.f, 0.166f, 2.685f},
                                      // long products only: three blocks a CU keep its matrix units busy between them, so that a round is of 256 (1200 x 8192 x
-                                     // 2048 306 us, 343 on 64 x 128; x 4384 185, 205; x 2048 95, 101; one block a CU alone is slower: 400 x 2048 x 8192 156, 143)
+                                     // 2048 306 us, 343 on 64 x 128; x 4384 185, 205; x 2048 95, 101; one block a CU alone is slower: 400 x 2048 x 8192 156, 143;
+                                     // row groups above five rounds, as their sizes fall: 150 random ones 0.95 of the time)
                                      {64, 64, 256, 0.f, 0.f, 0.475f, 0.5f, true}};
 
 static int pick_tile(const TileCost* tiles, int count, float part, int M, int N, int nk, int groups, bool by_rows, bool gated) {
@@ -696,7 +697,7 @@ static int pick_tile(const TileCost* tiles, int count, float part, int M, int N,
   float least = 0.f;
   for (int v = 0; v < count; ++v) {
     const TileCost& t = tiles[v];
-    const bool lng = nk >= LONG && !by_rows;
+    const bool lng = nk >= LONG && (!by_rows || t.shared);
     if ((gated && t.tn < 64) || (t.k_us == 0.f && !lng)) continue;      // (a wave of the 32-column tile has one half of a gated column only)
     const float k = (float)nk * (lng ? t.k_long : t.k_us), round = lng ? t.round_long : t.round_us;
     // (row groups: their sizes are on the device; each ends in a part of a tile, half of one on average, and how they fall on the
@@ -705,6 +706,7 @@ static int pick_tile(const TileCost* tiles, int count, float part, int M, int N,
     float us;
     if (by_rows) {
       const float full = ((float)M / t.tm + 0.5f * groups) * cols / t.slots;
+      if (t.shared && full <= 5.f) continue;
       us = (full <= 0.9f ? 1.f : full + 0.5f) * (k + round);
     } else {
       const long long blocks = (long long)((M + t.tm - 1) / t.tm) * groups * cols, rest = blocks % t.slots;

@@ -246,7 +246,7 @@ def test_grouped_few_rows_many_blocks(ops, cdt, tol, K):
 
 
 # fp32 on 64 x 64 tiles of three blocks a CU: long plain and gated products of more than a round, rows and columns past the last tile's end, an odd number
-# of K tiles; sums of 608 products in fp32: 1e-5 as above
+# of K tiles, and row groups, empty and of one row among them, as they are and gathered; sums of 608 products in fp32: 1e-5 as above
 @pytest.mark.parametrize("M,N", [(1100, 2056), (1037, 2056), (641, 4104)])
 def test_three_blocks_a_unit(ops, M, N):
     H, _ = ops
@@ -257,6 +257,14 @@ def test_three_blocks_a_unit(ops, M, N):
     z = a.double() @ w.double().t()
     close(H.matmul_nt(a, w), z, 1e-5)
     close(H.gated_matmul_nt(a, w, torch.float32), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
+    sizes, N = [0, M // 2, 1, M - M // 2 - 4, 0, 3], 6152
+    assert [H.k.fls_seq_gemm_tile_of(0, 0, M, N, K, 6, 1, g) for g in (0, 1)] == ([6, 6] if M > 700 else [2, 2])
+    offs, w = torch.tensor(np.cumsum([0] + sizes), dtype=torch.int32, device=DEV), 0.1 * torch.randn(6, N, K, device=DEV)
+    y = lambda x: torch.cat([x[offs[e]:offs[e + 1]].double() @ w[e].double().t() for e in range(6)])
+    close(H.grouped_matmul_nt(a, w, offs), y(a), 1e-5)
+    rows = torch.randperm(M, device=DEV).to(torch.int32) // 2
+    z = y(a[rows.long()])
+    close(H.gated_matmul_nt(a[:(M + 1) // 2], w, torch.float32, offs=offs, rows=rows), torch.nn.functional.silu(z[:, :N // 2]) * z[:, N // 2:], 2e-5)
 
 
 # few rows at the edges of what a pass takes; K of one lane's share, less than a K tile, a tile and a tail, more tiles than the waves' rings hold; columns
