@@ -245,6 +245,25 @@ def test_grouped_few_rows_many_blocks(ops, cdt, tol, K):
         close(H.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), R.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), 1e-5)
 
 
+# decays of -200 .. 200 through an identity product, and of infinities and NaN from the bias, in a few-row block and a tile.  The product of rate and softplus is good to a
+# unit of its last place, whose share of the result is that place itself, up to 88: 88 x 2^-24, and a unit each for the exponential and the sum
+@pytest.mark.parametrize("T", [5, 300])
+def test_decay_values(ops, T):
+    H, _ = ops
+    torch.manual_seed(T)
+    z = (torch.randn(T, 128, device=DEV) * 10 ** (torch.rand(T, 128, device=DEV) * 4 - 2)).clamp(-200, 200).bfloat16()
+    z[0, :2] = torch.tensor([0.0, -0.0], device=DEV)
+    rates = torch.tensor([-4.0, 0.0, 1.0, 2.8], device=DEV)
+    eye = torch.eye(128, device=DEV).bfloat16()
+    y = H.matmul_nt(z, eye, torch.zeros(128, device=DEV), decay=rates)
+    want = torch.exp(-rates.double().exp().repeat_interleave(32) * torch.nn.functional.softplus(z.double(), threshold=1000))
+    assert ((y.double() - want).abs() <= 90 * 2 ** -24 * want + 2.0 ** -126).all()
+    b = torch.zeros(128, device=DEV)
+    b[:3] = torch.tensor([float("inf"), float("-inf"), float("nan")], device=DEV)
+    y = H.matmul_nt(z, eye, b, decay=rates)
+    assert (y[:, 0] == 0).all() and (y[:, 1] == 1).all() and y[:, 2].isnan().all()
+
+
 # fp32 on 64 x 64 tiles of three blocks a CU: long plain and gated products of more than a round, rows and columns past the last tile's end, an odd number
 # of K tiles, and row groups, empty and of one row among them, as they are and gathered; sums of 608 products in fp32: 1e-5 as above
 @pytest.mark.parametrize("M,N", [(1100, 2056), (1037, 2056), (641, 4104)])
