@@ -34,7 +34,7 @@ __device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
 }
 // exp(ap softplus(z)), ap <= 0, in units of log 2: softplus as max(z, 0) + log(1 + exp(-|z|)) in two terms, of which the hardware's exponential and logarithm
 // give the first and exact residuals the second; near 1 a polynomial, where the exponential's last bit is the result's.  20 million of them 72 us by exp(ap
-// log1p(exp(z))) and 31 so (30 is their memory); from 64 bits, over normal z and ap of -1 .. -16, 3.3e-7 and 1.8e-7, largest 8.2e-6 and 2.7e-6.
+// log1p(exp(z))) and 31 so (30 is their memory); from 64 bits, over normal z and ap of -1 .. -16, 3.3e-7 and 1.3e-7, largest 8.2e-6 and 1.3e-6.
 __device__ __forceinline__ float decay_f(float ap, float z) {
   constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f, LN2 = 0.693147181f;
   const float a = fmaxf(-fabsf(z), -130.f), h = a * L2E, hl = __builtin_fmaf(a, L2E, -h) + a * L2E_LO;
