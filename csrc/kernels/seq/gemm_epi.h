@@ -34,19 +34,27 @@ __device__ __forceinline__ void epi_column(const Epi& e, EpiRegs& r, int col) {
 }
 // exp(ap softplus(z)), ap <= 0, in units of log 2: softplus as max(z, 0) + log(1 + exp(-|z|)) in two terms, of which the hardware's exponential and logarithm
 // give the first and exact residuals the second; near 1 a polynomial, where the exponential's last bit is the result's.  20 million of them 72 us by exp(ap
-// log1p(exp(z))) and 31 so (30 is their memory); from 64 bits, over normal z and ap of -1 .. -16, 3.3e-7 and 1.3e-7, largest 8.2e-6 and 1.3e-6.
+// log1p(exp(z))) and 33 so (30 is their memory); from 64 bits, over normal z and ap of -1 .. -16, 3.3e-7 and 1.3e-7, largest 8.2e-6 and 1.3e-6.
+// Infinities, NaN, and numbers that no model has, whose terms leave the range of fp32, go by the plain formula.  mh and t are held as rounded: fused into the
+// sums that follow, a product's rounding would be counted twice.
 __device__ __forceinline__ float decay_f(float ap, float z) {
+  if (!(z >= -80.f && z <= 1e30f && ap >= -1e30f)) return expf(ap * softplus_f(z));
   constexpr float L2E = 1.44269502f, L2E_LO = 1.92596299e-8f, LN2 = 0.693147181f;
-  const float a = fmaxf(-fabsf(z), -130.f), h = a * L2E, hl = __builtin_fmaf(a, L2E, -h) + a * L2E_LO;
+  const float a = -fabsf(z), h = a * L2E, hl = __builtin_fmaf(a, L2E, -h) + a * L2E_LO;
   float e = __builtin_amdgcn_exp2f(h);
   e = __builtin_fmaf(e, hl * LN2, e);
   const float u = 1.f + e, g = __builtin_amdgcn_logf(u), gl = (e - (u - 1.f)) * L2E * __builtin_amdgcn_rcpf(u);
-  const float m = z > 1e30f ? 1e30f : z < 0.f ? 0.f : z, mh = m * L2E, ml = __builtin_fmaf(m, L2E, -mh) + m * L2E_LO;      // (NaN stays)
-  const float s = mh + g, sl = (g - (s - mh)) + (ml + gl);
-  const float t = ap * s, tl = t > -200.f ? __builtin_fmaf(ap, s, -t) + ap * sl : 0.f;
-  const float d = __builtin_amdgcn_exp2f(t), y = (t + tl) * LN2;
+  const float m = fmaxf(z, 0.f);
+  float mh = m * L2E;
+  asm("" : "+v"(mh));
+  const float ml = __builtin_fmaf(m, L2E, -mh) + m * L2E_LO, s = mh + g, sl = (g - (s - mh)) + (ml + gl);
+  float t = ap * s;
+  asm("" : "+v"(t));
+  const float tl = t > -200.f ? __builtin_fmaf(ap, s, -t) + ap * sl : 0.f;
+  const bool low = t < -125.f;             // (the hardware's exponential has no subnormal results)
+  const float d = __builtin_amdgcn_exp2f(low ? t + 64.f : t), y = (t + tl) * LN2;
   const float near = __builtin_fmaf(y, __builtin_fmaf(y, __builtin_fmaf(y, __builtin_fmaf(y, 1.f / 24.f, 1.f / 6.f), 0.5f), 1.f), 1.f);
-  return t > -0.0625f ? near : __builtin_fmaf(d, tl * LN2, d);
+  return t > -0.0625f ? near : __builtin_amdgcn_ldexpf(__builtin_fmaf(d, tl * LN2, d), low ? -64 : 0);
 }
 template <int KIND, bool SIDES = true>
 __device__ __forceinline__ float epi_value_of(float v, const Epi& e, const EpiRegs& r) {

@@ -264,6 +264,26 @@ def test_decay_values(ops, T):
     assert (y[:, 0] == 0).all() and (y[:, 1] == 1).all() and y[:, 2].isnan().all()
 
 
+# decays at the ends of fp32, as exp(-exp(act) softplus(z)) has them: results below 2^-126 (within a unit of their last place beside the share above), rates of zero, of
+# next to nothing under a huge z, and infinite ones, each with the bias's infinities
+@pytest.mark.parametrize("T", [5, 300])
+def test_decay_edges(ops, T):
+    H, _ = ops
+    inf = float("inf")
+    eye, zero = torch.eye(128, device=DEV).bfloat16(), torch.zeros(T, 128, device=DEV).bfloat16()
+    z = torch.linspace(80, 110, T * 128, device=DEV).view(T, 128).bfloat16()
+    y = H.matmul_nt(z, eye, torch.zeros(128, device=DEV), decay=torch.zeros(4, device=DEV))
+    want = torch.exp(-z.double())
+    assert (want < 2.0 ** -126).any() and (want > 2.0 ** -126).any()
+    assert ((y.double() - want).abs() <= 110 * 2 ** -24 * want + 2.0 ** -149).all()
+    b = torch.tensor([inf, -inf, float("nan"), 1e33, 3e38, 0.0, -85.0, -60.0], device=DEV).repeat(16)
+    for act, want in ((-inf, [None, 1, None, 1, 1, 1, 1, 1]), (-75.0, [0, 1, None, math.exp(-1e33 * math.exp(-75.0)), 0, 1, 1, 1]), (inf, [0, None, None, 0, 0, 0, 0, 0])):
+        y = H.matmul_nt(zero, eye, b, decay=torch.full((4,), act, device=DEV)).view(T, 16, 8)
+        for i, v in enumerate(want):
+            got = y[:, :, i]
+            assert got.isnan().all() if v is None else ((got - v).abs() <= 1e-5 * v).all(), (act, i, got[0, 0])
+
+
 # fp32 on 64 x 64 tiles of three blocks a CU: long plain and gated products of more than a round, rows and columns past the last tile's end, an odd number
 # of K tiles, and row groups, empty and of one row among them, as they are and gathered; sums of 608 products in fp32: 1e-5 as above
 @pytest.mark.parametrize("M,N", [(1100, 2056), (1037, 2056), (641, 4104)])
