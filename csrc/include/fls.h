@@ -100,8 +100,9 @@ int fls_fold_norm(void* w, int ldw, int N, int K, const void* gamma, fls_stream_
 // y[dst_idx[r]] = x[src_idx[r]] for r < rows (fp16 rows of H elements; a null index = identity)
 // device-to-device copy: mode 0 HIP runtime (blit kernel), 1 SDMA engines (no CU), 2 `blocks` workgroups
 int fls_copy_d2d(void* dst, const void* src, uint64_t bytes, int mode, int blocks, fls_stream_t s);
-int fls_copy_rows(const void* x, int ldx, const int* src_idx, void* y, int ldy, const int* dst_idx, int rows, int H,
-                  fls_stream_t s);
+// (y_at: as kv0_at of fls_attention, null: y)
+int fls_copy_rows(const void* x, int ldx, const int* src_idx, void* y, int ldy, void* const* y_at, const int* dst_idx,
+                  int rows, int H, fls_stream_t s);
 int fls_gemm_set_splitk(int on);
 int fls_gemm_set_row_chunk(int rows);   // rows per main-path GEMM launch (default 16384; 0 = unlimited)
 int fls_gemm_set_v10_rows(int rows);    // rows of a 256-column main-path tile: 0 by shape, 128, 192 or 256 forced (tests / A-B)
@@ -126,6 +127,8 @@ int fls_gemm_set_mid(int on);   // 64x128-tile kernel for small / medium M (defa
 // shared-prefix / varlen flash attention over packed work items (int32 x8:
 // q_start q_len q_off r0_start r0_len r0_causal r1_start r1_len).
 // kv0 (optional, [P, 2*n_kv*hd] K then V, row stride ld_kv0): range 0 of every work item indexes it.
+// kv0_at (optional, with work2): a cell on the device that holds kv0 when the kernel runs, so that a captured step serves
+// K/V at any address; kv0 is not read then.
 // seg_lo (optional, [T] int32): first packed row of the suffix holding each row; range-1 key j is
 // visible to query row i iff seg_lo[i] <= j <= i, so an item may hold several suffixes of a prompt
 // (null: one suffix per item).  q_block: rows per work item (64 or 128).
@@ -138,8 +141,8 @@ int fls_attention_set_persistent(int on);   // persistent full-pass kernel (defa
 // ws / ws_bytes / n_rows (rows of qkv and out): fp32 scratch of the split-KV range-2 kernel (null: no split)
 int fls_attention(const void* qkv, void* out, const int* work, int n_items, int n_q_heads,
                   int n_kv_heads, int head_dim, int ld_qkv, int ld_out, float scale, const void* kv0,
-                  int ld_kv0, const int* seg_lo, int q_block, const int* work2, const int* r2win,
-                  void* ws, unsigned long long ws_bytes, int n_rows, fls_stream_t s);
+                  int ld_kv0, const void* const* kv0_at, const int* seg_lo, int q_block, const int* work2,
+                  const int* r2win, void* ws, unsigned long long ws_bytes, int n_rows, fls_stream_t s);
 int fls_headnorm_rope(void* x, int ldx, int rows, int n_q, int n_k, const void* qn, const void* kn, const int* pos,
                       const float* cos_t, const float* sin_t, int hd, float eps, fls_stream_t s);
 int fls_rmsnorm(const void* x, const void* w, void* y, const int* row_idx, int rows, int H,

@@ -114,6 +114,7 @@ __global__ __launch_bounds__(64 * WPH * HPB, 2) void attn_fwd(const half_t* __re
                                                     const int* __restrict__ work, const int* __restrict__ seg_lo,
                                                     int nh, int nkv, int ld_qkv, int ld_out, float scale_log2,
                                                     const half_t* __restrict__ kv0, int ld_kv0,
+                                                    const half_t* const* __restrict__ kv0_at,
                                                     const int* __restrict__ work2, const int* __restrict__ r2win,
                                                     float* __restrict__ part) {
   static_assert(!SPL || R2, "split-KV is built for the range-2 (suffix K/V reuse) kernel only");
@@ -136,6 +137,9 @@ __global__ __launch_bounds__(64 * WPH * HPB, 2) void attn_fwd(const half_t* __re
   const int* wi = work + blockIdx.x * 8;
   const int q_start = wi[0], q_len = wi[1], q_off = wi[2];
   if (q_len <= 0) return;                   // padding item (bucketed graph replays); block-uniform
+  if constexpr (R2) {
+    if (kv0_at != nullptr) kv0 = *kv0_at;   // (a captured step: where this replay's K/V lie)
+  }
   const int r_start0 = wi[3], r_len0 = wi[4], r_causal0 = wi[5];
   const int r_start1 = wi[6], r_len1 = wi[7];
   const int kend0 = r_len0 <= 0 ? 0 : (r_causal0 ? min(r_len0, q_off + q_len) : r_len0);
@@ -657,7 +661,8 @@ template <int HD, bool SPL, int NB>
 __global__ __launch_bounds__(256, 1) void attn_decode(const half_t* __restrict__ qkv, half_t* __restrict__ out,
                                                     const int* __restrict__ work, int nh, int nkv, int ld_qkv,
                                                     int ld_out, float scale_log2, const half_t* __restrict__ kv0,
-                                                    int ld_kv0, const int* __restrict__ work2,
+                                                    int ld_kv0, const half_t* const* __restrict__ kv0_at,
+                                                    const int* __restrict__ work2,
                                                     const int* __restrict__ r2win, float* __restrict__ part) {
   constexpr int NW = 4;                     // waves per block (16 packed rows each)
   // NB: tile ring depth (NB - 1 tiles in flight under the math of one)
@@ -678,6 +683,7 @@ __global__ __launch_bounds__(256, 1) void attn_decode(const half_t* __restrict__
   const int* wi = work + blockIdx.x * 8;
   const int q_start = wi[0], q_len = wi[1], q_off = wi[2];
   if (q_len <= 0) return;                   // padding item; block-uniform
+  if (kv0_at != nullptr) kv0 = *kv0_at;     // (a captured step: where this replay's K/V lie)
   const int r_start0 = wi[3], r_len0 = wi[4], r_causal0 = wi[5];
   const int kend0 = r_len0 <= 0 ? 0 : (r_causal0 ? min(r_len0, q_off + q_len) : r_len0);
   const int r_start2 = work2[blockIdx.x * 2];
@@ -879,16 +885,16 @@ constexpr int DECODE_RING = 3;
 
 template <int HD>
 int launch_decode(dim3 grid, int ns, hipStream_t st, const half_t* qkv, half_t* out, const int* work, int nh, int nkv,
-                  int ld_qkv, int ld_out, float scale_log2, const half_t* kv0, int ld_kv0, const int* work2,
-                  const int* r2win, float* part) {
+                  int ld_qkv, int ld_out, float scale_log2, const half_t* kv0, int ld_kv0,
+                  const half_t* const* kv0_at, const int* work2, const int* r2win, float* part) {
   if (ns > 1) {
     hipLaunchKernelGGL((attn_decode<HD, true, DECODE_RING>), dim3(grid.x, grid.y, ns), dim3(256), 0, st, qkv, out,
-                       work, nh, nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, work2, r2win, part);
+                       work, nh, nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, kv0_at, work2, r2win, part);
     FLS_CHECK_LAUNCH();
     hipLaunchKernelGGL((attn_split_combine<HD>), dim3(grid.x, nh), dim3(HD), 0, st, part, out, work, nh, ld_out, ns);
   } else {
     hipLaunchKernelGGL((attn_decode<HD, false, DECODE_RING>), grid, dim3(256), 0, st, qkv, out, work, nh, nkv, ld_qkv,
-                       ld_out, scale_log2, kv0, ld_kv0, work2, r2win, nullptr);
+                       ld_out, scale_log2, kv0, ld_kv0, kv0_at, work2, r2win, nullptr);
   }
   FLS_CHECK_LAUNCH();
   return 0;
@@ -897,13 +903,13 @@ int launch_decode(dim3 grid, int ns, hipStream_t st, const half_t* qkv, half_t* 
 template <int HD, int WPH, bool R2>
 int launch(int hpb, dim3 grid, hipStream_t st, const half_t* qkv, half_t* out, const int* work, const int* seg_lo,
            int nh, int nkv, int ld_qkv, int ld_out, float scale_log2, const half_t* kv0, int ld_kv0,
-           const int* work2, const int* r2win, float* part, int ns) {
+           const half_t* const* kv0_at, const int* work2, const int* r2win, float* part, int ns) {
   if constexpr (R2 && HD != 96) {
     if (ns > 1) {
       const dim3 g3(grid.x, grid.y, ns);
 #define FLS_ATTN_LAUNCH_SPL(HPB_)                                                                              \
   hipLaunchKernelGGL((attn_fwd<HD, HPB_, WPH, true, true>), g3, dim3(64 * WPH * HPB_), 0, st, qkv, out, work, seg_lo, \
-                     nh, nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, work2, r2win, part)
+                     nh, nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, kv0_at, work2, r2win, part)
       if constexpr (WPH == 1) {
         if (hpb == 8) FLS_ATTN_LAUNCH_SPL(8);
         else FLS_ATTN_LAUNCH_SPL(4);
@@ -924,7 +930,7 @@ int launch(int hpb, dim3 grid, hipStream_t st, const half_t* qkv, half_t* out, c
   }
 #define FLS_ATTN_LAUNCH(HPB_)                                                                                  \
   hipLaunchKernelGGL((attn_fwd<HD, HPB_, WPH, R2>), grid, dim3(64 * WPH * HPB_), 0, st, qkv, out, work, seg_lo, nh, \
-                     nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, work2, r2win, nullptr)
+                     nkv, ld_qkv, ld_out, scale_log2, kv0, ld_kv0, kv0_at, work2, r2win, nullptr)
   if constexpr (HD == 96) {
     FLS_ATTN_LAUNCH(1);                     // 12 chunks per row: one head per block divides the tile
   } else if constexpr (WPH == 1) {          // 4 or 8 heads (dispatch)
@@ -1015,8 +1021,8 @@ extern "C" int fls_attention_set_split(int ns) {
 namespace {
 template <bool R2>
 int dispatch(const void* qkv, void* out, const int* work, int n_items, int n_q_heads, int n_kv_heads, int head_dim,
-             int ld_qkv, int ld_out, float scale, const void* kv0, int ld_kv0, const int* seg_lo, int q_block,
-             const int* work2, const int* r2win, void* ws, unsigned long long ws_bytes, int n_rows,
+             int ld_qkv, int ld_out, float scale, const void* kv0, int ld_kv0, const half_t* const* kv0_at,
+             const int* seg_lo, int q_block, const int* work2, const int* r2win, void* ws, unsigned long long ws_bytes, int n_rows,
              fls_stream_t s) {
   if (n_q_heads % n_kv_heads) return -2;
   if (head_dim != 64 && head_dim != 96 && head_dim != 128) return -3;
@@ -1042,9 +1048,9 @@ int dispatch(const void* qkv, void* out, const int* work, int n_items, int n_q_h
       auto o = (half_t*)out;
       auto k0 = (const half_t*)kv0;
       return head_dim == 128 ? launch_decode<128>(grid, ns, st, q, o, work, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                                  scale_log2, k0, ld_kv0, work2, r2win, (float*)ws)
+                                                  scale_log2, k0, ld_kv0, kv0_at, work2, r2win, (float*)ws)
                              : launch_decode<64>(grid, ns, st, q, o, work, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                                 scale_log2, k0, ld_kv0, work2, r2win, (float*)ws);
+                                                 scale_log2, k0, ld_kv0, kv0_at, work2, r2win, (float*)ws);
     }
   }
   if (q_block == 8) q_block = 32;           // hd 96 (or the non-range-2 kernel): the per-head layout
@@ -1090,35 +1096,37 @@ int dispatch(const void* qkv, void* out, const int* work, int n_items, int n_q_h
   if constexpr (R2) {
     if (q_block == 32)                      // head_dim 64 / 128 here (96 fell back above)
       return head_dim == 128 ? launch<128, 1, true>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv,
-                                                    ld_out, scale_log2, k0, ld_kv0, work2, r2win, part, ns)
+                                                    ld_out, scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns)
                              : launch<64, 1, true>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv,
-                                                   ld_out, scale_log2, k0, ld_kv0, work2, r2win, part, ns);
+                                                   ld_out, scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns);
   }
   if (head_dim == 96)
     return q_block == 64 ? launch<96, 2, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                         scale_log2, k0, ld_kv0, work2, r2win, part, ns)
+                                         scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns)
                          : launch<96, 4, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                         scale_log2, k0, ld_kv0, work2, r2win, part, ns);
+                                         scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns);
   if (q_block == 64)
     return head_dim == 128 ? launch<128, 2, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                            scale_log2, k0, ld_kv0, work2, r2win, part, ns)
+                                            scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns)
                            : launch<64, 2, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                           scale_log2, k0, ld_kv0, work2, r2win, part, ns);
+                                           scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns);
   return head_dim == 128 ? launch<128, 4, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                          scale_log2, k0, ld_kv0, work2, r2win, part, ns)
+                                          scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns)
                          : launch<64, 4, R2>(hpb, grid, st, q, o, work, seg_lo, n_q_heads, n_kv_heads, ld_qkv, ld_out,
-                                         scale_log2, k0, ld_kv0, work2, r2win, part, ns);
+                                         scale_log2, k0, ld_kv0, kv0_at, work2, r2win, part, ns);
 }
 }  // namespace
 
 extern "C" int fls_attention(const void* qkv, void* out, const int* work, int n_items, int n_q_heads,
                              int n_kv_heads, int head_dim, int ld_qkv, int ld_out, float scale, const void* kv0,
-                             int ld_kv0, const int* seg_lo, int q_block, const int* work2, const int* r2win,
-                             void* ws, unsigned long long ws_bytes, int n_rows, fls_stream_t s) {
+                             int ld_kv0, const void* const* kv0_at, const int* seg_lo, int q_block, const int* work2,
+                             const int* r2win, void* ws, unsigned long long ws_bytes, int n_rows, fls_stream_t s) {
   if (n_items <= 0) return 0;
-  if (work2 && (!kv0 || !r2win)) return -6;   // range 2 indexes the K/V cache, per-row windows
+  if (work2 && ((!kv0 && !kv0_at) || !r2win)) return -6;   // range 2 indexes the K/V cache, per-row windows
+  if (kv0_at && !work2) return -6;            // (captured steps are range-2 steps)
   return work2 ? dispatch<true>(qkv, out, work, n_items, n_q_heads, n_kv_heads, head_dim, ld_qkv, ld_out, scale, kv0,
-                                ld_kv0, seg_lo, q_block, work2, r2win, ws, ws_bytes, n_rows, s)
+                                ld_kv0, (const half_t* const*)kv0_at, seg_lo, q_block, work2, r2win, ws, ws_bytes,
+                                n_rows, s)
                : dispatch<false>(qkv, out, work, n_items, n_q_heads, n_kv_heads, head_dim, ld_qkv, ld_out, scale, kv0,
-                                 ld_kv0, seg_lo, q_block, nullptr, nullptr, nullptr, 0, 0, s);
+                                 ld_kv0, nullptr, seg_lo, q_block, nullptr, nullptr, nullptr, 0, 0, s);
 }

@@ -165,11 +165,13 @@ __global__ __launch_bounds__(256) void fold_norm_kernel(half_t* __restrict__ w, 
 }
 
 // y[dst_idx[r]] = x[src_idx[r]] for fp16 rows of H elements (a null index is the identity):
-// row gathers / scatters of the pruned last layer and the prefix K/V cache
+// row gathers / scatters of the pruned last layer and the prefix K/V cache (y_at: the device cell that holds y, as in fls_attention)
 __global__ __launch_bounds__(256) void copy_rows_kernel(const half_t* __restrict__ x, int ldx,
                                                       const int* __restrict__ src_idx, half_t* __restrict__ y, int ldy,
-                                                      const int* __restrict__ dst_idx, int H) {
+                                                      half_t* const* __restrict__ y_at, const int* __restrict__ dst_idx,
+                                                      int H) {
   const int r = blockIdx.x;
+  if (y_at != nullptr) y = *y_at;
   const half8* src = (const half8*)(x + (size_t)(src_idx ? src_idx[r] : r) * ldx);
   half8* dst = (half8*)(y + (size_t)(dst_idx ? dst_idx[r] : r) * ldy);
   for (int c = threadIdx.x; c < H / 8; c += 256) dst[c] = src[c];
@@ -549,12 +551,12 @@ extern "C" int fls_copy_d2d(void* dst, const void* src, uint64_t bytes, int mode
                         (hipStream_t)s) == hipSuccess ? 0 : -1;
 }
 
-extern "C" int fls_copy_rows(const void* x, int ldx, const int* src_idx, void* y, int ldy, const int* dst_idx,
-                             int rows, int H, fls_stream_t s) {
+extern "C" int fls_copy_rows(const void* x, int ldx, const int* src_idx, void* y, int ldy, void* const* y_at,
+                             const int* dst_idx, int rows, int H, fls_stream_t s) {
   if (rows <= 0) return 0;
   if (H % 8 || ldx % 8 || ldy % 8 || (((uintptr_t)x | (uintptr_t)y) & 15)) return -2;
   hipLaunchKernelGGL(copy_rows_kernel, dim3(rows), dim3(256), 0, (hipStream_t)s, (const half_t*)x, ldx, src_idx,
-                     (half_t*)y, ldy, dst_idx, H);
+                     (half_t*)y, ldy, (half_t* const*)y_at, dst_idx, H);
   FLS_CHECK_LAUNCH();
   return 0;
 }

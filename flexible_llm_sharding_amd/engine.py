@@ -1101,7 +1101,7 @@ class ShardedRunner:
     def _run_graphed(self, tps, batches, t_start: float, entry=None) -> List[Optional[np.ndarray]]:
         """Static-weights path: one graph replay per micro-batch (runtime/graphs.py): resident
         full forwards (``--hip_graphs``), or decode-like calls on the prefix / suffix K/V cache
-        ``entry`` (exact shapes; the graph reads and writes the entry's per-layer K/V in place).
+        ``entry`` (exact shapes; the graph reads and writes the per-layer K/V of the step's entry in place).
 
         Activations never leave HBM (there is no shard boundary inside the
         graph), so ``storage_location`` has nothing to park.
@@ -1114,8 +1114,6 @@ class ShardedRunner:
         if entry is not None:
             if getattr(self, "_decode_graphs", None) is None:
                 self._decode_graphs = DecodeGraphs(self.dev, self._forward_all)
-                if self.prefix_cache is not None:
-                    self.prefix_cache.on_evict.append(self._decode_graphs.forget)
             graphs = self._decode_graphs
             run = lambda b: graphs.run(b, entry)          # noqa: E731
         else:

@@ -414,6 +414,7 @@ def _attention_whole(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tens
     qkv = _attn_inputs(ctx, W, x, meta["positions"], meta["last_idx"], prune, meta["last_pos"],
                        ss_key=(id(batch), li - 1, "mlp", x.shape[0]))
     kv0 = None
+    kv_at = meta["kv_at"][layer_name] if "kv_at" in meta else None       # (captured: where a replay finds the layer's K/V)
     pe = ctx.prefix_entry
     if pe is not None:
         qs, kv = cfg.q_size, 2 * cfg.num_key_value_heads * cfg.head_dim
@@ -424,7 +425,7 @@ def _attention_whole(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tens
         if "sfx_src" in meta:                # the suffix rows computed now (suffix K/V reuse)
             if kv0 is None:
                 kv0 = pe.buffer(layer_name, create=True)
-            ops.copy_rows(qkv[:, qs:qs + kv], meta["sfx_src"], kv0, meta["sfx_dst"])
+            ops.copy_rows(qkv[:, qs:qs + kv], meta["sfx_src"], kv0, meta["sfx_dst"], **({} if kv_at is None else {"y_at": kv_at}))
             if pe.host:                      # host-mode entry: the new rows into its host buffer too
                 pe.write_rows(ops, qkv[:, qs:qs + kv], meta["sfx_src"], meta["sfx_dst"], layer_name)
     work_items = getattr(ops, "uses_work_items", False)
@@ -437,6 +438,8 @@ def _attention_whole(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tens
     if work_items and "work2" in meta:       # suffix K/V reuse: range 2 = the suffixes' kept rows
         kw["work2"] = meta["work2_last"] if prune else meta["work2"]
         kw["r2win"] = meta["r2win"]
+        if kv_at is not None:
+            kw["kv0_at"] = kv_at
     qb = batch.r2_q_block if "work2" in kw else batch.q_block     # (work_last items: one row each)
     a = ops.attention(qkv, attn_arg, cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim,
                       kv0=kv0 if batch.kv_cached else None, q_block=qb, out=qkv[:, :cfg.q_size],

@@ -15,6 +15,7 @@ from __future__ import annotations
 import os
 import threading
 from dataclasses import dataclass
+from typing import Optional
 
 import torch
 
@@ -256,8 +257,9 @@ class HipOps:
         _chk(self.k.fls_fold_norm(w.data_ptr(), w.stride(0), w.shape[0], w.shape[1], gamma.data_ptr(), _stream()),
              "fls_fold_norm")
 
-    def copy_rows(self, x, src_idx, y, dst_idx):
-        """y[dst_idx[r]] = x[src_idx[r]] (int32 CUDA indices; None = identity; rows of x.shape[1])."""
+    def copy_rows(self, x, src_idx, y, dst_idx, y_at: Optional[int] = None):
+        """y[dst_idx[r]] = x[src_idx[r]] (int32 CUDA indices; None = identity; rows of x.shape[1]).  ``y_at``: as ``kv0_at`` of
+        :meth:`attention`."""
         _f16(x, "x")
         _f16(y, "y")
         idx = src_idx if src_idx is not None else dst_idx
@@ -268,8 +270,8 @@ class HipOps:
             raise ValueError(f"row width mismatch {tuple(x.shape)} -> {tuple(y.shape)}")
         rows = idx.shape[0] if idx is not None else x.shape[0]
         _chk(self.k.fls_copy_rows(x.data_ptr(), x.stride(0), src_idx.data_ptr() if src_idx is not None else None,
-                                  y.data_ptr(), y.stride(0), dst_idx.data_ptr() if dst_idx is not None else None,
-                                  rows, x.shape[1], _stream()), "fls_copy_rows")
+                                  y.data_ptr() if y_at is None else None, y.stride(0), y_at,
+                                  dst_idx.data_ptr() if dst_idx is not None else None, rows, x.shape[1], _stream()), "fls_copy_rows")
         return y
 
     def copy_rows_to(self, x, src_idx, y_ptr: int, y_ld: int, dst_idx):
@@ -281,7 +283,7 @@ class HipOps:
                 raise TypeError("row indices must be int32 CUDA")
         if y_ld < x.shape[1]:
             raise ValueError("destination rows narrower than the source rows")
-        _chk(self.k.fls_copy_rows(x.data_ptr(), x.stride(0), src_idx.data_ptr(), y_ptr, y_ld, dst_idx.data_ptr(),
+        _chk(self.k.fls_copy_rows(x.data_ptr(), x.stride(0), src_idx.data_ptr(), y_ptr, y_ld, None, dst_idx.data_ptr(),
                                   src_idx.shape[0], x.shape[1], _stream()), "fls_copy_rows")
 
     def gather_rows(self, x, idx, out=None):
@@ -420,12 +422,14 @@ class HipOps:
 
     # ----------------------------------------------------------- attention
     def attention(self, qkv, work, n_q_heads, n_kv_heads, head_dim, kv0=None, q_block: int = 64, out=None,
-                  seg_lo=None, work2=None, r2win=None, scale=None):
+                  seg_lo=None, work2=None, r2win=None, scale=None, kv0_at: Optional[int] = None):
         """kv0 ([P, 2 * n_kv * hd], K then V): range 0 of every work item reads these rows (prefix cache).
         seg_lo ([T] int32, first row of each row's suffix): work items may span several suffixes.
         work2 ([n_items, 2] int32: r2_start, r2_len) + r2win ([T, 2] int32: kv0 rows [lo, hi) per row):
         range 2 = the kv0 rows of the item's suffixes cached by an earlier call (suffix K/V reuse),
-        walked between the prefix and the new rows, each row seeing its own suffix's window."""
+        walked between the prefix and the new rows, each row seeing its own suffix's window.
+        kv0_at (with work2): the address of a device cell from which the kernel takes kv0's address (a captured step, whose
+        later replays read other K/V of kv0's width)."""
         _f16(qkv, "qkv")
         if work.dtype != torch.int32 or not work.is_cuda:
             raise TypeError("work items must be an int32 CUDA tensor")
@@ -452,8 +456,8 @@ class HipOps:
         rc = self.k.fls_attention(qkv.data_ptr(), out.data_ptr(), work.data_ptr(), work.shape[0],
                                   n_q_heads, n_kv_heads, head_dim, qkv.stride(0), out.stride(0),
                                   head_dim ** -0.5 if scale is None else float(scale),
-                                  kv0.data_ptr() if kv0 is not None else None,
-                                  kv0.stride(0) if kv0 is not None else 0,
+                                  kv0.data_ptr() if kv0 is not None and kv0_at is None else None,
+                                  kv0.stride(0) if kv0 is not None else 0, kv0_at,
                                   seg_lo.data_ptr() if seg_lo is not None else None, q_block,
                                   work2.data_ptr() if work2 is not None else None,
                                   r2win.data_ptr() if work2 is not None else None,

@@ -111,7 +111,6 @@ class _Graph:
         self.graph = torch.cuda.CUDAGraph()
         self.out: torch.Tensor = None        # static device output [S, V]
         self.replays = 0
-        self.kv: frozenset = frozenset()     # DecodeGraphs: the addresses of the K/V buffers that the graph reads and writes
         self.arrays: Optional[_Arrays] = None      # DecodeGraphs: ``meta``'s places in ``flat``
         self.flat: Optional[torch.Tensor] = None
         self.staging: List[Tuple[Dict[str, np.ndarray], torch.Tensor, Optional[torch.cuda.Event]]] = []
@@ -178,12 +177,12 @@ class DecodeGraphs:
     each; one graph replays them all.
 
     Unlike :class:`GraphedForward` the shapes are EXACT (no bucket padding: a padded row would
-    also be captured into the suffix K/V cache), keyed by the batch's array shapes and the addresses of the cache
-    entry's per-layer K/V buffers, which the graph reads and writes in place; consecutive steps of
-    one generation have the same shapes, so one capture serves them all, and the steps of a later entry in the same buffers
-    (``PrefixKVCache.begin``): nothing else of an entry is in a graph, its rows come with each step's metadata.  The metadata of each
-    step (new token ids, positions, work items, cache rows and windows) is copied into the
-    graph's static inputs before the replay."""
+    also be captured into the suffix K/V cache), keyed by the batch's array shapes; consecutive steps of
+    one generation have the same shapes, so one capture serves them all, and the steps of other cache entries of the
+    same shapes: nothing of an entry is in a graph.  The metadata of each step (new token ids, positions, work items,
+    cache rows and windows, and the addresses of the entry's per-layer K/V buffers, which the kernels read and write in
+    place) is copied into the graph's static inputs before the replay.  (A capture is 3 ms of a generation's 21: 16 steps
+    of 16 rows through four 7B layers.)"""
 
     def __init__(self, device, forward: Callable, max_graphs: int = 4):
         self.dev = torch.device(device)
@@ -196,23 +195,20 @@ class DecodeGraphs:
 
     @staticmethod
     def key(batch: PackedBatch, entry) -> tuple:
-        """The device address of every per-layer K/V buffer that the graph reads and writes, and the step's shapes."""
-        ptrs = tuple((n, t.data_ptr()) for n, t in sorted(entry.layers.items()))
-        return (ptrs, batch.r2_q_block, batch.q_block) + tuple(
+        """The layers whose K/V the graph reads and writes, and the step's shapes."""
+        return (tuple(entry.layers), batch.r2_q_block, batch.q_block) + tuple(
             (k, v.shape) for k, v in sorted(batch.host_meta().items()))
 
-    def forget(self, entry) -> None:
-        """Drop every graph captured on ``entry``'s buffers (called when the prefix cache frees them: a replay would read / write
-        freed HBM)."""
-        freed = {t.data_ptr() for held in (entry.memory, entry.spare) for t in held.values()}
-        for k in [k for k, g in self.graphs.items() if g.kv & freed]:
-            del self.graphs[k]
+    @staticmethod
+    def _put_addresses(words: np.ndarray, entry) -> None:
+        """``words``: the int32 head of a step's arrays, 64 bits a layer in the key's order."""
+        words[:2 * len(entry.layers)].view(np.int64)[:] = [t.data_ptr() for t in entry.layers.values()]
 
     # pinned staging sets per graph: a replay may be enqueued while the previous one (and its
     # metadata copies) still runs, so a set is refilled only after the copies that read it ran
     STAGING_SETS = 2
 
-    def _upload(self, g: _Graph, host: Dict[str, np.ndarray]) -> None:
+    def _upload(self, g: _Graph, host: Dict[str, np.ndarray], entry) -> None:
         """One stream-ordered copy of all metadata from the graph's persistent pinned staging buffers (with a copy for each of
         the 12 arrays, 17 steps of 16 rows through four 7B layers took 22.3 ms, with one 21.3)."""
         if not g.staging:
@@ -224,6 +220,7 @@ class DecodeGraphs:
             ev.synchronize()                                 # the copy that last read this set ran
         for k, v in host.items():
             np.copyto(views[k], v, casting="no")
+        self._put_addresses(pinned.numpy(), entry)
         g.flat.copy_(pinned, non_blocking=True)
         ev = torch.cuda.Event()
         ev.record(torch.cuda.current_stream(self.dev))
@@ -242,17 +239,18 @@ class DecodeGraphs:
         if g is None:
             if len(self.graphs) >= self.max_graphs:
                 self.graphs.popitem(last=False)
-            arrays = _Arrays(host)
+            arrays = _Arrays(host, _ceil(2 * len(entry.layers), 16))
             up = np.zeros(arrays.size, np.int32)
             for k, dst in arrays.views(up).items():
                 np.copyto(dst, host[k], casting="no")
+            self._put_addresses(up, entry)
             flat = torch.from_numpy(up).to(self.dev)
             meta = arrays.views(flat)
+            meta["kv_at"] = {name: flat.data_ptr() + 8 * i for i, name in enumerate(entry.layers)}
             if ids_dev is not None:
                 meta["ids"].copy_(ids_dev)
             g = _Graph(meta)
             g.arrays, g.flat = arrays, flat
-            g.kv = frozenset(p for _, p in key[0])
             s = torch.cuda.Stream(self.dev)
             s.wait_stream(torch.cuda.current_stream(self.dev))
             with torch.cuda.stream(s):
@@ -266,7 +264,7 @@ class DecodeGraphs:
             self.graphs[key] = g
             return eager
         self.graphs.move_to_end(key)
-        self._upload(g, host)
+        self._upload(g, host, entry)
         if ids_dev is not None:
             g.meta["ids"].copy_(ids_dev, non_blocking=True)
         g.graph.replay()

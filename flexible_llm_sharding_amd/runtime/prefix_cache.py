@@ -74,8 +74,7 @@ class PrefixEntry:
     REGION_ALIGN = 64      # attention key tile (csrc/kernels/attention.hip KT)
 
     def __init__(self, key: str, prefix_lens: Sequence[int], kv_cols: int, device, dtype,
-                 suffix_caps: Optional[Sequence[Sequence[int]]] = None, stage: Optional["HostStage"] = None,
-                 spare: Optional[Dict[str, torch.Tensor]] = None):
+                 suffix_caps: Optional[Sequence[Sequence[int]]] = None, stage: Optional["HostStage"] = None):
         self.key = key
         self.offsets: List[int] = []
         t = 0
@@ -101,9 +100,6 @@ class PrefixEntry:
         self.dev = torch.device(device)
         self.dtype = dtype
         self.layers: Dict[str, torch.Tensor] = {}
-        # device mode: the memory behind ``layers``, and an evicted entry's that this one takes over layer by layer
-        self.memory: Dict[str, torch.Tensor] = {}
-        self.spare: Dict[str, torch.Tensor] = spare if spare is not None else {}
         self.complete = False
         self.stage = stage            # host mode: the cache's staging buffers
         self._staged: Optional[tuple] = None     # (layer name, staging view) of the layer in flight
@@ -117,26 +113,11 @@ class PrefixEntry:
             return self._stage_in(layer_name, create)
         b = self.layers.get(layer_name)
         if b is None and create:
-            m = self.spare.pop(layer_name, None)
-            if m is None:
-                m = torch.empty(self.room(), self.kv_cols, dtype=self.dtype, device=self.dev)
             # zeroed: a reused step's key tiles cover the alignment gaps and unused region rows (masked,
             # P = 0 exactly, and 0 x a finite V adds nothing)
-            m.zero_()
-            self.memory[layer_name] = m
-            b = self.layers[layer_name] = m[:max(1, self.rows)]
+            b = torch.zeros(max(1, self.rows), self.kv_cols, dtype=self.dtype, device=self.dev)
+            self.layers[layer_name] = b
         return b
-
-    def room(self) -> int:
-        """Rows of a layer's memory: the entry's, up to the next quarter of a power of two, so that an entry a little larger
-        can take the memory over."""
-        n = max(1, self.rows)
-        step = max(self.REGION_ALIGN, 1 << max(0, n.bit_length() - 3))
-        return -(-n // step) * step
-
-    def can_take(self, memory: Dict[str, torch.Tensor]) -> bool:
-        """Does another entry's memory fit this one, without keeping more than four times what it needs?"""
-        return bool(memory) and all(self.rows <= m.shape[0] <= 4 * self.room() for m in memory.values())
 
     def _stage_in(self, layer_name: str, create: bool) -> Optional[torch.Tensor]:
         if self._staged is not None and self._staged[0] == layer_name:
@@ -337,8 +318,7 @@ class PrefixKVCache:
         self.entries: "OrderedDict[str, PrefixEntry]" = OrderedDict()
         self.hits = 0
         self.misses = 0
-        # called with an entry that leaves the cache and whose K/V buffers are freed with it: graphs
-        # captured on them must go first (runtime/graphs.py DecodeGraphs.forget)
+        # called with an entry that leaves the cache (its K/V buffers are freed with it)
         self.on_evict: List = []
 
     def _evict(self, e: Optional[PrefixEntry]) -> None:
@@ -381,23 +361,15 @@ class PrefixKVCache:
         return None
 
     def begin(self, tps: Sequence) -> PrefixEntry:
-        """A fresh entry the coming full pass fills (replaces any partial one).  In device mode it takes over the K/V buffers of an
-        entry that it evicts, where they fit: graphs captured on them then serve its steps too (a capture is 3 ms of a
-        generation's 21: 16 steps of 16 rows through four 7B layers)."""
+        """A fresh entry the coming full pass fills (replaces any partial one)."""
         key = prefix_fingerprint(tps)
-        gone = [e for e in (self.entries.pop(key, None),) if e is not None]
+        self._evict(self.entries.pop(key, None))
         while len(self.entries) >= self.max_entries:
-            gone.append(self.entries.popitem(last=False)[1])
+            self._evict(self.entries.popitem(last=False)[1])
         caps = ([[len(s) + self.suffix_growth for s in tp.suffixes] for tp in tps] if self.suffix_reuse else None)
         self.ensure_stage(tps)
         e = PrefixEntry(key, [len(tp.prefix) for tp in tps], self.kv_cols, self.dev, self.dtype, caps,
                         stage=self.stage)
-        heir = None if self.host else next((g for g in gone if g.complete and not g.spare and e.can_take(g.memory)), None)
-        if heir is not None:
-            e.spare, heir.memory, heir.layers = heir.memory, {}, {}
-        for g in gone:
-            if g is not heir:
-                self._evict(g)
         self.entries[key] = e
         return e
 

@@ -491,38 +491,27 @@ def test_row_exact_packing_and_regions():
     assert buf.shape[0] >= starts[-1] + 94 and not buf.any()
 
 
-def test_evicted_prefix_buffers_are_taken_over():
-    """One entry at a time: the next one's layers lie in the evicted one's memory where that fits, zeroed; one that is too small or more than
-    four times too large is freed, and so is an incomplete entry's, both reported to on_evict."""
+def test_prefix_entries_hold_what_the_plan_reserves():
+    """Entries of many sizes through a cache of two: each layer's memory is the entry's rows and no more (the planner reserves those), zeroed, and
+    an entry that leaves gives its own back."""
+    import gc
+    import weakref
+
     from flexible_llm_sharding_amd.runtime.prefix_cache import PrefixKVCache
     from flexible_llm_sharding_amd.utils.tokenizer import TokenizedPrompt
-    tps = lambda n: [TokenizedPrompt(list(range(3, 3 + n)), [[5, 6, 7]], 3, [2])]
-    pc, gone, names = PrefixKVCache(16, "cpu", torch.float16, max_entries=1), [], ("model.layers.0", "model.layers.1")
-    pc.on_evict.append(lambda e: gone.append(e))
-
-    def fill(n, complete=True):
-        e = pc.begin(tps(n))
-        bufs = [e.buffer(k, create=True) for k in names]
-        assert all(tuple(b.shape) == (e.rows, 16) and not b.any() for b in bufs)
-        for b in bufs:
+    pc, names, refs = PrefixKVCache(16, "cpu", torch.float16, max_entries=2), ("model.layers.0", "model.layers.1"), []
+    for n in (700, 650, 705, 5000, 40, 41, 1300, 1299):
+        e = pc.begin([TokenizedPrompt(list(range(3, 3 + n)), [[5, 6, 7]], 3, [2])])
+        for k in names:
+            b = e.buffer(k, create=True)
+            assert tuple(b.shape) == (e.rows, 16) and not b.any() and b.untyped_storage().nbytes() == e.rows * 32
             b.fill_(1.0)
-        e.complete = complete
-        return e, [b.data_ptr() for b in bufs]
-
-    e1, at1 = fill(700)
-    e2, at2 = fill(650)
-    assert at2 == at1 and not gone and not e1.layers and not e1.memory
-    e3, at3 = fill(e1.room() - 64 * 3)                               # (prefix and suffix region: the room to the last row)
-    assert at3 == at1 and not gone
-    e4, at4 = fill(5000)
-    assert at4 != at1 and gone == [e3]
-    e5, _ = fill(40)
-    assert gone == [e3, e4]
-    e6, at6 = fill(41, complete=False)
-    e7, at7 = fill(41)
-    assert gone[-1] is e6 and len(gone) == 3
-    pc.drop(e7)
-    assert gone[-1] is e7 and not pc.entries
+            refs.append(weakref.ref(b))
+        e.complete = True
+        assert pc.nbytes == sum(len(names) * x.rows * 32 for x in pc.entries.values()) and len(pc.entries) <= 2
+        del b
+        gc.collect()
+        assert sum(r() is not None for r in refs) == len(names) * len(pc.entries)
 
 
 def _host_mode(r):

@@ -760,8 +760,12 @@ def _suffix_rows_from_cache(ops, ref, nh, nkv, hd, prompts=None, keep=None, q_bl
     m = reuse.device_tensors(DEV)
     if q_block == 32:                                     # one wave per head: items of <= 32 rows
         q_block = 32 if int(reuse.work[:, 1].max()) <= 32 else 64
-    y = ops.attention(qkv_new.to(DEV), m["work"], nh, nkv, hd, kv0=cache.to(DEV), seg_lo=m["seg_lo"],
-                      work2=m["work2"], r2win=m["r2win"], q_block=q_block)
+    kv0, kw = cache.to(DEV), dict(seg_lo=m["seg_lo"], work2=m["work2"], r2win=m["r2win"], q_block=q_block)
+    y = ops.attention(qkv_new.to(DEV), m["work"], nh, nkv, hd, kv0=kv0, **kw)
+    # (the cache's address from a cell on the device: the same kernel, the same bits)
+    cells = torch.tensor([0, kv0.data_ptr()], dtype=torch.int64, device=DEV)
+    assert torch.equal(ops.attention(qkv_new.to(DEV), m["work"], nh, nkv, hd, kv0=torch.full_like(kv0, float("nan")),
+                                     kv0_at=cells.data_ptr() + 8, **kw), y)
     want = ref.attention(qkv.float(), full.segments, nh, nkv, hd)[sel]
     got_ref = ref.attention(qkv_new.float(), reuse.segments, nh, nkv, hd, kv0=cache.float())
     torch.cuda.synchronize()
@@ -1056,7 +1060,11 @@ def test_copy_rows(ops):
     ops.scatter_rows(g, dst, y)
     z = torch.zeros(40, 512, dtype=torch.float16, device=DEV)
     ops.copy_rows(x[:, 1024:1536], src, z, dst)            # strided source columns
+    z2, other = torch.zeros_like(z), torch.zeros_like(z)
+    cell = torch.tensor([z2.data_ptr()], dtype=torch.int64, device=DEV)
+    ops.copy_rows(x[:, 1024:1536], src, other, dst, y_at=cell.data_ptr())       # (the address from a cell on the device)
     torch.cuda.synchronize()
+    assert torch.equal(z2, z) and not other.any()
     assert torch.equal(g, x[src.long()])
     want = torch.zeros_like(y)
     want[dst.long()] = x[src.long()]
