@@ -2,7 +2,7 @@
 
 ``kernels()`` / ``runtime()`` raise if the library is missing — on a GPU the
 HIP path must be the one that runs (no silent fallback); CPU-only code paths
-call ``runtime_or_none()``.
+call ``runtime_or_none()`` and ``host_or_none()``.
 """
 from __future__ import annotations
 
@@ -52,6 +52,11 @@ def host():
     if _host is None:
         _host = _fastcall()
     return _host
+
+
+def host_or_none():
+    """:func:`host`, or None where the extension is not built: packing for the CPU backend needs numpy only (a GPU's libraries do not load without it)."""
+    return host() if _host is not None or os.path.exists(_FASTCALL) else None
 
 
 class _Quick:

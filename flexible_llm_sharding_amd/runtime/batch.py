@@ -47,13 +47,31 @@ WORK_ITEM_FIELDS = 8    # q_start q_len q_off r0_start r0_len r0_causal r1_start
 def _token_ids(parts: Sequence[Sequence[int]]) -> np.ndarray:
     """The parts' token ids one after the other, int32."""
     lens = [len(p) for p in parts]
-    out, at, int32s = np.empty(sum(lens), dtype=np.int32), 0, _native.host().int32s
+    out, at, host = np.empty(sum(lens), dtype=np.int32), 0, _native.host_or_none()
     for p, n in zip(parts, lens):
         part = out[at:at + n]
-        if not int32s(part, p):
+        if host is None or not host.int32s(part, p):
             part[...] = np.asarray(p, dtype=np.int32)
         at += n
     return out
+
+
+def _step_rows(cu: np.ndarray, pos0: np.ndarray, table: np.ndarray, page_size: int):
+    """-> (request, position and place in the page pools of every row, or None if a row's page is not in the table), int32: request b's rows
+    ``cu[b] .. cu[b + 1] - 1`` continue it from position ``pos0[b]``."""
+    host = _native.host_or_none()
+    if host is not None:
+        seq, pos, slot = (np.empty(int(cu[-1]), dtype=np.int32) for _ in range(3))
+        return (seq, pos, slot) if host.step_rows(cu, pos0, table, page_size, seq, pos, slot) else None
+    seq = np.repeat(np.arange(len(pos0), dtype=np.int64), np.diff(cu))
+    pos = np.arange(cu[-1], dtype=np.int64) - cu[seq] + pos0[seq]
+    at = pos // page_size
+    if at.size and at.max() >= table.shape[1]:
+        return None
+    pages = table[seq, at].astype(np.int64)
+    if (pages < 0).any():
+        return None
+    return tuple(a.astype(np.int32) for a in (seq, pos, pages * page_size + pos % page_size))
 
 
 def _table(rows: Sequence[Sequence[int]], width: int) -> np.ndarray:
@@ -561,9 +579,10 @@ def pack_step(entries: Sequence[StepEntry], cache) -> StepBatch:
     T = cu[-1]
     i32 = lambda a: np.asarray(a, dtype=np.int32)
     cu_a, pos0_a = i32(cu), i32(pos0)
-    seq, pos, kv_slot = (np.empty(T, dtype=np.int32) for _ in range(3))
-    if not _native.host().step_rows(cu_a, pos0_a, table, cache.page_size, seq, pos, kv_slot):
+    rows = _step_rows(cu_a, pos0_a, table, cache.page_size)
+    if rows is None:
         raise RuntimeError("a new token's page is missing from the page table")
+    seq, pos, kv_slot = rows
     prev = None
     if before:                                              # (each row's token before it: the row above, a request's first row its last one)
         prev = np.empty(T, dtype=np.int32)

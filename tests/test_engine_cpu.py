@@ -1056,3 +1056,56 @@ def test_one_token_steps_pack_like_portions(tmp_path, family):
         for more in ([], [StepEntry("other", [1, 2])]):
             with pytest.raises(ValueError, match="lies outside its 1 tokens"):
                 pack_step([StepEntry("x", [3], [bad])] + more, alone)
+
+
+def test_packing_without_the_extension(monkeypatch, tmp_path):
+    """Prompts and steps pack for the CPU where the native extension is not built, to the same arrays, and holes in a page table are still refused."""
+    import dataclasses
+
+    from flexible_llm_sharding_amd import _native
+    from flexible_llm_sharding_amd.runtime import batch as B
+    from flexible_llm_sharding_amd.utils.tokenizer import TokenizedPrompt
+    rng = np.random.default_rng(3)
+    ids = lambda n: rng.integers(3, 500, n).tolist()
+    tps = [TokenizedPrompt(p, ss, max(map(len, ss)), [len(s) - 1 for s in ss]) for p, ss in
+           ((ids(70), [ids(5), ids(80), ids(1)]), (ids(130), [ids(65)]), (ids(2), [ids(3), np.asarray(ids(140))]))]
+
+    class Pages:
+        page_size, prev_token, block_sizes = 16, True, ()
+
+        def __init__(self, hole):
+            self.at, self.hole = {"a": 0, "b": 37, "c": 5}, hole
+
+        def extend(self, rid, n):
+            p0 = self.at[rid]
+            self.at[rid] += n
+            return p0, ord(rid) - ord("a")
+
+        def advance_token(self, rid, token):
+            return 7
+
+        def page_table(self, rids):
+            t = np.random.default_rng(1).permutation(60).reshape(3, 20).astype(np.int32)
+            if self.hole:
+                t[1, 3] = -1
+            return t
+
+    steps = [B.StepEntry("a", ids(200), [199]), B.StepEntry("b", ids(33), [0, 32]), B.StepEntry("c", ids(1), [])]
+
+    def packed():
+        out = [B.pack_prompts(tps, [0, 1, 2], "causal"), B.pack_step(steps, Pages(False))]
+        with pytest.raises(RuntimeError, match="page table"):
+            B.pack_step(steps, Pages(True))
+        return [dataclasses.asdict(b) for b in out]
+
+    native = packed()
+    monkeypatch.setattr(_native, "_FASTCALL", str(tmp_path / "absent.so"))
+    monkeypatch.setattr(_native, "_host", None)
+    plain = packed()
+    for a, b in zip(native, plain):
+        assert a.keys() == b.keys()
+        for k in a:
+            if isinstance(a[k], np.ndarray):
+                assert a[k].dtype == b[k].dtype and np.array_equal(a[k], b[k]), k
+            else:
+                assert repr(a[k]) == repr(b[k]), k
