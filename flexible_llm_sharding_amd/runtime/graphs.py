@@ -29,6 +29,7 @@ from __future__ import annotations
 
 import contextlib
 import gc
+import threading
 from collections import OrderedDict
 from typing import Callable, Dict, List, Optional, Tuple
 
@@ -91,18 +92,35 @@ class _Arrays:
         return out
 
 
+class _CollectorHeld:
+    """Python's automatic collections off while any thread is in the context; when the last one leaves they are as the first one found them."""
+
+    def __init__(self):
+        self.lock, self.holders, self.collects = threading.Lock(), 0, False
+
+    def __enter__(self):
+        with self.lock:
+            if self.holders == 0:
+                self.collects = gc.isenabled()
+            self.holders += 1
+            gc.disable()
+
+    def __exit__(self, *exc):
+        with self.lock:
+            self.holders -= 1
+            if self.holders == 0 and self.collects:
+                gc.enable()
+
+
+_collector_held = _CollectorHeld()
+
+
 @contextlib.contextmanager
 def _capturing(graph: torch.cuda.CUDAGraph, pool, stream):
-    """Capture into ``graph`` without Python's automatic collections: one could free what a runner left in a cycle (pinned memory, events, graphs),
+    """Capture into ``graph`` without automatic collections: one could free what a runner left in a cycle (pinned memory, events, graphs),
     which is an error while a stream captures."""
-    collects = gc.isenabled()
-    gc.disable()
-    try:
-        with torch.cuda.graph(graph, pool=pool, stream=stream):
-            yield
-    finally:
-        if collects:
-            gc.enable()
+    with _collector_held, torch.cuda.graph(graph, pool=pool, stream=stream):
+        yield
 
 
 class _Graph:

@@ -1109,3 +1109,39 @@ def test_packing_without_the_extension(monkeypatch, tmp_path):
                 assert a[k].dtype == b[k].dtype and np.array_equal(a[k], b[k]), k
             else:
                 assert repr(a[k]) == repr(b[k]), k
+
+
+def test_captures_of_two_threads_hold_the_collector(monkeypatch):
+    """Python's collector stays off until the last of two overlapping captures is done, whichever began first, also where a capture fails; it is then as
+    it was before the first."""
+    import contextlib
+    import gc
+    import threading
+
+    from flexible_llm_sharding_amd.runtime import graphs
+    monkeypatch.setattr(torch.cuda, "graph", lambda *a, **k: contextlib.nullcontext())
+    was = gc.isenabled()
+    try:
+        for enabled in (True, False):
+            for fails in (False, True):
+                (gc.enable if enabled else gc.disable)()
+                inside, leave, seen = threading.Event(), threading.Event(), []
+
+                def other():
+                    with contextlib.suppress(KeyError), graphs._capturing(None, None, None):
+                        inside.set()
+                        leave.wait(10)
+                        seen.append(gc.isenabled())
+                        if fails:
+                            raise KeyError
+
+                with graphs._capturing(None, None, None):
+                    t = threading.Thread(target=other)
+                    t.start()
+                    assert inside.wait(10) and not gc.isenabled()
+                assert not gc.isenabled()                    # (the first one left: the other still captures)
+                leave.set()
+                t.join()
+                assert seen == [False] and gc.isenabled() == enabled
+    finally:
+        (gc.enable if was else gc.disable)()
