@@ -49,7 +49,18 @@ template <typename TA, typename TW, int XR, int HW> struct Ring {
   static constexpr int NST = stages_in(20480, STAGE), FEW = stages_in(10240, STAGE);
 };
 
-template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
+// 16 bytes of a row, zeros where the offset is out of range
+__device__ __forceinline__ floatx4 load16(__amdgpu_buffer_rsrc_t rs, unsigned off, int k0) {
+  return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, off, k0, 0));
+}
+__device__ __forceinline__ bf16x8 rounded(const floatx4& lo, const floatx4& hi) {       // fp32 rows against bf16 weights
+  typedef float floatx8 __attribute__((ext_vector_type(8)));
+  return __builtin_convertvector((floatx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), bf16x8);
+}
+
+// U > 0: operands straight to registers.  A short K is one chunk of U steps a wave, whose loads are all issued before the first product; what
+// counts there is the chain of one load, and the way through LDS adds to it: 8 rows x 11808 x 224 4.0 us so, 4.4 by the rings.
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED, int U>
 __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
                                         const int* offs, const int* a_rows, long long w_gs, int nst) {
   typedef typename Step<TW>::V V;
@@ -74,7 +85,9 @@ __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const
   // DMA pieces of 1 KB: 8 rows of 128 bytes, 16-byte chunk c of row r in place c ^ (r & 7) (rows of A of twice the size: 4 rows, c ^ (r & 15))
   const int lr = lane >> 3, lc = (lane & 7) ^ lr;
   const int kb = K * (int)sizeof(TW), stages = (kb + 127) / 128, mine = (stages - wave + WV - 1) / WV;
-  char* const ring = smem + wave * (nst * STAGE);
+  constexpr int SUMS = MG * HW * 1024;
+  const int share = U > 0 ? SUMS : nst * STAGE;            // of LDS, a wave's
+  char* const ring = smem + wave * share;
   __amdgpu_buffer_rsrc_t rw[HW];
   unsigned wo[HW][2];
 #pragma unroll
@@ -83,90 +96,119 @@ __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const
     const TW* p = W + (size_t)(n1 + (GATED && (h & 1) ? N : 0)) * ldw;
     rw[h] = rsrc_of(p);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) wo[h][j] = (unsigned)min(8 * j + lr, N - 1 - n1) * ldw * (unsigned)sizeof(TW) + lc * 16;
+    for (int j = 0; j < 2; ++j)
+      wo[h][j] = (unsigned)min(U > 0 ? fr : 8 * j + lr, N - 1 - n1) * ldw * (unsigned)sizeof(TW) + (U > 0 ? grp : lc) * 16;
   }
   const __amdgpu_buffer_rsrc_t ra = rsrc_of(A);
   const bool few = XR == 16 && M <= 8;                     // (a row group: half of its stages' pieces of A)
-  auto red = [&](int w, int at, int l) -> floatx4& { return *reinterpret_cast<floatx4*>(smem + w * (nst * STAGE) + (at * 64 + l) * 16); };
-  static_assert(MG * HW * 1024 <= STAGE, "a wave's sums fit its ring");
+  auto red = [&](int w, int at, int l) -> floatx4& { return *reinterpret_cast<floatx4*>(smem + w * share + (at * 64 + l) * 16); };
+  static_assert(SUMS <= STAGE, "a wave's sums fit its ring");
   for (int m0 = 0; m0 < M; m0 += 16 * MG) {
-    unsigned xo[XA];
-#pragma unroll
-    for (int i = 0; i < XA; ++i) {
-      const int row = XS == 1 ? 8 * i + lr : 4 * i + (lane >> 4), r = min(m0 + row, M - 1);
-      xo[i] = (unsigned)(a_rows != nullptr ? a_rows[r] : r) * lda * (unsigned)sizeof(TA) + (XS == 1 ? lc * 16 : ((lane ^ row) & 15) * 16);
-    }
     floatx4 acc[2][HW][MG];                // (the two steps of a tile in sums of their own, which rounds less)
 #pragma unroll
     for (int u = 0; u < MG; ++u)
 #pragma unroll
       for (int h = 0; h < HW; ++h) acc[0][h][u] = acc[1][h][u] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto fill = [&](int t, char* stg) {    // the wave's t-th stage (chunks past K: zeros)
-      const int k0 = (wave + t * WV) * 128;
-      const bool cut = k0 + 128 > kb;
-      const unsigned none = cut && k0 + lc * 16 >= kb ? 0x80000000u : 0u;
+    if constexpr (U > 0) {
+      unsigned xo[MG];
 #pragma unroll
-      for (int h = 0; h < HW; ++h)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) R_DMA(rw[h], wo[h][j] | none, k0, stg + (2 * h + j) * 1024);
-#pragma unroll
-      for (int i = 0; i < XA; ++i) {
-        unsigned no = none;
-        if (XS == 2) no = cut && k0 * 2 + (((lane ^ (4 * i + (lane >> 4))) & 15) * 16) >= kb * 2 ? 0x80000000u : 0u;
-        if (!(few && i >= XA / 2)) R_DMA(ra, xo[i] | no, k0 * XS, stg + R::SW + i * 1024);
+      for (int u = 0; u < MG; ++u) {       // (rows past M: zeros, no loads)
+        const int row = m0 + u * 16 + fr, r = min(row, M - 1);
+        xo[u] = row < M ? (unsigned)(a_rows != nullptr ? a_rows[r] : r) * lda * (unsigned)sizeof(TA) + grp * (16 * XS) : 0x80000000u;
       }
-    };
+      V w[HW][U], x[MG][U];
 #pragma unroll
-    for (int t = 0; t < NST; ++t)
-      if (t < min(nst, mine)) fill(t, ring + t * STAGE);
-    char* stg = ring;
-    for (int t = 0; t < mine; ++t) {
-      const int after = min(nst - 1, mine - 1 - t);        // stages that may stay in flight
-      asm volatile("" ::: "memory");
-#define R_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | ((n) >> 4) << 14 | 0x0f70)
-      if (after == 0) R_VM(0);
-#define R_WAIT(n)                            \
-  else if (NST > n && after == n) {          \
-    if (few) R_VM(n * (CNT - XA / 2));       \
-    else R_VM(n * CNT);                      \
-  }
-      R_WAIT(1)
-      R_WAIT(2)
-      R_WAIT(3)
-      R_WAIT(4)
-      R_WAIT(5)
-#undef R_WAIT
-#undef R_VM
-      asm volatile("" ::: "memory");
-      V w[HW][2], x[MG][2];
+      for (int i = 0; i < U; ++i) {        // steps of 64 bytes of a row of W
+        const int k0 = (wave * U + i) * 64;
+        const unsigned none = k0 + grp * 16 >= kb ? 0x80000000u : 0u;
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int c = ((4 * k + grp) ^ (fr & 7)) << 4;
-#pragma unroll
-        for (int h = 0; h < HW; ++h) w[h][k] = *reinterpret_cast<const V*>(stg + h * 2048 + fr * 128 + c);
+        for (int h = 0; h < HW; ++h) w[h][i] = __builtin_bit_cast(V, load16(rw[h], wo[h][0] | none, k0));
 #pragma unroll
         for (int u = 0; u < MG; ++u) {
-          const int r = min(u * 16 + fr, XR - 1);         // (rows past M: columns that are not stored)
-          if constexpr (XS == 1) {
-            x[u][k] = *reinterpret_cast<const V*>(stg + R::SW + r * 128 + (((4 * k + grp) ^ (r & 7)) << 4));
-          } else {
-            typedef float floatx8 __attribute__((ext_vector_type(8)));
-            const char* row = stg + R::SW + r * 256;
-            const int a = 8 * k + 2 * grp, sw = r & 15;
-            const floatx4 lo = *(const floatx4*)(row + ((a ^ sw) << 4)), hi = *(const floatx4*)(row + (((a + 1) ^ sw) << 4));
-            x[u][k] = __builtin_convertvector((floatx8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]}), V);
-          }
+          const floatx4 lo = load16(ra, xo[u] | none, k0 * XS);
+          if constexpr (XS == 1) x[u][i] = __builtin_bit_cast(V, lo);
+          else x[u][i] = rounded(lo, load16(ra, (xo[u] + 16) | none, k0 * XS));
         }
       }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      if (t + nst < mine) fill(t + nst, stg);
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+      for (int i = 0; i < U; ++i)
 #pragma unroll
         for (int u = 0; u < MG; ++u)
 #pragma unroll
-          for (int h = 0; h < HW; ++h) acc[k][h][u] = mfma_step(w[h][k], x[u][k], acc[k][h][u]);
-      stg = stg + STAGE == ring + nst * STAGE ? ring : stg + STAGE;
+          for (int h = 0; h < HW; ++h) acc[i & 1][h][u] = mfma_step(w[h][i], x[u][i], acc[i & 1][h][u]);
+    } else {
+      unsigned xo[XA];
+#pragma unroll
+      for (int i = 0; i < XA; ++i) {
+        const int row = XS == 1 ? 8 * i + lr : 4 * i + (lane >> 4), r = min(m0 + row, M - 1);
+        xo[i] = (unsigned)(a_rows != nullptr ? a_rows[r] : r) * lda * (unsigned)sizeof(TA) + (XS == 1 ? lc * 16 : ((lane ^ row) & 15) * 16);
+      }
+      auto fill = [&](int t, char* stg) {    // the wave's t-th stage (chunks past K: zeros)
+        const int k0 = (wave + t * WV) * 128;
+        const bool cut = k0 + 128 > kb;
+        const unsigned none = cut && k0 + lc * 16 >= kb ? 0x80000000u : 0u;
+#pragma unroll
+        for (int h = 0; h < HW; ++h)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) R_DMA(rw[h], wo[h][j] | none, k0, stg + (2 * h + j) * 1024);
+#pragma unroll
+        for (int i = 0; i < XA; ++i) {
+          unsigned no = none;
+          if (XS == 2) no = cut && k0 * 2 + (((lane ^ (4 * i + (lane >> 4))) & 15) * 16) >= kb * 2 ? 0x80000000u : 0u;
+          if (!(few && i >= XA / 2)) R_DMA(ra, xo[i] | no, k0 * XS, stg + R::SW + i * 1024);
+        }
+      };
+#pragma unroll
+      for (int t = 0; t < NST; ++t)
+        if (t < min(nst, mine)) fill(t, ring + t * STAGE);
+      char* stg = ring;
+      for (int t = 0; t < mine; ++t) {
+        const int after = min(nst - 1, mine - 1 - t);        // stages that may stay in flight
+        asm volatile("" ::: "memory");
+#define R_VM(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | ((n) >> 4) << 14 | 0x0f70)
+        if (after == 0) R_VM(0);
+#define R_WAIT(n)                            \
+    else if (NST > n && after == n) {          \
+      if (few) R_VM(n * (CNT - XA / 2));       \
+      else R_VM(n * CNT);                      \
+    }
+        R_WAIT(1)
+        R_WAIT(2)
+        R_WAIT(3)
+        R_WAIT(4)
+        R_WAIT(5)
+#undef R_WAIT
+#undef R_VM
+        asm volatile("" ::: "memory");
+        V w[HW][2], x[MG][2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int c = ((4 * k + grp) ^ (fr & 7)) << 4;
+#pragma unroll
+          for (int h = 0; h < HW; ++h) w[h][k] = *reinterpret_cast<const V*>(stg + h * 2048 + fr * 128 + c);
+#pragma unroll
+          for (int u = 0; u < MG; ++u) {
+            const int r = min(u * 16 + fr, XR - 1);         // (rows past M: columns that are not stored)
+            if constexpr (XS == 1) {
+              x[u][k] = *reinterpret_cast<const V*>(stg + R::SW + r * 128 + (((4 * k + grp) ^ (r & 7)) << 4));
+            } else {
+              const char* row = stg + R::SW + r * 256;
+              const int a = 8 * k + 2 * grp, sw = r & 15;
+              const floatx4 lo = *(const floatx4*)(row + ((a ^ sw) << 4)), hi = *(const floatx4*)(row + (((a + 1) ^ sw) << 4));
+              x[u][k] = rounded(lo, hi);
+            }
+          }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (t + nst < mine) fill(t + nst, stg);
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int u = 0; u < MG; ++u)
+#pragma unroll
+            for (int h = 0; h < HW; ++h) acc[k][h][u] = mfma_step(w[h][k], x[u][k], acc[k][h][u]);
+        stg = stg + STAGE == ring + nst * STAGE ? ring : stg + STAGE;
+      }
     }
 #pragma unroll
     for (int u = 0; u < MG; ++u)
@@ -216,24 +258,27 @@ __device__ __forceinline__ void rows_of(const TA* A, const TW* W, void* C, const
   }
 }
 
-template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED, int U>
 __global__ __launch_bounds__(64 * WV) void gemm_rows(const TA* __restrict__ A, const TW* __restrict__ W, void* __restrict__ C, Epi epi,
                                                      int M, int N, int K, int lda, int ldw, int ldc, const int* __restrict__ offs,
                                                      const int* __restrict__ a_rows, long long w_gs, int nst) {
-  rows_of<TA, TW, XR, WV, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs, nst);
+  rows_of<TA, TW, XR, WV, NB, GATED, U>(A, W, C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs, nst);
 }
 
-template <typename TA, typename TW, int XR, int WV, int NB, bool GATED>
+template <typename TA, typename TW, int XR, int WV, int NB, bool GATED, int U>
 int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc, int groups, const int* offs,
           const int* a_rows, long long w_gs, hipStream_t s) {
   typedef Ring<TA, TW, XR, GATED ? 2 * NB : NB> R;
-  static const hipError_t a = hipFuncSetAttribute((const void*)gemm_rows<TA, TW, XR, WV, NB, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, WV * R::NST * R::STAGE);
+  constexpr int SUMS = (XR + 15) / 16 * (GATED ? 2 * NB : NB) * 1024;
+  static const hipError_t a = hipFuncSetAttribute((const void*)gemm_rows<TA, TW, XR, WV, NB, GATED, U>, hipFuncAttributeMaxDynamicSharedMemorySize, WV * (U > 0 ? SUMS : R::NST * R::STAGE));
   if (a != hipSuccess) return -(int)a;
   const int cols = (N + 16 * NB - 1) / (16 * NB), gs = offs != nullptr ? groups : 1, stages = (K * (int)sizeof(TW) + 127) / 128;
   const bool deep = (long long)cols * gs <= (sizeof(TW) == 2 ? 1024 : 512);
-  const int nst = std::min((int)(deep ? R::NST : R::FEW), (stages + WV - 1) / WV);       // (a short K needs less)
-  hipLaunchKernelGGL((gemm_rows<TA, TW, XR, WV, NB, GATED>), dim3(cols, gs), dim3(64 * WV), WV * nst * R::STAGE, s, (const TA*)A, (const TW*)W, C, epi, M, N, K,
-                     lda, ldw, ldc, offs, a_rows, w_gs, nst);
+  int nst = std::min((int)(deep ? R::NST : R::FEW), (stages + WV - 1) / WV);       // (a short K needs less)
+  const int fit = 163840 / (WV * 2 * R::STAGE);            // blocks of two large stages a wave that a CU's LDS holds: where there are more, one stage and twice the blocks
+  if (nst == 2 && fit <= 2 && (stages <= 2 * WV || (fit == 1 && !GATED)) && (long long)cols * std::min(gs, M) > 256 * fit) nst = 1;
+  hipLaunchKernelGGL((gemm_rows<TA, TW, XR, WV, NB, GATED, U>), dim3(cols, gs), dim3(64 * WV), WV * (U > 0 ? SUMS : nst * R::STAGE), s, (const TA*)A, (const TW*)W,
+                     C, epi, M, N, K, lda, ldw, ldc, offs, a_rows, w_gs, nst);
   const hipError_t e = hipGetLastError();
   return e == hipSuccess ? 1 : -(int)e;
 }
@@ -245,9 +290,10 @@ int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const E
   // 16 rows a pass over W (8 if there are no more in all), without row groups up to 32 in one.  Eight waves share K where one block a CU or less
   // has all the columns and K is more than a tile for each (8 rows x 2048 x 2048 5.1 us, 5.4 with four; 24 rows 5.8 and 5.6, gated 8.1 and 7.8),
   // else four, two blocks a CU or more.  Blocks of 32 columns read half as much of A and leave no half-empty second round: from one round of
-  // 16-column blocks to 448 (8 rows x 6416 x 2048 9.3 -> 8.8 us; 8192, two full blocks a CU, 9.7 and 10.3), above 16 rows always (24 rows x 8192 x
-  // 2048 10.8 -> 10.4, x 32000 33.7 -> 29.3), plain bf16 products above 1024 blocks (8 rows x 32000 28.6 -> 27.2; fp32 49.5 and 55.4), and plain bf16 row
-  // groups of a row each or more (48 rows of 10 x 2048 x 2048 21.3 -> 19.9; 4 rows of 8 10.2 and 11.3).
+  // 16-column blocks (below it 1.04 to 1.4 of the time) to 448 (8 rows x 6416 x 2048 9.3 -> 8.8 us; of 1,500 random widths of 200 to 720 blocks 0.9 to 0.95 of the
+  // time up to 320, 0.83 to 1.05 to 448, and from 480 to 512 on slower but for the next kind), plain products of more than 16 rows above that too (24 rows x
+  // 8192 x 2048 10.8 -> 10.4, x 32000 33.7 -> 29.3; fp32 from 512 to 720 blocks is 1.1 to 1.19 so), plain bf16 products above 1024 blocks (8 rows x 32000
+  // 28.6 -> 27.2; fp32 49.5 and 55.4), and plain row groups of a row each or more on bf16 weights (48 rows of 10 x 2048 x 2048 21.3 -> 19.9; 4 rows of 8 10.2 and 11.3).
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
@@ -256,14 +302,30 @@ int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const E
   const long long blocks = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1);
   const bool wide = offs != nullptr ? !gated && tw == 1 && M >= groups : blocks > 256 && (blocks <= 448 || (!gated && (two || (tw == 1 && blocks > 1024))));
   const bool eight = !two && !gated && blocks <= 256 && K * ew > 512;
-#define START(TA, TW, XR, WV, NB, GATED) start<TA, TW, XR, WV, NB, GATED>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
+  // Straight to registers, in one chunk of 1, 2 or 3 steps for each of four waves (10,000 random products, times by the rings' with their spread over classes of rows
+  // and blocks): up to 256 bytes of a row of W 0.78 - 0.97, to 512 0.90 - 0.99 without gated row groups (1.00 - 1.04), to 768 0.92 - 1.02 for plain
+  // products of up to 16 rows and row groups; with eight waves to 1024 for those of up to 16 rows in a round of blocks (0.93 - 0.96).  A block reads its
+  // rows of A beside 16 columns: where that is more than 32 KB a CU in all, the rings' wider blocks are as fast or faster (1.1 - 1.4 above 1,500 blocks).
+  const int kb = K * ew;
+  const bool light = offs != nullptr || blocks <= 256 || blocks * ((gated ? 32 : 16) * kb + (long long)M * K * ea) <= 256 * 32768;
+  const int steps = !light ? 0 : kb <= 256 ? 1 : kb <= 512 && !(gated && offs != nullptr) ? 2 : kb <= 768 && !gated && !two ? 3 : 0;
+  const bool direct = steps > 0 || (kb <= 1024 && offs == nullptr && eight);
+#define START(TA, TW, XR, WV, NB, GATED, U) start<TA, TW, XR, WV, NB, GATED, U>(A, W, C, epi, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, s)
 #define PANELS(TA, TW, XR)                                                                                                 \
-  (gated ? (wide ? START(TA, TW, XR, 4, 2, true) : START(TA, TW, XR, 4, 1, true))                                          \
-         : wide ? START(TA, TW, XR, 4, 2, false) : eight ? START(TA, TW, XR <= 16 ? XR : 16, 8, 1, false) : START(TA, TW, XR, 4, 1, false))
-#define ROWS(TA, TW) (two ? (M <= 24 ? PANELS(TA, TW, 24) : PANELS(TA, TW, 32)) : M <= 8 ? PANELS(TA, TW, 8) : PANELS(TA, TW, 16))
+  (gated ? (wide ? START(TA, TW, XR, 4, 2, true, 0) : START(TA, TW, XR, 4, 1, true, 0))                                    \
+         : wide ? START(TA, TW, XR, 4, 2, false, 0) : eight ? START(TA, TW, XR <= 16 ? XR : 16, 8, 1, false, 0) : START(TA, TW, XR, 4, 1, false, 0))
+#define CHUNK(TA, TW, U)                                                                                                   \
+  (two ? (gated ? START(TA, TW, 32, 4, 1, true, U) : START(TA, TW, 32, 4, 1, false, U))                                    \
+       : gated ? START(TA, TW, 16, 4, 1, true, U) : START(TA, TW, 16, 4, 1, false, U))
+#define CHUNKS(TA, TW)                                                                                                     \
+  (steps == 1 ? CHUNK(TA, TW, 1) : steps == 2 ? CHUNK(TA, TW, 2) : steps == 3 ? START(TA, TW, 16, 4, 1, false, 3) : START(TA, TW, 16, 8, 1, false, 2))
+#define ROWS(TA, TW)                                                                                                       \
+  (direct ? CHUNKS(TA, TW) : two ? (M <= 24 ? PANELS(TA, TW, 24) : PANELS(TA, TW, 32)) : M <= 8 ? PANELS(TA, TW, 8) : PANELS(TA, TW, 16))
   if (tw == 0) return ROWS(float, float);
   return ta == 1 ? ROWS(bf16_t, bf16_t) : ROWS(float, bf16_t);
 #undef ROWS
+#undef CHUNKS
+#undef CHUNK
 #undef PANELS
 #undef START
 }

@@ -327,6 +327,33 @@ def test_few_rows_edges(ops, types, M):
             assert torch.equal(y[rest], H.matmul_nt(a, w)[rest]) and not y[[M - 1, M // 2 - 1]].isfinite().any()
 
 
+# short rows about the lengths (256, 512 and 1024 bytes of a weight row, by rows, columns and gates) up to which operands go straight to registers: whole
+# steps and tails, waves without a step, columns past a block's end, up to a round of blocks and more; row groups, empty and of more rows than a pass
+# takes, as they are and gathered.  fp32 sums of up to 520 products: 1e-5 as above
+@pytest.mark.parametrize("types", ["bf16", "mixed", "fp32"])
+@pytest.mark.parametrize("terms", [128, 136, 248, 256, 264, 504, 512, 520])
+def test_few_rows_of_few_terms(ops, types, terms):
+    H, _ = ops
+    ta, tw = {"bf16": (torch.bfloat16, torch.bfloat16), "mixed": (torch.float32, torch.bfloat16), "fp32": (torch.float32, torch.float32)}[types]
+    f64 = lambda t: (t.to(tw) if types == "mixed" else t).double()
+    gate = lambda z: torch.nn.functional.silu(z[:, :z.shape[1] // 2]) * z[:, z.shape[1] // 2:]
+    K = terms // 2 // 8 * 8 if types == "fp32" else terms
+    torch.manual_seed(terms)
+    for M, N in ((1, 20), (16, 4096), (16, 4136), (5, 8200), (17, 4096), (32, 4104), (20, 8200)):
+        a, w = torch.randn(M, K, device=DEV).to(ta), (0.1 * torch.randn(N, K, device=DEV)).to(tw)
+        z = f64(a) @ w.double().t()
+        close(H.matmul_nt(a, w), z, 1e-5)
+        close(H.gated_matmul_nt(a, w, torch.float32), gate(z), 2e-5)
+    sizes, N = [0, 1, 19, 0, 3, 0, 0, 2, 8], 136
+    M = sum(sizes)
+    offs, w = torch.tensor(np.cumsum([0] + sizes), dtype=torch.int32, device=DEV), (0.1 * torch.randn(len(sizes), N, K, device=DEV)).to(tw)
+    a, rows = torch.randn(M, K, device=DEV).to(ta), torch.randperm(M, device=DEV).to(torch.int32)
+    y = lambda x: torch.cat([f64(x[offs[e]:offs[e + 1]]) @ w[e].double().t() for e in range(len(sizes))])
+    close(H.grouped_matmul_nt(a, w, offs), y(a), 1e-5)
+    close(H.gated_matmul_nt(a, w, torch.float32, offs=offs), gate(y(a)), 2e-5)
+    close(H.gated_matmul_nt(a, w, torch.float32, offs=offs, rows=rows), gate(y(a[rows.long()])), 2e-5)
+
+
 # about the rows up to which row groups take the few-row kernel, spread over the groups and nearly all in one
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("M", [64, 65, 128, 129])
