@@ -17,6 +17,26 @@
 #include "gemm_epi.h"
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+
+// An accumulator's sixteen values: a loop over four at a time, moved on between them, so that there is one copy of the activations' code and no
+// index into registers.  (All copies laid out are more than the compiler unrolls, and accumulators that a loop indexes go to scratch: 1,011 rows x 6416 x
+// 1760 217 us, 104 without.)
+__device__ __forceinline__ floatx16 epi_values(floatx16 v, float bias, const Epi& e, const EpiRegs& r) {
+  v += bias;
+  if (e.kind != 0) {
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+      float o[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) o[x] = epi_value(v[x], e, r);
+#pragma unroll
+      for (int x = 0; x < 12; ++x) v[x] = v[x + 4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) v[12 + x] = o[x];
+    }
+  }
+  return v;
+}
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 
 #define BM 64
@@ -115,10 +135,11 @@ __global__ __launch_bounds__(256) void gemm_nt_any(const TA* __restrict__ A, con
   if (col < N) {
     const float bv = epi.bias != nullptr ? epi.bias[cbase + col] : 0.f;
     epi_column(epi, er, col);
+    const floatx16 v = epi_values(acc, bv, epi, er);
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int row = m0 + wm + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-      if (row < mend) emit(C, cbase + (size_t)row * ldc + col, acc[r] + bv, epi, er);
+      if (row < mend) emit(C, cbase + (size_t)row * ldc + col, v[r], epi);
     }
   }
 }
@@ -275,12 +296,14 @@ __global__ __launch_bounds__(64 * NWM * NWN) void gemm_nt_big(const TA* __restri
     const float bv = epi.bias != nullptr ? epi.bias[cbase + col] : 0.f;
     epi_column(epi, er, col);
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i) {
+      const floatx16 v = epi_values(acc[i][j], bv, epi, er);
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int row = m0 + wm + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        if (row < mend) emit(C, cbase + (size_t)row * ldc + col, acc[i][j][r] + bv, epi, er);
+        if (row < mend) emit(C, cbase + (size_t)row * ldc + col, v[r], epi);
       }
+    }
   }
 }
 
