@@ -656,6 +656,21 @@ def test_rows_written_to_the_host(ops, M, N, cdt):
         assert bool((down == -7.0).all())
 
 
+# the same for rows long enough for the rings, blocks of 16 and of 32 columns
+@pytest.mark.parametrize("M,N", [(1, 4), (8, 1000), (16, 6404), (17, 4100), (32, 6404), (9, 16400)])
+@pytest.mark.parametrize("cdt", [torch.bfloat16, torch.float32])
+def test_long_rows_written_to_the_host(ops, M, N, cdt):
+    H, _ = ops
+    torch.manual_seed(M + N)
+    a, w = torch.randn(M, 1032, device=DEV).to(cdt), torch.randn(N, 1032, device=DEV).to(cdt)
+    down = torch.full((M * N + 4,), -7.0, pin_memory=True)
+    mirror = H.host_rows(torch.tensor([down.data_ptr()], dtype=torch.int64, device=DEV))
+    c = H.matmul_nt(a, w, mirror=mirror)
+    torch.cuda.synchronize()
+    assert mirror.rows_there and torch.equal(c, H.matmul_nt(a, w))
+    assert torch.equal(down[:M * N].view(M, N), c.cpu()) and bool((down[M * N:] == -7.0).all())
+
+
 # weight rows so far apart (2^27 elements: past the few-row kernel's 32-bit offsets) that another kernel takes the product: the argmax then
 # writes the rows
 def test_rows_written_to_the_host_of_far_weight_rows(ops):
