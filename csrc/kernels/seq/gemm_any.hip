@@ -344,11 +344,11 @@ extern "C" int fls_seq_gemm(const void* A, int ta, const void* W, int tw, void* 
   if (mirror != nullptr && (tc != 0 || act_kind >= EPI_GATE || offs != nullptr || groups != 1 || M > 32 || N % 4 || !vec_a || !vec_w))
     return SEQ_NOT_SERVED;                 // (only the few-row kernel writes twice)
   if (vec_a && vec_w) {
-    // Few rows: bound by reading W, no tile to fill.  32 rows x 2048 x 2048 5.6 us, the best tile 6.5; 40 rows 8.5 and 6.4 (fp32 10.8, 14.2; 18.4,
-    // 14.0).  Row groups: 8 rows each on average, and 128 in all (64 in fp32), because their sizes are on the device and a router may send most
-    // rows to one: a block then reads its weight panel once per 16 rows.  128 groups (1536 x 2048, bf16), rows spread or all in one: 64 rows 58
-    // and 16 us, tiles 75 and 16; 128 rows 89 and 28, 109 and 16; 1024 rows 142 and 205, 156 and 29.  fp32: 64 rows 110 and 29, 132 and 25; 128
-    // rows 168 and 52, 200 and 25; 1024 rows 279 and 375, 314 and 81.
+    // Few rows: bound by reading W, no tile to fill.  32 rows x 2048 x 2048 6.5 us, the best tile 8.4; 40 rows 9.1 and 7.4 (fp32 10.5, 13.9; 17.8,
+    // 13.7).  Row groups: 8 rows each on average, and 128 in all (64 in fp32), because their sizes are on the device and a router may send most
+    // rows to one: a block then reads its weight panel once per 16 rows.  128 groups (1536 x 2048, bf16), rows spread or all in one: 64 rows 73
+    // and 16 us, tiles 92 and 17; 128 rows 141 and 29, 165 and 18; 1024 rows 148 and 193, 157 and 32.  fp32: 64 rows 136 and 33, 172 and 32; 128
+    // rows 273 and 56, 319 and 33; 1024 rows 293 and 361, 327 and 89.
     int rc = 0;
     if (offs != nullptr ? M <= 8 * groups && M <= (tw == 1 ? 128 : 64) : groups == 1 && M <= 32)
       rc = seq_gemm_rows(A, ta, W, tw, C, bias, M, N, K, lda, ldw, ldc, groups, offs, a_rows, w_gs, st);

@@ -5,9 +5,9 @@
 // sums, which meet in LDS in the order of the waves.  A tile is two steps of 32 elements of bf16 (a 16x16x32 MFMA each) or 16 of fp32 (four
 // 16x16x4 MFMAs, lane group g holding elements 4 g .. 4 g + 3).  Why not straight to registers: what a lane needs for an MFMA is 16 bytes of its own
 // row, so that neighbouring lanes' loads are rows apart, and a CU takes such loads at 16 bytes a cycle, 54 by DMA; with the loads of A, as many for 16
-// rows as for 16 columns, that was the bound.  Cold weights, before and so (us): 8 rows x 2048 x 2048 6.3, 5.1; x 2048 x 8192 15.6, 13.1; x 32000 x 2048
-// 31.5, 27.2 (the rate of a copy: 27.8); 24 rows x 2048 x 2048 8.2, 5.5; x 2048 x 8192 23.2, 15.0; x 32000 x 2048 37.5, 29.3; gated 5440 x 2048 18.3, 13.2;
-// fp32 8 rows x 2048 x 8192 28.3, 21.9, 24 rows 49.4, 30; 16 rows in 8 groups, gated 2048 x 2048 29.4, 29.1, 2048 x 2048 16.5, 14.6.
+// rows as for 16 columns, that was the bound.  Cold weights, before and so (us): 8 rows x 2048 x 2048 6.4, 5.2; x 2048 x 8192 15.1, 11.2; x 32000 x 2048
+// 30.7, 26.8 (the rate of a copy: 27.8); 24 rows x 2048 x 2048 8.7, 6.2; x 2048 x 8192 23.3, 14.3; x 32000 x 2048 37.3, 30.1; gated 5440 x 2048 17.4, 12.9;
+// fp32 8 rows x 2048 x 8192 27.8, 21.1, 24 rows 48.6, 30.3; 16 rows in 8 groups, gated 2048 x 2048 27.1, 24.3, 2048 x 2048 15.7, 14.2.
 #include <algorithm>
 
 #include "seq_common.h"
@@ -299,19 +299,20 @@ int start(const void* A, const void* W, void* C, const Epi& epi, int M, int N, i
 int seq_gemm_rows(const void* A, int ta, const void* W, int tw, void* C, const Epi& epi, int M, int N, int K, int lda, int ldw, int ldc,
                   int groups, const int* offs, const int* a_rows, long long w_gs, hipStream_t s) {
   // 16 rows a pass over W (8 if there are no more in all), without row groups up to 32 in one.  Eight waves share K where one block a CU or less
-  // has all the columns and K is more than a tile for each (8 rows x 2048 x 2048 5.1 us, 5.4 with four; 24 rows 5.8 and 5.6, gated 8.1 and 7.8),
+  // has all the columns and K is more than a tile for each (8 rows x 2048 x 2048 5.2 us, 5.3 with four; 24 rows 6.2 and 6.2, gated 7.2 and 7.0),
   // else four, two blocks a CU or more.  Blocks of 32 columns read half as much of A and leave no half-empty second round: from one round of
-  // 16-column blocks (below it 1.04 to 1.4 of the time) to 448 (8 rows x 6416 x 2048 9.3 -> 8.8 us; of 1,500 random widths of 200 to 720 blocks 0.9 to 0.95 of the
-  // time up to 320, 0.83 to 1.05 to 448, and from 480 to 512 on slower but for the next kind), plain products of more than 16 rows above that too (24 rows x
-  // 8192 x 2048 10.8 -> 10.4, x 32000 33.7 -> 29.3; fp32 from 512 to 720 blocks is 1.1 to 1.19 so), plain bf16 products above 1024 blocks (8 rows x 32000
-  // 28.6 -> 27.2; fp32 49.5 and 55.4), and plain row groups of a row each or more on bf16 weights (48 rows of 10 x 2048 x 2048 21.3 -> 19.9; 4 rows of 8 10.2 and 11.3).
+  // 16-column blocks (below it 1.04 to 1.4 of the time) to 448 (8 rows x 6416 x 2048 8.3 -> 7.8 us; of 1,500 random widths of 200 to 720 blocks 0.9 to 0.95 of the
+  // time up to 320, 0.83 to 1.05 to 448, and from 480 to 512 on slower but for the next kinds), plain products of more than 16 rows above that too (24 rows x
+  // 8192 x 2048 10.2 -> 9.5, x 32000 32.8 -> 30.1; fp32 from 512 to 720 blocks is 1.1 to 1.19 so), plain ones of more than 8 fp32 rows on bf16 weights above 1024
+  // blocks (16,400 to 66,000 columns 0.90 to 0.94; bf16 rows 0.96 to 1.03, up to 8 rows 0.97 to 1.08), and plain row groups of a row each or more on bf16
+  // weights (48 rows of 10 x 2048 x 2048 19.9 -> 18.9; 4 rows of 8 8.0 and 7.7).
   const bool gated = epi.kind >= EPI_GATE;
   if (gated) N >>= 1;                      // columns of C
   const int ea = ta == 1 ? 2 : 4, ew = tw == 1 ? 2 : 4;
   if (((long long)ldw * 16 + 8) * ew >= (1LL << 31) || (long long)lda * M * ea >= (1LL << 31)) return 0;      // (32-bit offsets within a panel, among the rows)
   const bool two = offs == nullptr && M > 16;
   const long long blocks = (long long)((N + 15) / 16) * (offs != nullptr ? groups : 1);
-  const bool wide = offs != nullptr ? !gated && tw == 1 && M >= groups : blocks > 256 && (blocks <= 448 || (!gated && (two || (tw == 1 && blocks > 1024))));
+  const bool wide = offs != nullptr ? !gated && tw == 1 && M >= groups : blocks > 256 && (blocks <= 448 || (!gated && (two || (ta != tw && M > 8 && blocks > 1024))));
   const bool eight = !two && !gated && blocks <= 256 && K * ew > 512;
   // Straight to registers, in one chunk of 1, 2 or 3 steps for each of four waves (10,000 random products, times by the rings' with their spread over classes of rows
   // and blocks): up to 256 bytes of a row of W 0.78 - 0.97, to 512 0.90 - 0.99 without gated row groups (1.00 - 1.04), to 768 0.92 - 1.02 for plain
