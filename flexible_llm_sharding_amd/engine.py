@@ -254,6 +254,7 @@ class ShardedRunner:
         self.stats: Dict[str, float] = {}
         self._fault = _parse_fault(self.comm.rank)
         self._store: Optional[ActivationStore] = None
+        self._results: Optional[hostmem.ResultBlocks] = None
         self._inbox: Optional[StageInbox] = None
         self._mp_start_layer = 0
         # whole-forward HIP graphs: only when every shard is local AND resident (fixed weight pointers)
@@ -961,9 +962,7 @@ class ShardedRunner:
             rx_stats = {f"rx_{k}": float(v) for k, v in px.inbox.stats.items()}
         self.last_tokens = [None] * len(px.tps)
         for batch, host, ev, pool_buf, am in px.out_pending:
-            self._collect(batch, host.numpy(), am, px.outputs)
-            if pool_buf is not None:
-                store.recycle_host(pool_buf)
+            self._collect(batch, host.numpy(), am, px.outputs, pool_buf)
         store.clear()
         store.trim()                   # pinned pool follows this call's shapes
         wait_s = pf.take_wait_seconds()
@@ -1153,15 +1152,11 @@ class ShardedRunner:
         """Replay every micro-batch (``run(batch, index) -> probs``), its row argmax and the D2H
         of both into pooled pinned buffers, all on the current stream -> (pending, argmax tensors,
         decoder FLOPs)."""
-        store = self._get_store()
         pending, ams, flops = [], [], 0.0
         for i, batch in enumerate(batches):
             probs = run(batch, i)
             am = self.ops.argmax_rows(probs)
-            nbytes = probs.numel() * probs.element_size()
-            pool_buf = store.host_buffer(nbytes + 4 * probs.shape[0])
-            host = pool_buf[:nbytes].view(probs.dtype).view(probs.shape)
-            host_am = pool_buf[nbytes:nbytes + 4 * probs.shape[0]].view(torch.int32)
+            pool_buf, host, host_am = self._output_block(probs)
             host.copy_(probs, non_blocking=True)     # same stream: ordered before the next replay
             host_am.copy_(am, non_blocking=True)
             pending.append((batch, host, pool_buf, host_am))
@@ -1176,11 +1171,9 @@ class ShardedRunner:
         return pending, ams, flops
 
     def _collect_graphed(self, pending, outputs, n_prompts: int) -> None:
-        store = self._get_store()
         self.last_tokens = [None] * n_prompts
         for batch, host, pool_buf, host_am in pending:
-            self._collect(batch, host.numpy(), host_am, outputs)
-            store.recycle_host(pool_buf)
+            self._collect(batch, host.numpy(), host_am, outputs, pool_buf)
 
     # ------------------------------------------------- speculative generation steps
     # A greedy generation step re-tokenizes ``suffix + decode(tokens)`` (main.py:86-88), which
@@ -1279,9 +1272,8 @@ class ShardedRunner:
 
     def _drop_spec(self, spec: dict) -> None:
         spec["done"].synchronize()
-        store = self._get_store()
         for _, _, pool_buf, _ in spec["pending"]:
-            store.recycle_host(pool_buf)
+            self._output_landed(pool_buf)
         self.spec_dropped += 1
 
     spec_dropped = 0
@@ -1353,20 +1345,45 @@ class ShardedRunner:
             print(f"rank{self.comm.rank}: resuming at shard {k0} from {ck.dir}")
         return ck, k0, (ck.load(k0) if k0 else {})
 
-    def _collect(self, batch: PackedBatch, probs: np.ndarray, am, outputs) -> None:
+    def _output_block(self, probs: torch.Tensor):
+        """Pinned memory for a micro-batch's results -> (its owner, the rows, their argmax): a block that the caller gets
+        (hostmem.ResultBlocks), or where none is to be had a buffer of the store's pool that the caller's copies are made from."""
+        nbytes, rows = probs.numel() * probs.element_size(), probs.shape[0]
+        at = -(-nbytes // 16) * 16
+        if self._results is None:
+            self._results = hostmem.ResultBlocks(pinned=self.cuda)
+        owner = self._results.take(at + 4 * rows)
+        if owner is not None:
+            buf = torch.from_numpy(owner)
+        else:
+            owner = buf = self._get_store().host_buffer(at + 4 * rows)
+        return owner, buf[:nbytes].view(probs.dtype).view(probs.shape), buf[at:at + 4 * rows].view(torch.int32)
+
+    def _output_landed(self, owner) -> None:
+        """The copies into a block of :meth:`_output_block` have been waited for (and a pool buffer's rows taken)."""
+        if isinstance(owner, np.ndarray):
+            hostmem.ResultBlocks.filled(owner)
+        else:
+            self._get_store().recycle_host(owner)
+
+    def _collect(self, batch: PackedBatch, probs: np.ndarray, am, outputs, owner=None) -> None:
         """Host scores of a finished micro-batch into ``outputs`` (prompt order) and its greedy
-        tokens into ``self.last_tokens`` (``am``: the rows' argmax, computed on the device)."""
+        tokens into ``self.last_tokens`` (``am``: the rows' argmax, computed on the device).  The rows go to the caller as
+        they lie in a block of its own, else (``owner`` a pool's buffer, or None) as copies."""
+        own = isinstance(owner, np.ndarray)
         am = am.numpy() if am is not None else None
         if isinstance(batch, StepBatch):
-            outputs[batch.prompt_ids[0]] = (np.array(probs, dtype=np.float32, copy=True), np.array(am, copy=True))
-            return
-        r = 0
-        for j, pid in enumerate(batch.prompt_ids):
-            ns = batch.n_suffix[j]
-            outputs[pid] = np.expand_dims(probs[r:r + ns].astype(np.float16, copy=True), axis=1)
-            if am is not None:
-                self.last_tokens[pid] = am[r:r + ns].astype(np.int64).reshape(ns, 1)
-            r += ns
+            outputs[batch.prompt_ids[0]] = (np.array(probs, dtype=np.float32, copy=None if own else True), np.array(am, copy=True))
+        else:
+            r = 0
+            for j, pid in enumerate(batch.prompt_ids):
+                ns = batch.n_suffix[j]
+                outputs[pid] = np.expand_dims(probs[r:r + ns].astype(np.float16, copy=not own), axis=1)
+                if am is not None:
+                    self.last_tokens[pid] = am[r:r + ns].astype(np.int64).reshape(ns, 1)
+                r += ns
+        if owner is not None:
+            self._output_landed(owner)
 
     def _start_output_copy(self, batch: PackedBatch, probs: torch.Tensor):
         """D2H of a micro-batch's probabilities and of their row argmax (the greedy token of
@@ -1377,11 +1394,7 @@ class ShardedRunner:
             am = self.ops.argmax_rows(probs) if hasattr(self.ops, "argmax_rows") else None
         if not self.cuda:
             return batch, probs.detach().to(torch.float32 if self.hybrid else torch.float16).cpu(), None, None, am
-        store = self._get_store()
-        nbytes = probs.numel() * probs.element_size()
-        pool_buf = store.host_buffer(nbytes + 4 * probs.shape[0])
-        host = pool_buf[:nbytes].view(probs.dtype).view(probs.shape)
-        host_am = pool_buf[nbytes:nbytes + 4 * probs.shape[0]].view(torch.int32)
+        pool_buf, host, host_am = self._output_block(probs)
         self.d2h_stream.wait_stream(torch.cuda.current_stream(self.dev))
         with torch.cuda.stream(self.d2h_stream):
             host.copy_(probs, non_blocking=True)
@@ -1412,4 +1425,7 @@ class ShardedRunner:
         if self._store is not None:
             self._store.close()
             self._store = None
+        if self._results is not None:
+            self._results.close()
+            self._results = None
         self._splitk_ws = self._splitk_own = None

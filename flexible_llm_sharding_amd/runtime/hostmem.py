@@ -12,8 +12,10 @@ from __future__ import annotations
 import ctypes
 import os
 import time
-from typing import Dict
+from collections import deque
+from typing import Dict, Optional
 
+import numpy as np
 import torch
 
 from .. import _native, knobs
@@ -84,6 +86,83 @@ def alloc_host(nbytes: int, pinned: bool = True) -> torch.Tensor:
                 return torch.frombuffer(arr, dtype=torch.uint8)[:nbytes]
         return torch.empty(nbytes, dtype=torch.uint8, pin_memory=True)
     return torch.empty(nbytes, dtype=torch.uint8)
+
+
+class _Lease:
+    """One block of a :class:`ResultBlocks` while arrays over it are alive: numpy keeps it as their base."""
+    __slots__ = ("pool", "block", "filled", "__array_interface__")
+
+    def __init__(self, pool: "ResultBlocks", block: torch.Tensor, nbytes: int):
+        self.pool, self.block, self.filled = pool, block, False
+        self.__array_interface__ = {"shape": (nbytes,), "typestr": "|u1", "data": (block.data_ptr(), False), "version": 3}
+
+    def __del__(self):
+        self.pool._out_bytes.append(-self.block.numel())
+        if self.filled and not self.pool.closed:       # (else the block goes, which waits for what still writes it)
+            self.pool._back.append(self.block)
+
+
+class ResultBlocks:
+    """Pinned blocks that calls' results are copied into by the GPU and handed to the caller in, without a second copy on the host
+    (a call with 48 rows of 151,936 fp16 probabilities spent 505 of 3,435 us on that copy).  A block comes back when the last array
+    over it is gone.  At most ``MOST`` blocks and ``MOST_BYTES`` are out or kept: :meth:`take` then gives None and the caller copies, so that results
+    that a program keeps for good pin no more than that.  A lease may die on any thread, within a collection too: it only appends to deques."""
+
+    MOST = 4
+    MOST_BYTES = 256 << 20
+
+    def __init__(self, pinned: bool = True):
+        self.pinned = pinned
+        self.closed = False
+        self._free: list = []
+        self._back: deque = deque()
+        self._out_bytes: deque = deque()      # + for a block handed out, - for one that died
+        self._out = self._out_n = 0
+
+    def _settle(self) -> None:
+        while self._out_bytes:
+            n = self._out_bytes.popleft()
+            self._out += n
+            self._out_n += 1 if n > 0 else -1
+        while self._back:
+            self._free.append(self._back.popleft())
+
+    @staticmethod
+    def _size(nbytes: int) -> int:
+        """Bytes of a block for ``nbytes``: sizes a quarter of a power of two apart, so that calls of about one size share theirs."""
+        n = max(1 << 16, nbytes)
+        q = 1 << (n.bit_length() - 3)
+        return -(-n // q) * q
+
+    def take(self, nbytes: int) -> Optional[np.ndarray]:
+        """A uint8 array of ``nbytes`` in a pinned block of its own, or None.  :meth:`filled` before the caller gets it."""
+        size = self._size(nbytes)
+        self._settle()
+        if self.closed or nbytes <= 0:
+            return None
+        fits = [b for b in self._free if size <= b.numel() <= 2 * size]
+        if fits:
+            block = min(fits, key=lambda b: b.numel())
+            self._free = [b for b in self._free if b is not block]
+        else:
+            while self._free and (self._out_n + len(self._free) >= self.MOST
+                                  or self._out + size + sum(b.numel() for b in self._free) > self.MOST_BYTES):
+                self._free.pop(0)
+            if self._out_n >= self.MOST or self._out + size > self.MOST_BYTES:
+                return None
+            block = alloc_host(size, pinned=self.pinned)
+        self._out_bytes.append(block.numel())
+        return np.asarray(_Lease(self, block, nbytes))
+
+    @staticmethod
+    def filled(array: np.ndarray) -> None:
+        """What writes ``array`` (as :meth:`take` gave it) has been waited for: its block may be used again once it is let go."""
+        array.base.filled = True
+
+    def close(self) -> None:
+        self.closed = True
+        self._settle()
+        self._free.clear()
 
 
 class _DeviceBlock:

@@ -662,3 +662,28 @@ def test_piece_pool_streams_layer_files(mid_model, tmp_path):
     assert r.stats["weight_h2d_bytes"] > 0
     r.close()
     torch.cuda.set_per_process_memory_fraction(1.0)
+
+
+@pytest.mark.parametrize("budget", [200, 4096])
+def test_results_kept_by_the_caller(setup, budget):
+    """More calls' results kept than there are pinned blocks, some let go in between, several micro-batches a call or one: every array keeps its
+    values, and what the caller writes into one changes no other."""
+    path, cfg, tok, prompts, ref = setup
+    r = ShardedRunner(cfg, HostStore.from_model_path(cfg, path), "cuda:0", tok, layer_num_per_shard=8, storage_location="gpu", resident=True,
+                      token_budget=budget)
+    want = [o.copy() for o in r(prompts)]
+    kept = [r(prompts) for _ in range(3)]
+    for k in range(6):
+        kept.append(r(prompts))
+        if k % 2:
+            kept.pop(0)
+        for o in kept[-1]:
+            o += 0                                # (writable)
+    kept[0][0][:] = 7
+    r.close()
+    for c in kept:
+        for i, o in enumerate(c):
+            if c is kept[0] and i == 0:
+                assert bool((o == 7).all())
+            else:
+                assert np.array_equal(o, want[i])

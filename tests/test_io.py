@@ -2,6 +2,7 @@
 import json
 import os
 
+import numpy as np
 import pytest
 import torch
 
@@ -281,3 +282,30 @@ def test_hf_moe_checkpoint_converts_and_matches(tmp_path, family):
             with torch.no_grad():
                 logits = hf(torch.tensor([tp.prefix + s])).logits[0, -1].float()
             assert np.abs(o[j, 0].astype(np.float32) - torch.softmax(logits, -1).numpy()).max() < 2e-3
+
+
+@pytest.mark.parametrize("nbytes", [1, 65536, 65537, 3000000])
+def test_result_blocks(nbytes):
+    """A block comes back only when the last view over it is gone and what writes it was waited for; no more of them than MOST and MOST_BYTES;
+    after close() none, and those still out keep their bytes."""
+    pool = hostmem.ResultBlocks(pinned=False)
+    out = [pool.take(nbytes) for _ in range(pool.MOST)]
+    assert pool.take(nbytes) is None and all(a.nbytes == nbytes and a.flags.writeable for a in out)
+    spans = sorted((a.ctypes.data, a.ctypes.data + nbytes) for a in out)
+    assert all(e <= s for (_, e), (s, _) in zip(spans, spans[1:]))
+    for i, a in enumerate(out):
+        a[:] = i
+        pool.filled(a)
+    view = out[1][:1].view(np.int8).reshape(1, 1)
+    place = out[1].ctypes.data
+    out[1] = None
+    assert pool.take(nbytes) is None                    # (a view is left)
+    del view, a
+    again = pool.take(nbytes)
+    assert again.ctypes.data == place
+    del again                                           # (not filled: given back to the system, not to the pool)
+    assert not pool._free and pool.take(nbytes) is not None and not pool._free
+    assert pool.take(pool.MOST_BYTES + 1) is None and pool.take(0) is None
+    pool.close()
+    assert pool.take(nbytes) is None
+    assert all((out[i] == i).all() for i in (0, 2, 3))
