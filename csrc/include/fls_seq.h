@@ -39,6 +39,10 @@ int fls_seq_group_rmsnorm(const float* x, int ldx, const int* idx, const float* 
 // that only fls_seq_moe_sum and fls_seq_group_rmsnorm take
 int fls_seq_moe_sum_add_group_rmsnorm(float* x, int ldx, const float* y, int ldy, const int* dest, const float* mw, int top, const float* w,
                                       float woff, int rows, int D, int groups, float eps, fls_stream_t s);
+// the same and then h = norm(x; w2 + woff2) of the new x, h of type th
+int fls_seq_moe_sum_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const int* dest, const float* mw, int top, const float* w,
+                                           float woff, const float* w2, float woff2, void* h, int th, int ldh, int rows, int D, int groups,
+                                           float eps, fls_stream_t s);
 // x += norm(y; w + woff), then h = norm(x; w2 + woff2) of the new x, both per group of D / groups columns; h of type th
 int fls_seq_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const float* w, float woff, const float* w2, float woff2,
                                    void* h, int th, int ldh, int rows, int D, int groups, float eps, fls_stream_t s);
@@ -252,6 +256,12 @@ int fls_seq_rmsnorm_pair(float* x, int ldx, const float* add, int ldadd, const f
 int fls_seq_parallel_update(float* x, int ldx, const float* a, int lda, const float* wa, const float* b, int ldb, const float* wb,
                             const float* y, int ldy, const int* dest, const float* w, const int* ids, int top, int E, const void* h,
                             int th, int ldh, int rows, int D, fls_stream_t s);
+// fls_seq_parallel_update and then fls_seq_rmsnorm_pair of the new x with outputs of type th (h's too); SEQ_NOT_SERVED: rows whose alignment or
+// width only those two take
+int fls_seq_parallel_update_norms(float* x, int ldx, const float* a, int lda, const float* wa, const float* b, int ldb, const float* wb,
+                                  const float* y, int ldy, const int* dest, const float* w, const int* ids, int top, int E, const void* h, int ldh,
+                                  const float* add, int ldadd, const float* w1, void* h1, int ld1, const float* w2, void* h2, int ld2, int th,
+                                  int rows, int D, float eps, fls_stream_t s);
 // rows z = [query latent (qr) | latent (r) | rotated key part (dr) | ...] of a latent attention: cq = rms(query latent) qw (qr = 0:
 // none), row kv_slot[t] of the pool (pw wide) = [rms(latent) kw | key part rotated in pairs (i, i + rot / 2), angle
 // tok_pos freqs[i]]; cq and the pool of type tp

@@ -175,7 +175,7 @@ def _load_kernels(path: str = _KERNELS):
     return _Quick(lib)
 
 
-SEQ_ABI = 21   # csrc/include/fls_seq.h
+SEQ_ABI = 22   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -188,6 +188,7 @@ def _load_seq():
     _bind(lib, "fls_seq_gemm", i, p, i, p, i, p, i, p, p, i, i, f, f, i, i, i, i, i, i, i, p, p, ll, i, ll, ll, p, p)
     _bind(lib, "fls_seq_gemm_tile_of", i, i, i, i, i, i, i, i, i)
     _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm", i, p, i, p, i, p, p, i, p, f, i, i, i, f, p)
+    _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm_next", i, p, i, p, i, p, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
     _bind(lib, "fls_seq_group_rmsnorm", i, p, i, p, p, p, i, i, i, i, i, f, i, f, i, p)
     _bind(lib, "fls_seq_residual_branches", i, p, i, i, p, i, p, p, i, p, f, p, i, p, i, i, p, i, i, i, f, p)
@@ -227,6 +228,7 @@ def _load_seq():
     _bind(lib, "fls_seq_moe_route_softmax_grouped", i, p, i, p, i, i, i, i, i, f, p, p, p, p, p, p, p)
     _bind(lib, "fls_seq_rmsnorm_pair", i, p, i, p, i, p, p, i, p, p, i, i, i, i, f, p)
     _bind(lib, "fls_seq_parallel_update", i, p, i, p, i, p, p, i, p, p, i, p, p, p, i, i, p, i, i, i, i, p)
+    _bind(lib, "fls_seq_parallel_update_norms", i, p, i, p, i, p, p, i, p, p, i, p, p, p, i, i, p, i, p, i, p, p, i, p, p, i, i, i, i, f, p)
     _bind(lib, "fls_seq_latent_rows", i, p, i, i, i, i, p, p, f, p, i, p, p, p, i, p, i, i, i, p)
     _bind(lib, "fls_seq_gated_delta_scan", i, p, i, p, i, p, i, p, i, p, p, p, p, i, i, p, p, p, i, i, i, i, i, i, i, f, f, f, i, p, i, p)
     _bind(lib, "fls_seq_streams_norm", i, p, i, p, p, p, p, i, i, i, i, i, f, p)

@@ -546,6 +546,20 @@ class ShardedRunner:
             self.seq_cache.release(rid)
         return out
 
+    def _in_turn(self, names, W):
+        """The layers ``names``, which run one behind the other on the same rows, each with the one ahead of it in a hybrid model's context."""
+        if not self.hybrid:
+            for name in names:
+                yield name
+            return
+        self.ctx.normed = None
+        try:
+            for name, nxt in zip(names, list(names[1:]) + [None]):
+                self.ctx.ahead = (nxt, W[nxt]) if nxt is not None else None
+                yield name
+        finally:
+            self.ctx.ahead = self.ctx.normed = None
+
     def _step_graphable(self, entries) -> bool:
         """A decode step (one token per request) on resident weights on one GPU: it replays as one
         captured HIP graph (runtime/graphs.py StepGraphs; FLS_DECODE_GRAPHS=0 turns it off)."""
@@ -561,7 +575,7 @@ class ShardedRunner:
         if self._decode_graphs is None:
             def forward(meta):
                 state = None
-                for name in self.names:
+                for name in self._in_turn(self.names, self._W_all):
                     state = self._run_layer(self.ctx, name, self._W_all[name], state, None, meta)
                 return state, self.ops.argmax_f32(state, meta["mirror"])
             self._decode_graphs = StepGraphs(self.dev, forward, self.ops, self.cfg.vocab_size)
@@ -860,8 +874,7 @@ class ShardedRunner:
         last_use = idx + 1 >= len(px.items) or px.items[idx + 1][0] != k
         tc = time.perf_counter()
         with trace.range(f"shard{k}:mb{b}:compute"):
-            for li in self.my_shards[k]:
-                name = self.names[li]
+            for name in self._in_turn([self.names[li] for li in self.my_shards[k]], px.W):
                 if hasattr(px.W[name], "final_use"):
                     px.W[name].final_use = last_use
                 state = self._run_layer(self.ctx, name, px.W[name], state, batch, meta)

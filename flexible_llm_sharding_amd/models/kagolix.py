@@ -151,6 +151,10 @@ class HybridContext:
     device: torch.device
     compute_dtype: torch.dtype
     cache: Optional[object] = None           # runtime.seq_state.SequenceStateCache
+    # The layer that runs on the rows right after this one, (name, weights), where the engine has its weights at hand (the same shard); a family
+    # whose layers end in a row-wise update may make its first norm in the same pass and leave it in ``normed``, which that layer takes.
+    ahead: Optional[tuple] = None
+    normed: Optional[object] = None
     embed_out: Optional[torch.Tensor] = None
     act_dtype: torch.dtype = torch.float32   # the residual stream
     # (fields the engine's pass machinery reads on every context)
@@ -210,14 +214,30 @@ def _moe(ctx, mlp: dict, W, h):
     return ops.grouped_matmul_nt(a, W["wdown"], route.offs), route        # fp32 rows by expert
 
 
+def _next_norm(ctx, meta):
+    """The weight of the norm that the rows go through next, if the layer ahead is known and takes every row."""
+    if ctx.ahead is None:
+        return None
+    name, W = ctx.ahead
+    if layer_kind(name) == "decoder":
+        return W["norm1"]
+    return W["norm"] if layer_kind(name) == "norm" and meta.get("all_rows") else None
+
+
 def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
     cfg, ops, cdt = ctx.cfg, ctx.ops, ctx.compute_dtype
     L = cfg.layer(name)
     ng, eps = cfg.norm_groups, cfg.norm_eps
-    h = ops.group_rmsnorm(x, W["norm1"], ng, eps, out_dtype=cdt)
+    h, ctx.normed = ctx.normed, None
+    if h is None:
+        h = ops.group_rmsnorm(x, W["norm1"], ng, eps, out_dtype=cdt)
     y = {"attention": _attention, "rglru": _rglru, "mamba2": _mamba2}[L.type](ctx, L.mixer, W, h, meta, name)
+    nw = _next_norm(ctx, meta)                   # with the next layer's norm in the last update's pass
     if L.mlp is None:
-        ops.add_group_rmsnorm_(x, y, W["norm1b"], ng, eps)
+        if nw is None:
+            ops.add_group_rmsnorm_(x, y, W["norm1b"], ng, eps)
+        else:
+            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], nw, ng, eps, out_dtype=cdt)
     else:
         h = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], W["norm2"], ng, eps, out_dtype=cdt)
         if L.mlp["kind"] == "dense":
@@ -225,8 +245,14 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
             y = ops.matmul_nt(ops.matmul_nt(h, W["wup"], xielu=W["act"], out_dtype=cdt), W["wdown"])
         else:
             y, route = _moe(ctx, L.mlp, W, h)
-            return ops.add_group_rmsnorm_moe_(x, y, route, W["norm2b"], ng, eps)
-        ops.add_group_rmsnorm_(x, y, W["norm2b"], ng, eps)
+            if nw is None:
+                return ops.add_group_rmsnorm_moe_(x, y, route, W["norm2b"], ng, eps)
+            ctx.normed = ops.add_group_rmsnorm_moe_next_(x, y, route, W["norm2b"], nw, ng, eps, out_dtype=cdt)
+            return x
+        if nw is None:
+            ops.add_group_rmsnorm_(x, y, W["norm2b"], ng, eps)
+        else:
+            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm2b"], nw, ng, eps, out_dtype=cdt)
     return x
 
 
@@ -241,6 +267,9 @@ def run_layer(ctx, name: str, W: Dict[str, torch.Tensor], state, batch, meta: di
     if kind == "decoder":
         return run_block(ctx, W, state, meta, name)
     if kind == "norm":
+        h, ctx.normed = ctx.normed, None
+        if h is not None:
+            return h
         return ops.group_rmsnorm(state, W["norm"], cfg.norm_groups, cfg.norm_eps, out_dtype=ctx.compute_dtype,
                                  row_idx=meta["want_idx"])
     return ops.matmul_nt(state, W["head"], softcap=cfg.logit_softcap, mirror=meta.get("mirror"))

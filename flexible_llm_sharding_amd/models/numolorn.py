@@ -247,14 +247,23 @@ def run_block(ctx, W, xs: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
     L, D = cfg.layer(name), cfg.width
     x = xs[:, :D]
     # both norms of the row in one pass; a pass other than the first adds the embedding row on the way
-    h1, h2 = ops.rmsnorm_pair(x, W["norm1"], W.get("norm2"), cfg.norm_eps, ctx.compute_dtype, add=xs[:, D:] if cfg.reenters(name) else None)
+    # (by the layer before, in the pass of its update, where this one's weights were at hand)
+    normed, ctx.normed = ctx.normed, None
+    norms = lambda n, w: dict(w1=w["norm1"], w2=w.get("norm2"), eps=cfg.norm_eps, out_dtype=ctx.compute_dtype,
+                              add=xs[:, D:] if cfg.reenters(n) else None)
+    h1, h2 = normed if normed is not None else ops.rmsnorm_pair(x, **norms(name, W))
     y = _MIXERS[L.type](ctx, L, W, h1, meta, name)
-    if L.mlp is None:
-        ops.parallel_update_(x, y, W["ls1"])
-    elif L.mlp["kind"] == "dense":
-        ops.parallel_update_(x, y, W["ls1"], _dense(ctx, L.mlp, W, h2), W["ls2"])
+    b = moe = None
+    if L.mlp is not None:
+        if L.mlp["kind"] == "dense":
+            b = _dense(ctx, L.mlp, W, h2)
+        else:
+            moe = _moe(ctx, L.mlp, W, h2)
+    wb = W["ls2"] if L.mlp is not None else None
+    if ctx.ahead is not None and layer_kind(ctx.ahead[0]) == "decoder":
+        ctx.normed = ops.parallel_update_norms_(x, y, W["ls1"], b, wb, moe, **norms(*ctx.ahead))
     else:
-        ops.parallel_update_(x, y, W["ls1"], wb=W["ls2"], moe=_moe(ctx, L.mlp, W, h2))
+        ops.parallel_update_(x, y, W["ls1"], b, wb, moe)
     return xs
 
 

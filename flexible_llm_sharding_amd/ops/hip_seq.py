@@ -46,6 +46,14 @@ def _vec(t: torch.Tensor, name: str, n: int, dtype=torch.float32):
     return t
 
 
+def _ptr(t):
+    return t.data_ptr() if t is not None else None
+
+
+def _ld(t):
+    return t.stride(0) if t is not None else 0
+
+
 class HostRows:
     """Where a step's logits and their argmax go on the host: ``cell`` (one int64 on the device) holds the address of rows x vocab
     floats and, behind them, the rows' argmax, or 0: nowhere; ``rows_there``: the logits are written already."""
@@ -178,7 +186,9 @@ class HipSeqOps:
                                          _CODE[out_dtype], T, D, float(eps), _stream()), "fls_seq_rmsnorm_pair")
         return h1, h2
 
-    def parallel_update_(self, x, a, wa, b=None, wb=None, moe=None):
+    @staticmethod
+    def _parallel_args(x, a, wa, b, wb, moe):
+        """The arguments of the residual update of two sublayers, checked -> (x .. ids, top, E as the kernels take them, the experts' input rows)."""
         _rows(x, "x", torch.float32)
         T, D = x.shape
         for nme, t in (("a", a), ("b", b)):
@@ -201,12 +211,35 @@ class HipSeqOps:
             _rows(h, "h")
             if y.shape != (T * top, D) or tuple(h.shape) != (T, D) or dest.shape[0] != T:
                 raise ValueError("parallel_update_: the experts' rows do not fit")
-        ptr = lambda t: t.data_ptr() if t is not None else None
-        ld = lambda t: t.stride(0) if t is not None else 0
-        _chk(self.k.fls_seq_parallel_update(x.data_ptr(), x.stride(0), a.data_ptr(), a.stride(0), wa.data_ptr(), ptr(b), ld(b), ptr(wb),
-                                            ptr(y), ld(y), ptr(dest), ptr(w), ptr(ids), top, int(E), ptr(h),
-                                            _code(h, "h") if h is not None else 0, ld(h), T, D, _stream()), "fls_seq_parallel_update")
+        return (x.data_ptr(), x.stride(0), a.data_ptr(), a.stride(0), wa.data_ptr(), _ptr(b), _ld(b), _ptr(wb), _ptr(y), _ld(y), _ptr(dest),
+                _ptr(w), _ptr(ids), top, int(E)), h
+
+    def parallel_update_(self, x, a, wa, b=None, wb=None, moe=None):
+        args, h = self._parallel_args(x, a, wa, b, wb, moe)
+        _chk(self.k.fls_seq_parallel_update(*args, _ptr(h), _code(h, "h") if h is not None else 0, _ld(h), x.shape[0], x.shape[1], _stream()),
+             "fls_seq_parallel_update")
         return x
+
+    def parallel_update_norms_(self, x, a, wa, b, wb, moe, w1, w2, eps, out_dtype, add=None):
+        args, h = self._parallel_args(x, a, wa, b, wb, moe)
+        T, D = x.shape
+        _vec(w1, "w1", D)
+        if w2 is not None:
+            _vec(w2, "w2", D)
+        if add is not None:
+            _rows(add, "add", torch.float32)
+            if tuple(add.shape) != (T, D):
+                raise ValueError("parallel_update_norms_: add is shaped unlike x")
+        if h is None or h.dtype == out_dtype:
+            h1 = torch.empty(T, D, dtype=out_dtype, device=x.device)
+            h2 = torch.empty(T, D, dtype=out_dtype, device=x.device) if w2 is not None else None
+            rc = self.k.fls_seq_parallel_update_norms(*args, _ptr(h), _ld(h), _ptr(add), _ld(add), w1.data_ptr(), h1.data_ptr(), D, _ptr(w2),
+                                                      _ptr(h2), D, _CODE[out_dtype], T, D, float(eps), _stream())
+            if rc != self.NOT_SERVED:
+                _chk(rc, "fls_seq_parallel_update_norms")
+                return h1, h2
+        self.parallel_update_(x, a, wa, b, wb, moe)
+        return self.rmsnorm_pair(x, w1, w2, eps, out_dtype, add=add)
 
     def latent_rows(self, z, q_rank, r, dr, q_norm, kv_norm, eps, rot, rows, meta, out_dtype):
         _rows(z, "z", torch.float32)
@@ -1047,6 +1080,24 @@ class HipSeqOps:
             return self.add_group_rmsnorm_(x, self.moe_weighted_sum(y, route), w, groups, eps)
         _chk(rc, "fls_seq_moe_sum_add_group_rmsnorm")
         return x
+
+    def add_group_rmsnorm_moe_next_(self, x, y, route, w, w2, groups, eps, out_dtype):
+        _rows(x, "x", torch.float32)
+        _rows(y, "y", torch.float32)
+        T, top = route.dest.shape
+        if x.shape != (T, y.shape[1]):
+            raise ValueError("add_group_rmsnorm_moe_next_: shapes differ")
+        _vec(w, "w", x.shape[1])
+        _vec(w2, "w2", x.shape[1])
+        h = torch.empty(x.shape, dtype=out_dtype, device=x.device)
+        rc = self.k.fls_seq_moe_sum_add_group_rmsnorm_next(x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), route.dest.data_ptr(),
+                                                           route.w.data_ptr(), top, w.data_ptr(), 0.0, w2.data_ptr(), 0.0, h.data_ptr(),
+                                                           _CODE[out_dtype], h.stride(0), T, x.shape[1], groups, float(eps), _stream())
+        if rc == self.NOT_SERVED:
+            self.add_group_rmsnorm_moe_(x, y, route, w, groups, eps)
+            return self.group_rmsnorm(x, w2, groups, eps, out_dtype)
+        _chk(rc, "fls_seq_moe_sum_add_group_rmsnorm_next")
+        return h
 
     def moe_weighted_sum(self, y, route):
         _rows(y, "y", torch.float32)

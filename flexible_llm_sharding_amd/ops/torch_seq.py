@@ -64,6 +64,11 @@ class TorchSeqOps:
         """``add_group_rmsnorm_`` of a mixture's output: the weighted sum of its rows ``y``, which lie sorted by expert."""
         return self.add_group_rmsnorm_(x, self.moe_weighted_sum(y, route), w, groups, eps)
 
+    def add_group_rmsnorm_moe_next_(self, x, y, route, w, w2, groups, eps, out_dtype):
+        """``add_group_rmsnorm_moe_`` and the norm of the new rows by ``w2``, which it returns."""
+        self.add_group_rmsnorm_moe_(x, y, route, w, groups, eps)
+        return self.group_rmsnorm(x, w2, groups, eps, out_dtype)
+
     def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype):
         """``add_group_rmsnorm_`` and the norm of the new rows by ``w2``, which it returns."""
         self.add_group_rmsnorm_(x, y, w, groups, eps)
@@ -109,6 +114,11 @@ class TorchSeqOps:
             new = new + b.float() * wb.float()
         x.add_(new)
         return x
+
+    def parallel_update_norms_(self, x, a, wa, b, wb, moe, w1, w2, eps, out_dtype, add=None):
+        """``parallel_update_`` and then ``rmsnorm_pair`` of the new rows."""
+        self.parallel_update_(x, a, wa, b, wb, moe)
+        return self.rmsnorm_pair(x, w1, w2, eps, out_dtype, add=add)
 
     def dyt_norm(self, x, wb, alpha, out_dtype, row_idx=None):
         """Dynamic Tanh: tanh(alpha x) w + b elementwise, no statistics of the row; ``wb`` = [w; b] ([2, D]),

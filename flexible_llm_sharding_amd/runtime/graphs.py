@@ -303,7 +303,7 @@ class _StepInputs:
         self.address = words[:2].view(np.int64)
         self.views = list(arrays.views(words).values())
         self.meta = arrays.views(self.flat)
-        self.meta.update(n_seqs=B, max_rows=1)
+        self.meta.update(n_seqs=B, max_rows=1, all_rows=True)          # (every row's logits)
 
     def fill(self, host: Dict[str, np.ndarray], address: int) -> None:
         """(the step that last read ``up`` has been waited for)"""

@@ -1912,6 +1912,42 @@ def test_side_by_side_rows(ops, cdt, tol, D):
         close(xa, xb, 1e-5)
 
 
+# a layer's last update with the next layer's norms in its pass: the bits of the two steps in turn, for widths about the pieces of 1,024 columns, the
+# widest that rows in registers take, and widths and alignments that only the two steps serve
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,pad", [(4, 0), (1020, 0), (1024, 4), (1028, 0), (2048, 0), (4100, 0), (8192, 0), (8196, 0), (35, 0), (64, 3)])
+def test_update_with_the_next_norms(ops, cdt, D, pad):
+    H, R = ops
+    torch.manual_seed(D + pad)
+    T, E, Z, top = 7, 5, 8, 3
+    wide = torch.randn(T, 2 * (D + pad), device=DEV)
+    w1, w2, n1, n2 = (torch.randn(D, device=DEV) for _ in range(4))
+    a, b = torch.randn(T, D, device=DEV), torch.randn(T, D, device=DEV)
+    h, y = torch.randn(T, D, device=DEV).to(cdt), torch.randn(T * top, D, device=DEV)
+    route = R.moe_route_softmax_grouped(torch.randn(T, Z, device=DEV) * 2, None, top, 4, 3, 1.3)
+    y[int(route.offs[E]):] = float("nan")                                   # (rows of identity experts are never made)
+    for bb, wb, moe in ((None, None, None), (b, w2, None), (None, w2, (y, route, h, E))):
+        for second, add in ((n2, False), (None, False), (n2, True)):
+            xa, xb = wide.clone(), wide.clone()
+            extra = lambda x: x[:, D + pad:2 * D + pad] if add else None
+            g = H.parallel_update_norms_(xa[:, :D], a, w1, bb, wb, moe, n1, second, 1e-5, cdt, add=extra(xa))
+            H.parallel_update_(xb[:, :D], a, w1, bb, wb, moe)
+            want = H.rmsnorm_pair(xb[:, :D], n1, second, 1e-5, cdt, add=extra(xb))
+            assert torch.equal(xa, xb) and torch.equal(g[0], want[0]) and (torch.equal(g[1], want[1]) if second is not None else g[1] is None)
+    route = H.moe_route_corrected(torch.randn(T, E, device=DEV), torch.randn(E, device=DEV) * 0.1, top)
+    y = torch.randn(T * top, D, device=DEV)
+    for groups in (1, 2):
+        if D % groups:
+            continue
+        xa, xb = wide.clone(), wide.clone()
+        g = H.add_group_rmsnorm_moe_next_(xa[:, :D], y, route, w1, n1, groups, 1e-6, cdt)
+        H.add_group_rmsnorm_moe_(xb[:, :D], y, route, w1, groups, 1e-6)
+        assert torch.equal(xa, xb) and torch.equal(g, H.group_rmsnorm(xb[:, :D], n1, groups, 1e-6, cdt))
+        g = H.add_group_rmsnorm_next_(xa[:, :D], a, w1, n1, groups, 1e-6, cdt)
+        H.add_group_rmsnorm_(xb[:, :D], a, w1, groups, 1e-6)
+        assert torch.equal(xa, xb) and torch.equal(g, H.group_rmsnorm(xb[:, :D], n1, groups, 1e-6, cdt))
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 @pytest.mark.parametrize("qr,r,dr,rot", [(9, 11, 8, 8), (1536, 512, 64, 64), (0, 40, 0, 0), (4, 12, 3, 2), (300, 1, 0, 0), (0, 512, 512, 64)])
 def test_latent_rows(ops, cdt, tol, qr, r, dr, rot):
