@@ -177,14 +177,37 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(const half_t* __restrict
   for (int c = threadIdx.x; c < H / 8; c += 256) dst[c] = src[c];
 }
 
+// greedy tokens: probabilities are >= 0, so their bit patterns order like their values; each thread keeps (bits, first index)
+__device__ __forceinline__ void argmax_join(unsigned& best, int& bi, unsigned b, int i) {
+  if (b > best || (b == best && i < bi)) {
+    best = b;
+    bi = i;
+  }
+}
+
+// over the block's threads; thread 0 gets the result
+template <int NT>
+__device__ __forceinline__ void argmax_block(unsigned& best, int& bi, unsigned* sb, int* si) {
+  for (int s = 32; s > 0; s >>= 1) argmax_join(best, bi, __shfl_xor(best, s, 64), __shfl_xor(bi, s, 64));
+  if ((threadIdx.x & 63) == 0) {
+    sb[threadIdx.x >> 6] = best;
+    si[threadIdx.x >> 6] = bi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int w = 1; w < NT / 64; ++w) argmax_join(best, bi, sb[w], si[w]);
+}
+
 // softmax over a row of fp16 logits -> fp16 probabilities (fp32 math),
 // online max/sum in one pass, normalisation in a second (row stays in L2).
 // inv_scale != 1: the logits are first fp16(l * inv_scale) (Granite's logits / logits_scaling).
 // One block a row and few rows a call: latency bound, so a wide vocabulary takes 1,024 threads (16 rows of 32,000:
 // 14.4 -> 8.7 us against 256 threads; of 151,936: 71 -> 35 us).
-template <int NT>
+// GREEDY: the first index of each row's largest probability too (argmax_rows_kernel's answer), found while they are written:
+// a launch and a pass over the rows less (16 rows of 32,000: 8.7 + 7.9 us).
+template <int NT, bool GREEDY>
 __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ logits, half_t* __restrict__ probs,
-                                                    int V, float inv_scale) {
+                                                    int V, float inv_scale, int* __restrict__ greedy) {
   const bool scaled = inv_scale != 1.f;
   auto ld = [=](half_t h) { return scaled ? (float)(half_t)((float)h * inv_scale) : (float)h; };
   __shared__ float red[NT / 64];
@@ -215,6 +238,8 @@ __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ 
   const float gm = block_max(m, red);
   const float gs = block_sum(m == -INFINITY ? 0.f : s * __expf(m - gm), red);
   const float inv = 1.f / gs;
+  unsigned best = 0;
+  int bi = 0x7fffffff;
   if (vec) {
     for (int c = threadIdx.x; c < V / 8; c += NT) {
       const half8 v = *(const half8*)(lr + c * 8);
@@ -222,24 +247,32 @@ __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ 
 #pragma unroll
       for (int j = 0; j < 8; ++j) o[j] = (half_t)(__expf(ld(v[j]) - gm) * inv);
       *(half8*)(pr + c * 8) = o;
+      if constexpr (GREEDY) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) argmax_join(best, bi, __builtin_bit_cast(unsigned short, (half_t)o[j]), c * 8 + j);
+      }
     }
   } else {
-    for (int c = threadIdx.x; c < V; c += NT) pr[c] = (half_t)(__expf(ld(lr[c]) - gm) * inv);
+    for (int c = threadIdx.x; c < V; c += NT) {
+      const half_t o = (half_t)(__expf(ld(lr[c]) - gm) * inv);
+      pr[c] = o;
+      if constexpr (GREEDY) argmax_join(best, bi, __builtin_bit_cast(unsigned short, o), c);
+    }
+  }
+  if constexpr (GREEDY) {
+    __shared__ unsigned sb[NT / 64];
+    __shared__ int si[NT / 64];
+    argmax_block<NT>(best, bi, sb, si);
+    if (threadIdx.x == 0) greedy[blockIdx.x] = bi == 0x7fffffff ? 0 : bi;
   }
 }
+
 
 // greedy token of each row of fp16 probabilities: the FIRST index of the row's maximum (numpy
 // argmax on the scores the reference hands back, main.py:85-88).  Probabilities are >= 0, so
 // their bit patterns order like their values; each thread keeps (bits, first index), then a reduction over
 // the lanes and the waves.  One block a row: latency bound, hence 1,024 threads and eight values a load where rows
 // are 16-byte aligned (16 rows of 32,000: 40 -> 7.9 us against 256 threads and one value a load; of 151,936: 201 -> 20 us).
-__device__ __forceinline__ void argmax_join(unsigned& best, int& bi, unsigned b, int i) {
-  if (b > best || (b == best && i < bi)) {
-    best = b;
-    bi = i;
-  }
-}
-
 __global__ __launch_bounds__(1024) void argmax_rows_kernel(const half_t* __restrict__ x, int ld, int V, int vec,
                                                          int* __restrict__ out) {
   __shared__ unsigned sb[16];
@@ -259,16 +292,8 @@ __global__ __launch_bounds__(1024) void argmax_rows_kernel(const half_t* __restr
     }
   }
   for (int c = nv * 8 + threadIdx.x; c < V; c += 1024) argmax_join(best, bi, r[c], c);
-  for (int s = 32; s > 0; s >>= 1) argmax_join(best, bi, __shfl_xor(best, s, 64), __shfl_xor(bi, s, 64));
-  if ((threadIdx.x & 63) == 0) {
-    sb[threadIdx.x >> 6] = best;
-    si[threadIdx.x >> 6] = bi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w) argmax_join(best, bi, sb[w], si[w]);
-    out[blockIdx.x] = bi == 0x7fffffff ? 0 : bi;
-  }
+  argmax_block<1024>(best, bi, sb, si);
+  if (threadIdx.x == 0) out[blockIdx.x] = bi == 0x7fffffff ? 0 : bi;
 }
 
 // counter-based normal generator (splitmix64 -> Box-Muller), 8 values/thread
@@ -478,14 +503,12 @@ extern "C" int fls_embed(const int* ids, const void* table, void* out, int T, in
   return 0;
 }
 
-extern "C" int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, fls_stream_t s) {
+extern "C" int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, int* greedy, fls_stream_t s) {
   if (rows <= 0) return 0;
-  if (V >= 4096)
-    hipLaunchKernelGGL(softmax_kernel<1024>, dim3(rows), dim3(1024), 0, (hipStream_t)s, (const half_t*)logits,
-                       (half_t*)probs, V, inv_scale);
-  else
-    hipLaunchKernelGGL(softmax_kernel<256>, dim3(rows), dim3(256), 0, (hipStream_t)s, (const half_t*)logits,
-                       (half_t*)probs, V, inv_scale);
+#define SOFTMAX(NT, GREEDY) hipLaunchKernelGGL((softmax_kernel<NT, GREEDY>), dim3(rows), dim3(NT), 0, (hipStream_t)s, (const half_t*)logits, (half_t*)probs, V, inv_scale, greedy)
+  if (V >= 4096) { if (greedy != nullptr) SOFTMAX(1024, true); else SOFTMAX(1024, false); }
+  else { if (greedy != nullptr) SOFTMAX(256, true); else SOFTMAX(256, false); }
+#undef SOFTMAX
   FLS_CHECK_LAUNCH();
   return 0;
 }

@@ -37,7 +37,7 @@ from . import knobs
 from .config import MAX_TOKEN_LEN, ModelConfig, is_hybrid
 from .models.layout import layer_kind
 from .models import hybrid_family
-from .models.llama import ExecContext, layer_flops, rope_tables, run_layer
+from .models.llama import ExecContext, Scored, layer_flops, rope_tables, run_layer
 from .ops import get_ops
 from .parallel.comm import Comm
 from .parallel.pipeline import StageInbox, build_programs, host_wait, rank_items, rx_key
@@ -662,7 +662,7 @@ class ShardedRunner:
             self.tps, self.batches, self.metas, self.store, self.items = tps, batches, metas, store, items
             self.pos = {it: i for i, it in enumerate(items)}
             self.outputs: List[Optional[np.ndarray]] = [None] * len(tps)
-            self.out_pending = []      # (batch, host tensor, event, pool buffer)
+            self.out_pending = []      # (batch, host tensor, its memory's owner, greedy tokens)
             self.carry = {}            # micro-batch -> device activation kept across a shard boundary
             self.sends = []            # (tensor, work) of outputs in flight to another rank
             self.shard_ev: List = []   # end-of-shard events on the compute stream (host run-ahead bound)
@@ -905,7 +905,8 @@ class ShardedRunner:
             # stays on this rank (contiguous stages) leaves the slot first
             state = state.clone()
         if last == self.L - 1:
-            px.out_pending.append(self._start_output_copy(px.batches[b], state))
+            # (nothing of the pass runs behind its last item: no other stream for its copy)
+            px.out_pending.append(self._start_output_copy(px.batches[b], state, px.prog is None and px.items[-1] == (k, b)))
         elif px.dst_rank != self.comm.rank:
             st = state.contiguous()
             w = self.comm.isend(st, px.dst_rank)
@@ -974,7 +975,7 @@ class ShardedRunner:
             px.inbox.end_call()
             rx_stats = {f"rx_{k}": float(v) for k, v in px.inbox.stats.items()}
         self.last_tokens = [None] * len(px.tps)
-        for batch, host, ev, pool_buf, am in px.out_pending:
+        for batch, host, pool_buf, am in px.out_pending:
             self._collect(batch, host.numpy(), am, px.outputs, pool_buf)
         store.clear()
         store.trim()                   # pinned pool follows this call's shapes
@@ -1093,12 +1094,17 @@ class ShardedRunner:
     ACT_BUFFER_SLACK = 1
 
     # ------------------------------------------------------ HIP graphs
-    def _forward_all(self, meta: dict, batch: PackedBatch) -> torch.Tensor:
+    def _forward_all(self, meta: dict, batch: PackedBatch) -> Scored:
         """embed -> every layer -> norm -> head on resident weights (captured by GraphedForward)."""
         state = None
         for name in self.names:
             state = run_layer(self.ctx, name, self._W_all[name], state, batch, meta)
-        return state
+        return self._scored(state)
+
+    def _scored(self, probs: torch.Tensor) -> Scored:
+        """The head's result with its greedy tokens, which the head made or which are made here."""
+        scored, self.ctx.scored = self.ctx.scored, None
+        return scored if scored is not None else Scored(probs, self.ops.argmax_rows(probs), None)
 
     def _decode_graphable(self, batches, cached: bool) -> bool:
         """A decode-like call (suffix K/V reuse: prefixes and kept suffix tokens from the cache)
@@ -1162,18 +1168,16 @@ class ShardedRunner:
         return outputs
 
     def _enqueue_graphed(self, batches, run):
-        """Replay every micro-batch (``run(batch, index) -> probs``), its row argmax and the D2H
-        of both into pooled pinned buffers, all on the current stream -> (pending, argmax tensors,
+        """Replay every micro-batch (``run(batch, index) -> Scored``) and the D2H
+        of its probabilities and greedy tokens into pooled pinned buffers, all on the current stream -> (pending, argmax tensors,
         decoder FLOPs)."""
         pending, ams, flops = [], [], 0.0
         for i, batch in enumerate(batches):
-            probs = run(batch, i)
-            am = self.ops.argmax_rows(probs)
-            pool_buf, host, host_am = self._output_block(probs)
-            host.copy_(probs, non_blocking=True)     # same stream: ordered before the next replay
-            host_am.copy_(am, non_blocking=True)
+            scored = run(batch, i)
+            pool_buf, host, host_am = self._output_down(scored)     # same stream: ordered before the next replay
             pending.append((batch, host, pool_buf, host_am))
-            ams.append(am)
+            # (a graph's own tokens: the step enqueued next reads them, perhaps after another replay of it)
+            ams.append(scored.greedy.clone() if self.spec_steps > 0 else scored.greedy)
             # every unpruned decoder layer has the same count: one evaluation each way (80 per step
             # cost 3.4 ms of host time, on the path that must stay under a generation step's GPU time)
             pruned = [self._pruned(n) for n in self.names if layer_kind(n) == "decoder"]
@@ -1358,9 +1362,11 @@ class ShardedRunner:
             print(f"rank{self.comm.rank}: resuming at shard {k0} from {ck.dir}")
         return ck, k0, (ck.load(k0) if k0 else {})
 
-    def _output_block(self, probs: torch.Tensor):
-        """Pinned memory for a micro-batch's results -> (its owner, the rows, their argmax): a block that the caller gets
-        (hostmem.ResultBlocks), or where none is to be had a buffer of the store's pool that the caller's copies are made from."""
+    def _output_down(self, scored: Scored):
+        """The copies of a micro-batch's results into pinned memory, on the current stream -> (the memory's owner, the rows and their argmax there).  The
+        owner: a block that the caller gets (hostmem.ResultBlocks), or where none is to be had a buffer of the store's pool that the
+        caller's copies are made from."""
+        probs = scored.probs
         nbytes, rows = probs.numel() * probs.element_size(), probs.shape[0]
         at = -(-nbytes // 16) * 16
         if self._results is None:
@@ -1370,10 +1376,16 @@ class ShardedRunner:
             buf = torch.from_numpy(owner)
         else:
             owner = buf = self._get_store().host_buffer(at + 4 * rows)
-        return owner, buf[:nbytes].view(probs.dtype).view(probs.shape), buf[at:at + 4 * rows].view(torch.int32)
+        host, host_am = buf[:nbytes].view(probs.dtype).view(probs.shape), buf[at:at + 4 * rows].view(torch.int32)
+        if scored.flat is not None:
+            buf[:at + 4 * rows].copy_(scored.flat, non_blocking=True)
+        else:
+            host.copy_(probs, non_blocking=True)
+            host_am.copy_(scored.greedy, non_blocking=True)
+        return owner, host, host_am
 
     def _output_landed(self, owner) -> None:
-        """The copies into a block of :meth:`_output_block` have been waited for (and a pool buffer's rows taken)."""
+        """The copies of :meth:`_output_down` have been waited for (and a pool buffer's rows taken)."""
         if isinstance(owner, np.ndarray):
             hostmem.ResultBlocks.filled(owner)
         else:
@@ -1398,26 +1410,28 @@ class ShardedRunner:
         if owner is not None:
             self._output_landed(owner)
 
-    def _start_output_copy(self, batch: PackedBatch, probs: torch.Tensor):
+    def _start_output_copy(self, batch: PackedBatch, probs: torch.Tensor, last: bool):
         """D2H of a micro-batch's probabilities and of their row argmax (the greedy token of
-        each suffix: api.generation_loop needs no host pass over the [n_s, V] scores)."""
+        each suffix: api.generation_loop needs no host pass over the [n_s, V] scores), beside what the pass computes next unless it is its
+        ``last``."""
         if isinstance(batch, StepBatch):
-            am = self.ops.argmax_f32(probs)                # (fp32 logits of the wanted rows)
+            scored = Scored(probs, self.ops.argmax_f32(probs), None)          # (fp32 logits of the wanted rows)
+        elif self.ctx.scored is not None or hasattr(self.ops, "argmax_rows"):
+            scored = self._scored(probs)
         else:
-            am = self.ops.argmax_rows(probs) if hasattr(self.ops, "argmax_rows") else None
+            scored = Scored(probs, None, None)
         if not self.cuda:
-            return batch, probs.detach().to(torch.float32 if self.hybrid else torch.float16).cpu(), None, None, am
-        pool_buf, host, host_am = self._output_block(probs)
-        self.d2h_stream.wait_stream(torch.cuda.current_stream(self.dev))
-        with torch.cuda.stream(self.d2h_stream):
-            host.copy_(probs, non_blocking=True)
-            probs.record_stream(self.d2h_stream)
-            if am is not None:
-                host_am.copy_(am, non_blocking=True)
-                am.record_stream(self.d2h_stream)
-            ev = torch.cuda.Event()
-            ev.record(self.d2h_stream)
-        return batch, host, ev, pool_buf, (host_am if am is not None else None)
+            return batch, probs.detach().to(torch.float32 if self.hybrid else torch.float16).cpu(), None, scored.greedy
+        if last:
+            owner, host, host_am = self._output_down(scored)
+        else:
+            self.d2h_stream.wait_stream(torch.cuda.current_stream(self.dev))
+            with torch.cuda.stream(self.d2h_stream):
+                owner, host, host_am = self._output_down(scored)
+                for t in scored:
+                    if t is not None:
+                        t.record_stream(self.d2h_stream)
+        return batch, host, owner, host_am
 
     def close(self):
         if self._spec is not None:             # an enqueued speculative step finishes first

@@ -18,7 +18,7 @@ from __future__ import annotations
 
 import math
 from dataclasses import dataclass
-from typing import Dict, Optional
+from typing import Dict, NamedTuple, Optional
 
 import torch
 
@@ -162,6 +162,13 @@ class Workspace:
         return 0 if self.buf is None else self.buf.numel() * self.buf.element_size()
 
 
+class Scored(NamedTuple):
+    """What the LM head leaves: the scored rows' probabilities, their argmax and, where they lie in one buffer, its bytes."""
+    probs: torch.Tensor
+    greedy: torch.Tensor
+    flat: Optional[torch.Tensor]
+
+
 @dataclass
 class ExecContext:
     cfg: ModelConfig
@@ -198,6 +205,7 @@ class ExecContext:
     ss_buf: Optional[torch.Tensor] = None      # the arena-backed buffer (grown, reused)
     ss_cur: Optional[torch.Tensor] = None      # the buffer the last residual GEMM wrote
     ss_key: Optional[tuple] = None
+    scored: Optional[Scored] = None            # of the head that ran last, until the engine takes it (backends that make both at once)
 
     def phase(self, *shapes) -> None:
         """Start a workspace phase that will carve ``shapes`` (rows, cols) in order."""
@@ -605,6 +613,9 @@ def run_norm(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, meta
 
 
 def run_head(ctx: ExecContext, W: Dict[str, torch.Tensor], h: torch.Tensor) -> torch.Tensor:
+    if hasattr(ctx.ops, "lm_head_scores"):
+        ctx.scored = Scored(*ctx.ops.lm_head_scores(h, W["head"], logits_scaling=ctx.cfg.logits_scaling))
+        return ctx.scored.probs
     return ctx.ops.lm_head_softmax(h, W["head"], logits_scaling=ctx.cfg.logits_scaling)
 
 

@@ -505,8 +505,20 @@ class HipOps:
         rows, V = logits.shape
         probs = torch.empty_like(logits)
         _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
-                                     _stream()), "fls_softmax")
+                                     None, _stream()), "fls_softmax")
         return probs
+
+    def softmax_greedy(self, logits, logits_scaling: float = 1.0):
+        """-> (:meth:`softmax`, its :meth:`argmax_rows`, the bytes of both in a row), in one launch."""
+        _f16(logits, "logits")
+        rows, V = logits.shape
+        n = 2 * rows * V
+        at = -(-n // 16) * 16                                # (host copies lay them out alike)
+        flat = torch.empty(at + 4 * rows, dtype=torch.uint8, device=logits.device)
+        probs, greedy = flat[:n].view(torch.float16).view(rows, V), flat[at:].view(torch.int32)
+        _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
+                                     greedy.data_ptr(), _stream()), "fls_softmax")
+        return probs, greedy, flat
 
     def argmax_rows(self, probs):
         """[rows] int32: the first index of each row's maximum (non-negative fp16 probabilities)."""
@@ -518,6 +530,9 @@ class HipOps:
 
     def lm_head_softmax(self, h, w, logits_scaling: float = 1.0):
         return self.softmax(self.linear(h, w), logits_scaling)
+
+    def lm_head_scores(self, h, w, logits_scaling: float = 1.0):
+        return self.softmax_greedy(self.linear(h, w), logits_scaling)
 
     def cast_f16(self, dst: torch.Tensor, src: torch.Tensor, src_code: int) -> None:
         """dst (fp16 bytes) = fp16(src bytes of bf16 (code 1; may be in place) or fp32 (code 2))."""

@@ -127,7 +127,7 @@ class _Graph:
     def __init__(self, meta: Dict[str, torch.Tensor]):
         self.meta = meta                     # static device inputs
         self.graph = torch.cuda.CUDAGraph()
-        self.out: torch.Tensor = None        # static device output [S, V]
+        self.out = None                      # static device output: llama.Scored, or a step's (logits, argmax)
         self.replays = 0
         self.arrays: Optional[_Arrays] = None      # DecodeGraphs: ``meta``'s places in ``flat``
         self.flat: Optional[torch.Tensor] = None
@@ -138,7 +138,7 @@ class _Graph:
 class GraphedForward:
     """LRU cache of captured whole-model forwards, keyed by the bucketed shape.
 
-    ``forward(meta, batch) -> probs`` must run embed..head for one micro-batch
+    ``forward(meta, batch) -> llama.Scored`` must run embed..head for one micro-batch
     on the current stream using only ``meta`` (device tensors) and resident
     weights; it is called eagerly once (warm-up) and then under capture.
     """
@@ -168,8 +168,8 @@ class GraphedForward:
         self.captures += 1
         return g
 
-    def run(self, batch: PackedBatch) -> torch.Tensor:
-        """Replay (capturing on first sight of the bucket); returns [n_scored, V] on the device."""
+    def run(self, batch: PackedBatch):
+        """Replay (capturing on first sight of the bucket) -> the scored rows on the device (llama.Scored)."""
         key = bucket_key(batch)
         g = self.graphs.get(key)
         if g is None:
@@ -184,7 +184,8 @@ class GraphedForward:
         g.graph.replay()
         g.replays += 1
         self.replays += 1
-        return g.out[:batch.n_scored]
+        n = batch.n_scored
+        return g.out._replace(probs=g.out.probs[:n], greedy=g.out.greedy[:n], flat=g.out.flat if n == g.out.probs.shape[0] else None)
 
 
 class DecodeGraphs:
@@ -245,8 +246,8 @@ class DecodeGraphs:
         g.staging[g.next_stage] = (views, pinned, ev)
         g.next_stage = (g.next_stage + 1) % len(g.staging)
 
-    def run(self, batch: PackedBatch, entry, ids_dev: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """Replay (capture on the first sight of the shape) -> the static [n_scored, V] output.
+    def run(self, batch: PackedBatch, entry, ids_dev: Optional[torch.Tensor] = None):
+        """Replay (capture on the first sight of the shape) -> the static output (llama.Scored).
         ``ids_dev``: the batch's token ids as a device int32 tensor, copied over ``batch.ids`` on
         the stream (a speculative step whose new tokens are the previous step's device argmax).
         The metadata goes in by a stream-ordered copy from pinned memory, so a replay can be

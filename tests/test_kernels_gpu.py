@@ -1242,6 +1242,26 @@ def test_argmax_rows_widths(ops, V):
         assert np.array_equal(ops.argmax_rows(x).cpu().numpy(), np.argmax(x.cpu().numpy(), axis=-1)), ld
 
 
+# the softmax with its greedy tokens: the bits of the two kernels, about a block's threads and eight values each, odd widths, ties and rows of one value, -inf
+# and NaN among the logits; both lie in the flat bytes as a host copy has them
+@pytest.mark.parametrize("V", [1, 7, 8, 1000, 2047, 4095, 4096, 8193, 32000, 32003])
+@pytest.mark.parametrize("scaling", [1.0, 8.0])
+def test_softmax_greedy(ops, V, scaling):
+    x = (torch.randn(5, V, generator=torch.Generator().manual_seed(V)) * 4).round().div(2).half()
+    x[1] = 0.25
+    x[2, V - 1] = 30.0
+    x[3, :V // 2] = float("-inf")
+    x[4, V // 3] = float("nan")
+    x = x.to(DEV)
+    probs, greedy, flat = ops.softmax_greedy(x, scaling)
+    want = ops.softmax(x, scaling)
+    assert torch.equal(probs.view(torch.int16), want.view(torch.int16)) and torch.equal(greedy, ops.argmax_rows(want))
+    assert np.array_equal(greedy[:4].cpu().numpy(), np.argmax(want[:4].cpu().numpy(), axis=-1))
+    host = flat.cpu()
+    at = (10 * V + 15) // 16 * 16
+    assert torch.equal(host[:10 * V].view(torch.int16), want.cpu().view(torch.int16).flatten()) and torch.equal(host[at:].view(torch.int32), greedy.cpu())
+
+
 # the statistic of a residual product's rows has the same bits from the partials it leaves and from its rows, on every path by rows (skinny,
 # blocks of 64 rows, split, tiles), and the product does not depend on which of the two is asked for
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 79, 128, 129, 300, 1000, 4100])
