@@ -17,7 +17,7 @@
 //     half-tile super-phases in flight, one counted vmcnt + raw s_barrier per
 //     two phases, LDS fragment reads and DMA interleaved into the MFMA stream.
 //     XCD-aware bijective block remap + grouped tile order (guide T1).
-//   * gemm_nt_col16 — 16-column blocks, K-tiles of 256, for M <= 64 and narrow outputs;
+//   * gemm_nt_col16 — blocks of 16 columns or pairs of columns, for M <= 64 and narrow outputs;
 //   * gemm_nt_mid — 64 x 128 x 64 tiles, 3-deep LDS-DMA ring, for M too small
 //     to fill 256 CUs with 256 x 256 tiles, and for odd K-tile counts (v10's
 //     body is unrolled over two K-tiles); 4 waves, or 8 (two per SIMD) for
@@ -334,42 +334,50 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   }
 }
 
-// 16-column blocks for M <= 64 and N below a round of 32-column mid blocks (the O / down projections of a 7B-sized
-// generation step: N = 4,096, 128 blocks of 32): what bounds those is the bytes in flight, one block's ring on half the
-// CUs, with 64 rows of A staged whatever M is.  Here every CU streams 16 weight rows, K-tiles of 256 (two rows a DMA
-// instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile; only ceil(M / 16) row
+// Blocks of 16 columns (N below a round of 32-column mid blocks: the O / down projections of a 7B-sized generation step, N = 4,096, 128 blocks
+// of 32), or of 16 pairs (a RoPE column and its partner, a gate and its up column), for M <= 64: what bounds the wider ones is the bytes in flight, one
+// block's ring on half the CUs, with 64 rows of A staged whatever M is.  Here a block streams 16 or 32 weight rows, K-tiles of 256 or 128 (two or four
+// rows a DMA instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile, pairs two blocks a CU; only ceil(M / 16) row
 // tiles of A are staged, wave w multiplies row tile w, the others only move data.  Same fragments, MFMA and K order as
 // the mid blocks: bitwise equal rows.  M = 16, K = 4,096 and 11,008 in turn (124 MB in both): 35.8 -> 16.6 us on average, 13 at
-// the rate of a large copy.
+// the rate of a large copy.  Pairs, M = 16 (us, 64-column mid blocks and these): 22,016 x 4,096 42.5, 35.2; 12,288 x 4,096 26.1, 25.3; 6,144 x 4,096
+// 22.5, 14.9; 5,120 x 2,048 12.7, 7.6; M = 64 23.9, 19.7 and 13.8, 11.4.  (A ring for W and a shorter one for A, loaded by waves of their own: 1.5 to 2 us slower.)
 namespace col16 {
-constexpr int KT = 256;
-constexpr int stage_bytes(int rt) { return 16 * (1 + rt) * KT * 2; }
-constexpr int stages(int rt) { return rt == 1 ? 8 : rt == 2 ? 6 : 3; }      // 128 / 144 / 120 KB
+constexpr int kt(int rt, int np) { return np == 2 && rt > 1 ? 128 : 256; }
+constexpr int stage_bytes(int rt, int np) { return 16 * (np + rt) * kt(rt, np) * 2; }
+constexpr int stages(int rt, int np) { return np == 2 ? (rt == 2 ? 5 : 3) : rt == 1 ? 8 : rt == 2 ? 6 : 3; }       // 128 / 144 / 120 KB; pairs 72 / 80 / 72
 }  // namespace col16
 
-template <int EPI, int RT>
+template <int EPI, int RT, int NP>
 __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
                                                    int ldc, Epi ep) {
-  constexpr int KT = col16::KT, NST = col16::stages(RT), STAGE = col16::stage_bytes(RT);
-  constexpr int PER_WAVE = 8 * (1 + RT) / 4;           // 1 KB DMA groups (two rows) of a stage, per wave
+  constexpr int KT = col16::kt(RT, NP), NST = col16::stages(RT, NP), STAGE = col16::stage_bytes(RT, NP);
+  constexpr int LPR = KT / 8, RPD = 64 / LPR, GP = 16 / RPD;               // lanes a row, rows a DMA group of 1 KB, groups a panel of 16 rows
+  constexpr int PER_WAVE = GP * (NP + RT) / 4;           // 1 KB DMA groups (two rows) of a stage, per wave
   extern __shared__ __attribute__((aligned(16))) char lds_c16[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
-  const int n0 = blockIdx.x * 16, nk = K / KT;
+  const int b = blockIdx.x, nk = K / KT;
+  // a pair's second column is hd / 2 rows on (SwiGLU: I rows)
+  const int n0 = EPI == FLS_EPI_ROPE ? (b >> 2) * 128 + (b & 3) * 16 : EPI == EPI_ROPE64 ? (b >> 1) * 64 + (b & 1) * 16 : b * 16;
+  const int second = EPI == FLS_EPI_ROPE ? 64 : EPI == EPI_ROPE64 ? 32 : ep.gu_rows;
   const half_t* src[PER_WAVE];                         // groups 0 .. 7: W rows, then A rows
 #pragma unroll
   for (int i = 0; i < PER_WAVE; ++i) {
-    const int g = wave + 4 * i, row = (g & 7) * 2 + (lane >> 5);          // row inside its tile of 16
-    const int kc = ((lane & 31) ^ row) * 8;
-    src[i] = g < 8 ? W + (size_t)(n0 + row) * ldw + kc : A + (size_t)min((g / 8 - 1) * 16 + row, M - 1) * lda + kc;
+    const int g = wave + 4 * i, row = g % GP * RPD + lane / LPR;           // row inside its panel
+    const int kc = ((lane % LPR) ^ row) * 8;
+    src[i] = g < GP * NP ? W + (size_t)(n0 + (NP == 2 && g >= GP ? second : 0) + row) * ldw + kc
+                         : A + (size_t)min((g / GP - NP) * 16 + row, M - 1) * lda + kc;
   }
   auto stage = [&](int s, int kt) {
     char* base = lds_c16 + (s % NST) * STAGE;
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) glds16(src[i] + (size_t)kt * KT, base + (wave + 4 * i) * 1024);
   };
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  floatx4 acc[NP];
+#pragma unroll
+  for (int h = 0; h < NP; ++h) acc[h] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int d = 0; d < NST - 1; ++d) stage(d, min(d, nk - 1));
   for (int kt = 0; kt < nk; ++kt) {
@@ -379,34 +387,42 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
     stage(kt + NST - 1, min(kt + NST - 1, nk - 1));    // (past the end: the last tile again, into a stage nobody reads)
     if (wave < RT) {
       const char* Ws = lds_c16 + (kt % NST) * STAGE + fr * (KT * 2);
-      const char* Xs = Ws + (1 + wave) * 16 * KT * 2;
-      half8 wf[KT / 32], xf[KT / 32];
+      const char* Xs = Ws + (NP + wave) * 16 * KT * 2;
+      half8 wf[NP][KT / 32], xf[KT / 32];
 #pragma unroll
       for (int ks = 0; ks < KT / 32; ++ks) {
         const int c = ((ks * 4 + grp) ^ fr) << 4;
-        wf[ks] = *(const half8*)(Ws + c);
+#pragma unroll
+        for (int h = 0; h < NP; ++h) wf[h][ks] = *(const half8*)(Ws + h * (16 * KT * 2) + c);
         xf[ks] = *(const half8*)(Xs + c);
       }
 #pragma unroll
-      for (int ks = 0; ks < KT / 32; ++ks) acc = mfma16x16x32(wf[ks], xf[ks], acc);
+      for (int ks = 0; ks < KT / 32; ++ks)
+#pragma unroll
+        for (int h = 0; h < NP; ++h) acc[h] = mfma16x16x32(wf[h][ks], xf[ks], acc[h]);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   const int m = wave * 16 + fr;
-  if (wave < RT && m < M) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc, ep);
+  if (wave < RT && m < M) {
+    if constexpr (NP == 1) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc[0], ep);
+    else if constexpr (is_rope(EPI)) store_rope_pair(C, ldc, m, n0 + 4 * grp, acc[0], acc[1], ep);
+    else store_pair_off<EPI>(C, ldc, m, b * 32, 4 * grp, acc[0], acc[1], ep);
+  }
 }
 
 template <int EPI, int RT>
 void launch_col16(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
                   const Epi& ep, hipStream_t s) {
-  constexpr int lds = col16::stages(RT) * col16::stage_bytes(RT);
+  constexpr int NP = EPI == FLS_EPI_NONE || EPI == FLS_EPI_RESID ? 1 : 2;
+  constexpr int lds = col16::stages(RT, NP) * col16::stage_bytes(RT, NP);
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm_nt_col16<EPI, RT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)hipFuncSetAttribute((const void*)gemm_nt_col16<EPI, RT, NP>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
-  hipLaunchKernelGGL((gemm_nt_col16<EPI, RT>), dim3(N / 16), dim3(256), lds, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
+  hipLaunchKernelGGL((gemm_nt_col16<EPI, RT, NP>), dim3(N / (16 * NP)), dim3(256), lds, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
 }
 
 int g_order = 0;             // 0: by shape, else a fixed signed group size (fls_gemm_set_order)
@@ -648,8 +664,16 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
   // down projections of generation steps with <= 12 prompts (M <= 64: 128 -> 256 blocks)
   const bool bn32 = !pairs && N % 32 == 0 && g_mid_waves != 4 &&
                     (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
-  // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
-  if (bn32 && g_mid_bn == 0 && N / 32 < 256 && K % col16::KT == 0) return MID_16;
+  // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks).  16 pairs a block: 672 random products
+  // that this rule gives them take 0.70 of the mid blocks' time (worst 1.02).  Up to a round of them the mid blocks leave half of the CUs idle; above
+  // it, up to 16 rows, they have the 64-row tile's staging of A to carry, but few K-tiles, or two rounds of the mid blocks that end together (768 .. 1,024), are
+  // as fast there (0.98 to 1.27), and with more rows everything above a round is (1.04 to 1.4).
+  const int pair_blocks = N / 32;
+  const bool few = M <= mid::BMm && K % 256 == 0 && g_mid_waves != 4;
+  if (few && pairs && (g_mid_bn == 16 || (g_mid_bn == 0 && (pair_blocks <= 256 || (M <= 16 && K >= 1024 && (pair_blocks <= 512 ||
+                                                            (K >= 1280 && pair_blocks <= 768) || pair_blocks > 1024))))))
+    return MID_16;
+  if (few && (g_mid_bn == 16 || (bn32 && g_mid_bn == 0 && N / 32 < 256))) return MID_16;
   if (bn32) return MID_32;
   if (bn64) return w8_64 ? MID_64 : MID_64_W4;
   if (w8) return r128 ? MID_128R : MID_128;
@@ -663,6 +687,9 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
 struct MidCost { float start, k_few, k_full, start2, k2, k2_more, tb; };       // tb: bytes of weight a us, in millions
 const MidCost MID_16_COST[3] = {{4.7f, 0.05f, 0.152f, 7.4f, 0.199f, 0.f, 4.76f}, {5.f, 0.092f, 0.165f, 7.8f, 0.247f, 0.f, 4.97f},
                                 {4.7f, 0.147f, 0.207f, 6.8f, 0.33f, 0.f, 4.99f}};        // up to 16, 32 and 64 rows
+// (pairs; their starts 2 us up: they were timed launch to launch in a graph)
+const MidCost MID_P16_COST[3] = {{4.7f, 0.111f, 0.17f, 6.2f, 0.25f, 0.13f, 5.5f}, {4.7f, 0.125f, 0.197f, 6.f, 0.25f, 0.13f, 5.2f},
+                                 {4.7f, 0.185f, 0.27f, 6.f, 0.27f, 0.13f, 5.2f}};
 const MidCost MID_32_COST = {4.4f, 0.269f, 0.337f, 6.f, 0.415f, 0.f, 4.2f};
 const MidCost MID_64_COST[2] = {{4.8f, 0.279f, 0.452f, 6.7f, 0.658f, 0.f, 4.8f}, {4.9f, 0.288f, 0.366f, 5.9f, 0.524f, 0.f, 5.f}};      // up to 64, 128 rows
 const MidCost MID_128_COST[2] = {{7.f, 0.38f, 0.543f, 8.9f, 0.833f, 0.173f, 5.6f}, {5.5f, 0.387f, 0.476f, 7.8f, 0.65f, 0.235f, 5.f}};
@@ -671,11 +698,11 @@ float mid_us(int M, int N, int K, bool pairs) {
   const MidForm form = mid_form(M, N, K, pairs, true);
   const int tiles_m = (M + 63) / 64;
   const float nk = (float)(K / BK), bytes = (float)N * K * 2.f;
-  const MidCost& c = form == MID_16 ? MID_16_COST[M <= 16 ? 0 : M <= 32 ? 1 : 2]
+  const MidCost& c = form == MID_16 ? (pairs ? MID_P16_COST : MID_16_COST)[M <= 16 ? 0 : M <= 32 ? 1 : 2]
                      : form == MID_32 ? MID_32_COST
                      : form == MID_64 || form == MID_64_W4 ? MID_64_COST[M > 64]
                      : form == MID_128R ? MID_128R_COST : MID_128_COST[M > 128];
-  const int width = form == MID_16 ? 16 : form == MID_32 ? 32 : form == MID_64 || form == MID_64_W4 ? 64 : 128;
+  const int width = form == MID_16 ? (pairs ? 32 : 16) : form == MID_32 ? 32 : form == MID_64 || form == MID_64_W4 ? 64 : 128;
   const float rounds = (float)((form == MID_128R ? (M + 127) / 128 : tiles_m) * (N / width)) / 256.f;
   if (form == MID_128_W4) return (4.f + 0.532f * nk) * powf(rounds, 0.842f);
   if (rounds <= 1.f) return c.start + fmaxf(bytes / (c.tb * 1e6f), (c.k_few + (c.k_full - c.k_few) * rounds) * nk);
@@ -747,7 +774,8 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
       least = us;
     }
   };
-  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs));
+  // (no lead for blocks of 16 pairs, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's)
+  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (rules == ROUTE_MID && pairs && mid_form(M, N, K, pairs, true) == MID_16 ? 1.f / 0.94f : 1.f));
   if (skinny) offer(ROUTE_SKINNY, skinny_us(M, N, K, bn, S));
   if (split) offer(ROUTE_SPLIT, split_us(M, N, K, S2));
   if (M > 64) {              // (up to 64 rows one row tile covers them all, and three quarters of a 256-row one are padding)
@@ -819,11 +847,9 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
     switch (mid_form(M, N, K, pairs, N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0))) {
       case MID_16:
-        if constexpr (!pairs) {
-          if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-          else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-          else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        }
+        if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         break;
       case MID_32:
         if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
@@ -944,11 +970,11 @@ extern "C" int fls_row_stat(const void* x, int ldx, int rows, int H, float eps, 
   return 0;
 }
 
-// mid-M block columns: 0 auto (default), 32, 64 or 128 forced where valid (tests / A-B; 32: NONE / RESID
-// epilogues, 8 waves); returns the previous
+// mid-M block columns: 0 auto (default), 16 (M <= 64), 32, 64 or 128 forced where valid (tests / A-B; 32: NONE / RESID
+// epilogues, 8 waves; 16: pairs of columns where the epilogue joins two); returns the previous
 extern "C" int fls_gemm_set_mid_bn(int bn) {
   const int old = g_mid_bn;
-  g_mid_bn = bn == 32 || bn == 64 || bn == 128 ? bn : 0;
+  g_mid_bn = bn == 16 || bn == 32 || bn == 64 || bn == 128 ? bn : 0;
   return old;
 }
 
