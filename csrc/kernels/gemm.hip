@@ -334,14 +334,15 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   }
 }
 
-// Blocks of 16 columns (N below a round of 32-column mid blocks: the O / down projections of a 7B-sized generation step, N = 4,096, 128 blocks
-// of 32), or of 16 pairs (a RoPE column and its partner, a gate and its up column), for M <= 64: what bounds the wider ones is the bytes in flight, one
+// Blocks of 16 columns (the O / down projections of a 7B-sized generation step, N = 4,096, 128 mid blocks
+// of 32), or of two panels of 16 (neighbours, or pairs: a RoPE column and its partner, a gate and its up column), for M <= 64: what bounds the wider ones is the bytes in flight, one
 // block's ring on half the CUs, with 64 rows of A staged whatever M is.  Here a block streams 16 or 32 weight rows, K-tiles of 256 or 128 (two or four
-// rows a DMA instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile, pairs two blocks a CU; only ceil(M / 16) row
+// rows a DMA instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile, of two panels two blocks a CU; only ceil(M / 16) row
 // tiles of A are staged, wave w multiplies row tile w, the others only move data.  Same fragments, MFMA and K order as
 // the mid blocks: bitwise equal rows.  M = 16, K = 4,096 and 11,008 in turn (124 MB in both): 35.8 -> 16.6 us on average, 13 at
 // the rate of a large copy.  Pairs, M = 16 (us, 64-column mid blocks and these): 22,016 x 4,096 42.5, 35.2; 12,288 x 4,096 26.1, 25.3; 6,144 x 4,096
-// 22.5, 14.9; 5,120 x 2,048 12.7, 7.6; M = 64 23.9, 19.7 and 13.8, 11.4.  (A ring for W and a shorter one for A, loaded by waves of their own: 1.5 to 2 us slower.)
+// 22.5, 14.9; 5,120 x 2,048 12.7, 7.6; M = 64 23.9, 19.7 and 13.8, 11.4.  Two panels, plain, 16 rows (32-column mid blocks
+// before): 8,192 x 8,192 45.1, 33.1; 8,192 x 28,672 147, 88.  (A ring for W and a shorter one for A, loaded by waves of their own: 1.5 to 2 us slower.)
 namespace col16 {
 constexpr int kt(int rt, int np) { return np == 2 && rt > 1 ? 128 : 256; }
 constexpr int stage_bytes(int rt, int np) { return 16 * (np + rt) * kt(rt, np) * 2; }
@@ -359,9 +360,10 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
   const int b = blockIdx.x, nk = K / KT;
-  // a pair's second column is hd / 2 rows on (SwiGLU: I rows)
-  const int n0 = EPI == FLS_EPI_ROPE ? (b >> 2) * 128 + (b & 3) * 16 : EPI == EPI_ROPE64 ? (b >> 1) * 64 + (b & 1) * 16 : b * 16;
-  const int second = EPI == FLS_EPI_ROPE ? 64 : EPI == EPI_ROPE64 ? 32 : ep.gu_rows;
+  // a pair's second column is hd / 2 rows on (SwiGLU: I rows; no pairs: the next 16)
+  const int n0 = EPI == FLS_EPI_ROPE ? (b >> 2) * 128 + (b & 3) * 16 : EPI == EPI_ROPE64 ? (b >> 1) * 64 + (b & 1) * 16
+                 : b * (EPI == FLS_EPI_SWIGLU ? 16 : 16 * NP);
+  const int second = EPI == FLS_EPI_ROPE ? 64 : EPI == EPI_ROPE64 ? 32 : EPI == FLS_EPI_SWIGLU ? ep.gu_rows : 16;
   const half_t* src[PER_WAVE];                         // groups 0 .. 7: W rows, then A rows
 #pragma unroll
   for (int i = 0; i < PER_WAVE; ++i) {
@@ -412,10 +414,9 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   }
 }
 
-template <int EPI, int RT>
+template <int EPI, int RT, int NP>
 void launch_col16(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
                   const Epi& ep, hipStream_t s) {
-  constexpr int NP = EPI == FLS_EPI_NONE || EPI == FLS_EPI_RESID ? 1 : 2;
   constexpr int lds = col16::stages(RT, NP) * col16::stage_bytes(RT, NP);
   static bool attr = false;
   if (!attr) {
@@ -639,7 +640,18 @@ int splitk_slices(int M, int N, int K, size_t tiles, size_t ws_bytes) {
 enum Route { ROUTE_NONE, ROUTE_SKINNY, ROUTE_SPLIT, ROUTE_MID, ROUTE_128, ROUTE_192, ROUTE_256, ROUTE_V11 };
 
 // The blocks that the mid-M path takes.
-enum MidForm { MID_16, MID_32, MID_64, MID_64_W4, MID_128R, MID_128, MID_128_W4 };
+enum MidForm { MID_16, MID_16X2, MID_32, MID_64, MID_64_W4, MID_128R, MID_128, MID_128_W4 };
+// Blocks of 16 pairs, or of two 16-column panels, for up to 64 rows.  Up to a round of them the mid blocks leave half of the CUs idle (plain
+// products of up to 128: the 16-column blocks fill them).  Above it, up to 16 rows (plain ones to 32), the mid blocks have the 64-row tile's staging of A to
+// carry, but few K-tiles, or two rounds of the mid blocks that end together (768 .. 1,024), are as fast there (0.98 to 1.27), and with more rows
+// everything above a round is (1.0 to 1.4).  Random products that this rule gives them: 672 pairs 0.70 of the mid blocks' time (worst 1.02), plain
+// ones 0.62 to 0.87 up to a round, 0.83 to 0.95 above.
+bool two_panels(int M, int N, int K, bool pairs) {
+  const int b = N / 32;
+  if (b <= 256) return pairs || b > 128;
+  if (!pairs && M <= 32 && K >= 2560 && b <= 768) return true;
+  return M <= 16 && K >= 1024 && (b <= 512 || (K >= 1280 && b <= 768) || (b > 1024 && (pairs || K >= 2048)));
+}
 // pairs: an epilogue that joins columns (SwiGLU, RoPE).  K % 128 == 0
 MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
   // 64-column blocks for a single row tile whose 128-column grid fills less than one round of the
@@ -664,16 +676,10 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
   // down projections of generation steps with <= 12 prompts (M <= 64: 128 -> 256 blocks)
   const bool bn32 = !pairs && N % 32 == 0 && g_mid_waves != 4 &&
                     (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
-  // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks).  16 pairs a block: 672 random products
-  // that this rule gives them take 0.70 of the mid blocks' time (worst 1.02).  Up to a round of them the mid blocks leave half of the CUs idle; above
-  // it, up to 16 rows, they have the 64-row tile's staging of A to carry, but few K-tiles, or two rounds of the mid blocks that end together (768 .. 1,024), are
-  // as fast there (0.98 to 1.27), and with more rows everything above a round is (1.04 to 1.4).
-  const int pair_blocks = N / 32;
+  // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
   const bool few = M <= mid::BMm && K % 256 == 0 && g_mid_waves != 4;
-  if (few && pairs && (g_mid_bn == 16 || (g_mid_bn == 0 && (pair_blocks <= 256 || (M <= 16 && K >= 1024 && (pair_blocks <= 512 ||
-                                                            (K >= 1280 && pair_blocks <= 768) || pair_blocks > 1024))))))
-    return MID_16;
-  if (few && (g_mid_bn == 16 || (bn32 && g_mid_bn == 0 && N / 32 < 256))) return MID_16;
+  if (few && (g_mid_bn == 33 || (g_mid_bn == 16 && pairs) || (g_mid_bn == 0 && two_panels(M, N, K, pairs)))) return MID_16X2;
+  if (few && !pairs && (g_mid_bn == 16 || (bn32 && g_mid_bn == 0 && N / 32 < 256))) return MID_16;
   if (bn32) return MID_32;
   if (bn64) return w8_64 ? MID_64 : MID_64_W4;
   if (w8) return r128 ? MID_128R : MID_128;
@@ -687,9 +693,9 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
 struct MidCost { float start, k_few, k_full, start2, k2, k2_more, tb; };       // tb: bytes of weight a us, in millions
 const MidCost MID_16_COST[3] = {{4.7f, 0.05f, 0.152f, 7.4f, 0.199f, 0.f, 4.76f}, {5.f, 0.092f, 0.165f, 7.8f, 0.247f, 0.f, 4.97f},
                                 {4.7f, 0.147f, 0.207f, 6.8f, 0.33f, 0.f, 4.99f}};        // up to 16, 32 and 64 rows
-// (pairs; their starts 2 us up: they were timed launch to launch in a graph)
-const MidCost MID_P16_COST[3] = {{4.7f, 0.111f, 0.17f, 6.2f, 0.25f, 0.13f, 5.5f}, {4.7f, 0.125f, 0.197f, 6.f, 0.25f, 0.13f, 5.2f},
-                                 {4.7f, 0.185f, 0.27f, 6.f, 0.27f, 0.13f, 5.2f}};
+// (two panels; their starts 2 us up: they were timed launch to launch in a graph)
+const MidCost MID_16X2_COST[3] = {{4.7f, 0.111f, 0.17f, 6.2f, 0.3f, 0.08f, 5.5f}, {4.7f, 0.125f, 0.197f, 6.2f, 0.33f, 0.08f, 5.2f},
+                                  {4.7f, 0.185f, 0.27f, 6.f, 0.27f, 0.13f, 5.2f}};
 const MidCost MID_32_COST = {4.4f, 0.269f, 0.337f, 6.f, 0.415f, 0.f, 4.2f};
 const MidCost MID_64_COST[2] = {{4.8f, 0.279f, 0.452f, 6.7f, 0.658f, 0.f, 4.8f}, {4.9f, 0.288f, 0.366f, 5.9f, 0.524f, 0.f, 5.f}};      // up to 64, 128 rows
 const MidCost MID_128_COST[2] = {{7.f, 0.38f, 0.543f, 8.9f, 0.833f, 0.173f, 5.6f}, {5.5f, 0.387f, 0.476f, 7.8f, 0.65f, 0.235f, 5.f}};
@@ -698,11 +704,11 @@ float mid_us(int M, int N, int K, bool pairs) {
   const MidForm form = mid_form(M, N, K, pairs, true);
   const int tiles_m = (M + 63) / 64;
   const float nk = (float)(K / BK), bytes = (float)N * K * 2.f;
-  const MidCost& c = form == MID_16 ? (pairs ? MID_P16_COST : MID_16_COST)[M <= 16 ? 0 : M <= 32 ? 1 : 2]
+  const MidCost& c = form == MID_16 || form == MID_16X2 ? (form == MID_16 ? MID_16_COST : MID_16X2_COST)[M <= 16 ? 0 : M <= 32 ? 1 : 2]
                      : form == MID_32 ? MID_32_COST
                      : form == MID_64 || form == MID_64_W4 ? MID_64_COST[M > 64]
                      : form == MID_128R ? MID_128R_COST : MID_128_COST[M > 128];
-  const int width = form == MID_16 ? (pairs ? 32 : 16) : form == MID_32 ? 32 : form == MID_64 || form == MID_64_W4 ? 64 : 128;
+  const int width = form == MID_16 ? 16 : form == MID_16X2 || form == MID_32 ? 32 : form == MID_64 || form == MID_64_W4 ? 64 : 128;
   const float rounds = (float)((form == MID_128R ? (M + 127) / 128 : tiles_m) * (N / width)) / 256.f;
   if (form == MID_128_W4) return (4.f + 0.532f * nk) * powf(rounds, 0.842f);
   if (rounds <= 1.f) return c.start + fmaxf(bytes / (c.tb * 1e6f), (c.k_few + (c.k_full - c.k_few) * rounds) * nk);
@@ -774,8 +780,8 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
       least = us;
     }
   };
-  // (no lead for blocks of 16 pairs, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's)
-  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (rules == ROUTE_MID && pairs && mid_form(M, N, K, pairs, true) == MID_16 ? 1.f / 0.94f : 1.f));
+  // (no lead for blocks of two panels, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's)
+  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (rules == ROUTE_MID && M <= 64 && two_panels(M, N, K, pairs) ? 1.f / 0.94f : 1.f));
   if (skinny) offer(ROUTE_SKINNY, skinny_us(M, N, K, bn, S));
   if (split) offer(ROUTE_SPLIT, split_us(M, N, K, S2));
   if (M > 64) {              // (up to 64 rows one row tile covers them all, and three quarters of a 256-row one are padding)
@@ -847,9 +853,16 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
     switch (mid_form(M, N, K, pairs, N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0))) {
       case MID_16:
-        if (M <= 16) launch_col16<EPI, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        else if (M <= 32) launch_col16<EPI, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        else launch_col16<EPI, 4>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        if constexpr (!pairs) {
+          if (M <= 16) launch_col16<EPI, 1, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+          else if (M <= 32) launch_col16<EPI, 2, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+          else launch_col16<EPI, 4, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        }
+        break;
+      case MID_16X2:
+        if (M <= 16) launch_col16<EPI, 1, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else if (M <= 32) launch_col16<EPI, 2, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else launch_col16<EPI, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         break;
       case MID_32:
         if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
@@ -971,10 +984,10 @@ extern "C" int fls_row_stat(const void* x, int ldx, int rows, int H, float eps, 
 }
 
 // mid-M block columns: 0 auto (default), 16 (M <= 64), 32, 64 or 128 forced where valid (tests / A-B; 32: NONE / RESID
-// epilogues, 8 waves; 16: pairs of columns where the epilogue joins two); returns the previous
+// epilogues, 8 waves; 16: two panels where the epilogue joins columns; 33: two panels); returns the previous
 extern "C" int fls_gemm_set_mid_bn(int bn) {
   const int old = g_mid_bn;
-  g_mid_bn = bn == 16 || bn == 32 || bn == 64 || bn == 128 ? bn : 0;
+  g_mid_bn = bn == 16 || bn == 33 || bn == 32 || bn == 64 || bn == 128 ? bn : 0;
   return old;
 }
 

@@ -560,20 +560,21 @@ def test_gemm_col16_bitwise(ops, N, K):
     assert rel_err(got[0], x.float() @ w.float().t() + b.float()) < 2e-3
 
 
-# pairs of columns, 16 a block (RoPE of both head sizes, with columns behind the rotated ones; SwiGLU): the 64-column mid blocks' bits, for rows about a
+# two panels of 16 columns a block (RoPE of both head sizes, with columns behind the rotated ones; SwiGLU; plain and residual): the 64-column mid blocks' bits, for rows about a
 # 16-row tile, a K of one tile, fewer and more than their ring, one block and a round of them
-@pytest.mark.parametrize("N,K", [(256, 256), (256, 1792), (1280, 4096), (8192, 512)])
-def test_gemm_col16_pairs_bitwise(ops, N, K):
+@pytest.mark.parametrize("N,K", [(256, 256), (256, 1792), (1280, 4096), (8192, 512), (8320, 2560)])
+def test_gemm_col16_two_panels_bitwise(ops, N, K):
     from flexible_llm_sharding_amd.config import ModelConfig
     from flexible_llm_sharding_amd.models.llama import rope_tables
-    x, w = rnd(64, K, seed=165), rnd(N, K, scale=0.03, seed=166)
+    x, w, r = rnd(64, K, seed=165), rnd(N, K, scale=0.03, seed=166), rnd(64, N, seed=168)
     rs, b = (torch.rand(64, device=DEV) + 0.5).float(), rnd(N, scale=0.5, seed=167)
     pos = torch.randint(0, 4096, (64,), dtype=torch.int32, device=DEV)
     tables = {hd: [t.to(DEV) for t in rope_tables(ModelConfig(hidden_size=256, num_attention_heads=256 // hd, num_key_value_heads=1), 4096)]
               for hd in (64, 128)}
     for m in (1, 15, 16, 17, 32, 33, 64):
         def run():
-            out = [ops.gemm(x[:m], w, EPI_SWIGLU, rscale=rs[:m])]
+            out = [ops.gemm(x[:m], w, EPI_SWIGLU, rscale=rs[:m]), ops.gemm(x[:m], w, bias=b),
+                   ops.gemm(x[:m], w, EPI_RESID, out=r[:m].clone(), resid=r[:m].clone(), rscale=rs[:m])]
             for hd, (cos, sin) in tables.items():
                 out.append(ops.gemm(x[:m], w, EPI_ROPE, positions=pos[:m], cos=cos, sin=sin, rope_cols=N - hd, head_dim=hd, bias=b, rscale=rs[:m]))
             return out
@@ -585,7 +586,7 @@ def test_gemm_col16_pairs_bitwise(ops, N, K):
             finally:
                 ops.k.fls_gemm_set_mid_bn(old)
         with ops.row_exact():
-            for a, c, e in zip(forced(16), forced(64), run()):
+            for a, c, e in zip(forced(33), forced(64), run()):
                 assert torch.equal(a, c) and torch.equal(a, e), m
 
 
