@@ -169,7 +169,7 @@ constexpr int BMm = 64, BNm = 128, BKm = 64, NTm = 256, NSTAGE = 3;
 // BNT: output columns per block, 128 (4 waves in 2 x 2, each 32 x 64) or 64 (each 32 x 32: twice the
 // blocks for grids of less than one round of 128-column tiles); 32 with 8 waves (below)
 // A rows 0 .. bmt-1 then W rows; LDS-DMA in 8-row (1 KiB) groups
-constexpr int stage_bytes(int bnt, int bmt = BMm) { return (bmt + bnt) * BKm * 2; }
+constexpr int stage_bytes(int bnt, int bmt = BMm, int bk = BKm) { return (bmt + bnt) * bk * 2; }
 }  // namespace mid
 
 // NST: LDS stages, NST - 1 K-tiles in flight ahead of the one being multiplied (3: 72 KB, two blocks
@@ -192,7 +192,12 @@ constexpr int stage_bytes(int bnt, int bmt = BMm) { return (bmt + bnt) * BKm * 2
 //   BNT = 32 : waves in 4 x 2, each 16 x 16 (plain / residual epilogues): 70B down at M = 64
 //              155 -> 139 us (profiles/r6_decode/mid8/bn32_*).
 // Same fragments, MFMA and K order in every shape, so all are bitwise equal.
-template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm>
+//
+// BNT = 64, WV = 8: K-tiles of BK = 128 (64 where K is no multiple of it), one barrier a K-tile: after it tile kt - 1 has been read, so that its stage takes
+// the tile NST - 1 ahead.  What bounds these grids of one row tile is the chain of one K-tile in few blocks a CU: M = 24, 50 and 64 (us, with K-tiles of 64 and
+// two barriers, and so) 12,288 x 4,096 27.9, 29.2, 28.2 -> 24.3, 27.1, 26.0; 10,240 x 8,192 49.2, 51.1, 52.1 -> 42.8, 46.9, 49.4 with three stages (one
+// block a CU); 22,016 x 4,096 43.4, 47.5, 49.6 -> 43.2, 46.3, 48.2 with two stages (two blocks; 47.6, 49.5, 51.0 with three).
+template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm, int BK = 64>
 __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                      half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
                                                      int ldc, Epi ep) {
@@ -204,9 +209,12 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   constexpr bool L24 = WV == 8 && BMT == 64 && BNT == 128;   // 2 x 4 waves of 32 x 32
   constexpr bool L42 = WV == 8 && BNT <= 64;                 // 4 x 2 waves of 16 x 32 (x 16 at BNT 32)
   constexpr int RW = L42 ? 16 : 32, U = RW / 16;             // rows per wave, 16-row subtiles per wave
-  // 8-row LDS-DMA groups: waves 0 .. NG % WV - 1 take one more when they do not divide evenly
-  constexpr int NG = (BMT + BNT) / 8, PER_WAVE = (NG + WV - 1) / WV, NG_REM = NG % WV;
-  constexpr int STAGE = stage_bytes(BNT, BMT), NSUB = L24 ? 2 : BNT == 32 ? 1 : BNT / 32;
+  constexpr bool ONE = BNT == 64 && WV == 8;                 // one barrier a K-tile
+  constexpr int LPR = BK / 8, RPD = 64 / LPR, KM = LPR - 1;  // lanes (16-byte chunks) a row, rows a DMA group of 1 KB
+  // LDS-DMA groups: waves 0 .. NG % WV - 1 take one more when they do not divide evenly
+  constexpr int NG = (BMT + BNT) / RPD, PER_WAVE = (NG + WV - 1) / WV, NG_REM = NG % WV;
+  static_assert(!ONE || NG_REM == 0, "one count of DMAs");
+  constexpr int STAGE = stage_bytes(BNT, BMT, BK), NSUB = L24 ? 2 : BNT == 32 ? 1 : BNT / 32;
   extern __shared__ __attribute__((aligned(16))) char lds_mid[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
@@ -222,7 +230,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   const int bn = bid / mt;
   const int n0 = bn * BNT;
   const int wm = L24 ? wave >> 2 : wave >> 1, wn = L24 ? wave & 3 : wave & 1;
-  const int nk = K / BKm;
+  const int nk = K / BK;
   const bool rope128 = EPI == FLS_EPI_ROPE;
   // BNT = 64 with RoPE over 128-wide heads: local W row l -> column of head bn / 2, quarter bn % 2
   const bool split_head = BNT == 64 && rope128;
@@ -231,18 +239,18 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
     return n0 + l;
   };
 
-  // this lane's LDS-DMA sources: group g = wave + WV*i covers tile rows 8*g .. 8*g+7
+  // this lane's LDS-DMA sources: group g = wave + WV*i covers tile rows RPD*g .. RPD*g+RPD-1
   const half_t* src[PER_WAVE];
-  const int sub = lane >> 3;                       // row inside the 8-row group
-  const int kc = ((lane & 7) ^ sub) * 8;           // source chunk pre-swizzled (read XORs it back)
+  const int sub = lane / LPR;                      // row inside the group
 #pragma unroll
   for (int i = 0; i < PER_WAVE; ++i) {
     const int g = min(wave + WV * i, NG - 1);       // (a group past NG is never issued)
-    if (g < BMT / 8) {
-      const int m = min(m0 + g * 8 + sub, M - 1);
+    const int kc = ((lane ^ (g * RPD + sub)) & KM) * 8;           // source chunk pre-swizzled (read XORs it back)
+    if (g < BMT / RPD) {
+      const int m = min(m0 + g * RPD + sub, M - 1);
       src[i] = A + (size_t)m * lda + kc;
     } else {
-      const int n = gcol((g - BMT / 8) * 8 + sub);
+      const int n = gcol((g - BMT / RPD) * RPD + sub);
       const int nr = EPI == FLS_EPI_SWIGLU ? gu_phys_row(n, ep.gu_rows) : n;
       src[i] = W + (size_t)nr * ldw + kc;
     }
@@ -254,7 +262,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i)
       if (NG_REM == 0 || i < PER_WAVE - 1 || wave < NG_REM)   // wave-uniform
-        glds16(src[i] + (size_t)kt * BKm, base + (wave + WV * i) * 1024);
+        glds16(src[i] + (size_t)kt * BK, base + (wave + WV * i) * 1024);
   };
   // local W rows of this wave's subtiles (RoPE: subtile t + NSUB / 2 is subtile t's partner)
   int wrow[NSUB];
@@ -275,27 +283,34 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
 #pragma unroll
   for (int d = 0; d < NST - 1; ++d) stage(d, min(d, nk - 1));
   for (int kt = 0; kt < nk; ++kt) {
+    if constexpr (ONE) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 2) * PER_WAVE) : "memory");
+      __builtin_amdgcn_s_barrier();                        // every wave's part of tile kt landed; tile kt - 1 has been read
+      asm volatile("" ::: "memory");
+    }
     // into the stage tile kt - 1 used (every wave passed that tile's closing barrier)
     stage(kt + NST - 1, min(kt + NST - 1, nk - 1));
     // tile kt landed
-    if (NG_REM == 0 || wave < NG_REM) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * PER_WAVE) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * (PER_WAVE - 1)) : "memory");
-    __builtin_amdgcn_s_barrier();                          // every wave's part of tile kt landed
+    if constexpr (!ONE) {
+      if (NG_REM == 0 || wave < NG_REM) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * PER_WAVE) : "memory");
+      else asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NST - 1) * (PER_WAVE - 1)) : "memory");
+      __builtin_amdgcn_s_barrier();                        // every wave's part of tile kt landed
+    }
     const char* Xs = lds_mid + (kt % NST) * STAGE;
-    const char* Ws = Xs + BMT * BKm * 2;
+    const char* Ws = Xs + BMT * BK * 2;
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int ks = 0; ks < BK / 32; ++ks) {
       const int c = ks * 4 + grp;                          // logical 16-byte chunk of this lane
       half8 xf[U], wf[NSUB];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int r = wm * RW + u * 16 + fr;
-        xf[u] = *(const half8*)(Xs + r * 128 + ((c ^ (r & 7)) << 4));
+        xf[u] = *(const half8*)(Xs + r * (BK * 2) + ((c ^ (r & KM)) << 4));
       }
 #pragma unroll
       for (int t = 0; t < NSUB; ++t) {
         const int r = wrow[t];
-        wf[t] = *(const half8*)(Ws + r * 128 + ((c ^ (r & 7)) << 4));
+        wf[t] = *(const half8*)(Ws + r * (BK * 2) + ((c ^ (r & KM)) << 4));
       }
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -304,7 +319,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
     }
     // WAR: the next iteration's DMA overwrites this stage; all reads are done
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
+    if constexpr (!ONE) __builtin_amdgcn_s_barrier();
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the redundant tail DMA, before LDS is handed on
 #pragma unroll
@@ -432,18 +447,18 @@ int g_mid_bn = 0;            // mid-M block columns: 0 auto, 64 / 128 forced whe
 int g_mid_waves = 0;         // 128-column mid blocks: 0 auto, 4 / 8 waves forced (fls_gemm_set_mid_waves)
 int g_mid_rows = 0;          // 8-wave mid blocks' rows: 0 auto, 64 / 128 forced (fls_gemm_set_mid_rows)
 
-template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm>
+template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm, int BK = 64>
 void launch_mid(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
                 const Epi& ep, hipStream_t s) {
   static bool attr = false;
-  constexpr int lds = NST * mid::stage_bytes(BNT, BMT);
+  constexpr int lds = NST * mid::stage_bytes(BNT, BMT, BK);
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm_nt_mid<EPI, NST, BNT, WV, BMT>,
+    (void)hipFuncSetAttribute((const void*)gemm_nt_mid<EPI, NST, BNT, WV, BMT, BK>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
   const int blocks = ((M + BMT - 1) / BMT) * (N / BNT);
-  hipLaunchKernelGGL((gemm_nt_mid<EPI, NST, BNT, WV, BMT>), dim3(blocks), dim3(64 * WV), lds, s, A, W, C, M, N, K,
+  hipLaunchKernelGGL((gemm_nt_mid<EPI, NST, BNT, WV, BMT, BK>), dim3(blocks), dim3(64 * WV), lds, s, A, W, C, M, N, K,
                      lda, ldw, ldc, ep);
 }
 
@@ -686,6 +701,8 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
   return MID_128_W4;
 }
 
+// (The 64-column blocks take 0.92 of what is estimated for them since their K-tiles are of 128 terms.  Fitted anew they took products of 65 to 128 rows from
+// K-split blocks, whose estimates are further off: 1.002 of the time of 180 random ones, up to 1.2, and 0.995, up to 1.04, with these.)
 // The estimates (us).  Fitted to 15,400 random products of 1 .. 3,000 rows, 512 .. 29,440 columns (and a gate / up of 57,344) and 256 .. 28,928 terms,
 // each timed on every path that it can take, with weights that no cache holds; profiles/cases/gemm_routes.txt has the errors of the fits, 5 to 9%
 // each, and what the choice makes of them.  The shortest form that tells the paths apart: a start, and the larger of the weight's stream
@@ -867,7 +884,11 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
       case MID_32:
         if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         break;
-      case MID_64: launch_mid<EPI, mid::NSTAGE, 64, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_64:
+        if (K % 128) launch_mid<EPI, 4, 64, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else if ((M + 63) / 64 * (N / 64) <= 256) launch_mid<EPI, 3, 64, 8, 64, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else launch_mid<EPI, 2, 64, 8, 64, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        break;
       case MID_64_W4: launch_mid<EPI, mid::NSTAGE, 64>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
       case MID_128R: launch_mid<EPI, mid::NSTAGE, 128, 8, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
       case MID_128: launch_mid<EPI, mid::NSTAGE, 128, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
