@@ -252,6 +252,147 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
   }
 }
 
+// Few rows (decoding, some requests): what bounds a (row, head) is the chain of one tile -- its keys' page entries, the keys, the weights, the values,
+// each a trip to memory -- and 64 keys a tile gave that chain 200 to 400 keys' work on four waves.  Here sixteen waves take tiles of 16 keys in turn: four
+// lanes share a key, each every fourth 16-byte piece of it, all of a head of 128 in flight at once, and the tile's values are one or two
+// batches of loads.  A row of fewer than 256 keys is one tile a wave.  (aligned rows, FOUR's head sizes, no blocks.)  us in turn, the other kernel with its
+// ranges over twice the blocks, bf16 heads of 128: 128 rows x heads of 220 keys 9.9 -> 8.0, 400 15.5 -> 10.8, 1,000 21.0 -> 17.3; 48 x 400 15.3 -> 10.2, 1,000 18.2
+// -> 11.8; fp32 48 x 400 18.0 -> 11.7; of 210 combinations of 8 to 256 rows x heads, 20 to 4,000 keys, heads of 64 to 256 0.77 of the time.
+template <typename TQ, typename T, typename TO>
+__global__ __launch_bounds__(1024) void attn_few_kernel(const TQ* __restrict__ q, int ldq, const T* __restrict__ kc, int ldk,
+                                                        const T* __restrict__ vc, int ldv, TO* __restrict__ out, int ldo,
+                                                        const int* __restrict__ tok_seq, const int* __restrict__ tok_pos,
+                                                        const int* __restrict__ page_table, int pt_stride, int H, int G,
+                                                        int d, int dv, float scale, float softcap,
+                                                        const float* __restrict__ r1, const float* __restrict__ r2,
+                                                        int chunk, int window, int keep_first,
+                                                        const float* __restrict__ gate_bias, float out_scale,
+                                                        int page_size, int vsh, float* __restrict__ part, int has_sink,
+                                                        float sink, const float* __restrict__ sink_h,
+                                                        const float* __restrict__ head_gate, int ldhg, int Gv) {
+  constexpr int WV = 16, KEYS = 16, PE = 16 / sizeof(T), KU = 4;      // elements of a piece, pieces in flight a lane
+  __shared__ __attribute__((aligned(16))) float qs[MAX_D];
+  __shared__ float pw[WV][KEYS];
+  __shared__ int prow[WV][KEYS];
+  __shared__ float mm[WV], ll[WV];
+  __shared__ __attribute__((aligned(16))) float accs[WV][256];
+  const int t = blockIdx.y, h = blockIdx.x;
+  const int g = h / (H / G), gv = g % Gv;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = tok_pos[t];
+  const int* table = page_table + (size_t)tok_seq[t] * pt_stride;
+  for (int c = threadIdx.x; c < d; c += 64 * WV) qs[c] = ldf(q + (size_t)t * ldq + (size_t)h * d, c);
+  __syncthreads();
+  int lo = chunk > 0 ? (i / chunk) * chunk : 0;
+  if (window > 0 && i - window + 1 > lo) lo = i - window + 1;
+  const int nkeep = min(keep_first, lo), nkeys = nkeep + i - lo + 1, ntiles = (nkeys + KEYS - 1) / KEYS;
+  const float a1 = r1 != nullptr ? r1[h] : 0.f, a2 = r2 != nullptr ? r2[h] : 0.f;
+  const bool gated = gate_bias != nullptr;
+  const float gb = gated ? gate_bias[h] : 0.f;
+  const float snk = has_sink && sink_h != nullptr ? sink_h[h] : sink;
+  const int key = lane >> 2, sub4 = lane & 3, pieces = d / PE;
+  const int at = 64 >> vsh, sub = lane >> vsh, col = 4 * (lane & ((1 << vsh) - 1));
+  float m = -1e30f, l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+  const int nsplit = gridDim.z, tps = (ntiles + nsplit - 1) / nsplit, tile_hi = min(ntiles, ((int)blockIdx.z + 1) * tps);
+  for (int tile = blockIdx.z * tps + wave; tile < tile_hi; tile += WV) {
+    const int n = tile * KEYS + key;
+    const bool valid = n < nkeys;
+    const int j = n < nkeep ? n : lo + (n - nkeep);
+    float sc = 0.f;
+    int row = 0;
+    if (valid) {
+      row = table[j / page_size] * page_size + j % page_size;
+      const T* k = kc + (size_t)row * ldk + (size_t)g * d;
+      for (int p0 = sub4; p0 < pieces; p0 += 4 * KU) {
+        uint4 v[KU];
+#pragma unroll
+        for (int x = 0; x < KU; ++x) v[x] = *reinterpret_cast<const uint4*>(k + min(p0 + 4 * x, pieces - 1) * PE);
+#pragma unroll
+        for (int x = 0; x < KU; ++x)
+          if (p0 + 4 * x < pieces) {
+            const T* e = reinterpret_cast<const T*>(&v[x]);
+            const float* qp = qs + (p0 + 4 * x) * PE;
+#pragma unroll
+            for (int y = 0; y < PE; ++y) sc += ldf(e, y) * qp[y];
+          }
+      }
+    }
+    sc += __shfl_xor(sc, 1, 64);
+    sc += __shfl_xor(sc, 2, 64);
+    sc *= scale;
+    if (softcap > 0.f) sc = softcap * tanhf(sc / softcap);
+    if (a1 != 0.f) sc -= a1 * log1pf(a2 * (float)max(i - j, 0));
+    if (!valid) sc = -1e30f;
+    float p, corr = 1.f;
+    if (gated) {
+      p = valid ? sigmoid_f(sc + gb) : 0.f;
+    } else {
+      const float mt = fmaxf(m, wave_max(sc));
+      p = valid ? expf(sc - mt) : 0.f;
+      corr = expf(m - mt);
+      l = l * corr + wave_sum(sub4 == 0 ? p : 0.f);
+      m = mt;
+    }
+    if (sub4 == 0) {
+      pw[wave][key] = p;
+      prow[wave][key] = row;
+    }
+    // (a wave reads back only what its own lanes wrote: no barrier, but the compiler must not move the loads above the stores)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const int nk = min(KEYS, nkeys - tile * KEYS);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] *= corr;
+    for (int j0 = sub; j0 - sub < nk; j0 += 8 * at) {
+      RowVec<4> v[8];
+      float pj[8];
+#pragma unroll
+      for (int x = 0; x < 8; ++x) {
+        const int jj = min(j0 + x * at, nk - 1);
+        pj[x] = pw[wave][jj];
+        v[x] = row_load<4>(vc + (size_t)gv * dv + (size_t)prow[wave][jj] * ldv + col);
+      }
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        if (j0 + x * at < nk) {
+#pragma unroll
+          for (int y = 0; y < 4; ++y) acc[y] += pj[x] * v[x].v[y];
+        }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (lane == 0) { mm[wave] = m; ll[wave] = l; }
+  for (int o = 1 << vsh; o < 64; o <<= 1)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) acc[x] += __shfl_xor(acc[x], o, 64);
+  if (lane >> vsh == 0) *reinterpret_cast<float4*>(&accs[wave][4 * lane]) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+  __syncthreads();
+  if (64 * wave >= dv) return;
+  // (lane w & 15: wave w's maximum and sum, in each wave that writes)
+  float f = 1.f, inv = out_scale, mx = 0.f, lt = 0.f;
+  if (!gated) {
+    const float mz = mm[lane & (WV - 1)];
+    mx = wave_max(mz);
+    if (has_sink && nsplit == 1) mx = fmaxf(mx, snk);
+    f = expf(mz - mx);
+    lt = wave_sum(lane < WV ? ll[lane & (WV - 1)] * f : 0.f);
+    if (has_sink && nsplit == 1) lt += expf(snk - mx);
+    inv = out_scale / lt;
+  }
+  if (head_gate != nullptr) inv *= sigmoid_f(head_gate[(size_t)t * ldhg + h]);
+  const int e = threadIdx.x;
+  float v = 0.f;
+#pragma unroll
+  for (int w = 0; w < WV; ++w) v += accs[w][e] * __shfl(f, w, 64);
+  if (nsplit > 1) {
+    float* pp = part + (((size_t)t * H + h) * nsplit + blockIdx.z) * (dv + 4);
+    if (e == 0) { pp[dv] = mx; pp[dv + 1] = lt; }
+    if (e < dv) pp[e] = v;
+  } else if (e < dv) {
+    stf(out + (size_t)t * ldo + (size_t)h * dv, e, v * inv);
+  }
+}
+
 // out[t, h] from the nsplit partial results of a (row, head): softmax parts are rescaled to the common
 // maximum and divided by the total sum, gated parts are added.  The nsplit weights are worked out once
 // per block (nsplit <= MERGE_MAX_SPLIT), then every thread sums its value columns over the parts.
@@ -321,6 +462,9 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   const int es = tc == 1 ? 2 : 4;
   const bool by4 = (uintptr_t)vc % (4 * es) == 0 && ldv % 4 == 0 && (pool_P == 0 || ((uintptr_t)vp % (4 * es) == 0 && ldvp % 4 == 0));
   const int vsh = !by4 ? -1 : dv == 32 ? 3 : dv == 64 ? 4 : dv == 128 ? 5 : dv == 256 ? 6 : -1;
+  // One block a CU (a second one waits: 384 and 512 blocks 1.0 to 1.4 of the other kernel's time) and keys of 256 bytes or more (128 bytes are two loads
+  // a lane here and eight there: 0.9 to 1.2)
+  const bool few_ok = vsh >= 0 && pool_P == 0 && (long long)T * H * nsplit <= 256 && d * es >= 256;
 #define ATTN_PAGED_ARGS ldq, (const TC*)kc, ldk, (const TC*)vc, ldv, (TOUT*)out, ldo, tok_seq, tok_pos, page_table, pt_stride, H, G, \
                         d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, vec, vsh, part, has_sink, sink, sink_h, \
                         nsplit > 1 ? nullptr : head_gate, ldhg, Gv, ab
@@ -328,7 +472,11 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   hipLaunchKernelGGL((attn_paged_kernel<TQ, TC, TOUT, POOL, FOUR, KU>), grid, dim3(256), 0, st, (const TQ*)q, ATTN_PAGED_ARGS)
 #define ATTN_PAGED_GO(TQ)                                         \
   do {                                                            \
-    if (pool_P > 0) {                                             \
+    if (few) {                                                    \
+      hipLaunchKernelGGL((attn_few_kernel<TQ, TC, TOUT>), grid, dim3(1024), 0, st, (const TQ*)q, ldq, (const TC*)kc, ldk, (const TC*)vc, ldv, (TOUT*)out, ldo, \
+                         tok_seq, tok_pos, page_table, pt_stride, H, G, d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, \
+                         vsh, part, has_sink, sink, sink_h, nsplit > 1 ? nullptr : head_gate, ldhg, Gv); \
+    } else if (pool_P > 0) {                                      \
       if (vsh < 0) ATTN_PAGED_FORM(TQ, true, false, 1);           \
       else if (dv == 256) ATTN_PAGED_FORM(TQ, true, true, 1);     \
       else ATTN_PAGED_FORM(TQ, true, true, 4);                    \
@@ -339,6 +487,7 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   if (tc == 1) {
     using TC = bf16_t;
     const int vec = d % 8 == 0 && (uintptr_t)kc % 16 == 0 && ldk % 8 == 0 && (pool_P == 0 || ((uintptr_t)kp % 16 == 0 && ldkp % 8 == 0));
+    const bool few = few_ok && vec;
     if (to == 0) {
       using TOUT = float;
       if (tq == 1) ATTN_PAGED_GO(bf16_t);
@@ -352,6 +501,7 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
     using TC = float;
     using TOUT = float;
     const int vec = d % 4 == 0 && (uintptr_t)kc % 16 == 0 && ldk % 4 == 0 && (pool_P == 0 || ((uintptr_t)kp % 16 == 0 && ldkp % 4 == 0));
+    const bool few = few_ok && vec;
     ATTN_PAGED_GO(float);
   }
 #undef ATTN_PAGED_GO

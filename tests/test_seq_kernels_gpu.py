@@ -446,6 +446,31 @@ def test_attention_values_by_columns(ops, dv, d, pad):
             assert float((got[t] - want).abs().max()) < 2e-5 * float(want.abs().max()), (i, window)
 
 
+# few rows on sixteen waves (256 rows x heads, ranges of keys among them) and the same rows too often for it on four: lengths about a tile of 16, a
+# wave's turn of 256 and ranges of their own, every option, shared values, heads whose pieces do not divide by four lanes.  fp32 throughout, sums
+# of up to 1,500 terms and weights of up to 20 in the exponent: 3e-5 of the largest
+@pytest.mark.parametrize("d,dv", [(64, 32), (96, 64), (72, 128), (128, 256), (200, 128)])
+@pytest.mark.parametrize("kind", ["plain", "penalty", "sigmoid", "sink"])
+def test_attention_few_rows(ops, d, dv, kind):
+    H, R = ops
+    Hh, G = 4, 2
+    torch.manual_seed(d + dv)
+    r1, r2 = (torch.rand(Hh, device=DEV), torch.rand(Hh, device=DEV)) if kind == "penalty" else (None, None)
+    kw = dict(gate_bias=torch.randn(Hh, device=DEV) - 2) if kind == "sigmoid" else \
+        dict(sink=torch.randn(Hh, device=DEV), head_gate=torch.randn(100, Hh, device=DEV)) if kind == "sink" else {}
+    for pos0, ps in (([0, 1, 14, 15, 16, 17, 63, 64, 240, 254, 255, 256, 257], 24), ([511, 512, 1500], 16)):
+        md, npages, _ = meta_of([1] * len(pos0), pos0, DEV, ps)
+        kc, vc = torch.randn(npages, ps, G * d, device=DEV), torch.randn(npages, ps, G * dv, device=DEV)
+        q = torch.randn(len(pos0), Hh * d, device=DEV)
+        for chunk, window, keep in ((0, 0, 0), (200, 0, 0), (0, 40, 0), (0, 40, 30)):
+            for rep in (1, 100 // len(pos0)):
+                m2 = dict(md, tok_seq=md["tok_seq"].repeat(rep), tok_pos=md["tok_pos"].repeat(rep))
+                k2 = dict(kw, head_gate=kw["head_gate"][:rep * len(pos0)]) if "head_gate" in kw else kw
+                args = (q.repeat(rep, 1), kc, vc, m2, Hh, G, d, dv, d ** -0.5, 20.0 if kind == "penalty" else 0.0, r1, r2, chunk, ps, torch.float32)
+                o1, o2 = (o.attn_paged(*args, window=window, keep_first=keep, v_heads=1 if kind == "sigmoid" and dv < 256 else None, **k2) for o in (H, R))
+                close(o1, o2, 3e-5)
+
+
 # prompt attention over 64-key tiles in two halves: lengths about a half, a tile and a 128-row block, windows and chunks that end inside
 # a half, kept first keys, pages of 24 (no power of two); `grow`: scores that rise along the keys in small steps or in large ones
 # (the running maximum grows key by key, or in jumps), with a sink far below, near and far above them.  bf16 tolerance as above
