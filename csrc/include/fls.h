@@ -68,7 +68,8 @@ enum { FLS_EPI_NONE = 0, FLS_EPI_RESID = 1, FLS_EPI_SWIGLU = 2, FLS_EPI_ROPE = 3
 // generation tie guard re-runs a subset of prompts bit-identically to the whole batch
 #define FLS_GEMM_ROW_EXACT 0x100
 // C[M, N'] = epi(acc), acc[m] = rscale[m] * (A[M,K] . W[N,K]^T)[m] (+ bias)  (rscale may be null:
-// 1; the RMSNorm statistic of a fused norm + projection).  fp16 in / fp32 accumulate / fp16 out.
+// 1; the RMSNorm statistic of a fused norm + projection; rs_eps > 0: fls_row_stat's of the rows of A with
+// that eps, made by this call, rscale its fp32 [M] scratch).  fp16 in / fp32 accumulate / fp16 out.
 //   RESID : C = alpha * acc + R (R may alias C; alpha: Granite's residual_multiplier, else 1)
 //   SWIGLU: W = [gate (N/2 rows); up (N/2 rows)]; C has N/2 columns = silu(g)*u
 //   ROPE  : columns < rope_cols are rotated (HF rotate-half, natural head-dim
@@ -77,7 +78,7 @@ enum { FLS_EPI_NONE = 0, FLS_EPI_RESID = 1, FLS_EPI_SWIGLU = 2, FLS_EPI_ROPE = 3
 int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K,
              int lda, int ldw, int ldc, int ldr, int epi, const int* pos, const float* cos_t,
              const float* sin_t, int rope_cols, int head_dim, const void* bias, const float* rscale,
-             float alpha, float* ss, int ss_ld, void* ws, uint64_t ws_bytes,
+             float rs_eps, float alpha, float* ss, int ss_ld, void* ws, uint64_t ws_bytes,
              fls_stream_t s);   // ws: device scratch for the small-M split-K path (may be null)
 // ss (RESID only, may be null): ss[m * ss_ld + j] = sum of the squares of the fp16 outputs of row m in
 // columns [128 j, 128 j + 128) -- the row statistic of the next norm-folded projection without a

@@ -364,7 +364,13 @@ constexpr int stage_bytes(int rt, int np) { return 16 * (np + rt) * kt(rt, np) *
 constexpr int stages(int rt, int np) { return np == 2 ? (rt == 2 ? 5 : 3) : rt == 1 ? 8 : rt == 2 ? 6 : 3; }       // 128 / 144 / 120 KB; pairs 72 / 80 / 72
 }  // namespace col16
 
-template <int EPI, int RT, int NP>
+//
+// STAT (up to 32 rows): the row statistic that the epilogue applies is made here, from the rows of A that pass through LDS anyway, by the waves that only move
+// data, in row_stat_kernel's order (same bits): a lane has one row's column group, its parts of 128 columns stay in registers, four to a lane
+// group, and are added as warp_sum adds them.  A launch less for every norm + projection of a generation step.  us with that launch in front and so:
+// 16 rows x 12,288 x 4,096 28.1, 26.3; x 22,016 x 4,096 37.3, 36.6 (one row 36.3, 37.6); x 10,240 x 8,192 45.1, 41.4; x 6,144 x 2,048 10.6, 9.3; 32 rows x 6,144 x
+// 2,048 11.5, 10.4.  Above 32 rows the multiplying waves would have to make it: 48 rows 12.8, 15.1.
+template <int EPI, int RT, int NP, bool STAT>
 __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
                                                    int ldc, Epi ep) {
@@ -395,6 +401,16 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   floatx4 acc[NP];
 #pragma unroll
   for (int h = 0; h < NP; ++h) acc[h] = floatx4{0.f, 0.f, 0.f, 0.f};
+  static_assert(!STAT || 2 * RT <= 4, "a wave beside each that multiplies");
+  const int srt = wave - RT;                             // row tile whose statistics the wave makes
+  const bool stat = STAT && srt >= 0 && srt < RT;
+  const int srow = ((NP + srt) * 16 + fr) * KT * 2;
+  unsigned so[8];                                        // a part's columns 32 p + 4 grp + 16 h of the row: 16-byte chunk 4 p + 2 h + grp / 2, half of it
+#pragma unroll
+  for (int x = 0; x < 8; ++x) so[x] = (((2 * x + (grp >> 1)) ^ fr) << 4) + (grp & 1) * 8;
+  float sp[STAT ? 16 : 1];
+#pragma unroll
+  for (int r = 0; r < (STAT ? 16 : 1); ++r) sp[r] = 0.f;
 #pragma unroll
   for (int d = 0; d < NST - 1; ++d) stage(d, min(d, nk - 1));
   for (int kt = 0; kt < nk; ++kt) {
@@ -419,26 +435,64 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
         for (int h = 0; h < NP; ++h) acc[h] = mfma16x16x32(wf[h][ks], xf[ks], acc[h]);
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
+    if (stat) {
+      const unsigned xs = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_c16 + (kt % NST) * STAGE + srow;
+      half4 q[KT / 128][8];
+#pragma unroll
+      for (int i = 0; i < KT / 128; ++i)                 // (in asm: of loads of its own the compiler believes that they want every DMA landed)
+        asm volatile("ds_read_b64 %0, %8 offset:%c16\n\tds_read_b64 %1, %9 offset:%c16\n\tds_read_b64 %2, %10 offset:%c16\n\tds_read_b64 %3, %11 offset:%c16\n\t"
+                     "ds_read_b64 %4, %12 offset:%c16\n\tds_read_b64 %5, %13 offset:%c16\n\tds_read_b64 %6, %14 offset:%c16\n\tds_read_b64 %7, %15 offset:%c16\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(q[i][0]), "=&v"(q[i][1]), "=&v"(q[i][2]), "=&v"(q[i][3]), "=&v"(q[i][4]), "=&v"(q[i][5]), "=&v"(q[i][6]), "=&v"(q[i][7])
+                     : "v"(xs + so[0]), "v"(xs + so[1]), "v"(xs + so[2]), "v"(xs + so[3]), "v"(xs + so[4]), "v"(xs + so[5]), "v"(xs + so[6]), "v"(xs + so[7]),
+                       "n"(i * 256) : "memory");
+#pragma unroll
+      for (int i = 0; i < KT / 128; ++i) {
+        float sq = 0.f;
+#pragma unroll
+        for (int p = 0; p < 4; ++p) sq = ss_accum_pair(sq, q[i][2 * p], q[i][2 * p + 1]);
+        sq = row_sum_4groups(sq);
+        const int j = kt * (KT / 128) + i;               // part j: lane group j % 4, register j / 4
+        if ((j & 3) == grp) {
+#pragma unroll
+          for (int r = 0; r < (STAT ? 16 : 1); ++r) sp[r] = (j >> 2) == r ? sq : sp[r];
+        }
+      }
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  Epi e2 = ep;
+  if constexpr (STAT) {
+    __syncthreads();                                     // (every wave's DMAs have landed and its reads are done)
+    if (stat) {
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+        for (int r = 0; r < o; ++r) sp[r] += sp[r + o];
+      const float v = row_sum_4groups(sp[0]);
+      if (grp == 0) reinterpret_cast<float*>(lds_c16)[srt * 16 + fr] = rsqrtf(v / (float)K + ep.rs_eps);
+    }
+    __syncthreads();
+    e2.rs = reinterpret_cast<const float*>(lds_c16);
+  }
   const int m = wave * 16 + fr;
   if (wave < RT && m < M) {
-    if constexpr (NP == 1) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc[0], ep);
-    else if constexpr (is_rope(EPI)) store_rope_pair(C, ldc, m, n0 + 4 * grp, acc[0], acc[1], ep);
-    else store_pair_off<EPI>(C, ldc, m, b * 32, 4 * grp, acc[0], acc[1], ep);
+    if constexpr (NP == 1) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc[0], e2);
+    else if constexpr (is_rope(EPI)) store_rope_pair(C, ldc, m, n0 + 4 * grp, acc[0], acc[1], e2);
+    else store_pair_off<EPI>(C, ldc, m, b * 32, 4 * grp, acc[0], acc[1], e2);
   }
 }
 
-template <int EPI, int RT, int NP>
+template <int EPI, int RT, int NP, bool STAT = false>
 void launch_col16(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
                   const Epi& ep, hipStream_t s) {
   constexpr int lds = col16::stages(RT, NP) * col16::stage_bytes(RT, NP);
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm_nt_col16<EPI, RT, NP>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    (void)hipFuncSetAttribute((const void*)gemm_nt_col16<EPI, RT, NP, STAT>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
-  hipLaunchKernelGGL((gemm_nt_col16<EPI, RT, NP>), dim3(N / (16 * NP)), dim3(256), lds, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
+  hipLaunchKernelGGL((gemm_nt_col16<EPI, RT, NP, STAT>), dim3(N / (16 * NP)), dim3(256), lds, s, A, W, C, M, N, K, lda, ldw, ldc, ep);
 }
 
 int g_order = 0;             // 0: by shape, else a fixed signed group size (fls_gemm_set_order)
@@ -626,6 +680,10 @@ __global__ __launch_bounds__(256) void row_stat_kernel(const half_t* __restrict_
   }
   v = warp_sum(v);
   if (lane == 0) rstd[m] = rsqrtf(v / (float)H + eps);
+}
+
+void row_stat(const half_t* x, int ldx, int rows, int H, float eps, float* rstd, hipStream_t s) {
+  hipLaunchKernelGGL(row_stat_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, ldx, rows, H / 128, H, eps, rstd);
 }
 
 void ss_partials_raw(const half_t* C, int ldc, int M, int N, float* ss, int ss_ld, hipStream_t s) {
@@ -831,6 +889,13 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
                         ((uintptr_t)C & 7) == 0 && ((uintptr_t)ws & 15) == 0 &&
                         (EPI != FLS_EPI_RESID || (ep.ldr % 4 == 0 && ((uintptr_t)ep.R & 7) == 0));
   if (!main_ok) route = ROUTE_NONE;
+  // The row statistic of A (rs_eps): made by the blocks of 16 pairs where they take the product, have waves for it and registers for its parts, else by a launch here.
+  constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
+  const bool to_mid = mid_ok && (ep.row_exact || route == ROUTE_MID) &&
+                      (!main_ok || route == ROUTE_MID || (route == ROUTE_NONE && g_mid && mid_rule(M, tiles256)));
+  const bool bn64_ok = N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0);
+  const bool stat = ep.rs_eps > 0.f && pairs && to_mid && M <= 32 && K <= 8192 && mid_form(M, N, K, pairs, bn64_ok) == MID_16X2;
+  if (ep.rs_eps > 0.f && !stat) row_stat(A, lda, M, K, ep.rs_eps, const_cast<float*>(ep.rs), s);
   if (!ep.row_exact && (route == ROUTE_NONE || route == ROUTE_SKINNY)) {
     const int rc = try_skinny<EPI>(A, W, C, M, N, K, lda, ldw, ldc, ep, s, ws, ws_bytes, route == ROUTE_SKINNY);
     if (rc > 0) ss_partials(C, ldc, M, N, ep, s);
@@ -867,8 +932,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   if (route == ROUTE_SPLIT) route = ROUTE_NONE;
   if (mid_ok && (!main_ok || route == ROUTE_MID ||
                  (route == ROUTE_NONE && g_mid && mid_rule(M, tiles256)))) {
-    constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
-    switch (mid_form(M, N, K, pairs, N % 64 == 0 && (EPI != FLS_EPI_ROPE || N % 128 == 0))) {
+    switch (mid_form(M, N, K, pairs, bn64_ok)) {
       case MID_16:
         if constexpr (!pairs) {
           if (M <= 16) launch_col16<EPI, 1, 1>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
@@ -877,6 +941,13 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
         }
         break;
       case MID_16X2:
+        if constexpr (pairs) {
+          if (stat) {
+            if (M <= 16) launch_col16<EPI, 1, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+            else launch_col16<EPI, 2, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+            break;
+          }
+        }
         if (M <= 16) launch_col16<EPI, 1, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else if (M <= 32) launch_col16<EPI, 2, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else launch_col16<EPI, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
@@ -937,7 +1008,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
 
 }  // namespace
 
-extern "C" int fls_kernels_version(void) { return 37; }
+extern "C" int fls_kernels_version(void) { return 38; }
 
 // tile order: 0 = by shape (default); g > 0: groups of g M tiles; g < 0: groups of -g N tiles (A/B, tests)
 extern "C" int fls_gemm_set_order(int order) {
@@ -998,8 +1069,7 @@ extern "C" int fls_row_ss(const void* x, int ldx, int rows, int H, float* ss, in
 extern "C" int fls_row_stat(const void* x, int ldx, int rows, int H, float eps, float* rstd, fls_stream_t s) {
   if (rows <= 0) return 0;
   if (H % 128 || H / 128 > ROW_STAT_MAX_PARTS || ldx % 8 || ((uintptr_t)x & 15)) return -2;
-  hipLaunchKernelGGL(row_stat_kernel, dim3((rows + 3) / 4), dim3(256), 0, (hipStream_t)s, (const half_t*)x, ldx, rows,
-                     H / 128, H, eps, rstd);
+  row_stat((const half_t*)x, ldx, rows, H, eps, rstd, (hipStream_t)s);
   FLS_CHECK_LAUNCH();
   return 0;
 }
@@ -1052,7 +1122,7 @@ extern "C" int fls_gemm_leaves_ss(int M, int N, int K, uint64_t ws_bytes) {
 
 extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
                         int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
-                        int rope_cols, int head_dim, const void* bias, const float* rscale, float alpha, float* ss,
+                        int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, float alpha, float* ss,
                         int ss_ld, void* ws, uint64_t ws_bytes, fls_stream_t s) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int row_exact = (epi & FLS_GEMM_ROW_EXACT) ? 1 : 0;
@@ -1063,8 +1133,16 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
   if ((epi == FLS_EPI_SWIGLU || epi == FLS_EPI_ROPE) && (N % 32)) return -2;
   if (epi == FLS_EPI_ROPE && ((head_dim != 64 && head_dim != 128) || rope_cols % head_dim || N % head_dim))
     return -3;
+  // rscale made here: by the path itself or by fls_row_stat's kernel in front of it
+  if (rs_eps > 0.f) {
+    if (!rscale || K % 128 || K / 128 > ROW_STAT_MAX_PARTS || lda % 8 || ((uintptr_t)A & 15)) return -2;
+    if (M > 64) {
+      row_stat((const half_t*)A, lda, M, K, rs_eps, const_cast<float*>(rscale), (hipStream_t)s);
+      rs_eps = 0.f;
+    }
+  }
   Route route = N % BN == 0 && K % (2 * BK) == 0 ? route_of(M, N, K, epi, row_exact != 0, ws ? ws_bytes : 0) : ROUTE_NONE;
-  {
+  if (M > 64) {
     const int rc = fls_gemm_v11_try(A, W, C, R, M, N, K, lda, ldw, ldc, ldr, epi, pos, cos_t, sin_t, rope_cols,
                                     head_dim, bias, rscale, alpha, ss, ss_ld,
                                     route == ROUTE_NONE ? 0 : route == ROUTE_V11 ? 1 : -1, s);
@@ -1074,6 +1152,7 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
   Epi ep{(const half_t*)R, ldr, pos, cos_t, sin_t, rope_cols, head_dim, (const half_t*)bias, N / 2, 0,
          nullptr, nullptr, 0, 0};
   ep.rs = rscale;
+  ep.rs_eps = rs_eps;
   ep.alpha = alpha;
   ep.ss = ss;
   ep.ss_ld = ss_ld;

@@ -48,6 +48,8 @@ struct Epi {
   // rsqrt(mean(x^2) + eps) of a GEMM that reads the un-normalised hidden state x with the norm
   // weight folded into W (fused RMSNorm + projection); applied before the bias
   const float* rs = nullptr;
+  // > 0: the 16-pair blocks make that statistic themselves, of the rows of A (and rs is not read)
+  float rs_eps = 0.f;
   // scale of (product + bias) before the residual add (Granite's residual_multiplier)
   float alpha = 1.f;
   // optional (RESID): per-row partial sums of squares of the fp16 output, one fp32 per 128 output

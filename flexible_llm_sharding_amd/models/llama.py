@@ -254,14 +254,14 @@ class ExecContext:
         return self.row_stat(x, out=out)
 
     def row_stat(self, x: torch.Tensor, out=None) -> torch.Tensor:
-        """The statistic from a pass over x.  With 128-column partials it is computed exactly as the
+        """The statistic from a pass over x, for the one product of x that it scales (which makes it, or has it made).  With 128-column partials it is computed exactly as the
         residual GEMM epilogue's partials + rstd_from_ss would give it, so a row's statistic (and the
         scores) do not depend on whether its partials survived: a state received from another
         pipeline rank, parked in host memory, after grouped attention or in the pruned last layer
         gets the same bits as one straight from the residual GEMM."""
         H, eps = self.cfg.hidden_size, self.cfg.rms_norm_eps
-        if H % 128 == 0 and H <= 16384 and hasattr(self.ops, "row_stat"):
-            return self.ops.row_stat(x, eps, out=out)
+        if H % 128 == 0 and H <= 16384 and hasattr(self.ops, "pending_stat"):
+            return self.ops.pending_stat(x, eps, out=out)
         return self.ops.row_rstd(x, eps, out=out)
 
 

@@ -15,7 +15,7 @@ from __future__ import annotations
 import os
 import threading
 from dataclasses import dataclass
-from typing import Optional
+from typing import NamedTuple, Optional
 
 import torch
 
@@ -60,6 +60,12 @@ class MoeRoute:
     k: int
 
 
+class RowStat(NamedTuple):
+    """A row statistic (:meth:`HipOps.row_stat`) that the one product it scales makes: fp32 scratch of a value a row, epsilon."""
+    buf: torch.Tensor
+    eps: float
+
+
 class HipOps:
     name = "hip"
     uses_work_items = True
@@ -81,11 +87,14 @@ class HipOps:
              resid: torch.Tensor = None, positions=None, cos=None, sin=None, rope_cols: int = 0,
              head_dim: int = 0, bias: torch.Tensor = None, rscale: torch.Tensor = None,
              alpha: float = 1.0, ss: torch.Tensor = None) -> torch.Tensor:
-        """rscale ([M] fp32): per-row scale of the raw product (before bias / epilogue); alpha:
+        """rscale ([M] fp32, or the :class:`RowStat` of x): per-row scale of the raw product (before bias / epilogue); alpha:
         RESID's C = alpha * (product + bias) + R; ss ([>= M, N / 128] fp32, RESID): each output
         row's partial sums of squares per 128 columns (:meth:`rstd_from_ss`)."""
         _f16(x, "x")
         _f16(w, "w")
+        rs_eps = 0.0
+        if isinstance(rscale, RowStat):
+            rscale, rs_eps = rscale
         if rscale is not None and (rscale.dtype != torch.float32 or not rscale.is_cuda
                                    or rscale.numel() < x.shape[0] or not rscale.is_contiguous()):
             raise TypeError("rscale must be a contiguous fp32 CUDA vector with one entry per row")
@@ -112,7 +121,7 @@ class HipOps:
                              cos.data_ptr() if cos is not None else None,
                              sin.data_ptr() if sin is not None else None,
                              rope_cols, head_dim, bias.data_ptr() if bias is not None else None,
-                             rscale.data_ptr() if rscale is not None else None, float(alpha),
+                             rscale.data_ptr() if rscale is not None else None, rs_eps, float(alpha),
                              ss.data_ptr() if ss is not None else None, ss.stride(0) if ss is not None else 0,
                              ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream())
         _chk(rc, "fls_gemm")
@@ -236,6 +245,13 @@ class HipOps:
         _chk(self.k.fls_row_stat(x.data_ptr(), x.stride(0), rows, H, float(eps), r.data_ptr(), _stream()),
              "fls_row_stat")
         return r
+
+    def pending_stat(self, x, eps, out=None):
+        """:meth:`row_stat` of x for the one product of x that it scales (``rscale``): made there, within the product's own
+        launch where its path can."""
+        if x.stride(0) % 8 or x.data_ptr() % 16 or eps <= 0:
+            return self.row_stat(x, eps, out=out)
+        return RowStat(out if out is not None else torch.empty(x.shape[0], dtype=torch.float32, device=x.device), float(eps))
 
     def row_rstd(self, x, eps, row_idx=None, out=None):
         """[rows] fp32 rsqrt(mean(x[row]^2) + eps) (rows = row_idx or every row of x)."""

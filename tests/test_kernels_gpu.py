@@ -590,6 +590,34 @@ def test_gemm_col16_two_panels_bitwise(ops, N, K):
                 assert torch.equal(a, c) and torch.equal(a, e), m
 
 
+# a norm's statistic made by its product: the bits of row_stat's launch before it, where the blocks of 16 pairs make it (both tile depths, an odd count of parts of 128
+# columns to a lane group, all of its registers) and on every other path (K above them, more rows, plain products)
+@pytest.mark.parametrize("N,K", [(256, 256), (512, 768), (1280, 4096), (8192, 512), (1024, 8192), (512, 8448)])
+def test_gemm_makes_row_stat(ops, N, K):
+    from flexible_llm_sharding_amd.config import ModelConfig
+    from flexible_llm_sharding_amd.models.llama import rope_tables
+    from flexible_llm_sharding_amd.ops.hip_backend import RowStat
+    x, w, b = rnd(200, K, seed=171) * 3, rnd(N, K, scale=0.03, seed=172), rnd(N, scale=0.5, seed=173)
+    x[5] = 0
+    pos = torch.randint(0, 4096, (200,), dtype=torch.int32, device=DEV)
+    tables = {hd: [t.to(DEV) for t in rope_tables(ModelConfig(hidden_size=256, num_attention_heads=256 // hd, num_key_value_heads=1), 4096)]
+              for hd in (64, 128)}
+    for m in (1, 15, 16, 17, 32, 33, 64, 65, 200):
+        xm = x[:m]
+
+        def run(make):
+            out = [ops.gemm(xm, w, EPI_SWIGLU, rscale=make()), ops.gemm(xm, w, bias=b, rscale=make())]
+            for hd, (cos, sin) in tables.items():
+                out.append(ops.gemm(xm, w, EPI_ROPE, positions=pos[:m], cos=cos, sin=sin, rope_cols=N - hd, head_dim=hd, bias=b, rscale=make()))
+            return out
+        for exact in (True, False):
+            with ops.row_exact(exact):
+                for a, c in zip(run(lambda: RowStat(torch.full((m,), float("nan"), device=DEV), 1e-5)), run(lambda: ops.row_stat(xm, 1e-5))):
+                    assert torch.equal(a, c), (m, exact)
+    wide = rnd(4, K + 4, seed=174)[:, :K]                       # rows that vectors do not fit: the statistic first
+    assert torch.is_tensor(ops.pending_stat(wide, 1e-5)) and isinstance(ops.pending_stat(x, 1e-5), RowStat)
+
+
 def test_row_ss_matches_residual_epilogue(ops):
     """fls_row_ss on a hidden state == the partial sums of squares the residual GEMM epilogue wrote
     for the same rows (v10 / v11 tiles and the mid-M kernel + ss_partials), bit for bit, and the
