@@ -321,7 +321,10 @@ __global__ __launch_bounds__(256, 2) void delta_walk_kernel(Delta a) {
   int buf = 0;
   for (int r0 = first; r0 < stop; r0 += CH, buf ^= 1) {
     const floatx4 v = vn, zero = {0.f, 0.f, 0.f, 0.f};
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");        // this wave's part of the chunk's factors is here ...
+    // (a builtin, which the compiler counts: behind the same wait in asm it believed the state's registers, loaded in front of the loop, still on their
+    // way and had each chunk wait for half of the next one's factors before its first product)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x70);                                  // vmcnt(0) lgkmcnt(0): this wave's part of the chunk's factors is here ...
     __builtin_amdgcn_s_barrier();                                      // ... and everybody's; the other buffer has been read
     asm volatile("" ::: "memory");
     if (r0 > first) store_o(r0 - CH);
