@@ -150,7 +150,8 @@ int fls_rmsnorm(const void* x, const void* w, void* y, const int* row_idx, int r
                 int ldx, int ldy, float eps, fls_stream_t s);
 int fls_embed(const int* ids, const void* table, void* out, int T, int H, int V, float scale, fls_stream_t s);
 // greedy (nullable): the rows' argmax too, as fls_argmax_rows gives it
-int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, int* greedy, fls_stream_t s);
+int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, int* greedy, float* part,
+                     fls_stream_t s);     // part: 128 floats of scratch a row for rows of more than 32,768 values (null: one block a row)
 // dst = fp16(src): src_dtype 1 = bf16 (in place allowed), 2 = fp32 (no overlap)
 int fls_cast_f16(void* dst, const void* src, int src_dtype, uint64_t n, fls_stream_t s);
 // C[M,N] = X[M,K] W[N,K]^T for M <= 16 (skinny LM head); K % 32 == 0

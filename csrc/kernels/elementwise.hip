@@ -3,6 +3,8 @@
 // skinny-M GEMV.
 // All loads/stores are 16-byte vectors (guide G13: scalar fp16 loads cost
 // ~2x); one 256-thread block per row; fp32 statistics.
+#include <algorithm>
+
 #include "common.h"
 #include "fls.h"
 
@@ -202,7 +204,7 @@ __device__ __forceinline__ void argmax_block(unsigned& best, int& bi, unsigned* 
 // online max/sum in one pass, normalisation in a second (row stays in L2).
 // inv_scale != 1: the logits are first fp16(l * inv_scale) (Granite's logits / logits_scaling).
 // One block a row and few rows a call: latency bound, so a wide vocabulary takes 1,024 threads (16 rows of 32,000:
-// 14.4 -> 8.7 us against 256 threads; of 151,936: 71 -> 35 us).
+// 14.4 -> 8.7 us against 256 threads; of 151,936: 71 -> 35 us).  Rows in eights of 4,096 and more take softmax_regs_kernel.
 // GREEDY: the first index of each row's largest probability too (argmax_rows_kernel's answer), found while they are written:
 // a launch and a pass over the rows less (16 rows of 32,000: 8.7 + 7.9 us).
 template <int NT, bool GREEDY>
@@ -267,6 +269,88 @@ __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ 
   }
 }
 
+// The same with the row in registers, NC times eight values a thread (rows of up to 32,768 in eights): all of its loads in flight at once and none a second time,
+// one exponential a value for the sum instead of the running maximum's rescaling too, and the greedy token as the first value with the largest one's
+// bits.  16 rows of 32,000 with greedy tokens 12.3 -> 7.3 us, one of 8,192 6.3 -> 4.6.
+// PASS 1 and 2: wider rows, bound by what one CU computes, cut over gridDim.x blocks of slices: each slice's maximum and sum to `part`, then the
+// probabilities: one row of 65,544 19.8 -> 6.7 us, of 151,936 39.2 -> 6.9; 48 43.6 -> 14.2, 120 47.0 -> 24.2.
+template <int NT, int NC, bool GREEDY, int PASS>
+__global__ __launch_bounds__(NT) void softmax_regs_kernel(const half_t* __restrict__ logits, half_t* __restrict__ probs,
+                                                        int V, float inv_scale, int* __restrict__ greedy, float2* __restrict__ part) {
+  __shared__ float red[NT / 64];
+  const int row = PASS == 0 ? blockIdx.x : blockIdx.y, z = PASS == 0 ? 0 : blockIdx.x, nz = PASS == 0 ? 1 : gridDim.x;
+  const half8* lr = (const half8*)(logits + (size_t)row * V);
+  half8* pr = (half8*)(probs + (size_t)row * V);
+  const int per = (V / 8 + nz - 1) / nz, c0 = z * per, n = min(V / 8, c0 + per);       // the slice's chunks of eight (per <= NC NT)
+  half8 v[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) v[i] = lr[min(c0 + (int)threadIdx.x + i * NT, V / 8 - 1)];
+  if (inv_scale != 1.f) {
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[i][j] = (half_t)((float)v[i][j] * inv_scale);
+  }
+  float gm, gs;
+  if constexpr (PASS == 2) {
+    const float2 p = part[(size_t)row * nz + min((int)(threadIdx.x & 63), nz - 1)];      // (nz <= 64; every wave adds them up)
+    gm = warp_max(p.x);
+    gs = warp_sum((threadIdx.x & 63) < nz ? p.y * __expf(p.x - gm) : 0.f);
+  } else {
+    float m = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (c0 + (int)threadIdx.x + i * NT < n) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m = fmaxf(m, (float)v[i][j]);
+      }
+    gm = block_max(m, red);
+    float s = 0.f;
+    const float base = gm == -INFINITY ? 0.f : gm;       // (a slice of -inf: zeros)
+#pragma unroll
+    for (int i = 0; i < NC; ++i)
+      if (c0 + (int)threadIdx.x + i * NT < n) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s += __expf((float)v[i][j] - base);
+      }
+    gs = block_sum(s, red);
+    if constexpr (PASS == 1) {
+      if (threadIdx.x == 0) part[(size_t)row * nz + z] = make_float2(gm, gs);
+      if (GREEDY && z == 0 && threadIdx.x == 0) greedy[row] = 0x7fffffff;
+      return;
+    }
+  }
+  const float inv = 1.f / gs;
+  const unsigned short top = __builtin_bit_cast(unsigned short, (half_t)inv);        // the largest probability's bits
+  int bi = 0x7fffffff;
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = c0 + threadIdx.x + i * NT;
+    if (c < n) {
+      half8 o;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) o[j] = (half_t)(__expf((float)v[i][j] - gm) * inv);
+      pr[c] = o;
+      if constexpr (GREEDY) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bi = min(bi, __builtin_bit_cast(unsigned short, (half_t)o[j]) == top ? c * 8 + j : 0x7fffffff);
+      }
+    }
+  }
+  if constexpr (GREEDY) {
+    __shared__ int si[NT / 64];
+    for (int o = 32; o > 0; o >>= 1) bi = min(bi, __shfl_xor(bi, o, 64));
+    if ((threadIdx.x & 63) == 0) si[threadIdx.x >> 6] = bi;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < NT / 64; ++w) bi = min(bi, si[w]);
+      const bool none = !(gs >= 1.f) || gm == INFINITY;        // (no finite maximum: no largest value to find)
+      if (none) bi = 0;
+      if (PASS == 0) greedy[row] = bi;
+      else if (bi != 0x7fffffff) atomicMin(greedy + row, bi);
+    }
+  }
+}
 
 // greedy token of each row of fp16 probabilities: the FIRST index of the row's maximum (numpy
 // argmax on the scores the reference hands back, main.py:85-88).  Probabilities are >= 0, so
@@ -503,12 +587,33 @@ extern "C" int fls_embed(const int* ids, const void* table, void* out, int T, in
   return 0;
 }
 
-extern "C" int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, int* greedy, fls_stream_t s) {
+extern "C" int fls_softmax_rows(const void* logits, void* probs, int rows, int V, float inv_scale, int* greedy, float* part, fls_stream_t s) {
   if (rows <= 0) return 0;
-#define SOFTMAX(NT, GREEDY) hipLaunchKernelGGL((softmax_kernel<NT, GREEDY>), dim3(rows), dim3(NT), 0, (hipStream_t)s, (const half_t*)logits, (half_t*)probs, V, inv_scale, greedy)
-  if (V >= 4096) { if (greedy != nullptr) SOFTMAX(1024, true); else SOFTMAX(1024, false); }
-  else { if (greedy != nullptr) SOFTMAX(256, true); else SOFTMAX(256, false); }
+  const bool regs = V % 8 == 0 && V >= 4096 && (((uintptr_t)logits | (uintptr_t)probs) & 15) == 0;
+#define SOFTMAX_ARGS (hipStream_t)s, (const half_t*)logits, (half_t*)probs, V, inv_scale, greedy
+#define SOFTMAX(NT, GREEDY) hipLaunchKernelGGL((softmax_kernel<NT, GREEDY>), dim3(rows), dim3(NT), 0, SOFTMAX_ARGS)
+#define SOFTMAX_REGS(NT, NC, PASS, GRID)                                                                                     \
+  do {                                                                                                                       \
+    if (greedy != nullptr) hipLaunchKernelGGL((softmax_regs_kernel<NT, NC, true, PASS>), GRID, dim3(NT), 0, SOFTMAX_ARGS, (float2*)part); \
+    else hipLaunchKernelGGL((softmax_regs_kernel<NT, NC, false, PASS>), GRID, dim3(NT), 0, SOFTMAX_ARGS, (float2*)part);    \
+  } while (0)
+  if (regs && V <= 32768) {
+    SOFTMAX_REGS(1024, 4, 0, dim3(rows));
+  } else if (regs && part != nullptr && V <= 64 * 16384 && rows <= 65535) {
+    // slices of up to 16,384 values, or of fewer where the rows would leave CUs idle
+    const int nz = std::max((V + 16383) / 16384, std::min(std::min(256 / rows, V / 4096), 64));
+    SOFTMAX_REGS(256, 8, 1, dim3(nz, rows));
+    SOFTMAX_REGS(256, 8, 2, dim3(nz, rows));
+  } else if (V >= 4096) {
+    if (greedy != nullptr) SOFTMAX(1024, true);
+    else SOFTMAX(1024, false);
+  } else {
+    if (greedy != nullptr) SOFTMAX(256, true);
+    else SOFTMAX(256, false);
+  }
+#undef SOFTMAX_REGS
 #undef SOFTMAX
+#undef SOFTMAX_ARGS
   FLS_CHECK_LAUNCH();
   return 0;
 }

@@ -60,6 +60,12 @@ class MoeRoute:
     k: int
 
 
+def _softmax_part(logits):
+    # (stream-ordered scratch: the allocator hands it out again only behind the kernels that use it)
+    rows, V = logits.shape
+    return torch.empty(rows * 128, dtype=torch.float32, device=logits.device).data_ptr() if V > 32768 else None
+
+
 class RowStat(NamedTuple):
     """A row statistic (:meth:`HipOps.row_stat`) that the one product it scales makes: fp32 scratch of a value a row, epsilon."""
     buf: torch.Tensor
@@ -521,11 +527,11 @@ class HipOps:
         rows, V = logits.shape
         probs = torch.empty_like(logits)
         _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
-                                     None, _stream()), "fls_softmax")
+                                     None, _softmax_part(logits), _stream()), "fls_softmax")
         return probs
 
     def softmax_greedy(self, logits, logits_scaling: float = 1.0):
-        """-> (:meth:`softmax`, its :meth:`argmax_rows`, the bytes of both in a row), in one launch."""
+        """-> (:meth:`softmax`, its :meth:`argmax_rows`, the bytes of both in a row), in one launch (two for very wide rows)."""
         _f16(logits, "logits")
         rows, V = logits.shape
         n = 2 * rows * V
@@ -533,7 +539,7 @@ class HipOps:
         flat = torch.empty(at + 4 * rows, dtype=torch.uint8, device=logits.device)
         probs, greedy = flat[:n].view(torch.float16).view(rows, V), flat[at:].view(torch.int32)
         _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
-                                     greedy.data_ptr(), _stream()), "fls_softmax")
+                                     greedy.data_ptr(), _softmax_part(logits), _stream()), "fls_softmax")
         return probs, greedy, flat
 
     def argmax_rows(self, probs):

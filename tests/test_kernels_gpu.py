@@ -1320,6 +1320,30 @@ def test_softmax_greedy(ops, V, scaling):
     assert torch.equal(host[:10 * V].view(torch.int16), want.cpu().view(torch.int16).flatten()) and torch.equal(host[at:].view(torch.int32), greedy.cpu())
 
 
+# rows in registers, in one block and cut over several (their limits, few rows and many, the widest and one that is wider): probabilities
+# against fp64 (half a step of fp16, 2^-11, and 1e-5 for the hardware's exponential, or half the smallest step), the greedy token and the bits without it; ties across
+# slices, a slice of -inf, NaN
+@pytest.mark.parametrize("V", [4104, 32768, 32776, 65536, 65544, 131080, 151936, 1048576, 1048584])
+@pytest.mark.parametrize("rows", [4, 70])
+def test_softmax_wide_rows(ops, V, rows):
+    rows = min(rows, 4 + (1 << 23) // V)
+    x = (torch.randn(rows, V, generator=torch.Generator().manual_seed(V)) * 4).round().div(2).half()
+    x[1] = 0.25
+    x[1, V // 2] = x[1, V - 3] = 9.0
+    x[2, :V // 2] = float("-inf") if V <= 1 << 20 else -60000.0        # (one block of any width: NaN where a thread begins with eight of them)
+    x[3, V // 3] = float("nan")
+    x = x.to(DEV)
+    for scaling in (1.0, 8.0):
+        probs, greedy, _ = ops.softmax_greedy(x, scaling)
+        assert torch.equal(probs.view(torch.int16), ops.softmax(x, scaling).view(torch.int16)) and torch.equal(greedy, ops.argmax_rows(probs))
+        assert bool(torch.isnan(probs[3]).all()) and greedy[1].item() == V // 2
+        ok = [r for r in range(rows) if r != 3]
+        z = (x[ok].float() * (1.0 / scaling)).half().double()
+        want = torch.softmax(z, -1)
+        assert bool(((probs[ok].double() - want).abs() <= want * (2.0 ** -11 + 1e-5) + 2.0 ** -25).all())
+        assert np.array_equal(greedy[ok].cpu().numpy(), np.argmax(probs[ok].cpu().numpy(), axis=-1))
+
+
 # the statistic of a residual product's rows has the same bits from the partials it leaves and from its rows, on every path by rows (skinny,
 # blocks of 64 rows, split, tiles), and the product does not depend on which of the two is asked for
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 65, 79, 128, 129, 300, 1000, 4100])
