@@ -193,10 +193,12 @@ constexpr int stage_bytes(int bnt, int bmt = BMm, int bk = BKm) { return (bmt + 
 //              155 -> 139 us (profiles/r6_decode/mid8/bn32_*).
 // Same fragments, MFMA and K order in every shape, so all are bitwise equal.
 //
-// BNT = 64, WV = 8: K-tiles of BK = 128 (64 where K is no multiple of it), one barrier a K-tile: after it tile kt - 1 has been read, so that its stage takes
+// BNT = 64 and 128, WV = 8: K-tiles of BK = 128 (64 where K is no multiple of it), one barrier a K-tile: after it tile kt - 1 has been read, so that its stage takes
 // the tile NST - 1 ahead.  What bounds these grids of one row tile is the chain of one K-tile in few blocks a CU: M = 24, 50 and 64 (us, with K-tiles of 64 and
 // two barriers, and so) 12,288 x 4,096 27.9, 29.2, 28.2 -> 24.3, 27.1, 26.0; 10,240 x 8,192 49.2, 51.1, 52.1 -> 42.8, 46.9, 49.4 with three stages (one
 // block a CU); 22,016 x 4,096 43.4, 47.5, 49.6 -> 43.2, 46.3, 48.2 with two stages (two blocks; 47.6, 49.5, 51.0 with three).
+// So BNT = 128 up to a round of blocks and from 2,048 terms on (1,024: 1.03 of the time): M = 65, 128 x 12,288 x 4,096 30.7, 35.2 -> 28.9, 33.3; 150, 256 x 4,096
+// x 11,008 71.6, 79.0 -> 66.8, 72.8; 192 x 8,192 x 4,096 31.1 -> 29.8.
 template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm, int BK = 64>
 __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                      half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   constexpr bool L24 = WV == 8 && BMT == 64 && BNT == 128;   // 2 x 4 waves of 32 x 32
   constexpr bool L42 = WV == 8 && BNT <= 64;                 // 4 x 2 waves of 16 x 32 (x 16 at BNT 32)
   constexpr int RW = L42 ? 16 : 32, U = RW / 16;             // rows per wave, 16-row subtiles per wave
-  constexpr bool ONE = BNT == 64 && WV == 8;                 // one barrier a K-tile
+  constexpr bool ONE = WV == 8 && (BNT == 64 || BK == 128);  // one barrier a K-tile
   constexpr int LPR = BK / 8, RPD = 64 / LPR, KM = LPR - 1;  // lanes (16-byte chunks) a row, rows a DMA group of 1 KB
   // LDS-DMA groups: waves 0 .. NG % WV - 1 take one more when they do not divide evenly
   constexpr int NG = (BMT + BNT) / RPD, PER_WAVE = (NG + WV - 1) / WV, NG_REM = NG % WV;
@@ -962,7 +964,10 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
         break;
       case MID_64_W4: launch_mid<EPI, mid::NSTAGE, 64>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
       case MID_128R: launch_mid<EPI, mid::NSTAGE, 128, 8, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
-      case MID_128: launch_mid<EPI, mid::NSTAGE, 128, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
+      case MID_128:
+        if (K % 128 == 0 && K >= 2048 && (M + 63) / 64 * (N / 128) <= 256) launch_mid<EPI, 3, 128, 8, 64, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        else launch_mid<EPI, mid::NSTAGE, 128, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
+        break;
       case MID_128_W4: launch_mid<EPI, mid::NSTAGE, 128>(A, W, C, M, N, K, lda, ldw, ldc, ep, s); break;
     }
     FLS_CHECK_LAUNCH();

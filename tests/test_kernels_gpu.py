@@ -618,6 +618,33 @@ def test_gemm_makes_row_stat(ops, N, K):
     assert torch.is_tensor(ops.pending_stat(wide, 1e-5)) and isinstance(ops.pending_stat(x, 1e-5), RowStat)
 
 
+# 64 x 128 blocks of eight waves with K-tiles of 128 terms (K of 2,048 and more up to a round of blocks): the bits of four waves' with tiles of 64, for rows about
+# a row tile, K-tiles that are no multiple of the ring, a K that 128 does not divide and more than a round
+@pytest.mark.parametrize("N,K", [(256, 2048), (512, 2304), (1280, 4096), (256, 2112), (8192, 2048)])
+def test_gemm_mid_long_tiles_bitwise(ops, N, K):
+    from flexible_llm_sharding_amd.config import ModelConfig
+    from flexible_llm_sharding_amd.models.llama import rope_tables
+    x, w, r = rnd(330, K, seed=181), rnd(N, K, scale=0.03, seed=182), rnd(330, N, seed=183)
+    pos = torch.randint(0, 4096, (330,), dtype=torch.int32, device=DEV)
+    cos, sin = [t.to(DEV) for t in rope_tables(ModelConfig(hidden_size=256, num_attention_heads=2, num_key_value_heads=1), 4096)]
+
+    def forced(waves, fn):
+        old = (ops.k.fls_gemm_set_mid_bn(128), ops.k.fls_gemm_set_mid_waves(waves), ops.k.fls_gemm_set_mid_rows(64))
+        try:
+            return fn()
+        finally:
+            ops.k.fls_gemm_set_mid_bn(old[0])
+            ops.k.fls_gemm_set_mid_waves(old[1])
+            ops.k.fls_gemm_set_mid_rows(old[2])
+    for m in (1, 63, 64, 65, 128, 129, 256, 330):
+        def run():
+            return (ops.gemm(x[:m], w, EPI_SWIGLU), ops.gemm(x[:m], w, EPI_RESID, out=r[:m].clone(), resid=r[:m].clone()),
+                    ops.gemm(x[:m], w, EPI_ROPE, positions=pos[:m], cos=cos, sin=sin, rope_cols=N - 128, head_dim=128))
+        with ops.row_exact():
+            for a, b in zip(forced(8, run), forced(4, run)):
+                assert torch.equal(a, b), m
+
+
 def test_row_ss_matches_residual_epilogue(ops):
     """fls_row_ss on a hidden state == the partial sums of squares the residual GEMM epilogue wrote
     for the same rows (v10 / v11 tiles and the mid-M kernel + ss_partials), bit for bit, and the
