@@ -80,6 +80,12 @@ int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N,
              const float* sin_t, int rope_cols, int head_dim, const void* bias, const float* rscale,
              float rs_eps, float alpha, float* ss, int ss_ld, void* ws, uint64_t ws_bytes,
              fls_stream_t s);   // ws: device scratch for the small-M split-K path (may be null)
+// A RoPE product that also writes columns kv_col0 .. N - 1 of row m into row kv_dst[m] of a K/V buffer of ld kv_ld (kv, or the address that
+// the device cell kv_at holds)
+int fls_gemm_kv(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int epi,
+                const int* pos, const float* cos_t, const float* sin_t, int rope_cols, int head_dim, const void* bias,
+                const float* rscale, float rs_eps, void* kv, void* const* kv_at, const int* kv_dst, int kv_col0,
+                int kv_ld, void* ws, uint64_t ws_bytes, fls_stream_t s);
 // ss (RESID only, may be null): ss[m * ss_ld + j] = sum of the squares of the fp16 outputs of row m in
 // columns [128 j, 128 j + 128) -- the row statistic of the next norm-folded projection without a
 // pass over the hidden state (fls_rstd_from_ss)

@@ -480,7 +480,7 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   const int m = wave * 16 + fr;
   if (wave < RT && m < M) {
     if constexpr (NP == 1) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc[0], e2);
-    else if constexpr (is_rope(EPI)) store_rope_pair(C, ldc, m, n0 + 4 * grp, acc[0], acc[1], e2);
+    else if constexpr (is_rope(EPI)) store_rope_pair<true>(C, ldc, m, n0 + 4 * grp, acc[0], acc[1], e2);
     else store_pair_off<EPI>(C, ldc, m, b * 32, 4 * grp, acc[0], acc[1], e2);
   }
 }
@@ -868,6 +868,7 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
   return best;
 }
 
+// -> 0; 1 where the product has also written the K/V rows (Epi::kv_dst)
 template <int EPI>
 int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
            const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes, Route route) {
@@ -947,13 +948,15 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
           if (stat) {
             if (M <= 16) launch_col16<EPI, 1, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
             else launch_col16<EPI, 2, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-            break;
+            FLS_CHECK_LAUNCH();
+            return ep.kv_dst != nullptr;
           }
         }
         if (M <= 16) launch_col16<EPI, 1, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else if (M <= 32) launch_col16<EPI, 2, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else launch_col16<EPI, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        break;
+        FLS_CHECK_LAUNCH();
+        return is_rope(EPI) && ep.kv_dst != nullptr;
       case MID_32:
         if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         break;
@@ -1013,7 +1016,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
 
 }  // namespace
 
-extern "C" int fls_kernels_version(void) { return 39; }
+extern "C" int fls_kernels_version(void) { return 40; }
 
 // tile order: 0 = by shape (default); g > 0: groups of g M tiles; g < 0: groups of -g N tiles (A/B, tests)
 extern "C" int fls_gemm_set_order(int order) {
@@ -1125,10 +1128,18 @@ extern "C" int fls_gemm_leaves_ss(int M, int N, int K, uint64_t ws_bytes) {
   return route == ROUTE_NONE ? (long)((M + 255) / 256) * (N / BN) >= 128 : route >= ROUTE_128;
 }
 
-extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
-                        int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
-                        int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, float alpha, float* ss,
-                        int ss_ld, void* ws, uint64_t ws_bytes, fls_stream_t s) {
+namespace {
+struct KvOut {
+  half_t* kv;
+  half_t* const* kv_at;
+  const int* dst;
+  int col0, ld;
+};
+// fls_gemm; 1 where the product has also written the K/V rows
+int gemm_entry(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
+               int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
+               int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, float alpha, float* ss,
+               int ss_ld, const KvOut* kv, void* ws, uint64_t ws_bytes, fls_stream_t s) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const int row_exact = (epi & FLS_GEMM_ROW_EXACT) ? 1 : 0;
   epi &= 0xff;
@@ -1158,6 +1169,13 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
          nullptr, nullptr, 0, 0};
   ep.rs = rscale;
   ep.rs_eps = rs_eps;
+  if (kv != nullptr) {
+    ep.kv = kv->kv;
+    ep.kv_at = kv->kv_at;
+    ep.kv_dst = kv->dst;
+    ep.kv_col0 = kv->col0;
+    ep.kv_ld = kv->ld;
+  }
   ep.alpha = alpha;
   ep.ss = ss;
   ep.ss_ld = ss_ld;
@@ -1175,4 +1193,29 @@ extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, in
                              : launch<EPI_ROPE64>(a, w, c, M, N, K, lda, ldw, ldc, ep, st, ws, ws_bytes, route);
   }
   return -1;
+}
+}  // namespace
+
+extern "C" int fls_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
+                        int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
+                        int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, float alpha, float* ss,
+                        int ss_ld, void* ws, uint64_t ws_bytes, fls_stream_t s) {
+  return gemm_entry(A, W, C, R, M, N, K, lda, ldw, ldc, ldr, epi, pos, cos_t, sin_t, rope_cols, head_dim, bias, rscale, rs_eps, alpha, ss, ss_ld, nullptr, ws,
+                    ws_bytes, s);
+}
+
+// A RoPE product whose rows' columns from kv_col0 on (new keys and values) also go to rows kv_dst of a K/V buffer: from the blocks of 16 pairs with
+// their own stores, else by fls_copy_rows behind it (16 rows x 8,192 columns: 4.6 us and a launch of a generation step's layer)
+extern "C" int fls_gemm_kv(const void* A, const void* W, void* C, int M, int N, int K, int lda, int ldw, int ldc, int epi, const int* pos, const float* cos_t,
+                           const float* sin_t, int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, void* kv, void* const* kv_at,
+                           const int* kv_dst, int kv_col0, int kv_ld, void* ws, uint64_t ws_bytes, fls_stream_t s) {
+  if (M <= 0) return 0;
+  if ((epi & 0xff) != FLS_EPI_ROPE || !kv_dst || kv_col0 < 0 || kv_col0 >= N || kv_col0 % 8 || (head_dim > 0 && kv_col0 % head_dim) || kv_ld % 8 || ldc % 8 || N % 8 ||
+      (kv_at == nullptr && (!kv || ((uintptr_t)kv & 15))) || ((uintptr_t)C & 15))
+    return -2;
+  const KvOut out = {(half_t*)kv, (half_t* const*)kv_at, kv_dst, kv_col0, kv_ld};
+  const int rc = gemm_entry(A, W, C, C, M, N, K, lda, ldw, ldc, ldc, epi, pos, cos_t, sin_t, rope_cols, head_dim, bias, rscale, rs_eps, 1.f, nullptr, 0, &out, ws,
+                            ws_bytes, s);
+  if (rc) return rc > 0 ? 0 : rc;
+  return fls_copy_rows((const half_t*)C + kv_col0, ldc, nullptr, kv, kv_ld, kv_at, kv_dst, M, N - kv_col0, s);
 }

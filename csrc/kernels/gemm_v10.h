@@ -48,6 +48,11 @@ struct Epi {
   // rsqrt(mean(x^2) + eps) of a GEMM that reads the un-normalised hidden state x with the norm
   // weight folded into W (fused RMSNorm + projection); applied before the bias
   const float* rs = nullptr;
+  // RoPE products of 16-pair blocks (fls_gemm_kv): row m's columns from kv_col0 on into row kv_dst[m] of a K/V buffer too (kv, or what lies at kv_at)
+  half_t* kv = nullptr;
+  half_t* const* kv_at = nullptr;
+  const int* kv_dst = nullptr;
+  int kv_col0 = 0, kv_ld = 0;
   // > 0: the 16-pair blocks make that statistic themselves, of the rows of A (and rs is not read)
   float rs_eps = 0.f;
   // scale of (product + bias) before the residual add (Granite's residual_multiplier)
@@ -133,6 +138,7 @@ __device__ __forceinline__ void store_pair_off(half_t* __restrict__ C, int ldc, 
 // RoPE pair: columns ca (first half of a head) and ca + hd/2 of row m; f = ca % hd.  The arithmetic
 // is epilogue_rope's, expression for expression (x = acc * s + bias, then the rotation), so the mid-M
 // kernel's rows are bitwise the v10 / v11 rows (row-exact calls take either)
+template <bool KV = false>
 __device__ __forceinline__ void store_rope_pair(half_t* __restrict__ C, int ldc, int m, int ca, const floatx4& acc_a,
                                                 const floatx4& acc_b, const Epi& ep) {
   const int hd = ep.head_dim, half_hd = hd >> 1;
@@ -165,6 +171,13 @@ __device__ __forceinline__ void store_rope_pair(half_t* __restrict__ C, int ldc,
   }
   *(half4*)(C + (size_t)m * ldc + ca) = oa;
   *(half4*)(C + (size_t)m * ldc + cb) = ob;
+  if constexpr (KV) {
+    if (ep.kv_dst != nullptr && ca >= ep.kv_col0) {        // (a pair lies in one head: both or none)
+      half_t* const row = (ep.kv_at != nullptr ? *ep.kv_at : ep.kv) + (size_t)ep.kv_dst[m] * ep.kv_ld - ep.kv_col0;
+      *(half4*)(row + ca) = oa;
+      *(half4*)(row + cb) = ob;
+    }
+  }
 }
 
 // 16-byte stores of a pair of neighbouring 16-column subtiles (columns c .. c+31 of one row).

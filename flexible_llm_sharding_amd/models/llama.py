@@ -321,11 +321,14 @@ def balanced_step(rows: int, limit: int, align: int = 0) -> int:
     return limit
 
 
-def _proj(ctx: ExecContext, W: Dict[str, torch.Tensor], h, wr, p, n_q, n_k, bias, out=None, rscale=None):
+def _proj(ctx: ExecContext, W: Dict[str, torch.Tensor], h, wr, p, n_q, n_k, bias, out=None, rscale=None, kv=None):
     """QKV-shaped projection of ``h`` by ``wr`` with RoPE on the first n_q + n_k heads (Qwen3:
-    per-head q / k RMSNorm first); ``rscale``: per-row scale of the fused RMSNorm (HIP only)."""
+    per-head q / k RMSNorm first); ``rscale``: per-row scale of the fused RMSNorm (HIP only); ``kv`` = (buffer, the cell of its
+    address, row of it for each row): its K/V columns go there too (backends with ``writes_kv``)."""
     cfg = ctx.cfg
     kw = {"rscale": rscale} if rscale is not None else {}
+    if kv is not None:
+        kw["kv"] = (*kv, n_q * cfg.head_dim)
     if cfg.qk_norm:
         return ctx.ops.qkv_norm_rope(h, wr, p, ctx.cos, ctx.sin, n_q, n_k, cfg.head_dim, W["qn"], W["kn"],
                                      cfg.rms_norm_eps, bias=bias, out=out, **kw)
@@ -348,14 +351,15 @@ def _scored_q(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, las
 
 def _attn_inputs(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, pos: torch.Tensor,
                  last_idx: Optional[torch.Tensor], prune: bool, last_pos: Optional[torch.Tensor] = None,
-                 q_scored: Optional[torch.Tensor] = None, ss_key: Optional[tuple] = None) -> torch.Tensor:
+                 q_scored: Optional[torch.Tensor] = None, ss_key: Optional[tuple] = None, kv_out: Optional[tuple] = None) -> torch.Tensor:
     """RMSNorm + QKV projection (+ RoPE, + bias) of every row into one [T, qkv] buffer.
     ``prune`` (the last decoder layer): K/V (+ RoPE on K) for every row, Q only for the scored rows,
     scattered into the Q columns of those rows — the other rows' Q columns stay unwritten, the last
     layer's attention work items (``work_last``) query only scored rows (Q is q_size / qkv_size of
     the projection: 80% for Llama-2-70B).  ``q_scored``: that Q, already projected (the grouped
     attention phase projects every group's scored rows in one GEMM, as the whole-batch path does).
-    ``ss_key``: the previous layer's residual GEMM whose partial sums give the row statistic.
+    ``ss_key``: the previous layer's residual GEMM whose partial sums give the row statistic.  ``kv_out``: _proj's ``kv`` of
+    every row (fused only).
 
     Fused (``ctx.fused_norm``, HIP): one GEMM over the raw hidden state with ln1 folded into W_qkv
     and each row scaled by its rsqrt(mean(x^2) + eps) in the epilogue — the workspace holds only
@@ -368,8 +372,8 @@ def _attn_inputs(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, 
     T0 = x.shape[0]
     w, b = W["wqkv"], W.get("bqkv")
 
-    def proj(h, wr, p, n_q, n_k, bias, out=None, rscale=None):
-        return _proj(ctx, W, h, wr, p, n_q, n_k, bias, out=out, rscale=rscale)
+    def proj(h, wr, p, n_q, n_k, bias, out=None, rscale=None, kv=None):
+        return _proj(ctx, W, h, wr, p, n_q, n_k, bias, out=out, rscale=rscale, kv=kv)
 
     def put(r, dst):
         if r.data_ptr() != dst.data_ptr():
@@ -386,9 +390,9 @@ def _attn_inputs(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tensor, 
             qkv = torch.empty(T0, Qn, dtype=x.dtype, device=x.device)
         rstd = ctx.rstd(x, ss_key, out=ctx.scratch_f32(T0))
         if not prune:
-            put(proj(x, w, pos, nq, nkv, b, out=qkv, rscale=rstd), qkv)
+            put(proj(x, w, pos, nq, nkv, b, out=qkv, rscale=rstd, kv=kv_out), qkv)
             return qkv
-        put(proj(x, w[qs:], pos, 0, nkv, b[qs:] if b is not None else None, out=qkv[:, qs:], rscale=rstd),
+        put(proj(x, w[qs:], pos, 0, nkv, b[qs:] if b is not None else None, out=qkv[:, qs:], rscale=rstd, kv=kv_out),
             qkv[:, qs:])
         scored_q()
         return qkv
@@ -419,18 +423,25 @@ def _attention_whole(ctx: ExecContext, W: Dict[str, torch.Tensor], x: torch.Tens
     projection + residual (in place on x; the pruned last layer returns its scored rows)."""
     cfg, ops = ctx.cfg, ctx.ops
     li = _decoder_index(layer_name)
-    qkv = _attn_inputs(ctx, W, x, meta["positions"], meta["last_idx"], prune, meta["last_pos"],
-                       ss_key=(id(batch), li - 1, "mlp", x.shape[0]))
     kv0 = None
     kv_at = meta["kv_at"][layer_name] if "kv_at" in meta else None       # (captured: where a replay finds the layer's K/V)
     pe = ctx.prefix_entry
+    # Suffix K/V reuse, a step whose rows are all new suffix tokens (then sfx_src, in row order, is each row): the projection writes them
+    kv_out = None
+    if pe is not None and batch.kv_cached and not pe.host and "sfx_src" in meta and meta["sfx_src"].shape[0] == x.shape[0] and ctx.fused_norm \
+            and hasattr(ops, "writes_kv") and ops.writes_kv(cfg):
+        kv0 = pe.buffer(layer_name)
+        if kv0 is not None:
+            kv_out = (kv0, kv_at, meta["sfx_dst"])
+    qkv = _attn_inputs(ctx, W, x, meta["positions"], meta["last_idx"], prune, meta["last_pos"],
+                       ss_key=(id(batch), li - 1, "mlp", x.shape[0]), kv_out=kv_out)
     if pe is not None:
         qs, kv = cfg.q_size, 2 * cfg.num_key_value_heads * cfg.head_dim
         if batch.kv_cached:                  # prefix K/V of every prompt from the cache
             kv0 = pe.buffer(layer_name)
         elif "pfx_src" in meta:              # full pass: keep the prefix rows' post-RoPE K/V
             ops.copy_rows(qkv[:, qs:qs + kv], meta["pfx_src"], pe.buffer(layer_name, create=True), meta["pfx_dst"])
-        if "sfx_src" in meta:                # the suffix rows computed now (suffix K/V reuse)
+        if "sfx_src" in meta and kv_out is None:     # the suffix rows computed now (suffix K/V reuse)
             if kv0 is None:
                 kv0 = pe.buffer(layer_name, create=True)
             ops.copy_rows(qkv[:, qs:qs + kv], meta["sfx_src"], kv0, meta["sfx_dst"], **({} if kv_at is None else {"y_at": kv_at}))

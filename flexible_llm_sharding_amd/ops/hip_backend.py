@@ -92,10 +92,11 @@ class HipOps:
     def gemm(self, x: torch.Tensor, w: torch.Tensor, epi: int = EPI_NONE, out: torch.Tensor = None,
              resid: torch.Tensor = None, positions=None, cos=None, sin=None, rope_cols: int = 0,
              head_dim: int = 0, bias: torch.Tensor = None, rscale: torch.Tensor = None,
-             alpha: float = 1.0, ss: torch.Tensor = None) -> torch.Tensor:
+             alpha: float = 1.0, ss: torch.Tensor = None, kv=None) -> torch.Tensor:
         """rscale ([M] fp32, or the :class:`RowStat` of x): per-row scale of the raw product (before bias / epilogue); alpha:
         RESID's C = alpha * (product + bias) + R; ss ([>= M, N / 128] fp32, RESID): each output
-        row's partial sums of squares per 128 columns (:meth:`rstd_from_ss`)."""
+        row's partial sums of squares per 128 columns (:meth:`rstd_from_ss`); kv (RoPE): (buffer, the cell that holds its
+        address or None, row of it for each row, first column): the columns from there on go there too."""
         _f16(x, "x")
         _f16(w, "w")
         rs_eps = 0.0
@@ -121,6 +122,17 @@ class HipOps:
         if ss is not None and (ss.dtype != torch.float32 or not ss.is_cuda or ss.dim() != 2 or ss.shape[0] < M
                                or ss.shape[1] < N // 128 or ss.stride(1) != 1):
             raise TypeError(f"ss must be an fp32 CUDA [>= {M}, >= {N // 128}] matrix with unit column stride")
+        if kv is not None:
+            buf, at, dst, col0 = kv
+            _f16(buf, "kv buffer")
+            if dst.dtype != torch.int32 or not dst.is_cuda or dst.numel() != M or not dst.is_contiguous() or buf.shape[1] != N - col0:
+                raise ValueError("kv: one int32 row of the buffer for each row of x, and columns that fit it")
+            _chk(self.k.fls_gemm_kv(x.data_ptr(), w.data_ptr(), out.data_ptr(), M, N, K, x.stride(0), w.stride(0), out.stride(0), code,
+                                    positions.data_ptr(), cos.data_ptr(), sin.data_ptr(), rope_cols, head_dim,
+                                    bias.data_ptr() if bias is not None else None, rscale.data_ptr() if rscale is not None else None, rs_eps,
+                                    buf.data_ptr() if at is None else None, at, dst.data_ptr(), col0, buf.stride(0),
+                                    ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0, _stream()), "fls_gemm_kv")
+            return out
         rc = self.k.fls_gemm(x.data_ptr(), w.data_ptr(), out.data_ptr(), R.data_ptr(), M, N, K,
                              x.stride(0), w.stride(0), out.stride(0), R.stride(0), code,
                              positions.data_ptr() if positions is not None else None,
@@ -317,8 +329,12 @@ class HipOps:
         """y[idx] = x in place (distinct indices)."""
         return self.copy_rows(x, None, y, idx)
 
+    def writes_kv(self, cfg) -> bool:
+        """Does :meth:`qkv_rope` of such a model take ``kv``?"""
+        return not cfg.qk_norm and cfg.head_dim in (64, 128)
+
     def qkv_rope(self, x, wqkv, positions, cos, sin, n_q_heads, n_kv_heads, head_dim, bias=None, out=None,
-                 rscale=None):
+                 rscale=None, kv=None):
         if positions.dtype != torch.int32:
             raise TypeError("positions must be int32")
         rope_cols = (n_q_heads + n_kv_heads) * head_dim
@@ -332,7 +348,7 @@ class HipOps:
             _chk(rc, "fls_headnorm_rope")
             return y
         return self.gemm(x, wqkv, EPI_ROPE, out=out, positions=positions, cos=cos, sin=sin,
-                         rope_cols=rope_cols, head_dim=head_dim, bias=bias, rscale=rscale)
+                         rope_cols=rope_cols, head_dim=head_dim, bias=bias, rscale=rscale, kv=kv)
 
     def qkv_norm_rope(self, x, wqkv, positions, cos, sin, n_q_heads, n_kv_heads, head_dim, qn, kn, eps,
                       bias=None, out=None, rscale=None):

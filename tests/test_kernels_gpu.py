@@ -618,6 +618,34 @@ def test_gemm_makes_row_stat(ops, N, K):
     assert torch.is_tensor(ops.pending_stat(wide, 1e-5)) and isinstance(ops.pending_stat(x, 1e-5), RowStat)
 
 
+# a RoPE product that also writes its rows' keys and values into a K/V buffer (a row of it each, by address or through a cell): the bits of the product and of
+# copy_rows behind it, from the 16-pair blocks (with the row statistic and without) and on every other path; rows that no product names stay as they were
+@pytest.mark.parametrize("nq,nkv,hd,K", [(8, 2, 128, 256), (4, 4, 64, 512), (32, 8, 128, 1024), (0, 8, 64, 512)])
+def test_gemm_writes_kv(ops, nq, nkv, hd, K):
+    from flexible_llm_sharding_amd.config import ModelConfig
+    from flexible_llm_sharding_amd.models.llama import rope_tables
+    from flexible_llm_sharding_amd.ops.hip_backend import RowStat
+    N, col0 = (nq + 2 * nkv) * hd, nq * hd
+    x, w, b = rnd(200, K, seed=191), rnd(N, K, scale=0.03, seed=192), rnd(N, scale=0.5, seed=193)
+    pos = torch.randint(0, 4096, (200,), dtype=torch.int32, device=DEV)
+    cos, sin = [t.to(DEV) for t in rope_tables(ModelConfig(hidden_size=hd * 2, num_attention_heads=2, num_key_value_heads=1), 4096)]
+    for m in (1, 15, 16, 17, 33, 64, 65, 200):
+        dst = torch.randperm(300, generator=torch.Generator().manual_seed(m))[:m].to(torch.int32).to(DEV)
+        for exact in (True, False):
+            for stat in (False, True):
+                rs = lambda: RowStat(torch.empty(m, device=DEV), 1e-5) if stat else None
+                kw = dict(positions=pos[:m], cos=cos, sin=sin, rope_cols=(nq + nkv) * hd, head_dim=hd, bias=b)
+                with ops.row_exact(exact):
+                    want = ops.gemm(x[:m], w, EPI_ROPE, rscale=rs(), **kw)
+                    kv_want = torch.full((300, N - col0), 7.0, dtype=torch.float16, device=DEV)
+                    ops.copy_rows(want[:, col0:], None, kv_want, dst)
+                    for at in (False, True):
+                        kv = torch.full((300, N - col0), 7.0, dtype=torch.float16, device=DEV)
+                        cell = torch.tensor([kv.data_ptr()], dtype=torch.int64, device=DEV)
+                        got = ops.gemm(x[:m], w, EPI_ROPE, rscale=rs(), kv=(kv, cell.data_ptr() if at else None, dst, col0), **kw)
+                        assert torch.equal(got, want) and torch.equal(kv, kv_want), (m, exact, stat, at)
+
+
 # 64 x 128 blocks of eight waves with K-tiles of 128 terms (K of 2,048 and more up to a round of blocks): the bits of four waves' with tiles of 64, for rows about
 # a row tile, K-tiles that are no multiple of the ring, a K that 128 does not divide and more than a round
 @pytest.mark.parametrize("N,K", [(256, 2048), (512, 2304), (1280, 4096), (256, 2112), (8192, 2048)])
