@@ -311,19 +311,35 @@ extern "C" int fls_seq_add_scaled_dyt(float* x, int ldx, const float* y, int ldy
 }
 
 // ------------------------------------------------------------------------------- embedding
-template <typename T>
-__global__ void embed_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int D, int V, float scale) {
+// (four columns a lane and four of its pieces' loads in flight where the rows allow it: single columns took
+// a load, a wait and a store for each 256: us, 8 rows of 2,048 in bf16 2.5 -> 2.1, of 4,096 3.5 -> 2.2, 1,024 of 4,096 9.1 -> 5.9, 9,000 64.7 -> 35.8)
+template <typename T, int VE>
+__global__ __launch_bounds__(256) void embed_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int D, int V, float scale) {
   const int t = blockIdx.x;
   int id = ids[t];
   id = id < 0 ? 0 : (id >= V ? V - 1 : id);
   const T* row = table + (size_t)id * D;
-  for (int c = threadIdx.x; c < D; c += blockDim.x) out[(size_t)t * D + c] = ldf(row, c) * scale;
+  float* o = out + (size_t)t * D;
+  for (int c0 = VE * threadIdx.x; c0 < D; c0 += 4 * 256 * VE) {
+    RowVec<VE> v[4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) v[x] = row_load<VE>(row + min(c0 + x * 256 * VE, D - VE));
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+#pragma unroll
+      for (int e = 0; e < VE; ++e) v[x].v[e] *= scale;
+      if (c0 + x * 256 * VE < D) row_store<VE>(o + c0 + x * 256 * VE, v[x]);
+    }
+  }
 }
 
 extern "C" int fls_seq_embed(const int* ids, const void* table, int tt, float* out, int T, int D, int V, float scale, fls_stream_t s) {
-  if (T <= 0) return 0;
-  if (tt == 1) hipLaunchKernelGGL((embed_kernel<bf16_t>), dim3(T), dim3(256), 0, (hipStream_t)s, ids, (const bf16_t*)table, out, D, V, scale);
-  else hipLaunchKernelGGL((embed_kernel<float>), dim3(T), dim3(256), 0, (hipStream_t)s, ids, (const float*)table, out, D, V, scale);
+  if (T <= 0 || D <= 0) return 0;
+  const bool vec = D % 4 == 0 && (((uintptr_t)table | (uintptr_t)out) & 15) == 0;
+#define EMBED(TT, VE) hipLaunchKernelGGL((embed_kernel<TT, VE>), dim3(T), dim3(256), 0, (hipStream_t)s, ids, (const TT*)table, out, D, V, scale)
+  if (tt == 1) { if (vec) EMBED(bf16_t, 4); else EMBED(bf16_t, 1); }
+  else { if (vec) EMBED(float, 4); else EMBED(float, 1); }
+#undef EMBED
   SEQ_LAUNCH_CHECK();
   return 0;
 }

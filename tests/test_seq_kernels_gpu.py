@@ -1451,6 +1451,24 @@ def test_dyt_norm_scaled_add_and_embedding_scale(ops, cdt, tol):
     close(H.embed_rows(ids, table, scale=0.37), R.embed_rows(ids, table, scale=0.37), 1e-6)
 
 
+# embedding rows by four columns a lane and by one: widths about a block's turn of 1,024 columns and the four or two of them in flight, tables that vectors do
+# not fit; ids out of range; with positions, pairs and copies.  Sums of three values of the table's type in fp32, whose order is the oracle's: 1e-6
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [4, 1020, 1024, 1028, 2052, 4096, 4100, 1023])
+def test_embedding_widths(ops, cdt, D):
+    H, R = ops
+    torch.manual_seed(D)
+    flat = torch.randn(60 * D + 1, device=DEV).to(cdt)
+    ids = torch.tensor([3, 59, 0, 77, -1, 12], dtype=torch.int32, device=DEV)
+    clamped = ids.clamp(0, 59)
+    for table in (flat[:60 * D].view(60, D), flat[1:].view(60, D)):
+        close(H.embed_rows(ids, table, scale=0.37), R.embed_rows(clamped, table, scale=0.37), 1e-6)
+        ptab, pairs = torch.randn(9, D, device=DEV).to(cdt), torch.randn(12, D, device=DEV).to(cdt)
+        pos, prev = torch.arange(6, dtype=torch.int32, device=DEV), torch.tensor([-1, 3, 4, 0, 9, 50], dtype=torch.int32, device=DEV)
+        for kw in (dict(pos_table=ptab, tok_pos=pos), dict(bigram=(pairs, prev, 31, 17)), dict(pos_table=ptab, tok_pos=pos, copies=3)):
+            close(H.embed_rows(ids, table, **kw), R.embed_rows(clamped, table, **kw), 1e-6)
+
+
 @pytest.mark.parametrize("cdt,tol", DTYPES)
 def test_rotation_with_rescaled_frequencies_then_unit_norm(ops, cdt, tol):
     """Pair rotation with wavelength-rescaled frequencies followed by the weightless RMS norm, into rows and into pools;
