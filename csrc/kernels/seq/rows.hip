@@ -999,7 +999,7 @@ __global__ __launch_bounds__(64 * NW) void moe_route_softmax_grouped_kernel(cons
   __syncthreads();
   if constexpr (!FUSED) {                            // (one number per block and expert)
     for (int e = threadIdx.x; e < E; e += 64 * NW)
-      if (cnt[e]) atomicAdd(hist + e, cnt[e]);
+      if (hist != nullptr && cnt[e]) atomicAdd(hist + e, cnt[e]);
   } else {
     if (wave == 0) {
       const int per = (E + 63) / 64, e0 = min(E, lane * per), e1 = min(E, e0 + per);
@@ -1065,7 +1065,7 @@ extern "C" int fls_seq_moe_route_grouped(const float* logits, int ldl, int T, in
   hipLaunchKernelGGL(moe_route_grouped_kernel, dim3((T + 127) / 128), dim3(128), 0, (hipStream_t)s, logits, ldl, T, E, top, groups,
                      keep, scale, ids, w);
   SEQ_LAUNCH_CHECK();
-  hipLaunchKernelGGL(moe_hist_kernel, dim3((T * top + 4095) / 4096), dim3(256), 0, (hipStream_t)s, ids, T * top, E, hist);
+  if (hist != nullptr) hipLaunchKernelGGL(moe_hist_kernel, dim3((T * top + 4095) / 4096), dim3(256), 0, (hipStream_t)s, ids, T * top, E, hist);
   SEQ_LAUNCH_CHECK();
   return 0;
 }
@@ -1077,7 +1077,7 @@ extern "C" int fls_seq_moe_route(const float* logits, int ldl, const float* corr
   if (corr != nullptr) return moe_route_softmax(logits, ldl, corr, T, E, top, 0, 0, 1.f, 1, ids, w, hist, offs, dest, rows, (hipStream_t)s);
   hipLaunchKernelGGL(moe_route_kernel, dim3((T + 127) / 128), dim3(128), 0, (hipStream_t)s, logits, ldl, T, E, top, ids, w);
   SEQ_LAUNCH_CHECK();
-  hipLaunchKernelGGL(moe_hist_kernel, dim3((T * top + 4095) / 4096), dim3(256), 0, (hipStream_t)s, ids, T * top, E, hist);
+  if (hist != nullptr) hipLaunchKernelGGL(moe_hist_kernel, dim3((T * top + 4095) / 4096), dim3(256), 0, (hipStream_t)s, ids, T * top, E, hist);
   SEQ_LAUNCH_CHECK();
   return 0;
 }
@@ -1085,17 +1085,42 @@ extern "C" int fls_seq_moe_route(const float* logits, int ldl, const float* corr
 // Entries to their rows: every block scans the counts for itself (lane l of its first wave sums a run of ceil(E / 64) experts, the runs'
 // starts come from a prefix sum over the lanes), the first one leaves them in offs; it ranks its entries in LDS and takes its places with
 // one atomic per expert (32768 entries of 8 experts: 50 us with an atomic per wave and expert, 6.8 here).
+// SELF (few entries): every block counts all of them for itself, and those of the blocks before it for its places: no counts and cursors that have to be zeroed
+// first, and no atomics on memory (a launch less for each layer with experts of a prompt's portion).
 #define PLACE_THREADS 1024
+template <bool SELF>
 __global__ __launch_bounds__(PLACE_THREADS) void moe_place_kernel(const int* __restrict__ ids, int n, int top, const int* __restrict__ hist, int E,
                                                         int* __restrict__ offs, int* __restrict__ cursor, int* __restrict__ dest,
                                                         int* __restrict__ rows) {
-  __shared__ int start[MOE_MAX_E], cnt[MOE_MAX_E];
-  for (int e = threadIdx.x; e < E; e += PLACE_THREADS) cnt[e] = 0;
+  __shared__ int start[MOE_MAX_E], cnt[MOE_MAX_E], tot[SELF ? MOE_MAX_E : 1], bef[SELF ? MOE_MAX_E : 1];
+  for (int e = threadIdx.x; e < E; e += PLACE_THREADS) {
+    cnt[e] = 0;
+    if constexpr (SELF) tot[e] = bef[e] = 0;
+  }
+  if constexpr (SELF) {
+    __syncthreads();
+    for (int base = threadIdx.x & ~63; base < n; base += PLACE_THREADS) {        // 64 entries a wave; the lanes of one expert count together
+      const int at = base + (threadIdx.x & 63);
+      const int e = at < n ? ids[at] : -1;
+      unsigned long long todo = __ballot(at < n);
+      while (todo) {
+        const int leader = __ffsll((long long)todo) - 1, el = __shfl(e, leader, 64);
+        const unsigned long long same = __ballot(e == el);
+        if ((int)(threadIdx.x & 63) == leader) {
+          atomicAdd(&tot[el], __popcll(same));
+          if (base < (int)blockIdx.x * PLACE_THREADS) atomicAdd(&bef[el], __popcll(same));
+        }
+        todo &= ~same;
+      }
+    }
+    __syncthreads();
+  }
+  const auto count = [&](int e) { return SELF ? tot[SELF ? e : 0] : hist[e]; };
   if (threadIdx.x < 64) {
     const int lane = threadIdx.x, per = (E + 63) / 64;
     const int e0 = min(E, lane * per), e1 = min(E, e0 + per);
     int own = 0;
-    for (int e = e0; e < e1; ++e) own += hist[e];
+    for (int e = e0; e < e1; ++e) own += count(e);
     int acc = own;
     for (int o = 1; o < 64; o <<= 1) {
       const int v = __shfl_up(acc, o, 64);
@@ -1105,9 +1130,9 @@ __global__ __launch_bounds__(PLACE_THREADS) void moe_place_kernel(const int* __r
     if (first && lane == 63) offs[E] = acc;
     acc -= own;
     for (int e = e0; e < e1; ++e) {
-      start[e] = acc;
+      start[e] = acc + (SELF ? bef[SELF ? e : 0] : 0);
       if (first) offs[e] = acc;
-      acc += hist[e];
+      acc += count(e);
     }
   }
   __syncthreads();
@@ -1129,9 +1154,11 @@ __global__ __launch_bounds__(PLACE_THREADS) void moe_place_kernel(const int* __r
     todo &= ~same;
   }
   __syncthreads();
-  for (int g = threadIdx.x; g < E; g += PLACE_THREADS)
-    if (cnt[g]) start[g] += atomicAdd(cursor + g, cnt[g]);
-  __syncthreads();
+  if constexpr (!SELF) {
+    for (int g = threadIdx.x; g < E; g += PLACE_THREADS)
+      if (cnt[g]) start[g] += atomicAdd(cursor + g, cnt[g]);
+    __syncthreads();
+  }
   if (valid) {
     const int p = start[e] + rank;
     dest[i] = p;
@@ -1143,7 +1170,13 @@ extern "C" int fls_seq_moe_place(const int* ids, int n, int top, const int* hist
                                  fls_stream_t s) {
   if (n <= 0) return 0;
   if (E < 1 || E > MOE_MAX_E) return -1;
-  hipLaunchKernelGGL(moe_place_kernel, dim3((n + PLACE_THREADS - 1) / PLACE_THREADS), dim3(PLACE_THREADS), 0, (hipStream_t)s, ids, n, top, hist, E, offs, cursor, dest, rows);
+  const dim3 blocks((n + PLACE_THREADS - 1) / PLACE_THREADS);
+  if (hist == nullptr) {
+    if (n > FLS_SEQ_PLACE_SELF) return -1;
+    hipLaunchKernelGGL((moe_place_kernel<true>), blocks, dim3(PLACE_THREADS), 0, (hipStream_t)s, ids, n, top, hist, E, offs, cursor, dest, rows);
+  } else {
+    hipLaunchKernelGGL((moe_place_kernel<false>), blocks, dim3(PLACE_THREADS), 0, (hipStream_t)s, ids, n, top, hist, E, offs, cursor, dest, rows);
+  }
   SEQ_LAUNCH_CHECK();
   return 0;
 }
@@ -1190,4 +1223,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 22; }
+extern "C" int fls_seq_version(void) { return 23; }

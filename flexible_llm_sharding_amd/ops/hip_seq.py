@@ -393,20 +393,30 @@ class HipSeqOps:
         # every head's output over its own root mean square, times the weight the heads share
         return self.head_norm_rope(raw, heads, vdim, 0, vdim, out, 0, vdim, meta, w=norm_w, eps=eps)
 
+    # Up to so many entries (the limit in csrc/include/fls_seq.h) of so many experts their placement counts them itself: us of the whole route in a
+    # graph, with the launch that zeroes the counts and so, 8 experts: 130 entries 8.7, 7.1; 1,024 9.4, 7.9; 2,048 9.7, 9.1; 4,096 10.6, 11.6; 1,600 of 128 18.8, 25.7
+    PLACE_SELF, PLACE_SELF_EXPERTS = 2048, 16
+
+    def _route_ints(self, E, n, dev, fused=False):
+        """-> (row offsets per expert, address of the zeroed counts or None, of the zeroed cursors or None) of n entries."""
+        if fused or (n <= self.PLACE_SELF and E <= self.PLACE_SELF_EXPERTS):
+            return torch.empty(E + 1, dtype=torch.int32, device=dev), None, None
+        ints = torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)          # offs | hist | cursor
+        return ints[:E + 1], ints.data_ptr() + 4 * (E + 1), ints.data_ptr() + 4 * (2 * E + 1)
+
     def moe_route_grouped(self, logits, top, groups, keep, scale):
         _rows(logits, "logits", torch.float32)
         T, E = logits.shape
         dev = logits.device
         ids = torch.empty(T, top, dtype=torch.int32, device=dev)
         w = torch.empty(T, top, dtype=torch.float32, device=dev)
-        ints = torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)          # hist | cursor | offs
-        hist, cursor, offs = ints[:E], ints[E:2 * E], ints[2 * E:]
+        offs, hist, cursor = self._route_ints(E, T * top, dev)
         dest = torch.empty(T, top, dtype=torch.int32, device=dev)
         rows = torch.empty(T * top, dtype=torch.int32, device=dev)
         s = _stream()
         _chk(self.k.fls_seq_moe_route_grouped(logits.data_ptr(), logits.stride(0), T, E, top, int(groups or 0), int(keep or 0),
-                                              float(scale), ids.data_ptr(), w.data_ptr(), hist.data_ptr(), s), "fls_seq_moe_route_grouped")
-        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+                                              float(scale), ids.data_ptr(), w.data_ptr(), hist, s), "fls_seq_moe_route_grouped")
+        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist, E, offs.data_ptr(), cursor, dest.data_ptr(),
                                       rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 
@@ -421,17 +431,16 @@ class HipSeqOps:
         fused = T <= self.ROUTE_FUSED
         ids = torch.empty(T, top, dtype=torch.int32, device=dev)
         w = torch.empty(T, top, dtype=torch.float32, device=dev)
-        ints = torch.empty(E + 1, dtype=torch.int32, device=dev) if fused else torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)
-        offs, hist, cursor = ints[:E + 1], ints[E + 1:2 * E + 1], ints[2 * E + 1:]
+        offs, hist, cursor = self._route_ints(E, T * top, dev, fused)
         dest = torch.empty(T, top, dtype=torch.int32, device=dev)
         rows = torch.empty(T * top, dtype=torch.int32, device=dev)
         s = _stream()
         _chk(self.k.fls_seq_moe_route_softmax_grouped(logits.data_ptr(), logits.stride(0), corr.data_ptr() if corr is not None else None,
                                                       T, E, top, int(groups or 0), int(keep or 0), float(scale), ids.data_ptr(),
-                                                      w.data_ptr(), hist.data_ptr(), offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
+                                                      w.data_ptr(), hist, offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s),
              "fls_seq_moe_route_softmax_grouped")
         if not fused:
-            _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+            _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist, E, offs.data_ptr(), cursor, dest.data_ptr(),
                                           rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 
@@ -1056,16 +1065,15 @@ class HipSeqOps:
         ids = torch.empty(T, top, dtype=torch.int32, device=dev)
         w = torch.empty(T, top, dtype=torch.float32, device=dev)
         fused = corr is not None and 0 < T <= self.ROUTE_FUSED
-        ints = torch.empty(E + 1, dtype=torch.int32, device=dev) if fused else torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)
-        offs, hist, cursor = ints[:E + 1], ints[E + 1:2 * E + 1], ints[2 * E + 1:]
+        offs, hist, cursor = self._route_ints(E, T * top, dev, fused)
         dest = torch.empty(T, top, dtype=torch.int32, device=dev)
         rows = torch.empty(T * top, dtype=torch.int32, device=dev)
         s = _stream()
         _chk(self.k.fls_seq_moe_route(logits.data_ptr(), logits.stride(0), corr.data_ptr() if corr is not None else None, T, E, top, ids.data_ptr(),
-                                      w.data_ptr(), hist.data_ptr(), offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s), "fls_seq_moe_route")
+                                      w.data_ptr(), hist, offs.data_ptr(), dest.data_ptr(), rows.data_ptr(), s), "fls_seq_moe_route")
         if fused:
             return SeqRoute(ids, w, offs, rows, dest, top)
-        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist.data_ptr(), E, offs.data_ptr(), cursor.data_ptr(), dest.data_ptr(),
+        _chk(self.k.fls_seq_moe_place(ids.data_ptr(), T * top, top, hist, E, offs.data_ptr(), cursor, dest.data_ptr(),
                                       rows.data_ptr(), s), "fls_seq_moe_place")
         return SeqRoute(ids, w, offs, rows, dest, top)
 

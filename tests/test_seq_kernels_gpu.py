@@ -1451,6 +1451,27 @@ def test_dyt_norm_scaled_add_and_embedding_scale(ops, cdt, tol):
     close(H.embed_rows(ids, table, scale=0.37), R.embed_rows(ids, table, scale=0.37), 1e-6)
 
 
+# entries to their experts' rows, counted by the placement itself (up to 2,048 entries of 16 experts) and from counts: one block and several, wave and block edges, one expert and
+# the most, one that nobody takes; every entry in its expert's range, once
+@pytest.mark.parametrize("T,top", [(65, 1), (127, 2), (512, 2), (513, 2), (512, 4), (513, 4), (1500, 1), (2048, 1), (2049, 1)])
+@pytest.mark.parametrize("E", [1, 8, 10, 16, 17, 130])
+def test_placement_counts_itself(ops, T, top, E):
+    H, R = ops
+    if top > E:
+        return
+    torch.manual_seed(T + E)
+    logits = torch.randn(T, E, device=DEV)
+    logits[:, E // 2:E // 2 + 1] -= 50.0 if E > top else 0.0                     # (an expert that nobody takes)
+    for r in (H.moe_route_softmax_grouped(logits, None, top, 0, 0, 1.0), H.moe_route_corrected(logits, torch.zeros(E, device=DEV), top),
+              H.moe_route_corrected(logits, None, top), H.moe_route_grouped(logits, top, 0, 0, 1.0)):
+        ids = r.ids.long().flatten().cpu()
+        assert torch.equal(r.offs.long().cpu(), torch.cat([torch.zeros(1, dtype=torch.long), torch.bincount(ids, minlength=E).cumsum(0)]))
+        dest = r.dest.long().flatten().cpu()
+        assert torch.equal(dest.sort().values, torch.arange(T * top))
+        assert torch.equal(torch.bucketize(dest, r.offs.long().cpu()[1:], right=True), ids)
+        assert torch.equal(r.rows.long().cpu()[dest], torch.arange(T).repeat_interleave(top))
+
+
 # embedding rows by four columns a lane and by one: widths about a block's turn of 1,024 columns and the four or two of them in flight, tables that vectors do
 # not fit; ids out of range; with positions, pairs and copies.  Sums of three values of the table's type in fp32, whose order is the oracle's: 1e-6
 @pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
