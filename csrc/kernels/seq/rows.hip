@@ -344,17 +344,22 @@ extern "C" int fls_seq_embed(const int* ids, const void* table, int tt, float* o
   return 0;
 }
 
-template <typename T>
-__global__ void gather_rows_kernel(const T* __restrict__ x, int ldx, const int* __restrict__ idx, T* __restrict__ y, int ldy, int D) {
-  const T* xr = x + (size_t)idx[blockIdx.x] * ldx;
-  T* yr = y + (size_t)blockIdx.x * ldy;
+// (V: 16 bytes where rows and strides are multiples of them, else an element)
+template <typename V>
+__global__ void gather_rows_kernel(const V* __restrict__ x, int ldx, const int* __restrict__ idx, V* __restrict__ y, int ldy, int D) {
+  const V* xr = x + (size_t)idx[blockIdx.x] * ldx;
+  V* yr = y + (size_t)blockIdx.x * ldy;
   for (int c = threadIdx.x; c < D; c += blockDim.x) yr[c] = xr[c];
 }
 
 extern "C" int fls_seq_gather_rows(const void* x, int tx, int ldx, const int* idx, void* y, int ldy, int rows, int D,
                                    fls_stream_t s) {
   if (rows <= 0) return 0;
-  if (tx == 1) hipLaunchKernelGGL((gather_rows_kernel<bf16_t>), dim3(rows), dim3(256), 0, (hipStream_t)s, (const bf16_t*)x, ldx, idx, (bf16_t*)y, ldy, D);
+  const int per = tx == 1 ? 8 : 4;
+  // (us, bf16: 9,000 rows of 2,048 23.3 -> 12.9, of 576 10.1 -> 5.0)
+  if (D % per == 0 && ldx % per == 0 && ldy % per == 0 && (((uintptr_t)x | (uintptr_t)y) & 15) == 0)
+    hipLaunchKernelGGL((gather_rows_kernel<uint4>), dim3(rows), dim3(D / per <= 64 ? 64 : D / per <= 128 ? 128 : 256), 0, (hipStream_t)s, (const uint4*)x, ldx / per, idx, (uint4*)y, ldy / per, D / per);
+  else if (tx == 1) hipLaunchKernelGGL((gather_rows_kernel<bf16_t>), dim3(rows), dim3(256), 0, (hipStream_t)s, (const bf16_t*)x, ldx, idx, (bf16_t*)y, ldy, D);
   else hipLaunchKernelGGL((gather_rows_kernel<float>), dim3(rows), dim3(256), 0, (hipStream_t)s, (const float*)x, ldx, idx, (float*)y, ldy, D);
   SEQ_LAUNCH_CHECK();
   return 0;

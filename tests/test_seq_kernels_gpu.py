@@ -1472,6 +1472,17 @@ def test_placement_counts_itself(ops, T, top, E):
         assert torch.equal(r.rows.long().cpu()[dest], torch.arange(T).repeat_interleave(top))
 
 
+# gathered rows by 16 bytes and by elements: the same bytes, for widths about a block's threads, column slices and rows that vectors do not fit
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D", [8, 36, 512, 520, 1032, 2056, 4])
+def test_gathered_rows(ops, cdt, D):
+    H, _ = ops
+    x = torch.randn(50, D + 16, device=DEV).to(cdt)
+    idx = torch.tensor([49, 0, 7, 7, 31], dtype=torch.int32, device=DEV)
+    for a in (x[:, :D], x[:, 8:8 + D], x[:, 1:1 + D], x[:, :D].contiguous()):
+        assert torch.equal(H.gather_rows(a, idx), a[idx.long()])
+
+
 # embedding rows by four columns a lane and by one: widths about a block's turn of 1,024 columns and the four or two of them in flight, tables that vectors do
 # not fit; ids out of range; with positions, pairs and copies.  Sums of three values of the table's type in fp32, whose order is the oracle's: 1e-6
 @pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
