@@ -647,45 +647,38 @@ __global__ __launch_bounds__(256) void ss_partials_kernel(const half_t* __restri
   if (grp == 0 && m < M) ss[(size_t)m * ss_ld + j] = sq;
 }
 
-// the fused norm's statistic straight from x, one wave per row: lane j computes the 128-column
-// partials j, j + 64, ... itself, with ss_partials_kernel's per-lane FMA chains (one per 4-column group
-// g) combined as row_sum_4groups does, (g0 + g2) + (g1 + g3), and sums them in rstd_from_ss_kernel's
-// order (lane j takes parts j, j + 64, ..., then warp_sum): the same bits as fls_row_ss followed by
-// fls_rstd_from_ss, in one launch (generation steps run two per layer).  The 16-row lane layout of
-// the GEMM epilogue, kept here first, cost 16 us per launch at any row count (16 rows per block, 32
-// rows' worth of scattered 32-byte pieces per load); lane-per-part loads stream each row.
+// the fused norm's statistic straight from x: the 128-column parts of a row with ss_partials_kernel's per-lane FMA chains (one per
+// 4-column group g) combined as row_sum_4groups does, (g0 + g2) + (g1 + g3), and summed in rstd_from_ss_kernel's order
+// (lane j takes parts j, j + 64, ..., then warp_sum): the same bits as fls_row_ss followed by fls_rstd_from_ss, in one launch.
+// What bounds it is one row's chain: four lanes a part, one for each of its column groups, 128 lanes a row (us, a lane for a whole part before: 65 rows
+// of 4,096 3.03 -> 2.58, of 8,192 3.68 -> 2.90, 6,400 of 4,096 14.8 -> 10.7; one row 2.06 -> 2.21).
 constexpr int ROW_STAT_MAX_PARTS = 128;              // H <= 16,384
 __global__ __launch_bounds__(256) void row_stat_kernel(const half_t* __restrict__ x, int ldx, int M, int nparts, int H,
                                                        float eps, float* __restrict__ rstd) {
-  const int lane = threadIdx.x & 63;
-  const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (m >= M) return;                               // wave-uniform (no block barrier)
-  const half_t* row = x + (size_t)m * ldx;
-  float v = 0.f;
-  for (int j = lane; j < nparts; j += 64) {
-    half4 q[32];                                    // the part's 128 columns
+  __shared__ float parts[2][ROW_STAT_MAX_PARTS];
+  const int r = threadIdx.x >> 7, l = threadIdx.x & 127, g = l & 3, m = blockIdx.x * 2 + r;
+  const half_t* row = x + (size_t)min(m, M - 1) * ldx + 4 * g;
+  for (int j = l >> 2; j < nparts; j += 32) {
+    half4 q[8];
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const half8 c = *(const half8*)(row + j * 128 + k * 8);
-      q[2 * k] = c.lo;
-      q[2 * k + 1] = c.hi;
-    }
-    float sg[4];
+    for (int k = 0; k < 8; ++k) q[k] = *(const half4*)(row + j * 128 + k * 16);
+    float sq = 0.f;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float sq = 0.f;
-#pragma unroll
-      for (int p = 0; p < 4; ++p) sq = ss_accum_pair(sq, q[p * 8 + g], q[p * 8 + 4 + g]);
-      sg[g] = sq;
-    }
-    v += (sg[0] + sg[2]) + (sg[1] + sg[3]);
+    for (int p = 0; p < 4; ++p) sq = ss_accum_pair(sq, q[2 * p], q[2 * p + 1]);
+    sq += __shfl_xor(sq, 2, 64);
+    sq += __shfl_xor(sq, 1, 64);                    // (g0 + g2) + (g1 + g3)
+    if (g == 0) parts[r][j] = sq;
   }
+  __syncthreads();
+  if (l >= 64 || m >= M) return;                    // wave-uniform
+  float v = 0.f;
+  for (int j = l; j < nparts; j += 64) v += parts[r][j];
   v = warp_sum(v);
-  if (lane == 0) rstd[m] = rsqrtf(v / (float)H + eps);
+  if (l == 0) rstd[m] = rsqrtf(v / (float)H + eps);
 }
 
 void row_stat(const half_t* x, int ldx, int rows, int H, float eps, float* rstd, hipStream_t s) {
-  hipLaunchKernelGGL(row_stat_kernel, dim3((rows + 3) / 4), dim3(256), 0, s, x, ldx, rows, H / 128, H, eps, rstd);
+  hipLaunchKernelGGL(row_stat_kernel, dim3((rows + 1) / 2), dim3(256), 0, s, x, ldx, rows, H / 128, H, eps, rstd);
 }
 
 void ss_partials_raw(const half_t* C, int ldc, int M, int N, float* ss, int ss_ld, hipStream_t s) {
