@@ -850,8 +850,11 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
       least = us;
     }
   };
-  // (no lead for blocks of two panels, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's)
-  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (rules == ROUTE_MID && M <= 64 && two_panels(M, N, K, pairs) ? 1.f / 0.94f : 1.f));
+  // (no lead for blocks of two panels, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's.
+  // Above 16 rows and 4,096 terms the skinny path's blocks, the rules' choice there, are estimated up to 20% worse than they are: by the bare estimates plain products
+  // of 4,352 .. 14,336 columns took up to 1.22 of their time before there were two panels, 20% of them more than 1.04; so 0.99, 10% and 1.05 (1.3: up to 1.09)
+  const bool panels = M <= 64 && two_panels(M, N, K, pairs);
+  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (!panels ? 1.f : rules == ROUTE_MID ? 1.f / 0.94f : !pairs && M > 16 && K > 4096 ? 1.4f : 1.f));
   if (skinny) offer(ROUTE_SKINNY, skinny_us(M, N, K, bn, S));
   if (split) offer(ROUTE_SPLIT, split_us(M, N, K, S2));
   if (M > 64) {              // (up to 64 rows one row tile covers them all, and three quarters of a 256-row one are padding)

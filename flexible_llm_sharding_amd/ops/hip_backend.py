@@ -60,12 +60,6 @@ class MoeRoute:
     k: int
 
 
-def _softmax_part(logits):
-    # (stream-ordered scratch: the allocator hands it out again only behind the kernels that use it)
-    rows, V = logits.shape
-    return torch.empty(rows * 128, dtype=torch.float32, device=logits.device).data_ptr() if V > 32768 else None
-
-
 class RowStat(NamedTuple):
     """A row statistic (:meth:`HipOps.row_stat`) that the one product it scales makes: fp32 scratch of a value a row, epsilon."""
     buf: torch.Tensor
@@ -537,13 +531,19 @@ class HipOps:
              "fls_embed")
         return out
 
+    def _softmax_rows(self, logits, probs, logits_scaling, greedy):
+        rows, V = logits.shape
+        # (scratch of wide rows, held until their kernels are in the stream)
+        part = torch.empty(rows * 128, dtype=torch.float32, device=logits.device) if V > 32768 else None
+        _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
+                                     greedy.data_ptr() if greedy is not None else None, part.data_ptr() if part is not None else None, _stream()),
+             "fls_softmax")
+
     def softmax(self, logits, logits_scaling: float = 1.0):
         """Row softmax of fp16 logits (logits_scaling != 1: of fp16(logits / logits_scaling))."""
         _f16(logits, "logits")
-        rows, V = logits.shape
         probs = torch.empty_like(logits)
-        _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
-                                     None, _softmax_part(logits), _stream()), "fls_softmax")
+        self._softmax_rows(logits, probs, logits_scaling, None)
         return probs
 
     def softmax_greedy(self, logits, logits_scaling: float = 1.0):
@@ -554,8 +554,7 @@ class HipOps:
         at = -(-n // 16) * 16                                # (host copies lay them out alike)
         flat = torch.empty(at + 4 * rows, dtype=torch.uint8, device=logits.device)
         probs, greedy = flat[:n].view(torch.float16).view(rows, V), flat[at:].view(torch.int32)
-        _chk(self.k.fls_softmax_rows(logits.data_ptr(), probs.data_ptr(), rows, V, 1.0 / float(logits_scaling),
-                                     greedy.data_ptr(), _softmax_part(logits), _stream()), "fls_softmax")
+        self._softmax_rows(logits, probs, logits_scaling, greedy)
         return probs, greedy, flat
 
     def argmax_rows(self, probs):
