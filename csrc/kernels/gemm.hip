@@ -368,10 +368,10 @@ constexpr int stages(int rt, int np) { return np == 2 ? (rt == 2 ? 5 : 3) : rt =
 
 //
 // STAT (up to 32 rows): the row statistic that the epilogue applies is made here, from the rows of A that pass through LDS anyway, by the waves that only move
-// data, in row_stat_kernel's order (same bits): a lane has one row's column group, its parts of 128 columns stay in registers, four to a lane
-// group, and are added as warp_sum adds them.  A launch less for every norm + projection of a generation step.  us with that launch in front and so:
-// 16 rows x 12,288 x 4,096 28.1, 26.3; x 22,016 x 4,096 37.3, 36.6 (one row 36.3, 37.6); x 10,240 x 8,192 45.1, 41.4; x 6,144 x 2,048 10.6, 9.3; 32 rows x 6,144 x
-// 2,048 11.5, 10.4.  Above 32 rows the multiplying waves would have to make it: 48 rows 12.8, 15.1.
+// data (a wave for each part of 128 columns of a K-tile), in row_stat_kernel's order (same bits): a lane has one row's column group, its parts
+// stay in registers, four to a lane group, and are added as warp_sum adds them.  A launch less for every norm + projection of a generation step.  us with
+// that launch in front and so: 16 rows x 12,288 x 4,096 27.8, 26.0; x 22,016 x 4,096 36.9, 35.1; x 10,240 x 8,192 44.8, 42.9; x 6,144 x 2,048 10.4, 8.6; 32 rows
+// x 6,144 x 2,048 11.3, 10.4.  (Both parts of a tile in one wave: x 22,016 36.6.  Above 32 rows the multiplying waves would have to make it: 48 rows 12.8, 15.1.)
 template <int EPI, int RT, int NP, bool STAT>
 __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
@@ -403,9 +403,10 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   floatx4 acc[NP];
 #pragma unroll
   for (int h = 0; h < NP; ++h) acc[h] = floatx4{0.f, 0.f, 0.f, 0.f};
-  static_assert(!STAT || 2 * RT <= 4, "a wave beside each that multiplies");
-  const int srt = wave - RT;                             // row tile whose statistics the wave makes
-  const bool stat = STAT && srt >= 0 && srt < RT;
+  constexpr int SPW = KT / 128;                          // parts of 128 columns in a K-tile: a wave each
+  static_assert(!STAT || RT * (1 + SPW) <= 4, "waves beside those that multiply");
+  const int srt = (wave - RT) / SPW, spart = (wave - RT) % SPW;             // row tile and part whose statistics the wave makes
+  const bool stat = STAT && wave >= RT && srt < RT;
   const int srow = ((NP + srt) * 16 + fr) * KT * 2;
   unsigned so[8];                                        // a part's columns 32 p + 4 grp + 16 h of the row: 16-byte chunk 4 p + 2 h + grp / 2, half of it
 #pragma unroll
@@ -438,27 +439,21 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
     if (stat) {
-      const unsigned xs = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_c16 + (kt % NST) * STAGE + srow;
-      half4 q[KT / 128][8];
+      const unsigned xs = (unsigned)(size_t)(__attribute__((address_space(3))) char*)lds_c16 + (kt % NST) * STAGE + srow + spart * 256;
+      half4 q[8];                                        // (in asm: of loads of its own the compiler believes that they want every DMA landed)
+      asm volatile("ds_read_b64 %0, %8\n\tds_read_b64 %1, %9\n\tds_read_b64 %2, %10\n\tds_read_b64 %3, %11\n\t"
+                   "ds_read_b64 %4, %12\n\tds_read_b64 %5, %13\n\tds_read_b64 %6, %14\n\tds_read_b64 %7, %15\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(q[0]), "=&v"(q[1]), "=&v"(q[2]), "=&v"(q[3]), "=&v"(q[4]), "=&v"(q[5]), "=&v"(q[6]), "=&v"(q[7])
+                   : "v"(xs + so[0]), "v"(xs + so[1]), "v"(xs + so[2]), "v"(xs + so[3]), "v"(xs + so[4]), "v"(xs + so[5]), "v"(xs + so[6]), "v"(xs + so[7])
+                   : "memory");
+      float sq = 0.f;
 #pragma unroll
-      for (int i = 0; i < KT / 128; ++i)                 // (in asm: of loads of its own the compiler believes that they want every DMA landed)
-        asm volatile("ds_read_b64 %0, %8 offset:%c16\n\tds_read_b64 %1, %9 offset:%c16\n\tds_read_b64 %2, %10 offset:%c16\n\tds_read_b64 %3, %11 offset:%c16\n\t"
-                     "ds_read_b64 %4, %12 offset:%c16\n\tds_read_b64 %5, %13 offset:%c16\n\tds_read_b64 %6, %14 offset:%c16\n\tds_read_b64 %7, %15 offset:%c16\n\t"
-                     "s_waitcnt lgkmcnt(0)"
-                     : "=&v"(q[i][0]), "=&v"(q[i][1]), "=&v"(q[i][2]), "=&v"(q[i][3]), "=&v"(q[i][4]), "=&v"(q[i][5]), "=&v"(q[i][6]), "=&v"(q[i][7])
-                     : "v"(xs + so[0]), "v"(xs + so[1]), "v"(xs + so[2]), "v"(xs + so[3]), "v"(xs + so[4]), "v"(xs + so[5]), "v"(xs + so[6]), "v"(xs + so[7]),
-                       "n"(i * 256) : "memory");
+      for (int p = 0; p < 4; ++p) sq = ss_accum_pair(sq, q[2 * p], q[2 * p + 1]);
+      sq = row_sum_4groups(sq);
+      const int part = kt * SPW + spart;                 // lane group part % 4, register part / 4
+      if ((part & 3) == grp) {
 #pragma unroll
-      for (int i = 0; i < KT / 128; ++i) {
-        float sq = 0.f;
-#pragma unroll
-        for (int p = 0; p < 4; ++p) sq = ss_accum_pair(sq, q[i][2 * p], q[i][2 * p + 1]);
-        sq = row_sum_4groups(sq);
-        const int j = kt * (KT / 128) + i;               // part j: lane group j % 4, register j / 4
-        if ((j & 3) == grp) {
-#pragma unroll
-          for (int r = 0; r < (STAT ? 16 : 1); ++r) sp[r] = (j >> 2) == r ? sq : sp[r];
-        }
+        for (int r = 0; r < (STAT ? 16 : 1); ++r) sp[r] = (part >> 2) == r ? sq : sp[r];
       }
     }
   }
@@ -466,12 +461,17 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   Epi e2 = ep;
   if constexpr (STAT) {
     __syncthreads();                                     // (every wave's DMAs have landed and its reads are done)
+    float* const sums = reinterpret_cast<float*>(lds_c16) + 64;
     if (stat) {
 #pragma unroll
       for (int o = 8; o > 0; o >>= 1)
 #pragma unroll
         for (int r = 0; r < o; ++r) sp[r] += sp[r + o];
-      const float v = row_sum_4groups(sp[0]);
+      if (SPW == 2 && (grp & 1) == spart) sums[srt * 64 + lane] = sp[0];          // (a wave's parts lie in every other lane group)
+    }
+    if constexpr (SPW == 2) __syncthreads();
+    if (stat && spart == 0) {
+      const float v = row_sum_4groups(SPW == 2 ? sums[srt * 64 + lane] : sp[0]);
       if (grp == 0) reinterpret_cast<float*>(lds_c16)[srt * 16 + fr] = rsqrtf(v / (float)K + ep.rs_eps);
     }
     __syncthreads();
