@@ -1117,7 +1117,7 @@ extern "C" int fls_gemm_v11_try(const void* A, const void* W, void* C, const voi
 
 // Does a residual product of M x N x K write its rows' partial sums of squares in its epilogue (v10 and v11 tiles)?  On the other paths
 // they are a launch of their own behind it and a second one sums them; fls_row_stat gives the same bits in one (79 rows x 4,096:
-// 3.5 + 2.7 us and a launch more, 4.6 here).
+// 3.5 + 2.7 us and a launch more, 2.6 here).
 extern "C" int fls_gemm_leaves_ss(int M, int N, int K, uint64_t ws_bytes) {
   if (M <= 64 || N % BN || K % (2 * BK)) return 0;
   const Route route = route_of(M, N, K, FLS_EPI_RESID, false, ws_bytes);
