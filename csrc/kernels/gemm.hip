@@ -931,6 +931,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
   if (route == ROUTE_SPLIT) route = ROUTE_NONE;
   if (mid_ok && (!main_ok || route == ROUTE_MID ||
                  (route == ROUTE_NONE && g_mid && mid_rule(M, tiles256)))) {
+    bool kv_written = false;
     switch (mid_form(M, N, K, pairs, bn64_ok)) {
       case MID_16:
         if constexpr (!pairs) {
@@ -940,19 +941,18 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
         }
         break;
       case MID_16X2:
+        kv_written = is_rope(EPI) && ep.kv_dst != nullptr;
         if constexpr (pairs) {
           if (stat) {
             if (M <= 16) launch_col16<EPI, 1, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
             else launch_col16<EPI, 2, 2, true>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-            FLS_CHECK_LAUNCH();
-            return ep.kv_dst != nullptr;
+            break;
           }
         }
         if (M <= 16) launch_col16<EPI, 1, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else if (M <= 32) launch_col16<EPI, 2, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         else launch_col16<EPI, 4, 2>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
-        FLS_CHECK_LAUNCH();
-        return is_rope(EPI) && ep.kv_dst != nullptr;
+        break;
       case MID_32:
         if constexpr (!pairs) launch_mid<EPI, mid::NSTAGE, 32, 8>(A, W, C, M, N, K, lda, ldw, ldc, ep, s);
         break;
@@ -972,7 +972,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     FLS_CHECK_LAUNCH();
     ss_partials(C, ldc, M, N, ep, s);
     FLS_CHECK_LAUNCH();
-    return 0;
+    return kv_written;
   }
   if (!main_ok) {
     dim3 grid((M + 31) / 32, (N + 255) / 256);

@@ -1411,3 +1411,23 @@ def test_residual_statistic_from_partials_or_rows(ops, M, N, K):
     assert torch.equal(a, b)
     assert torch.equal(ops.rstd_from_ss(ss, N, 1e-5), ops.row_stat(b, 1e-5))
     assert ops.leaves_ss(M, N, K) == (M == 4100 or (M == 1000 and N == 4096))      # (the tiles' epilogue leaves them)
+
+
+# the same of blocks of two panels (wide products of up to 64 rows, chosen and forced), partials that were not there before, and of a chunk of
+# many rows with a tail of few: what the MLP of a capped plan leaves for the next layer's norm
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 32, 33, 64, 3088])
+@pytest.mark.parametrize("N,K", [(8192, 1024), (8192, 8192), (5120, 13824)])
+def test_residual_statistic_of_two_panels(ops, M, N, K):
+    g = torch.Generator().manual_seed(M + N)
+    x, w, r = ((torch.randn(*s, generator=g) * f).half().to(DEV) for s, f in (((M, K), 1.0), ((N, K), K ** -0.5), ((M, N), 1.0)))
+    for bn in (0, 33):
+        old = ops.k.fls_gemm_set_mid_bn(bn)
+        try:
+            for exact in (False, True):
+                ss, y = torch.full((M, N // 128), float("nan"), device=DEV), r.clone()
+                with ops.row_exact(exact):
+                    for s in range(0, M, 3072):
+                        ops.linear_residual(x[s:s + 3072], w, y[s:s + 3072], ss=ss[s:s + 3072])
+                assert torch.equal(ops.rstd_from_ss(ss, N, 1e-5), ops.row_stat(y, 1e-5)), (bn, exact)
+        finally:
+            ops.k.fls_gemm_set_mid_bn(old)
