@@ -864,7 +864,10 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
   return best;
 }
 
-// -> 0; 1 where the product has also written the K/V rows (Epi::kv_dst)
+// what launch returns where the product has also written the K/V rows (Epi::kv_dst): no error code of HIP's
+constexpr int KV_WRITTEN = 1 << 24;
+
+// -> 0, KV_WRITTEN, or an error
 template <int EPI>
 int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int lda, int ldw, int ldc,
            const Epi& ep, hipStream_t s, void* ws, size_t ws_bytes, Route route) {
@@ -972,7 +975,7 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
     FLS_CHECK_LAUNCH();
     ss_partials(C, ldc, M, N, ep, s);
     FLS_CHECK_LAUNCH();
-    return kv_written;
+    return kv_written ? KV_WRITTEN : 0;
   }
   if (!main_ok) {
     dim3 grid((M + 31) / 32, (N + 255) / 256);
@@ -1131,7 +1134,7 @@ struct KvOut {
   const int* dst;
   int col0, ld;
 };
-// fls_gemm; 1 where the product has also written the K/V rows
+// fls_gemm; KV_WRITTEN where the product has also written the K/V rows
 int gemm_entry(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldw,
                int ldc, int ldr, int epi, const int* pos, const float* cos_t, const float* sin_t,
                int rope_cols, int head_dim, const void* bias, const float* rscale, float rs_eps, float alpha, float* ss,
@@ -1212,6 +1215,6 @@ extern "C" int fls_gemm_kv(const void* A, const void* W, void* C, int M, int N, 
   const KvOut out = {(half_t*)kv, (half_t* const*)kv_at, kv_dst, kv_col0, kv_ld};
   const int rc = gemm_entry(A, W, C, C, M, N, K, lda, ldw, ldc, ldc, epi, pos, cos_t, sin_t, rope_cols, head_dim, bias, rscale, rs_eps, 1.f, nullptr, 0, &out, ws,
                             ws_bytes, s);
-  if (rc) return rc > 0 ? 0 : rc;
+  if (rc) return rc == KV_WRITTEN ? 0 : rc;
   return fls_copy_rows((const half_t*)C + kv_col0, ldc, nullptr, kv, kv_ld, kv_at, kv_dst, M, N - kv_col0, s);
 }

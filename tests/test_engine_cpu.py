@@ -985,6 +985,22 @@ def test_activation_store_buffer_bound():
     st.trim()
 
 
+@pytest.mark.skipif(torch.cuda.is_available(), reason="without a device, so that no launch can start")
+@pytest.mark.parametrize("M,K", [(4, 256), (4, 4096), (48, 256), (100, 4096)])
+def test_gemm_kv_reports_failed_launches(M, K):
+    """A RoPE product that also writes K/V rows returns its launches' errors (blocks of 16 pairs, other few-row blocks, tiles), as one without them does."""
+    from flexible_llm_sharding_amd import _native
+    try:
+        k = _native.kernels()
+    except Exception as e:  # noqa: BLE001 (library not built in this checkout)
+        pytest.skip(f"kernel library unavailable: {e}")
+    p = (np.zeros(1 << 10, np.uint8).ctypes.data + 15) // 16 * 16
+    N, rope, rs_eps = 1280, 3, 0.0
+    plain = k.fls_gemm(p, p, p, p, M, N, K, K, K, N, N, rope, p, p, p, 1152, 128, None, None, rs_eps, 1.0, None, 0, None, 0, None)
+    kv = k.fls_gemm_kv(p, p, p, M, N, K, K, K, N, rope, p, p, p, 1152, 128, None, None, rs_eps, p, None, p, 1024, 256, None, 0, None)
+    assert plain > 0 and kv == plain
+
+
 def test_gemm_v11_round_rule():
     """The GEMM launcher's v10 / v11 choice (csrc/kernels/gemm_v11.hip v11_pays, a host-side rule):
     whole 256-CU tile rounds of each kernel, a 384 x 256 tile priced at 1.45 256 x 256 tiles
