@@ -43,9 +43,10 @@ int fls_seq_moe_sum_add_group_rmsnorm(float* x, int ldx, const float* y, int ldy
 int fls_seq_moe_sum_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const int* dest, const float* mw, int top, const float* w,
                                            float woff, const float* w2, float woff2, void* h, int th, int ldh, int rows, int D, int groups,
                                            float eps, fls_stream_t s);
-// x += norm(y; w + woff), then h = norm(x; w2 + woff2) of the new x, both per group of D / groups columns; h of type th
+// x += norm(y; w + woff), then h = norm(x; w2 + woff2) of the new x, both per group of D / groups columns; h of type th; in_turn: with the bits of
+// fls_seq_group_rmsnorm called for the one and then for the other
 int fls_seq_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const float* w, float woff, const float* w2, float woff2,
-                                   void* h, int th, int ldh, int rows, int D, int groups, float eps, fls_stream_t s);
+                                   void* h, int th, int ldh, int rows, int D, int groups, float eps, int in_turn, fls_stream_t s);
 // new = (keep ? x : 0) + coef (rms(a) wa + rms(b) wb) + f (all fp32 rows; a and b nullable together, f nullable), x <- new;
 // h != null: h = rms(new) hw as type th, hw a vector or (hw_one) one number
 int fls_seq_residual_branches(float* x, int ldx, int keep, const float* a, int lda, const float* wa, const float* b,

@@ -32,11 +32,14 @@ __global__ __launch_bounds__(256) void group_rmsnorm_kernel(const float* __restr
 // post-norm, the residual update and the next sublayer's norm in one pass.  Bound by its bytes from some hundred rows on
 // and by a launch and two memory latencies below.  16384 rows of 4096 in two groups, a column a thread before: norm 146 -> 82 us,
 // residual update 199 -> 140, update and next norm in turn 345, here 182.  SUM: x is a mixture's rows, sorted by expert; row r of the sum is
-// sum_k mw[r, k] x[idx[r, k]], k < top, made on the way in (moe_sum_kernel's order).  MODE 2 rounds as MODE 1 and then MODE 0 do, so that a layer's last
-// update gives the same bits with the next layer's norm and without it (16,384 rows of 4096 in three layers 16.42 -> 16.28 ms, a captured step of 8 rows
-// of 2048, three launches fewer, 258 -> 253 us).
-// (its fused steps spelt out: the same rounding in every kernel)
-__device__ __forceinline__ float squares(const float4& v) { return fmaf(v.w, v.w, fmaf(v.z, v.z, fmaf(v.y, v.y, v.x * v.x))); }
+// sum_k mw[r, k] x[idx[r, k]], k < top, made on the way in (moe_sum_kernel's order).  MODE 3: as MODE 2, rounded as MODE 1 and then MODE 0, so that a
+// layer's last update gives the same bits with the next layer's norm and without it (16,384 rows of 4096 in three layers 16.42 -> 16.28 ms, a captured
+// step of 8 rows of 2048, three launches fewer, 258 -> 253 us).  MODE 2's rounding, of the update and norm within a layer, is its own.
+// (The fused steps of the sums are spelt out, so that no compiler's choice moves them: the second square first but in MODE 2 of up to 1,024 columns.)
+template <bool X_FIRST>
+__device__ __forceinline__ float squares(const float4& v) {
+  return fmaf(v.w, v.w, fmaf(v.z, v.z, X_FIRST ? fmaf(v.y, v.y, v.x * v.x) : fmaf(v.x, v.x, v.y * v.y)));
+}
 
 template <typename TO, int MODE, int NV, bool SUM = false>
 __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, const int* __restrict__ idx,
@@ -44,6 +47,7 @@ __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __r
                                                                 float eps, float woff, int w_one, const float* __restrict__ w2,
                                                                 TO* __restrict__ h, int ldh, float woff2,
                                                                 const float* __restrict__ mw, int top) {
+  constexpr bool NEXT = MODE >= 2, X_FIRST = MODE == 2 && NV == 1;
   __shared__ float red[8];
   const int r = blockIdx.x, g = blockIdx.y;
   const float* xr = x + (size_t)(!SUM && idx != nullptr ? idx[r] : r) * ldx + (size_t)g * n;
@@ -77,9 +81,9 @@ __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __r
       if constexpr (!SUM) v[i] = *reinterpret_cast<const float4*>(xr + c);
       if constexpr (MODE != 0) u[i] = *reinterpret_cast<const float4*>(yr + c);
       if (!w_one) a[i] = *reinterpret_cast<const float4*>(wg + c);
-      if constexpr (MODE == 2) b[i] = *reinterpret_cast<const float4*>(w2 + (size_t)g * n + c);
+      if constexpr (NEXT) b[i] = *reinterpret_cast<const float4*>(w2 + (size_t)g * n + c);
     }
-    ss += squares(v[i]);
+    ss += squares<X_FIRST>(v[i]);
   }
   const float rs = 1.f / sqrtf(block_sum_256(ss, red) / (float)n + eps);
   float s2 = 0.f;
@@ -87,19 +91,22 @@ __global__ __launch_bounds__(256) void group_rmsnorm_vec_kernel(const float* __r
   for (int i = 0; i < NV; ++i) {
     v[i].x = u[i].x + v[i].x * rs * (a[i].x + woff); v[i].y = u[i].y + v[i].y * rs * (a[i].y + woff);
     v[i].z = u[i].z + v[i].z * rs * (a[i].z + woff); v[i].w = u[i].w + v[i].w * rs * (a[i].w + woff);
-    if constexpr (MODE == 2) s2 += squares(v[i]);
+    if constexpr (NEXT) s2 += squares<X_FIRST>(v[i]);
   }
   float rs2 = 0.f;
-  if constexpr (MODE == 2) rs2 = 1.f / sqrtf(block_sum_256(s2, red + 4) / (float)n + eps);
+  if constexpr (NEXT) rs2 = 1.f / sqrtf(block_sum_256(s2, red + 4) / (float)n + eps);
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int c = (threadIdx.x + 256 * i) * 4;
     if (c >= n) continue;
     if constexpr (MODE != 0) *reinterpret_cast<float4*>(yr + c) = v[i];
     if constexpr (MODE != 1) {
-      TO* hr = MODE == 2 ? h + (size_t)r * ldh + (size_t)g * n : reinterpret_cast<TO*>(y) + (size_t)r * ldy + (size_t)g * n;
+      TO* hr = NEXT ? h + (size_t)r * ldh + (size_t)g * n : reinterpret_cast<TO*>(y) + (size_t)r * ldy + (size_t)g * n;
       float4 o = v[i];
       if constexpr (MODE == 2) {
+        o.x *= rs2 * (b[i].x + woff2); o.y *= rs2 * (b[i].y + woff2); o.z *= rs2 * (b[i].z + woff2); o.w *= rs2 * (b[i].w + woff2);
+      }
+      if constexpr (MODE == 3) {
         o.x = o.x * rs2 * (b[i].x + woff2); o.y = o.y * rs2 * (b[i].y + woff2);
         o.z = o.z * rs2 * (b[i].z + woff2); o.w = o.w * rs2 * (b[i].w + woff2);
       }
@@ -167,8 +174,8 @@ extern "C" int fls_seq_moe_sum_add_group_rmsnorm_next(float* x, int ldx, const f
   if (rows <= 0) return 0;
   if (groups < 1 || D % groups || top < 1) return -1;
   hipStream_t st = (hipStream_t)s;
-  if (!(th == 1 ? group_rmsnorm_vec<bf16_t, 2, true>(y, ldy, dest, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (bf16_t*)h, ldh, woff2, st, mw, top)
-                : group_rmsnorm_vec<float, 2, true>(y, ldy, dest, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (float*)h, ldh, woff2, st, mw, top)))
+  if (!(th == 1 ? group_rmsnorm_vec<bf16_t, 3, true>(y, ldy, dest, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (bf16_t*)h, ldh, woff2, st, mw, top)
+                : group_rmsnorm_vec<float, 3, true>(y, ldy, dest, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (float*)h, ldh, woff2, st, mw, top)))
     return SEQ_NOT_SERVED;
   SEQ_LAUNCH_CHECK();
   return 0;
@@ -176,15 +183,16 @@ extern "C" int fls_seq_moe_sum_add_group_rmsnorm_next(float* x, int ldx, const f
 
 extern "C" int fls_seq_add_group_rmsnorm_next(float* x, int ldx, const float* y, int ldy, const float* w, float woff, const float* w2,
                                               float woff2, void* h, int th, int ldh, int rows, int D, int groups, float eps,
-                                              fls_stream_t s) {
+                                              int in_turn, fls_stream_t s) {
   if (rows <= 0) return 0;
   if (groups < 1 || D % groups) return -1;
   hipStream_t st = (hipStream_t)s;
-  if (th == 1 ? group_rmsnorm_vec<bf16_t, 2>(y, ldy, nullptr, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (bf16_t*)h, ldh, woff2, st)
-              : group_rmsnorm_vec<float, 2>(y, ldy, nullptr, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (float*)h, ldh, woff2, st)) {
+#define GN_NEXT(TO, MODE) group_rmsnorm_vec<TO, MODE>(y, ldy, nullptr, w, x, ldx, rows, D, groups, eps, woff, 0, w2, (TO*)h, ldh, woff2, st)
+  if (in_turn ? (th == 1 ? GN_NEXT(bf16_t, 3) : GN_NEXT(float, 3)) : (th == 1 ? GN_NEXT(bf16_t, 2) : GN_NEXT(float, 2))) {
     SEQ_LAUNCH_CHECK();
     return 0;
   }
+#undef GN_NEXT
   const int rc = fls_seq_group_rmsnorm(y, ldy, nullptr, w, x, 0, ldx, rows, D, groups, eps, 1, woff, 0, s);
   return rc ? rc : fls_seq_group_rmsnorm(x, ldx, nullptr, w2, h, th, ldh, rows, D, groups, eps, 0, woff2, 0, s);
 }
@@ -1228,4 +1236,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 23; }
+extern "C" int fls_seq_version(void) { return 24; }

@@ -177,7 +177,7 @@ def _load_kernels(path: str = _KERNELS):
     return _Quick(lib)
 
 
-SEQ_ABI = 23   # csrc/include/fls_seq.h
+SEQ_ABI = 24   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -191,7 +191,7 @@ def _load_seq():
     _bind(lib, "fls_seq_gemm_tile_of", i, i, i, i, i, i, i, i, i)
     _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm", i, p, i, p, i, p, p, i, p, f, i, i, i, f, p)
     _bind(lib, "fls_seq_moe_sum_add_group_rmsnorm_next", i, p, i, p, i, p, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
-    _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, p)
+    _bind(lib, "fls_seq_add_group_rmsnorm_next", i, p, i, p, i, p, f, p, f, p, i, i, i, i, i, f, i, p)
     _bind(lib, "fls_seq_group_rmsnorm", i, p, i, p, p, p, i, i, i, i, i, f, i, f, i, p)
     _bind(lib, "fls_seq_residual_branches", i, p, i, i, p, i, p, p, i, p, f, p, i, p, i, i, p, i, i, i, f, p)
     _bind(lib, "fls_seq_block_means", i, p, i, p, i, i, p, p, i, i, i, i, p, i, i, i, p, i, p, i, p, i, p)

@@ -237,7 +237,7 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
         if nw is None:
             ops.add_group_rmsnorm_(x, y, W["norm1b"], ng, eps)
         else:
-            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], nw, ng, eps, out_dtype=cdt)
+            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], nw, ng, eps, out_dtype=cdt, in_turn=True)
     else:
         h = ops.add_group_rmsnorm_next_(x, y, W["norm1b"], W["norm2"], ng, eps, out_dtype=cdt)
         if L.mlp["kind"] == "dense":
@@ -252,7 +252,7 @@ def run_block(ctx, W, x: torch.Tensor, meta: dict, name: str) -> torch.Tensor:
         if nw is None:
             ops.add_group_rmsnorm_(x, y, W["norm2b"], ng, eps)
         else:
-            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm2b"], nw, ng, eps, out_dtype=cdt)
+            ctx.normed = ops.add_group_rmsnorm_next_(x, y, W["norm2b"], nw, ng, eps, out_dtype=cdt, in_turn=True)
     return x
 
 

@@ -127,7 +127,7 @@ class HipSeqOps:
              "fls_seq_group_rmsnorm")
         return x
 
-    def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype):
+    def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype, in_turn=False):
         _rows(x, "x", torch.float32)
         _rows(y, "y", torch.float32)
         if x.shape != y.shape:
@@ -137,7 +137,7 @@ class HipSeqOps:
         h = torch.empty(x.shape, dtype=out_dtype, device=x.device)
         _chk(self.k.fls_seq_add_group_rmsnorm_next(x.data_ptr(), x.stride(0), y.data_ptr(), y.stride(0), w.data_ptr(), 0.0, w2.data_ptr(),
                                                    0.0, h.data_ptr(), _CODE[out_dtype], h.stride(0), x.shape[0], x.shape[1], groups,
-                                                   float(eps), _stream()), "fls_seq_add_group_rmsnorm_next")
+                                                   float(eps), 1 if in_turn else 0, _stream()), "fls_seq_add_group_rmsnorm_next")
         return h
 
     def residual_branches_(self, x, branches=None, coef=1.0, add=None, keep=True, eps=0.0, norm_w=None, out_dtype=torch.float32):

@@ -69,8 +69,9 @@ class TorchSeqOps:
         self.add_group_rmsnorm_moe_(x, y, route, w, groups, eps)
         return self.group_rmsnorm(x, w2, groups, eps, out_dtype)
 
-    def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype):
-        """``add_group_rmsnorm_`` and the norm of the new rows by ``w2``, which it returns."""
+    def add_group_rmsnorm_next_(self, x, y, w, w2, groups, eps, out_dtype, in_turn=False):
+        """``add_group_rmsnorm_`` and the norm of the new rows by ``w2``, which it returns; ``in_turn``: with the bits of the two steps (here
+        always)."""
         self.add_group_rmsnorm_(x, y, w, groups, eps)
         return self.group_rmsnorm(x, w2, groups, eps, out_dtype)
 

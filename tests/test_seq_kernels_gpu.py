@@ -1987,6 +1987,41 @@ def test_side_by_side_rows(ops, cdt, tol, D):
         close(xa, xb, 1e-5)
 
 
+# the rounding of group norms, step for step: rows whose values lie in one thread's four columns, so that nothing but them is summed.  The
+# second square comes first, but in an update and norm in one pass of up to 1,024 columns; that pass multiplies scale and weight first, the two
+# steps in turn the row and its scale
+@pytest.mark.parametrize("D", [4, 1024, 1028, 4096, 8192])
+@pytest.mark.parametrize("form", ["norm", "add", "next", "in turn"])
+def test_group_norm_rounding(ops, D, form):
+    H, _ = ops
+    f32 = np.float32
+    fma = lambda a, b, c: f32(np.longdouble(a) * np.longdouble(b) + np.longdouble(c))
+    rng = np.random.default_rng(D)
+    T, eps = 200, f32(1e-6)
+    x, y = np.zeros((T, D), f32), np.zeros((T, D), f32)
+    x[:, :4], y[:, :4] = rng.standard_normal((2, T, 4))
+    w, w2 = rng.standard_normal((2, D)).astype(f32)
+    x_first = form == "next" and D <= 1024
+
+    def scale(v):                                  # 1 / rms of rows of four values
+        sq = lambda i: (v[:, i] * v[:, i]).astype(f32)
+        ss = fma(v[:, 1], v[:, 1], sq(0)) if x_first else fma(v[:, 0], v[:, 0], sq(1))
+        ss = fma(v[:, 3], v[:, 3], fma(v[:, 2], v[:, 2], ss))
+        return (f32(1) / np.sqrt(ss / f32(D) + eps))[:, None]
+    dev = lambda a: torch.from_numpy(a.copy()).to(DEV)
+    new = fma(y[:, :4] * scale(y[:, :4]), w[None, :4], x[:, :4])
+    xd = dev(x)
+    if form == "norm":
+        assert np.array_equal(H.group_rmsnorm(dev(y), dev(w), 1, float(eps), torch.float32).cpu().numpy()[:, :4], y[:, :4] * scale(y[:, :4]) * w[:4])
+        return
+    if form == "add":
+        H.add_group_rmsnorm_(xd, dev(y), dev(w), 1, float(eps))
+    else:
+        h = H.add_group_rmsnorm_next_(xd, dev(y), dev(w), dev(w2), 1, float(eps), torch.float32, in_turn=form == "in turn").cpu().numpy()[:, :4]
+        assert np.array_equal(h, new * scale(new) * w2[:4] if form == "in turn" else new * (scale(new) * w2[:4]))
+    assert np.array_equal(xd.cpu().numpy()[:, :4], new)
+
+
 # a layer's last update with the next layer's norms in its pass: the bits of the two steps in turn, for widths about the pieces of 1,024 columns, the
 # widest that rows in registers take, and widths and alignments that only the two steps serve
 @pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
@@ -2018,7 +2053,7 @@ def test_update_with_the_next_norms(ops, cdt, D, pad):
         g = H.add_group_rmsnorm_moe_next_(xa[:, :D], y, route, w1, n1, groups, 1e-6, cdt)
         H.add_group_rmsnorm_moe_(xb[:, :D], y, route, w1, groups, 1e-6)
         assert torch.equal(xa, xb) and torch.equal(g, H.group_rmsnorm(xb[:, :D], n1, groups, 1e-6, cdt))
-        g = H.add_group_rmsnorm_next_(xa[:, :D], a, w1, n1, groups, 1e-6, cdt)
+        g = H.add_group_rmsnorm_next_(xa[:, :D], a, w1, n1, groups, 1e-6, cdt, in_turn=True)
         H.add_group_rmsnorm_(xb[:, :D], a, w1, groups, 1e-6)
         assert torch.equal(xa, xb) and torch.equal(g, H.group_rmsnorm(xb[:, :D], n1, groups, 1e-6, cdt))
 
