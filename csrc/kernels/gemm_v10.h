@@ -48,13 +48,6 @@ struct Epi {
   // rsqrt(mean(x^2) + eps) of a GEMM that reads the un-normalised hidden state x with the norm
   // weight folded into W (fused RMSNorm + projection); applied before the bias
   const float* rs = nullptr;
-  // RoPE products of 16-pair blocks (fls_gemm_kv): row m's columns from kv_col0 on into row kv_dst[m] of a K/V buffer too (kv, or what lies at kv_at)
-  half_t* kv = nullptr;
-  half_t* const* kv_at = nullptr;
-  const int* kv_dst = nullptr;
-  int kv_col0 = 0, kv_ld = 0;
-  // > 0: the 16-pair blocks make that statistic themselves, of the rows of A (and rs is not read)
-  float rs_eps = 0.f;
   // scale of (product + bias) before the residual add (Granite's residual_multiplier)
   float alpha = 1.f;
   // optional (RESID): per-row partial sums of squares of the fp16 output, one fp32 per 128 output
@@ -65,6 +58,13 @@ struct Epi {
   // FLS_GEMM_ROW_EXACT: only the row-independent paths (v10 / v11 / mid-M tiles, or the generic kernel
   // for shapes they do not take): every output row gets the same arithmetic whatever M and the other rows
   int row_exact = 0;
+  // RoPE products of 16-pair blocks (fls_gemm_kv): row m's columns from kv_col0 on into row kv_dst[m] of a K/V buffer too (kv, or what lies at kv_at)
+  half_t* kv = nullptr;
+  half_t* const* kv_at = nullptr;
+  const int* kv_dst = nullptr;
+  int kv_col0 = 0, kv_ld = 0;
+  // > 0: the 16-pair blocks make that statistic themselves, of the rows of A (and rs is not read)
+  float rs_eps = 0.f;
 };
 
 // sum of v over the 4 lanes of one output row (lanes l, l^16, l^32, l^48: one 16-column group
