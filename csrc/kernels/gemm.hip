@@ -726,8 +726,8 @@ bool two_panels(int M, int N, int K, bool pairs) {
   if (!pairs && M <= 32 && K >= 2560 && b <= 768) return true;
   return M <= 16 && K >= 1024 && (b <= 512 || (K >= 1280 && b <= 768) || (b > 1024 && (pairs || K >= 2048)));
 }
-// pairs: an epilogue that joins columns (SwiGLU, RoPE).  K % 128 == 0
-MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
+// pairs: an epilogue that joins columns (SwiGLU, RoPE).  panels: two-panel blocks among them.  K % 128 == 0
+MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok, bool panels = true) {
   // 64-column blocks for a single row tile whose 128-column grid fills less than one round of the
   // 256 CUs: 70B generation steps with 8 prompts (M = 40) 39.7 vs 46.7 ms per step; with 32 prompts
   // (M = 160, three row tiles) the 128-column blocks are faster, 53 vs 55.5 ms (profiles/r6_decode/
@@ -752,7 +752,7 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
                     (g_mid_bn == 32 || (g_mid_bn == 0 && M <= mid::BMm && blocks64 < 256));
   // 16-column ones where 32-column ones leave CUs idle too (g_mid_bn: a forced width keeps the mid blocks)
   const bool few = M <= mid::BMm && K % 256 == 0 && g_mid_waves != 4;
-  if (few && (g_mid_bn == 33 || (g_mid_bn == 16 && pairs) || (g_mid_bn == 0 && two_panels(M, N, K, pairs)))) return MID_16X2;
+  if (panels && few && (g_mid_bn == 33 || (g_mid_bn == 16 && pairs) || (g_mid_bn == 0 && two_panels(M, N, K, pairs)))) return MID_16X2;
   if (few && !pairs && (g_mid_bn == 16 || (bn32 && g_mid_bn == 0 && N / 32 < 256))) return MID_16;
   if (bn32) return MID_32;
   if (bn64) return w8_64 ? MID_64 : MID_64_W4;
@@ -769,15 +769,14 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok) {
 struct MidCost { float start, k_few, k_full, start2, k2, k2_more, tb; };       // tb: bytes of weight a us, in millions
 const MidCost MID_16_COST[3] = {{4.7f, 0.05f, 0.152f, 7.4f, 0.199f, 0.f, 4.76f}, {5.f, 0.092f, 0.165f, 7.8f, 0.247f, 0.f, 4.97f},
                                 {4.7f, 0.147f, 0.207f, 6.8f, 0.33f, 0.f, 4.99f}};        // up to 16, 32 and 64 rows
-// (two panels; their starts 2 us up: they were timed launch to launch in a graph)
-const MidCost MID_16X2_COST[3] = {{4.7f, 0.111f, 0.17f, 6.2f, 0.3f, 0.08f, 5.5f}, {4.7f, 0.125f, 0.197f, 6.2f, 0.33f, 0.08f, 5.2f},
-                                  {4.7f, 0.185f, 0.27f, 6.f, 0.27f, 0.13f, 5.2f}};
+// (two panels: of 2,600 random products launch to launch in a graph, so that only SKINNY_COST's last compares with them; 5% off)
+const MidCost MID_16X2_COST[3] = {{2.9f, 0.112f, 0.147f, 3.7f, 0.273f, 0.277f, 5.63f}, {3.f, 0.123f, 0.183f, 5.6f, 0.301f, 0.048f, 5.23f},
+                                  {2.7f, 0.177f, 0.242f, 4.f, 0.27f, 0.13f, 5.2f}};
 const MidCost MID_32_COST = {4.4f, 0.269f, 0.337f, 6.f, 0.415f, 0.f, 4.2f};
 const MidCost MID_64_COST[2] = {{4.8f, 0.279f, 0.452f, 6.7f, 0.658f, 0.f, 4.8f}, {4.9f, 0.288f, 0.366f, 5.9f, 0.524f, 0.f, 5.f}};      // up to 64, 128 rows
 const MidCost MID_128_COST[2] = {{7.f, 0.38f, 0.543f, 8.9f, 0.833f, 0.173f, 5.6f}, {5.5f, 0.387f, 0.476f, 7.8f, 0.65f, 0.235f, 5.f}};
 const MidCost MID_128R_COST = {-14.f, 0.514f, 0.7f, 18.f, 0.6f, 0.3f, 3.8f};
-float mid_us(int M, int N, int K, bool pairs) {
-  const MidForm form = mid_form(M, N, K, pairs, true);
+float mid_us(int M, int N, int K, MidForm form) {
   const int tiles_m = (M + 63) / 64;
   const float nk = (float)(K / BK), bytes = (float)N * K * 2.f;
   const MidCost& c = form == MID_16 || form == MID_16X2 ? (form == MID_16 ? MID_16_COST : MID_16X2_COST)[M <= 16 ? 0 : M <= 32 ? 1 : 2]
@@ -788,7 +787,9 @@ float mid_us(int M, int N, int K, bool pairs) {
   const float rounds = (float)((form == MID_128R ? (M + 127) / 128 : tiles_m) * (N / width)) / 256.f;
   if (form == MID_128_W4) return (4.f + 0.532f * nk) * powf(rounds, 0.842f);
   if (rounds <= 1.f) return c.start + fmaxf(bytes / (c.tb * 1e6f), (c.k_few + (c.k_full - c.k_few) * rounds) * nk);
-  return c.start2 + fmaxf(bytes / (c.tb * 1e6f), (c.k2 + c.k2_more * (rounds - 1.f)) * nk);
+  // (two blocks of two panels share a CU: up to two rounds some CUs have both and take as long as all with both)
+  const float more = form == MID_16X2 ? fmaxf(rounds - 2.f, 0.f) : rounds - 1.f;
+  return c.start2 + fmaxf(bytes / (c.tb * 1e6f), (c.k2 + c.k2_more * more) * nk);
 }
 
 // Tiles of `rows` x 256: whole rounds of 256 blocks and a last one.  A weight that one or two row tiles read comes from memory and not from
@@ -813,12 +814,12 @@ float split_us(int M, int N, int K, int S) {
   const float tiles = (float)(blocks / 256) * full + (fill > 0.f ? part + (full - part) * powf(fill, 0.349f) : 0.f);
   return 12.2f + fmaxf((float)N * K * 2.f / 4.04e6f, tiles) + S * ((float)M * N * 1.314e-6f + 0.094f);
 }
-// K-split blocks of all rows (gemm_skinny.h): up to 64 rows, more without a split, more
+// K-split blocks of all rows (gemm_skinny.h): up to 64 rows, more without a split, more; up to 64 beside blocks of two panels, timed as those
 struct SkinnyCost { float start, tb, k, k_rows, k_fill, over, slab, slice, sum; };
-const SkinnyCost SKINNY_COST[3] = {{4.9f, 4.48f, 0.2f, 0.1115f, 0.408f, 1.097f, 2.19f, 0.41f, 2.4f}, {7.f, 4.94f, -0.15f, 0.167f, 0.785f, 1.f, 0.f, 0.f, 0.f},
-                                   {0.f, 4.55f, 0.194f, 0.0955f, 0.231f, 1.167f, 1.73f, 0.17f, 9.5f}};
-float skinny_us(int M, int N, int K, int bn, int S) {
-  const SkinnyCost& c = SKINNY_COST[M <= 64 ? 0 : S == 1 ? 1 : 2];
+const SkinnyCost SKINNY_COST[4] = {{4.9f, 4.48f, 0.2f, 0.1115f, 0.408f, 1.097f, 2.19f, 0.41f, 2.4f}, {7.f, 4.94f, -0.15f, 0.167f, 0.785f, 1.f, 0.f, 0.f, 0.f},
+                                   {0.f, 4.55f, 0.194f, 0.0955f, 0.231f, 1.167f, 1.73f, 0.17f, 9.5f}, {2.3f, 5.81f, 0.246f, 0.09f, 0.262f, 1.174f, 1.73f, 0.49f, 1.7f}};
+float skinny_us(int M, int N, int K, int bn, int S, bool beside_panels = false) {
+  const SkinnyCost& c = SKINNY_COST[beside_panels ? 3 : M <= 64 ? 0 : S == 1 ? 1 : 2];
   const float rounds = (float)(N / bn) * S / 256.f;
   const float k = (c.k + c.k_rows * ((M + 31) / 32) + c.k_fill * fminf(rounds, 1.f)) * powf(fmaxf(rounds, 1.f), c.over);
   return c.start + fmaxf((float)N * K * 2.f / (c.tb * 1e6f), k * (float)(K / BK) / S) +
@@ -856,16 +857,17 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
       least = us;
     }
   };
-  // (no lead for blocks of two panels, which those rules have not been measured with: M <= 16, K above 6,000 on up to 100 of them 1.1 to 1.16 of the skinny path's.
-  // Above 16 rows and 4,096 terms the skinny path's blocks, the rules' choice there, are estimated up to 20% worse than they are: by the bare estimates plain products
-  // of 4,352 .. 14,336 columns took up to 1.22 of their time before there were two panels, 20% of them more than 1.04; so 0.99, 10% and 1.05 (1.3: up to 1.09)
-  const bool panels = M <= 64 && two_panels(M, N, K, pairs);
-  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, pairs) * (!panels ? 1.f : rules == ROUTE_MID ? 1.f / 0.94f : !pairs && M > 16 && K > 4096 ? 1.4f : 1.f));
+  if (g_mid) offer(ROUTE_MID, mid_us(M, N, K, mid_form(M, N, K, pairs, true, false)));
   if (skinny) offer(ROUTE_SKINNY, skinny_us(M, N, K, bn, S));
   if (split) offer(ROUTE_SPLIT, split_us(M, N, K, S2));
   if (M > 64) {              // (up to 64 rows one row tile covers them all, and three quarters of a 256-row one are padding)
     for (int i = 0; i < 3; ++i) offer((Route)(ROUTE_128 + i), rounds_us(ROUNDS[i], M, N, K));
     if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], M, N, K));
+  } else if (best == ROUTE_SKINNY && mid_form(M, N, K, pairs, true) == MID_16X2 &&
+             1.04f * mid_us(M, N, K, MID_16X2) < skinny_us(M, N, K, bn, S, true)) {
+    // Two panels take what the mid blocks would, and of the K-split blocks' products those that they are estimated 4% faster for.  2,600 random ones of up to
+    // 64 rows, against the time before there were two panels: 0.896, 6 of them more than 5% slower (no margin: 0.894, 32; each on the faster of the two: 0.890)
+    best = ROUTE_MID;
   }
   return best;
 }
