@@ -398,7 +398,9 @@ class HipSeqOps:
     PLACE_SELF, PLACE_SELF_EXPERTS = 2048, 16
 
     def _route_ints(self, E, n, dev, fused=False):
-        """-> (row offsets per expert, address of the zeroed counts or None, of the zeroed cursors or None) of n entries."""
+        """-> (row offsets per expert, address of the zeroed counts or None, of the zeroed cursors or None) of n entries (of none nothing is launched: zeros)."""
+        if n == 0:
+            return torch.zeros(E + 1, dtype=torch.int32, device=dev), None, None
         if fused or (n <= self.PLACE_SELF and E <= self.PLACE_SELF_EXPERTS):
             return torch.empty(E + 1, dtype=torch.int32, device=dev), None, None
         ints = torch.zeros(3 * E + 1, dtype=torch.int32, device=dev)          # offs | hist | cursor

@@ -1472,6 +1472,19 @@ def test_placement_counts_itself(ops, T, top, E):
         assert torch.equal(r.rows.long().cpu()[dest], torch.arange(T).repeat_interleave(top))
 
 
+# no tokens: no rows of any expert, whatever the memory held
+@pytest.mark.parametrize("E", [8, 40])
+def test_routes_of_no_tokens(ops, E):
+    H, _ = ops
+    logits = torch.randn(0, E, device=DEV)
+    for route in (lambda: H.moe_route_softmax_grouped(logits, None, 2, 0, 0, 1.0), lambda: H.moe_route_grouped(logits, 2, 0, 0, 1.0),
+                  lambda: H.moe_route_corrected(logits, torch.zeros(E, device=DEV), 2), lambda: H.moe_route_corrected(logits, None, 2)):
+        junk = torch.full((E + 1,), 7, dtype=torch.int32, device=DEV)
+        del junk
+        r = route()
+        assert r.offs.shape == (E + 1,) and not bool(r.offs.any()) and r.dest.shape == (0, 2) and r.rows.numel() == 0
+
+
 # gathered rows by 16 bytes and by elements: the same bytes, for widths about a block's threads, column slices and rows that vectors do not fit
 @pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("D", [8, 36, 512, 520, 1032, 2056, 4])
