@@ -223,17 +223,17 @@ __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ 
       float vm = ld(v[0]);
 #pragma unroll
       for (int j = 1; j < 8; ++j) vm = fmaxf(vm, ld(v[j]));
-      const float nm = fmaxf(m, vm);
-      s *= __expf(m - nm);
+      const float nm = fmaxf(m, vm), base = nm == -INFINITY ? 0.f : nm;       // (nothing but -inf so far: zeros)
+      s *= __expf(m - base);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) s += __expf(ld(v[j]) - nm);
+      for (int j = 0; j < 8; ++j) s += __expf(ld(v[j]) - base);
       m = nm;
     }
   } else {
     for (int c = threadIdx.x; c < V; c += NT) {
       const float v = ld(lr[c]);
-      const float nm = fmaxf(m, v);
-      s = s * __expf(m - nm) + __expf(v - nm);
+      const float nm = fmaxf(m, v), base = nm == -INFINITY ? 0.f : nm;
+      s = s * __expf(m - base) + __expf(v - base);
       m = nm;
     }
   }

@@ -1375,6 +1375,22 @@ def test_softmax_greedy(ops, V, scaling):
     assert torch.equal(host[:10 * V].view(torch.int16), want.cpu().view(torch.int16).flatten()) and torch.equal(host[at:].view(torch.int32), greedy.cpu())
 
 
+# logits of -inf, before and behind the others and all but one: zeros, and the others' probabilities; widths of each form (one block of either size, by eights and
+# singly; in registers; wider than slices).  Tolerance as below
+@pytest.mark.parametrize("V", [7, 8, 1000, 2048, 4095, 4096, 8193, 32003, 65544, 1048584])
+def test_softmax_of_minus_infinities(ops, V):
+    x = (torch.randn(4, V, generator=torch.Generator().manual_seed(V)) * 4).half()
+    x[0, :V // 2] = float("-inf")
+    x[1, V // 3:] = float("-inf")
+    x[2] = float("-inf")
+    x[2, V - 2] = -3.0
+    for scaling in (1.0, 8.0):
+        probs, greedy, _ = ops.softmax_greedy(x.to(DEV), scaling)
+        want = torch.softmax((x.float() * (1.0 / scaling)).half().double(), -1)
+        assert bool(((probs.cpu().double() - want).abs() <= want * (2.0 ** -11 + 1e-5) + 2.0 ** -25).all())
+        assert np.array_equal(greedy.cpu().numpy(), np.argmax(probs.cpu().numpy(), axis=-1))
+
+
 # rows in registers, in one block and cut over several (their limits, few rows and many, the widest and one that is wider): probabilities
 # against fp64 (half a step of fp16, 2^-11, and 1e-5 for the hardware's exponential, or half the smallest step), the greedy token and the bits without it; ties across
 # slices, a slice of -inf, NaN
@@ -1385,7 +1401,7 @@ def test_softmax_wide_rows(ops, V, rows):
     x = (torch.randn(rows, V, generator=torch.Generator().manual_seed(V)) * 4).round().div(2).half()
     x[1] = 0.25
     x[1, V // 2] = x[1, V - 3] = 9.0
-    x[2, :V // 2] = float("-inf") if V <= 1 << 20 else -60000.0        # (one block of any width: NaN where a thread begins with eight of them)
+    x[2, :V // 2] = float("-inf")
     x[3, V // 3] = float("nan")
     x = x.to(DEV)
     for scaling in (1.0, 8.0):
