@@ -111,6 +111,8 @@ int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc, int ldk, 
                        const float* gate_bias, float out_scale, int page_size, int nsplit, float* part,
                        int has_sink, float sink, const float* sink_h, const float* head_gate, int ldhg, int Gv,
                        int pool_P, const void* kp, int ldkp, const void* vp, int ldvp, const int* block_table, int bt_stride, fls_stream_t s);
+// its nsplit for rows of up to `bound` keys: what fills the chip with the blocks that these pools get
+int fls_seq_attn_ranges(const void* kc, int ldk, const void* vc, int ldv, int tc, int T, int H, int d, int dv, int pool_P, int bound);
 // the same attention on the matrix cores for bf16 pools and rows in tiles: tiles[n_tiles][2] = (first packed
 // row, rows <= 128) of one request each, covering every row of the step; q of type tq.  -2: shape not
 // served (use the above)

@@ -437,6 +437,26 @@ int seq_attn_merge(const float* part, void* out, int tc, int ldo, int T, int H, 
   return 0;
 }
 
+// lanes (a power of two, as an exponent) that share a row of values, four columns each; -1: not so many columns or not so aligned
+static int value_lanes(const void* vc, int ldv, int es, int dv) {
+  if ((uintptr_t)vc % (4 * es) || ldv % 4) return -1;
+  return dv == 32 ? 3 : dv == 64 ? 4 : dv == 128 ? 5 : dv == 256 ? 6 : -1;
+}
+static bool keys_by_16(const void* kc, int ldk, int es, int d) { return d * es % 16 == 0 && (uintptr_t)kc % 16 == 0 && ldk * es % 16 == 0; }
+// Sixteen waves a (row, head) and range of its keys?  One block a CU (a second one waits: 384 and 512 blocks 1.0 to 1.4 of the other kernel's time) and keys
+// of 256 bytes or more (128 bytes are two loads a lane here and eight there: 0.9 to 1.2)
+static bool few_rows(const void* kc, int ldk, const void* vc, int ldv, int es, int d, int dv, int pool_P, long long blocks) {
+  return pool_P == 0 && blocks <= 256 && d * es >= 256 && keys_by_16(kc, ldk, es, d) && value_lanes(vc, ldv, es, dv) >= 0;
+}
+
+// Ranges of keys for rows of up to `bound` keys: of 256 keys or more, so many that the launch has a block a CU of sixteen waves, or two of four
+extern "C" int fls_seq_attn_ranges(const void* kc, int ldk, const void* vc, int ldv, int tc, int T, int H, int d, int dv, int pool_P, int bound) {
+  const long long rows = (long long)T * H;
+  if (rows < 1) return 1;
+  const long long n = (few_rows(kc, ldk, vc, ldv, tc == 1 ? 2 : 4, d, dv, pool_P, rows) ? 256 : 512) / rows;
+  return max(1, min(min(8, (int)n), pool_P == 0 ? bound / 256 : (bound + 255) / 256));
+}
+
 // tq: type of q; tc: type of the pools; to: type of out (fp32 over bf16 pools allowed)
 extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc, int ldk, const void* vc, int ldv, int tc,
                                   void* out, int to, int ldo, const int* tok_seq, const int* tok_pos, const int* page_table,
@@ -458,13 +478,10 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   const AttnBlocks ab = {pool_P, kp, ldkp, vp, ldvp, block_table, bt_stride};
   dim3 grid(H, T, nsplit);
   hipStream_t st = (hipStream_t)s;
-  // lanes (a power of two, as an exponent) that share a row of values, four columns each; -1: not so many columns or not so aligned
   const int es = tc == 1 ? 2 : 4;
-  const bool by4 = (uintptr_t)vc % (4 * es) == 0 && ldv % 4 == 0 && (pool_P == 0 || ((uintptr_t)vp % (4 * es) == 0 && ldvp % 4 == 0));
-  const int vsh = !by4 ? -1 : dv == 32 ? 3 : dv == 64 ? 4 : dv == 128 ? 5 : dv == 256 ? 6 : -1;
-  // One block a CU (a second one waits: 384 and 512 blocks 1.0 to 1.4 of the other kernel's time) and keys of 256 bytes or more (128 bytes are two loads
-  // a lane here and eight there: 0.9 to 1.2)
-  const bool few_ok = vsh >= 0 && pool_P == 0 && (long long)T * H * nsplit <= 256 && d * es >= 256;
+  const int vsh = pool_P == 0 || value_lanes(vp, ldvp, es, dv) >= 0 ? value_lanes(vc, ldv, es, dv) : -1;
+  const int vec = keys_by_16(kc, ldk, es, d) && (pool_P == 0 || keys_by_16(kp, ldkp, es, d));
+  const bool few = few_rows(kc, ldk, vc, ldv, es, d, dv, pool_P, (long long)T * H * nsplit);
 #define ATTN_PAGED_ARGS ldq, (const TC*)kc, ldk, (const TC*)vc, ldv, (TOUT*)out, ldo, tok_seq, tok_pos, page_table, pt_stride, H, G, \
                         d, dv, scale, softcap, r1, r2, chunk, window, keep_first, gate_bias, out_scale, page_size, vec, vsh, part, has_sink, sink, sink_h, \
                         nsplit > 1 ? nullptr : head_gate, ldhg, Gv, ab
@@ -486,8 +503,6 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   } while (0)
   if (tc == 1) {
     using TC = bf16_t;
-    const int vec = d % 8 == 0 && (uintptr_t)kc % 16 == 0 && ldk % 8 == 0 && (pool_P == 0 || ((uintptr_t)kp % 16 == 0 && ldkp % 8 == 0));
-    const bool few = few_ok && vec;
     if (to == 0) {
       using TOUT = float;
       if (tq == 1) ATTN_PAGED_GO(bf16_t);
@@ -500,8 +515,6 @@ extern "C" int fls_seq_attn_paged(const void* q, int ldq, int tq, const void* kc
   } else {
     using TC = float;
     using TOUT = float;
-    const int vec = d % 4 == 0 && (uintptr_t)kc % 16 == 0 && ldk % 4 == 0 && (pool_P == 0 || ((uintptr_t)kp % 16 == 0 && ldkp % 4 == 0));
-    const bool few = few_ok && vec;
     ATTN_PAGED_GO(float);
   }
 #undef ATTN_PAGED_GO

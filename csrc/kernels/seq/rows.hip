@@ -1236,4 +1236,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 24; }
+extern "C" int fls_seq_version(void) { return 25; }

@@ -177,7 +177,7 @@ def _load_kernels(path: str = _KERNELS):
     return _Quick(lib)
 
 
-SEQ_ABI = 24   # csrc/include/fls_seq.h
+SEQ_ABI = 25   # csrc/include/fls_seq.h
 
 
 def _load_seq():
@@ -211,6 +211,7 @@ def _load_seq():
     _bind(lib, "fls_seq_argmax", i, p, i, i, i, p, p, i, p)
     _bind(lib, "fls_seq_copy_words", i, p, p, i, p)
     _bind(lib, "fls_seq_kv_store", i, p, i, p, f, p, i, p, p, i, p, i, i, i, p)
+    _bind(lib, "fls_seq_attn_ranges", i, p, i, p, i, i, i, i, i, i, i, i)
     _bind(lib, "fls_seq_attn_paged", i, p, i, i, p, i, p, i, i, p, i, i, p, p, p, i, i, i, i, i, i, f, f, p, p, i, i, i, p, f, i, i, p,
           i, f, p, p, i, i, i, p, i, p, i, p, i, p)
     _bind(lib, "fls_seq_attn_prefill", i, p, i, i, p, i, p, i, p, i, i, p, i, p, p, p, i, i, i, i, i, f, f, p, p, i, i, i, p, f, i,

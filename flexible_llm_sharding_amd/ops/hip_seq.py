@@ -854,9 +854,7 @@ class HipSeqOps:
                 _chk(rc, "fls_seq_attn_heads")
         # few rows over many keys (decoding a small batch): cut every row's keys into ranges that run as
         # blocks of their own, so that the launch has a few hundred blocks
-        # (blocks of sixteen waves, one a CU, where the kernel takes them: see attn_few_kernel)
-        few = T * H <= 256 and d * kcache.element_size() >= 256 and d % 8 == 0 and dv in (32, 64, 128, 256) and blocks is None
-        nsplit = max(1, min(8, (256 if few else 512) // max(1, T * H), bound // 256 if blocks is None else -(-bound // 256)))
+        nsplit = self.k.fls_seq_attn_ranges(kcache.data_ptr(), ldk, vcache.data_ptr(), ldv, _code(kcache, "kcache"), T, H, d, dv, blk[0], bound)
         part = torch.empty(T * H * nsplit * (dv + 4), dtype=torch.float32, device=q.device) if nsplit > 1 else None
         _chk(self.k.fls_seq_attn_paged(q.data_ptr(), q.stride(0), _code(q, "q"), kcache.data_ptr(), ldk, vcache.data_ptr(), ldv,
                                        _code(kcache, "kcache"), out.data_ptr(), to, out.stride(0), meta["tok_seq"].data_ptr(),

@@ -1001,6 +1001,25 @@ def test_gemm_kv_reports_failed_launches(M, K):
     assert plain > 0 and kv == plain
 
 
+@pytest.mark.parametrize("tc,d,dv", [(1, 128, 128), (0, 64, 32), (0, 128, 256), (1, 256, 64)])
+def test_paged_attention_key_ranges(tc, d, dv):
+    """Ranges of keys a row (a host-side rule of csrc/kernels/seq/attn_paged.hip): a block a CU where the sixteen-wave blocks take the pools, two where they
+    do not (keys or values not so aligned or wide, blocks), none below 256 keys each."""
+    from flexible_llm_sharding_amd import _native
+    try:
+        k = _native.seq_kernels()
+    except Exception as e:  # noqa: BLE001 (library not built in this checkout)
+        pytest.skip(f"kernel library unavailable: {e}")
+    es, G = 2 if tc else 4, 4
+    ranges = lambda T, H, kc=1 << 12, ldk=G * d, vc=1 << 12, ldv=G * dv, bound=1 << 14, dd=d, ddv=dv, pool=0: \
+        k.fls_seq_attn_ranges(kc, ldk, vc, ldv, tc, T, H, dd, ddv, pool, bound)
+    assert [ranges(T, 16) for T in (1, 2, 4, 8, 16, 17)] == [8, 8, 4, 2, 1, 1]
+    for other in (dict(kc=(1 << 12) + 8), dict(ldk=G * d + 8 // es), dict(vc=(1 << 12) + es), dict(ldv=G * dv + 1), dict(ddv=dv + 1), dict(dd=256 // es - 16 // es), dict(pool=16)):
+        assert [ranges(T, 16, **other) for T in (1, 4, 8, 16, 32, 33)] == [8, 8, 4, 2, 1, 1], other
+    assert [ranges(1, 16, bound=n) for n in (1, 255, 512, 1000, 1 << 20)] == [1, 1, 2, 3, 8]
+    assert [ranges(1, 16, bound=n, pool=16) for n in (1, 257, 512)] == [1, 2, 2] and ranges(0, 16) == 1
+
+
 def test_gemm_v11_round_rule():
     """The GEMM launcher's v10 / v11 choice (csrc/kernels/gemm_v11.hip v11_pays, a host-side rule):
     whole 256-CU tile rounds of each kernel, a 384 x 256 tile priced at 1.45 256 x 256 tiles
