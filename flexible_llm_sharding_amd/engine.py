@@ -546,19 +546,18 @@ class ShardedRunner:
             self.seq_cache.release(rid)
         return out
 
-    def _in_turn(self, names, W):
-        """The layers ``names``, which run one behind the other on the same rows, each with the one ahead of it in a hybrid model's context."""
-        if not self.hybrid:
-            for name in names:
-                yield name
-            return
-        self.ctx.normed = None
+    def _run_in_turn(self, names, W, state, batch, meta):
+        """The layers ``names``, which run one behind the other on the same rows, each with the one ahead of it in a hybrid model's context -> the last one's output."""
+        ctx = self.ctx
         try:
-            for name, nxt in zip(names, list(names[1:]) + [None]):
-                self.ctx.ahead = (nxt, W[nxt]) if nxt is not None else None
-                yield name
+            for i, name in enumerate(names):
+                if self.hybrid:
+                    ctx.ahead = (names[i + 1], W[names[i + 1]]) if i + 1 < len(names) else None
+                state = self._run_layer(ctx, name, W[name], state, batch, meta)
         finally:
-            self.ctx.ahead = self.ctx.normed = None
+            if self.hybrid:
+                ctx.ahead = ctx.normed = None
+        return state
 
     def _step_graphable(self, entries) -> bool:
         """A decode step (one token per request) on resident weights on one GPU: it replays as one
@@ -574,9 +573,7 @@ class ShardedRunner:
                 self._W_all.update(self.prefetcher.acquire(k))
         if self._decode_graphs is None:
             def forward(meta):
-                state = None
-                for name in self._in_turn(self.names, self._W_all):
-                    state = self._run_layer(self.ctx, name, self._W_all[name], state, None, meta)
+                state = self._run_in_turn(self.names, self._W_all, None, None, meta)
                 return state, self.ops.argmax_f32(state, meta["mirror"])
             self._decode_graphs = StepGraphs(self.dev, forward, self.ops, self.cfg.vocab_size)
         batch = pack_step(entries, self.seq_cache)
@@ -874,10 +871,12 @@ class ShardedRunner:
         last_use = idx + 1 >= len(px.items) or px.items[idx + 1][0] != k
         tc = time.perf_counter()
         with trace.range(f"shard{k}:mb{b}:compute"):
-            for name in self._in_turn([self.names[li] for li in self.my_shards[k]], px.W):
+            names = [self.names[li] for li in self.my_shards[k]]
+            for name in names:
                 if hasattr(px.W[name], "final_use"):
                     px.W[name].final_use = last_use
-                state = self._run_layer(self.ctx, name, px.W[name], state, batch, meta)
+            state = self._run_in_turn(names, px.W, state, batch, meta)
+            for name in names:
                 if self.hybrid:
                     if layer_kind(name) == "decoder":
                         px.flops += self.family.layer_flops(self.cfg, name, batch.num_tokens)

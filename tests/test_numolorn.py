@@ -445,6 +445,48 @@ def test_few_layers_per_shard_stream_weights(tmp_path, device, lnps):
 
 
 @pytest.mark.parametrize("device", DEVICES)
+def test_shards_give_the_bits_of_one(tmp_path, device):
+    """All layers in one shard (each leaves the next one's norms), a few a shard and one a shard: the same logits, prompts, portions and decode steps."""
+    cfg = nu.config(STACK, loop=LOOP, width=64)
+    path = nu.write_model(str(tmp_path / "s"), cfg, nu.random_weights(cfg, 15))
+    toks = nu.tokens(44, cfg["vocab"], 5)
+    got = []
+    for lnps in (None, 3, 2, 1):
+        runner = load_runner(path, torch.float32, device, max_tokens=64, layer_num_per_shard=lnps)
+        got.append(run_cut(runner, "r", toks, [23, 3, 14]))
+        runner.close()
+    for g in got[1:]:
+        assert np.array_equal(g, got[0])
+
+
+def test_a_failed_pass_leaves_the_next_one_alone(tmp_path):
+    """A pass that an error ends in mid-stack, whose traceback lives on and is let go while a later pass runs: that one's logits are what they are without."""
+    cfg, _, runner, _ = build(tmp_path, STACK, 16, loop=LOOP, max_seqs=3)
+    toks = nu.tokens(20, cfg["vocab"], 6)
+    want = run_cut(runner, "a", toks, [20])
+    inner, held, names = runner._run_layer, [], runner.cfg.layer_names()
+    at = next(i for i, n in enumerate(names) if n.split("@")[0] != n) - 1          # the first layer of a looped layer's second pass comes next
+
+    def layer(ctx, name, W, state, batch, meta):
+        if fail and name == names[at]:
+            raise RuntimeError("planted")
+        out = inner(ctx, name, W, state, batch, meta)
+        if name == names[at]:
+            held.clear()
+        return out
+    runner._run_layer, fail = layer, True
+    try:
+        runner.step([StepEntry("b", toks, range(20))])
+    except RuntimeError as e:
+        held.append(e)
+    assert held
+    fail = False
+    got = runner.step([StepEntry("c", toks, range(20))], ["c"])[0][0]
+    assert not held and np.array_equal(got, want)
+    runner.close()
+
+
+@pytest.mark.parametrize("device", DEVICES)
 def test_bf16_products_stay_close(tmp_path, device):
     """(Every expert is chosen, so that rounding cannot flip a choice.)"""
     f = nu.moe(experts=3, identity=1, top=4, groups=(2, 2))
