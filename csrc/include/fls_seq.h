@@ -215,8 +215,7 @@ int fls_seq_moe_route_grouped(const float* logits, int ldl, int T, int E, int to
 int fls_seq_moe_route_softmax_grouped(const float* logits, int ldl, const float* corr, int T, int E, int top, int groups, int keep,
                                       float scale, int* ids, float* w, int* hist, int* offs, int* dest, int* rows, fls_stream_t s);
 // offs[E+1] = exclusive scan of hist; dest[t, k] = a row in its expert's range; rows[dest] = t (cursor[E]: zeros from the caller).
-// hist null (up to FLS_SEQ_PLACE_SELF entries; cursor is not read): the launch counts for itself, and the routes above need no hist either
-#define FLS_SEQ_PLACE_SELF 2048
+// hist null (cursor is not read): every block of the launch counts all entries for itself, and the routes above need no hist either
 int fls_seq_moe_place(const int* ids, int n, int top, const int* hist, int E, int* offs, int* cursor, int* dest, int* rows, fls_stream_t s);
 // out[t] = sum_k w[t, k] y[dest[t, k]] (fp32, k in order)
 int fls_seq_moe_sum(const float* y, int ldy, const int* dest, const float* w, float* out, int ldo, int T, int top,

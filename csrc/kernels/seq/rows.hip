@@ -1185,7 +1185,6 @@ extern "C" int fls_seq_moe_place(const int* ids, int n, int top, const int* hist
   if (E < 1 || E > MOE_MAX_E) return -1;
   const dim3 blocks((n + PLACE_THREADS - 1) / PLACE_THREADS);
   if (hist == nullptr) {
-    if (n > FLS_SEQ_PLACE_SELF) return -1;
     hipLaunchKernelGGL((moe_place_kernel<true>), blocks, dim3(PLACE_THREADS), 0, (hipStream_t)s, ids, n, top, hist, E, offs, cursor, dest, rows);
   } else {
     hipLaunchKernelGGL((moe_place_kernel<false>), blocks, dim3(PLACE_THREADS), 0, (hipStream_t)s, ids, n, top, hist, E, offs, cursor, dest, rows);
@@ -1236,4 +1235,4 @@ extern "C" int fls_seq_moe_combine(float* x, int ldx, const float* y, int ldy, c
   return 0;
 }
 
-extern "C" int fls_seq_version(void) { return 25; }
+extern "C" int fls_seq_version(void) { return 26; }

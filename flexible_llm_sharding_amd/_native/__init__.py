@@ -177,7 +177,7 @@ def _load_kernels(path: str = _KERNELS):
     return _Quick(lib)
 
 
-SEQ_ABI = 25   # csrc/include/fls_seq.h
+SEQ_ABI = 26   # csrc/include/fls_seq.h
 
 
 def _load_seq():

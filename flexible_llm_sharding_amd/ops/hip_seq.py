@@ -393,8 +393,8 @@ class HipSeqOps:
         # every head's output over its own root mean square, times the weight the heads share
         return self.head_norm_rope(raw, heads, vdim, 0, vdim, out, 0, vdim, meta, w=norm_w, eps=eps)
 
-    # Up to so many entries (the limit in csrc/include/fls_seq.h) of so many experts their placement counts them itself: us of the whole route in a
-    # graph, with the launch that zeroes the counts and so, 8 experts: 130 entries 8.7, 7.1; 1,024 9.4, 7.9; 2,048 9.7, 9.1; 4,096 10.6, 11.6; 1,600 of 128 18.8, 25.7
+    # Up to so many entries of so many experts their placement counts them itself: us of the whole route in a graph, with the launch that zeroes
+    # the counts and so, 8 experts: 130 entries 8.7, 7.1; 1,024 9.4, 7.9; 2,048 9.7, 9.1; 4,096 10.6, 11.6; 1,600 of 128 18.8, 25.7
     PLACE_SELF, PLACE_SELF_EXPERTS = 2048, 16
 
     def _route_ints(self, E, n, dev, fused=False):
