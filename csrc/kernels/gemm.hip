@@ -168,7 +168,7 @@ namespace mid {
 constexpr int BMm = 64, BNm = 128, BKm = 64, NTm = 256, NSTAGE = 3;
 // BNT: output columns per block, 128 (4 waves in 2 x 2, each 32 x 64) or 64 (each 32 x 32: twice the
 // blocks for grids of less than one round of 128-column tiles); 32 with 8 waves (below)
-// A rows 0 .. bmt-1 then W rows; LDS-DMA in 8-row (1 KiB) groups
+// A rows 0 .. bmt-1 then W rows; LDS-DMA in groups of 1 KiB: 8 rows, of K-tiles of 128 terms 4
 constexpr int stage_bytes(int bnt, int bmt = BMm, int bk = BKm) { return (bmt + bnt) * bk * 2; }
 }  // namespace mid
 
@@ -290,7 +290,7 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
       __builtin_amdgcn_s_barrier();                        // every wave's part of tile kt landed; tile kt - 1 has been read
       asm volatile("" ::: "memory");
     }
-    // into the stage tile kt - 1 used (every wave passed that tile's closing barrier)
+    // into the stage tile kt - 1 used (every wave passed the barrier behind its reads: the one above, or that tile's closing one)
     stage(kt + NST - 1, min(kt + NST - 1, nk - 1));
     // tile kt landed
     if constexpr (!ONE) {
@@ -351,15 +351,17 @@ __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict_
   }
 }
 
-// Blocks of 16 columns (the O / down projections of a 7B-sized generation step, N = 4,096, 128 mid blocks
-// of 32), or of two panels of 16 (neighbours, or pairs: a RoPE column and its partner, a gate and its up column), for M <= 64: what bounds the wider ones is the bytes in flight, one
-// block's ring on half the CUs, with 64 rows of A staged whatever M is.  Here a block streams 16 or 32 weight rows, K-tiles of 256 or 128 (two or four
-// rows a DMA instruction, XOR chunk swizzle on the source), a ring of NST stages with one barrier a K-tile, of two panels two blocks a CU; only ceil(M / 16) row
-// tiles of A are staged, wave w multiplies row tile w, the others only move data.  Same fragments, MFMA and K order as
-// the mid blocks: bitwise equal rows.  M = 16, K = 4,096 and 11,008 in turn (124 MB in both): 35.8 -> 16.6 us on average, 13 at
-// the rate of a large copy.  Pairs, M = 16 (us, 64-column mid blocks and these): 22,016 x 4,096 42.5, 35.2; 12,288 x 4,096 26.1, 25.3; 6,144 x 4,096
-// 22.5, 14.9; 5,120 x 2,048 12.7, 7.6; M = 64 23.9, 19.7 and 13.8, 11.4.  Two panels, plain, 16 rows (32-column mid blocks
-// before): 8,192 x 8,192 45.1, 33.1; 8,192 x 28,672 147, 88.  (A ring for W and a shorter one for A, loaded by waves of their own: 1.5 to 2 us slower.)
+// Blocks of 16 columns (the O / down projections of a 7B-sized generation step, N = 4,096: 128 mid blocks of 32 columns), or of two panels
+// of 16 (neighbours, or pairs: a RoPE column and its partner, a gate and its up column), for M <= 64.  What bounds the wider mid blocks there is the
+// bytes in flight: one block's ring on half of the CUs, with 64 rows of A staged whatever M is.
+// Here a block streams 16 or 32 weight rows in K-tiles of 256 or 128 (two or four rows a DMA instruction, XOR chunk swizzle on the source) through
+// a ring of NST stages with one barrier a K-tile; of two panels a CU has two blocks.  Only ceil(M / 16) row tiles of A are staged, wave w multiplies
+// row tile w, the others only move data.  Same fragments, MFMA and K order as the mid blocks: bitwise equal rows.
+// One panel, M = 16, K = 4,096 and 11,008 in turn (124 MB in both): 35.8 -> 16.6 us on average, 13 at the rate of a large copy.
+// Pairs (us, 64-column mid blocks and these), M = 16: 22,016 x 4,096 42.5, 35.2; 12,288 x 4,096 26.1, 25.3; 6,144 x 4,096 22.5, 14.9;
+// 5,120 x 2,048 12.7, 7.6; M = 64, the last two: 23.9, 19.7 and 13.8, 11.4.
+// Two panels, plain, 16 rows (32-column mid blocks before): 8,192 x 8,192 45.1, 33.1; 8,192 x 28,672 147, 88.
+// (A ring for W and a shorter one for A, loaded by waves of their own: 1.5 to 2 us slower.)
 namespace col16 {
 constexpr int kt(int rt, int np) { return np == 2 && rt > 1 ? 128 : 256; }
 constexpr int stage_bytes(int rt, int np) { return 16 * (np + rt) * kt(rt, np) * 2; }
@@ -378,7 +380,7 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
                                                    int ldc, Epi ep) {
   constexpr int KT = col16::kt(RT, NP), NST = col16::stages(RT, NP), STAGE = col16::stage_bytes(RT, NP);
   constexpr int LPR = KT / 8, RPD = 64 / LPR, GP = 16 / RPD;               // lanes a row, rows a DMA group of 1 KB, groups a panel of 16 rows
-  constexpr int PER_WAVE = GP * (NP + RT) / 4;           // 1 KB DMA groups (two rows) of a stage, per wave
+  constexpr int PER_WAVE = GP * (NP + RT) / 4;           // DMA groups of a stage, per wave
   extern __shared__ __attribute__((aligned(16))) char lds_c16[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int fr = lane & 15, grp = lane >> 4;
@@ -387,7 +389,7 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   const int n0 = EPI == FLS_EPI_ROPE ? (b >> 2) * 128 + (b & 3) * 16 : EPI == EPI_ROPE64 ? (b >> 1) * 64 + (b & 1) * 16
                  : b * (EPI == FLS_EPI_SWIGLU ? 16 : 16 * NP);
   const int second = EPI == FLS_EPI_ROPE ? 64 : EPI == EPI_ROPE64 ? 32 : EPI == FLS_EPI_SWIGLU ? ep.gu_rows : 16;
-  const half_t* src[PER_WAVE];                         // groups 0 .. 7: W rows, then A rows
+  const half_t* src[PER_WAVE];                         // groups 0 .. GP NP - 1: W rows, panel by panel, then A rows
 #pragma unroll
   for (int i = 0; i < PER_WAVE; ++i) {
     const int g = wave + 4 * i, row = g % GP * RPD + lane / LPR;           // row inside its panel

@@ -313,7 +313,8 @@ class ShardedRunner:
 
     # ------------------------------------------------------------- main
     def __call__(self, prompts) -> List[np.ndarray]:
-        """Reference API: list of (prefix, suffixes) -> list of [n_s, 1, V] fp16 arrays."""
+        """Reference API: list of (prefix, suffixes) -> list of [n_s, 1, V] fp16 arrays (the caller's own, but on a GPU views of one pinned block a
+        micro-batch: an array kept keeps the block, at most hostmem.ResultBlocks.MOST of them; copy what is to stay for long)."""
         if self.my_shards and prompts and not self.resume_dir and not self.hip_graphs:
             # the first shards' weights do not depend on the prompts: their H2D overlaps tokenization
             if self._h2d0 is None:
@@ -511,7 +512,7 @@ class ShardedRunner:
         """One serving step of a hybrid stack: every entry's next tokens run through all shards from
         the state earlier steps left (``self.seq_cache``); requests named in ``end`` give their pages
         and slots back afterwards.  -> per entry (logits [len(want), vocab] fp32, their argmax) or
-        None when it wants nothing.  Entries are cut into micro-batches of whole requests under the
+        None when it wants nothing (logits: the caller's own, views of pinned blocks as a scoring call's).  Entries are cut into micro-batches of whole requests under the
         token budget and scheduled over the shards like a scoring call's micro-batches.  No row's result
         contains another request's; how its sums are split (the products' tiles by the micro-batch's rows,
         recurrences row by row or in chunks by its longest request) follows the micro-batch, so with other
