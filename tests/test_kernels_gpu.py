@@ -1394,10 +1394,10 @@ def test_softmax_of_minus_infinities(ops, V):
 # rows in registers, in one block and cut over several (their limits, few rows and many, the widest and one that is wider): probabilities
 # against fp64 (half a step of fp16, 2^-11, and 1e-5 for the hardware's exponential, or half the smallest step), the greedy token and the bits without it; ties across
 # slices, a slice of -inf, NaN
-@pytest.mark.parametrize("V", [4104, 32768, 32776, 65536, 65544, 131080, 151936, 1048576, 1048584])
-@pytest.mark.parametrize("rows", [4, 70])
+@pytest.mark.parametrize("V", [4104, 8192, 8200, 32768, 32776, 65536, 65544, 131080, 151936, 1048576, 1048584])
+@pytest.mark.parametrize("rows", [4, 70, 420])
 def test_softmax_wide_rows(ops, V, rows):
-    rows = min(rows, 4 + (1 << 23) // V)
+    rows = min(rows, 4 + (1 << (25 if rows == 420 else 23)) // V)
     x = (torch.randn(rows, V, generator=torch.Generator().manual_seed(V)) * 4).round().div(2).half()
     x[1] = 0.25
     x[1, V // 2] = x[1, V - 3] = 9.0
