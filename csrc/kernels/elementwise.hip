@@ -269,12 +269,12 @@ __global__ __launch_bounds__(NT) void softmax_kernel(const half_t* __restrict__ 
   }
 }
 
-// The same with the row in registers, NC times eight values a thread (rows of up to 32,768 in eights): all of its loads in flight at once and none a second time,
-// one exponential a value for the sum instead of the running maximum's rescaling too, and the greedy token as the first value with the largest one's
-// bits.  16 rows of 32,000 with greedy tokens 12.3 -> 7.3 us, one of 8,192 6.3 -> 4.6.  (Up to 8,192 columns eight values a thread: of more each thread loads the row's end
-// again, 48 rows of 4,096 3.81 us in the kernel above, 4.01 of 32, 3.78 of eight.)
-// PASS 1 and 2: wider rows, bound by what one CU computes, cut over gridDim.x blocks of slices: each slice's maximum and sum to `part`, then the
-// probabilities: one row of 65,544 19.8 -> 6.7 us, of 151,936 39.2 -> 6.9; 48 43.6 -> 14.2, 120 47.0 -> 24.2.
+// The same with the row in registers, NC times eight values a thread (rows of up to 32,768 in eights): all of its loads in flight at once
+// and none a second time, one exponential a value for the sum instead of the running maximum's rescaling too, and the greedy token as the
+// first value with the largest one's bits.  16 rows of 32,000 with greedy tokens 12.3 -> 7.3 us, one of 8,192 6.3 -> 4.6.  (Up to 8,192
+// columns eight values a thread: of more each thread loads the row's end again, 48 rows of 4,096 3.81 us in the kernel above, 4.01 of 32,
+// 3.78 of eight.) PASS 1 and 2: wider rows, bound by what one CU computes, cut over gridDim.x blocks of slices: each slice's maximum and
+// sum to `part`, then the probabilities: one row of 65,544 19.8 -> 6.7 us, of 151,936 39.2 -> 6.9; 48 43.6 -> 14.2, 120 47.0 -> 24.2.
 template <int NT, int NC, bool GREEDY, int PASS>
 __global__ __launch_bounds__(NT) void softmax_regs_kernel(const half_t* __restrict__ logits, half_t* __restrict__ probs,
                                                         int V, float inv_scale, int* __restrict__ greedy, float2* __restrict__ part) {
@@ -603,8 +603,9 @@ extern "C" int fls_softmax_rows(const void* logits, void* probs, int rows, int V
   } else if (regs && V <= 32768) {
     SOFTMAX_REGS(1024, 4, 0, dim3(rows));
   } else if (regs && part != nullptr && V <= 64 * 16384 && rows <= 65535) {
-    // slices of up to 16,384 values, or of fewer where the rows would leave CUs idle.  (400 rows and more of up to 65,536 are faster in a block each
-    // where no greedy tokens are wanted, 1,000 x 50,304 46.3 us for 55.3, but not with them, 56.3 for 55.4, 400 27.2 for 29.8; and the two are to give the same bits.)
+    // slices of up to 16,384 values, or of fewer where the rows would leave CUs idle.  (400 rows and more of up to 65,536 are faster in a
+    // block each where no greedy tokens are wanted, 1,000 x 50,304 46.3 us for 55.3, but not with them, 56.3 for 55.4, 400 27.2 for 29.8;
+    // and the two are to give the same bits.)
     const int nz = std::max((V + 16383) / 16384, std::min(std::min(256 / rows, V / 4096), 64));
     SOFTMAX_REGS(256, 8, 1, dim3(nz, rows));
     SOFTMAX_REGS(256, 8, 2, dim3(nz, rows));

@@ -193,12 +193,13 @@ constexpr int stage_bytes(int bnt, int bmt = BMm, int bk = BKm) { return (bmt + 
 //              155 -> 139 us (profiles/r6_decode/mid8/bn32_*).
 // Same fragments, MFMA and K order in every shape, so all are bitwise equal.
 //
-// BNT = 64 and 128, WV = 8: K-tiles of BK = 128 (64 where K is no multiple of it), one barrier a K-tile: after it tile kt - 1 has been read, so that its stage takes
-// the tile NST - 1 ahead.  What bounds these grids of one row tile is the chain of one K-tile in few blocks a CU: M = 24, 50 and 64 (us, with K-tiles of 64 and
-// two barriers, and so) 12,288 x 4,096 27.9, 29.2, 28.2 -> 24.3, 27.1, 26.0; 10,240 x 8,192 49.2, 51.1, 52.1 -> 42.8, 46.9, 49.4 with three stages (one
-// block a CU); 22,016 x 4,096 43.4, 47.5, 49.6 -> 43.2, 46.3, 48.2 with two stages (two blocks; 47.6, 49.5, 51.0 with three).
-// So BNT = 128 up to a round of blocks and from 2,048 terms on (1,024: 1.03 of the time): M = 65, 128 x 12,288 x 4,096 30.7, 35.2 -> 28.9, 33.3; 150, 256 x 4,096
-// x 11,008 71.6, 79.0 -> 66.8, 72.8; 192 x 8,192 x 4,096 31.1 -> 29.8.
+// BNT = 64 and 128, WV = 8: K-tiles of BK = 128 (64 where K is no multiple of it), one barrier a K-tile: after it tile kt - 1 has been
+// read, so that its stage takes the tile NST - 1 ahead.  What bounds these grids of one row tile is the chain of one K-tile in few blocks
+// a CU: M = 24, 50 and 64 (us, with K-tiles of 64 and two barriers, and so) 12,288 x 4,096 27.9, 29.2, 28.2 -> 24.3, 27.1, 26.0; 10,240 x
+// 8,192 49.2, 51.1, 52.1 -> 42.8, 46.9, 49.4 with three stages (one block a CU); 22,016 x 4,096 43.4, 47.5, 49.6 -> 43.2, 46.3, 48.2 with
+// two stages (two blocks; 47.6, 49.5, 51.0 with three). So BNT = 128 up to a round of blocks and from 2,048 terms on (1,024: 1.03 of the
+// time): M = 65, 128 x 12,288 x 4,096 30.7, 35.2 -> 28.9, 33.3; 150, 256 x 4,096 x 11,008 71.6, 79.0 -> 66.8, 72.8; 192 x 8,192 x 4,096
+// 31.1 -> 29.8.
 template <int EPI, int NST, int BNT, int WV = 4, int BMT = mid::BMm, int BK = 64>
 __global__ __launch_bounds__(64 * WV) void gemm_nt_mid(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                      half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
@@ -369,11 +370,12 @@ constexpr int stages(int rt, int np) { return np == 2 ? (rt == 2 ? 5 : 3) : rt =
 }  // namespace col16
 
 //
-// STAT (up to 32 rows): the row statistic that the epilogue applies is made here, from the rows of A that pass through LDS anyway, by the waves that only move
-// data (a wave for each part of 128 columns of a K-tile), in row_stat_kernel's order (same bits): a lane has one row's column group, its parts
-// stay in registers, four to a lane group, and are added as warp_sum adds them.  A launch less for every norm + projection of a generation step.  us with
-// that launch in front and so: 16 rows x 12,288 x 4,096 27.8, 26.0; x 22,016 x 4,096 36.9, 35.1; x 10,240 x 8,192 44.8, 42.9; x 6,144 x 2,048 10.4, 8.6; 32 rows
-// x 6,144 x 2,048 11.3, 10.4.  (Both parts of a tile in one wave: x 22,016 36.6.  Above 32 rows the multiplying waves would have to make it: 48 rows 12.8, 15.1.)
+// STAT (up to 32 rows): the row statistic that the epilogue applies is made here, from the rows of A that pass through LDS anyway, by the
+// waves that only move data (a wave for each part of 128 columns of a K-tile), in row_stat_kernel's order (same bits): a lane has one
+// row's column group, its parts stay in registers, four to a lane group, and are added as warp_sum adds them.  A launch less for every
+// norm + projection of a generation step.  us with that launch in front and so: 16 rows x 12,288 x 4,096 27.8, 26.0; x 22,016 x 4,096
+// 36.9, 35.1; x 10,240 x 8,192 44.8, 42.9; x 6,144 x 2,048 10.4, 8.6; 32 rows x 6,144 x 2,048 11.3, 10.4.  (Both parts of a tile in one
+// wave: x 22,016 36.6.  Above 32 rows the multiplying waves would have to make it: 48 rows 12.8, 15.1.)
 template <int EPI, int RT, int NP, bool STAT>
 __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ A, const half_t* __restrict__ W,
                                                    half_t* __restrict__ C, int M, int N, int K, int lda, int ldw,
@@ -461,8 +463,8 @@ __global__ __launch_bounds__(256) void gemm_nt_col16(const half_t* __restrict__ 
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   const int m = wave * 16 + fr;
-  // (of ep itself but for the statistic: of a copy the compiler loads what it needs from the arguments only here, a trip to memory after another: residual
-  // products of up to 3,000 columns 0.3 us slower)
+  // (of ep itself but for the statistic: of a copy the compiler loads what it needs from the arguments only here, a trip to memory after
+  // another: residual products of up to 3,000 columns 0.3 us slower)
   auto finish = [&](const Epi& e) {
     if (wave >= RT || m >= M) return;
     if constexpr (NP == 1) store_one<EPI>(C, ldc, m, n0 + 4 * grp, acc[0], e);
@@ -658,8 +660,8 @@ __global__ __launch_bounds__(256) void ss_partials_kernel(const half_t* __restri
 // the fused norm's statistic straight from x: the 128-column parts of a row with ss_partials_kernel's per-lane FMA chains (one per
 // 4-column group g) combined as row_sum_4groups does, (g0 + g2) + (g1 + g3), and summed in rstd_from_ss_kernel's order
 // (lane j takes parts j, j + 64, ..., then warp_sum): the same bits as fls_row_ss followed by fls_rstd_from_ss, in one launch.
-// What bounds it is one row's chain: four lanes a part, one for each of its column groups, 128 lanes a row (us, a lane for a whole part before: 65 rows
-// of 4,096 3.03 -> 2.58, of 8,192 3.68 -> 2.90, 6,400 of 4,096 14.8 -> 10.7; one row 2.06 -> 2.21).
+// What bounds it is one row's chain: four lanes a part, one for each of its column groups, 128 lanes a row (us, a lane for a whole part
+// before: 65 rows of 4,096 3.03 -> 2.58, of 8,192 3.68 -> 2.90, 6,400 of 4,096 14.8 -> 10.7; one row 2.06 -> 2.21).
 constexpr int ROW_STAT_MAX_PARTS = 128;              // H <= 16,384
 __global__ __launch_bounds__(256) void row_stat_kernel(const half_t* __restrict__ x, int ldx, int M, int nparts, int H,
                                                        float eps, float* __restrict__ rstd) {
@@ -717,11 +719,11 @@ enum Route { ROUTE_NONE, ROUTE_SKINNY, ROUTE_SPLIT, ROUTE_MID, ROUTE_128, ROUTE_
 
 // The blocks that the mid-M path takes.
 enum MidForm { MID_16, MID_16X2, MID_32, MID_64, MID_64_W4, MID_128R, MID_128, MID_128_W4 };
-// Blocks of 16 pairs, or of two 16-column panels, for up to 64 rows.  Up to a round of them the mid blocks leave half of the CUs idle (plain
-// products of up to 128: the 16-column blocks fill them).  Above it, up to 16 rows (plain ones to 32), the mid blocks have the 64-row tile's staging of A to
-// carry, but few K-tiles, or two rounds of the mid blocks that end together (768 .. 1,024), are as fast there (0.98 to 1.27), and with more rows
-// everything above a round is (1.0 to 1.4).  Random products that this rule gives them: 672 pairs 0.70 of the mid blocks' time (worst 1.02), plain
-// ones 0.62 to 0.87 up to a round, 0.83 to 0.95 above.
+// Blocks of 16 pairs, or of two 16-column panels, for up to 64 rows.  Up to a round of them the mid blocks leave half of the CUs idle
+// (plain products of up to 128: the 16-column blocks fill them).  Above it, up to 16 rows (plain ones to 32), the mid blocks have the
+// 64-row tile's staging of A to carry, but few K-tiles, or two rounds of the mid blocks that end together (768 .. 1,024), are as fast
+// there (0.98 to 1.27), and with more rows everything above a round is (1.0 to 1.4).  Random products that this rule gives them: 672 pairs
+// 0.70 of the mid blocks' time (worst 1.02), plain ones 0.62 to 0.87 up to a round, 0.83 to 0.95 above.
 bool two_panels(int M, int N, int K, bool pairs) {
   const int b = N / 32;
   if (b <= 256) return pairs || b > 128;
@@ -762,12 +764,13 @@ MidForm mid_form(int M, int N, int K, bool pairs, bool bn64_ok, bool panels = tr
   return MID_128_W4;
 }
 
-// (The 64-column blocks take 0.92 of what is estimated for them since their K-tiles are of 128 terms.  Fitted anew they took products of 65 to 128 rows from
-// K-split blocks, whose estimates are further off: 1.002 of the time of 180 random ones, up to 1.2, and 0.995, up to 1.04, with these.)
-// The estimates (us).  Fitted to 15,400 random products of 1 .. 3,000 rows, 512 .. 29,440 columns (and a gate / up of 57,344) and 256 .. 28,928 terms,
-// each timed on every path that it can take, with weights that no cache holds; profiles/cases/gemm_routes.txt has the errors of the fits, 5 to 9%
-// each, and what the choice makes of them.  The shortest form that tells the paths apart: a start, and the larger of the weight's stream
-// and the K tiles of 64 terms (nk), which take longer the more blocks pull on memory and power at once.
+// (The 64-column blocks take 0.92 of what is estimated for them since their K-tiles are of 128 terms.  Fitted anew they took products of
+// 65 to 128 rows from K-split blocks, whose estimates are further off: 1.002 of the time of 180 random ones, up to 1.2, and 0.995, up to
+// 1.04, with these.) The estimates (us).  Fitted to 15,400 random products of 1 .. 3,000 rows, 512 .. 29,440 columns (and a gate / up of
+// 57,344) and 256 .. 28,928 terms, each timed on every path that it can take, with weights that no cache holds;
+// profiles/cases/gemm_routes.txt has the errors of the fits, 5 to 9% each, and what the choice makes of them.  The shortest form that
+// tells the paths apart: a start, and the larger of the weight's stream and the K tiles of 64 terms (nk), which take longer the more
+// blocks pull on memory and power at once.
 struct MidCost { float start, k_few, k_full, start2, k2, k2_more, tb; };       // tb: bytes of weight a us, in millions
 const MidCost MID_16_COST[3] = {{4.7f, 0.05f, 0.152f, 7.4f, 0.199f, 0.f, 4.76f}, {5.f, 0.092f, 0.165f, 7.8f, 0.247f, 0.f, 4.97f},
                                 {4.7f, 0.147f, 0.207f, 6.8f, 0.33f, 0.f, 4.99f}};        // up to 16, 32 and 64 rows
@@ -867,8 +870,9 @@ Route route_of(int M, int N, int K, int epi, bool row_exact, size_t ws_bytes) {
     if (M >= 384) offer(ROUTE_V11, rounds_us(ROUNDS[3], M, N, K));
   } else if (best == ROUTE_SKINNY && mid_form(M, N, K, pairs, true) == MID_16X2 &&
              1.04f * mid_us(M, N, K, MID_16X2) < skinny_us(M, N, K, bn, S, true)) {
-    // Two panels take what the mid blocks would, and of the K-split blocks' products those that they are estimated 4% faster for.  2,600 random ones of up to
-    // 64 rows, against the time before there were two panels: 0.896, 6 of them more than 5% slower (no margin: 0.894, 32; each on the faster of the two: 0.890)
+    // Two panels take what the mid blocks would, and of the K-split blocks' products those that they are estimated 4% faster for.  2,600
+    // random ones of up to 64 rows, against the time before there were two panels: 0.896, 6 of them more than 5% slower (no margin: 0.894,
+    // 32; each on the faster of the two: 0.890)
     best = ROUTE_MID;
   }
   return best;
@@ -901,7 +905,8 @@ int launch(const half_t* A, const half_t* W, half_t* C, int M, int N, int K, int
                         ((uintptr_t)C & 7) == 0 && ((uintptr_t)ws & 15) == 0 &&
                         (EPI != FLS_EPI_RESID || (ep.ldr % 4 == 0 && ((uintptr_t)ep.R & 7) == 0));
   if (!main_ok) route = ROUTE_NONE;
-  // The row statistic of A (rs_eps): made by the blocks of 16 pairs where they take the product, have waves for it and registers for its parts, else by a launch here.
+  // The row statistic of A (rs_eps): made by the blocks of 16 pairs where they take the product, have waves for it and registers for its
+  // parts, else by a launch here.
   constexpr bool pairs = EPI != FLS_EPI_NONE && EPI != FLS_EPI_RESID;
   const bool to_mid = mid_ok && (ep.row_exact || route == ROUTE_MID) &&
                       (!main_ok || route == ROUTE_MID || (route == ROUTE_NONE && g_mid && mid_rule(M, tiles256)));

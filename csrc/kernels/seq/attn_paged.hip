@@ -23,13 +23,14 @@
 // one row, so its block walks the (bounded) chunk or window with four waves; a prompt has one block
 // per row and head, which fills the chip without a second kernel.
 //
-// What bounds a decoded row is latency: a key's 16-byte loads came in two or three at a time, a value's columns 2 or 4 bytes a lane.  With KU
-// of a key's 16-byte pieces and eight keys' values in flight: 16 requests of 1,000 keys, 32 heads of 128 on 8, 61.7 -> 45.6 us; 8 of 90 .. 240,
-// 16 heads 10.3 -> 9.4; in fp32 prompts of 400, 300 and 210 rows 217 -> 200.  What bounds many rows is how many waves a SIMD holds, so each form is a
-// kernel of its own (bf16: 64 registers a lane without FOUR, 94 with KU = 4, 87 with 8; both in one 136, and prompts of heads of 96 took 1.4 to
-// 1.8 times as long).  6,500 random calls, mean over the lane = column kernel by heads of values: 32 (KU = 4) 0.64 .. 0.82, with KU = 8 0.73 .. 1.02
-// and up to 1.2; 64 .. 256 (KU = 8) 0.57 .. 0.86, with KU = 4 0 to 3 hundredths more; any other (KU = 1) the same, with KU = 8 up to 1.3.  With blocks
-// (POOL, 4,300 calls) 32 .. 128 (KU = 4) 0.70 .. 0.89, with KU = 8 0.71 .. 0.89 and up to 1.2; 256 (KU = 1) 0.74 .. 0.89, with KU = 8 up to 1.3.
+// What bounds a decoded row is latency: a key's 16-byte loads came in two or three at a time, a value's columns 2 or 4 bytes a lane.  With
+// KU of a key's 16-byte pieces and eight keys' values in flight: 16 requests of 1,000 keys, 32 heads of 128 on 8, 61.7 -> 45.6 us; 8 of 90
+// .. 240, 16 heads 10.3 -> 9.4; in fp32 prompts of 400, 300 and 210 rows 217 -> 200.  What bounds many rows is how many waves a SIMD
+// holds, so each form is a kernel of its own (bf16: 64 registers a lane without FOUR, 94 with KU = 4, 87 with 8; both in one 136, and
+// prompts of heads of 96 took 1.4 to 1.8 times as long).  6,500 random calls, mean over the lane = column kernel by heads of values: 32
+// (KU = 4) 0.64 .. 0.82, with KU = 8 0.73 .. 1.02 and up to 1.2; 64 .. 256 (KU = 8) 0.57 .. 0.86, with KU = 4 0 to 3 hundredths more; any
+// other (KU = 1) the same, with KU = 8 up to 1.3.  With blocks (POOL, 4,300 calls) 32 .. 128 (KU = 4) 0.70 .. 0.89, with KU = 8 0.71 ..
+// 0.89 and up to 1.2; 256 (KU = 1) 0.74 .. 0.89, with KU = 8 up to 1.3.
 #include "seq_common.h"
 #include "fls_seq.h"
 #include "row_vec.h"
@@ -252,12 +253,13 @@ __global__ __launch_bounds__(256) void attn_paged_kernel(const TQ* __restrict__ 
   }
 }
 
-// Few rows (decoding, some requests): what bounds a (row, head) is the chain of one tile -- its keys' page entries, the keys, the weights, the values,
-// each a trip to memory -- and 64 keys a tile gave that chain 200 to 400 keys' work on four waves.  Here sixteen waves take tiles of 16 keys in turn: four
-// lanes share a key, each every fourth 16-byte piece of it, all of a head of 128 in flight at once, and the tile's values are one or two
-// batches of loads.  A row of fewer than 256 keys is one tile a wave.  (aligned rows, FOUR's head sizes, no blocks.)  us in turn, the other kernel with its
-// ranges over twice the blocks, bf16 heads of 128: 128 rows x heads of 220 keys 9.9 -> 8.0, 400 15.5 -> 10.8, 1,000 21.0 -> 17.3; 48 x 400 15.3 -> 10.2, 1,000 18.2
-// -> 11.8; fp32 48 x 400 18.0 -> 11.7; of 210 combinations of 8 to 256 rows x heads, 20 to 4,000 keys, heads of 64 to 256 0.77 of the time.
+// Few rows (decoding, some requests): what bounds a (row, head) is the chain of one tile -- its keys' page entries, the keys, the weights,
+// the values, each a trip to memory -- and 64 keys a tile gave that chain 200 to 400 keys' work on four waves.  Here sixteen waves take
+// tiles of 16 keys in turn: four lanes share a key, each every fourth 16-byte piece of it, all of a head of 128 in flight at once, and the
+// tile's values are one or two batches of loads.  A row of fewer than 256 keys is one tile a wave.  (aligned rows, FOUR's head sizes, no
+// blocks.)  us in turn, the other kernel with its ranges over twice the blocks, bf16 heads of 128: 128 rows x heads of 220 keys 9.9 ->
+// 8.0, 400 15.5 -> 10.8, 1,000 21.0 -> 17.3; 48 x 400 15.3 -> 10.2, 1,000 18.2 -> 11.8; fp32 48 x 400 18.0 -> 11.7; of 210 combinations of
+// 8 to 256 rows x heads, 20 to 4,000 keys, heads of 64 to 256 0.77 of the time.
 template <typename TQ, typename T, typename TO>
 __global__ __launch_bounds__(1024) void attn_few_kernel(const TQ* __restrict__ q, int ldq, const T* __restrict__ kc, int ldk,
                                                         const T* __restrict__ vc, int ldv, TO* __restrict__ out, int ldo,
@@ -443,8 +445,8 @@ static int value_lanes(const void* vc, int ldv, int es, int dv) {
   return dv == 32 ? 3 : dv == 64 ? 4 : dv == 128 ? 5 : dv == 256 ? 6 : -1;
 }
 static bool keys_by_16(const void* kc, int ldk, int es, int d) { return d * es % 16 == 0 && (uintptr_t)kc % 16 == 0 && ldk * es % 16 == 0; }
-// Sixteen waves a (row, head) and range of its keys?  One block a CU (a second one waits: 384 and 512 blocks 1.0 to 1.4 of the other kernel's time) and keys
-// of 256 bytes or more (128 bytes are two loads a lane here and eight there: 0.9 to 1.2)
+// Sixteen waves a (row, head) and range of its keys?  One block a CU (a second one waits: 384 and 512 blocks 1.0 to 1.4 of the other
+// kernel's time) and keys of 256 bytes or more (128 bytes are two loads a lane here and eight there: 0.9 to 1.2)
 static bool few_rows(const void* kc, int ldk, const void* vc, int ldv, int es, int d, int dv, int pool_P, long long blocks) {
   return pool_P == 0 && blocks <= 256 && d * es >= 256 && keys_by_16(kc, ldk, es, d) && value_lanes(vc, ldv, es, dv) >= 0;
 }

@@ -145,9 +145,10 @@ extern "C" int fls_seq_parallel_update(float* x, int ldx, const float* a, int ld
   return 0;
 }
 
-// The update and the next layer's two norms in one pass: a layer's new row is read by nothing else in between.  A row stays in a block's registers, NP
-// pieces of 1,024 columns, and rounds as in the two kernels above, so that a layer that ends a shard gives the same bits.  Bound by its bytes (9,000 rows
-// of 2048: three passes' prompt step 7.27 -> 7.08 ms), for few rows by a launch and its latencies (a captured step of 24 rows, five of them fewer, 672 -> 667 us).
+// The update and the next layer's two norms in one pass: a layer's new row is read by nothing else in between.  A row stays in a block's
+// registers, NP pieces of 1,024 columns, and rounds as in the two kernels above, so that a layer that ends a shard gives the same bits. 
+// Bound by its bytes (9,000 rows of 2048: three passes' prompt step 7.27 -> 7.08 ms), for few rows by a launch and its latencies (a
+// captured step of 24 rows, five of them fewer, 672 -> 667 us).
 template <typename T, int NP>
 __global__ __launch_bounds__(256) void parallel_update_norms_kernel(float* __restrict__ x, int ldx, const float* __restrict__ a, int lda,
                                                                     const float* __restrict__ wa, const float* __restrict__ b, int ldb,

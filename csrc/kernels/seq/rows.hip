@@ -31,11 +31,12 @@ __global__ __launch_bounds__(256) void group_rmsnorm_kernel(const float* __restr
 // reduction.  MODE 0: y = norm(x); 1: y += norm(x); 2: y += norm(x), then h = norm(y; w2) of the new row: a sublayer's
 // post-norm, the residual update and the next sublayer's norm in one pass.  Bound by its bytes from some hundred rows on
 // and by a launch and two memory latencies below.  16384 rows of 4096 in two groups, a column a thread before: norm 146 -> 82 us,
-// residual update 199 -> 140, update and next norm in turn 345, here 182.  SUM: x is a mixture's rows, sorted by expert; row r of the sum is
-// sum_k mw[r, k] x[idx[r, k]], k < top, made on the way in (moe_sum_kernel's order).  MODE 3: as MODE 2, rounded as MODE 1 and then MODE 0, so that a
-// layer's last update gives the same bits with the next layer's norm and without it (16,384 rows of 4096 in three layers 16.42 -> 16.28 ms, a captured
-// step of 8 rows of 2048, three launches fewer, 258 -> 253 us).  MODE 2's rounding, of the update and norm within a layer, is its own.
-// (The fused steps of the sums are spelt out, so that no compiler's choice moves them: the second square first but in MODE 2 of up to 1,024 columns.)
+// residual update 199 -> 140, update and next norm in turn 345, here 182.  SUM: x is a mixture's rows, sorted by expert; row r of the sum
+// is sum_k mw[r, k] x[idx[r, k]], k < top, made on the way in (moe_sum_kernel's order).  MODE 3: as MODE 2, rounded as MODE 1 and then
+// MODE 0, so that a layer's last update gives the same bits with the next layer's norm and without it (16,384 rows of 4096 in three layers
+// 16.42 -> 16.28 ms, a captured step of 8 rows of 2048, three launches fewer, 258 -> 253 us).  MODE 2's rounding, of the update and norm
+// within a layer, is its own. (The fused steps of the sums are spelt out, so that no compiler's choice moves them: the second square first
+// but in MODE 2 of up to 1,024 columns.)
 template <bool X_FIRST>
 __device__ __forceinline__ float squares(const float4& v) {
   return fmaf(v.w, v.w, fmaf(v.z, v.z, X_FIRST ? fmaf(v.y, v.y, v.x * v.x) : fmaf(v.x, v.x, v.y * v.y)));
@@ -320,7 +321,8 @@ extern "C" int fls_seq_add_scaled_dyt(float* x, int ldx, const float* y, int ldy
 
 // ------------------------------------------------------------------------------- embedding
 // (four columns a lane and four of its pieces' loads in flight where the rows allow it: single columns took
-// a load, a wait and a store for each 256: us, 8 rows of 2,048 in bf16 2.5 -> 2.1, of 4,096 3.5 -> 2.2, 1,024 of 4,096 9.1 -> 5.9, 9,000 64.7 -> 35.8)
+// a load, a wait and a store for each 256: us, 8 rows of 2,048 in bf16 2.5 -> 2.1, of 4,096 3.5 -> 2.2, 1,024 of 4,096 9.1 -> 5.9, 9,000
+// 64.7 -> 35.8)
 template <typename T, int VE>
 __global__ __launch_bounds__(256) void embed_kernel(const int* __restrict__ ids, const T* __restrict__ table, float* __restrict__ out, int D, int V, float scale) {
   const int t = blockIdx.x;
@@ -1098,8 +1100,8 @@ extern "C" int fls_seq_moe_route(const float* logits, int ldl, const float* corr
 // Entries to their rows: every block scans the counts for itself (lane l of its first wave sums a run of ceil(E / 64) experts, the runs'
 // starts come from a prefix sum over the lanes), the first one leaves them in offs; it ranks its entries in LDS and takes its places with
 // one atomic per expert (32768 entries of 8 experts: 50 us with an atomic per wave and expert, 6.8 here).
-// SELF (few entries): every block counts all of them for itself, and those of the blocks before it for its places: no counts and cursors that have to be zeroed
-// first, and no atomics on memory (a launch less for each layer with experts of a prompt's portion).
+// SELF (few entries): every block counts all of them for itself, and those of the blocks before it for its places: no counts and cursors
+// that have to be zeroed first, and no atomics on memory (a launch less for each layer with experts of a prompt's portion).
 #define PLACE_THREADS 1024
 template <bool SELF>
 __global__ __launch_bounds__(PLACE_THREADS) void moe_place_kernel(const int* __restrict__ ids, int n, int top, const int* __restrict__ hist, int E,
